@@ -60,8 +60,10 @@ __device__ __forceinline__ void route_wave(const float* __restrict__ z, int expe
 }
 
 // VEC: the prologue keeps its vectors in registers as float4 (k a multiple of 4, at most what the S pieces per thread cover);
-// else any k, through LDS.
-template <typename ET, int R, int S, int PRO, bool VEC>
+// else any k, through LDS.  NT: the weights are read once on this chip and are requested as such (non-temporal): what they
+// would push out of the caches stays, and the stream itself runs faster (16384 x 2048 bfloat16: 14.6 -> 13.9 us, the head of
+// 128256 x 2048 90 -> 82 us).  With several tokens the grid rows share the weights through L2 and the ordinary loads stay.
+template <typename ET, int R, int S, int PRO, bool VEC, bool NT>
 __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
     constexpr int CE = Chunk<ET>::N;
     extern __shared__ __attribute__((aligned(16))) float xs[];     // [kpad] the vector
@@ -105,7 +107,11 @@ __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
     const int nchunk = g.kpad / CE;                       // 16-byte pieces of a row
     const int ng = (g.n + R - 1) / R, G = gridDim.x;      // groups of R rows, dealt to the workgroups in turn
     i32x4 buf[2][R][S];
-    auto piece = [&](int row, int c) { return *reinterpret_cast<const i32x4*>(w + (size_t)min(row, g.n - 1) * g.kpad + c * CE); };
+    auto piece = [&](int row, int c) {
+        const i32x4* p = reinterpret_cast<const i32x4*>(w + (size_t)min(row, g.n - 1) * g.kpad + c * CE);
+        if constexpr (NT) return __builtin_nontemporal_load(p);
+        else return *p;
+    };
     auto load = [&](int b, int grp) {
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -244,7 +250,8 @@ __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
 }
 
 template <typename ET, int R, int S>
-static int launch_gemv_rs(const GemvArgs& g, int pro, int rows_y, hipStream_t st) {
+static int launch_gemv_rs(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
+    const int rows_y = pro == 2 ? tokens * g.top : tokens;
     // workgroups that share the chip at a time (two per CU where the vector takes a third of LDS or more); each walks its
     // groups with the next one's weights in flight
     int wgs = (S > 4 ? 512 : 1024) / rows_y;
@@ -255,8 +262,9 @@ static int launch_gemv_rs(const GemvArgs& g, int pro, int rows_y, hipStream_t st
     const bool vec = g.k % 4 == 0 && g.ldx % 4 == 0 && g.ldy % 4 == 0 && g.ldh % 4 == 0 && g.kpad <= 256 * Chunk<ET>::N * S;
 #define FX_GEMV(PRO)                                                                               \
     do {                                                                                           \
-        if (vec) gemv_float_kernel<ET, R, S, PRO, true><<<grid, 256, lds, st>>>(g);                \
-        else gemv_float_kernel<ET, R, S, PRO, false><<<grid, 256, lds, st>>>(g);                   \
+        if (vec && tokens == 1) gemv_float_kernel<ET, R, S, PRO, true, true><<<grid, 256, lds, st>>>(g); \
+        else if (vec) gemv_float_kernel<ET, R, S, PRO, true, false><<<grid, 256, lds, st>>>(g);    \
+        else gemv_float_kernel<ET, R, S, PRO, false, false><<<grid, 256, lds, st>>>(g);            \
     } while (0)
     if (pro == 0) FX_GEMV(0);
     if constexpr (S <= 4) {                               // longer rows: gemv_float asks for the plain linear only
@@ -275,14 +283,14 @@ int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     FX_REQUIRE(pro != 2 || (g.experts > 0 && g.experts <= kMaxExperts && g.top > 0 && g.top <= kMaxTop && g.top <= g.experts),
                "gemv_float: %d experts, top %d (at most %d, %d)", g.experts, g.top, kMaxExperts, kMaxTop);
     const int per = 256 * Chunk<ET>::N, steps = (g.kpad + per - 1) / per;
-    const int rows_y = pro == 2 ? tokens * g.top : tokens;
-    if (steps == 1) {
-        if ((g.n + 7) / 8 * rows_y >= 512) return launch_gemv_rs<ET, 8, 1>(g, pro, rows_y, st);
-        return launch_gemv_rs<ET, 4, 1>(g, pro, rows_y, st);
-    }
-    if (steps == 2) return launch_gemv_rs<ET, 4, 2>(g, pro, rows_y, st);
-    if (steps > 4 && pro == 0) return launch_gemv_rs<ET, 2, 8>(g, pro, rows_y, st);
-    return launch_gemv_rs<ET, 2, 4>(g, pro, rows_y, st);
+    // Rows per group: four pieces per thread and group where workgroups walk several groups (a group's sums and barrier then
+    // overlap the next group's loads: 16384 x 2048 13.9 us with eight, 12.9 with four; 28672 x 4096 42.2 -> 37.7 us), eight
+    // where a workgroup has a single group anyway (4096 x 4096: 7.65 us with eight, 7.96 with four) and for rows so long
+    // that two rows are eight pieces (2048 x 8192: 8.2 us, 8.4 one row at a time; 4096 x 14336: 21.1 and 23.1).
+    if (steps == 1) return launch_gemv_rs<ET, 4, 1>(g, pro, tokens, st);
+    if (steps == 2) return (g.n + 3) / 4 <= 1024 ? launch_gemv_rs<ET, 4, 2>(g, pro, tokens, st) : launch_gemv_rs<ET, 2, 2>(g, pro, tokens, st);
+    if (steps > 4 && pro == 0) return launch_gemv_rs<ET, 2, 8>(g, pro, tokens, st);
+    return launch_gemv_rs<ET, 2, 4>(g, pro, tokens, st);
 }
 template int gemv_float<bf16_t>(const GemvArgs&, int, int, hipStream_t);
 template int gemv_float<float>(const GemvArgs&, int, int, hipStream_t);
