@@ -34,6 +34,11 @@ template <> struct Chunk<float> {
     }
 };
 
+// Words that workgroups of one launch hand to each other.  The L2 caches of the chip's eight dies do not see each other's lines, so
+// such words go past them both ways; the writer waits for its stores (vmcnt) before it says that they are there.
+__device__ __forceinline__ void store_past(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_past(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
 __device__ __forceinline__ float fma_f(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + exp_f(-v)); }
 

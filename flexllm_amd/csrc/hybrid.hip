@@ -73,7 +73,7 @@ struct flexllm_hybrid {
     // one-token workspace
     float *x0 = nullptr, *xa = nullptr, *xb = nullptr, *proj = nullptr, *f32 = nullptr, *att = nullptr, *y = nullptr, *hn = nullptr, *hid = nullptr, *hs = nullptr, *route = nullptr;
     float *pick_w = nullptr, *scratch = nullptr, *logits = nullptr, *hw = nullptr;
-    int *pick = nullptr, *want = nullptr;
+    int *pick = nullptr, *want = nullptr, *tickets = nullptr;
     float* am_v = nullptr;
     int* am_i = nullptr;
     float* topk_val = nullptr;
@@ -421,6 +421,9 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
     FX_TRY(own(m, m->pick, T * m->max_top));
     FX_TRY(own(m, m->pick_w, T * m->max_top));
     FX_TRY(own(m, m->scratch, (size_t)kAbsorbTokens * m->absorbed + 1));
+    int heads = 1;
+    for (const HybridLayer& L : m->layers) heads = L.d.heads > heads ? L.d.heads : heads;
+    FX_TRY(own(m, m->tickets, (size_t)kAbsorbTokens * heads * kTicketPitch));
     FX_TRY(own(m, m->logits, c.vocab));
     FX_TRY(own(m, m->want, kPieceTokens));
     FX_TRY(own(m, m->am_v, kArgmaxParts));
@@ -547,7 +550,7 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
         FX_TRY(norm_linear(a, L.g1, m->runs[r].again));
         if (L.d.mixer == FLEXLLM_MIX_SHARED_KV) {
             const SharedKvRows<ET> rows = {static_cast<ET*>(s.rows[r]), s.inv_rms[r]};
-            FX_TRY(shared_kv_splits<ET>(L.sd, m->proj, m->max_et, m->f32, nf, L.kv_norm, rows, s.pos, 0, T, m->scratch, m->att, m->max_att, 1, st));
+            FX_TRY(shared_kv_splits<ET>(L.sd, m->proj, m->max_et, m->f32, nf, L.kv_norm, rows, s.pos, 0, T, m->scratch, m->tickets, m->att, m->max_att, 1, st));
         } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {
             ET* rows = static_cast<ET*>(s.rows[r]);
             FX_TRY(latent_decode<ET>(L.ld, m->proj, m->max_et, nf ? m->f32 : nullptr, nf, L.latent_norm, L.cos_t, L.sin_t, static_cast<ET*>(L.uk),
@@ -654,7 +657,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
             if (!flash)
                 for (int t0 = 0; t0 < T; t0 += kAbsorbTokens) {
                     const int n = T - t0 < kAbsorbTokens ? T - t0 : kAbsorbTokens;
-                    FX_TRY(shared_kv_splits<ET>(L.sd, proj + (size_t)t0 * ldp, ldp, nullptr, 0, L.kv_norm, rows, s.pos, t0, n, m->scratch, att + (size_t)t0 * lda, lda, 0, st));
+                    FX_TRY(shared_kv_splits<ET>(L.sd, proj + (size_t)t0 * ldp, ldp, nullptr, 0, L.kv_norm, rows, s.pos, t0, n, m->scratch, m->tickets, att + (size_t)t0 * lda, lda, 0, st));
                 }
         } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {
             ET *cache = static_cast<ET*>(s.rows[r]), *uk = static_cast<ET*>(L.uk), *uv = static_cast<ET*>(L.uv);

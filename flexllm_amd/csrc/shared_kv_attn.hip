@@ -4,7 +4,8 @@
 //
 // Few tokens: a workgroup takes a split of the visible rows for up to GH query heads of a key/value head.  16-byte pieces of a
 // row live in the registers of LPK neighbouring lanes, which sum the score among themselves and then add the same registers,
-// weighted, to their columns; groups of lanes walk over the rows with running maxima of their own and meet at the end.
+// weighted, to their columns; groups of lanes walk over the rows with running maxima of their own and meet at the end.  The
+// split that is done last joins them all.
 // Many tokens: flash-style on v_mfma_f32_32x32x16_bf16 with one LDS tile of rows for both products, the second one reading
 // it transposed (ds_read_b64_tr_b16).  Scores and weights are float32 throughout: the weights enter the second product as
 // the sum of two bfloat16 halves, which keeps 16 bits of each.
@@ -77,20 +78,24 @@ template int shared_kv_store<bf16_t>(const SharedKvDims&, const float*, int, Sha
 template int shared_kv_store<float>(const SharedKvDims&, const float*, int, SharedKvRows<float>, const int*, int, hipStream_t);
 
 // ---- few tokens -----------------------------------------------------------------------------------------------------
-constexpr int kKvSplits = 64, kKvStats = 4;               // most splits; floats behind a split's sums (maximum, weight sum)
+constexpr int kKvSplits = 32, kKvStats = 4;               // most splits; floats behind a split's sums (maximum, weight sum)
 
 static int kv_head_group(const SharedKvDims& d) {         // query heads per workgroup
     const int r = d.heads / d.kv_heads;
     return r >= 4 ? 4 : r >= 2 ? 2 : 1;
 }
-static int kv_split_count(const SharedKvDims& d) {
-    const int gh = kv_head_group(d), blocks = d.kv_heads * ((d.heads / d.kv_heads + gh - 1) / gh);
+// One workgroup per CU.  The position is known on the device only, so workgroups beyond the rows that there are start too, and
+// every split stands in line at the ticket.  32 heads on 8, dim 64, behind a linear: one token at 1531 rows 10.9 us with 32 splits and
+// 17.9 with 64, five tokens at 5 rows 8.4 us with 8 splits each and 17.9 with 32.  Wider workgroups, with as many rows at once
+// in 8 or 16 waves, are no faster (11.4 and 14.7 us): what their waves save in steps they cost to start.
+static int kv_split_count(const SharedKvDims& d, int tokens) {
+    const int gh = kv_head_group(d), blocks = tokens * d.kv_heads * ((d.heads / d.kv_heads + gh - 1) / gh);
     int s = 1;
-    while (s < kKvSplits && s * blocks < 512) s *= 2;
+    while (s < kKvSplits && s * blocks < 256) s *= 2;
     const int most = (d.capacity + 31) / 32;
     return s < most ? s : most;
 }
-size_t shared_kv_scratch(const SharedKvDims& d) { return (size_t)d.heads * kv_split_count(d) * (d.dimp + kKvStats); }
+size_t shared_kv_scratch(const SharedKvDims& d) { return (size_t)d.heads * kv_split_count(d, 1) * (d.dimp + kKvStats); }
 
 // N consecutive float32 (N a multiple of 4, 16-byte aligned), zeros where there are none.
 template <int N>
@@ -110,25 +115,52 @@ __device__ __forceinline__ int kv_splits_used(int n, int rows) { return max((n +
 template <typename ET, int LPK, int GH, int CPL>
 __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, const void* __restrict__ q, int ldq, int q_f32, const float* __restrict__ k, int ldk,
                                                               const float* __restrict__ norm_w, SharedKvRows<ET> c, const int* __restrict__ state, int tok0,
-                                                              int splits, float* __restrict__ part) {
-    constexpr int CE = Chunk<ET>::N, KS = 256 / LPK, U = 4, N = CPL * CE;
-    extern __shared__ __attribute__((aligned(16))) float sums[];   // [4][GH][dimp]
-    __shared__ float sm_m[4][GH], sm_l[4][GH];
+                                                              int splits, float* __restrict__ part, int* __restrict__ tickets, void* __restrict__ o, int ldo, int o_f32) {
+    constexpr int CE = Chunk<ET>::N, NW = 4, NT = 64 * NW, KS = NT / LPK, U = 4, N = CPL * CE;
+    extern __shared__ __attribute__((aligned(16))) float wsp[];    // weights of the splits [GH][kKvSplits], sums [NW][GH][dimp]
+    float* const sums = wsp + GH * kKvSplits;
+    __shared__ float sm_m[NW][GH], sm_l[NW][GH];
+    __shared__ int done;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lc = lane % LPK, ks = wave * (64 / LPK) + lane / LPK;
     const int rep = d.heads / d.kv_heads, hb = (rep + GH - 1) / GH, g = blockIdx.y / hb, h0 = (blockIdx.y % hb) * GH, tok = blockIdx.z;
-    const int base = state[0], pos = base + tok0 + tok, held = k ? base : pos + 1;      // rows 0 .. held-1 are in the cache
-    const int per = kv_split_rows(held, splits), first = blockIdx.x * per, last = min(held, first + per);
-    if ((int)blockIdx.x >= kv_splits_used(held, per) || pos >= d.capacity) return;
-    const ET* rows = c.row + (size_t)g * d.capacity * d.dimp;
-    const float* inv = c.inv_rms + (size_t)g * d.capacity;
     int col[CPL];
     bool in[CPL];
 #pragma unroll
     for (int j = 0; j < CPL; j++) { col[j] = (lc + j * LPK) * CE; in[j] = col[j] < d.dimp; }
+    // ---- what does not hang on the position is requested ahead of it: the queries' columns of this lane, the norms' weights
+    // and this step's rows, which are not in the cache yet (the first split takes them; the first KS of them here)
+    float qv[GH][N], wv[N], xo[N];
+    const bool own = k && blockIdx.x == 0;
+#pragma unroll
+    for (int j = 0; j < CPL; j++) {
+        load_floats<CE>(norm_w + col[j], in[j], wv + j * CE);
+        if (own) load_floats<CE>(k + (size_t)min(ks, tok) * ldk + g * d.dimp + col[j], in[j], xo + j * CE);
+    }
+#pragma unroll
+    for (int h = 0; h < GH; h++) {
+        const size_t at = (size_t)tok * ldq + (size_t)(g * rep + min(h0 + h, rep - 1)) * d.dimp;
+#pragma unroll
+        for (int j = 0; j < CPL; j++) {
+            if (q_f32) {
+                load_floats<CE>(static_cast<const float*>(q) + at + col[j], in[j], &qv[h][j * CE]);
+            } else {
+                uint4 u = make_uint4(0, 0, 0, 0);
+                if (in[j]) u = *reinterpret_cast<const uint4*>(static_cast<const ET*>(q) + at + col[j]);
+                Chunk<ET>::unpack(u, reinterpret_cast<float (&)[CE]>(qv[h][j * CE]));
+            }
+        }
+    }
+    const int base = state[0], pos = base + tok0 + tok, held = k ? base : pos + 1;      // rows 0 .. held-1 are in the cache
+    const int per = kv_split_rows(held, splits), first = blockIdx.x * per, last = min(held, first + per), ns = kv_splits_used(held, per);
+    if ((int)blockIdx.x >= ns || pos >= d.capacity) return;
+    const ET* rows = c.row + (size_t)g * d.capacity * d.dimp;
+    const float* inv = c.inv_rms + (size_t)g * d.capacity;
 
+    auto rows_at = [&](int b, int i) { return i == 0 || first + (b * U + i) * KS < last; };     // otherwise nobody has a row there
     auto load = [&](int b, i32x4 (&u)[U][CPL], float (&r)[U]) {
 #pragma unroll
         for (int i = 0; i < U; i++) {
+            if (!rows_at(b, i)) break;
             const int key = min(first + (b * U + i) * KS + ks, last - 1);
 #pragma unroll
             for (int j = 0; j < CPL; j++) u[i][j] = in[j] ? *reinterpret_cast<const i32x4*>(rows + (size_t)key * d.dimp + col[j]) : i32x4{0, 0, 0, 0};
@@ -140,27 +172,12 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
     const int nb = last > first ? (last - first + U * KS - 1) / (U * KS) : 0;
     if (nb > 0) load(0, ua, ra);
 
-    // ---- the queries' columns of this lane, normed and scaled
-    float qv[GH][N];
+    // ---- the queries, normed and scaled
     {
-        float wv[N];
-#pragma unroll
-        for (int j = 0; j < CPL; j++) load_floats<CE>(norm_w + col[j], in[j], wv + j * CE);
         const float f = query_factor(d, pos);
 #pragma unroll
         for (int h = 0; h < GH; h++) {
-            const size_t at = (size_t)tok * ldq + (size_t)(g * rep + min(h0 + h, rep - 1)) * d.dimp;
             float ss = 0.0f;
-#pragma unroll
-            for (int j = 0; j < CPL; j++) {
-                if (q_f32) {
-                    load_floats<CE>(static_cast<const float*>(q) + at + col[j], in[j], &qv[h][j * CE]);
-                } else {
-                    uint4 u = make_uint4(0, 0, 0, 0);
-                    if (in[j]) u = *reinterpret_cast<const uint4*>(static_cast<const ET*>(q) + at + col[j]);
-                    Chunk<ET>::unpack(u, reinterpret_cast<float (&)[CE]>(qv[h][j * CE]));
-                }
-            }
 #pragma unroll
             for (int e = 0; e < N; e++) ss = fma_f(qv[h][e], qv[h][e], ss);
             const float s = f / sqrtf(group_sum<LPK>(ss) / (float)d.dim + d.eps);
@@ -187,6 +204,11 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
         float s[GH][U];
 #pragma unroll
         for (int i = 0; i < U; i++) {
+            if (!rows_at(b, i)) {
+#pragma unroll
+                for (int h = 0; h < GH; h++) s[h][i] = -INFINITY;
+                continue;
+            }
             float x[N];
 #pragma unroll
             for (int j = 0; j < CPL; j++) Chunk<ET>::unpack(make_uint4(u[i][j][0], u[i][j][1], u[i][j][2], u[i][j][3]), reinterpret_cast<float (&)[CE]>(x[j * CE]));
@@ -212,6 +234,7 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
         }
 #pragma unroll
         for (int i = 0; i < U; i++) {
+            if (!rows_at(b, i)) break;
             float x[N];
 #pragma unroll
             for (int j = 0; j < CPL; j++) Chunk<ET>::unpack(make_uint4(u[i][j][0], u[i][j][1], u[i][j][2], u[i][j][3]), reinterpret_cast<float (&)[CE]>(x[j * CE]));
@@ -228,14 +251,18 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
         if (b + 2 < nb) load(b + 2, ua, ra);
         take(b + 1, ub, rb);
     }
-    // ---- rows of this step, which are not in the cache yet: taken by the first split, stored by their own token
-    if (k && blockIdx.x == 0) {
+    // ---- rows of this step: stored by their own token
+    if (own) {
         for (int n0 = 0; n0 <= tok; n0 += KS) {
-            const int n = min(n0 + ks, tok);
-            const float* src = k + (size_t)n * ldk + g * d.dimp;
+            const float* src = k + (size_t)min(n0 + ks, tok) * ldk + g * d.dimp;
             float x[N], ss = 0.0f;
 #pragma unroll
-            for (int j = 0; j < CPL; j++) load_floats<CE>(src + col[j], in[j], x + j * CE);
+            for (int j = 0; j < CPL; j++) {
+                if (n0 > 0) load_floats<CE>(src + col[j], in[j], x + j * CE);
+                else
+#pragma unroll
+                    for (int e = 0; e < CE; e++) x[j * CE + e] = xo[j * CE + e];
+            }
 #pragma unroll
             for (int e = 0; e < N; e++) {
                 ss = fma_f(x[e], x[e], ss);
@@ -257,8 +284,8 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
             }
 #pragma unroll
             for (int h = 0; h < GH; h++) {
-                const float v = score(x, h) * r, s = mine ? v : -INFINITY;
-                const float mx = fmaxf(m[h], s), al = __builtin_amdgcn_exp2f(m[h] - mx), p = __builtin_amdgcn_exp2f(s - mx);
+                const float v = score(x, h) * r, sc = mine ? v : -INFINITY;
+                const float mx = fmaxf(m[h], sc), al = __builtin_amdgcn_exp2f(m[h] - mx), p = __builtin_amdgcn_exp2f(sc - mx);
                 m[h] = mx;
                 l[h] = l[h] * al + p;
 #pragma unroll
@@ -276,7 +303,9 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < GH; h++) {
-        mt[h] = fmaxf(fmaxf(sm_m[0][h], sm_m[1][h]), fmaxf(sm_m[2][h], sm_m[3][h]));
+        mt[h] = sm_m[0][h];
+#pragma unroll
+        for (int i = 1; i < NW; i++) mt[h] = fmaxf(mt[h], sm_m[i][h]);
         const float w = __builtin_amdgcn_exp2f(m[h] - mt[h]);
         const float lw = wave_sum(lc == 0 ? l[h] * w : 0.0f);
         if (lane == 0) sm_l[wave][h] = lw;
@@ -307,81 +336,114 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
                     if (in[j]) sums[(wave * GH + h) * d.dimp + col[j] + e] = acc[h][j * CE + e];
     }
     __syncthreads();
-    const int ld = d.dimp + kKvStats, step = GH * d.dimp;
-    for (int i = t; i < step; i += 256) {
-        const int h = i / d.dimp, e = i - h * d.dimp;
-        if (h0 + h < rep)
-            part[(((size_t)tok * d.heads + g * rep + h0 + h) * splits + blockIdx.x) * ld + e] = (sums[i] + sums[step + i]) + (sums[2 * step + i] + sums[3 * step + i]);
-    }
-    if (t < GH && h0 + t < rep) {
-        float* o = part + (((size_t)tok * d.heads + g * rep + h0 + t) * splits + blockIdx.x) * ld + d.dimp;
-        o[0] = fmaxf(fmaxf(sm_m[0][t], sm_m[1][t]), fmaxf(sm_m[2][t], sm_m[3][t]));
-        o[1] = (sm_l[0][t] + sm_l[1][t]) + (sm_l[2][t] + sm_l[3][t]);
-    }
-}
-
-// Join the splits of one (token, head); here the sink enters the sum of the weights.
-template <typename OT>
-__global__ __launch_bounds__(256) void shared_kv_join_kernel(SharedKvDims d, const float* __restrict__ part, const int* __restrict__ state, int tok0, int held_only,
-                                                             int splits, OT* __restrict__ o, int ldo) {
-    __shared__ float wsp[kKvSplits];
-    __shared__ float sums[256];
-    const int t = threadIdx.x, lane = t & 63, h = blockIdx.x, tok = blockIdx.y, ld = d.dimp + kKvStats;
-    const int pos = state[0] + tok0 + tok, held = held_only ? state[0] : pos + 1;
-    if (pos >= d.capacity) return;
-    const int ns = kv_splits_used(held, kv_split_rows(held, splits));
-    const float* p = part + ((size_t)tok * d.heads + h) * splits * ld;
-    {
-        const float ms = lane < ns ? p[lane * ld + d.dimp] : -1e30f, ls = lane < ns ? p[lane * ld + d.dimp + 1] : 0.0f;
-        float m = wave_max(ms);
-        if (d.sink) m = fmaxf(m, 0.0f);
-        const float w = lane < ns ? __builtin_amdgcn_exp2f(ms - m) : 0.0f;
-        float l = wave_sum(ls * w);
-        if (d.sink) l += __builtin_amdgcn_exp2f(-m);
-        if (t < 64) wsp[lane] = w / l;
-    }
-    __syncthreads();
-    int width = 64;                                       // threads that share a split's columns
-    while (width < d.dim && width < 256) width *= 2;
-    const int parts = 256 / width, my = t / width;
-    for (int c0 = 0; c0 < d.dim; c0 += width) {
-        const int e = c0 + t % width;
-        float v = 0.0f;
-        if (e < d.dim)
-#pragma unroll 16
-            for (int s = my; s < ns; s += parts) v = fma_f(p[s * ld + e], wsp[s], v);
-        sums[t] = v;
+    // ---- a split's sums to where the last one finds them: past the caches of the dies, which do not see each other's lines
+    const int ld = d.dimp + kKvStats, step = GH * d.dimp, nh = min(GH, rep - h0), head0 = g * rep + h0;
+    auto split_at = [&](int h, int sp) { return part + (((size_t)tok * d.heads + head0 + h) * splits + sp) * ld; };
+    auto of_waves = [&](const float* p, int stride) {     // sum over the waves, neighbours first
+        float v[NW];
+#pragma unroll
+        for (int i = 0; i < NW; i++) v[i] = p[i * stride];
+#pragma unroll
+        for (int n = NW / 2; n >= 1; n /= 2)
+#pragma unroll
+            for (int i = 0; i < n; i++) v[i] = v[2 * i] + v[2 * i + 1];
+        return v[0];
+    };
+    if (ns > 1) {
+        for (int i = t; i < nh * d.dimp; i += NT) store_past(split_at(i / d.dimp, blockIdx.x) + i % d.dimp, of_waves(sums + i, step));
+        if (lane == 0 && wave < nh) {
+            float* p = split_at(wave, blockIdx.x) + d.dimp;
+            float mj = sm_m[0][wave];
+#pragma unroll
+            for (int i = 1; i < NW; i++) mj = fmaxf(mj, sm_m[i][wave]);
+            store_past(p, mj);
+            store_past(p + 1, of_waves(&sm_l[0][wave], GH));
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): this wave's sums have arrived
         __syncthreads();
-        if (my == 0 && e < d.dim) {
-            for (int i = 1; i < parts; i++) v += sums[i * width + t];
-            o[(size_t)tok * ldo + h * d.dim + e] = (OT)v;
+        if (t == 0) {
+            int* ticket = tickets + ((size_t)tok * gridDim.y + blockIdx.y) * kTicketPitch;
+            done = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+            if (done == ns) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // for the next launch
         }
         __syncthreads();
+        if (done != ns) return;
+    }
+    // ---- the join, one wave per head for the weights; here the sink enters the sum of the weights.  The first columns of all
+    // splits are requested ahead of that: one trip to memory instead of three.
+    const int outs = nh * d.dim;
+    float u[kKvSplits];
+    auto request = [&](int i) {
+        const int h = min(i / d.dim, nh - 1), e = i % d.dim;
+#pragma unroll
+        for (int j = 0; j < kKvSplits; j += 8) {
+            if (j >= ns) break;
+#pragma unroll
+            for (int n = j; n < j + 8; n++) u[n] = load_past(split_at(h, min(n, ns - 1)) + e);
+        }
+    };
+    if (ns > 1) request(t);
+    if (wave < nh) {
+        float ms = -1e30f, ls = 0.0f;
+        if (ns == 1) {
+            if (lane < NW) { ms = sm_m[lane][wave]; ls = sm_l[lane][wave]; }      // the waves' sums have one maximum already
+        } else if (lane < ns) {
+            const float* p = split_at(wave, lane) + d.dimp;
+            ms = load_past(p);
+            ls = load_past(p + 1);
+        }
+        const float top = wave_max(ms), mj = d.sink ? fmaxf(top, 0.0f) : top;
+        float w = lane < ns ? __builtin_amdgcn_exp2f(ms - mj) : 0.0f;
+        if (ns == 1) w = __builtin_amdgcn_exp2f(top - mj);
+        float lj = wave_sum(ls * w);
+        if (d.sink) lj += __builtin_amdgcn_exp2f(-mj);
+        if (lane < kKvSplits) wsp[wave * kKvSplits + lane] = w / lj;
+    }
+    static_assert(GH <= NW && kKvSplits <= 64 && kKvSplits % 8 == 0, "a wave per head, a lane per split");
+    __syncthreads();
+    for (int i = t; i < outs; i += NT) {
+        const int h = i / d.dim, e = i - h * d.dim;
+        float v = 0.0f;
+        if (ns == 1) {
+            v = of_waves(sums + h * d.dimp + e, step) * wsp[h * kKvSplits];
+        } else {
+            if (i >= NT) request(i);
+#pragma unroll
+            for (int j = 0; j < kKvSplits; j += 8) {
+                if (j >= ns) break;
+#pragma unroll
+                for (int n = j; n < j + 8; n++) v = fma_f(u[n], wsp[h * kKvSplits + n], v);      // weight 0 beyond the last split
+            }
+        }
+        const size_t out = (size_t)tok * ldo + (size_t)(head0 + h) * d.dim + e;
+        if (o_f32) static_cast<float*>(o)[out] = v;
+        else static_cast<ET*>(o)[out] = (ET)v;
     }
 }
 
 template <typename ET, int LPK, int GH, int CPL>
 static int launch_splits(const SharedKvDims& d, const void* q, int ldq, const float* k, int ldk, const float* norm_w, const SharedKvRows<ET>& c,
-                         const int* state, int tok0, int tokens, float* scratch, int f32, hipStream_t st) {
-    const int splits = kv_split_count(d), rep = d.heads / d.kv_heads;
+                         const int* state, int tok0, int tokens, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
+    const int splits = kv_split_count(d, tokens), rep = d.heads / d.kv_heads;
     const dim3 grid(splits, d.kv_heads * ((rep + GH - 1) / GH), tokens);
-    shared_kv_split_kernel<ET, LPK, GH, CPL><<<grid, 256, 4 * GH * d.dimp * sizeof(float), st>>>(d, q, ldq, f32, k, ldk, norm_w, c, state, tok0, splits, scratch);
+    const size_t lds = GH * (kKvSplits + 4 * (size_t)d.dimp) * sizeof(float);
+    shared_kv_split_kernel<ET, LPK, GH, CPL><<<grid, 256, lds, st>>>(d, q, ldq, f32, k, ldk, norm_w, c, state, tok0, splits, scratch, tickets, o, ldo, f32);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
 
 template <typename ET>
 int shared_kv_splits(const SharedKvDims& d, const void* q, int ldq, const float* k, int ldk, const float* norm_w, SharedKvRows<ET> c, const int* state,
-                     int tok0, int tokens, float* scratch, void* o, int ldo, int f32, hipStream_t st) {
-    FX_REQUIRE(q && norm_w && c.row && c.inv_rms && state && scratch && o && tokens > 0 && (!k || tok0 == 0), "shared_kv_splits: null pointer, or %d tokens at %d", tokens, tok0);
+                     int tok0, int tokens, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
+    FX_REQUIRE(q && norm_w && c.row && c.inv_rms && state && scratch && tickets && o && tokens > 0 && (!k || tok0 == 0), "shared_kv_splits: null pointer, or %d tokens at %d", tokens, tok0);
     FX_REQUIRE(d.heads % d.kv_heads == 0 && d.dimp % 8 == 0 && d.dimp >= d.dim && d.dimp <= 512 && ldq % (f32 ? 4 : 8) == 0 && ldk % 4 == 0,
                "shared_kv_splits: %d heads on %d, rows of %d, strides %d %d", d.heads, d.kv_heads, d.dimp, ldq, ldk);
     const int chunks = d.dimp / Chunk<ET>::N, gh = kv_head_group(d);
     int rc;
 #define FX_SPLITS(LPK, CPL)                                                                                                                \
-    (gh == 4   ? launch_splits<ET, LPK, 4, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, f32, st)                    \
-     : gh == 2 ? launch_splits<ET, LPK, 2, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, f32, st)                    \
-               : launch_splits<ET, LPK, 1, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, f32, st))
+    (gh == 4   ? launch_splits<ET, LPK, 4, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st)                    \
+     : gh == 2 ? launch_splits<ET, LPK, 2, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st)                    \
+               : launch_splits<ET, LPK, 1, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st))
     if (chunks <= 8) rc = FX_SPLITS(8, 1);
     else if (chunks <= 16) rc = FX_SPLITS(16, 1);
     else if (chunks <= 32) rc = FX_SPLITS(32, 1);
@@ -389,16 +451,10 @@ int shared_kv_splits(const SharedKvDims& d, const void* q, int ldq, const float*
     else if constexpr (std::is_same<ET, float>::value) rc = FX_SPLITS(64, 2);
     else rc = FLEXLLM_EINVAL;                             // not reached: rows of 512 are 64 pieces
 #undef FX_SPLITS
-    if (rc) return rc;
-    const int splits = kv_split_count(d);
-    const dim3 grid(d.heads, tokens);
-    if (f32) shared_kv_join_kernel<float><<<grid, 256, 0, st>>>(d, scratch, state, tok0, k != nullptr, splits, static_cast<float*>(o), ldo);
-    else shared_kv_join_kernel<ET><<<grid, 256, 0, st>>>(d, scratch, state, tok0, k != nullptr, splits, static_cast<ET*>(o), ldo);
-    FX_LAUNCH_CHECK();
-    return FLEXLLM_OK;
+    return rc;
 }
-template int shared_kv_splits<bf16_t>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<bf16_t>, const int*, int, int, float*, void*, int, int, hipStream_t);
-template int shared_kv_splits<float>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<float>, const int*, int, int, float*, void*, int, int, hipStream_t);
+template int shared_kv_splits<bf16_t>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<bf16_t>, const int*, int, int, float*, int*, void*, int, int, hipStream_t);
+template int shared_kv_splits<float>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<float>, const int*, int, int, float*, int*, void*, int, int, hipStream_t);
 
 // ---- many tokens ----------------------------------------------------------------------------------------------------
 // Workgroup: NW waves x 32 queries over tiles of 64 rows.  The queries of a key/value head are numbered token by token, the

@@ -41,3 +41,13 @@ def check_lopazen(cfg, dtype, n, *cuts, max_pos=512):
 @pytest.mark.parametrize("width,vocab", [(64, 4), (2048, 8191), (2112, 4096), (2112, 4097), (2304, 8301), (4096, 4099), (4160, 515)])
 def test_one_token_linears(width, vocab, dtype):
     check_lopazen(lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(97))], width=width, vocab=vocab), dtype, 6, [1], [3])
+
+
+# splits of the rows in the step kernel: one split, the first two, a last one of one row, more columns than threads, several
+# tokens (fewer splits each) ahead of and behind the borders
+@BOTH
+@pytest.mark.parametrize("heads,kv_heads,dim", [(8, 2, 64), (8, 1, 128), (3, 3, 264), (2, 1, 8)])
+def test_few_token_attention_splits(heads, kv_heads, dim, dtype):
+    cfg = lc.config([lc.layer(heads=heads, kv_heads=kv_heads, dim=dim, scale=0.8 * dim ** -0.5)])
+    check_lopazen(cfg, dtype, 75, [1], [31, 1, 1, 8, 5], [3, 8])
+    check_lopazen(cfg, dtype, 1100, [1021, 2, 1, 1, 8, 7, 1], max_pos=1100)
