@@ -103,6 +103,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const GemmTile&
         }
 }
 
+// A stage is 128 bytes of k of the tile's rows and columns; STAGES of them form the ring in LDS.
+// What bounds it: with one workgroup per CU the trip of a stage's bytes, so that everything LDS holds is in flight (two stages of
+// 128 x 128 in four waves, two workgroups per CU: 213 us for 777 x 4096 x 14336; four stages, eight waves: 117 us), and for the
+// largest tile LDS itself, which hands out 6 KiB of operands for 8 matrix instructions per wave.
 template <int BM, int BN, int STAGES, int WPE, int NW>
 __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g, int tiles_m, int tiles_n) {
     constexpr int BKB = 128, GW = NW, WGN = GW / 2;
@@ -294,12 +298,25 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         FX_LAUNCH_CHECK();
         g.n = g.n_split;
     }
-    auto tiles = [&](int bm, int bn) { return ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn); };
-    const int t256 = tiles(256, 256);
-    if (t256 >= 256 && (t256 % 256 == 0 || t256 >= 1024)) return launch_bf16<256, 256, 2, 2, 8>(g, st);
-    if (tiles(128, 128) >= 256) return launch_bf16<128, 128, 2, 2, 4>(g, st);
-    if (tiles(64, 64) >= 768) return launch_bf16<64, 64, 3, 3, 4>(g, st);
-    return launch_bf16<64, 64, 4, 2, 4>(g, st);
+    // The tile whose rounds over the chip (a workgroup per CU) take the least time.  Cost of a round per 64 k, in 0.01 us, as
+    // measured where all CUs are busy: 256 x 256 2.1 us, 128 x 256 1.1 us, 128 x 128 0.6 us, 64 x 128 0.4 us, 64 x 64 0.28 us.  So 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us;
+    // 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3 rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336
+    // 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048 64 x 128 (14.8 us; 128 x 128: 19.4 us).
+    struct Tile { int bm, bn, cost; };
+    constexpr Tile tiles[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}};
+    long best = 0;
+    int pick = -1;
+    for (int i = 0; i < 5; i++) {
+        const long n = (long)((g.m + tiles[i].bm - 1) / tiles[i].bm) * ((g.n + tiles[i].bn - 1) / tiles[i].bn), cost = (n + 255) / 256 * tiles[i].cost;
+        if (pick < 0 || cost < best) { best = cost; pick = i; }
+    }
+    switch (pick) {
+        case 0: return launch_bf16<256, 256, 2, 2, 8>(g, st);
+        case 1: return launch_bf16<128, 256, 3, 2, 8>(g, st);
+        case 2: return launch_bf16<128, 128, 4, 2, 8>(g, st);
+        case 3: return launch_bf16<64, 128, 4, 2, 8>(g, st);
+        default: return launch_bf16<64, 64, 4, 2, 4>(g, st);
+    }
 }
 
 template <int BM>

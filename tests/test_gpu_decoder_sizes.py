@@ -51,3 +51,24 @@ def test_few_token_attention_splits(heads, kv_heads, dim, dtype):
     cfg = lc.config([lc.layer(heads=heads, kv_heads=kv_heads, dim=dim, scale=0.8 * dim ** -0.5)])
     check_lopazen(cfg, dtype, 75, [1], [31, 1, 1, 8, 5], [3, 8])
     check_lopazen(cfg, dtype, 1100, [1021, 2, 1, 1, 8, 7, 1], max_pos=1100)
+
+
+# every tile of the GEMM: one k-stage, fewer and more than the ring holds, rows and columns that do not fill the last tile
+@pytest.mark.parametrize("k", [64, 128, 256, 448])
+@pytest.mark.parametrize("m,n,split,glu", [(1024, 16380, 16380, 0), (1021, 16384, 16384, 1), (1100, 16384, 16000, 0), (1000, 4000, 4000, 2), (897, 4096, 0, 0),
+                                           (1000, 2040, 1024, 0), (961, 2048, 2048, 1), (65, 1028, 1028, 0), (1, 64, 0, 0)])
+def test_gemm_tiles(m, n, split, glu, k):
+    from flexllm_amd import ops, to_device
+    from flexllm_amd.loader import from_bf16, to_bf16
+    from oracle import nifunex_ref
+    r = np.random.default_rng(m + n + k)
+    a, w = [lc.round_bf16(r.standard_normal(s)) for s in ((m, k), (n, k))]
+    y, y32 = ops.linear_float(to_device(to_bf16(a)), to_device(to_bf16(w)), split, glu, 3.0)
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    # float32 sums of k products of O(1): 1e-5 of sqrt(k); a bfloat16 result is within 2^-9 of the value, the unit's slope is at most 1.2
+    if split:
+        g, u = want[:, 0:split:2], want[:, 1:split:2]
+        first = want[:, :split] if not glu else nifunex_ref.clamped_glu(g, u, 3.0) if glu == 1 else lopazen_ref.gelu(g) * u
+        assert np.all(np.abs(from_bf16(y.numpy()) - first) <= 5e-3 * (np.abs(first) + np.sqrt(k)))
+    if split < n:
+        assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * (np.abs(want[:, split:]) + np.sqrt(k)))
