@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import lopazen_cases as lc
-from oracle import lopazen_ref
+import nifunex_cases as nc
+from oracle import lopazen_ref, nifunex_ref
 
 pytestmark = pytest.mark.gpu
 BOTH = pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
@@ -23,17 +24,28 @@ def logits(model, toks, cuts, max_pos=512):
     return np.concatenate(out)
 
 
-def check_lopazen(cfg, dtype, n, *cuts, max_pos=512):
-    from flexllm_amd.lopazen import Lopazen
-    w, toks = lc.weights(cfg, 11), lc.tokens(cfg, n)
-    want = lopazen_ref.Reference(cfg, w).run(toks)
-    m = Lopazen.from_tensors(cfg, w, dtype=dtype, max_pos=max_pos)
+def check(cls, w, toks, want, cfg, dtype, cuts, max_pos, skip=0.0):
+    """skip: share of the places that a close call of a router may leave out."""
+    m = cls.from_tensors(cfg, w, dtype=dtype, max_pos=max_pos)
     for c in cuts:
         got = logits(m, toks, c)
         assert np.isfinite(got).all(), c
         err = lc.rel_err(got, want)
-        assert err.max() < lc.LIMIT[dtype], "portions %s: error %.3g at place %d" % (c, err.max(), err.argmax())
+        worst = np.sort(err)[:len(err) - int(skip * len(err))].max()
+        assert worst < lc.LIMIT[dtype], "portions %s: error %.3g (all places: %.3g at %d)" % (c, worst, err.max(), err.argmax())
     m.close()
+
+
+def check_lopazen(cfg, dtype, n, *cuts, max_pos=512):
+    from flexllm_amd.lopazen import Lopazen
+    w, toks = lc.weights(cfg, 11), lc.tokens(cfg, n)
+    check(Lopazen, w, toks, lopazen_ref.Reference(cfg, w).run(toks), cfg, dtype, cuts, max_pos)
+
+
+def check_nifunex(cfg, dtype, n, *cuts, max_pos=512, skip=0.0):
+    from flexllm_amd.nifunex import Nifunex
+    w, toks = nc.weights(cfg, 11), nc.tokens(cfg, n)
+    check(Nifunex, w, toks, nifunex_ref.Reference(cfg, w).run(toks), cfg, dtype, cuts, max_pos, skip if dtype == "bfloat16" else 0.0)
 
 
 # rows and lengths of the one-token linears: rows per group and pieces per thread change with both
@@ -60,7 +72,6 @@ def test_few_token_attention_splits(heads, kv_heads, dim, dtype):
 def test_gemm_tiles(m, n, split, glu, k):
     from flexllm_amd import ops, to_device
     from flexllm_amd.loader import from_bf16, to_bf16
-    from oracle import nifunex_ref
     r = np.random.default_rng(m + n + k)
     a, w = [lc.round_bf16(r.standard_normal(s)) for s in ((m, k), (n, k))]
     y, y32 = ops.linear_float(to_device(to_bf16(a)), to_device(to_bf16(w)), split, glu, 3.0)
@@ -72,3 +83,11 @@ def test_gemm_tiles(m, n, split, glu, k):
         assert np.all(np.abs(from_bf16(y.numpy()) - first) <= 5e-3 * (np.abs(first) + np.sqrt(k)))
     if split < n:
         assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * (np.abs(want[:, split:]) + np.sqrt(k)))
+
+
+# grouped products of the experts: tiles of 64 and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
+@BOTH
+@pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70)])
+def test_grouped_tiles(experts, top, ff, tokens, dtype):
+    cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=192)
+    check_nifunex(cfg, dtype, tokens, [tokens], skip=0.05)
