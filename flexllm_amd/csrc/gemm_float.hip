@@ -6,7 +6,10 @@
 // matrix each (experts), the epilogue adds a bias, splits the columns between an ET and a float32 output and applies the
 // gated unit to interleaved gate/up columns.
 //
-// float32: v_mfma_f32_32x32x2_f32 (full float32 products and sums) on register-staged 64x64 tiles, same epilogue.
+// float32: the same kernel on v_mfma_f32_32x32x2_f32 (full float32 products and sums).  The 16 bytes that a lane holds are four k of
+// a row, and instruction e of four takes its e-th: the two halves of the wave then stand for k apart, the same ones in
+// both operands, and a sum does not mind.  (A register-staged 64 x 64 tile, which this took the place of: 333 x 2048 x 8192 345 us,
+// now 173; 2048 x 4096 x 4096 950 us, now 602.)
 #include "float_ops.h"
 #include "gemm_i8.h"
 
@@ -107,8 +110,8 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const GemmTile&
 // What bounds it: with one workgroup per CU the trip of a stage's bytes, so that everything LDS holds is in flight (two stages of
 // 128 x 128 in four waves, two workgroups per CU: 213 us for 777 x 4096 x 14336; four stages, eight waves: 117 us), and for the
 // largest tile LDS itself, which hands out 6 KiB of operands for 8 matrix instructions per wave.
-template <int BM, int BN, int STAGES, int WPE, int NW>
-__global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g, int tiles_m, int tiles_n) {
+template <typename ET, int BM, int BN, int STAGES, int WPE, int NW>
+__global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g, int tiles_m, int tiles_n) {
     constexpr int BKB = 128, GW = NW, WGN = GW / 2;
     constexpr int WM = BM / 2, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     constexpr int CPR = BKB / 16, RPI = 64 / CPR;
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
     const int8_t* const a = static_cast<const int8_t*>(g.a);
-    const int8_t* const w = static_cast<const int8_t*>(g.w) + (size_t)tl.group * g.w_stride * sizeof(bf16_t);
+    const int8_t* const w = static_cast<const int8_t*>(g.w) + (size_t)tl.group * g.w_stride * sizeof(ET);
 
     unsigned offa[A_INSTR], offb[B_INSTR];
 #pragma unroll
@@ -133,12 +136,12 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
         const int r = (wave * A_INSTR + j) * RPI + lane / CPR;
         int row = min(tl.row0 + r, tl.row_end - 1);
         if (g.row_src) row = g.row_src[row];
-        offa[j] = (unsigned)row * (unsigned)g.lda * 2u + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
+        offa[j] = (unsigned)row * (unsigned)(g.lda * sizeof(ET)) + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
     }
 #pragma unroll
     for (int j = 0; j < B_INSTR; j++) {
         const int r = (wave * B_INSTR + j) * RPI + lane / CPR;
-        offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)g.ldw * 2u + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
+        offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)(g.ldw * sizeof(ET)) + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
     }
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)gemm_smem;
     auto issue_stage = [&](int kt) {
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-    const int nk = g.k * 2 / BKB;
+    const int nk = g.k * (int)sizeof(ET) / BKB;
     constexpr int PER = A_INSTR + B_INSTR;
     // everything the compiler loaded itself (tile table, gathered row numbers) has to be in before the counted loads start
     gemm_wait_vmcnt<0>();
@@ -166,25 +169,33 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
     for (int s0 = 0; s0 < STAGES - 1; s0++)
         if (s0 < nk) issue_stage(s0);
     const int fr = lane & 31, fg = lane >> 5;
-    auto read_frags = [&](int kt, int ks, bf16x8 (&fa)[TM], bf16x8 (&fb)[TN]) {
+    using Frag = std::conditional_t<std::is_same<ET, float>::value, f32x4, bf16x8>;
+    auto read_frags = [&](int kt, int ks, Frag (&fa)[TM], Frag (&fb)[TN]) {
         const int8_t* sa = gemm_smem + (kt % STAGES) * STAGE;
         const int8_t* sb = sa + BM * BKB;
 #pragma unroll
         for (int i = 0; i < TM; i++) {
             const int r = wm + i * 32 + fr;
-            fa[i] = *reinterpret_cast<const bf16x8*>(sa + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
+            fa[i] = *reinterpret_cast<const Frag*>(sa + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
         }
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int r = wn + j * 32 + fr;
-            fb[j] = *reinterpret_cast<const bf16x8*>(sb + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
+            fb[j] = *reinterpret_cast<const Frag*>(sb + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
         }
     };
-    auto mma = [&](const bf16x8 (&fa)[TM], const bf16x8 (&fb)[TN]) {
+    auto mma = [&](const Frag (&fa)[TM], const Frag (&fb)[TN]) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; j++) {
+                if constexpr (std::is_same<ET, float>::value) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[i][j], 0, 0, 0);
+                } else {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+                }
+            }
     };
     auto wait_stage = [&](int kt) {
         const int younger = min(STAGES - 2, nk - 1 - kt);
@@ -194,7 +205,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
     };
     static_assert(STAGES <= 4 && 2 * PER < 64, "the wait distinguishes up to two younger stages");
 
-    bf16x8 fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+    Frag fa0[TM], fb0[TN], fa1[TM], fb1[TN];
     wait_stage(0);
     __syncthreads();
     read_frags(0, 0, fa0, fb0);
@@ -219,25 +230,25 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_bf16_dma_kernel(GemmArgs g,
         }
     }
     __syncthreads();
-    gemm_epilogue<bf16_t, TM, TN>(g, tl, col0, wm, wn, lane, reinterpret_cast<float*>(gemm_smem) + wave * (32 * 36), acc);
+    gemm_epilogue<ET, TM, TN>(g, tl, col0, wm, wn, lane, reinterpret_cast<float*>(gemm_smem) + wave * (32 * 36), acc);
 }
 
-constexpr int gemm_bf16_lds(int bm, int bn, int stages, int nw) {
+constexpr int gemm_float_lds(int bm, int bn, int stages, int nw) {
     const int ring = stages * (bm + bn) * 128, epi = nw * 32 * 36 * 4;
     return ring > epi ? ring : epi;
 }
 
-template <int BM, int BN, int STAGES, int WPE, int NW>
-static int launch_bf16(const GemmArgs& g, hipStream_t st) {
-    constexpr int lds = gemm_bf16_lds(BM, BN, STAGES, NW);
+template <typename ET, int BM, int BN, int STAGES, int WPE, int NW>
+static int launch_dma(const GemmArgs& g, hipStream_t st) {
+    constexpr int lds = gemm_float_lds(BM, BN, STAGES, NW);
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_dma_kernel<BM, BN, STAGES, WPE, NW>),
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         opted_in.store(true, std::memory_order_release);
     }
     const int tm = g.tiles ? g.max_tiles : (g.m + BM - 1) / BM, tn = (g.n + BN - 1) / BN;
-    gemm_bf16_dma_kernel<BM, BN, STAGES, WPE, NW><<<tm * tn, NW * 64, lds, st>>>(g, tm, tn);
+    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<tm * tn, NW * 64, lds, st>>>(g, tm, tn);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
@@ -285,6 +296,20 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
     return FLEXLLM_OK;
 }
 
+// The tile whose rounds over the chip (a workgroup per CU) take the least time; cost: of a round, as measured where all CUs are
+// busy, in any unit.
+struct GemmTileCost { int bm, bn, cost; };
+template <int N>
+static int gemm_cheapest_tile(const GemmArgs& g, const GemmTileCost (&tiles)[N]) {
+    long best = 0;
+    int pick = -1;
+    for (int i = 0; i < N; i++) {
+        const long n = (long)((g.m + tiles[i].bm - 1) / tiles[i].bm) * ((g.n + tiles[i].bn - 1) / tiles[i].bn), cost = (n + 255) / 256 * tiles[i].cost;
+        if (pick < 0 || cost < best) { best = cost; pick = i; }
+    }
+    return pick;
+}
+
 template <>
 int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
@@ -298,24 +323,17 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         FX_LAUNCH_CHECK();
         g.n = g.n_split;
     }
-    // The tile whose rounds over the chip (a workgroup per CU) take the least time.  Cost of a round per 64 k, in 0.01 us, as
-    // measured where all CUs are busy: 256 x 256 2.1 us, 128 x 256 1.1 us, 128 x 128 0.6 us, 64 x 128 0.4 us, 64 x 64 0.28 us.  So 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us;
-    // 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3 rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336
-    // 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048 64 x 128 (14.8 us; 128 x 128: 19.4 us).
-    struct Tile { int bm, bn, cost; };
-    constexpr Tile tiles[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}};
-    long best = 0;
-    int pick = -1;
-    for (int i = 0; i < 5; i++) {
-        const long n = (long)((g.m + tiles[i].bm - 1) / tiles[i].bm) * ((g.n + tiles[i].bn - 1) / tiles[i].bn), cost = (n + 255) / 256 * tiles[i].cost;
-        if (pick < 0 || cost < best) { best = cost; pick = i; }
-    }
+    // 256 x 256 2.1 us per 64 k, 128 x 256 1.1 us, 128 x 128 0.6 us, 64 x 128 0.4 us, 64 x 64 0.28 us.  So 777 x 28672 x 4096 takes 256 x 256
+    // (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3 rounds, 113 us; 256 x 256: 2 rounds, 141 us),
+    // 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048 64 x 128 (14.8 us; 128 x 128: 19.4 us).
+    constexpr GemmTileCost tiles[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}};
+    const int pick = gemm_cheapest_tile(g, tiles);
     switch (pick) {
-        case 0: return launch_bf16<256, 256, 2, 2, 8>(g, st);
-        case 1: return launch_bf16<128, 256, 3, 2, 8>(g, st);
-        case 2: return launch_bf16<128, 128, 4, 2, 8>(g, st);
-        case 3: return launch_bf16<64, 128, 4, 2, 8>(g, st);
-        default: return launch_bf16<64, 64, 4, 2, 4>(g, st);
+        case 0: return launch_dma<bf16_t, 256, 256, 2, 2, 8>(g, st);
+        case 1: return launch_dma<bf16_t, 128, 256, 3, 2, 8>(g, st);
+        case 2: return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
+        case 3: return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
+        default: return launch_dma<bf16_t, 64, 64, 4, 2, 4>(g, st);
     }
 }
 
@@ -327,74 +345,40 @@ static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
-    if constexpr (BM == 128) return launch_bf16<128, 128, 4, 2, 8>(g, st);
-    else return launch_bf16<64, 128, 4, 2, 8>(g, st);
+    if constexpr (BM == 128) return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
+    else return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
 }
 
 // ---- float32 -----------------------------------------------------------------------------------------------------
-// 64x64 tile, four waves 2x2, 16 k per step staged through registers.
-template <int BM>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs g, int tiles_m, int tiles_n) {
-    constexpr int BN = 64, BK = 16, P = 65, TM = BM / 64;
-    __shared__ float la[BK][BM + 1], lb[BK][P];
-    __shared__ float patch[4][32 * 36];
-    GemmTile tl;
-    int col0;
-    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, tl, col0)) return;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * 32;
-    const float* a = static_cast<const float*>(g.a);
-    const float* w = static_cast<const float*>(g.w) + (size_t)tl.group * g.w_stride;
-    f32x16 acc[TM][1];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][0][r] = 0.0f;
-    for (int k0 = 0; k0 < g.k; k0 += BK) {
-        __syncthreads();
-        for (int c = t; c < BM * 4; c += 256) {
-            int row = min(tl.row0 + (c >> 2), tl.row_end - 1);
-            if (g.row_src) row = g.row_src[row];
-            const float4 v = *reinterpret_cast<const float4*>(a + (size_t)row * g.lda + k0 + (c & 3) * 4);
-            la[(c & 3) * 4][c >> 2] = v.x; la[(c & 3) * 4 + 1][c >> 2] = v.y; la[(c & 3) * 4 + 2][c >> 2] = v.z; la[(c & 3) * 4 + 3][c >> 2] = v.w;
-        }
-        {
-            const int c = t;
-            const float4 v = *reinterpret_cast<const float4*>(w + (size_t)min(col0 + (c >> 2), g.n - 1) * g.ldw + k0 + (c & 3) * 4);
-            lb[(c & 3) * 4][c >> 2] = v.x; lb[(c & 3) * 4 + 1][c >> 2] = v.y; lb[(c & 3) * 4 + 2][c >> 2] = v.z; lb[(c & 3) * 4 + 3][c >> 2] = v.w;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < BK / 2; s++) {
-            const float fb = lb[2 * s + (lane >> 5)][wn + (lane & 31)];
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const float fa = la[2 * s + (lane >> 5)][wm + i * 32 + (lane & 31)];
-                acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa, fb, acc[i][0], 0, 0, 0);
-            }
-        }
-    }
-    gemm_epilogue<float, TM, 1>(g, tl, col0, wm, wn, lane, patch[wave], acc);
-}
-
-template <int BM>
-static int launch_f32(const GemmArgs& args, hipStream_t st) {
+template <>
+int gemm_float<float>(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 4);
     if (rc) return rc;
-    const int tm = g.tiles ? g.max_tiles : (g.m + BM - 1) / BM, tn = (g.n + 63) / 64;
-    gemm_f32_kernel<BM><<<tm * tn, 256, 0, st>>>(g, tm, tn);
-    FX_LAUNCH_CHECK();
-    return FLEXLLM_OK;
+    FX_REQUIRE(!g.tiles, "gemm_float: a tile table goes to gemm_grouped");
+    // 128 x 128 2.35 us per 32 k, 64 x 128 1.26 us, 64 x 64 0.66 us: 333 x 16384 x 2048 takes 64 x 128 (251 us; 64 x 64: 265, 128 x 128: 289 us),
+    // 333 x 2048 x 8192 64 x 64 (173 us; 64 x 128: 276 us), 2048 x 4096 x 4096 128 x 128 (602 us, 114 TFLOP/s; 64 x 64: 656 us).
+    constexpr GemmTileCost tiles[] = {{128, 128, 235}, {64, 128, 126}, {64, 64, 66}};
+    switch (gemm_cheapest_tile(g, tiles)) {
+        case 0: return launch_dma<float, 128, 128, 4, 2, 8>(g, st);
+        case 1: return launch_dma<float, 64, 128, 4, 2, 8>(g, st);
+        default: return launch_dma<float, 64, 64, 4, 2, 4>(g, st);
+    }
 }
 
-template <>
-int gemm_float<float>(const GemmArgs& g, hipStream_t st) { return launch_f32<64>(g, st); }
+template <int BM>
+static int gemm_grouped_f32(const GemmArgs& args, hipStream_t st) {
+    GemmArgs g = args;
+    int rc = gemm_check(g, g.m, 4);
+    if (rc) return rc;
+    if constexpr (BM == 128) return launch_dma<float, 128, 64, 4, 2, 4>(g, st);
+    else return launch_dma<float, 64, 64, 4, 2, 4>(g, st);
+}
 
 template <typename ET>
 int gemm_grouped(const GemmArgs& g, int tile_rows, hipStream_t st) {
     FX_REQUIRE(g.tiles && (tile_rows == 64 || tile_rows == 128), "gemm_grouped: tile table of %d rows", tile_rows);
-    if constexpr (std::is_same<ET, float>::value) return tile_rows == 128 ? launch_f32<128>(g, st) : launch_f32<64>(g, st);
+    if constexpr (std::is_same<ET, float>::value) return tile_rows == 128 ? gemm_grouped_f32<128>(g, st) : gemm_grouped_f32<64>(g, st);
     else return tile_rows == 128 ? gemm_grouped_bf16<128>(g, st) : gemm_grouped_bf16<64>(g, st);
 }
 template int gemm_grouped<bf16_t>(const GemmArgs&, int, hipStream_t);

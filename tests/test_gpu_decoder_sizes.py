@@ -66,23 +66,29 @@ def test_few_token_attention_splits(heads, kv_heads, dim, dtype):
 
 
 # every tile of the GEMM: one k-stage, fewer and more than the ring holds, rows and columns that do not fill the last tile
+@BOTH
 @pytest.mark.parametrize("k", [64, 128, 256, 448])
 @pytest.mark.parametrize("m,n,split,glu", [(1024, 16380, 16380, 0), (1021, 16384, 16384, 1), (1100, 16384, 16000, 0), (1000, 4000, 4000, 2), (897, 4096, 0, 0),
                                            (1000, 2040, 1024, 0), (961, 2048, 2048, 1), (65, 1028, 1028, 0), (1, 64, 0, 0)])
-def test_gemm_tiles(m, n, split, glu, k):
+def test_gemm_tiles(m, n, split, glu, k, dtype):
     from flexllm_amd import ops, to_device
     from flexllm_amd.loader import from_bf16, to_bf16
     r = np.random.default_rng(m + n + k)
     a, w = [lc.round_bf16(r.standard_normal(s)) for s in ((m, k), (n, k))]
-    y, y32 = ops.linear_float(to_device(to_bf16(a)), to_device(to_bf16(w)), split, glu, 3.0)
+    dev = to_device if dtype == "float32" else lambda x: to_device(to_bf16(x))
+    y, y32 = ops.linear_float(dev(a), dev(w), split, glu, 3.0)
     want = a.astype(np.float64) @ w.astype(np.float64).T
-    # float32 sums of k products of O(1): 1e-5 of sqrt(k); a bfloat16 result is within 2^-9 of the value, the unit's slope is at most 1.2
+    # A float32 sum of k products of O(1) is within d = 1e-5 sqrt(k).  A unit act(g) u has slopes of at most 1.2 |u| in g and |g| in u
+    # (the clamped one: u + 1 with |u| <= 3); a bfloat16 result is besides within 2^-9 of the value.
+    d = 1e-5 * np.sqrt(k)
     if split:
         g, u = want[:, 0:split:2], want[:, 1:split:2]
         first = want[:, :split] if not glu else nifunex_ref.clamped_glu(g, u, 3.0) if glu == 1 else lopazen_ref.gelu(g) * u
-        assert np.all(np.abs(from_bf16(y.numpy()) - first) <= 5e-3 * (np.abs(first) + np.sqrt(k)))
+        got, tol = (y.numpy(), 1e-5) if dtype == "float32" else (from_bf16(y.numpy()), 5e-3)
+        slope = 1.2 * (np.abs(u) + 1) + np.abs(g) if glu else 1.0
+        assert np.all(np.abs(got - first) <= tol * np.abs(first) + d * slope)
     if split < n:
-        assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * (np.abs(want[:, split:]) + np.sqrt(k)))
+        assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * np.abs(want[:, split:]) + d)
 
 
 # grouped products of the experts: tiles of 64 and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
