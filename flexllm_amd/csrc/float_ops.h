@@ -22,8 +22,11 @@ struct GemmArgs {
     const int* row_src = nullptr;
     const int4* tiles = nullptr; const int* n_tiles = nullptr; int max_tiles = 0;
     size_t w_stride = 0;
+    int parts = 1; size_t part_stride = 0;                // n_split 0 only: k in `parts` parts, whose sums leave part_stride apart in y32
 };
 template <typename ET> int gemm_float(const GemmArgs& g, hipStream_t st);
+// Parts (at most `most`) that suit a product with n_split 0 whose reader adds the parts' sums up.
+template <typename ET> int gemm_parts(const GemmArgs& g, int most);
 // The grouped form; the table is cut for tiles of tile_rows (64 or 128) rows, gemm_group_tile_rows says which suits.
 template <typename ET> int gemm_grouped(const GemmArgs& g, int tile_rows, hipStream_t st);
 int gemm_group_tile_rows(int rows_per_group);
@@ -77,7 +80,7 @@ int advance_launch(int* state, int n, hipStream_t st);
 struct RowArgs {
     float *x = nullptr, *x_new = nullptr;
     const float* x0 = nullptr;
-    const float* y = nullptr; int ldy = 0;
+    const float* y = nullptr; int ldy = 0, y_parts = 1; size_t y_stride = 0;      // y is the sum of y_parts parts, y_stride apart
     const float *gb = nullptr, *g = nullptr;
     float eps = 0.0f;
     int width = 0, rows = 0;

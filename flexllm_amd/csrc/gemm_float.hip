@@ -19,15 +19,15 @@ struct GemmTile { int row0, row_end, group; };
 
 // Which tile this workgroup works on: row tiles fastest inside a range of weight columns per XCD, as in gemm_i8_kernel.
 template <int BM, int BN>
-__device__ __forceinline__ bool gemm_pick_tile(const GemmArgs& g, int tiles_m, int tiles_n, GemmTile& t, int& col0) {
+__device__ __forceinline__ bool gemm_pick_tile(const GemmArgs& g, int tiles_m, int tiles_n, int tile, GemmTile& t, int& col0) {
     int tm, tn;
     if ((tiles_n & 7) == 0) {
-        const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+        const int xcd = tile & 7, idx = tile >> 3;
         tn = xcd * (tiles_n >> 3) + idx / tiles_m;
         tm = idx % tiles_m;
     } else {
-        tm = blockIdx.x % tiles_m;
-        tn = blockIdx.x / tiles_m;
+        tm = tile % tiles_m;
+        tn = tile / tiles_m;
     }
     col0 = tn * BN;
     if (g.tiles) {
@@ -123,12 +123,14 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
 
     GemmTile tl;
     int col0;
-    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, tl, col0)) return;
+    const int part = blockIdx.x / (tiles_m * tiles_n), stages = g.k * (int)sizeof(ET) / BKB, k0 = part * stages / g.parts;
+    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, blockIdx.x - part * (tiles_m * tiles_n), tl, col0)) return;
+    g.y32 += part * g.part_stride;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
-    const int8_t* const a = static_cast<const int8_t*>(g.a);
-    const int8_t* const w = static_cast<const int8_t*>(g.w) + (size_t)tl.group * g.w_stride * sizeof(ET);
+    const int8_t* const a = static_cast<const int8_t*>(g.a) + (size_t)k0 * BKB;
+    const int8_t* const w = static_cast<const int8_t*>(g.w) + (size_t)tl.group * g.w_stride * sizeof(ET) + (size_t)k0 * BKB;
 
     unsigned offa[A_INSTR], offb[B_INSTR];
 #pragma unroll
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-    const int nk = g.k * (int)sizeof(ET) / BKB;
+    const int nk = (part + 1) * stages / g.parts - k0;
     constexpr int PER = A_INSTR + B_INSTR;
     // everything the compiler loaded itself (tile table, gathered row numbers) has to be in before the counted loads start
     gemm_wait_vmcnt<0>();
@@ -248,7 +250,7 @@ static int launch_dma(const GemmArgs& g, hipStream_t st) {
         opted_in.store(true, std::memory_order_release);
     }
     const int tm = g.tiles ? g.max_tiles : (g.m + BM - 1) / BM, tn = (g.n + BN - 1) / BN;
-    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<tm * tn, NW * 64, lds, st>>>(g, tm, tn);
+    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<tm * tn * g.parts, NW * 64, lds, st>>>(g, tm, tn);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
@@ -293,22 +295,51 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
     FX_REQUIRE(g.n_split >= 0 && g.n_split <= g.n && (g.n_split == 0 || g.y) && (g.n_split == g.n || g.y32), "gemm_float: output pointers");
     FX_REQUIRE(!g.glu || g.n_split % 2 == 0, "gemm_float: odd number of gate/up rows");
     FX_REQUIRE(!g.tiles || (g.n_tiles && g.max_tiles > 0), "gemm_float: tile table");
+    FX_REQUIRE(g.parts >= 1 && (g.parts == 1 || (g.n_split == 0 && !g.bias && !g.tiles && g.parts <= g.k * es / 128)), "gemm_float: %d parts of k=%d", g.parts, g.k);
     return FLEXLLM_OK;
 }
 
-// The tile whose rounds over the chip (a workgroup per CU) take the least time; cost: of a round, as measured where all CUs are
-// busy, in any unit.
+// The tile whose rounds over the chip (a workgroup per CU) take the least time; cost: of a round of one stage, in 0.01 us, as
+// measured where all CUs are busy.
+//
+// bfloat16 (64 k): 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3
+// rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048
+// 64 x 128 (14.8 us; 128 x 128: 19.4 us).
+// float32 (32 k): 333 x 16384 x 2048 takes 64 x 128 (251 us; 64 x 64: 265, 128 x 128: 289 us), 333 x 2048 x 8192 64 x 64 (173 us; 64 x 128:
+// 276 us), 2048 x 4096 x 4096 128 x 128 (602 us, 114 TFLOP/s; 64 x 64: 656 us).
 struct GemmTileCost { int bm, bn, cost; };
-template <int N>
-static int gemm_cheapest_tile(const GemmArgs& g, const GemmTileCost (&tiles)[N]) {
-    long best = 0;
-    int pick = -1;
-    for (int i = 0; i < N; i++) {
-        const long n = (long)((g.m + tiles[i].bm - 1) / tiles[i].bm) * ((g.n + tiles[i].bn - 1) / tiles[i].bn), cost = (n + 255) / 256 * tiles[i].cost;
+template <typename ET> struct GemmTiles;
+template <> struct GemmTiles<bf16_t> { static constexpr GemmTileCost list[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}}; };
+template <> struct GemmTiles<float> { static constexpr GemmTileCost list[] = {{128, 128, 235}, {64, 128, 126}, {64, 64, 66}}; };
+
+template <typename ET>
+static int gemm_cheapest_tile(const GemmArgs& g, int parts, long& best) {
+    const long stages = (long)g.k * sizeof(ET) / 128;
+    int pick = -1, i = 0;
+    for (const GemmTileCost& t : GemmTiles<ET>::list) {
+        const long n = (long)((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn) * parts, cost = (n + 255) / 256 * t.cost * ((stages + parts - 1) / parts);
         if (pick < 0 || cost < best) { best = cost; pick = i; }
+        i++;
     }
     return pick;
 }
+
+// Few rows of a long k leave most CUs without a tile, so k is shared out.  A part costs its sums' way to memory and back (8 bytes
+// each at 5 TB/s, besides the launch that it does not add) and has at least a ring of stages to walk.
+template <typename ET>
+int gemm_parts(const GemmArgs& g, int most) {
+    long best = 0;
+    int parts = 1;
+    for (int p = 1; p <= most && p * 4 <= (int)(g.k * sizeof(ET) / 128); p *= 2) {
+        long cost;
+        gemm_cheapest_tile<ET>(g, p, cost);
+        cost += (long)p * g.m * g.n * 8 / 50000;
+        if (p == 1 || cost < best) { best = cost; parts = p; }
+    }
+    return parts;
+}
+template int gemm_parts<bf16_t>(const GemmArgs&, int);
+template int gemm_parts<float>(const GemmArgs&, int);
 
 template <>
 int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
@@ -323,12 +354,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         FX_LAUNCH_CHECK();
         g.n = g.n_split;
     }
-    // 256 x 256 2.1 us per 64 k, 128 x 256 1.1 us, 128 x 128 0.6 us, 64 x 128 0.4 us, 64 x 64 0.28 us.  So 777 x 28672 x 4096 takes 256 x 256
-    // (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3 rounds, 113 us; 256 x 256: 2 rounds, 141 us),
-    // 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048 64 x 128 (14.8 us; 128 x 128: 19.4 us).
-    constexpr GemmTileCost tiles[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}};
-    const int pick = gemm_cheapest_tile(g, tiles);
-    switch (pick) {
+    long cost;
+    switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
         case 0: return launch_dma<bf16_t, 256, 256, 2, 2, 8>(g, st);
         case 1: return launch_dma<bf16_t, 128, 256, 3, 2, 8>(g, st);
         case 2: return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
@@ -356,10 +383,8 @@ int gemm_float<float>(const GemmArgs& args, hipStream_t st) {
     int rc = gemm_check(g, g.m, 4);
     if (rc) return rc;
     FX_REQUIRE(!g.tiles, "gemm_float: a tile table goes to gemm_grouped");
-    // 128 x 128 2.35 us per 32 k, 64 x 128 1.26 us, 64 x 64 0.66 us: 333 x 16384 x 2048 takes 64 x 128 (251 us; 64 x 64: 265, 128 x 128: 289 us),
-    // 333 x 2048 x 8192 64 x 64 (173 us; 64 x 128: 276 us), 2048 x 4096 x 4096 128 x 128 (602 us, 114 TFLOP/s; 64 x 64: 656 us).
-    constexpr GemmTileCost tiles[] = {{128, 128, 235}, {64, 128, 126}, {64, 64, 66}};
-    switch (gemm_cheapest_tile(g, tiles)) {
+    long cost;
+    switch (gemm_cheapest_tile<float>(g, g.parts, cost)) {
         case 0: return launch_dma<float, 128, 128, 4, 2, 8>(g, st);
         case 1: return launch_dma<float, 64, 128, 4, 2, 8>(g, st);
         default: return launch_dma<float, 64, 64, 4, 2, 4>(g, st);

@@ -21,6 +21,8 @@ namespace fx {
 constexpr int kSmallTokens = 8;
 constexpr int kPieceTokens = 4096;
 constexpr int kHeadRows = 256;          // rows of logits formed at a time
+constexpr int kMaxParts = 8;            // parts that the k of a product with few rows is shared out in,
+constexpr int kPartRows = 4096;         // and rows of all parts together
 // Prompts without a matrix-core attention (float32, long heads) take the attention kernels for few tokens in slices of this many
 // (333 tokens of ten layers in float32: 16 at a time 17.2 ms, 64 at a time 14.7 ms: more workgroups per launch, fewer splits to join).
 constexpr int kAbsorbTokens = 64;
@@ -82,7 +84,7 @@ struct flexllm_hybrid {
     int* topk_idx = nullptr;
     int* gen_token = nullptr;
     // many-token workspace
-    int rows = 0;
+    int rows = 0, ly_rows = 0;
     float *lx0 = nullptr, *lx = nullptr, *lf32 = nullptr, *ly = nullptr, *lys = nullptr, *lroute = nullptr, *lgla = nullptr, *lpick_w = nullptr;
     void *lh = nullptr, *lproj = nullptr, *latt = nullptr, *lhid = nullptr, *lhs = nullptr, *lk = nullptr, *lvt = nullptr, *lhead = nullptr;
     int *lpick = nullptr, *lpos_of = nullptr, *lrow_src = nullptr, *lcounts = nullptr, *lntiles = nullptr;
@@ -472,7 +474,8 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
     FX_TRY(pool(m->lx, R * W));
     if (c.loop_times > 1) FX_TRY(pool(m->lx0, R * W));
     FX_TRY(pool(m->lf32, R * (m->max_f32 + 4)));
-    FX_TRY(pool(m->ly, R * W));
+    m->ly_rows = (int)(R > kPartRows ? R : R * kMaxParts < kPartRows ? R * kMaxParts : kPartRows);
+    FX_TRY(pool(m->ly, (size_t)m->ly_rows * W));
     FX_TRY(pool_et(m->lh, R * pad_k((int)W)));
     FX_TRY(pool_et(m->lproj, R * ((size_t)(m->max_et + 7) / 8 * 8)));
     FX_TRY(pool_et(m->latt, R * pad_k(m->max_att)));
@@ -633,9 +636,13 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         g.a = a; g.lda = lda; g.w = w; g.m = rows; g.n = n; g.k = pad_k(k);
         return g;
     };
+    // a product that the next row kernel takes in, which adds the parts that k is shared out in
     auto to_y = [&](const void* a, int lda, const void* w, int k) {
         GemmArgs g = gemm(a, lda, w, T, W, k);
         g.n_split = 0; g.y32 = m->ly; g.ldy32 = W;
+        g.parts = gemm_parts<ET>(g, kMaxParts < m->ly_rows / T ? kMaxParts : m->ly_rows / T);
+        g.part_stride = (size_t)T * W;
+        pend.y = m->ly; pend.ldy = W; pend.y_parts = g.parts; pend.y_stride = g.part_stride;
         return gemm_float<ET>(g, st);
     };
     const int runs = (int)m->runs.size();
@@ -696,7 +703,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
             FX_TRY(gla_steps<ET>(L.gd, proj, ldp, 0, m->lf32, nf, static_cast<ET*>(L.a2), L.a2_bias, L.head_norm, s.state[r], s.pos, 0, T, att, lda, 0, st));
         }
         FX_TRY(to_y(att, lda, L.w_o, L.k_o));
-        pend.y = m->ly; pend.ldy = W; pend.gb = L.g1b;
+        pend.gb = L.g1b;
         if (L.d.ff_kind == FLEXLLM_FF_NONE) continue;
         const int kf = pad_k(L.d.ff);
         FX_TRY(rows_h(L.g2));
@@ -705,7 +712,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
             g.n_split = 2 * L.d.ff; g.glu = 1 + L.d.glu; g.limit = L.d.limit; g.y = m->lhid; g.ldy = kf;
             FX_TRY(gemm_float<ET>(g, st));
             FX_TRY(to_y(m->lhid, kf, L.w_d, L.d.ff));
-            pend.y = m->ly; pend.ldy = W; pend.gb = L.g2b;
+            pend.gb = L.g2b;
             continue;
         }
         const int sf = L.d.shared_ff, ldr = L.n_side - 2 * sf, top = L.d.top, ks = pad_k(sf > 0 ? sf : 1);
@@ -729,7 +736,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         FX_TRY(gemm_grouped<ET>(g, tile, st));
         if (sf) {
             FX_TRY(to_y(m->lhs, ks, L.w_sd, sf));
-            pend.y = m->ly; pend.route = m->lroute; pend.ld_route = ldr; pend.experts = L.d.experts;
+            pend.route = m->lroute; pend.ld_route = ldr; pend.experts = L.d.experts;
         }
         pend.ldy = W; pend.gb = L.g2b; pend.ys = m->lys; pend.pos_of = m->lpos_of; pend.pick_w = m->lpick_w; pend.top = top;
     }

@@ -61,6 +61,15 @@ int advance_launch(int* state, int n, hipStream_t st) {
     return FLEXLLM_OK;
 }
 
+// y at `at`, its parts in order.
+template <typename V>
+__device__ __forceinline__ V sum_parts(const RowArgs& a, size_t at) {
+    V v = *reinterpret_cast<const V*>(a.y + at);
+#pragma unroll 4
+    for (int p = 1; p < a.y_parts; p++) v += *reinterpret_cast<const V*>(a.y + p * a.y_stride + at);
+    return v;
+}
+
 // One workgroup per row; the row stays in LDS between the two norms.
 template <typename ET>
 __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
@@ -78,9 +87,9 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
             float v = 0.0f;
             if (mix) {
                 for (int k = 0; k < a.top; k++) v = fma_f(a.pick_w[r * a.top + k], a.ys[(size_t)a.pos_of[r * a.top + k] * a.ldy + i], v);
-                if (a.y) v = fma_f(sg, a.y[(size_t)r * a.ldy + i], v);
+                if (a.y) v = fma_f(sg, sum_parts<float>(a, (size_t)r * a.ldy + i), v);
             } else if (a.y) {
-                v = a.y[(size_t)r * a.ldy + i];
+                v = sum_parts<float>(a, (size_t)r * a.ldy + i);
             }
             row[i] = v;
             ss = fma_f(v, v, ss);
@@ -140,12 +149,12 @@ __global__ __launch_bounds__(256) void norm_rows_vec_kernel(RowArgs a) {
                         for (int e = 0; e < 4; e++) y[i][e] = fma_f(w, u[e], y[i][e]);
                     }
                     if (a.y) {
-                        const f32x4 u = *reinterpret_cast<const f32x4*>(a.y + (size_t)r * a.ldy + c * 4);
+                        const f32x4 u = sum_parts<f32x4>(a, (size_t)r * a.ldy + c * 4);
 #pragma unroll
                         for (int e = 0; e < 4; e++) y[i][e] = fma_f(sg, u[e], y[i][e]);
                     }
                 } else if (a.y) {
-                    y[i] = *reinterpret_cast<const f32x4*>(a.y + (size_t)r * a.ldy + c * 4);
+                    y[i] = sum_parts<f32x4>(a, (size_t)r * a.ldy + c * 4);
                 }
             }
 #pragma unroll

@@ -97,3 +97,20 @@ def test_gemm_tiles(m, n, split, glu, k, dtype):
 def test_grouped_tiles(experts, top, ff, tokens, dtype):
     cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=192)
     check_nifunex(cfg, dtype, tokens, [tokens], skip=0.05)
+
+
+# prompts of few rows, whose down and output projections share k out: no row tile filled, one and two of them, parts of uneven lengths,
+# with and without a norm behind the sublayer, a mixture's shared expert
+@BOTH
+@pytest.mark.parametrize("tokens,ff", [(9, 2048), (65, 1100), (130, 4200)])
+def test_shared_out_k(tokens, ff, dtype):
+    check_lopazen(lc.config([lc.layer(heads=12, kv_heads=3, dim=64, mlp=lc.dense(ff)), lc.layer()], width=192), dtype, tokens, [tokens])
+    check_nifunex(nc.config([nc.gla(heads=9, dim=32, vdim=64, mlp=nc.dense(ff)), nc.gla(heads=1, mlp=nc.moe(4, 2, 72, 1.5, ff))], width=192), dtype, tokens, [tokens], skip=0.05)
+
+
+@BOTH
+def test_slices_of_a_prompt(dtype):
+    """Prompts that go through the step's attention in slices of 64 tokens: whole slices, one token more, one less."""
+    for n in (63, 64, 65, 129):
+        check_lopazen(lc.config([lc.layer(heads=4, kv_heads=2, dim=264, scale=0.06)]), dtype, n, [n], [9, n])
+        check_nifunex(nc.config([nc.latent(heads=2, dim=264, rot_dim=8, vdim=16, kv_rank=48, window=50, scale=0.06)]), dtype, n, [n], [9, n])
