@@ -11,7 +11,6 @@
 #include "attn_decode_kernels.h"
 #include "common.h"
 #include <atomic>
-#include <stdlib.h>
 
 namespace fx {
 
@@ -202,15 +201,13 @@ __global__ __launch_bounds__(256) void gemm_i8_kernel(const int8_t* __restrict__
 //
 // The loads are issued from inline assembly: the compiler does not track them, so the k-loop waits for them
 // with explicit counters (results return in issue order).
-__host__ __device__ constexpr int gemm_dma_lds_bytes(int bm, int bn, int stages, int bkb = 64, int nw = 4, int ksplit = 1) {
-    // the stage rings (one per k-group), or the epilogue: one patch per wave plus, with two k-groups, the second
-    // group's accumulators
-    const int rings = ksplit * stages * (bm + bn) * bkb;
-    const int epi = nw * 32 * 36 * 4 + (ksplit > 1 ? bm * bn * 4 : 0);
-    return rings > epi ? rings : epi;
-}
-
 enum GemmDmaEpi { kDmaRaw = 0, kDmaDequant = 1, kDmaSwiglu = 2, kDmaQkv = 3, kDmaDequantAsym = 4, kDmaSwigluAsym = 5 };
+
+// The stage ring, or the epilogue: a patch per wave, for q/k/v the dequantised tile.
+__host__ __device__ constexpr int gemm_dma_lds_bytes(int bm, int bn, int stages, int bkb, int nw, int epilogue) {
+    const int ring = stages * (bm + bn) * bkb, epi = epilogue == kDmaQkv ? bm * (bn + 1) * 4 : nw * 32 * 36 * 4;
+    return ring > epi ? ring : epi;
+}
 
 // Arguments of the q/k/v epilogue: the 64-column tile of the fused [q | k | v] projection is one attention head,
 // so RoPE (pairs k, k+32), the static int8 quantisation and the store into q8 / the K cache / the transposed V
@@ -246,24 +243,18 @@ __device__ __forceinline__ void gemm_wait_vmcnt() {            // s_waitcnt vmcn
 // 23 TB/s into LDS in whole 128-byte lines and 14.5 TB/s in halves.  With 128-byte rows the slot rotation is
 // s ^ ((r >> 1) & 7): two rows span the 64 banks, so 16 consecutive rows of one chunk fall on 16 different bank groups.
 // NW = waves per workgroup, 4 (2x2 wave grid) or 8 (2x4): eight waves let a 256x256 tile keep two waves per SIMD.
-// KSPLIT = 2 (with NW = 8): two groups of four waves work on the same output tile, group g on the stages
-// kt with kt % 2 == g, each with its own ring of LDS stages; the second group's accumulators are added to the first's
-// through LDS before the epilogue (integer sums: exact in any order).  For outputs too narrow to give every CU two
-// workgroups (down projection: 256 tiles of 64x128) this puts two independent load pipelines on a CU all the same.
-template <int BM, int BN, int EPI, int kDmaStages, int WPE, int BKB, int NW, int KSPLIT>   // at most 7 stages (the wait below distinguishes up to 5 younger ones)
+template <int BM, int BN, int EPI, int kDmaStages, int WPE, int BKB, int NW>   // at most 4 stages (the wait below distinguishes up to 2 younger ones)
 __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ w,
                                                           int32_t* __restrict__ c_out, const float* __restrict__ s_x,
                                                           const float* __restrict__ w_s, const float* __restrict__ residual,
                                                           float* __restrict__ y, int m, int k, int n, int tiles_m, int tiles_n,
                                                           QkvEpiArgs qa) {
     static_assert(NW == 4 || NW == 8, "four or eight waves");
-    static_assert(KSPLIT == 1 || (KSPLIT == 2 && NW == 8 && EPI != kDmaQkv), "two k-groups need eight waves");
-    constexpr int GW = NW / KSPLIT;                           // waves per k-group
-    constexpr int WGN = GW / 2;                               // waves along N
+    constexpr int WGN = NW / 2;                               // waves along N
     constexpr int WM = BM / 2, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     static_assert(BKB == 64 || BKB == 128, "64 or 128 k-bytes per row and stage");
     constexpr int CPR = BKB / 16, RPI = 64 / CPR;             // 16-byte chunks per row; rows per direct load (1 KiB)
-    constexpr int A_INSTR = BM / (GW * RPI), B_INSTR = BN / (GW * RPI);   // direct loads per wave per stage
+    constexpr int A_INSTR = BM / (NW * RPI), B_INSTR = BN / (NW * RPI);   // direct loads per wave per stage
     static_assert(A_INSTR >= 1 && B_INSTR >= 1 && TM >= 1 && TN >= 1, "tile too small for this wave count");
     constexpr int STAGE = (BM + BN) * BKB, KS = BKB / 32;     // KS MFMA k-steps per stage
     auto rot = [](int r) { return BKB == 64 ? (r >> 2) & 3 : (r >> 1) & 7; };
@@ -280,10 +271,9 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
     }
     int row0 = tm * BM, col0 = tn * BN;
     const int t = threadIdx.x, lane = t & 63;
-    const int wave_wg = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int grp = wave_wg / GW, wave = wave_wg % GW;         // k-group, wave within the group
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
-    int8_t* const ring = gemm_smem + grp * (kDmaStages * STAGE);
+    int8_t* const ring = gemm_smem;
 
     // per-lane global offsets of this wave's direct loads (without the k offset, which is uniform)
     unsigned offa[A_INSTR], offb[B_INSTR];
@@ -298,10 +288,9 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
         offb[j] = (unsigned)min(col0 + r, n - 1) * (unsigned)k + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
     }
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)ring;
-    // kt counts the stages of this k-group; the group's stage kt is stage kt * KSPLIT + grp of the whole K range
     auto issue_stage = [&](int kt) {
         const unsigned sb = lds0 + (unsigned)(kt % kDmaStages) * STAGE;
-        const size_t koff = (size_t)(kt * KSPLIT + grp) * BKB;
+        const size_t koff = (size_t)kt * BKB;
 #pragma unroll
         for (int j = 0; j < A_INSTR; j++) gemm_dma_issue(a + koff, offa[j], sb + (wave * A_INSTR + j) * 1024);
 #pragma unroll
@@ -316,7 +305,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
 
-    const int nk = k / (BKB * KSPLIT);                         // stages per k-group (the launcher checks divisibility)
+    const int nk = k / BKB;                                    // the launcher checks divisibility
     constexpr int PER = A_INSTR + B_INSTR;                     // direct loads per wave per stage
 #pragma unroll
     for (int s0 = 0; s0 < kDmaStages - 1; s0++)
@@ -344,13 +333,11 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
             for (int j = 0; j < TN; j++)
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
     };
+    static_assert(kDmaStages <= 4 && 2 * PER < 64, "the wait distinguishes up to two younger stages");
     // stage kt has landed once only the younger stages in flight remain outstanding
     auto wait_stage = [&](int kt) {
         const int younger = min(kDmaStages - 2, nk - 1 - kt);
-        if (younger >= 5) gemm_wait_vmcnt<(5 * PER < 64 ? 5 * PER : 63)>();
-        else if (younger == 4) gemm_wait_vmcnt<(4 * PER < 64 ? 4 * PER : 63)>();
-        else if (younger == 3) gemm_wait_vmcnt<3 * PER>();
-        else if (younger == 2) gemm_wait_vmcnt<2 * PER>();
+        if (younger >= 2) gemm_wait_vmcnt<2 * PER>();
         else if (younger == 1) gemm_wait_vmcnt<PER>();
         else gemm_wait_vmcnt<0>();
     };
@@ -389,80 +376,69 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
     // (32 x 36 words) and then owns 4 consecutive columns of a row: 16-byte loads of the residual, 16-byte stores
     // (8 bytes for the SiLU*up pairs), 128 contiguous bytes per row.
     __syncthreads();                                           // all waves are done with the stage buffers
-    if constexpr (KSPLIT == 2) {
-        // the second k-group hands its accumulators over, lane-contiguous (conflict-free), behind the patch area
-        int* xch = reinterpret_cast<int*>(gemm_smem) + NW * 32 * 36 + wave * (TM * TN * 16 * 64) + lane;
-        if (grp == 1) {
+    if constexpr (EPI == kDmaQkv) {
+        static_assert(BM % 64 == 0 && BN % 64 == 0 && NW % 4 == 0, "blocks of 64 tokens x one head");
+        constexpr int TP = BN + 1;                             // odd pitch: a column walk hits every bank once
+        float* tile = reinterpret_cast<float*>(gemm_smem);     // dequantised tile [BM tokens][BN channels]
+        const bool asym = qa.b_x != nullptr;                  // asymmetric activations: + zero point x row sum of the dequantised weights
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int cl = wn + j * 32 + (lane & 31), col = min(col0 + cl, n - 1);
+            const float ws = w_s[col];
+            const float wq = asym ? qa.w_sum[col] : 0.0f;
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) xch[((i * TN + j) * 16 + r) * 64] = acc[i][j][r];
-        }
-        __syncthreads();
-        if (grp == 1) return;
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][j][r] += xch[((i * TN + j) * 16 + r) * 64];
-    }
-    if constexpr (EPI == kDmaQkv) {
-        static_assert(EPI != kDmaQkv || (BM == 64 && BN == 64 && NW == 4), "the q/k/v epilogue works on 64x64 tiles with four waves");
-        constexpr int TP = 65;                                 // odd pitch: a column walk hits every bank once
-        float* tile = reinterpret_cast<float*>(gemm_smem);     // dequantised tile [64 tokens][64 channels]
-        {
-            const int col = col0 + wn + (lane & 31);
-            const float ws = w_s[col];
-            const bool asym = qa.b_x != nullptr;              // asymmetric activations: + zero point x row sum of the dequantised weights
-            const float wq = asym ? qa.w_sum[col] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int lr = wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                const int row = min(row0 + lr, m - 1);
-                float v = (float)acc[0][0][r] * s_x[row] * ws;
-                if (asym) v = v + qa.b_x[row] * wq;
-                tile[lr * TP + wn + (lane & 31)] = v;
-            }
-        }
-        __syncthreads();
-        const int head = col0 / kHd;                           // uniform: 0..q_heads-1 q, then k heads, then v heads
-        const int sel = t & 63, part = t >> 6;
-        if (head < qa.q_heads + qa.kv_heads) {
-            // RoPE + static quantisation: thread = (token sel, pairs 8*part .. 8*part+7)
-            const int row = row0 + sel, pos = qa.pos0 + row;
-            if (row < m) {
-                const bool is_q = head < qa.q_heads;
-                const int hk = is_q ? head : head - qa.q_heads;
-                const float div = is_q ? 8.0f * qa.q_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
-                const float* sn = qa.sin_t + (size_t)pos * 32 + part * 8;
-                const float* cs = qa.cos_t + (size_t)pos * 32 + part * 8;
-                uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float t0 = tile[sel * TP + part * 8 + j], t1 = tile[sel * TP + part * 8 + j + 32];
-                    const float o0 = t0 * cs[j] - t1 * sn[j];
-                    const float o1 = t0 * sn[j] + t1 * cs[j];
-                    lo[j >> 2] |= (uint32_t)(static_q8(o0, div) & 0xff) << (8 * (j & 3));
-                    hi[j >> 2] |= (uint32_t)(static_q8(o1, div) & 0xff) << (8 * (j & 3));
+                for (int r = 0; r < 16; r++) {
+                    const int lr = wm + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                    const int row = min(row0 + lr, m - 1);
+                    float v = (float)acc[i][j][r] * s_x[row] * ws;
+                    if (asym) v = v + qa.b_x[row] * wq;
+                    tile[lr * TP + cl] = v;
                 }
-                int8_t* dst = is_q ? qa.q8 + ((size_t)row * qa.q_heads + hk) * kHd : qa.kc + k_index(hk, pos, qa.max_pos);
-                *reinterpret_cast<uint2*>(dst + part * 8) = make_uint2(lo[0], lo[1]);
-                *reinterpret_cast<uint2*>(dst + part * 8 + 32) = make_uint2(hi[0], hi[1]);
-            }
-        } else {
-            // V: thread = (channel sel, 16 consecutive positions 16*part ..): one 16-byte run of the transposed cache block
-            const int hv = head - qa.q_heads - qa.kv_heads;
-            const int rbase = row0 + part * 16;
-            if (rbase < m) {                                   // m is a multiple of 32 (checked by the launcher)
-                const float div = 1.0f * qa.v_s[hv];
-                uint32_t wv4[4] = {0, 0, 0, 0};
+        }
+        __syncthreads();
+        // four waves at a time take a block of 64 tokens x one head
+        constexpr int HM = BM / 64, HN = BN / 64, TEAMS = NW / 4;
+        const int sel = t & 63, part = (t >> 6) & 3;
+        for (int blk = t >> 8; blk < HM * HN; blk += TEAMS) {
+            const int tr = (blk % HM) * 64, tc = (blk / HM) * 64, head = (col0 + tc) / kHd;      // 0..q_heads-1 q, then k heads, then v heads
+            if (col0 + tc >= n) break;
+            const float* sub = tile + tr * TP + tc;
+            if (head < qa.q_heads + qa.kv_heads) {
+                // RoPE + static quantisation: thread = (token sel, pairs 8*part .. 8*part+7)
+                const int row = row0 + tr + sel, pos = qa.pos0 + row;
+                if (row < m) {
+                    const bool is_q = head < qa.q_heads;
+                    const int hk = is_q ? head : head - qa.q_heads;
+                    const float div = is_q ? 8.0f * qa.q_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
+                    const float* sn = qa.sin_t + (size_t)pos * 32 + part * 8;
+                    const float* cs = qa.cos_t + (size_t)pos * 32 + part * 8;
+                    uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};
 #pragma unroll
-                for (int i = 0; i < 16; i++)
-                    wv4[i >> 2] |= (uint32_t)(static_q8(tile[(part * 16 + i) * TP + sel], div) & 0xff) << (8 * (i & 3));
-                *reinterpret_cast<uint4*>(qa.vc + v_index(hv, qa.pos0 + rbase, sel, qa.max_pos)) = make_uint4(wv4[0], wv4[1], wv4[2], wv4[3]);
+                    for (int j = 0; j < 8; j++) {
+                        const float t0 = sub[sel * TP + part * 8 + j], t1 = sub[sel * TP + part * 8 + j + 32];
+                        const float o0 = t0 * cs[j] - t1 * sn[j];
+                        const float o1 = t0 * sn[j] + t1 * cs[j];
+                        lo[j >> 2] |= (uint32_t)(static_q8(o0, div) & 0xff) << (8 * (j & 3));
+                        hi[j >> 2] |= (uint32_t)(static_q8(o1, div) & 0xff) << (8 * (j & 3));
+                    }
+                    int8_t* dst = is_q ? qa.q8 + ((size_t)row * qa.q_heads + hk) * kHd : qa.kc + k_index(hk, pos, qa.max_pos);
+                    *reinterpret_cast<uint2*>(dst + part * 8) = make_uint2(lo[0], lo[1]);
+                    *reinterpret_cast<uint2*>(dst + part * 8 + 32) = make_uint2(hi[0], hi[1]);
+                }
+            } else {
+                // V: thread = (channel sel, 16 consecutive positions 16*part ..): one 16-byte run of the transposed cache block
+                const int hv = head - qa.q_heads - qa.kv_heads;
+                const int rbase = row0 + tr + part * 16;
+                if (rbase < m) {                               // m is a multiple of 32 (checked by the launcher)
+                    const float div = 1.0f * qa.v_s[hv];
+                    uint32_t wv4[4] = {0, 0, 0, 0};
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        wv4[i >> 2] |= (uint32_t)(static_q8(sub[(part * 16 + i) * TP + sel], div) & 0xff) << (8 * (i & 3));
+                    *reinterpret_cast<uint4*>(qa.vc + v_index(hv, qa.pos0 + rbase, sel, qa.max_pos)) = make_uint4(wv4[0], wv4[1], wv4[2], wv4[3]);
+                }
             }
         }
         return;
@@ -571,62 +547,56 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
     }
 }
 
-template <int BM, int BN, int EPI, int STAGES = 3, int WPE = 1, int BKB = 64, int NW = 4, int KSPLIT = 1>
+template <int BM, int BN, int EPI, int STAGES = 3, int WPE = 1, int BKB = 64, int NW = 4>
 inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s,
                            const float* residual, float* y, int m, int k, int n, hipStream_t st, QkvEpiArgs qa = QkvEpiArgs()) {
     static std::atomic<bool> opted_in{false};             // more than the default 64 KiB of LDS per workgroup
     if (!opted_in.load(std::memory_order_acquire)) {   // idempotent: two threads racing here both set the same attribute
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_i8_dma_kernel<BM, BN, EPI, STAGES, WPE, BKB, NW, KSPLIT>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dma_lds_bytes(BM, BN, STAGES, BKB, NW, KSPLIT)));
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_i8_dma_kernel<BM, BN, EPI, STAGES, WPE, BKB, NW>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dma_lds_bytes(BM, BN, STAGES, BKB, NW, EPI)));
         opted_in.store(true, std::memory_order_release);
     }
     const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;
-    gemm_i8_dma_kernel<BM, BN, EPI, STAGES, WPE, BKB, NW, KSPLIT><<<tm * tn, NW * 64, gemm_dma_lds_bytes(BM, BN, STAGES, BKB, NW, KSPLIT), st>>>(a, w, c, s_x, w_s, residual, y, m, k, n, tm, tn, qa);
+    gemm_i8_dma_kernel<BM, BN, EPI, STAGES, WPE, BKB, NW><<<tm * tn, NW * 64, gemm_dma_lds_bytes(BM, BN, STAGES, BKB, NW, EPI), st>>>(a, w, c, s_x, w_s, residual, y, m, k, n, tm, tn, qa);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
+}
+
+// The direct-load kernel on the tile whose rounds over the 256 CUs (a workgroup per CU) cost least, in 0.01 us: per stage of 128 k,
+// and once per round for what lies around them (first loads, epilogue).  From products of 2048 and 8192 k where all CUs are
+// busy.  Measured against the fixed choices before (us): 512 x 16384 x 2048 43.8 -> 24.8 (128 x 256), 2048 x 2048 x 8192 62.7 -> 45.8
+// (128 x 128), 2528 x 2048 x 8192 85.1 -> 65.1 (128 x 256), 1536 x 2048 x 8192 53.4 -> 41.3 (128 x 128), 4096 x 2048 x 8192 91.0 -> 80.4
+// (128 x 256), 1024 x 2048 x 2048 12.1 -> 11.3 (64 x 128); 1024 x 16384 x 2048 stays on 256 x 256, 41.5.
+template <int EPI>
+inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s, const float* residual, float* y,
+                             int m, int k, int n, hipStream_t st, QkvEpiArgs qa = QkvEpiArgs()) {
+    // whole 128-byte lines per row and stage where k allows
+    if (k % 128 != 0) return launch_gemm_dma<64, 64, EPI>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    struct Tile { int bm, bn, stage, round; };
+    constexpr Tile tiles[] = {{256, 256, 180, 1200}, {128, 256, 95, 950}, {128, 128, 65, 520}, {64, 128, 41, 220}, {64, 64, 35, 300}};
+    long best = 0;
+    int pick = -1;
+    for (int i = EPI == kDmaQkv ? 1 : 0; i < 5; i++) {         // the q/k/v epilogue's tile has to fit in LDS
+        const Tile& t = tiles[i];
+        const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), cost = (wgs + 255) / 256 * (t.stage * (k / 128) + t.round);
+        if (pick < 0 || cost < best) { best = cost; pick = i; }
+    }
+    if constexpr (EPI != kDmaQkv)
+        if (pick == 0) return launch_gemm_dma<256, 256, EPI, 2, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    if (pick == 1) return launch_gemm_dma<128, 256, EPI, 3, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    if (pick == 2) return launch_gemm_dma<128, 128, EPI, 4, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    if (pick == 3) return launch_gemm_dma<64, 128, EPI, 4, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    return launch_gemm_dma<64, 64, EPI, 4, 2, 128>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
 }
 
 template <int EPI>
 inline int launch_gemm(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s,
                        const float* residual, float* y, int m, int k, int n, hipStream_t st) {
-    // Measured on MI355X at M=1024: the direct-load kernel wins wherever it applies; 128x128 tiles once they fill
-    // the chip about three times over, 64x64 tiles for the narrow projections.  FLEXLLM_GEMM_TILE forces a variant
-    // (0..2: register-staged 128x128 / 64x128 / 64x64; direct-load: 11 = 128x128, 12 = 128x128 with two stages of
-    // 128-byte rows, 13 = 64x64, 19 = 64x128 four
-    // stages, all with 64-byte rows; 36 = 64x64 four stages and 38 = 64x64 three stages with 128-byte rows; 60 = 64x128
-    // three stages with 128-byte rows and two k-groups).
-    auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
-    static const char* force = getenv("FLEXLLM_GEMM_TILE");
     // the direct-load kernel needs 32-bit element offsets into both operands and 16-byte aligned output rows
-    const bool dma_ok = (size_t)m * k < (1ull << 31) && (size_t)n * k < (1ull << 31) && n % 4 == 0;
-    int mode = dma_ok ? (tiles(128, 128) >= 768 ? 11 : (k >= 4096 && tiles(64, 128) >= 256) ? 19 : 13) : (tiles(128, 128) >= 1024 ? 0 : 2);
-    // whole 128-byte lines per row and stage where K allows: three workgroups of 48 KiB per CU when the grid has
-    // that many, else two of 64 KiB with a fourth stage (the narrow projections stream their weights cold)
-    // Long K and an output too narrow for two workgroups per CU (down projection): 64x128 tiles, two k-groups of
-    // four waves per workgroup (32 us against 36 us for 64x64 tiles, two workgroups per CU).
-    // 384..767 tiles of 128x128 (o and down projections from M = 3072): two stages of 128-byte rows, two workgroups
-    // per CU.  At M = 4096: 36 us against 47 us (o) and 102 us against 133 us (down) for the narrow-tile choices below;
-    // at M = 3072: 30 / 87 us against 35 / 109 us; at M = 2048 (256 tiles) the narrow tiles are level or ahead.
-    if (dma_ok && mode != 11 && k % 128 == 0 && tiles(128, 128) >= 384) mode = 12;
-    if (mode == 19 && k % 256 == 0) mode = 60;
-    if ((mode == 13 || mode == 19) && k % 128 == 0) mode = tiles(64, 64) >= 768 ? 38 : 36;
-    if (force) mode = atoi(force);
-    if (mode >= 10 && !dma_ok) mode = 2;
+    if ((size_t)m * k < (1ull << 31) && (size_t)n * k < (1ull << 31) && n % 4 == 0)
+        return launch_gemm_tiles<EPI == kGemmDequant ? kDmaDequant : kDmaRaw>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
+    const int mode = ((m + 127) / 128) * ((n + 127) / 128) >= 1024 ? 0 : 2;
     const int nk = k / kGemmBK;
-    if (mode >= 10) {
-        constexpr int DE = EPI == kGemmDequant ? kDmaDequant : kDmaRaw;
-        if (mode == 12 && k % 128 == 0) return launch_gemm_dma<128, 128, DE, 2, 2, 128>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-        if (mode == 11) return launch_gemm_dma<128, 128, DE>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-        if (mode == 19) return launch_gemm_dma<64, 128, DE, 4, 2>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-        if (k % 128 == 0) {
-            if (mode == 36) return launch_gemm_dma<64, 64, DE, 4, 2, 128>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-            if (mode == 38) return launch_gemm_dma<64, 64, DE, 3, 3, 128>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-            if (k % 256 == 0) {
-                if (mode == 60) return launch_gemm_dma<64, 128, DE, 3, 2, 128, 8, 2>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-            }
-        }
-        return launch_gemm_dma<64, 64, DE>(a, w, c, s_x, w_s, residual, y, m, k, n, st);
-    }
 #define FX_GEMM_LAUNCH(BM, BN, DD)                                                                                \
     do {                                                                                                          \
         const int tm = (m + BM - 1) / BM, tn = (n + BN - 1) / BN;                                                 \
@@ -634,7 +604,6 @@ inline int launch_gemm(const int8_t* a, const int8_t* w, int32_t* c, const float
     } while (0)
     const bool deep = nk % 4 == 0;      // prefetch depth 4 needs the k-steps in groups of 4 (K % 256 == 0)
     if (mode == 0) { if (deep) FX_GEMM_LAUNCH(128, 128, 4); else FX_GEMM_LAUNCH(128, 128, 1); }
-    else if (mode == 1) { if (deep) FX_GEMM_LAUNCH(64, 128, 4); else FX_GEMM_LAUNCH(64, 128, 1); }
     else { if (deep) FX_GEMM_LAUNCH(64, 64, 4); else FX_GEMM_LAUNCH(64, 64, 1); }
 #undef FX_GEMM_LAUNCH
     FX_LAUNCH_CHECK();
@@ -647,48 +616,21 @@ inline int launch_gemm_asym(const int8_t* a, const int8_t* w, const float* s_x, 
                             const float* w_sum, const float* residual, float* y, int m, int k, int n, hipStream_t st) {
     FX_REQUIRE((size_t)m * k < (1ull << 31) && (size_t)n * k < (1ull << 31) && n % 4 == 0,
                "linear_i8_gemm_dequant_asym: m=%d k=%d n=%d outside the direct-load kernel's range", m, k, n);
-    auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     QkvEpiArgs qa = QkvEpiArgs();
     qa.b_x = b_x; qa.w_sum = w_sum;
-    constexpr int DE = kDmaDequantAsym;
-    static const char* force = getenv("FLEXLLM_GEMM_TILE");
-    const int fm = force ? atoi(force) : 0;
-    // Wide outputs (the separate gate and up projections of the W4A4 graph, 2048 -> 8192 at M = 1024), measured (us):
-    // 128x128 tiles, two stages of 128-byte rows 26.7; 128x128, three stages of 64-byte rows 31.8; 128x256 on four
-    // waves 38.7; 64x64 tiles 41.0.
-    if (k % 128 == 0 && (fm == 12 || (!fm && tiles(128, 128) >= 384)))
-        return launch_gemm_dma<128, 128, DE, 2, 2, 128>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (fm == 11 || (!fm && tiles(128, 128) >= 768)) return launch_gemm_dma<128, 128, DE>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (k % 256 == 0 && k >= 4096 && tiles(64, 128) >= 256 && (!fm || fm == 60))
-        return launch_gemm_dma<64, 128, DE, 3, 2, 128, 8, 2>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (k % 128 == 0) {
-        if (tiles(64, 64) >= 768) return launch_gemm_dma<64, 64, DE, 3, 3, 128>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
-        return launch_gemm_dma<64, 64, DE, 4, 2, 128>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
-    }
-    return launch_gemm_dma<64, 64, DE>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
+    return launch_gemm_tiles<kDmaDequantAsym>(a, w, nullptr, s_x, w_s, residual, y, m, k, n, st, qa);
 }
 
 // The gate/up projection of the W4A4 graph (interleaved rows, asymmetric activations held one value per byte) with
 // SiLU(gate)*up in the epilogue: the asymmetric dequantisation of launch_gemm_asym followed by the product that the
 // Hadamard kernel would otherwise form from the interleaved fp32 columns - the same arithmetic, half the output.
-// Tiles as in launch_gemm_swiglu: 256x256 where its grid fills the CUs in whole rounds (1024 tokens: 44 us against
-// 50 us for the unfused 128x128 kernel, and the transform after it reads half as much), smaller ones otherwise.
 inline int launch_gemm_swiglu_asym(const int8_t* a, const int8_t* w_gu, const float* s_x, const float* b_x, const float* w_s_gu,
                                    const float* w_sum_gu, float* h, int m, int k, int n2, hipStream_t st) {
     FX_REQUIRE((size_t)m * k < (1ull << 31) && (size_t)n2 * k < (1ull << 31) && n2 % 4 == 0,
                "linear_i8_gemm_swiglu_asym: m=%d k=%d n=%d outside the direct-load kernel's range", m, k, n2 / 2);
-    auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n2 + bn - 1) / bn); };
     QkvEpiArgs qa = QkvEpiArgs();
     qa.b_x = b_x; qa.w_sum = w_sum_gu;
-    constexpr int E = kDmaSwigluAsym;
-    if (k % 128 == 0) {
-        const int t256 = tiles(256, 256);
-        if (t256 >= 256 && (t256 % 256 == 0 || t256 >= 1024))
-            return launch_gemm_dma<256, 256, E, 2, 2, 128, 8>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st, qa);
-        if (tiles(128, 128) >= 384) return launch_gemm_dma<128, 128, E, 2, 2, 128>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st, qa);
-        return launch_gemm_dma<64, 64, E, 4, 2, 128>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st, qa);
-    }
-    return launch_gemm_dma<64, 64, E>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st, qa);
+    return launch_gemm_tiles<kDmaSwigluAsym>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st, qa);
 }
 
 // W4A4 prefill GEMM on nibble-packed operands (register-staged kernel, nibbles widened on the way to LDS).
@@ -714,20 +656,7 @@ inline int launch_gemm_swiglu(const int8_t* a, const int8_t* w_gu, const float* 
                               int k, int n2, hipStream_t st) {
     FX_REQUIRE((size_t)m * k < (1ull << 31) && (size_t)n2 * k < (1ull << 31) && n2 % 4 == 0,
                "linear_i8_gemm_swiglu: m=%d k=%d n=%d outside the direct-load kernel's range", m, k, n2 / 2);
-    // Measured at M=1024, 2048 -> 2x8192 (us): 256x256 tiles on eight waves, two stages of 128-byte rows, one
-    // workgroup per CU: 42.0; the same with four stages of 64-byte rows: 43.6; 128x256 tiles on four waves, two
-    // stages of 64-byte rows, two workgroups per CU: 49.3; 128x256 on eight waves: 48-57; 128x128 tiles (two or
-    // three per CU) and 256x256 on four waves: 48-58.  The big tile is taken when its grid fills the 256 CUs in
-    // whole rounds (or many of them); FLEXLLM_GEMM_TILE forces 50 / 16 / 13 (the 64x64 fallback).
-    static const char* force = getenv("FLEXLLM_GEMM_TILE");
-    const int tiles_256 = ((m + 255) / 256) * ((n2 + 255) / 256);
-    const int tiles_big = ((m + 127) / 128) * ((n2 + 255) / 256);
-    int mode = (k % 128 == 0 && tiles_256 >= 256 && (tiles_256 % 256 == 0 || tiles_256 >= 1024)) ? 50 : tiles_big >= 384 ? 16 : 13;
-    if (force) mode = atoi(force);
-    if (mode == 50 && k % 128 == 0)
-        return launch_gemm_dma<256, 256, kDmaSwiglu, 2, 2, 128, 8>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st);
-    if (mode == 16) return launch_gemm_dma<128, 256, kDmaSwiglu, 2, 2>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st);
-    return launch_gemm_dma<64, 64, kDmaSwiglu>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st);
+    return launch_gemm_tiles<kDmaSwiglu>(a, w_gu, nullptr, s_x, w_s_gu, nullptr, h, m, k, n2, st);
 }
 
 // Fused q/k/v projection: GEMM over the concatenated [q | k | v] weight rows with RoPE, static int8 quantisation and
@@ -738,13 +667,7 @@ inline int launch_gemm_qkv(const int8_t* a, const int8_t* w_qkv, const float* s_
     const int n = (qa.q_heads + 2 * qa.kv_heads) * kHd;
     FX_REQUIRE(m % 32 == 0 && qa.pos0 % 64 == 0 && qa.pos0 + m <= qa.max_pos, "gemm_qkv: m=%d pos0=%d max_pos=%d", m, qa.pos0, qa.max_pos);
     FX_REQUIRE((size_t)m * k < (1ull << 31) && (size_t)n * k < (1ull << 31), "gemm_qkv: m=%d k=%d outside the direct-load kernel's range", m, k);
-    static const char* force = getenv("FLEXLLM_GEMM_TILE");
-    const int mode = force ? atoi(force) : (((m + 63) / 64) * (n / 64) >= 768 ? 38 : 36);
-    if (k % 128 == 0) {
-        if (mode == 36) return launch_gemm_dma<64, 64, kDmaQkv, 4, 2, 128>(a, w_qkv, nullptr, s_x, w_s, nullptr, nullptr, m, k, n, st, qa);
-        if (mode == 38) return launch_gemm_dma<64, 64, kDmaQkv, 3, 3, 128>(a, w_qkv, nullptr, s_x, w_s, nullptr, nullptr, m, k, n, st, qa);
-    }
-    return launch_gemm_dma<64, 64, kDmaQkv>(a, w_qkv, nullptr, s_x, w_s, nullptr, nullptr, m, k, n, st, qa);
+    return launch_gemm_tiles<kDmaQkv>(a, w_qkv, nullptr, s_x, w_s, nullptr, nullptr, m, k, n, st, qa);
 }
 
 }  // namespace fx
