@@ -53,7 +53,12 @@ struct GemvArgs {
     const float* route = nullptr; int ld_route = 0, experts = 0, top = 0;
     int* pick = nullptr; float* pick_w = nullptr;
     size_t w_stride = 0;
+    // several tokens at prologue 0: each reads the weights for itself; or one pass over them, whose k may be shared out (n_split 0,
+    // no bias) as in GemmArgs, in gemv_parts parts
+    bool per_token = false;
+    int parts = 1; size_t part_stride = 0;
 };
+template <typename ET> int gemv_parts(int n, int kpad, int most);
 template <typename ET> int gemv_float(const GemvArgs& g, int prologue, int tokens, hipStream_t st);
 // y[t] = sum_i pick_w[t][i] * W_down[pick[t][i]] h[t*top+i]  (+ sigmoid(gate) * W_shared hs[t], gate = route[t][experts])
 struct MoeDownArgs {

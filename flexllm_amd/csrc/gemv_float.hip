@@ -4,10 +4,12 @@
 // The first two groups are requested before the prologue (residual, norms) runs, so that its latency lies under the weight
 // stream, and two groups stay in flight after that.  The R sums are reduced together (multi_sum_step).
 #include "float_ops.h"
+#include <atomic>
 
 namespace fx {
 
 constexpr int kMaxExperts = 1024, kMaxTop = 32;
+constexpr size_t kGemvTokensLds = 128 * 1024;             // vectors of gemv_tokens_kernel
 
 // Expert choice of one token by one wave: softmax over the router outputs, the `top` largest (ties: lower index), their
 // weights divided by their sum.  Lane k < top gets choice k and its weight.  NE: 64-expert pieces (experts <= 64 NE).
@@ -276,12 +278,274 @@ static int launch_gemv_rs(const GemvArgs& g, int pro, int tokens, hipStream_t st
     return FLEXLLM_OK;
 }
 
+// The same linear for TT tokens at a time (prologue 0): a piece of a weight row in registers meets the TT vectors in LDS, so the
+// weights are read once per TT tokens instead of once per token.  A thread's floats of the vectors lie in planes of 4 (one for
+// float32, two for bfloat16 pieces of 8), so that neighbouring lanes read neighbouring 16 bytes.
+template <typename ET, int TT, int R, int S>
+__global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens) {
+    constexpr int CE = Chunk<ET>::N, PL = CE / 4;
+    constexpr int SUMS = R * TT <= 4 ? 4 : R * TT <= 8 ? 8 : R * TT <= 16 ? 16 : 32;
+    static_assert(R * TT <= 32, "sums per lane");
+    extern __shared__ __attribute__((aligned(16))) float xs[];     // [TT][PL][nchunk][4]
+    __shared__ float red[2][4 * SUMS];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, tok0 = blockIdx.y * TT;
+    const ET* w = static_cast<const ET*>(g.w);
+    const int nchunk = g.kpad / CE, ng = (g.n + R - 1) / R, G = gridDim.x;
+    // the vectors first: loads return in order, and the weights behind them are a long stream
+    const bool vec = (g.k & 3) == 0 && (g.ldx & 3) == 0;
+#pragma unroll
+    for (int j = 0; j < TT; j++) {
+        const float* x = g.x + (size_t)min(tok0 + j, tokens - 1) * g.ldx;
+        for (int c = t; c < g.kpad / 4; c += 256) {
+            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (vec) {
+                if (4 * c < g.k) v = *reinterpret_cast<const f32x4*>(x + 4 * c);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = 4 * c + e < g.k ? x[4 * c + e] : 0.0f;
+            }
+            *reinterpret_cast<f32x4*>(xs + ((size_t)(j * PL + c % PL) * nchunk + c / PL) * 4) = v;
+        }
+    }
+    i32x4 buf[2][R][S];
+    auto piece = [&](int row, int c) { return *reinterpret_cast<const i32x4*>(w + (size_t)min(row, g.n - 1) * g.kpad + c * CE); };
+    auto load = [&](int b, int grp) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                const int c = s * 256 + t;
+                buf[b][r][s] = c < nchunk ? piece(grp * R + r, c) : i32x4{0, 0, 0, 0};
+            }
+    };
+    const int g0 = blockIdx.x;
+    load(0, g0);
+    if (g0 + G < ng) load(1, g0 + G);
+    __syncthreads();
+    // piece c of R rows (u[.][s]) meets the vectors' piece c
+    auto take = [&](const i32x4 (&u)[R][S], int s, int c, float (&acc)[SUMS]) {
+        float wv[R][CE];
+#pragma unroll
+        for (int r = 0; r < R; r++) Chunk<ET>::unpack(make_uint4(u[r][s][0], u[r][s][1], u[r][s][2], u[r][s][3]), wv[r]);
+#pragma unroll
+        for (int j = 0; j < TT; j++)
+#pragma unroll
+            for (int q = 0; q < PL; q++) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(xs + ((j * PL + q) * nchunk + c) * 4);
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[r * TT + j] = fma_f(wv[r][q * 4 + e], v[e], acc[r * TT + j]);
+            }
+    };
+    auto process = [&](int b, int grp) {
+        float acc[SUMS];
+#pragma unroll
+        for (int i = 0; i < SUMS; i++) acc[i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < S; s++) take(buf[b], s, min(s * 256 + t, nchunk - 1), acc);     // pieces beyond the row were filled with zeros
+        for (int c = S * 256 + t; c < nchunk; c += 256) {
+            i32x4 more[R][S];
+#pragma unroll
+            for (int r = 0; r < R; r++) more[r][0] = piece(grp * R + r, c);
+            take(more, 0, c, acc);
+        }
+        multi_sum_step<SUMS, 1>(acc, lane);
+        if (lane < SUMS) red[b][wave * SUMS + multi_row<SUMS>(lane)] = acc[0];
+        __syncthreads();                                  // red alternates with the buffer: one barrier per group is enough
+        const int r = t / TT, j = t - r * TT, row = grp * R + r, tok = tok0 + j;
+        if (t < R * TT && row < g.n && tok < tokens) {
+            auto total = [&](int i) {
+                const float* p = red[b] + min(r + i, R - 1) * TT + j;
+                const float v = (p[0] + p[SUMS]) + (p[2 * SUMS] + p[3 * SUMS]);
+                return g.bias ? v + g.bias[min(row + i, g.n - 1)] : v;
+            };
+            if (row >= g.n_split) g.out32[(size_t)tok * g.ldo32 + row - g.n_split] = total(0);
+            else if (!g.glu) g.out[(size_t)tok * g.ldo + row] = total(0);
+            else if ((row & 1) == 0) g.out[(size_t)tok * g.ldo + (row >> 1)] = glu_f(g.glu, total(0), total(1), g.limit);
+        }
+    };
+    for (int grp = g0; grp < ng; grp += 2 * G) {
+        process(0, grp);
+        if (grp + 2 * G < ng) load(0, grp + 2 * G);
+        if (grp + G < ng) {
+            process(1, grp + G);
+            if (grp + 3 * G < ng) load(1, grp + 3 * G);
+        }
+    }
+}
+
+template <typename ET, int TT, int R, int S>
+static int launch_gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
+    const size_t lds = (size_t)TT * g.kpad * sizeof(float);
+    static std::atomic<bool> opted_in{false};
+    if (!opted_in.load(std::memory_order_acquire)) {
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_tokens_kernel<ET, TT, R, S>), hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTokensLds));
+        opted_in.store(true, std::memory_order_release);
+    }
+    const int groups = (tokens + TT - 1) / TT, per_cu = lds <= 36 * 1024 ? 4 : lds <= 72 * 1024 ? 2 : 1, ng = (g.n + R - 1) / R;
+    const int wgs = 256 * per_cu / groups;                // what is resident at a time
+    gemv_tokens_kernel<ET, TT, R, S><<<dim3(ng < wgs ? ng : wgs, groups), 256, lds, st>>>(g, tokens);
+    FX_LAUNCH_CHECK();
+    return FLEXLLM_OK;
+}
+
+// R x S pieces per thread and group as for one token, TT as many tokens as LDS holds.
+template <typename ET, int R, int S>
+static int gemv_tokens_rs(const GemvArgs& g, int tokens, hipStream_t st) {
+    const int fit = (int)(kGemvTokensLds / (g.kpad * sizeof(float))), most = fit < 32 / R ? fit : 32 / R;
+    const int cap = most >= 8 ? 8 : most >= 6 ? 6 : most >= 4 ? 4 : 2, groups = (tokens + cap - 1) / cap, tt = (tokens + groups - 1) / groups;
+    if constexpr (R <= 4) if (tt > 6) return launch_gemv_tokens<ET, 8, R, S>(g, tokens, st);
+    if (tt > 4) return launch_gemv_tokens<ET, 6, R, S>(g, tokens, st);
+    if (tt > 2) return launch_gemv_tokens<ET, 4, R, S>(g, tokens, st);
+    return launch_gemv_tokens<ET, 2, R, S>(g, tokens, st);
+}
+
+template <typename ET>
+static int gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
+    const int per = 256 * Chunk<ET>::N, steps = (g.kpad + per - 1) / per;
+    if (steps == 1) return gemv_tokens_rs<ET, 4, 1>(g, tokens, st);
+    if (steps == 2) return gemv_tokens_rs<ET, 2, 2>(g, tokens, st);
+    if (steps <= 4 || g.glu) return gemv_tokens_rs<ET, 2, 4>(g, tokens, st);      // a pair of the gated unit lies in one group
+    return gemv_tokens_rs<ET, 1, 8>(g, tokens, st);
+}
+
+// bfloat16 weights on the matrix cores: a float32 vector is the sum of three bfloat16 parts to 24 bits and their products with the
+// weights are exact in float32, so three instructions per 16 rows x 32 k give what the float32 products give (vector
+// instructions: 16384 x 2048 for 5 tokens 24 us, the weights' stream is 10).  A workgroup of eight waves walks tiles of 16 rows; the
+// waves share its stretch of k (KW steps of 32 each), whose vectors lie in LDS as [part][token][stretch, padded by 16 bytes: the
+// tokens of an operand read are then on different banks], and meet through LDS per tile, two tiles' weights in flight.
+constexpr int kMfmaTokens = 16, kMfmaWaves = 8;
+constexpr int gemv_mfma_row(int stretch) { return stretch * 2 + 16; }      // bytes of a token's part
+template <int KW>
+__global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, int tokens, int group) {
+    constexpr int NT = kMfmaWaves * 64, STRETCH = KW * kMfmaWaves * 32, ROW = gemv_mfma_row(STRETCH);
+    extern __shared__ __attribute__((aligned(16))) int8_t xp[];    // [3][group][ROW]
+    __shared__ float red[2][kMfmaWaves][16 * 17];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int part = blockIdx.x % g.parts, walker = blockIdx.x / g.parts, walkers = gridDim.x / g.parts;
+    const int tok0 = blockIdx.y * group, nt = min(group, tokens - tok0), k0 = part * STRETCH, tiles = (g.n + 15) / 16;
+    for (int i = t; i < nt * (STRETCH / 4); i += NT) {
+        const int j = i / (STRETCH / 4), c = i - j * (STRETCH / 4), k = k0 + 4 * c;
+        const float* x = g.x + (size_t)(tok0 + j) * g.ldx;
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if ((g.k & 3) == 0 && (g.ldx & 3) == 0) {
+            if (k < g.k) v = *reinterpret_cast<const f32x4*>(x + k);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = k + e < g.k ? x[k + e] : 0.0f;
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            bf16x4 b;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                b[e] = (bf16_t)v[e];
+                v[e] -= (float)b[e];
+            }
+            *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
+        }
+    }
+    const int wk = wave * (KW * 32) + (lane >> 4) * 8;    // this lane's k within the stretch
+    const bf16_t* w = static_cast<const bf16_t*>(g.w) + k0 + wk;
+    bf16x8 buf[2][KW];
+    auto load = [&](int b, int tile) {
+        const bf16_t* row = w + (size_t)min(tile * 16 + (lane & 15), g.n - 1) * g.kpad;
+#pragma unroll
+        for (int s = 0; s < KW; s++)
+            if (k0 + wave * (KW * 32) + s * 32 < g.kpad) buf[b][s] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(row + s * 32));
+            else
+#pragma unroll
+                for (int e = 0; e < 8; e++) buf[b][s][e] = (bf16_t)0.0f;
+    };
+    load(0, walker);
+    if (walker + walkers < tiles) load(1, walker + walkers);
+    __syncthreads();
+    const int8_t* xl = xp + min(lane & 15, nt - 1) * ROW + wk * 2;
+    auto process = [&](int b, int tile) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < KW; s++)
+#pragma unroll
+            for (int p = 2; p >= 0; p--)                  // the small parts first
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf[b][s], *reinterpret_cast<const bf16x8*>(xl + p * group * ROW + s * 64), acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[b][wave][((lane >> 4) * 4 + i) * 17 + (lane & 15)] = acc[i];
+        __syncthreads();                                  // red alternates with the buffer: one barrier per tile is enough
+        const int r = t & 15, j = t >> 4, row = tile * 16 + r, tok = tok0 + j;
+        if (j < nt && row < g.n) {
+            auto total = [&](int i) {
+                const float* p = red[b][0] + (r + i) * 17 + j;
+                float v[kMfmaWaves];
+#pragma unroll
+                for (int q = 0; q < kMfmaWaves; q++) v[q] = p[q * 16 * 17];
+                const float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+                return g.bias ? s + g.bias[min(row + i, g.n - 1)] : s;
+            };
+            if (row >= g.n_split) g.out32[part * g.part_stride + (size_t)tok * g.ldo32 + row - g.n_split] = total(0);
+            else if (!g.glu) g.out[(size_t)tok * g.ldo + row] = total(0);
+            else if ((row & 1) == 0) g.out[(size_t)tok * g.ldo + (row >> 1)] = glu_f(g.glu, total(0), total(1), g.limit);
+        }
+    };
+    for (int tile = walker; tile < tiles; tile += 2 * walkers) {
+        process(0, tile);
+        if (tile + 2 * walkers < tiles) load(0, tile + 2 * walkers);
+        if (tile + walkers < tiles) {
+            process(1, tile + walkers);
+            if (tile + 3 * walkers < tiles) load(1, tile + 3 * walkers);
+        }
+    }
+}
+
+template <int KW>
+static int launch_gemv_mfma(const GemvArgs& g, int tokens, hipStream_t st) {
+    constexpr int STRETCH = KW * kMfmaWaves * 32, fit = (int)(kGemvTokensLds / (3 * gemv_mfma_row(STRETCH)));
+    constexpr int most = fit < kMfmaTokens ? fit : kMfmaTokens;
+    static_assert(most >= 4, "tokens that fit");
+    static std::atomic<bool> opted_in{false};
+    if (!opted_in.load(std::memory_order_acquire)) {
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mfma_kernel<KW>), hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTokensLds));
+        opted_in.store(true, std::memory_order_release);
+    }
+    const int groups = (tokens + most - 1) / most, group = (tokens + groups - 1) / groups, tiles = (g.n + 15) / 16;
+    const size_t lds = (size_t)3 * group * gemv_mfma_row(STRETCH);
+    int walkers = 256 / (g.parts * groups);               // one workgroup per CU: a second one does not speed the stream up
+    if (walkers < 1) walkers = 1;
+    if (walkers > tiles) walkers = tiles;
+    gemv_mfma_kernel<KW><<<dim3(walkers * g.parts, groups), kMfmaWaves * 64, lds, st>>>(g, tokens, group);
+    FX_LAUNCH_CHECK();
+    return FLEXLLM_OK;
+}
+
+// k of a workgroup: 1024, 2048 or 4096.  Parts of a product whose reader adds them: as few as that takes, one more doubling where the
+// rows alone leave CUs without a tile (2048 x 2048).
+template <>
+int gemv_parts<bf16_t>(int n, int kpad, int most) {
+    int parts = (kpad + 2047) / 2048;
+    if (parts > most) return 1;
+    if (parts * 2 <= most && kpad >= parts * 2048 && (n + 15) / 16 * parts < 256) parts *= 2;
+    return parts;
+}
+template <>
+int gemv_parts<float>(int, int, int) { return 1; }
+
 template <typename ET>
 int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     FX_REQUIRE(g.w && g.x && g.n > 0 && g.k > 0 && g.kpad >= g.k && g.kpad % kKPad == 0 && tokens > 0, "gemv_float: n=%d k=%d", g.n, g.k);
     FX_REQUIRE(g.kpad <= 15360, "gemv_float: k=%d beyond 15360 (the vector is held in LDS)", g.k);
     FX_REQUIRE(pro != 2 || (g.experts > 0 && g.experts <= kMaxExperts && g.top > 0 && g.top <= kMaxTop && g.top <= g.experts),
                "gemv_float: %d experts, top %d (at most %d, %d)", g.experts, g.top, kMaxExperts, kMaxTop);
+    FX_REQUIRE(g.parts == 1 || (std::is_same<ET, bf16_t>::value && pro == 0 && tokens > 1 && g.n_split == 0 && !g.bias), "gemv_float: %d parts", g.parts);
+    if (pro == 0 && tokens > 1 && !g.per_token) {
+        if constexpr (std::is_same<ET, bf16_t>::value) {
+            const int stretch = (g.kpad + g.parts - 1) / g.parts;
+            if (stretch <= 1024) return launch_gemv_mfma<4>(g, tokens, st);
+            if (stretch <= 2048) return launch_gemv_mfma<8>(g, tokens, st);
+            if (stretch <= 4096) return launch_gemv_mfma<16>(g, tokens, st);
+            FX_REQUIRE(g.parts == 1, "gemv_float: %d parts of k=%d", g.parts, g.k);
+        }
+        return gemv_tokens<ET>(g, tokens, st);
+    }
     const int per = 256 * Chunk<ET>::N, steps = (g.kpad + per - 1) / per;
     // Rows per group: four pieces per thread and group where workgroups walk several groups (a group's sums and barrier then
     // overlap the next group's loads: 16384 x 2048 13.9 us with eight, 12.9 with four; 28672 x 4096 42.2 -> 37.7 us), eight

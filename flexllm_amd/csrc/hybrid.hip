@@ -414,7 +414,7 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
     FX_TRY(own(m, m->xa, T * W));
     FX_TRY(own(m, m->xb, T * W));
     FX_TRY(own(m, m->hn, T * W));
-    FX_TRY(own(m, m->y, T * W));
+    FX_TRY(own(m, m->y, kMaxParts * T * W));
     FX_TRY(own(m, m->hw, T * W));
     FX_TRY(own(m, m->proj, T * m->max_et));
     FX_TRY(own(m, m->f32, T * (m->max_f32 + 4)));
@@ -500,8 +500,14 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
     return FLEXLLM_OK;
 }
 
+// A linear behind a norm, for T tokens of a step: every token reads the weights (from L2, behind the first) under its own norm's
+// prologue while the bytes read again are few, else the norms have a launch of their own (4.6 us) ahead of one pass over the
+// weights.  Two tokens, 16 layers of 2048: 1162 us with the former everywhere, 1390 us with the latter; four layers of 4096: 952
+// and 874 us; five tokens, gate and up of 2048 x 8192: 35 us and 4.6 + 17.
+static bool reads_again(int T, int n, int kpad, int es) { return T == 1 || (size_t)(T - 1) * n * kpad * es <= ((size_t)72 << 20); }
+
 // ---- one to kSmallTokens tokens --------------------------------------------------------------------------------------
-struct Pending { bool on = false; const float* gb = nullptr; };      // the last sublayer's output in y still has to be added
+struct Pending { bool on = false; const float* gb = nullptr; int parts = 1; };      // the last sublayer's output in y (in parts) still has to be added
 
 template <typename ET>
 static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, const int* want, int n_want, float* logits, float* layers_out, hipStream_t st) {
@@ -518,12 +524,12 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
     auto settle = [&] {                                   // take the pending output in, without a norm behind it
         if (!pend.on) return FLEXLLM_OK;
         RowArgs r;
-        r.x = x; r.x_new = other; r.y = m->y; r.ldy = W; r.gb = pend.gb; r.eps = c.eps; r.width = W; r.rows = T;
+        r.x = x; r.x_new = other; r.y = m->y; r.ldy = W; r.y_parts = pend.parts; r.y_stride = (size_t)T * W; r.gb = pend.gb; r.eps = c.eps; r.width = W; r.rows = T;
         const int rc = norm_rows<ET>(r, st);
         moved();
         return rc;
     };
-    auto pending = [&](const float* gb) { pend.on = true; pend.gb = gb; };
+    auto pending = [&](const float* gb, int parts = 1) { pend.on = true; pend.gb = gb; pend.parts = parts; };
     auto base = [&](const void* w, int n, int k) {
         GemvArgs a;
         a.w = w; a.n = n; a.k = k; a.kpad = pad_k(k); a.eps = c.eps;
@@ -531,6 +537,17 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
     };
     // linear on norm(x + pending [+ x0])
     auto norm_linear = [&](GemvArgs a, const float* g, bool add_x0 = false) {
+        if (pend.parts > 1 || !reads_again(T, a.n, a.kpad, sizeof(ET))) {
+            RowArgs r;
+            r.x = x; r.eps = c.eps; r.width = W; r.rows = T; r.h = m->hn; r.ldh = W; r.h_f32 = 1; r.g = g;
+            if (pend.on) { r.y = m->y; r.ldy = W; r.y_parts = pend.parts; r.y_stride = (size_t)T * W; r.gb = pend.gb; }
+            if (add_x0) r.x0 = m->x0;
+            if (pend.on || add_x0) r.x_new = other;
+            FX_TRY(norm_rows<ET>(r, st));
+            if (r.x_new) moved();
+            a.x = m->hn; a.ldx = W;
+            return gemv_float<ET>(a, 0, T, st);
+        }
         if (add_x0 && pend.gb) FX_TRY(settle());          // the kernel takes a norm's weight or x0
         a.x = x; a.ldx = W; a.g = g;
         if (pend.on) { a.y = m->y; a.ldy = W; a.gb = pend.gb; }
@@ -541,9 +558,13 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
         if (changes) moved();
         return rc;
     };
-    auto plain_linear = [&](const void* w, int n, int k, const float* v, int ldv, float* out) {
-        GemvArgs a = base(w, n, k);
-        a.x = v; a.ldx = ldv; a.n_split = 0; a.out32 = out; a.ldo32 = n;
+    // linear onto the pending output
+    auto to_y = [&](const void* w, int k, const float* v, int ldv, const float* gb, bool shared) {      // shared: k may be shared out
+        GemvArgs a = base(w, W, k);
+        a.x = v; a.ldx = ldv; a.n_split = 0; a.out32 = m->y; a.ldo32 = W;
+        a.per_token = T == 2 && W * sizeof(ET) <= 4096;   // short rows: as cheap, and the next linear's prologue takes the sum as it is
+        if (T > 1 && !a.per_token && shared) { a.parts = gemv_parts<ET>(W, a.kpad, kMaxParts); a.part_stride = (size_t)T * W; }
+        pending(gb, a.parts);
         return gemv_float<ET>(a, 0, T, st);
     };
     const int runs = (int)m->runs.size();
@@ -567,14 +588,12 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
         } else {
             FX_TRY(gla_steps<ET>(L.gd, m->proj, m->max_et, 1, m->f32, nf, static_cast<ET*>(L.a2), L.a2_bias, L.head_norm, s.state[r], s.pos, 0, T, m->att, m->max_att, 1, st));
         }
-        FX_TRY(plain_linear(L.w_o, W, L.k_o, m->att, m->max_att, m->y));
-        pending(L.g1b);
+        FX_TRY(to_y(L.w_o, L.k_o, m->att, m->max_att, L.g1b, L.d.ff_kind == FLEXLLM_FF_DENSE && !reads_again(T, 2 * L.d.ff, kw, sizeof(ET))));
         if (L.d.ff_kind == FLEXLLM_FF_DENSE) {
             a = base(L.w_gu, 2 * L.d.ff, W);
             a.n_split = 2 * L.d.ff; a.glu = 1 + L.d.glu; a.limit = L.d.limit; a.out = m->hid; a.ldo = L.d.ff;
             FX_TRY(norm_linear(a, L.g2));
-            FX_TRY(plain_linear(L.w_d, W, L.d.ff, m->hid, L.d.ff, m->y));
-            pending(L.g2b);
+            FX_TRY(to_y(L.w_d, L.d.ff, m->hid, L.d.ff, L.g2b, true));
         } else if (L.d.ff_kind == FLEXLLM_FF_MOE) {
             const int sf = L.d.shared_ff, ldr = L.n_side - 2 * sf;
             a = base(L.w_side, L.n_side, W);

@@ -114,3 +114,17 @@ def test_slices_of_a_prompt(dtype):
     for n in (63, 64, 65, 129):
         check_lopazen(lc.config([lc.layer(heads=4, kv_heads=2, dim=264, scale=0.06)]), dtype, n, [n], [9, n])
         check_nifunex(nc.config([nc.latent(heads=2, dim=264, rot_dim=8, vdim=16, kv_rank=48, window=50, scale=0.06)]), dtype, n, [n], [9, n])
+
+
+# two to eight tokens in one step: every number of tokens per pass over the weights, vectors of one to fifteen pieces per thread, a
+# gated unit on vectors so long that its pairs need two rows per group, odd lengths, a mixture
+@BOTH
+@pytest.mark.parametrize("width,ff", [(160, 88), (90, 33), (2112, 2050), (64, 4100), (64, 8200), (64, 15360), (8256, 40)])
+def test_step_of_several_tokens(width, ff, dtype):
+    cfg = lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff))], width=width, vocab=131, loop=(0, 1, 2))
+    check_lopazen(cfg, dtype, 35, [2, 3, 4, 5, 6, 7, 8])
+
+
+@BOTH
+def test_step_of_several_tokens_nifunex(dtype):
+    check_nifunex(nc.mixed(), dtype, 35, [2, 3, 4, 5, 6, 7, 8], skip=0.05)
