@@ -560,37 +560,67 @@ template int gemv_float<bf16_t>(const GemvArgs&, int, int, hipStream_t);
 template int gemv_float<float>(const GemvArgs&, int, int, hipStream_t);
 
 // Down projections of the chosen experts and of the shared one, summed with their weights.  The sources lie one after
-// the other in a list of 16-byte pieces, which the threads walk together; R = 4 output rows per workgroup.
-template <typename ET>
+// the other in a list of 16-byte pieces, which the threads walk together; R = 4 output rows per workgroup.  The trips to
+// memory bound it: a pick, the weights behind it, the sum.  So a thread requests B = 4 pieces of each row, and what they
+// meet, before it takes the first one in.  Six experts of 2048 x 1024 and a shared one of 2048, one token, 33.5 MB: 12.4 us
+// with one piece after the other, 9.6 us so (3.5 TB/s).  NT: one token, whose weights are read once; several tokens share
+// them through the L2.
+template <typename ET, bool NT>
 __global__ __launch_bounds__(256) void moe_down_kernel(MoeDownArgs a) {
-    constexpr int CE = Chunk<ET>::N, R = 4;
+    constexpr int CE = Chunk<ET>::N, R = 4, B = 4;
     __shared__ float red[4 * R];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, tok = blockIdx.y, row0 = blockIdx.x * R;
     const int ce = a.kpad / CE, cs = a.ws ? a.ks_pad / CE : 0, total = a.top * ce + cs;
+    const bool vec = ((a.k | a.ldh) & 3) == 0 && (!a.ws || ((a.ks | a.ldhs) & 3) == 0);
     float acc[R] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float sg = 0.0f;
-    if (a.ws) sg = sigmoid_f(a.route[(size_t)tok * a.ld_route + a.experts]);
-#pragma unroll 4
-    for (int it = t; it < total; it += 256) {
-        const bool sh = it >= a.top * ce;
-        const int slot = sh ? 0 : it / ce, c = sh ? it - a.top * ce : it - slot * ce;
-        const int kp = sh ? a.ks_pad : a.kpad, kk = sh ? a.ks : a.k;
-        const ET* w = sh ? static_cast<const ET*>(a.ws) : static_cast<const ET*>(a.w) + (size_t)a.pick[tok * a.top + slot] * a.w_stride;
-        const float wt = sh ? sg : a.pick_w[tok * a.top + slot];
-        const float* h = sh ? a.hs + (size_t)tok * a.ldhs : a.h + (size_t)(tok * a.top + slot) * a.ldh;
-        uint4 u[R];
+    for (int i0 = t; i0 < total; i0 += 256 * B) {
+        i32x4 u[B][R];
+        float x[B][CE], wt[B];
 #pragma unroll
-        for (int r = 0; r < R; r++) u[r] = *reinterpret_cast<const uint4*>(w + (size_t)min(row0 + r, a.n - 1) * kp + c * CE);
-        float xv[CE];
+        for (int b = 0; b < B; b++) {
+            const int it = min(i0 + 256 * b, total - 1);
+            const bool sh = it >= a.top * ce;
+            const int slot = sh ? 0 : it / ce, c = sh ? it - a.top * ce : it - slot * ce, kp = sh ? a.ks_pad : a.kpad;
+            const ET* w = sh ? static_cast<const ET*>(a.ws) : static_cast<const ET*>(a.w) + (size_t)a.pick[tok * a.top + slot] * a.w_stride;
 #pragma unroll
-        for (int e = 0; e < CE; e++) xv[e] = c * CE + e < kk ? h[c * CE + e] : 0.0f;
+            for (int r = 0; r < R; r++) {
+                const i32x4* p = reinterpret_cast<const i32x4*>(w + (size_t)min(row0 + r, a.n - 1) * kp + c * CE);
+                if constexpr (NT) u[b][r] = __builtin_nontemporal_load(p);
+                else u[b][r] = *p;
+            }
+        }
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            float wv[CE], s = 0.0f;
-            Chunk<ET>::unpack(u[r], wv);
+        for (int b = 0; b < B; b++) {
+            const int it = min(i0 + 256 * b, total - 1);
+            const bool sh = it >= a.top * ce;
+            const int slot = sh ? 0 : it / ce, c = sh ? it - a.top * ce : it - slot * ce, kk = sh ? a.ks : a.k;
+            const float* h = sh ? a.hs + (size_t)tok * a.ldhs : a.h + (size_t)(tok * a.top + slot) * a.ldh;
+            wt[b] = sh ? a.route[(size_t)tok * a.ld_route + a.experts] : a.pick_w[tok * a.top + slot];
+            if (vec) {
 #pragma unroll
-            for (int e = 0; e < CE; e++) s = fma_f(wv[e], xv[e], s);
-            acc[r] = fma_f(wt, s, acc[r]);
+                for (int q = 0; q < CE; q += 4) {
+                    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (c * CE + q < kk) v = *reinterpret_cast<const f32x4*>(h + c * CE + q);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[b][q + e] = v[e];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < CE; e++) x[b][e] = c * CE + e < kk ? h[c * CE + e] : 0.0f;
+            }
+            if (sh) wt[b] = sigmoid_f(wt[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            if (i0 + 256 * b >= total) break;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float wv[CE], s = 0.0f;
+                Chunk<ET>::unpack(make_uint4(u[b][r][0], u[b][r][1], u[b][r][2], u[b][r][3]), wv);
+#pragma unroll
+                for (int e = 0; e < CE; e++) s = fma_f(wv[e], x[b][e], s);
+                acc[r] = fma_f(wt[b], s, acc[r]);
+            }
         }
     }
     multi_sum_step<R, 1>(acc, lane);
@@ -603,7 +633,9 @@ __global__ __launch_bounds__(256) void moe_down_kernel(MoeDownArgs a) {
 template <typename ET>
 int moe_down_small(const MoeDownArgs& a, int tokens, hipStream_t st) {
     FX_REQUIRE(a.w && a.h && a.pick && a.pick_w && a.y && a.n > 0 && tokens > 0, "moe_down: null pointer");
-    moe_down_kernel<ET><<<dim3((a.n + 3) / 4, tokens), 256, 0, st>>>(a);
+    const dim3 grid((a.n + 3) / 4, tokens);
+    if (tokens == 1) moe_down_kernel<ET, true><<<grid, 256, 0, st>>>(a);
+    else moe_down_kernel<ET, false><<<grid, 256, 0, st>>>(a);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }

@@ -128,3 +128,12 @@ def test_step_of_several_tokens(width, ff, dtype):
 @BOTH
 def test_step_of_several_tokens_nifunex(dtype):
     check_nifunex(nc.mixed(), dtype, 35, [2, 3, 4, 5, 6, 7, 8], skip=0.05)
+
+
+# the experts' down projections of a step: fewer pieces than threads, more than one pass of them, a last pass that is ragged, units that
+# are read four at a time and such that are not, no shared expert, rows that do not fill a group
+@BOTH
+@pytest.mark.parametrize("top,ff,shared,width", [(1, 8, 0, 66), (2, 41, 56, 90), (3, 40, 57, 130), (6, 1024, 2048, 160), (4, 2100, 0, 70), (5, 822, 410, 64)])
+def test_experts_down(top, ff, shared, width, dtype):
+    cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(top + 1, top, ff, 1.5, shared)), nc.gla(heads=1, mlp=nc.dense(72))], width=width)
+    check_nifunex(cfg, dtype, 20, [1], [3], skip=0.1)
