@@ -441,7 +441,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 b[e] = (bf16_t)v[e];
-                v[e] -= (float)b[e];
+                v[e] = isinf(v[e]) ? 0.0f : v[e] - (float)b[e];     // an infinity has no rest
             }
             *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
         }

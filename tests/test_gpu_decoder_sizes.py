@@ -137,3 +137,28 @@ def test_step_of_several_tokens_nifunex(dtype):
 def test_experts_down(top, ff, shared, width, dtype):
     cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(top + 1, top, ff, 1.5, shared)), nc.gla(heads=1, mlp=nc.dense(72))], width=width)
     check_nifunex(cfg, dtype, 20, [1], [3], skip=0.1)
+
+
+@BOTH
+@pytest.mark.parametrize("ff", [88, 2050])
+def test_infinite_units(ff, dtype):
+    """A unit beyond float32 leaves infinities of the same signs in the residual, however many tokens a step has.  (The gate itself
+    stays small enough for its cube, which gelu forms, to be finite: about 1e12.)"""
+    from flexllm_amd.lopazen import Lopazen
+    cfg = lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff))])
+    w, toks = lc.weights(cfg, 11), lc.tokens(cfg, 6)
+    for name in w:
+        if name.endswith((".gate", ".up")):
+            w[name][5] = lc.round_bf16(w[name][5] * np.float32(1e4 if name.endswith("gate") else 1e36))
+        if name.endswith(".down"):
+            w[name][:, 5] = np.where(w[name][:, 5] < 0, -1.0, 1.0)
+    m = Lopazen.from_tensors(cfg, w, dtype=dtype, max_pos=64)
+    got = {}
+    for n in (1, 3):
+        slot = m.pool.acquire(n)
+        got[n] = np.concatenate([m.step(slot, toks[p:p + n], [n - 1], layers=True)[1] for p in range(0, 6, n)], 1)
+        m.pool.release(n)
+    m.close()
+    assert np.isinf(got[1]).any()
+    for same in (np.isposinf, np.isneginf, np.isnan):
+        assert (same(got[1]) == same(got[3])).all()
