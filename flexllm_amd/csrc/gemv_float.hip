@@ -416,6 +416,7 @@ static int gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
 // waves share its stretch of k (KW steps of 32 each), whose vectors lie in LDS as [part][token][stretch, padded by 16 bytes: the
 // tokens of an operand read are then on different banks], and meet through LDS per tile, two tiles' weights in flight.
 constexpr int kMfmaTokens = 16, kMfmaWaves = 8;
+constexpr float kBf16Max = 3.38953139e38f;
 constexpr int gemv_mfma_row(int stretch) { return stretch * 2 + 16; }      // bytes of a token's part
 template <int KW>
 __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, int tokens, int group) {
@@ -440,8 +441,11 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
             bf16x4 b;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                b[e] = (bf16_t)v[e];
-                v[e] = isinf(v[e]) ? 0.0f : v[e] - (float)b[e];     // an infinity has no rest
+                // what is beyond the largest bfloat16 lies in the rest (a part that rounds to infinity would leave infinity
+                // less infinity); an infinity has no rest
+                const bool finite = isfinite(v[e]);
+                b[e] = (bf16_t)(finite ? fminf(fmaxf(v[e], -kBf16Max), kBf16Max) : v[e]);
+                v[e] = finite ? v[e] - (float)b[e] : 0.0f;
             }
             *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
         }
@@ -717,3 +721,22 @@ int moe_plan(const float* route, int ld_route, int rows, int experts, int top, i
 }
 
 }  // namespace fx
+
+using namespace fx;
+
+extern "C" {
+
+int flexllm_linear_float_step(const float* x, const void* w, const float* bias, float* y, float* y32, int tokens, int k, int n, int n_split, int glu, float limit,
+                              int parts, int dtype, void* stream) {
+    FX_REQUIRE((dtype == 0 || dtype == 1) && glu >= 0 && glu <= 1 + FLEXLLM_GLU_GELU, "linear_float_step: dtype=%d glu=%d", dtype, glu);
+    FX_REQUIRE(tokens > 0 && tokens <= 8 && k > 0 && n > 0 && n_split >= 0 && n_split <= n && (n_split == 0 || y) && (n_split == n || y32) && (!glu || n_split % 2 == 0),
+               "linear_float_step: tokens=%d k=%d n=%d n_split=%d", tokens, k, n, n_split);
+    FX_REQUIRE(parts >= 1 && parts <= 8 && (size_t)x % 16 == 0 && (size_t)w % 16 == 0, "linear_float_step: %d parts, or an operand off 16 bytes", parts);
+    GemvArgs g;
+    g.w = w; g.n = n; g.k = k; g.kpad = pad_k(k); g.x = x; g.ldx = k; g.bias = bias;
+    g.out = y; g.ldo = glu ? n_split / 2 : n_split; g.out32 = y32; g.ldo32 = n - n_split; g.n_split = n_split; g.glu = glu; g.limit = limit;
+    g.parts = parts; g.part_stride = (size_t)tokens * n;
+    return dtype == 0 ? gemv_float<bf16_t>(g, 0, tokens, as_stream(stream)) : gemv_float<float>(g, 0, tokens, as_stream(stream));
+}
+
+}  // extern "C"

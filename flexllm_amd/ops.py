@@ -433,3 +433,18 @@ def linear_float(a, w, n_split=None, glu=0, limit=0.0, bias=None, stream=None):
     check(lib().flexllm_linear_float_gemm(_p(a), _p(w), _p(bias), _p(y), _p(y32), m, k, n, n_split, int(glu), C.c_float(limit),
                                           int(a.dtype == np.float32), _s(stream)))
     return y, y32
+
+
+def linear_float_step(x, w, n_split=None, glu=0, limit=0.0, bias=None, parts=1, stream=None):
+    """linear_float for the 1 to 8 tokens of a step: x float32 [tokens][k], w [n][k rounded up to 64] with zeros behind k; both
+    outputs are float32.  parts > 1 (n_split 0, no bias, bfloat16 weights): the second output is [parts][tokens][n], to be summed."""
+    tokens, k = x.shape
+    n, kpad = w.shape
+    if kpad != (k + 63) // 64 * 64:
+        raise ValueError("linear_float_step: rows of %d for %d columns" % (kpad, k))
+    n_split = n if n_split is None else n_split
+    y = DeviceArray((tokens, n_split // 2 if glu else n_split), np.float32) if n_split else None
+    y32 = DeviceArray((parts, tokens, n) if parts > 1 else (tokens, n - n_split), np.float32) if n_split < n else None
+    check(lib().flexllm_linear_float_step(_p(x), _p(w), _p(bias), _p(y), _p(y32), tokens, k, n, n_split, int(glu), C.c_float(limit), int(parts),
+                                          int(w.dtype == np.float32), _s(stream)))
+    return y, y32

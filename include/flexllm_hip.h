@@ -596,6 +596,11 @@ int flexllm_hybrid_check(flexllm_hybrid* m);
  * bias [n] or NULL is added first; glu: 0, or 1 + FLEXLLM_GLU_*. */
 int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, void* y, float* y32, int m, int k, int n, int n_split, int glu, float limit,
                               int dtype, void* stream);
+/* The linear behind the steps of a few tokens (1 to 8) on its own: x float32 [tokens][k], w [n][k rounded up to 64] of the
+ * element type, zeros behind a row's k; both 16-byte aligned.  Outputs as above, all float32.  With n_split 0 and no bias a
+ * bfloat16 product of several tokens may be asked for in `parts` sums over k, which leave y32 as [parts][tokens][n]. */
+int flexllm_linear_float_step(const float* x, const void* w, const float* bias, float* y, float* y32, int tokens, int k, int n, int n_split, int glu, float limit,
+                              int parts, int dtype, void* stream);
 int flexllm_rt_fill_uniform_bf16(uint16_t* dst, size_t n, uint64_t seed, float lo, float hi, void* stream);
 
 #ifdef __cplusplus
