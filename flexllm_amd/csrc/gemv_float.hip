@@ -466,6 +466,21 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
     if (walker + walkers < tiles) load(1, walker + walkers);
     __syncthreads();
     const int8_t* xl = xp + min(lane & 15, nt - 1) * ROW + wk * 2;
+    // Not a number may be of the parts' own making, where an infinite weight meets parts of zero or of both signs: the same sum with
+    // a float32 product per weight has the right of it.
+    auto whole = [&](int row, int j) __attribute__((always_inline)) {
+        const bf16_t* wr = static_cast<const bf16_t*>(g.w) + (size_t)row * g.kpad + k0;
+        float s = 0.0f;
+        for (int c = 0; c < min(STRETCH, g.kpad - k0); c += 8) {
+            const bf16x8 u = *reinterpret_cast<const bf16x8*>(wr + c);
+            bf16x8 b[3];
+#pragma unroll
+            for (int p = 0; p < 3; p++) b[p] = *reinterpret_cast<const bf16x8*>(xp + (p * group + j) * ROW + c * 2);
+#pragma unroll
+            for (int e = 0; e < 8; e++) s = fma_f((float)u[e], (float)b[0][e] + ((float)b[1][e] + (float)b[2][e]), s);
+        }
+        return s;
+    };
     auto process = [&](int b, int tile) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -483,7 +498,8 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
                 float v[kMfmaWaves];
 #pragma unroll
                 for (int q = 0; q < kMfmaWaves; q++) v[q] = p[q * 16 * 17];
-                const float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+                float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+                if (isnan(s)) s = whole(min(row + i, g.n - 1), j);
                 return g.bias ? s + g.bias[min(row + i, g.n - 1)] : s;
             };
             if (row >= g.n_split) g.out32[part * g.part_stride + (size_t)tok * g.ldo32 + row - g.n_split] = total(0);

@@ -35,3 +35,23 @@ def test_values_beyond_bfloat16(k, tokens, dtype):
     w = lc.round_bf16(r.uniform(0.5, 1.0, (37, k)) * 2.0 ** -20)
     x[:, [0, 7, k // 2, k - 1]] = [3.4e38, -3.3962e38, np.finfo(np.float32).max, -3.39e38]
     near(step(x, w, dtype)[0], x, w)
+
+
+@BOTH
+@pytest.mark.parametrize("tokens", [1, 2, 3, 8])
+@pytest.mark.parametrize("k", [100, 2048, 2112, 8200])
+def test_infinite_weights(k, tokens, dtype):
+    """An infinite weight gives infinities of the sign that the products have, whichever bits the vector has set; not a number only
+    where it meets zero or infinities of both signs meet."""
+    r = np.random.default_rng(k + tokens)
+    x = (r.standard_normal((tokens, k)) + 0.1).astype(np.float32)
+    w = lc.round_bf16(r.standard_normal((37, k)))
+    x[:, :4] = [1.0, -1.5, 1.0 + 2.0 ** -9 - 2.0 ** -20, 0.0]        # nothing behind the first bfloat16, the same below zero, parts of both signs
+    w[2, 0], w[3, 1], w[5, 2], w[16, k - 1], w[17, 3], w[36, [0, 1]] = np.inf, np.inf, -np.inf, -np.inf, np.inf, np.inf
+    with np.errstate(invalid="ignore"):
+        want = (x[:, None, :].astype(np.float64) * w[None].astype(np.float64)).sum(-1)
+    got = step(x, w, dtype)[0]
+    for same in (np.isposinf, np.isneginf, np.isnan):
+        assert (same(got) == same(want)).all()
+    rows = np.isfinite(want[0])
+    near(got[:, rows], x, w[rows])
