@@ -68,7 +68,7 @@ __device__ __forceinline__ void route_wave(const float* __restrict__ z, int expe
 template <typename ET, int R, int S, int PRO, bool VEC, bool NT>
 __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
     constexpr int CE = Chunk<ET>::N;
-    extern __shared__ __attribute__((aligned(16))) float xs[];     // [kpad] the vector
+    extern __shared__ __attribute__((aligned(16))) float xs[];     // [kpad] the vector, and a piece of zeros for threads without one
     __shared__ float red[2][4 * R];
     __shared__ float nred[4];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -127,6 +127,7 @@ __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
     load(0, g0);
     if (g0 + G < ng) load(1, g0 + G);
     __builtin_amdgcn_sched_barrier(0);
+    if (t < CE) xs[g.kpad + t] = 0.0f;
     // ---- the vector
     if constexpr (PRO == 1 && VEC) {
         float rs = 0.0f;
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(256) void gemv_float_kernel(GemvArgs g) {
         for (int r = 0; r < R; r++) acc[r] = 0.0f;
 #pragma unroll
         for (int s = 0; s < S; s++) {
-            const int c = min(s * 256 + t, nchunk - 1);   // pieces beyond the row were filled with zeros
+            const int c = min(s * 256 + t, nchunk);       // pieces beyond the row meet the zeros
 #pragma unroll
             for (int r = 0; r < R; r++) dot(c, buf[b][r][s], acc[r]);
         }
@@ -260,7 +261,7 @@ static int launch_gemv_rs(const GemvArgs& g, int pro, int tokens, hipStream_t st
     if (wgs < 128) wgs = 128;
     const int ng = (g.n + R - 1) / R;
     const dim3 grid(ng < wgs ? ng : wgs, rows_y);
-    const size_t lds = (size_t)g.kpad * sizeof(float);
+    const size_t lds = (size_t)(g.kpad + Chunk<ET>::N) * sizeof(float);
     const bool vec = g.k % 4 == 0 && g.ldx % 4 == 0 && g.ldy % 4 == 0 && g.ldh % 4 == 0 && g.kpad <= 256 * Chunk<ET>::N * S;
 #define FX_GEMV(PRO)                                                                               \
     do {                                                                                           \
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens
     constexpr int CE = Chunk<ET>::N, PL = CE / 4;
     constexpr int SUMS = R * TT <= 4 ? 4 : R * TT <= 8 ? 8 : R * TT <= 16 ? 16 : 32;
     static_assert(R * TT <= 32, "sums per lane");
-    extern __shared__ __attribute__((aligned(16))) float xs[];     // [TT][PL][nchunk][4]
+    extern __shared__ __attribute__((aligned(16))) float xs[];     // [TT][PL][nchunk + 1][4], the last piece zeros for threads without one
     __shared__ float red[2][4 * SUMS];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, tok0 = blockIdx.y * TT;
     const ET* w = static_cast<const ET*>(g.w);
@@ -304,9 +305,10 @@ __global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens
 #pragma unroll
                 for (int e = 0; e < 4; e++) v[e] = 4 * c + e < g.k ? x[4 * c + e] : 0.0f;
             }
-            *reinterpret_cast<f32x4*>(xs + ((size_t)(j * PL + c % PL) * nchunk + c / PL) * 4) = v;
+            *reinterpret_cast<f32x4*>(xs + ((size_t)(j * PL + c % PL) * (nchunk + 1) + c / PL) * 4) = v;
         }
     }
+    if (t < TT * PL) *reinterpret_cast<f32x4*>(xs + ((size_t)t * (nchunk + 1) + nchunk) * 4) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     i32x4 buf[2][R][S];
     auto piece = [&](int row, int c) { return *reinterpret_cast<const i32x4*>(w + (size_t)min(row, g.n - 1) * g.kpad + c * CE); };
     auto load = [&](int b, int grp) {
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens
         for (int j = 0; j < TT; j++)
 #pragma unroll
             for (int q = 0; q < PL; q++) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(xs + ((j * PL + q) * nchunk + c) * 4);
+                const f32x4 v = *reinterpret_cast<const f32x4*>(xs + ((j * PL + q) * (nchunk + 1) + c) * 4);
 #pragma unroll
                 for (int r = 0; r < R; r++)
 #pragma unroll
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens
 #pragma unroll
         for (int i = 0; i < SUMS; i++) acc[i] = 0.0f;
 #pragma unroll
-        for (int s = 0; s < S; s++) take(buf[b], s, min(s * 256 + t, nchunk - 1), acc);     // pieces beyond the row were filled with zeros
+        for (int s = 0; s < S; s++) take(buf[b], s, min(s * 256 + t, nchunk), acc);     // pieces beyond the row meet the zeros
         for (int c = S * 256 + t; c < nchunk; c += 256) {
             i32x4 more[R][S];
 #pragma unroll
@@ -377,13 +379,13 @@ __global__ __launch_bounds__(256) void gemv_tokens_kernel(GemvArgs g, int tokens
 
 template <typename ET, int TT, int R, int S>
 static int launch_gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
-    const size_t lds = (size_t)TT * g.kpad * sizeof(float);
+    const size_t lds = (size_t)TT * (g.kpad + Chunk<ET>::N) * sizeof(float);
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
         FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_tokens_kernel<ET, TT, R, S>), hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTokensLds));
         opted_in.store(true, std::memory_order_release);
     }
-    const int groups = (tokens + TT - 1) / TT, per_cu = lds <= 36 * 1024 ? 4 : lds <= 72 * 1024 ? 2 : 1, ng = (g.n + R - 1) / R;
+    const int groups = (tokens + TT - 1) / TT, per_cu = lds <= 37 * 1024 ? 4 : lds <= 73 * 1024 ? 2 : 1, ng = (g.n + R - 1) / R;
     const int wgs = 256 * per_cu / groups;                // what is resident at a time
     gemv_tokens_kernel<ET, TT, R, S><<<dim3(ng < wgs ? ng : wgs, groups), 256, lds, st>>>(g, tokens);
     FX_LAUNCH_CHECK();
@@ -393,7 +395,7 @@ static int launch_gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
 // R x S pieces per thread and group as for one token, TT as many tokens as LDS holds.
 template <typename ET, int R, int S>
 static int gemv_tokens_rs(const GemvArgs& g, int tokens, hipStream_t st) {
-    const int fit = (int)(kGemvTokensLds / (g.kpad * sizeof(float))), most = fit < 32 / R ? fit : 32 / R;
+    const int fit = (int)(kGemvTokensLds / ((g.kpad + Chunk<ET>::N) * sizeof(float))), most = fit < 32 / R ? fit : 32 / R;
     const int cap = most >= 8 ? 8 : most >= 6 ? 6 : most >= 4 ? 4 : 2, groups = (tokens + cap - 1) / cap, tt = (tokens + groups - 1) / groups;
     if constexpr (R <= 4) if (tt > 6) return launch_gemv_tokens<ET, 8, R, S>(g, tokens, st);
     if (tt > 4) return launch_gemv_tokens<ET, 6, R, S>(g, tokens, st);

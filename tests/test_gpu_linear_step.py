@@ -55,3 +55,15 @@ def test_infinite_weights(k, tokens, dtype):
         assert (same(got) == same(want)).all()
     rows = np.isfinite(want[0])
     near(got[:, rows], x, w[rows])
+
+
+@BOTH
+@pytest.mark.parametrize("tokens", [1, 2, 3, 8])
+@pytest.mark.parametrize("k", [64, 192, 2048, 2112, 4160, 8192, 8256])
+def test_infinity_in_the_last_piece(k, tokens, dtype):
+    """Threads that have no piece of a row add nothing, whatever the vector's last piece holds."""
+    r = np.random.default_rng(k + tokens)
+    x = r.standard_normal((tokens, k)).astype(np.float32)
+    w = lc.round_bf16(r.standard_normal((37, k)))
+    x[:, k - 1] = np.inf
+    assert np.array_equal(step(x, w, dtype)[0], np.broadcast_to(np.inf * w[:, k - 1], (tokens, 37)))
