@@ -414,6 +414,10 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
 #pragma unroll
                 for (int n = j; n < j + 8; n++) v = fma_f(u[n], wsp[h * kKvSplits + n], v);      // weight 0 beyond the last split
             }
+            if (isnan(v)) {                               // an infinite sum of the last split is not nothing at weight 0: the splits alone
+                v = 0.0f;
+                for (int n = 0; n < ns; n++) v = fma_f(load_past(split_at(h, n) + e), wsp[h * kKvSplits + n], v);
+            }
         }
         const size_t out = (size_t)tok * ldo + (size_t)(head0 + h) * d.dim + e;
         if (o_f32) static_cast<float*>(o)[out] = v;

@@ -162,3 +162,20 @@ def test_infinite_units(ff, dtype):
     assert np.isinf(got[1]).any()
     for same in (np.isposinf, np.isneginf, np.isnan):
         assert (same(got[1]) == same(got[3])).all()
+
+
+# the last split of the rows repeats in the join of fewer splits than it reads at a time
+@BOTH
+@pytest.mark.parametrize("rows", [40, 96, 200, 256, 270])
+def test_infinite_sums_of_the_splits(rows, dtype):
+    """Rows so large that their sum leaves float32 give an infinity in that column, of any number of splits."""
+    from flexllm_amd.lopazen import Lopazen
+    cfg = lc.config([lc.layer(heads=1, kv_heads=1, dim=8)])
+    w, toks = lc.weights(cfg, 11), lc.tokens(cfg, rows + 1)
+    w["l0.mix.k.b"][3], w["l0.mix.q.norm"][3] = 2.0 ** 126, 0.0      # this column is in no score
+    m = Lopazen.from_tensors(cfg, w, dtype=dtype, max_pos=512)
+    slot = m.pool.acquire("t")
+    m.step(slot, toks[:rows])
+    got = m.step(slot, toks[rows:], layers=True)[1][0, 0]
+    m.close()
+    assert np.array_equal(got, np.where(w["l0.mix.o"][:, 3] < 0, -np.inf, np.inf))
