@@ -547,7 +547,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
     }
 }
 
-template <int BM, int BN, int EPI, int STAGES = 3, int WPE = 1, int BKB = 64, int NW = 4>
+template <int BM, int BN, int EPI, int STAGES, int WPE, int BKB, int NW = 4>
 inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s,
                            const float* residual, float* y, int m, int k, int n, hipStream_t st, QkvEpiArgs qa = QkvEpiArgs()) {
     static std::atomic<bool> opted_in{false};             // more than the default 64 KiB of LDS per workgroup
@@ -562,31 +562,49 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
     return FLEXLLM_OK;
 }
 
-// The direct-load kernel on the tile whose rounds over the 256 CUs (a workgroup per CU) cost least, in 0.01 us: per stage of 128 k,
-// and once per round for what lies around them (first loads, epilogue).  From products of 2048 and 8192 k where all CUs are
-// busy.  Measured against the fixed choices before (us): 512 x 16384 x 2048 43.8 -> 24.8 (128 x 256), 2048 x 2048 x 8192 62.7 -> 45.8
+// The direct-load kernel runs on the tile whose rounds over the 256 CUs (a workgroup per CU) cost least, in 0.01 us: per stage, and
+// once per round for what lies around them (first loads, epilogue).  From products of 2048 and 8192 k (whole 128-byte lines per row
+// and stage) and of 2112 and 8256 k (a multiple of 64 only: 64-byte rows) where all CUs are busy.
+// 128-byte rows, measured against the fixed choices before (us): 512 x 16384 x 2048 43.8 -> 24.8 (128 x 256), 2048 x 2048 x 8192 62.7 -> 45.8
 // (128 x 128), 2528 x 2048 x 8192 85.1 -> 65.1 (128 x 256), 1536 x 2048 x 8192 53.4 -> 41.3 (128 x 128), 4096 x 2048 x 8192 91.0 -> 80.4
 // (128 x 256), 1024 x 2048 x 2048 12.1 -> 11.3 (64 x 128); 1024 x 16384 x 2048 stays on 256 x 256, 41.5.
+// 64-byte rows, against 64 x 64 everywhere (us): 1024 x 8192 x 2112 41.6 -> 25.3 (128 x 256), 1024 x 16384 x 2112 85.2 -> 40.3 and
+// 4096 x 16384 x 2112 427 -> 192 (256 x 256), 1024 x 2048 x 8256 42.1 -> 32.3 (64 x 128), 2048 x 2048 x 8256 95.9 -> 47.6 (128 x 128).
+struct GemmI8Tile { int bm, bn, stage, round; };
+constexpr GemmI8Tile kGemmI8Tiles[2][5] = {{{256, 256, 180, 1200}, {128, 256, 95, 950}, {128, 128, 65, 520}, {64, 128, 41, 220}, {64, 64, 35, 300}},
+                                           {{256, 256, 88, 1120}, {128, 256, 61, 500}, {128, 128, 32, 580}, {64, 128, 22, 400}, {64, 64, 17, 350}}};
+inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
+    const bool half = k % 128 != 0;
+    long best = 0;
+    int pick = -1;
+    for (int i = qkv ? 1 : 0; i < 5; i++) {                    // the q/k/v epilogue's tile has to fit in LDS
+        const GemmI8Tile& t = kGemmI8Tiles[half][i];
+        const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), cost = (wgs + 255) / 256 * (t.stage * (k / (half ? 64 : 128)) + t.round);
+        if (pick < 0 || cost < best) { best = cost; pick = i; }
+    }
+    return pick;
+}
+
 template <int EPI>
 inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s, const float* residual, float* y,
                              int m, int k, int n, hipStream_t st, QkvEpiArgs qa = QkvEpiArgs()) {
-    // whole 128-byte lines per row and stage where k allows
-    if (k % 128 != 0) return launch_gemm_dma<64, 64, EPI>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
-    struct Tile { int bm, bn, stage, round; };
-    constexpr Tile tiles[] = {{256, 256, 180, 1200}, {128, 256, 95, 950}, {128, 128, 65, 520}, {64, 128, 41, 220}, {64, 64, 35, 300}};
-    long best = 0;
-    int pick = -1;
-    for (int i = EPI == kDmaQkv ? 1 : 0; i < 5; i++) {         // the q/k/v epilogue's tile has to fit in LDS
-        const Tile& t = tiles[i];
-        const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), cost = (wgs + 255) / 256 * (t.stage * (k / 128) + t.round);
-        if (pick < 0 || cost < best) { best = cost; pick = i; }
+    const int pick = gemm_i8_tile(m, k, n, EPI == kDmaQkv);
+#define FX_GEMM_TILE(BM, BN, ...) launch_gemm_dma<BM, BN, EPI, __VA_ARGS__>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa)
+    if (k % 128 != 0) {
+        if constexpr (EPI != kDmaQkv)
+            if (pick == 0) return FX_GEMM_TILE(256, 256, 4, 2, 64, 8);
+        if (pick == 1) return FX_GEMM_TILE(128, 256, 4, 2, 64, 8);
+        if (pick == 2) return FX_GEMM_TILE(128, 128, 4, 2, 64, 8);
+        if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 64);
+        return FX_GEMM_TILE(64, 64, 4, 2, 64);
     }
     if constexpr (EPI != kDmaQkv)
-        if (pick == 0) return launch_gemm_dma<256, 256, EPI, 2, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (pick == 1) return launch_gemm_dma<128, 256, EPI, 3, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (pick == 2) return launch_gemm_dma<128, 128, EPI, 4, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
-    if (pick == 3) return launch_gemm_dma<64, 128, EPI, 4, 2, 128, 8>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
-    return launch_gemm_dma<64, 64, EPI, 4, 2, 128>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+        if (pick == 0) return FX_GEMM_TILE(256, 256, 2, 2, 128, 8);
+    if (pick == 1) return FX_GEMM_TILE(128, 256, 3, 2, 128, 8);
+    if (pick == 2) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
+    if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 128, 8);
+    return FX_GEMM_TILE(64, 64, 4, 2, 128);
+#undef FX_GEMM_TILE
 }
 
 template <int EPI>

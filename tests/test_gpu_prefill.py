@@ -109,10 +109,10 @@ def test_gemm_swiglu(fx, oracle, m, k, n):
 
 
 @pytest.mark.parametrize("m,qh,kvh,pos0", [(128, 32, 8, 0), (96, 8, 2, 64), (32, 4, 4, 0), (1024, 32, 8, 0)])
-def test_gemm_qkv_rope_cache_fused(fx, oracle, m, qh, kvh, pos0):
+def test_gemm_qkv_rope_cache_fused(fx, oracle, m, qh, kvh, pos0, k=2048):
     """q/k/v GEMM with RoPE + static quantisation + cache stores in the epilogue: int8 outputs bit-exact against the
     oracle's chain (linear -> dequant -> RoPE -> static quant) and against the unfused device entry points."""
-    k, max_pos = 2048, 1280
+    max_pos = 1280
     n = (qh + 2 * kvh) * 64
     x = rng.standard_normal((m, k)).astype(np.float32)
     w = rng.integers(-127, 128, (n, k)).astype(np.int8)
