@@ -19,7 +19,8 @@ struct GemmTile { int row0, row_end, group; };
 
 // Which tile this workgroup works on: row tiles fastest inside a range of weight columns per XCD, as in gemm_i8_kernel.
 template <int BM, int BN>
-__device__ __forceinline__ bool gemm_pick_tile(const GemmArgs& g, int tiles_m, int tiles_n, int tile, GemmTile& t, int& col0) {
+__device__ __forceinline__ bool gemm_pick_tile(const GemmArgs& g, int tiles_m, int tiles_n, GemmTile& t, int& col0) {
+    const int tile = blockIdx.x;
     int tm, tn;
     if ((tiles_n & 7) == 0) {
         const int xcd = tile & 7, idx = tile >> 3;
@@ -123,8 +124,10 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
 
     GemmTile tl;
     int col0;
-    const int part = blockIdx.x / (tiles_m * tiles_n), stages = g.k * (int)sizeof(ET) / BKB, k0 = part * stages / g.parts;
-    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, blockIdx.x - part * (tiles_m * tiles_n), tl, col0)) return;
+    // scalar registers for the ends of the part: divisions are made in vector ones, and the loop would carry them along
+    const int part = blockIdx.y, stages = g.k * (int)sizeof(ET) / BKB;
+    const int k0 = __builtin_amdgcn_readfirstlane(part * stages / g.parts);
+    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, tl, col0)) return;
     g.y32 += part * g.part_stride;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
-    const int nk = (part + 1) * stages / g.parts - k0;
+    const int nk = __builtin_amdgcn_readfirstlane((part + 1) * stages / g.parts) - k0;
     constexpr int PER = A_INSTR + B_INSTR;
     // everything the compiler loaded itself (tile table, gathered row numbers) has to be in before the counted loads start
     gemm_wait_vmcnt<0>();
@@ -211,17 +214,18 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
     wait_stage(0);
     __syncthreads();
     read_frags(0, 0, fa0, fb0);
-    for (int kt = 0; kt < nk; kt++) {
+    // The last stage stands by itself, a branch less in the loop: 2 x 72 x 9024, one tile of 141 stages, 36.7 -> 31.0 us.
+    auto stage = [&](int kt, auto more) __attribute__((always_inline)) {
 #pragma unroll
         for (int ks = 0; ks < KS; ks += 2) {
             read_frags(kt, ks + 1, fa1, fb1);
-            if (ks == 0 && kt + STAGES - 1 < nk) issue_stage(kt + STAGES - 1);
+            if (more && ks == 0 && kt + STAGES - 1 < nk) issue_stage(kt + STAGES - 1);
             __builtin_amdgcn_sched_barrier(0);
             mma(fa0, fb0);
             __builtin_amdgcn_sched_barrier(0);
             if (ks + 2 < KS) {
                 read_frags(kt, ks + 2, fa0, fb0);
-            } else if (kt + 1 < nk) {
+            } else if (more) {
                 wait_stage(kt + 1);
                 __syncthreads();
                 read_frags(kt + 1, 0, fa0, fb0);
@@ -230,7 +234,9 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g
             mma(fa1, fb1);
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
+    };
+    for (int kt = 0; kt < nk - 1; kt++) stage(kt, std::true_type());
+    stage(nk - 1, std::false_type());
     __syncthreads();
     gemm_epilogue<ET, TM, TN>(g, tl, col0, wm, wn, lane, reinterpret_cast<float*>(gemm_smem) + wave * (32 * 36), acc);
 }
@@ -250,7 +256,7 @@ static int launch_dma(const GemmArgs& g, hipStream_t st) {
         opted_in.store(true, std::memory_order_release);
     }
     const int tm = g.tiles ? g.max_tiles : (g.m + BM - 1) / BM, tn = (g.n + BN - 1) / BN;
-    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<tm * tn * g.parts, NW * 64, lds, st>>>(g, tm, tn);
+    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<dim3(tm * tn, g.parts), NW * 64, lds, st>>>(g, tm, tn);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
