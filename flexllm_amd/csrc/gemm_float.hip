@@ -109,7 +109,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const GemmTile&
 
 // A stage is 128 bytes of k of the tile's rows and columns; STAGES of them form the ring in LDS.
 // What bounds it: with one workgroup per CU the trip of a stage's bytes, so that everything LDS holds is in flight (two stages of
-// 128 x 128 in four waves, two workgroups per CU: 213 us for 777 x 4096 x 14336; four stages, eight waves: 117 us), and for the
+// 128 x 128 in four waves, of which a CU could hold two: 213 us for 777 x 4096 x 14336, 224 tiles; four stages, eight waves: 117 us), and for the
 // largest tile LDS itself, which hands out 6 KiB of operands for 8 matrix instructions per wave.
 template <typename ET, int BM, int BN, int STAGES, int WPE, int NW>
 __global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g, int tiles_m, int tiles_n) {
@@ -305,25 +305,30 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
     return FLEXLLM_OK;
 }
 
-// The tile whose rounds over the chip (a workgroup per CU) take the least time; cost: of a round of one stage, in 0.01 us, as
-// measured where all CUs are busy.
+// The tile whose rounds over the chip take the least time.  cost: of one stage of a round, and `round` once per round, in 0.01 us, as
+// measured where all CUs are busy; per_cu: workgroups that a CU holds at a time.  (A fit over 300 sizes from 1 to 5000 rows gives a
+// constant per round to the 64 x 128 tiles only; the tiles picked are within 1 % of the best ones on average.)
 //
 // bfloat16 (64 k): 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3
 // rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048
-// 64 x 128 (14.8 us; 128 x 128: 19.4 us).
+// 64 x 128 (14.4 us; 128 x 128: 19.4 us).  128 x 128 in four waves with two stages fits twice into a CU: 3700 x 2064 x 8576, 493 tiles,
+// takes one round of it (130 us; two rounds of the one with four stages: 181 us).
 // float32 (32 k): 333 x 16384 x 2048 takes 64 x 128 (251 us; 64 x 64: 265, 128 x 128: 289 us), 333 x 2048 x 8192 64 x 64 (173 us; 64 x 128:
 // 276 us), 2048 x 4096 x 4096 128 x 128 (602 us, 114 TFLOP/s; 64 x 64: 656 us).
-struct GemmTileCost { int bm, bn, cost; };
+struct GemmTileCost { int bm, bn, cost, round, per_cu; };
 template <typename ET> struct GemmTiles;
-template <> struct GemmTiles<bf16_t> { static constexpr GemmTileCost list[] = {{256, 256, 210}, {128, 256, 110}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}}; };
-template <> struct GemmTiles<float> { static constexpr GemmTileCost list[] = {{128, 128, 235}, {64, 128, 126}, {64, 64, 66}}; };
+template <> struct GemmTiles<bf16_t> {
+    static constexpr GemmTileCost list[] = {{256, 256, 200, 0, 1}, {128, 256, 110, 0, 1}, {128, 128, 64, 0, 1}, {64, 128, 42, 100, 1}, {64, 64, 28, 0, 1}, {128, 128, 113, 0, 2}};
+};
+template <> struct GemmTiles<float> { static constexpr GemmTileCost list[] = {{128, 128, 235, 0, 1}, {64, 128, 126, 100, 1}, {64, 64, 66, 0, 1}}; };
 
 template <typename ET>
 static int gemm_cheapest_tile(const GemmArgs& g, int parts, long& best) {
     const long stages = (long)g.k * sizeof(ET) / 128;
     int pick = -1, i = 0;
     for (const GemmTileCost& t : GemmTiles<ET>::list) {
-        const long n = (long)((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn) * parts, cost = (n + 255) / 256 * t.cost * ((stages + parts - 1) / parts);
+        const long n = (long)((g.m + t.bm - 1) / t.bm) * ((g.n + t.bn - 1) / t.bn) * parts, slots = 256 * t.per_cu;
+        const long cost = (n + slots - 1) / slots * (t.cost * ((stages + parts - 1) / parts) + t.round);
         if (pick < 0 || cost < best) { best = cost; pick = i; }
         i++;
     }
@@ -366,7 +371,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         case 1: return launch_dma<bf16_t, 128, 256, 3, 2, 8>(g, st);
         case 2: return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
         case 3: return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
-        default: return launch_dma<bf16_t, 64, 64, 4, 2, 4>(g, st);
+        case 4: return launch_dma<bf16_t, 64, 64, 4, 2, 4>(g, st);
+        default: return launch_dma<bf16_t, 128, 128, 2, 2, 4>(g, st);
     }
 }
 
@@ -428,6 +434,18 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
     g.a = a; g.w = w; g.lda = k; g.m = m; g.n = n; g.k = k; g.n_split = n_split; g.glu = glu; g.limit = limit; g.bias = bias;
     g.y = y; g.ldy = glu ? n_split / 2 : n_split; g.y32 = y32; g.ldy32 = n - n_split;
     return dtype == 0 ? gemm_float<bf16_t>(g, as_stream(stream)) : gemm_float<float>(g, as_stream(stream));
+}
+
+int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu) {
+    FX_REQUIRE((dtype == 0 || dtype == 1) && m > 0 && n > 0 && k > 0 && k % kKPad == 0 && rows && cols && per_cu, "linear_float_gemm_tile: m=%d k=%d n=%d dtype=%d", m, k, n, dtype);
+    GemmArgs g;
+    g.m = m; g.k = k; g.n = n;
+    long cost;
+    const GemmTileCost& t = dtype == 0 ? GemmTiles<bf16_t>::list[gemm_cheapest_tile<bf16_t>(g, 1, cost)] : GemmTiles<float>::list[gemm_cheapest_tile<float>(g, 1, cost)];
+    *rows = t.bm;
+    *cols = t.bn;
+    *per_cu = t.per_cu;
+    return FLEXLLM_OK;
 }
 
 }  // extern "C"

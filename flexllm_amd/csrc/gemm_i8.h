@@ -570,16 +570,22 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
 // (128 x 256), 1024 x 2048 x 2048 12.1 -> 11.3 (64 x 128); 1024 x 16384 x 2048 stays on 256 x 256, 41.5.
 // 64-byte rows, against 64 x 64 everywhere (us): 1024 x 8192 x 2112 41.6 -> 25.3 (128 x 256), 1024 x 16384 x 2112 85.2 -> 40.3 and
 // 4096 x 16384 x 2112 427 -> 192 (256 x 256), 1024 x 2048 x 8256 42.1 -> 32.3 (64 x 128), 2048 x 2048 x 8256 95.9 -> 47.6 (128 x 128).
-struct GemmI8Tile { int bm, bn, stage, round; };
-constexpr GemmI8Tile kGemmI8Tiles[2][5] = {{{256, 256, 180, 1200}, {128, 256, 95, 950}, {128, 128, 65, 520}, {64, 128, 41, 220}, {64, 64, 35, 300}},
-                                           {{256, 256, 88, 1120}, {128, 256, 61, 500}, {128, 128, 32, 580}, {64, 128, 22, 400}, {64, 64, 17, 350}}};
+// Outputs that a short k hardly fills are bound by their stores, which is what the costs per round were set by: 731 x 27176 x 128
+// 28.8 us on 64 x 128, 23.0 on 128 x 128; 917 x 19348 x 704 40.7 us on 128 x 256, 29.8 on 128 x 128.
+// 128 x 128 in four waves with two stages fits twice into a CU (per_cu): 3700 x 2064 x 8576, 493 tiles, 74.6 us in one round of it, 86.2 in
+// two of the one with four stages.
+struct GemmI8Tile { int bm, bn, stage, round, per_cu; };
+constexpr GemmI8Tile kGemmI8Tiles[2][6] = {
+    {{256, 256, 180, 1200, 1}, {128, 256, 95, 950, 1}, {128, 128, 65, 470, 1}, {64, 128, 41, 320, 1}, {64, 64, 35, 200, 1}, {128, 128, 113, 900, 2}},
+    {{256, 256, 88, 1120, 1}, {128, 256, 61, 650, 1}, {128, 128, 32, 440, 1}, {64, 128, 22, 400, 1}, {64, 64, 17, 350, 1}, {}}};
 inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
     const bool half = k % 128 != 0;
     long best = 0;
     int pick = -1;
-    for (int i = qkv ? 1 : 0; i < 5; i++) {                    // the q/k/v epilogue's tile has to fit in LDS
+    for (int i = qkv ? 1 : 0; i < (half || qkv ? 5 : 6); i++) {     // the q/k/v epilogue's tile has to fit in LDS, with per_cu of them
         const GemmI8Tile& t = kGemmI8Tiles[half][i];
-        const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), cost = (wgs + 255) / 256 * (t.stage * (k / (half ? 64 : 128)) + t.round);
+        const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), slots = 256 * t.per_cu;
+        const long cost = (wgs + slots - 1) / slots * (t.stage * (k / (half ? 64 : 128)) + t.round);
         if (pick < 0 || cost < best) { best = cost; pick = i; }
     }
     return pick;
@@ -598,8 +604,10 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
         if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 64);
         return FX_GEMM_TILE(64, 64, 4, 2, 64);
     }
-    if constexpr (EPI != kDmaQkv)
+    if constexpr (EPI != kDmaQkv) {
         if (pick == 0) return FX_GEMM_TILE(256, 256, 2, 2, 128, 8);
+        if (pick == 5) return FX_GEMM_TILE(128, 128, 2, 2, 128);
+    }
     if (pick == 1) return FX_GEMM_TILE(128, 256, 3, 2, 128, 8);
     if (pick == 2) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
     if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 128, 8);

@@ -48,11 +48,12 @@ int flexllm_linear_i8_gemm_qkv_rope_cache(const int8_t* a, const float* s_x, con
     return launch_gemm_qkv(a, w_qkv, s_x, w_s, m, k, qa, as_stream(stream));
 }
 
-int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols) {
-    FX_REQUIRE(m > 0 && n > 0 && k > 0 && k % 64 == 0 && rows && cols, "linear_i8_gemm_tile: m=%d k=%d n=%d", m, k, n);
+int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols, int* per_cu) {
+    FX_REQUIRE(m > 0 && n > 0 && k > 0 && k % 64 == 0 && rows && cols && per_cu, "linear_i8_gemm_tile: m=%d k=%d n=%d", m, k, n);
     const GemmI8Tile& t = kGemmI8Tiles[k % 128 != 0][gemm_i8_tile(m, k, n, qkv != 0)];
     *rows = t.bm;
     *cols = t.bn;
+    *per_cu = t.per_cu;
     return FLEXLLM_OK;
 }
 

@@ -138,8 +138,9 @@ int flexllm_linear_i8_gemv_swiglu(const int8_t* x, const float* s_x, const int8_
  * pref_Linear_Layer_i4xi4 (Modules/Linear_Layer.h:293-341) with the int8 systolic array
  * (Modules/MHA.h:113-187, Modules/PE.h:526-583).  k % 64 == 0. */
 int flexllm_linear_i8_gemm(const int8_t* a, const int8_t* w, int32_t* acc, int m, int k, int n, void* stream);
-/* Rows and columns of the tile that an int8 product (qkv: the fused q/k/v projection) of these sizes runs on.  Needs no GPU. */
-int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols);
+/* Rows and columns of the tile that an int8 product (qkv: the fused q/k/v projection) of these sizes runs on, and how many of them
+ * a CU holds at a time.  Needs no GPU. */
+int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols, int* per_cu);
 /* The same exact product with UNSIGNED 8-bit activations (0..255), the reference's is_uint_input instantiation of its
  * int8 arrays (Modules/MHA.h:339-344, :854-859 with is_uint_input = true; Modules/PE.h:526-583, is_uint_A): used for
  * P.V with the uint8 softmax probabilities as a stand-alone stage.  a [m][k] uint8, w [n][k] int8, acc [m][n] int32;
@@ -598,6 +599,8 @@ int flexllm_hybrid_check(flexllm_hybrid* m);
  * bias [n] or NULL is added first; glu: 0, or 1 + FLEXLLM_GLU_*. */
 int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, void* y, float* y32, int m, int k, int n, int n_split, int glu, float limit,
                               int dtype, void* stream);
+/* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
+int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
 /* The linear behind the steps of a few tokens (1 to 8) on its own: x float32 [tokens][k], w [n][k rounded up to 64] of the
  * element type, zeros behind a row's k; both 16-byte aligned.  Outputs as above, all float32.  With n_split 0 and no bias a
  * bfloat16 product of several tokens may be asked for in `parts` sums over k, which leave y32 as [parts][tokens][n]. */

@@ -1,31 +1,64 @@
-"""Which tile a product runs on is arithmetic on the host: the tests on the GPU reach every tile, and wide products take wide ones."""
+"""Which tile a product runs on is arithmetic on the host: the tests on the GPU reach every tile, and products take the ones that
+measured best."""
 import ctypes as C
 
 import pytest
 
+import test_gpu_decoder_sizes as floats
 import test_gpu_gemm_tiles as gpu
 
 
-def tile(m, k, n, qkv=False):
+def ask(name, *sizes):
     from flexllm_amd import lib
-    rows, cols = C.c_int(), C.c_int()
-    assert lib().flexllm_linear_i8_gemm_tile(m, k, n, int(qkv), C.byref(rows), C.byref(cols)) == 0
-    return rows.value, cols.value
+    out = [C.c_int() for _ in range(3)]
+    assert getattr(lib(), name)(*sizes, *(C.byref(v) for v in out)) == 0
+    return tuple(v.value for v in out)
 
 
-ALL = {(256, 256), (128, 256), (128, 128), (64, 128), (64, 64)}
+def tile(m, k, n, qkv=False):
+    return ask("flexllm_linear_i8_gemm_tile", m, k, n, int(qkv))
+
+
+def float_tile(m, k, n, dtype="bfloat16"):
+    return ask("flexllm_linear_float_gemm_tile", m, k, n, int(dtype == "float32"))
+
+
+ONE = {(256, 256, 1), (128, 256, 1), (128, 128, 1), (64, 128, 1), (64, 64, 1)}      # rows, columns, workgroups per CU
+TWO = {(128, 128, 2)}
 
 
 def test_every_int8_tile_is_under_test():
-    assert {tile(*s) for s in gpu.TILES if s[1] % 128 == 0} == ALL
-    assert {tile(*s) for s in gpu.HALF} == ALL
-    assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV} == ALL - {(256, 256)}
+    assert {tile(*s) for s in gpu.TILES if s[1] % 128 == 0} == ONE | TWO
+    assert {tile(*s) for s in gpu.HALF} == ONE
+    assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV} == ONE - {(256, 256, 1)}
+
+
+def test_every_float_tile_is_under_test():
+    at = {k: {float_tile(m, k, n) for m, n, _, _ in floats.GEMM} for k in floats.GEMM_K}
+    assert at[576] == ONE | TWO
+    assert all(at[k] == ONE - {(64, 128, 1)} | TWO for k in floats.GEMM_K if k < 512)      # short k never runs on 64 x 128
+    for k in floats.GEMM_K[1:]:
+        assert {float_tile(m, k, n, "float32") for m, n, _, _ in floats.GEMM} == {(128, 128, 1), (64, 128, 1), (64, 64, 1)}
 
 
 @pytest.mark.parametrize("k", [2048, 2112])
 def test_wide_int8_products_take_wide_tiles(k):
-    assert tile(4096, k, 16384) == tile(1024, k, 16384) == (256, 256)
-    assert tile(4096, 4 * k, 2048) == (128, 256)
-    assert tile(2048, k, 2048) == (128, 128)
-    assert tile(1024, k, 2048) == (64, 128)
-    assert tile(32, k, 2048) == (64, 64)
+    assert tile(4096, k, 16384) == tile(1024, k, 16384) == (256, 256, 1)
+    assert tile(4096, 4 * k, 2048) == (128, 256, 1)
+    assert tile(2048, k, 2048) == (128, 128, 1)
+    assert tile(1024, k, 2048) == (64, 128, 1)
+    assert tile(32, k, 2048) == (64, 64, 1)
+
+
+def test_tiles_that_measured_best():
+    """Sizes at which another tile was 5 to 40 % slower."""
+    assert float_tile(3700, 8576, 2064) == tile(3700, 8576, 2064) == (128, 128, 2)      # 493 tiles
+    assert float_tile(3700, 4096, 28672) == float_tile(3072, 4096, 28672) == (256, 256, 1)
+    assert float_tile(1621, 320, 22276) == (128, 256, 1)
+    assert float_tile(777, 4096, 28672) == (256, 256, 1)
+    assert float_tile(1531, 2048, 16384) == (128, 256, 1)
+    assert float_tile(777, 14336, 4096) == (128, 128, 1)
+    assert float_tile(1024, 2048, 2048) == (64, 128, 1)
+    assert tile(731, 128, 27176) == tile(917, 704, 19348) == (128, 128, 1)
+    assert tile(2528, 2048, 8192) == tile(3072, 2048, 2048) == (128, 256, 1)
+    assert float_tile(266, 128, 18912, "float32") == (64, 64, 1)

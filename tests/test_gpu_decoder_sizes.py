@@ -66,10 +66,14 @@ def test_few_token_attention_splits(heads, kv_heads, dim, dtype):
 
 
 # every tile of the GEMM: one k-stage, fewer and more than the ring holds, rows and columns that do not fill the last tile
+GEMM_K = [64, 128, 256, 448, 576]
+GEMM = [(1024, 16380, 16380, 0), (1021, 16384, 16384, 1), (1100, 16384, 16000, 0), (1000, 4000, 4000, 2), (897, 4096, 0, 0), (1000, 2040, 1024, 0), (961, 2048, 2048, 1),
+        (65, 1028, 1028, 0), (1, 64, 0, 0), (1531, 16384, 16384, 1), (1500, 16380, 16000, 0), (3700, 2064, 2064, 2), (3699, 2060, 1000, 0), (2040, 4100, 4100, 0)]
+
+
 @BOTH
-@pytest.mark.parametrize("k", [64, 128, 256, 448])
-@pytest.mark.parametrize("m,n,split,glu", [(1024, 16380, 16380, 0), (1021, 16384, 16384, 1), (1100, 16384, 16000, 0), (1000, 4000, 4000, 2), (897, 4096, 0, 0),
-                                           (1000, 2040, 1024, 0), (961, 2048, 2048, 1), (65, 1028, 1028, 0), (1, 64, 0, 0)])
+@pytest.mark.parametrize("k", GEMM_K)
+@pytest.mark.parametrize("m,n,split,glu", GEMM)
 def test_gemm_tiles(m, n, split, glu, k, dtype):
     from flexllm_amd import ops, to_device
     from flexllm_amd.loader import from_bf16, to_bf16

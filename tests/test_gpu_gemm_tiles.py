@@ -9,7 +9,7 @@ from test_gpu_prefill import fx  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 TILES = [(1024, 128, 16384), (1021, 256, 16380), (1000, 128, 8192), (897, 384, 8188), (1000, 1024, 4096), (1023, 1024, 3972), (1000, 512, 2048),
-         (961, 128, 1924), (100, 640, 1028), (1, 128, 4), (200, 192, 516), (100, 2048, 1028)]
+         (961, 128, 1924), (100, 640, 1028), (1, 128, 4), (200, 192, 516), (100, 2048, 1028), (3700, 1152, 2060)]
 # k a multiple of 64 alone: stages of 64-byte rows, fewer and more of them than the four of the ring
 HALF = [(1021, 320, 16380), (1024, 2112, 16384), (1000, 64, 8192), (897, 320, 8188), (1023, 2112, 3972), (1000, 192, 4096), (961, 64, 1924), (1000, 1088, 2048),
         (1, 64, 4), (100, 448, 1028)]
