@@ -336,16 +336,22 @@ static int gemm_cheapest_tile(const GemmArgs& g, int parts, long& best) {
 }
 
 // Few rows of a long k leave most CUs without a tile, so k is shared out.  A part costs its sums' way to memory and back (8 bytes
-// each at 5 TB/s, besides the launch that it does not add) and has at least a ring of stages to walk.
+// each at 5 TB/s, besides the launch that it does not add) and has at least a ring of stages to walk.  The costs are good to a few
+// per cent, so that more parts have to be a 32nd cheaper; and the sums of all parts have to fit into the 32 MiB of the dies' L2 caches: beyond
+// them they cost more than that.  Whole prompts of the layers of width 4096 (four) and 2048 (sixteen), with the parts taken here and
+// in one part: 200 rows 1024 and 1120 us, 1700 and 1949; 1024 rows 2459 and 2532, 3596 and 3688; 1531 rows 3644 in two parts and 3516 in one (50
+// MB of sums: one), 4879 and 5040 (25 MB).
 template <typename ET>
 int gemm_parts(const GemmArgs& g, int most) {
+    constexpr size_t kSums = (size_t)32 << 20;
     long best = 0;
     int parts = 1;
     for (int p = 1; p <= most && p * 4 <= (int)(g.k * sizeof(ET) / 128); p *= 2) {
+        if (p > 1 && (size_t)p * g.m * g.n * sizeof(float) > kSums) break;
         long cost;
         gemm_cheapest_tile<ET>(g, p, cost);
         cost += (long)p * g.m * g.n * 8 / 50000;
-        if (p == 1 || cost < best) { best = cost; parts = p; }
+        if (p == 1 || cost < best - best / 32) { best = cost; parts = p; }
     }
     return parts;
 }
@@ -446,6 +452,13 @@ int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, in
     *cols = t.bn;
     *per_cu = t.per_cu;
     return FLEXLLM_OK;
+}
+
+int flexllm_linear_float_gemm_parts(int m, int k, int n, int dtype, int most) {
+    FX_REQUIRE((dtype == 0 || dtype == 1) && m > 0 && n > 0 && k > 0 && k % kKPad == 0 && most > 0, "linear_float_gemm_parts: m=%d k=%d n=%d dtype=%d", m, k, n, dtype);
+    GemmArgs g;
+    g.m = m; g.k = k; g.n = n;
+    return dtype == 0 ? gemm_parts<bf16_t>(g, most) : gemm_parts<float>(g, most);
 }
 
 }  // extern "C"

@@ -601,6 +601,9 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
                               int dtype, void* stream);
 /* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
 int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
+/* Parts (at most `most`) that k of such a product is shared out in where its reader adds the parts' sums up; negative: an error code.
+ * Needs no GPU. */
+int flexllm_linear_float_gemm_parts(int m, int k, int n, int dtype, int most);
 /* The linear behind the steps of a few tokens (1 to 8) on its own: x float32 [tokens][k], w [n][k rounded up to 64] of the
  * element type, zeros behind a row's k; both 16-byte aligned.  Outputs as above, all float32.  With n_split 0 and no bias a
  * bfloat16 product of several tokens may be asked for in `parts` sums over k, which leave y32 as [parts][tokens][n]. */

@@ -63,3 +63,19 @@ def test_tiles_that_measured_best():
     assert tile(731, 128, 27176) == tile(917, 704, 19348) == (128, 128, 1)
     assert tile(2528, 2048, 8192) == tile(3072, 2048, 2048) == (128, 256, 1)
     assert float_tile(266, 128, 18912, "float32") == (64, 64, 1)
+
+
+def parts(m, k, n, dtype="bfloat16", most=8):
+    from flexllm_amd import lib
+    return lib().flexllm_linear_float_gemm_parts(m, k, n, int(dtype == "float32"), most)
+
+
+def test_parts_of_k():
+    """Shared out for few rows; not for next to nothing, nor where the sums leave the caches (measured slower in parts)."""
+    assert parts(64, 14336, 4096) == 8 and parts(200, 8192, 2048) == 8 and parts(200, 8192, 2048, most=4) == 4
+    assert parts(64, 8192, 2048, "float32") == 8
+    assert parts(1024, 14336, 4096) == parts(1531, 8192, 2048) == 2
+    assert parts(640, 14336, 4096) == 2 and parts(777, 8192, 2048) == 2
+    assert parts(777, 4096, 4096) == 1
+    assert parts(1300, 14336, 4096) == parts(1531, 14336, 4096) == parts(2048, 14336, 4096) == 1
+    assert parts(64, 64, 2048) == 1
