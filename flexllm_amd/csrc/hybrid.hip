@@ -91,7 +91,7 @@ struct flexllm_hybrid {
     int4* ltiles = nullptr;
     // captured decode step
     hipGraphExec_t graph = nullptr;
-    int graph_slot = -1, graph_topk = 0;
+    int graph_slot = -1, graph_topk = 0, graph_splits = 0;
     const void *graph_io = nullptr, *graph_out = nullptr, *graph_rands = nullptr;
     hipStream_t graph_stream = nullptr;
 };
@@ -506,11 +506,11 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 // and 874 us; five tokens, gate and up of 2048 x 8192: 35 us and 4.6 + 17.
 static bool reads_again(int T, int n, int kpad, int es) { return T == 1 || (size_t)(T - 1) * n * kpad * es <= ((size_t)72 << 20); }
 
-// ---- one to kSmallTokens tokens --------------------------------------------------------------------------------------
+// ---- one to kSmallTokens tokens, behind which there are at most `held` --------------------------------------------------------------------------------------
 struct Pending { bool on = false; const float* gb = nullptr; int parts = 1; };      // the last sublayer's output in y (in parts) still has to be added
 
 template <typename ET>
-static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, const int* want, int n_want, float* logits, float* layers_out, hipStream_t st) {
+static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, int held, const int* want, int n_want, float* logits, float* layers_out, hipStream_t st) {
     const flexllm_hybrid_config& c = m->cfg;
     const int W = c.width, kw = pad_k(W);
     float *x = m->x0, *other = m->xa;                     // the embedding output stays in x0, later residuals alternate
@@ -580,7 +580,7 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
         FX_TRY(norm_linear(a, L.g1, m->runs[r].again));
         if (L.d.mixer == FLEXLLM_MIX_SHARED_KV) {
             const SharedKvRows<ET> rows = {static_cast<ET*>(s.rows[r]), s.inv_rms[r]};
-            FX_TRY(shared_kv_splits<ET>(L.sd, m->proj, m->max_et, m->f32, nf, L.kv_norm, rows, s.pos, 0, T, m->scratch, m->tickets, m->att, m->max_att, 1, st));
+            FX_TRY(shared_kv_splits<ET>(L.sd, m->proj, m->max_et, m->f32, nf, L.kv_norm, rows, s.pos, 0, T, held, m->scratch, m->tickets, m->att, m->max_att, 1, st));
         } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {
             ET* rows = static_cast<ET*>(s.rows[r]);
             FX_TRY(latent_decode<ET>(L.ld, m->proj, m->max_et, nf ? m->f32 : nullptr, nf, L.latent_norm, L.cos_t, L.sin_t, static_cast<ET*>(L.uk),
@@ -689,7 +689,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
             if (!flash)
                 for (int t0 = 0; t0 < T; t0 += kAbsorbTokens) {
                     const int n = T - t0 < kAbsorbTokens ? T - t0 : kAbsorbTokens;
-                    FX_TRY(shared_kv_splits<ET>(L.sd, proj + (size_t)t0 * ldp, ldp, nullptr, 0, L.kv_norm, rows, s.pos, t0, n, m->scratch, m->tickets, att + (size_t)t0 * lda, lda, 0, st));
+                    FX_TRY(shared_kv_splits<ET>(L.sd, proj + (size_t)t0 * ldp, ldp, nullptr, 0, L.kv_norm, rows, s.pos, t0, n, pos0 + t0 + n, m->scratch, m->tickets, att + (size_t)t0 * lda, lda, 0, st));
                 }
         } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {
             ET *cache = static_cast<ET*>(s.rows[r]), *uk = static_cast<ET*>(L.uk), *uv = static_cast<ET*>(L.uv);
@@ -798,7 +798,7 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
         while (w1 < n_want && want[w1] < t0 + T) part.push_back(want[w1++] - t0);
         float* lg = n_want ? logits + (size_t)w0 * m->cfg.vocab : nullptr;
         if (T <= kSmallTokens && (!layers_out || t0 == 0))
-            FX_TRY(run_small<ET>(m, s, tokens + t0, T, part.data(), (int)part.size(), lg, layers_out, st));
+            FX_TRY(run_small<ET>(m, s, tokens + t0, T, s.length + T, part.data(), (int)part.size(), lg, layers_out, st));
         else
             FX_TRY(run_many<ET>(m, s, tokens + t0, T, part.data(), (int)part.size(), lg, layers_out ? layers_out + (size_t)t0 * W : nullptr, (size_t)n * W, st));
         FX_TRY(advance_launch(s.pos, T, st));
@@ -811,10 +811,10 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
 
 // One token of the decode loop: *token_io -> logits -> next token, position and step advance on the device.
 template <typename ET>
-static int decode_token(flexllm_hybrid* m, int slot, int* token_io, const float* rands, int top_k, int* tokens_out, hipStream_t st) {
+static int decode_token(flexllm_hybrid* m, int slot, int held, int* token_io, const float* rands, int top_k, int* tokens_out, hipStream_t st) {
     HybridSlot& s = m->slots[slot];
     const int zero = 0, V = m->cfg.vocab;
-    FX_TRY(run_small<ET>(m, s, token_io, 1, &zero, 1, m->logits, nullptr, st));
+    FX_TRY(run_small<ET>(m, s, token_io, 1, held, &zero, 1, m->logits, nullptr, st));
     if (top_k == 0) {
         argmax_partial_kernel<<<kArgmaxParts, 256, 0, st>>>(m->logits, V, m->am_v, m->am_i);
         argmax_final_advance_kernel<<<1, 64, 0, st>>>(m->am_v, m->am_i, kArgmaxParts, token_io, tokens_out, s.pos);
@@ -827,9 +827,9 @@ static int decode_token(flexllm_hybrid* m, int slot, int* token_io, const float*
     return FLEXLLM_OK;
 }
 
-static int decode_any(flexllm_hybrid* m, int slot, int* token_io, const float* rands, int top_k, int* tokens_out, hipStream_t st) {
-    return m->cfg.dtype == 0 ? decode_token<bf16_t>(m, slot, token_io, rands, top_k, tokens_out, st)
-                             : decode_token<float>(m, slot, token_io, rands, top_k, tokens_out, st);
+static int decode_any(flexllm_hybrid* m, int slot, int held, int* token_io, const float* rands, int top_k, int* tokens_out, hipStream_t st) {
+    return m->cfg.dtype == 0 ? decode_token<bf16_t>(m, slot, held, token_io, rands, top_k, tokens_out, st)
+                             : decode_token<float>(m, slot, held, token_io, rands, top_k, tokens_out, st);
 }
 
 }  // namespace fx
@@ -905,15 +905,18 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
     if (steps == 0) return FLEXLLM_OK;
     FX_TRY(set_state_launch(s.pos, s.length, 0, st));
     if (!use_graph) {
-        for (int i = 0; i < steps; i++) FX_TRY(decode_any(m, slot, token_io, rands, top_k, tokens_out, st));
+        for (int i = 0; i < steps; i++) FX_TRY(decode_any(m, slot, s.length + steps, token_io, rands, top_k, tokens_out, st));
     } else {
+        int splits = 0;                                   // of all layers together: none has fewer at more rows
+        for (const HybridLayer& L : m->layers)
+            if (L.d.mixer == FLEXLLM_MIX_SHARED_KV) splits += shared_kv_split_count(L.sd, 1, s.length + steps);
         if (!m->graph || m->graph_slot != slot || m->graph_topk != top_k || m->graph_io != token_io || m->graph_out != tokens_out ||
-            m->graph_rands != rands || m->graph_stream != st) {
+            m->graph_rands != rands || m->graph_stream != st || m->graph_splits != splits) {
             if (m->graph) { (void)hipGraphExecDestroy(m->graph); m->graph = nullptr; }
             FX_HIP(hipStreamSynchronize(st));
             hipGraph_t graph;
             FX_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            const int rc = decode_any(m, slot, token_io, rands, top_k, tokens_out, st);
+            const int rc = decode_any(m, slot, s.length + steps, token_io, rands, top_k, tokens_out, st);
             hipError_t e = hipStreamEndCapture(st, &graph);
             if (rc) { if (e == hipSuccess) (void)hipGraphDestroy(graph); return rc; }
             FX_HIP(e);
@@ -921,7 +924,7 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
             (void)hipGraphDestroy(graph);
             if (e != hipSuccess) m->graph = nullptr;
             FX_HIP(e);
-            m->graph_slot = slot; m->graph_topk = top_k; m->graph_io = token_io; m->graph_out = tokens_out; m->graph_rands = rands; m->graph_stream = st;
+            m->graph_slot = slot; m->graph_topk = top_k; m->graph_io = token_io; m->graph_out = tokens_out; m->graph_rands = rands; m->graph_stream = st; m->graph_splits = splits;
         }
         for (int i = 0; i < steps; i++) FX_HIP(hipGraphLaunch(m->graph, st));
     }

@@ -78,24 +78,31 @@ template int shared_kv_store<bf16_t>(const SharedKvDims&, const float*, int, Sha
 template int shared_kv_store<float>(const SharedKvDims&, const float*, int, SharedKvRows<float>, const int*, int, hipStream_t);
 
 // ---- few tokens -----------------------------------------------------------------------------------------------------
-constexpr int kKvSplits = 32, kKvStats = 4;               // most splits; floats behind a split's sums (maximum, weight sum)
+constexpr int kKvSplits = 64, kKvRead = 32, kKvStats = 4;               // most splits, and those that the join reads at a time; floats behind a split's sums (maximum, weight sum)
 
 static int kv_head_group(const SharedKvDims& d) {         // query heads per workgroup
     const int r = d.heads / d.kv_heads;
     return r >= 4 ? 4 : r >= 2 ? 2 : 1;
 }
-// One workgroup per CU.  The position is known on the device only, so workgroups beyond the rows that there are start too, and
-// every split stands in line at the ticket.  32 heads on 8, dim 64, behind a linear: one token at 1531 rows 10.9 us with 32 splits and
-// 17.9 with 64, five tokens at 5 rows 8.4 us with 8 splits each and 17.9 with 32.  Wider workgroups, with as many rows at once
+// Splits for up to `rows` rows.  At first one workgroup per CU, at most 32 splits: every split stands in line at the ticket, and
+// workgroups beyond the rows that there are start too.  32 heads on 8, dim 64, behind a linear: one token at 1531 rows 10.9 us with 32
+// splits and 17.9 with 64, five tokens at 5 rows 8.4 us with 8 splits each and 17.9 with 32.  Wider workgroups, with as many rows at once
 // in 8 or 16 waves, are no faster (11.4 and 14.7 us): what their waves save in steps they cost to start.
-static int kv_split_count(const SharedKvDims& d, int tokens) {
+// Long caches take twice the splits, from 384 rows per split on where CUs are without one, from 768 where they then hold two.
+// A decode step per layer, rows in the cache, 32 splits (8 for 32 heads on 32) and twice those: 4 heads on 1, dim 128, 16384 rows 40.1 and
+// 36.5 us, 32000 rows 53.0 and 43.4; 16 on 2, dim 128, 16384 rows 42.7 and 39.2; 32 on 8, dim 64, 16384 rows 34.8 and 36.4, 32000 rows 39.8
+// and 39.7; 32 on 32, dim 64, 4096 rows 29.3 and 29.7, 8192 rows 34.9 and 32.1, 32000 rows 63.5 and 53.7.  The host says how many rows
+// there are, since workgroups that find none are not for nothing (256 of them 2 us).
+static int kv_split_count(const SharedKvDims& d, int tokens, int rows) {
     const int gh = kv_head_group(d), blocks = tokens * d.kv_heads * ((d.heads / d.kv_heads + gh - 1) / gh);
     int s = 1;
-    while (s < kKvSplits && s * blocks < 256) s *= 2;
+    while (s < 32 && s * blocks < 256) s *= 2;
+    while (s < kKvSplits && 2 * s * blocks <= 512 && rows >= s * (2 * s * blocks <= 256 ? 384 : 768)) s *= 2;
     const int most = (d.capacity + 31) / 32;
     return s < most ? s : most;
 }
-size_t shared_kv_scratch(const SharedKvDims& d) { return (size_t)d.heads * kv_split_count(d, 1) * (d.dimp + kKvStats); }
+int shared_kv_split_count(const SharedKvDims& d, int tokens, int rows) { return kv_split_count(d, tokens, rows); }
+size_t shared_kv_scratch(const SharedKvDims& d) { return (size_t)d.heads * kv_split_count(d, 1, d.capacity) * (d.dimp + kKvStats); }
 
 // N consecutive float32 (N a multiple of 4, 16-byte aligned), zeros where there are none.
 template <int N>
@@ -372,17 +379,17 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
     // ---- the join, one wave per head for the weights; here the sink enters the sum of the weights.  The first columns of all
     // splits are requested ahead of that: one trip to memory instead of three.
     const int outs = nh * d.dim;
-    float u[kKvSplits];
-    auto request = [&](int i) {
+    float u[kKvRead];
+    auto request = [&](int i, int s0) {
         const int h = min(i / d.dim, nh - 1), e = i % d.dim;
 #pragma unroll
-        for (int j = 0; j < kKvSplits; j += 8) {
-            if (j >= ns) break;
+        for (int j = 0; j < kKvRead; j += 8) {
+            if (s0 + j >= ns) break;
 #pragma unroll
-            for (int n = j; n < j + 8; n++) u[n] = load_past(split_at(h, min(n, ns - 1)) + e);
+            for (int n = j; n < j + 8; n++) u[n] = load_past(split_at(h, min(s0 + n, ns - 1)) + e);
         }
     };
-    if (ns > 1) request(t);
+    if (ns > 1) request(t, 0);
     if (wave < nh) {
         float ms = -1e30f, ls = 0.0f;
         if (ns == 1) {
@@ -397,9 +404,9 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
         if (ns == 1) w = __builtin_amdgcn_exp2f(top - mj);
         float lj = wave_sum(ls * w);
         if (d.sink) lj += __builtin_amdgcn_exp2f(-mj);
-        if (lane < kKvSplits) wsp[wave * kKvSplits + lane] = w / lj;
+        wsp[wave * kKvSplits + lane] = w / lj;
     }
-    static_assert(GH <= NW && kKvSplits <= 64 && kKvSplits % 8 == 0, "a wave per head, a lane per split");
+    static_assert(GH <= NW && kKvSplits == 64 && kKvRead % 8 == 0, "a wave per head, a lane per split");
     __syncthreads();
     for (int i = t; i < outs; i += NT) {
         const int h = i / d.dim, e = i - h * d.dim;
@@ -407,12 +414,14 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
         if (ns == 1) {
             v = of_waves(sums + h * d.dimp + e, step) * wsp[h * kKvSplits];
         } else {
-            if (i >= NT) request(i);
+            for (int s0 = 0; s0 < ns; s0 += kKvRead) {
+                if (i >= NT || s0 > 0) request(i, s0);
 #pragma unroll
-            for (int j = 0; j < kKvSplits; j += 8) {
-                if (j >= ns) break;
+                for (int j = 0; j < kKvRead; j += 8) {
+                    if (s0 + j >= ns) break;
 #pragma unroll
-                for (int n = j; n < j + 8; n++) v = fma_f(u[n], wsp[h * kKvSplits + n], v);      // weight 0 beyond the last split
+                    for (int n = j; n < j + 8; n++) v = fma_f(u[n], wsp[h * kKvSplits + s0 + n], v);      // weight 0 beyond the last split
+                }
             }
             if (isnan(v)) {                               // an infinite sum of the last split is not nothing at weight 0: the splits alone
                 v = 0.0f;
@@ -427,8 +436,8 @@ __global__ __launch_bounds__(256) void shared_kv_split_kernel(SharedKvDims d, co
 
 template <typename ET, int LPK, int GH, int CPL>
 static int launch_splits(const SharedKvDims& d, const void* q, int ldq, const float* k, int ldk, const float* norm_w, const SharedKvRows<ET>& c,
-                         const int* state, int tok0, int tokens, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
-    const int splits = kv_split_count(d, tokens), rep = d.heads / d.kv_heads;
+                         const int* state, int tok0, int tokens, int held, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
+    const int splits = kv_split_count(d, tokens, held), rep = d.heads / d.kv_heads;
     const dim3 grid(splits, d.kv_heads * ((rep + GH - 1) / GH), tokens);
     const size_t lds = GH * (kKvSplits + 4 * (size_t)d.dimp) * sizeof(float);
     shared_kv_split_kernel<ET, LPK, GH, CPL><<<grid, 256, lds, st>>>(d, q, ldq, f32, k, ldk, norm_w, c, state, tok0, splits, scratch, tickets, o, ldo, f32);
@@ -438,16 +447,16 @@ static int launch_splits(const SharedKvDims& d, const void* q, int ldq, const fl
 
 template <typename ET>
 int shared_kv_splits(const SharedKvDims& d, const void* q, int ldq, const float* k, int ldk, const float* norm_w, SharedKvRows<ET> c, const int* state,
-                     int tok0, int tokens, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
+                     int tok0, int tokens, int held, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st) {
     FX_REQUIRE(q && norm_w && c.row && c.inv_rms && state && scratch && tickets && o && tokens > 0 && (!k || tok0 == 0), "shared_kv_splits: null pointer, or %d tokens at %d", tokens, tok0);
     FX_REQUIRE(d.heads % d.kv_heads == 0 && d.dimp % 8 == 0 && d.dimp >= d.dim && d.dimp <= 512 && ldq % (f32 ? 4 : 8) == 0 && ldk % 4 == 0,
                "shared_kv_splits: %d heads on %d, rows of %d, strides %d %d", d.heads, d.kv_heads, d.dimp, ldq, ldk);
     const int chunks = d.dimp / Chunk<ET>::N, gh = kv_head_group(d);
     int rc;
 #define FX_SPLITS(LPK, CPL)                                                                                                                \
-    (gh == 4   ? launch_splits<ET, LPK, 4, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st)                    \
-     : gh == 2 ? launch_splits<ET, LPK, 2, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st)                    \
-               : launch_splits<ET, LPK, 1, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, scratch, tickets, o, ldo, f32, st))
+    (gh == 4   ? launch_splits<ET, LPK, 4, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, held, scratch, tickets, o, ldo, f32, st)                    \
+     : gh == 2 ? launch_splits<ET, LPK, 2, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, held, scratch, tickets, o, ldo, f32, st)                    \
+               : launch_splits<ET, LPK, 1, CPL>(d, q, ldq, k, ldk, norm_w, c, state, tok0, tokens, held, scratch, tickets, o, ldo, f32, st))
     if (chunks <= 8) rc = FX_SPLITS(8, 1);
     else if (chunks <= 16) rc = FX_SPLITS(16, 1);
     else if (chunks <= 32) rc = FX_SPLITS(32, 1);
@@ -457,8 +466,8 @@ int shared_kv_splits(const SharedKvDims& d, const void* q, int ldq, const float*
 #undef FX_SPLITS
     return rc;
 }
-template int shared_kv_splits<bf16_t>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<bf16_t>, const int*, int, int, float*, int*, void*, int, int, hipStream_t);
-template int shared_kv_splits<float>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<float>, const int*, int, int, float*, int*, void*, int, int, hipStream_t);
+template int shared_kv_splits<bf16_t>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<bf16_t>, const int*, int, int, int, float*, int*, void*, int, int, hipStream_t);
+template int shared_kv_splits<float>(const SharedKvDims&, const void*, int, const float*, int, const float*, SharedKvRows<float>, const int*, int, int, int, float*, int*, void*, int, int, hipStream_t);
 
 // ---- many tokens ----------------------------------------------------------------------------------------------------
 // Workgroup: NW waves x 32 queries over tiles of 64 rows.  The queries of a key/value head are numbered token by token, the

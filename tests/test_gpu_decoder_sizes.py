@@ -168,6 +168,32 @@ def test_infinite_units(ff, dtype):
         assert (same(got[1]) == same(got[3])).all()
 
 
+def test_splits_of_long_caches():
+    """From 12288 rows on these heads have twice the splits: steps on both sides of the border, and decoding across it, whose graph
+    is made for the rows that there will be."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd.lopazen import Lopazen
+    cfg = lc.config([lc.layer(heads=2, kv_heads=1, dim=16)])
+    cuts = [12270, 7, 8, 2, 1, 1, 3, 4, 8, 2]
+    check_lopazen(cfg, "float32", sum(cuts), cuts, max_pos=12544)
+    check_lopazen(cfg, "bfloat16", sum(cuts), cuts, max_pos=12544)
+    w, toks = lc.weights(cfg, 11), lc.tokens(cfg, 12281)
+    m = Lopazen.from_tensors(cfg, w, dtype="float32", max_pos=12544, slots=2)
+    slots = [m.pool.acquire(n) for n in "ab"]
+    for s in slots:
+        m.step(s, toks[:-1])
+    token, got, want = to_device(np.array(toks[-1:], np.int32)), [], toks[-1:]
+    for n in (4, 20, 5):
+        out = zeros((n,), np.int32)
+        m.decode(slots[0], token, n, out)
+        m.check()
+        got += out.numpy().tolist()
+    for _ in got:
+        want.append(int(m.step(slots[1], want[-1:], [0])[0].argmax()))
+    m.close()
+    assert got == want[1:]
+
+
 # the last split of the rows repeats in the join of fewer splits than it reads at a time
 @BOTH
 @pytest.mark.parametrize("rows", [40, 96, 200, 256, 270])
