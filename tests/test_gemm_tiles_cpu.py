@@ -24,13 +24,13 @@ def float_tile(m, k, n, dtype="bfloat16"):
 
 
 ONE = {(256, 256, 1), (128, 256, 1), (128, 128, 1), (64, 128, 1), (64, 64, 1)}      # rows, columns, workgroups per CU
-TWO = {(128, 128, 2)}
+TWO, THREE = {(128, 128, 2)}, {(64, 64, 3)}
 
 
 def test_every_int8_tile_is_under_test():
-    assert {tile(*s) for s in gpu.TILES if s[1] % 128 == 0} == ONE | TWO
+    assert {tile(*s) for s in gpu.TILES if s[1] % 128 == 0} == ONE | TWO | THREE
     assert {tile(*s) for s in gpu.HALF} == ONE
-    assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV} == ONE - {(256, 256, 1)}
+    assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV} == ONE - {(256, 256, 1)} | THREE
 
 
 def test_every_float_tile_is_under_test():
@@ -60,7 +60,8 @@ def test_tiles_that_measured_best():
     assert float_tile(1531, 2048, 16384) == (128, 256, 1)
     assert float_tile(777, 14336, 4096) == (128, 128, 1)
     assert float_tile(1024, 2048, 2048) == (64, 128, 1)
-    assert tile(731, 128, 27176) == tile(917, 704, 19348) == (128, 128, 1)
+    assert tile(917, 704, 19348) == (128, 128, 1)
+    assert tile(1536, 2048, 2048) == tile(2176, 512, 2048) == tile(1536, 512, 2048) == tile(393, 128, 9536) == (64, 64, 3)
     assert tile(2528, 2048, 8192) == tile(3072, 2048, 2048) == (128, 256, 1)
     assert float_tile(266, 128, 18912, "float32") == (64, 64, 1)
 
