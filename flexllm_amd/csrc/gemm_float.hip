@@ -306,8 +306,10 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
 }
 
 // The tile whose rounds over the chip take the least time.  cost: of one stage of a round, and `round` once per round, in 0.01 us, as
-// measured where all CUs are busy; per_cu: workgroups that a CU holds at a time.  (A fit over 300 sizes from 1 to 5000 rows gives a
-// constant per round to the 64 x 128 tiles only; the tiles picked are within 1 % of the best ones on average.)
+// measured where all CUs are busy; per_cu: workgroups that a CU holds at a time.  The bfloat16 ones are those that lose least over 520 sizes of 1
+// to 4096 rows and 64 to 14336 k: the tiles picked are 0.6 % from the best ones on average.  What a round costs besides its stages decides where k
+// is short and the outputs' stores bound the product: 2409 x 5608 x 256 23.7 us on 256 x 256, 20.5 on 128 x 128 twice per CU,
+// where 1621 x 22276 x 320 takes 54.8 us on 128 x 256 and 63.4 on those; 2070 x 9468 x 5632 293 us on 128 x 128, 253 on 128 x 256.
 //
 // bfloat16 (64 k): 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3
 // rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048
@@ -318,7 +320,7 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
 struct GemmTileCost { int bm, bn, cost, round, per_cu; };
 template <typename ET> struct GemmTiles;
 template <> struct GemmTiles<bf16_t> {
-    static constexpr GemmTileCost list[] = {{256, 256, 200, 0, 1}, {128, 256, 110, 0, 1}, {128, 128, 64, 0, 1}, {64, 128, 42, 100, 1}, {64, 64, 28, 0, 1}, {128, 128, 113, 0, 2}};
+    static constexpr GemmTileCost list[] = {{256, 256, 190, 520, 1}, {128, 256, 107, 180, 1}, {128, 128, 64, 150, 1}, {64, 128, 51, 170, 1}, {64, 64, 37, 40, 1}, {128, 128, 120, 120, 2}};
 };
 template <> struct GemmTiles<float> { static constexpr GemmTileCost list[] = {{128, 128, 235, 0, 1}, {64, 128, 126, 100, 1}, {64, 64, 66, 0, 1}}; };
 

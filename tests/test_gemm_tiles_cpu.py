@@ -35,8 +35,9 @@ def test_every_int8_tile_is_under_test():
 
 def test_every_float_tile_is_under_test():
     at = {k: {float_tile(m, k, n) for m, n, _, _ in floats.GEMM} for k in floats.GEMM_K}
-    assert at[576] == ONE | TWO
-    assert all(at[k] == ONE - {(64, 128, 1)} | TWO for k in floats.GEMM_K if k < 512)      # short k never runs on 64 x 128
+    assert at[448] == at[576] == ONE | TWO
+    assert at[256] == {(128, 128, 1), (64, 128, 1), (64, 64, 1)} | TWO                        # short k never runs on the wide tiles,
+    assert at[64] == at[128] == {(128, 128, 1), (64, 64, 1)} | TWO                            # nor the shortest on 64 x 128
     at = {k: {float_tile(m, k, n, "float32") for m, n, _, _ in floats.GEMM} for k in floats.GEMM_K}
     assert at[576] == {(128, 128, 1), (64, 128, 1), (64, 64, 1)}
     assert all(at[k] == {(128, 128, 1), (64, 64, 1)} for k in floats.GEMM_K if k < 512)
@@ -56,6 +57,9 @@ def test_tiles_that_measured_best():
     assert float_tile(3700, 8576, 2064) == tile(3700, 8576, 2064) == (128, 128, 2)      # 493 tiles
     assert float_tile(3700, 4096, 28672) == float_tile(3072, 4096, 28672) == (256, 256, 1)
     assert float_tile(1621, 320, 22276) == (128, 256, 1)
+    assert float_tile(2409, 256, 5608) == float_tile(1468, 128, 23752) == float_tile(639, 128, 16380) == (128, 128, 2)
+    assert float_tile(2070, 5632, 9468) == float_tile(3072, 2048, 6144) == (128, 256, 1)
+    assert float_tile(288, 1664, 23660) == (128, 128, 1)
     assert float_tile(777, 4096, 28672) == (256, 256, 1)
     assert float_tile(1531, 2048, 16384) == (128, 256, 1)
     assert float_tile(777, 14336, 4096) == (128, 128, 1)
