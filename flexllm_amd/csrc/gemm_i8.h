@@ -566,24 +566,25 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
     return FLEXLLM_OK;
 }
 
-// The direct-load kernel runs on the tile whose rounds over the 256 CUs (a workgroup per CU) cost least, in 0.01 us: per stage, and
-// once per round for what lies around them (first loads, epilogue).  From products of 2048 and 8192 k (whole 128-byte lines per row
-// and stage) and of 2112 and 8256 k (a multiple of 64 only: 64-byte rows) where all CUs are busy.
+// The direct-load kernel runs on the tile whose rounds over the 256 CUs (per_cu at a time) cost least, in about 0.01 us: per stage, and
+// once per round for what lies around them (first loads, epilogue).  Rows of a stage are whole 128-byte lines where k
+// allows, 64 bytes where it is a multiple of 64 alone.
 // 128-byte rows, measured against the fixed choices before (us): 512 x 16384 x 2048 43.8 -> 24.8 (128 x 256), 2048 x 2048 x 8192 62.7 -> 45.8
 // (128 x 128), 2528 x 2048 x 8192 85.1 -> 65.1 (128 x 256), 1536 x 2048 x 8192 53.4 -> 41.3 (128 x 128), 4096 x 2048 x 8192 91.0 -> 80.4
 // (128 x 256), 1024 x 2048 x 2048 12.1 -> 11.3 (64 x 128); 1024 x 16384 x 2048 stays on 256 x 256, 41.5.
 // 64-byte rows, against 64 x 64 everywhere (us): 1024 x 8192 x 2112 41.6 -> 25.3 (128 x 256), 1024 x 16384 x 2112 85.2 -> 40.3 and
 // 4096 x 16384 x 2112 427 -> 192 (256 x 256), 1024 x 2048 x 8256 42.1 -> 32.3 (64 x 128), 2048 x 2048 x 8256 95.9 -> 47.6 (128 x 128).
-// Outputs that a short k hardly fills are bound by their stores, which is what the costs per round were set by: 731 x 27176 x 128
-// 28.8 us on 64 x 128, 23.0 on 128 x 128; 917 x 19348 x 704 40.7 us on 128 x 256, 29.8 on 128 x 128.
+// A product of a short k is bound by the stores of its output: 917 x 19348 x 704 40.7 us on 128 x 256, 29.8 on 128 x 128; 3575 x 2548 x 192
+// 26.2 us on 256 x 256, 17.1 on 64 x 64.
 // 128 x 128 in four waves with two stages fits twice into a CU (per_cu): 3700 x 2064 x 8576, 493 tiles, 74.6 us in one round of it, 86.2 in
-// two of the one with four stages.  64 x 64 with three stages fits three times: 1536 x 2048 x 2048, 768 tiles, 13.3 us in one
-// round of it, 14.3 on 128 x 128; 393 x 9536 x 128 7.9 us, 9.6 on 128 x 128 twice per CU.  The costs of 128-byte rows are the ones that lose least over
-// 260 sizes of 1 to 4096 rows: their tiles are 0.8 % from the best ones on average.
+// two of the one with four stages.  64 x 64 with three stages fits three times: 1536 x 2048 x 2048, 768 tiles, 14.4 us in one
+// round of it, 15.8 on 128 x 128; 393 x 9536 x 128 7.5 us, 9.5 on 128 x 128 twice per CU.
+// The costs are the ones that lose least over 384 sizes (128-byte rows) and 136 sizes (64-byte rows) of 1 to 4096 rows and 64 to 14336 k: their
+// tiles are 0.6 and 0.2 % from the best ones on average.
 struct GemmI8Tile { int bm, bn, stage, round, per_cu; };
 constexpr GemmI8Tile kGemmI8Tiles[2][7] = {
-    {{256, 256, 128, 1750, 1}, {128, 256, 68, 890, 1}, {128, 128, 72, 340, 1}, {64, 128, 57, 290, 1}, {64, 64, 52, 75, 1}, {64, 64, 80, 210, 3}, {128, 128, 88, 770, 2}},
-    {{256, 256, 88, 1120, 1}, {128, 256, 61, 650, 1}, {128, 128, 32, 440, 1}, {64, 128, 22, 400, 1}, {64, 64, 17, 350, 1}, {}, {}}};
+    {{256, 256, 108, 2230, 1}, {128, 256, 75, 1130, 1}, {128, 128, 75, 370, 1}, {64, 128, 60, 490, 1}, {64, 64, 28, 410, 1}, {64, 64, 76, 350, 3}, {128, 128, 106, 920, 2}},
+    {{256, 256, 40, 1640, 1}, {128, 256, 29, 1180, 1}, {128, 128, 25, 260, 1}, {64, 128, 18, 390, 1}, {64, 64, 13, 70, 1}, {}, {}}};
 inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
     const bool half = k % 128 != 0;
     long best = 0;
