@@ -259,6 +259,9 @@ static int launch_gemv_rs(const GemvArgs& g, int pro, int tokens, hipStream_t st
     // groups with the next one's weights in flight
     int wgs = (S > 4 ? 512 : 1024) / rows_y;
     if (wgs < 128) wgs = 128;
+    // the workgroups of one walk for all tokens belong on one die, whose L2 hands the weights on: dies take workgroups in turn
+    // (three tokens of 16 layers of 2048, 341 workgroups each: 1107 us, 336: 1031)
+    if (tokens > 1) wgs &= ~7;
     const int ng = (g.n + R - 1) / R;
     const dim3 grid(ng < wgs ? ng : wgs, rows_y);
     const size_t lds = (size_t)(g.kpad + Chunk<ET>::N) * sizeof(float);
@@ -573,6 +576,9 @@ int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     // overlap the next group's loads: 16384 x 2048 13.9 us with eight, 12.9 with four; 28672 x 4096 42.2 -> 37.7 us), eight
     // where a workgroup has a single group anyway (4096 x 4096: 7.65 us with eight, 7.96 with four) and for rows so long
     // that two rows are eight pieces (2048 x 8192: 8.2 us, 8.4 one row at a time; 4096 x 14336: 21.1 and 23.1).
+    // Several tokens wait for the L2, with eight in flight again from the third on (four tokens as in reads_again: 1349 us with eight,
+    // 1444 with four; two tokens 1058 and 1030).
+    if (steps == 1 && pro != 2 && tokens > 2 && (g.n + 7) / 8 * tokens >= 512) return launch_gemv_rs<ET, 8, 1>(g, pro, tokens, st);
     if (steps == 1) return launch_gemv_rs<ET, 4, 1>(g, pro, tokens, st);
     if (steps == 2) return (g.n + 3) / 4 <= 1024 ? launch_gemv_rs<ET, 4, 2>(g, pro, tokens, st) : launch_gemv_rs<ET, 2, 2>(g, pro, tokens, st);
     if (steps > 4 && pro == 0) return launch_gemv_rs<ET, 2, 8>(g, pro, tokens, st);

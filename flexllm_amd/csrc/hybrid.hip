@@ -501,12 +501,15 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 }
 
 // A linear behind a norm, for T tokens of a step: every token reads the weights (from L2, behind the first) under its own norm's
-// prologue while the bytes read again are few, else the norms have a launch of their own (4.6 us) ahead of one pass over the
-// weights.  Two tokens, 16 layers of 2048: 1162 us with the former everywhere, 1390 us with the latter; four layers of 4096: 952
-// and 874 us; five tokens, gate and up of 2048 x 8192: 35 us and 4.6 + 17.
-static bool reads_again(int T, int n, int kpad, int es) { return T == 1 || (size_t)(T - 1) * n * kpad * es <= ((size_t)72 << 20); }
+// prologue while that is cheap, else the norms have a launch of their own (5 us) ahead of one pass over the weights.
+// Rows of at most 4 KiB, a piece per thread, are cheap up to four tokens: 16 layers of 2048, bfloat16, three tokens 945 us against 1107
+// (with a recurrence in every second layer 1208 and 1370), four 1013 and 1114 (1349 and 1480), six 1243 and 1203.
+// Longer rows and more tokens while the bytes read again are few.  Four layers of 4096, two tokens: 952 us with the former everywhere,
+// 874 with the latter; three tokens 671 and 588.
+static bool short_rows(int kpad, int es) { return kpad * es <= 4096; }
+static bool reads_again(int T, int n, int kpad, int es) { return T == 1 || (T <= 4 && short_rows(kpad, es)) || (size_t)(T - 1) * n * kpad * es <= ((size_t)72 << 20); }
 
-// ---- one to kSmallTokens tokens, behind which there are at most `held` --------------------------------------------------------------------------------------
+// ---- one to kSmallTokens tokens, behind which there are at most `held` ------------------------------------------------
 struct Pending { bool on = false; const float* gb = nullptr; int parts = 1; };      // the last sublayer's output in y (in parts) still has to be added
 
 template <typename ET>
@@ -562,7 +565,7 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
     auto to_y = [&](const void* w, int k, const float* v, int ldv, const float* gb, bool shared) {      // shared: k may be shared out
         GemvArgs a = base(w, W, k);
         a.x = v; a.ldx = ldv; a.n_split = 0; a.out32 = m->y; a.ldo32 = W;
-        a.per_token = T == 2 && W * sizeof(ET) <= 4096;   // short rows: as cheap, and the next linear's prologue takes the sum as it is
+        a.per_token = T > 1 && T <= 4 && short_rows(kw, sizeof(ET));      // then the next linear's prologue takes the sum as it is
         if (T > 1 && !a.per_token && shared) { a.parts = gemv_parts<ET>(W, a.kpad, kMaxParts); a.part_stride = (size_t)T * W; }
         pending(gb, a.parts);
         return gemv_float<ET>(a, 0, T, st);

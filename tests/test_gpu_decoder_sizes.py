@@ -123,7 +123,7 @@ def test_slices_of_a_prompt(dtype):
 # two to eight tokens in one step: every number of tokens per pass over the weights, vectors of one to fifteen pieces per thread, a
 # gated unit on vectors so long that its pairs need two rows per group, odd lengths, a mixture
 @BOTH
-@pytest.mark.parametrize("width,ff", [(160, 88), (90, 33), (2112, 2050), (64, 4100), (64, 8200), (64, 15360), (8256, 40)])
+@pytest.mark.parametrize("width,ff", [(160, 88), (160, 1029), (90, 33), (2112, 2050), (64, 4100), (64, 8200), (64, 15360), (8256, 40)])
 def test_step_of_several_tokens(width, ff, dtype):
     cfg = lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff))], width=width, vocab=131, loop=(0, 1, 2))
     check_lopazen(cfg, dtype, 35, [2, 3, 4, 5, 6, 7, 8])
