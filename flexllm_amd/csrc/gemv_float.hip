@@ -576,11 +576,11 @@ int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     // overlap the next group's loads: 16384 x 2048 13.9 us with eight, 12.9 with four; 28672 x 4096 42.2 -> 37.7 us), eight
     // where a workgroup has a single group anyway (4096 x 4096: 7.65 us with eight, 7.96 with four) and for rows so long
     // that two rows are eight pieces (2048 x 8192: 8.2 us, 8.4 one row at a time; 4096 x 14336: 21.1 and 23.1).
-    // Several tokens wait for the L2, with eight in flight again from the third on (four tokens as in reads_again: 1349 us with eight,
-    // 1444 with four; two tokens 1058 and 1030).
+    // Several tokens wait for the L2, with eight in flight again: of rows of two pieces always, of one piece from the third token on (four
+    // tokens of 16 layers of 2048, bfloat16, half of them recurrences: 1349 us with eight, 1444 with four; two tokens 1058 and 1030).
     if (steps == 1 && pro != 2 && tokens > 2 && (g.n + 7) / 8 * tokens >= 512) return launch_gemv_rs<ET, 8, 1>(g, pro, tokens, st);
     if (steps == 1) return launch_gemv_rs<ET, 4, 1>(g, pro, tokens, st);
-    if (steps == 2) return (g.n + 3) / 4 <= 1024 ? launch_gemv_rs<ET, 4, 2>(g, pro, tokens, st) : launch_gemv_rs<ET, 2, 2>(g, pro, tokens, st);
+    if (steps == 2) return (g.n + 3) / 4 <= 1024 || tokens > 1 ? launch_gemv_rs<ET, 4, 2>(g, pro, tokens, st) : launch_gemv_rs<ET, 2, 2>(g, pro, tokens, st);
     if (steps > 4 && pro == 0) return launch_gemv_rs<ET, 2, 8>(g, pro, tokens, st);
     return launch_gemv_rs<ET, 2, 4>(g, pro, tokens, st);
 }

@@ -504,10 +504,14 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 // prologue while that is cheap, else the norms have a launch of their own (5 us) ahead of one pass over the weights.
 // Rows of at most 4 KiB, a piece per thread, are cheap up to four tokens: 16 layers of 2048, bfloat16, three tokens 945 us against 1107
 // (with a recurrence in every second layer 1208 and 1370), four 1013 and 1114 (1349 and 1480), six 1243 and 1203.
-// Longer rows and more tokens while the bytes read again are few.  Four layers of 4096, two tokens: 952 us with the former everywhere,
-// 874 with the latter; three tokens 671 and 588.
+// Longer rows and more tokens while the bytes read again are few.  A mixture of 8 layers of 2048 in float32, four tokens, 4161 rows
+// (97 MiB) read again or not: 1369 and 1404 us; five tokens (130 MiB) 1655 and 1686; 16 layers of 2048 in float32, two tokens, 16384 rows (128
+// MiB): 1541 and 1453, five, 3072 rows (96 MiB): 1680 and 1750.  Four layers of 4096 in bfloat16, two tokens, 28672 rows (224 MiB): 633 and 579,
+// in float32 (16 KiB), four tokens, up to 240 MiB: 1224 and 1175.
 static bool short_rows(int kpad, int es) { return kpad * es <= 4096; }
-static bool reads_again(int T, int n, int kpad, int es) { return T == 1 || (T <= 4 && short_rows(kpad, es)) || (size_t)(T - 1) * n * kpad * es <= ((size_t)72 << 20); }
+static bool reads_again(int T, int n, int kpad, int es) {
+    return T == 1 || (T <= 4 && short_rows(kpad, es)) || (size_t)(T - 1) * n * kpad * es <= (size_t)(kpad * es > 8192 ? 72 : T == 2 ? 104 : 240) << 20;
+}
 
 // ---- one to kSmallTokens tokens, behind which there are at most `held` ------------------------------------------------
 struct Pending { bool on = false; const float* gb = nullptr; int parts = 1; };      // the last sublayer's output in y (in parts) still has to be added
