@@ -22,6 +22,7 @@ struct GemmArgs {
     const int* row_src = nullptr;
     const int4* tiles = nullptr; const int* n_tiles = nullptr; int max_tiles = 0;
     size_t w_stride = 0;
+    int group_rows = 0;                                   // rows that a group has on average
     int parts = 1; size_t part_stride = 0;                // n_split 0 only: k in `parts` parts, whose sums leave part_stride apart in y32
 };
 template <typename ET> int gemm_float(const GemmArgs& g, hipStream_t st);

@@ -386,13 +386,16 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
 
 // Experts: their weights are read once and little else, so the tiles keep as many bytes in flight as LDS holds (64 experts of
 // 2048 x 2048 and 2048 x 1024, 1024 tokens, top 6: 134 us on average with two stages in four waves, 122 with four in eight;
-// the weights alone are 73 us at 5.5 TB/s).
+// the weights alone are 73 us at 5.5 TB/s).  With fewer than 45 rows per expert most of a wide tile's rows are none, and three workgroups per
+// CU on 64 x 64 hide more of each other's trips (the mixture's whole prompt of 9 rows 1711 -> 1666 us, 333 rows 2743 -> 2669, 450 rows
+// 2830 -> 2772; 500 rows, 47 per expert, 2841 and 2850, 600 rows 3093 and 3143).
 template <int BM>
 static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
     if constexpr (BM == 128) return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
+    else if (g.group_rows < 45) return launch_dma<bf16_t, 64, 64, 3, 3, 4>(g, st);
     else return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
 }
 

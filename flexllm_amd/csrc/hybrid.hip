@@ -754,11 +754,11 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         if (max_tiles > T * top) max_tiles = T * top;
         g = gemm(m->lh, kw, L.w_gu, T * top, 2 * L.d.ff, W);
         g.n_split = 2 * L.d.ff; g.glu = 1 + L.d.glu; g.limit = L.d.limit; g.y = m->lhid; g.ldy = kf;
-        g.row_src = m->lrow_src; g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)2 * L.d.ff * kw;
+        g.row_src = m->lrow_src; g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)2 * L.d.ff * kw; g.group_rows = T * top / L.d.experts;
         FX_TRY(gemm_grouped<ET>(g, tile, st));
         g = gemm(m->lhid, kf, L.w_d, T * top, W, L.d.ff);
         g.n_split = 0; g.y32 = m->lys; g.ldy32 = W;
-        g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)W * kf;
+        g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)W * kf; g.group_rows = T * top / L.d.experts;
         FX_TRY(gemm_grouped<ET>(g, tile, st));
         if (sf) {
             FX_TRY(to_y(m->lhs, ks, L.w_sd, sf));
