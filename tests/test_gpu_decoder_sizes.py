@@ -24,15 +24,15 @@ def logits(model, toks, cuts, max_pos=512):
     return np.concatenate(out)
 
 
-def check(cls, w, toks, want, cfg, dtype, cuts, max_pos, skip=0.0):
-    """skip: share of the places that a close call of a router may leave out."""
+def check(cls, w, toks, want, cfg, dtype, cuts, max_pos, close=()):
+    """close: places where a router's choice may fall either way; they have to be finite, no more."""
+    clear = np.setdiff1d(np.arange(len(toks)), close)
     m = cls.from_tensors(cfg, w, dtype=dtype, max_pos=max_pos)
     for c in cuts:
         got = logits(m, toks, c)
         assert np.isfinite(got).all(), c
         err = lc.rel_err(got, want)
-        worst = np.sort(err)[:len(err) - int(skip * len(err))].max()
-        assert worst < lc.LIMIT[dtype], "portions %s: error %.3g (all places: %.3g at %d)" % (c, worst, err.max(), err.argmax())
+        assert err[clear].max() < lc.LIMIT[dtype], "portions %s: error %.3g at %d" % (c, err[clear].max(), clear[err[clear].argmax()])
     m.close()
 
 
@@ -42,10 +42,27 @@ def check_lopazen(cfg, dtype, n, *cuts, max_pos=512):
     check(Lopazen, w, toks, lopazen_ref.Reference(cfg, w).run(toks), cfg, dtype, cuts, max_pos)
 
 
-def check_nifunex(cfg, dtype, n, *cuts, max_pos=512, skip=0.0):
+# Router outputs are of size 2 and in bfloat16 off by up to a 100th of that: a choice is clear when the last one taken is further than this
+# ahead of the first one left.
+CLOSE = 0.04
+
+
+def check_nifunex(cfg, dtype, n, *cuts, max_pos=512):
     from flexllm_amd.nifunex import Nifunex
     w, toks = nc.weights(cfg, 11), nc.tokens(cfg, n)
-    check(Nifunex, w, toks, nifunex_ref.Reference(cfg, w).run(toks), cfg, dtype, cuts, max_pos, skip if dtype == "bfloat16" else 0.0)
+    lead, route = [], nifunex_ref.route
+
+    def noted(z, top):
+        s = np.sort(z)[::-1]
+        lead.append(s[top - 1] - s[top] if top < len(s) else np.inf)
+        return route(z, top)
+
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(nifunex_ref, "route", noted)
+        want = nifunex_ref.Reference(cfg, w).run(toks)
+    close = np.nonzero((np.reshape(lead, (-1, n)) < CLOSE).any(0))[0] if dtype == "bfloat16" and lead else ()
+    assert len(close) < max(n // 4, 2)
+    check(Nifunex, w, toks, want, cfg, dtype, cuts, max_pos, close)
 
 
 # rows and lengths of the one-token linears: rows per group and pieces per thread change with both
@@ -95,12 +112,12 @@ def test_gemm_tiles(m, n, split, glu, k, dtype):
         assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * np.abs(want[:, split:]) + d)
 
 
-# grouped products of the experts: tiles of 64 and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
+# grouped products of the experts: tiles of 64 rows, narrow and wide ones, and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
 @BOTH
-@pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70)])
+@pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70), (4, 2, 100, 130), (2, 1, 40, 130)])
 def test_grouped_tiles(experts, top, ff, tokens, dtype):
     cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=192)
-    check_nifunex(cfg, dtype, tokens, [tokens], skip=0.05)
+    check_nifunex(cfg, dtype, tokens, [tokens])
 
 
 # prompts of few rows, whose down and output projections share k out: no row tile filled, one and two of them, parts of uneven lengths,
@@ -109,7 +126,7 @@ def test_grouped_tiles(experts, top, ff, tokens, dtype):
 @pytest.mark.parametrize("tokens,ff", [(9, 2048), (65, 1100), (130, 4200)])
 def test_shared_out_k(tokens, ff, dtype):
     check_lopazen(lc.config([lc.layer(heads=12, kv_heads=3, dim=64, mlp=lc.dense(ff)), lc.layer()], width=192), dtype, tokens, [tokens])
-    check_nifunex(nc.config([nc.gla(heads=9, dim=32, vdim=64, mlp=nc.dense(ff)), nc.gla(heads=1, mlp=nc.moe(4, 2, 72, 1.5, ff))], width=192), dtype, tokens, [tokens], skip=0.05)
+    check_nifunex(nc.config([nc.gla(heads=9, dim=32, vdim=64, mlp=nc.dense(ff)), nc.gla(heads=1, mlp=nc.moe(4, 2, 72, 1.5, ff))], width=192), dtype, tokens, [tokens])
 
 
 @BOTH
@@ -131,7 +148,7 @@ def test_step_of_several_tokens(width, ff, dtype):
 
 @BOTH
 def test_step_of_several_tokens_nifunex(dtype):
-    check_nifunex(nc.mixed(), dtype, 35, [2, 3, 4, 5, 6, 7, 8], skip=0.05)
+    check_nifunex(nc.mixed(), dtype, 35, [2, 3, 4, 5, 6, 7, 8])
 
 
 # the experts' down projections of a step: fewer pieces than threads, more than one pass of them, a last pass that is ragged, units that
@@ -140,7 +157,7 @@ def test_step_of_several_tokens_nifunex(dtype):
 @pytest.mark.parametrize("top,ff,shared,width", [(1, 8, 0, 66), (2, 41, 56, 90), (3, 40, 57, 130), (6, 1024, 2048, 160), (4, 2100, 0, 70), (5, 822, 410, 64)])
 def test_experts_down(top, ff, shared, width, dtype):
     cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(top + 1, top, ff, 1.5, shared)), nc.gla(heads=1, mlp=nc.dense(72))], width=width)
-    check_nifunex(cfg, dtype, 20, [1], [3], skip=0.1)
+    check_nifunex(cfg, dtype, 20, [1], [3])
 
 
 @BOTH

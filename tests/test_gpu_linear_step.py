@@ -67,3 +67,50 @@ def test_infinity_in_the_last_piece(k, tokens, dtype):
     w = lc.round_bf16(r.standard_normal((37, k)))
     x[:, k - 1] = np.inf
     assert np.array_equal(step(x, w, dtype)[0], np.broadcast_to(np.inf * w[:, k - 1], (tokens, 37)))
+
+
+@BOTH
+@pytest.mark.parametrize("tokens", range(1, 9))
+@pytest.mark.parametrize("k,n,split", [(1000, 37, 12), (2048, 130, 128), (2112, 131, 0), (4160, 67, 67), (8256, 45, 32)])
+def test_columns_of_both_outputs(k, n, split, tokens, dtype):
+    """A bias, columns in the first output, in the second, in both; rows that do not fill a group or a tile; every number of tokens per pass."""
+    from flexllm_amd import to_device
+    r = np.random.default_rng(k + tokens)
+    x, bias = r.standard_normal((tokens, k)).astype(np.float32), r.standard_normal(n).astype(np.float32)
+    w = lc.round_bf16(r.standard_normal((n, k)))
+    y, y32 = step(x, w, dtype, n_split=split, bias=to_device(bias))
+    got = np.concatenate([a for a in (y, y32) if a is not None], 1)
+    one = lambda a: np.concatenate([a, np.ones((len(a), 1))], 1)      # the bias is one product more
+    near(got, one(x), np.concatenate([w, bias[:, None]], 1))
+
+
+@BOTH
+@pytest.mark.parametrize("glu", [1, 2])
+@pytest.mark.parametrize("tokens", range(1, 9))
+@pytest.mark.parametrize("k,n,split", [(1000, 38, 38), (2048, 131, 128), (4160, 67, 66), (8256, 46, 32)])
+def test_gated_unit(k, n, split, tokens, glu, dtype):
+    """The unit of neighbouring rows in the epilogue: both rows of a pair lie in one group, whatever the rows' length."""
+    from oracle import lopazen_ref, nifunex_ref
+    r = np.random.default_rng(k + tokens)
+    x = r.standard_normal((tokens, k)).astype(np.float32)
+    w = lc.round_bf16(r.standard_normal((n, k)) * k ** -0.5)
+    y, y32 = step(x, w, dtype, n_split=split, glu=glu, limit=3.0)
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    z, d = x @ w.T, EPS * (np.abs(x) @ np.abs(w).T)
+    g, u, dg, du = [a[:, i:split:2] for a in (z, d) for i in (0, 1)]
+    want = nifunex_ref.clamped_glu(g, u, 3.0) if glu == 1 else lopazen_ref.gelu(g) * u
+    # act(g) u has slopes of at most 1.2 (|u| + 1) in g and |g| in u; the function itself is good to 1e-6 of its arguments
+    slope_g, slope_u = 1.2 * (np.abs(u) + 1), np.abs(g) + 0.2
+    assert np.all(np.abs(y - want) <= slope_g * (dg + 1e-6 * np.abs(g)) + slope_u * (du + 1e-6 * np.abs(u)))
+    if split < n:
+        assert np.all(np.abs(y32 - z[:, split:]) <= d[:, split:])
+
+
+@pytest.mark.parametrize("tokens", range(2, 9))
+@pytest.mark.parametrize("k,parts", [(2048, 2), (2112, 2), (4160, 3), (8192, 8), (14336, 7), (8200, 5)])
+def test_parts_of_k(k, parts, tokens):
+    """Sums over parts of k, the last one of any length, add up to the product."""
+    r = np.random.default_rng(k + tokens)
+    x = r.standard_normal((tokens, k)).astype(np.float32)
+    w = lc.round_bf16(r.standard_normal((45, k)))
+    near(step(x, w, "bfloat16", n_split=0, parts=parts)[1].astype(np.float64).sum(0), x, w)
