@@ -190,8 +190,7 @@ __global__ __launch_bounds__(256) void gemm_i8_kernel(const int8_t* __restrict__
 
 // ---------------------------------------------------------------------------------------------------------
 // Second kernel: tiles go global -> LDS by direct loads (global_load_lds_dwordx4), bypassing registers, two to four
-// stages deep.  Tile BM x BN, BKB = 64 or 128 k-bytes per row and stage, four waves (2x2) or eight (2x4, or two
-// k-groups of 2x2); the wave tile is a grid of 32x32 MFMA tiles, and the wider it is the more MFMAs every fragment
+// stages deep.  Tile BM x BN, BKB = 64 or 128 k-bytes per row and stage, four waves (2x2) or eight (2x4); the wave tile is a grid of 32x32 MFMA tiles, and the wider it is the more MFMAs every fragment
 // read from LDS feeds (a 128x64 wave tile: six reads for eight MFMAs).
 //
 // LDS stage layout: row-major, BKB bytes (= BKB/16 16-byte k-chunks) per tile row.  A direct load writes lane i
@@ -210,9 +209,9 @@ __host__ __device__ constexpr int gemm_dma_lds_bytes(int bm, int bn, int stages,
     return ring > epi ? ring : epi;
 }
 
-// Arguments of the q/k/v epilogue: the 64-column tile of the fused [q | k | v] projection is one attention head,
+// Arguments of the q/k/v epilogue: 64 columns of the fused [q | k | v] projection are one attention head, a tile holds whole heads,
 // so RoPE (pairs k, k+32), the static int8 quantisation and the store into q8 / the K cache / the transposed V
-// cache blocks all happen on the tile (64 tokens x 64 channels; a V cache block is 64 positions x 64 channels).
+// cache blocks all happen on the tile, 64 tokens x 64 channels at a time (a V cache block is 64 positions x 64 channels).
 struct QkvEpiArgs {
     const float *sin_t = nullptr, *cos_t = nullptr, *q_s = nullptr, *k_s = nullptr, *v_s = nullptr;
     int8_t *q8 = nullptr, *kc = nullptr, *vc = nullptr;

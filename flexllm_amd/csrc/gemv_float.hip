@@ -400,7 +400,8 @@ template <typename ET, int R, int S>
 static int gemv_tokens_rs(const GemvArgs& g, int tokens, hipStream_t st) {
     const int fit = (int)(kGemvTokensLds / ((g.kpad + Chunk<ET>::N) * sizeof(float))), most = fit < 32 / R ? fit : 32 / R;
     const int cap = most >= 8 ? 8 : most >= 6 ? 6 : most >= 4 ? 4 : 2, groups = (tokens + cap - 1) / cap, tt = (tokens + groups - 1) / groups;
-    if constexpr (R <= 4) if (tt > 6) return launch_gemv_tokens<ET, 8, R, S>(g, tokens, st);
+    // rows that the others are called with are too long for eight vectors
+    if constexpr (std::is_same<ET, float>::value && R > 1) if (tt > 6) return launch_gemv_tokens<ET, 8, R, S>(g, tokens, st);
     if (tt > 4) return launch_gemv_tokens<ET, 6, R, S>(g, tokens, st);
     if (tt > 2) return launch_gemv_tokens<ET, 4, R, S>(g, tokens, st);
     return launch_gemv_tokens<ET, 2, R, S>(g, tokens, st);
@@ -409,8 +410,10 @@ static int gemv_tokens_rs(const GemvArgs& g, int tokens, hipStream_t st) {
 template <typename ET>
 static int gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
     const int per = 256 * Chunk<ET>::N, steps = (g.kpad + per - 1) / per;
-    if (steps == 1) return gemv_tokens_rs<ET, 4, 1>(g, tokens, st);
-    if (steps == 2) return gemv_tokens_rs<ET, 2, 2>(g, tokens, st);
+    if constexpr (std::is_same<ET, float>::value) {       // bfloat16: beyond what gemv_mfma_kernel takes, more than two pieces
+        if (steps == 1) return gemv_tokens_rs<ET, 4, 1>(g, tokens, st);
+        if (steps == 2) return gemv_tokens_rs<ET, 2, 2>(g, tokens, st);
+    }
     if (steps <= 4 || g.glu) return gemv_tokens_rs<ET, 2, 4>(g, tokens, st);      // a pair of the gated unit lies in one group
     return gemv_tokens_rs<ET, 1, 8>(g, tokens, st);
 }

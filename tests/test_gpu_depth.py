@@ -372,7 +372,7 @@ def test_repeated_runs_are_identical_to_the_byte(two_layer, top_k):
 
 # ---------------------------------------------------------------------------------------------------------------
 # The 1024-token prefill of the full-size model: the size at which the launcher picks the 256x256 gate/up tile, the
-# two-k-group down tile and the eight-wave attention with four key tiles per wave.
+# 64x128 down tile and the eight-wave attention with four key tiles per wave.
 
 def _stage_chain_with_substitution(fx, oracle, cfg, host_w, dev_w, l, x):
     """Layer l of the full-size model on S rows of input x, stage by stage through the module entry points, next to

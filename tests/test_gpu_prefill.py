@@ -25,7 +25,7 @@ def test_gemm_int32_exact(fx, m, k, n):
 
 
 def test_gemm_down_projection_shape(fx, oracle):
-    """1024 x 8192 -> 2048, the shape that takes 64x128 tiles with two k-groups per workgroup: raw int32 and the
+    """1024 x 8192 -> 2048, the down projection of a 1024-token prefill: raw int32 and the
     dequantised + residual epilogue.  float64 BLAS is exact here (|sum| < 2^31)."""
     m, k, n = 1024, 8192, 2048
     a = rng.integers(-128, 128, (m, k)).astype(np.int8)
@@ -41,7 +41,7 @@ def test_gemm_down_projection_shape(fx, oracle):
 
 
 def test_gemm_all_tile_shapes_and_extremes(fx):
-    # 128x128 tiles (>= 512 workgroups), 64x128 and 64x64 paths; saturated operands
+    # one stage of k, from many tiles to few; saturated operands
     for m, k, n in [(1024, 128, 8192), (512, 128, 4096), (256, 128, 256)]:
         a = rng.integers(-128, 128, (m, k)).astype(np.int8)
         w = rng.integers(-128, 128, (n, k)).astype(np.int8)
@@ -53,9 +53,8 @@ def test_gemm_all_tile_shapes_and_extremes(fx):
 
 @pytest.mark.parametrize("m,k,n", [(4096, 2048, 2048), (2048, 128, 4096), (2000, 384, 4100), (3072, 256, 2048), (1024, 2048, 2048)])
 def test_gemm_long_prefill_shapes(fx, oracle, m, k, n):
-    """Shapes with 384..767 tiles of 128x128 (the o projection of a 4096-token prefill, shallow ones, a ragged one):
-    the 128x128 variant with two stages of 128-byte rows; and the o projection of a 1024-token prefill (1024 x 2048 ->
-    2048, the narrow-tile instance the layer graph runs at that length).  Raw int32 and dequantised + residual, float64 BLAS as the
+    """The o projections of a 4096-token and of a 1024-token prefill (1024 x 2048 -> 2048), shallow products of as many
+    tiles, a ragged one.  Raw int32 and dequantised + residual, float64 BLAS as the
     exact reference (|sum| < 2^31)."""
     a = rng.integers(-128, 128, (m, k)).astype(np.int8)
     w = rng.integers(-128, 128, (n, k)).astype(np.int8)
