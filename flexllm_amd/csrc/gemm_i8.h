@@ -577,18 +577,19 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
 // 26.2 us on 256 x 256, 17.1 on 64 x 64.
 // 128 x 128 in four waves with two stages fits twice into a CU (per_cu): 3700 x 2064 x 8576, 493 tiles, 74.6 us in one round of it, 86.2 in
 // two of the one with four stages.  64 x 64 with three stages fits three times: 1536 x 2048 x 2048, 768 tiles, 14.4 us in one
-// round of it, 15.8 on 128 x 128; 393 x 9536 x 128 7.5 us, 9.5 on 128 x 128 twice per CU.
+// round of it, 15.8 on 128 x 128; 393 x 9536 x 128 7.5 us, 9.5 on 128 x 128 twice per CU.  The q/k/v
+// epilogue turns whole heads, for which small tiles are no better: 1024 x 3072 x 2048 stays on 128 x 128.
 // The costs are the ones that lose least over 384 sizes (128-byte rows) and 136 sizes (64-byte rows) of 1 to 4096 rows and 64 to 14336 k: their
 // tiles are 0.6 and 0.2 % from the best ones on average.
 struct GemmI8Tile { int bm, bn, stage, round, per_cu; };
 constexpr GemmI8Tile kGemmI8Tiles[2][7] = {
-    {{256, 256, 108, 2230, 1}, {128, 256, 75, 1130, 1}, {128, 128, 75, 370, 1}, {64, 128, 60, 490, 1}, {64, 64, 28, 410, 1}, {64, 64, 76, 350, 3}, {128, 128, 106, 920, 2}},
+    {{256, 256, 126, 2000, 1}, {128, 256, 81, 1140, 1}, {128, 128, 74, 400, 1}, {64, 128, 60, 410, 1}, {64, 64, 27, 450, 1}, {64, 64, 77, 350, 3}, {128, 128, 112, 950, 2}},
     {{256, 256, 40, 1640, 1}, {128, 256, 29, 1180, 1}, {128, 128, 25, 260, 1}, {64, 128, 18, 390, 1}, {64, 64, 13, 70, 1}, {}, {}}};
 inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
     const bool half = k % 128 != 0;
     long best = 0;
     int pick = -1;
-    for (int i = qkv ? 1 : 0; i < (half ? 5 : qkv ? 6 : 7); i++) {     // the q/k/v epilogue's tile has to fit in LDS, with per_cu of them
+    for (int i = qkv ? 1 : 0; i < (half || qkv ? 5 : 7); i++) {     // the q/k/v epilogue's tile has to fit in LDS, with per_cu of them
         const GemmI8Tile& t = kGemmI8Tiles[half][i];
         const long wgs = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn), slots = 256 * t.per_cu;
         const long cost = (wgs + slots - 1) / slots * (t.stage * (k / (half ? 64 : 128)) + t.round);
@@ -612,12 +613,12 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
     }
     if constexpr (EPI != kDmaQkv) {
         if (pick == 0) return FX_GEMM_TILE(256, 256, 2, 2, 128, 8);
+        if (pick == 5) return FX_GEMM_TILE(64, 64, 3, 3, 128);
         if (pick == 6) return FX_GEMM_TILE(128, 128, 2, 2, 128);
     }
     if (pick == 1) return FX_GEMM_TILE(128, 256, 3, 2, 128, 8);
     if (pick == 2) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
     if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 128, 8);
-    if (pick == 5) return FX_GEMM_TILE(64, 64, 3, 3, 128);
     return FX_GEMM_TILE(64, 64, 4, 2, 128);
 #undef FX_GEMM_TILE
 }

@@ -30,8 +30,8 @@ TWO, THREE = {(128, 128, 2)}, {(64, 64, 3)}
 def test_every_int8_tile_is_under_test():
     assert {tile(*s) for s in gpu.TILES if s[1] % 128 == 0} == ONE | TWO | THREE
     assert {tile(*s) for s in gpu.HALF} == ONE
-    for half, want in ((0, ONE - {(256, 256, 1), (64, 64, 1)} | THREE), (64, ONE - {(256, 256, 1)})):
-        assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV if k % 128 == half} == want
+    for half in (0, 64):
+        assert {tile(m, k, (qh + 2 * kvh) * 64, True) for m, qh, kvh, _, k in gpu.QKV if k % 128 == half} == ONE - {(256, 256, 1)}
 
 
 def test_every_float_tile_is_under_test():
@@ -68,6 +68,7 @@ def test_tiles_that_measured_best():
     assert tile(917, 704, 19348) == tile(1621, 320, 22276) == tile(838, 192, 10668) == (128, 128, 1)
     assert tile(3575, 192, 2548) == tile(260, 64, 3440) == tile(530, 192, 3580) == (64, 64, 1)
     assert tile(1536, 2048, 2048) == tile(2176, 512, 2048) == tile(1536, 512, 2048) == tile(393, 128, 9536) == (64, 64, 3)
+    assert tile(2528, 2048, 16384) == (256, 256, 1) and tile(1024, 2048, 3072, True) == tile(3072, 2048, 3072, True) == (128, 128, 1)
     assert tile(2528, 2048, 8192) == tile(3072, 2048, 2048) == (128, 256, 1)
     assert float_tile(266, 128, 18912, "float32") == (64, 64, 1)
 

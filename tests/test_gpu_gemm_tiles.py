@@ -15,7 +15,7 @@ TILES = [(1024, 128, 16384), (1021, 256, 16380), (1000, 128, 8192), (897, 384, 8
 HALF = [(1021, 320, 16380), (1024, 2112, 16384), (1000, 64, 8192), (897, 320, 8188), (1023, 2112, 3972), (1000, 192, 4096), (961, 64, 1924), (1000, 1088, 2048),
         (1, 64, 4), (100, 448, 1028), (900, 2112, 8188), (900, 2112, 2052)]
 QKV = [(1056, 33, 11, 64, 2048), (640, 96, 32, 0, 2048), (1024, 16, 4, 0, 2048), (1056, 33, 11, 64, 1088), (640, 96, 32, 0, 64), (1024, 16, 4, 0, 320),
-       (96, 8, 2, 64, 192), (1120, 24, 4, 64, 512), (640, 96, 32, 0, 2112), (1024, 16, 4, 0, 2112)]
+       (96, 8, 2, 64, 192), (1120, 24, 4, 64, 512), (640, 96, 32, 0, 2112), (1024, 16, 4, 0, 2112), (96, 8, 2, 64, 256)]
 
 
 @pytest.mark.parametrize("m,k,n", TILES + HALF)
