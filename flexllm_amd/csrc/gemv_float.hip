@@ -444,19 +444,23 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] = k + e < g.k ? x[k + e] : 0.0f;
         }
+        auto split = [&](auto big) {
 #pragma unroll
-        for (int p = 0; p < 3; p++) {
-            bf16x4 b;
+            for (int p = 0; p < 3; p++) {
+                bf16x4 b;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                // what is beyond the largest bfloat16 lies in the rest (a part that rounds to infinity would leave infinity
-                // less infinity); an infinity has no rest
-                const bool finite = isfinite(v[e]);
-                b[e] = (bf16_t)(finite ? fminf(fmaxf(v[e], -kBf16Max), kBf16Max) : v[e]);
-                v[e] = finite ? v[e] - (float)b[e] : 0.0f;
+                for (int e = 0; e < 4; e++) {
+                    // what is beyond the largest bfloat16 lies in the rest (a part that rounds to infinity would leave infinity
+                    // less infinity); an infinity has no rest
+                    const bool finite = !big || isfinite(v[e]);
+                    b[e] = (bf16_t)(big && finite ? fminf(fmaxf(v[e], -kBf16Max), kBf16Max) : v[e]);
+                    v[e] = finite ? v[e] - (float)b[e] : 0.0f;
+                }
+                *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
             }
-            *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
-        }
+        };
+        if (fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) > kBf16Max) split(std::true_type());
+        else split(std::false_type());                    // not a number stays what it is in every part
     }
     const int wk = wave * (KW * 32) + (lane >> 4) * 8;    // this lane's k within the stretch
     const bf16_t* w = static_cast<const bf16_t*>(g.w) + k0 + wk;
