@@ -500,6 +500,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
 #pragma unroll
             for (int p = 2; p >= 0; p--)                  // the small parts first
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf[b][s], *reinterpret_cast<const bf16x8*>(xl + p * group * ROW + s * 64), acc, 0, 0, 0);
+        if (tile + 2 * walkers < tiles) load(b, tile + 2 * walkers);      // ahead of the branches below
 #pragma unroll
         for (int i = 0; i < 4; i++) red[b][wave][((lane >> 4) * 4 + i) * 17 + (lane & 15)] = acc[i];
         __syncthreads();                                  // red alternates with the buffer: one barrier per tile is enough
@@ -521,11 +522,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, 
     };
     for (int tile = walker; tile < tiles; tile += 2 * walkers) {
         process(0, tile);
-        if (tile + 2 * walkers < tiles) load(0, tile + 2 * walkers);
-        if (tile + walkers < tiles) {
-            process(1, tile + walkers);
-            if (tile + 3 * walkers < tiles) load(1, tile + 3 * walkers);
-        }
+        if (tile + walkers < tiles) process(1, tile + walkers);
     }
 }
 
