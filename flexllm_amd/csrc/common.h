@@ -53,6 +53,22 @@ enum ScratchKind { kScratchArgmax = 0, kScratchTopK = 1, kScratchMhaDecode = 2, 
 int stream_scratch(ScratchKind kind, hipStream_t st, size_t bytes, void** out);
 void stream_scratch_release(hipStream_t st);
 
+// Launches of kernels whose workgroups wait for each other and so have to be resident all at once.  Two of them side by side could each
+// hold a part of the chip and wait for the rest of it, so on a device they run one after the other, whatever streams they are
+// launched on: each waits for the event behind the one before.  (Kernels of other kinds end by themselves.)  In a
+// stream that is being captured there is no such order to keep.
+int resident_begin(hipStream_t st, bool& ordered);       // takes the device's turn
+int resident_end(hipStream_t st, bool ordered);
+template <class F>
+int resident_launch(hipStream_t st, F launch) {
+    bool ordered = false;
+    int rc = resident_begin(st, ordered);
+    if (rc) return rc;
+    rc = launch();
+    const int end = resident_end(st, ordered);
+    return rc ? rc : end;
+}
+
 // ---------------------------------------------------------------- cross-lane exchange
 // Value held by lane (lane ^ MASK).  1,2: DPP quad_perm; 8: DPP row rotate by 8; 4: two DPP row shifts, each
 // writing the banks (groups of four lanes) it is right for; 16: ds_swizzle bit mode (no LDS traffic, crossbar

@@ -1,0 +1,70 @@
+// One kernel for whole decode steps of one token (csrc/decode_float.hip): what it is given, and when it can be used.
+#pragma once
+#include "float_ops.h"
+
+namespace fx {
+
+constexpr int kWalkWG = 256;               // workgroups, one per CU: all of them have to be resident at once
+constexpr int kWalkMaxPhases = 512;
+constexpr int kWalkMaxWidth = 4096;
+constexpr size_t kWalkLdsMax = 160 * 1024;
+constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 8, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
+constexpr int kWalkRow = 4096;             // bytes that the rows of all linears are a multiple of
+
+// A linear of the step: n rows of kpad elements, dealt to the workgroups in runs of neighbouring rows (walk_rows).
+struct WalkPhase {
+    const void* w;
+    int n, kpad;
+};
+enum WalkMixer { kWalkSharedKv = 0 };
+struct WalkRun {
+    const float *g1, *g1b, *g2, *g2b;      // norms ahead of and behind (null: none) the two sublayers
+    const float *in_bias, *kv_norm;
+    void* rows;
+    float* inv_rms;
+    int mixer, again, n_in, n_et, k_o, ff, glu;
+    float limit;
+    // shared key/value rows
+    int kv_heads, rep, splits, dim, sink, temp_every, capacity;
+    float scale, temp_coef;
+    // where the words that the workgroups hand to each other lie, in floats from the start of a set
+    unsigned x_in, x_part, x_att, x_y, x_hid, x_y2;
+};
+struct WalkArgs {
+    const WalkRun* runs;
+    const WalkPhase* phases;
+    int n_runs, n_phases;                  // without the head's phase, which is entry n_phases
+    int width, vocab, segs_max;
+    float eps, embed_scale;
+    const bf16_t* embed;
+    const float* g_final;
+    float* words;                          // two sets of `set` floats
+    size_t set;
+    unsigned x_cand;                       // candidates of the arg-max
+    int parity;                            // set of the first token
+    int* err;                              // raised when a wait has timed out
+    int* state;                            // HybridSlot::pos
+    int* token;                            // token fed in; after greedy steps the last one found
+    int* tokens_out;                       // greedy steps: tokens_out[state[1] + step]; null: a single step
+    float* logits;                         // null: not wanted
+    int steps, head;
+    int lds_xs, lds_red;                   // floats
+};
+// Rows r0 .. r1-1 of n belong to workgroup w: pairs of rows stay together.
+__host__ __device__ inline int walk_rows(int n, int w) {
+    const int r = 2 * (int)(((long long)w * ((n + 1) / 2)) / kWalkWG);
+    return r < n ? r : n;
+}
+size_t walk_lds(const WalkArgs& a);        // bytes
+template <typename ET> int walk_launch(const WalkArgs& a, hipStream_t st);
+// Attention over shared key/value rows: splits of the rows per query head (one workgroup each, and at least four columns of the head for
+// each in the join), and the words of a split: the sums, maximum and weight sum.
+inline int walk_splits(int heads, int dim) {
+    int s = 4;
+    while (s < 16 && 2 * s * heads <= kWalkWG && 8 * s <= dim) s *= 2;
+    return s;
+}
+__host__ __device__ constexpr int walk_part(int dim) { return dim + 4; }
+inline bool walk_shared_kv_ok(const SharedKvDims& d) { return (d.dim == 64 || d.dim == 128) && d.dimp == d.dim && 4 * d.heads <= kWalkWG; }
+
+}  // namespace fx

@@ -1,0 +1,766 @@
+// Whole decode steps of one token in one kernel: 256 workgroups, one per CU, stay resident and walk through the linears and
+// the attention of all layers, the head and the choice of the next token.
+//
+// What bounds a step of one token: a layer is a chain of five linears and attentions, each of which needs all of the one before.  As
+// kernels of their own every link costs 3.5 us of launch and ramp beside its stream of weights: 16 layers of 2048, feed-forward 8192, bfloat16, 1531
+// tokens held, take 43 us each for 122 MB (17 us at the rate of a read stream).  Here a link costs an exchange between resident
+// workgroups, 1.3 us behind the slowest of them, and the weights, which do not hang on the activations, are asked for ahead of it: 33 us per
+// layer, 771 -> 615 us per token (four layers of 4096: 535 -> 478; ten layers, six of them twice, float32: 1098 -> 922).
+// Eight of a workgroup's twelve waves ("stream waves") do nothing but walk through the workgroup's rows of all linears.  The other four ("service
+// waves") wait for the vectors, norm them, attend, finish the sums.  They meet at workgroup barriers: the vector is in LDS / the sums
+// are in LDS.  Answers of vector memory return to a wave in order, so a wave that streams could not see a word of another workgroup before its weights.
+//
+// Words between workgroups: a float32 goes past the L2 caches (which do not see each other's lines) to a place of its own per layer run,
+// which holds kUnset until then; readers poll the places themselves, 16 bytes per lane.  There are two sets of places, for tokens in
+// turn: who writes a word of one set puts kUnset back in the other one, whose readers were done a token ago (a token ends with an exchange that all
+// workgroups take part in, or with the kernel).  A result that happens to have kUnset's bits leaves as another NaN.
+// All waits are bounded: a wait that times out raises a flag, everybody then runs to the end without waiting.
+#include "decode_float.h"
+#include <atomic>
+
+namespace fx {
+
+constexpr int kSvcWaves = 4, kSvcT = kSvcWaves * 64, kStrWaves = 8, kWalkT = kSvcT + kStrWaves * 64;
+constexpr unsigned kUnset = 0xFFFFFFFFu;
+constexpr int kWalkSpin = 1 << 20, kWalkErrPeriod = 64;
+constexpr int kQuad = 4096;                               // bytes that a stream wave asks for at a time: 4 x 16 per lane
+
+// Pointers out of tables are global ones: as the generic ones that the compiler takes them for, their loads would count as LDS accesses
+// too, and every wait for LDS would wait for all of them.
+template <typename T> using Global = T __attribute__((address_space(1)));
+template <typename T> __device__ __forceinline__ const Global<T>* global(const T* p) { return (const Global<T>*)p; }
+using RunPtr = const WalkRun __attribute__((address_space(4)))*;       // read-only for the whole launch: scalar loads
+
+__device__ __forceinline__ bool unset(float v) { return (unsigned)__float_as_int(v) == kUnset; }
+
+struct Wait {
+    int* err;
+    bool dead;
+    __device__ __forceinline__ bool give_up(int it) {
+        if (it % kWalkErrPeriod != 0) return false;
+        if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) dead = true;
+        else if (it >= kWalkSpin) { __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); dead = true; }
+        return dead;
+    }
+};
+// N x 16 bytes per lane from base + off[i] (bytes), past the L2
+template <int N>
+__device__ __forceinline__ void load_words(const float* base, const unsigned (&off)[N], f32x4 (&v)[N]) {
+    if constexpr (N == 1) {
+        asm volatile("global_load_dwordx4 %0, %1, %2 sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v[0]) : "v"(off[0]), "s"(base) : "memory");
+    } else if constexpr (N == 2) {
+        asm volatile("global_load_dwordx4 %0, %2, %4 sc1\n\tglobal_load_dwordx4 %1, %3, %4 sc1\n\ts_waitcnt vmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]) : "v"(off[0]), "v"(off[1]), "s"(base) : "memory");
+    } else if constexpr (N == 4) {
+        asm volatile("global_load_dwordx4 %0, %4, %8 sc1\n\tglobal_load_dwordx4 %1, %5, %8 sc1\n\tglobal_load_dwordx4 %2, %6, %8 sc1\n\t"
+                     "global_load_dwordx4 %3, %7, %8 sc1\n\ts_waitcnt vmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base) : "memory");
+    } else {
+        static_assert(N == 8, "words at a time");
+        asm volatile("global_load_dwordx4 %0, %8, %16 sc1\n\tglobal_load_dwordx4 %1, %9, %16 sc1\n\tglobal_load_dwordx4 %2, %10, %16 sc1\n\t"
+                     "global_load_dwordx4 %3, %11, %16 sc1\n\tglobal_load_dwordx4 %4, %12, %16 sc1\n\tglobal_load_dwordx4 %5, %13, %16 sc1\n\t"
+                     "global_load_dwordx4 %6, %14, %16 sc1\n\tglobal_load_dwordx4 %7, %15, %16 sc1\n\ts_waitcnt vmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+                     : "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]), "v"(off[6]), "v"(off[7]), "s"(base) : "memory");
+    }
+}
+// The same, until none of the words is unset; of the last 16 bytes the first LAST words count.
+template <int N, int LAST = 4>
+__device__ __forceinline__ void poll_words(const float* base, const unsigned (&off)[N], bool need, f32x4 (&v)[N], Wait& w) {
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bool ok = !need || w.dead;
+    int it = 0;
+    for (;;) {
+        if (!ok) {
+            load_words<N>(base, off, v);
+            ok = true;
+#pragma unroll
+            for (int i = 0; i < N; i++)
+#pragma unroll
+                for (int e = 0; e < (i == N - 1 ? LAST : 4); e++) ok = ok && !unset(v[i][e]);
+        }
+        if (__builtin_amdgcn_ballot_w64(!ok) == 0) break;
+        if (w.give_up(++it)) break;
+    }
+}
+
+template <int N>
+__device__ __forceinline__ float lanes_sum(float v) {     // over groups of N neighbouring lanes
+    if constexpr (N > 1) v += lane_xor_f<1>(v);
+    if constexpr (N > 2) v += lane_xor_f<2>(v);
+    if constexpr (N > 4) v += lane_xor_f<4>(v);
+    if constexpr (N > 8) v += lane_xor_f<8>(v);
+    if constexpr (N > 16) v += lane_xor_f<16>(v);
+    return v;
+}
+// f for the masks of a butterfly over groups of n neighbouring lanes, n a power of two up to 16
+template <class F>
+__device__ __forceinline__ void group(int n, F f) {
+    f(std::integral_constant<int, 1>());
+    f(std::integral_constant<int, 2>());
+    if (n > 4) f(std::integral_constant<int, 4>());
+    if (n > 8) f(std::integral_constant<int, 8>());
+}
+
+constexpr float kWalkLog2e = 1.44269504088896340736f;
+
+struct WalkLds {                                          // ahead of the vector and the sums
+    __attribute__((aligned(16))) int4 phase[kWalkMaxPhases + 1];       // address of the workgroup's rows, 1 KiB units, [pieces of 64 per row | 8 mod that | barriers]
+    __attribute__((aligned(16))) float q[128];
+    __attribute__((aligned(16))) float kx[128];
+    __attribute__((aligned(16))) float sums[kSvcWaves][128];
+    float m[kSvcWaves], l[kSvcWaves];
+    int met, ready, sent;                                 // service waves' barrier; linears whose vector is there, whose sums have left
+    float norm[2][kSvcWaves];
+    float bestv[2][kSvcWaves];
+    int besti[2][kSvcWaves];
+};
+
+// ---- stream waves ---------------------------------------------------------------------------------------------------
+// A workgroup's rows of a linear are one stretch of memory, dealt to the stream waves in turn in quads of 4 KiB, of which a row is a whole
+// number.  Each wave has a ring of `slots` quads in LDS.  The trip is direct (the compiler does not see it: a wait names how many
+// younger quads are on their way), so a request holds no register and may be made at any time.  When it is made matters: a CU takes
+// 32 KiB of requests or so, then the wave that asks stands still until bytes arrive.  Freed slots are therefore filled at once only from the same
+// linear; what belongs to the next ones is asked for behind the barrier that hands the sums on, beside the exchange.  (With register buffers that the
+// compiler waits for, refilled on the spot, the last products of a linear wait until the next one's first quads are asked for: gate/up of
+// 16384 x 2048 8.7 us behind a full ring, 7.1 so.  Eight waves: with four, one per SIMD, a quad's 100 instructions are not hidden, 13 us.)
+__device__ __forceinline__ void quad_to_lds(const char* base, unsigned voff, unsigned dst) {
+    unsigned saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\t"
+                 "s_mov_b32 m0, %3\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2 nt\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:1024 nt\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:2048 nt\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:3072 nt\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "v"(voff), "s"(base), "s"(dst) : "memory");
+}
+// Until all but the youngest n quads have arrived.
+__device__ __forceinline__ void wait_quads(int n) {
+    switch (n) {
+        case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+        case 1: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+        case 2: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
+        case 3: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
+        case 4: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;
+        case 5: asm volatile("s_waitcnt vmcnt(20)" ::: "memory"); break;
+        case 6: asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(28)" ::: "memory"); break;
+    }
+}
+__device__ __forceinline__ int flag(const int& f) { return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)); }
+template <typename ET>
+__device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, float* red, const char* ring, int slots, int phases, int tokens) {
+    constexpr int CE = Chunk<ET>::N, PL = CE / 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) - kSvcWaves;
+    auto word = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const char* mine = ring + (size_t)wave * slots * kQuad;
+    const unsigned dst = word((int)(unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)mine);
+    // what is asked for next: quad iq of linear ip of token it
+    int ip = 0, it = 0, iq = wave, itotal = word(L.phase[0].z), islot = 0, ahead = 0;       // ahead: quads asked for and not taken in
+    auto base_of = [&](int p) { return reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(L.phase[p].y) << 32) | (unsigned)word(L.phase[p].x)); };
+    const char* ibase = base_of(0);
+    auto settle = [&] {                                   // on to a linear of which this wave has a quad
+        while (iq >= itotal && it < tokens) {
+            iq = wave;
+            if (++ip == phases) { ip = 0; it++; }
+            itotal = word(L.phase[ip].z);
+            ibase = base_of(ip);
+        }
+    };
+    auto ask = [&] {
+        quad_to_lds(ibase, (unsigned)iq * kQuad + lane * 16, dst + islot * kQuad);
+        islot = islot + 1 == slots ? 0 : islot + 1;
+        ahead++;
+        iq += kStrWaves;
+        settle();
+    };
+    settle();
+    // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (without that 624 us per
+    // token where it is 610; nothing asked for between linears: 658).
+    auto calm = [&](int n) {
+        while (flag(L.ready) < n) {
+            if (ahead < slots && it < tokens) {
+                ask();
+                wait_quads(0);
+            } else {
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+    };
+    int slot = 0, n = 0;
+    for (int ct = 0; ct < tokens; ct++)
+        for (int cp = 0; cp < phases; cp++) {
+            const int total = word(L.phase[cp].z), rq = word(L.phase[cp].w), segs = 4 * rq;       // quads, and those of a row
+            int at = wave;                                // place of the quad in its row
+            while (at >= rq) at -= rq;
+            const bool held = kStrWaves % rq == 0;        // the same in all rows
+            float xr[4][CE];
+            auto vector = [&](float (&x)[4][CE], int at) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int q = 0; q < PL; q++) {
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(xs + ((q * segs + 4 * at + i) * 64 + lane) * 4);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) x[i][q * 4 + e] = v[e];
+                    }
+            };
+            auto read = [&](i32x4 (&u)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) u[i] = *reinterpret_cast<const i32x4*>(mine + slot * kQuad + i * 1024 + lane * 16);
+                slot = slot + 1 == slots ? 0 : slot + 1;
+                ahead--;
+            };
+            auto dot = [&](const i32x4 (&u)[4], const float (&x)[4][CE]) {
+                float s[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float wv[CE];
+                    Chunk<ET>::unpack(make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]), wv);
+                    s[i] = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < CE; e++) s[i] = fma_f(wv[e], x[i][e], s[i]);
+                }
+                return (s[0] + s[1]) + (s[2] + s[3]);
+            };
+            auto next = [&] {
+                at += kStrWaves;
+                while (at >= rq) at -= rq;
+            };
+            calm(++n);
+            __syncthreads();                              // the vector is there
+            while (ahead < slots && ip == cp && it == ct) ask();
+            if (wave < total) vector(xr, at);
+            int q = wave;
+            for (; q + kStrWaves < total; q += 2 * kStrWaves) {        // two at a time, which hide each other's latencies
+                wait_quads(ahead - 2);
+                i32x4 u[2][4];
+                read(u[0]);
+                read(u[1]);
+                float v[2];
+                if (held) {
+                    v[0] = dot(u[0], xr);
+                    v[1] = dot(u[1], xr);
+                } else {
+                    float x2[4][CE];
+                    if (q > wave) vector(xr, at);
+                    next();
+                    vector(x2, at);
+                    next();
+                    v[0] = dot(u[0], xr);
+                    v[1] = dot(u[1], x2);
+                }
+                if (ip == cp && it == ct) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
+                    ask();
+                    if (ip == cp && it == ct) ask();
+                }
+                multi_sum_step<2, 1>(v, lane);
+                if (lane < 2) red[q + kStrWaves * lane] = v[0];
+            }
+            if (q < total) {
+                wait_quads(ahead - 1);
+                i32x4 u[4];
+                read(u);
+                if (!held && q > wave) vector(xr, at);
+                const float v = wave_sum(dot(u, xr));
+                if (lane == 0) red[q] = v;
+            }
+            __syncthreads();                              // the sums are there
+        }
+}
+
+// ---- service waves ----------------------------------------------------------------------------------------------------
+template <typename ET, int QW>
+struct Service {
+    static constexpr int CE = Chunk<ET>::N, PL = CE / 4, QE = kQuad / sizeof(ET);      // elements of a quad
+    const WalkArgs& a;
+    WalkLds& L;
+    float *xs, *red;
+    const int t, lane, wave, wg;
+    Wait wait;
+    float *now, *other;                                   // the two sets
+    f32x4 x[QW];                                          // residual: float4 t + 256 i
+    int normed = 0;                                       // L.norm in turn
+    int meetings = 0, ready = 0, sent = 0;
+
+    __device__ __forceinline__ Service(const WalkArgs& a_, WalkLds& L_, float* xs_, float* red_)
+        : a(a_), L(L_), xs(xs_), red(red_), t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {
+        wait.err = a.err;
+        wait.dead = false;
+    }
+    // Barrier of the service waves among themselves: the others may stand still for the sake of their requests.
+    __device__ __forceinline__ void meet() {
+        meetings += kSvcWaves;
+        if (lane == 0) __hip_atomic_fetch_add(&L.met, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        while (__hip_atomic_load(&L.met, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < meetings) {}
+    }
+    __device__ __forceinline__ void say(int& f, int n) {
+        if (t == 0) __hip_atomic_store(&f, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    // to the stream waves: the vector is there; then, behind put(): the sums have left
+    __device__ __forceinline__ void vector_done() {
+        say(L.ready, ++ready);
+        __syncthreads();
+    }
+    __device__ __forceinline__ void sums_done() { say(L.sent, ++sent); }
+    __device__ __forceinline__ void put(unsigned at, float v) {
+        store_past(now + at, unset(v) ? __int_as_float(0x7FC00000) : v);
+        unput(at);
+    }
+    __device__ __forceinline__ void unput(unsigned at) { store_past(other + at, __int_as_float((int)kUnset)); }
+    __device__ __forceinline__ void put_x(int segs, int c, const f32x4& v) {       // float4 c of the vector
+        const int at = PL == 1 ? c : (c & 1) * segs * 64 + (c >> 1);
+        *reinterpret_cast<f32x4*>(xs + 4 * at) = v;
+    }
+    // total of local row r, of rq quads
+    __device__ __forceinline__ float total(int rq, int r) const {
+        const float* p = red + r * rq;
+        float s = p[0];
+        for (int i = 1; i < rq; i++) s += p[i];
+        return s;
+    }
+    // A vector of k words as it is
+    __device__ __forceinline__ void take(unsigned at, int k) {
+        const int n4 = k / 4, segs = k / (CE * 64);
+        auto some = [&](auto n, int c0) {
+            constexpr int N = decltype(n)::value;
+            unsigned off[N];
+            f32x4 v[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) off[i] = 16u * (unsigned)min(c0 + t + kSvcT * i, n4 - 1);
+            poll_words<N>(now + at, off, c0 + wave * 64 < n4, v, wait);
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (c0 + t + kSvcT * i < n4) put_x(segs, c0 + t + kSvcT * i, v[i]);
+        };
+        int c0 = 0;
+        while (n4 - c0 > 4 * kSvcT) { some(std::integral_constant<int, 8>(), c0); c0 += 8 * kSvcT; }
+        if (n4 - c0 > 2 * kSvcT) some(std::integral_constant<int, 4>(), c0);
+        else if (n4 - c0 > kSvcT) some(std::integral_constant<int, 2>(), c0);
+        else if (n4 - c0 > 0) some(std::integral_constant<int, 1>(), c0);
+        vector_done();
+    }
+    // x += y (normed and times gb where there is one) + the embedding of `again`; the vector becomes norm(x) * g.
+    __device__ __forceinline__ void norm(bool have, unsigned at, const float* gb, const float* g, int again_token) {
+        const int n4 = a.width / 4, segs = a.width / (CE * 64);
+        f32x4 gv[QW], gbv[QW];
+        unsigned off[QW];
+#pragma unroll
+        for (int i = 0; i < QW; i++) {
+            const int c = min(t + kSvcT * i, n4 - 1);
+            off[i] = 16u * (unsigned)c;
+            gv[i] = *global(reinterpret_cast<const f32x4*>(g + 4 * c));
+            if (have && gb) gbv[i] = *global(reinterpret_cast<const f32x4*>(gb + 4 * c));
+        }
+        if (have) {
+            f32x4 y[QW];
+            poll_words<QW>(now + at, off, wave * 64 < n4, y, wait);
+            float rs = 0.0f;
+            if (gb) {
+                float ss = 0.0f;
+#pragma unroll
+                for (int i = 0; i < QW; i++)
+                    if (t + kSvcT * i < n4)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) ss = fma_f(y[i][e], y[i][e], ss);
+                rs = root(ss);
+            }
+#pragma unroll
+            for (int i = 0; i < QW; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[i][e] = gb ? x[i][e] + y[i][e] * rs * gbv[i][e] : x[i][e] + y[i][e];
+        }
+        if (again_token >= 0)
+#pragma unroll
+            for (int i = 0; i < QW; i++) x[i] += embedding(again_token, min(t + kSvcT * i, n4 - 1));
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < QW; i++)
+            if (t + kSvcT * i < n4)
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss = fma_f(x[i][e], x[i][e], ss);
+        const float rx = root(ss);
+#pragma unroll
+        for (int i = 0; i < QW; i++) {
+            f32x4 h;
+#pragma unroll
+            for (int e = 0; e < 4; e++) h[e] = x[i][e] * rx * gv[i][e];
+            if (t + kSvcT * i < n4) put_x(segs, t + kSvcT * i, h);
+        }
+        vector_done();
+    }
+    // 1 / rms of a vector of the model's width from the threads' sums of squares
+    __device__ __forceinline__ float root(float ss) {
+        ss = wave_sum(ss);
+        if (lane == 0) L.norm[normed][wave] = ss;
+        meet();
+        const float* n = L.norm[normed];
+        normed ^= 1;
+        return 1.0f / sqrtf(((n[0] + n[1]) + (n[2] + n[3])) / (float)a.width + a.eps);
+    }
+    __device__ __forceinline__ f32x4 embedding(int token, int c) const {
+        const bf16x4 b = *global(reinterpret_cast<const bf16x4*>(a.embed + (size_t)token * a.width + 4 * c));
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = (float)b[e] * a.embed_scale;
+        return v;
+    }
+    __device__ __forceinline__ void embed(int token) {
+#pragma unroll
+        for (int i = 0; i < QW; i++) x[i] = embedding(token, min(t + kSvcT * i, a.width / 4 - 1));
+    }
+
+    // ---- attention over shared key/value rows (see shared_kv_attn.hip): a workgroup takes a split of the rows for one query head;
+    // the heads that share rows are on one die.  (All four heads of a key/value head in one workgroup and four times the splits: 2.9 us
+    // instead of 1.9 for 1531 rows, for the norms and sums of four heads.)  A split has a batch of rows for every group of lanes at
+    // least: up to 256 rows of 64 then need no join, which is 2.4 us.
+    template <int D>
+    __device__ __forceinline__ void shared_kv(RunPtr r, int pos) {
+        constexpr int LPK = D / CE, KS = kSvcT / LPK, U = 4, N = CE, PW = walk_part(D);
+        const int G = r->kv_heads, rep = r->rep, S = r->splits, g = wg % G, idx = wg / G, split = idx / rep, head = g * rep + idx % rep;
+        const int held = pos, per = max(((held + S - 1) / S + KS - 1) / KS * KS, U * KS), ns = max((held + per - 1) / per, 1);
+        const int first = split * per, last = min(held, first + per);
+        const int lc = lane % LPK, ks = wave * (64 / LPK) + lane / LPK, col = lc * CE;
+        const unsigned part = r->x_part + (unsigned)((head * S + split) * PW);
+        if (split < ns && pos < r->capacity) {            // others only take part in the join
+            const bool own = split == 0;
+            const auto* rows = global(static_cast<const ET*>(r->rows)) + (size_t)g * r->capacity * D;
+            const auto* inv = global(r->inv_rms) + (size_t)g * r->capacity;
+            i32x4 ua[U], ub[U];
+            float ra[U], rb[U], wv[N];
+            auto rows_at = [&](int b, int i) { return i == 0 || first + (b * U + i) * KS < last; };
+            auto load = [&](int b, i32x4 (&u)[U], float (&ri)[U]) {
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    if (!rows_at(b, i)) break;
+                    const int key = min(first + (b * U + i) * KS + ks, last - 1);
+                    u[i] = *reinterpret_cast<const Global<i32x4>*>(rows + (size_t)key * D + col);
+                    ri[i] = inv[key];
+                }
+            };
+            const int nb = last > first ? (last - first + U * KS - 1) / (U * KS) : 0;
+            if (nb > 0) load(0, ua, ra);
+#pragma unroll
+            for (int q = 0; q < N; q += 4) {
+                const f32x4 v = *global(reinterpret_cast<const f32x4*>(r->kv_norm + col + q));
+#pragma unroll
+                for (int e = 0; e < 4; e++) wv[q + e] = v[e];
+            }
+            float f = r->scale * kWalkLog2e;
+            if (r->temp_coef != 0.0f) f *= 1.0f + r->temp_coef * logf((float)((pos + 1) / r->temp_every) + 1.0f);
+            if (wave == 0) {                              // the query, and the row of this step, into LDS
+                unsigned off[1];
+                f32x4 v[1];
+                const bool isq = lane < D / 4, isk = own && lane >= D / 4 && lane < D / 2;
+                off[0] = isq ? 4u * (unsigned)(head * D) + 16u * (unsigned)lane : 4u * (unsigned)(r->n_et + g * D) + 16u * (unsigned)(isk ? lane - D / 4 : 0);
+                poll_words<1>(now + r->x_in, off, isq || isk, v, wait);
+                if (isq) *reinterpret_cast<f32x4*>(L.q + 4 * lane) = v[0];
+                if (isk) *reinterpret_cast<f32x4*>(L.kx + 4 * (lane - D / 4)) = v[0];
+            }
+            meet();
+            float qv[N], acc[N], m = -1e30f, l = 0.0f;    // m finite, so that differences stay defined
+            {
+                float ss = 0.0f;
+#pragma unroll
+                for (int q = 0; q < N; q += 4) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(L.q + col + q);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) { qv[q + e] = v[e]; ss = fma_f(v[e], v[e], ss); }
+                }
+                const float s = f / sqrtf(lanes_sum<LPK>(ss) / (float)D + a.eps);
+#pragma unroll
+                for (int e = 0; e < N; e++) { qv[e] *= s * wv[e]; acc[e] = 0.0f; }
+            }
+            auto score = [&](const float (&v)[N]) {
+                float s = 0.0f;
+#pragma unroll
+                for (int e = 0; e < N; e++) s = fma_f(qv[e], v[e], s);
+                return lanes_sum<LPK>(s);
+            };
+            auto take_rows = [&](int b, const i32x4 (&u)[U], const float (&ri)[U]) {
+                float s[U], mx = m;
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    s[i] = -INFINITY;
+                    if (!rows_at(b, i)) continue;
+                    float v[N];
+                    Chunk<ET>::unpack(make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]), v);
+                    const float z = score(v) * ri[i];
+                    if (first + (b * U + i) * KS + ks < last) s[i] = z;
+                    mx = fmaxf(mx, s[i]);
+                }
+                const float al = __builtin_amdgcn_exp2f(m - mx);
+                m = mx;
+                l *= al;
+#pragma unroll
+                for (int e = 0; e < N; e++) acc[e] *= al;
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    if (!rows_at(b, i)) break;
+                    const float p = __builtin_amdgcn_exp2f(s[i] - mx);
+                    l += p;
+                    float v[N];
+                    Chunk<ET>::unpack(make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]), v);
+#pragma unroll
+                    for (int e = 0; e < N; e++) acc[e] = fma_f(p, v[e], acc[e]);
+                }
+            };
+            for (int b = 0; b < nb; b += 2) {
+                if (b + 1 < nb) load(b + 1, ub, rb);
+                take_rows(b, ua, ra);
+                if (b + 1 >= nb) break;
+                if (b + 2 < nb) load(b + 2, ua, ra);
+                take_rows(b + 1, ub, rb);
+            }
+            if (own && wave == 0) {                       // the row of this step: the first group of lanes takes it in, one head's workgroup stores it
+                float v[N], ss = 0.0f;
+#pragma unroll
+                for (int e = 0; e < N; e++) {
+                    v[e] = L.kx[col + e];
+                    ss = fma_f(v[e], v[e], ss);
+                    v[e] = (float)(ET)v[e];               // as a later step reads it
+                }
+                const float ri = 1.0f / sqrtf(lanes_sum<LPK>(ss) / (float)D + a.eps);
+                if (ks == 0 && head == g * rep) {
+                    const size_t row = (size_t)g * r->capacity + pos;
+                    __attribute__((aligned(16))) ET o[N];
+#pragma unroll
+                    for (int e = 0; e < N; e++) o[e] = (ET)v[e];
+                    float* dst = reinterpret_cast<float*>(static_cast<ET*>(r->rows) + row * D + col);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) store_past(dst + i, reinterpret_cast<const float*>(o)[i]);
+                    if (lc == 0) store_past(r->inv_rms + row, ri);
+                }
+                const float z = score(v) * ri, sc = ks == 0 ? z : -INFINITY;
+                const float mx = fmaxf(m, sc), al = __builtin_amdgcn_exp2f(m - mx), p = __builtin_amdgcn_exp2f(sc - mx);
+                m = mx;
+                l = l * al + p;
+#pragma unroll
+                for (int e = 0; e < N; e++) acc[e] = fma_f(p, v[e], acc[e] * al);
+            }
+            // the groups of lanes of a wave meet
+            const float mw = wave_max(m), w = __builtin_amdgcn_exp2f(m - mw), lw = wave_sum(lc == 0 ? l * w : 0.0f);
+            if (lane == 0) { L.m[wave] = mw; L.l[wave] = lw; }
+#pragma unroll
+            for (int e = 0; e < N; e++) acc[e] *= w;
+            constexpr int LEFT = N / (64 / LPK) > 0 ? N / (64 / LPK) : 1;
+            multi_sum_step<N, LPK>(acc, lane);
+            int r0 = 0;
+#pragma unroll
+            for (int mask = LPK, half = N / 2; mask < 64 && half > 0; mask *= 2, half /= 2)
+                if (lane & mask) r0 += half;
+#pragma unroll
+            for (int i = 0; i < LEFT; i++) L.sums[wave][col + r0 + i] = acc[i];
+            meet();
+            // and the waves
+            if (t < D) {
+                const bool sink = ns == 1 && r->sink;
+                float mt = fmaxf(fmaxf(L.m[0], L.m[1]), fmaxf(L.m[2], L.m[3])), v = 0.0f, lt = 0.0f;
+                if (sink) mt = fmaxf(mt, 0.0f);
+#pragma unroll
+                for (int i = 0; i < kSvcWaves; i++) {
+                    const float e = __builtin_amdgcn_exp2f(L.m[i] - mt);
+                    v += e == 0.0f ? 0.0f : L.sums[i][t] * e;
+                    lt = fma_f(L.l[i], e, lt);
+                }
+                if (sink) lt += __builtin_amdgcn_exp2f(-mt);
+                if (ns == 1) {
+                    put(r->x_att + (unsigned)(head * D + t), v / lt);
+                    unput(part + t);
+                    if (t < 2) unput(part + D + t);
+                } else {
+                    put(part + t, v);
+                    if (t == 0) { put(part + D, mt); put(part + D + 1, lt); }
+                }
+            }
+            sums_done();
+        } else if (split < S) {
+            for (int i = t; i < D + 2; i += kSvcT) unput(part + i);
+        }
+        // the join: columns split * cw .. of the head belong to this workgroup; a lane per split and four columns
+        if (ns > 1 && split < S && wave == 0) {
+            const int cw = D / S, s = lane & (S - 1), c4 = lane / S, c = split * cw + 4 * c4;
+            const bool cols = 4 * c4 < cw, mine = cols && s < ns;
+            const unsigned at = 4u * (unsigned)((head * S + (mine ? s : 0)) * PW);
+            unsigned off[2] = {at + 4u * (unsigned)(mine ? c : 0), at + 4u * (unsigned)D};
+            f32x4 v[2];
+            // the words behind the two of the second piece are never set
+            poll_words<2, 2>(now + r->x_part, off, mine, v, wait);
+            const float ms = mine ? v[1][0] : -INFINITY;
+            float mt = ms;
+            group(S, [&](auto k) { mt = fmaxf(mt, lane_xor_f<decltype(k)::value>(mt)); });
+            if (r->sink) mt = fmaxf(mt, 0.0f);
+            const float e = mine ? __builtin_amdgcn_exp2f(ms - mt) : 0.0f;
+            float o[5];
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[i] = e == 0.0f ? 0.0f : v[0][i] * e;
+            o[4] = e == 0.0f ? 0.0f : v[1][1] * e;
+            group(S, [&](auto k) {
+#pragma unroll
+                for (int i = 0; i < 5; i++) o[i] += lane_xor_f<decltype(k)::value>(o[i]);
+            });
+            const float lt = r->sink ? o[4] + __builtin_amdgcn_exp2f(-mt) : o[4];
+            if (cols && s < 4) put(r->x_att + (unsigned)(head * D + c + s), (s == 0 ? o[0] : s == 1 ? o[1] : s == 2 ? o[2] : o[3]) / lt);
+        }
+        sums_done();
+    }
+
+    // ---- one token: returns the next one
+    __device__ __forceinline__ int rows_of(int n, int& r0) const {
+        r0 = walk_rows(n, wg);
+        return walk_rows(n, wg + 1) - r0;
+    }
+    // the sums of a linear of n rows of k leave as they are
+    __device__ __forceinline__ void plain(int n, int k, unsigned at, const float* bias) {
+        int r0;
+        const int rows = rows_of(n, r0);
+        const float b = bias && t < rows ? *global(bias + r0 + t) : 0.0f;      // under the products
+        __syncthreads();                                  // the sums are there
+        for (int j = t; j < rows; j += kSvcT) put(at + (unsigned)(r0 + j), total(k / QE, j) + (j == t ? b : bias ? *global(bias + r0 + j) : 0.0f));
+        sums_done();
+    }
+    __device__ __forceinline__ int step(int token, int pos, bool choose) {
+        const int W = a.width;
+        RunPtr runs = (RunPtr)(uintptr_t)a.runs;
+        embed(token);
+        bool have = false;
+        unsigned y = 0;
+        const float* gb = nullptr;
+        for (int i = 0; i < a.n_runs; i++) {
+            RunPtr r = runs + i;
+            norm(have, y, gb, r->g1, r->again ? token : -1);
+            plain(r->n_in, W, r->x_in, r->in_bias);
+            if (r->dim == 64) shared_kv<64>(r, pos);
+            else shared_kv<128>(r, pos);
+            take(r->x_att, r->k_o);
+            plain(W, r->k_o, r->x_y, nullptr);
+            have = true; y = r->x_y; gb = r->g1b;
+            if (r->ff == 0) continue;
+            norm(true, y, gb, r->g2, -1);
+            __syncthreads();
+            int r0;
+            const int rows = rows_of(2 * r->ff, r0);
+            for (int j = t; j < rows / 2; j += kSvcT)
+                put(r->x_hid + (unsigned)(r0 / 2 + j), glu_f(r->glu, total(W / QE, 2 * j), total(W / QE, 2 * j + 1), r->limit));
+            sums_done();
+            take(r->x_hid, r->ff);
+            plain(W, r->ff, r->x_y2, nullptr);
+            y = r->x_y2; gb = r->g2b;
+        }
+        if (!a.head) return 0;
+        norm(have, y, gb, a.g_final, -1);
+        __syncthreads();
+        int r0;
+        const int rows = rows_of(a.vocab, r0);
+        float best = -INFINITY;
+        int bi = 0x7fffffff;
+        for (int j = t; j < rows; j += kSvcT) {
+            const float v = total(W / QE, j);
+            if (a.logits) a.logits[r0 + j] = v;
+            if (v > best) { best = v; bi = r0 + j; }
+        }
+        sums_done();
+        if (!choose) return 0;
+        auto better = [&](float ov, int oi) {
+            if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+        };
+        auto reduce = [&](int n) {
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) better(__shfl_xor(best, k), __shfl_xor(bi, k));
+            if (lane == 0) { L.bestv[n][wave] = best; L.besti[n][wave] = bi; }
+            meet();
+            best = L.bestv[n][0]; bi = L.besti[n][0];
+#pragma unroll
+            for (int w = 1; w < kSvcWaves; w++) better(L.bestv[n][w], L.besti[n][w]);
+        };
+        __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): what this wave stored in this step has arrived
+        reduce(0);
+        if (t == 0) { put(a.x_cand + 2 * wg, best); put(a.x_cand + 2 * wg + 1, __int_as_float(bi)); }
+        unsigned off[1] = {16u * (unsigned)min(t, kWalkWG / 2 - 1)};
+        f32x4 v[1];
+        poll_words<1>(now + a.x_cand, off, t < kWalkWG / 2, v, wait);
+        best = -INFINITY;
+        bi = 0x7fffffff;
+        if (t < kWalkWG / 2) {
+            better(v[0][0], __float_as_int(v[0][1]));
+            better(v[0][2], __float_as_int(v[0][3]));
+        }
+        reduce(1);
+        return (unsigned)bi < (unsigned)a.vocab ? bi : 0;
+    }
+};
+
+template <typename ET, int QW>
+__global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
+    constexpr int QE = kQuad / sizeof(ET);
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    WalkLds& L = *reinterpret_cast<WalkLds*>(lds);
+    float* xs = reinterpret_cast<float*>(lds + sizeof(WalkLds));
+    float* red = xs + a.lds_xs;
+    const int phases = a.n_phases + (a.head ? 1 : 0);
+    for (int p = threadIdx.x; p < phases; p += kWalkT) {
+        const WalkPhase ph = a.phases[p];
+        const int r0 = walk_rows(ph.n, blockIdx.x), rows = walk_rows(ph.n, blockIdx.x + 1) - r0, rq = ph.kpad / QE;
+        const uintptr_t w = reinterpret_cast<uintptr_t>(static_cast<const ET*>(ph.w) + (size_t)r0 * ph.kpad);
+        L.phase[p] = make_int4((int)(unsigned)w, (int)(unsigned)(w >> 32), rows * rq, rq);
+    }
+    if (threadIdx.x == 0) L.met = L.ready = L.sent = 0;
+    __syncthreads();
+    if (threadIdx.x >= kSvcT) {
+        stream_waves<ET>(L, xs, red, reinterpret_cast<const char*>(red + a.lds_red), slots, phases, a.steps);
+        return;
+    }
+    Service<ET, QW> s(a, L, xs, red);
+    const int pos0 = a.state[0], step0 = a.state[1];
+    int token = a.token[0];
+    if ((unsigned)token >= (unsigned)a.vocab) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.state[3] = 2;
+        token = 0;
+    }
+    for (int i = 0; i < a.steps; i++) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");             // rows that other workgroups stored a token ago
+        const int set = (a.parity + i) & 1;
+        s.now = a.words + set * a.set;
+        s.other = a.words + (1 - set) * a.set;
+        token = s.step(token, pos0 + i, a.tokens_out != nullptr);
+        if (a.tokens_out && blockIdx.x == 0 && threadIdx.x == 0) a.tokens_out[step0 + i] = token;
+    }
+    if (a.tokens_out && blockIdx.x == 0 && threadIdx.x == 0) {
+        a.token[0] = token;
+        a.state[0] = pos0 + a.steps;
+        a.state[1] = step0 + a.steps;
+    }
+}
+
+// What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.
+size_t walk_lds(const WalkArgs& a) { return sizeof(WalkLds) + sizeof(float) * ((size_t)a.lds_xs + a.lds_red); }
+static_assert(kStrWaves * kQuad == kWalkSlotBytes && kQuad == kWalkRow, "a quad per wave");
+
+template <typename ET>
+int walk_launch(const WalkArgs& a, hipStream_t st) {
+    FX_REQUIRE(a.n_phases + 1 <= kWalkMaxPhases && a.width % 512 == 0 && a.width <= kWalkMaxWidth && a.vocab >= kWalkWG && a.steps > 0, "walk: %d linears, width %d, vocabulary %d", a.n_phases, a.width, a.vocab);
+    const size_t used = walk_lds(a);
+    FX_REQUIRE(used + kWalkMinSlots * kWalkSlotBytes <= kWalkLdsMax, "walk: %zu bytes of LDS", used);
+    int slots = (int)((kWalkLdsMax - used) / kWalkSlotBytes);
+    if (slots > kWalkMaxSlots) slots = kWalkMaxSlots;
+    const size_t lds = used + slots * kWalkSlotBytes;
+    auto go = [&](auto* k, std::atomic<bool>& opted_in) {
+        if (!opted_in.load(std::memory_order_acquire)) {
+            FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWalkLdsMax));
+            opted_in.store(true, std::memory_order_release);
+        }
+        k<<<kWalkWG, kWalkT, lds, st>>>(a, slots);
+        FX_LAUNCH_CHECK();
+        return FLEXLLM_OK;
+    };
+    static std::atomic<bool> opted2{false}, opted4{false};
+    return a.width <= 2048 ? go(walk_kernel<ET, 2>, opted2) : go(walk_kernel<ET, 4>, opted4);
+}
+template int walk_launch<bf16_t>(const WalkArgs&, hipStream_t);
+template int walk_launch<float>(const WalkArgs&, hipStream_t);
+
+}  // namespace fx

@@ -10,7 +10,7 @@
 // graph serves every token), more go through the GEMMs in pieces of at most kPieceTokens.  In both, the norm after a
 // sublayer, the residual and the norm before the next one are one step: the sublayer's output is kept "pending" until the
 // next sublayer's first kernel takes it in.
-#include "float_ops.h"
+#include "decode_float.h"
 #include "logits_kernels.h"
 #include <math.h>
 #include <string.h>
@@ -94,6 +94,10 @@ struct flexllm_hybrid {
     int graph_slot = -1, graph_topk = 0, graph_splits = 0;
     const void *graph_io = nullptr, *graph_out = nullptr, *graph_rands = nullptr;
     hipStream_t graph_stream = nullptr;
+    // steps of one token in one kernel (csrc/decode_float.hip); walk.phases null: this model has none
+    fx::WalkArgs walk = {};
+    fx::WalkRun* walk_runs = nullptr;         // [slots][runs]
+    unsigned walk_steps = 0;                  // steps taken so far
 };
 
 namespace fx {
@@ -370,6 +374,80 @@ static int create_layer(flexllm_hybrid* m, int i, const flexllm_hybrid_layer_wei
     return FLEXLLM_OK;
 }
 
+// Steps of one token as one kernel: where the chip and the sizes are those that csrc/decode_float.hip is made for.
+template <typename ET>
+static int create_walk(flexllm_hybrid* m) {
+    const flexllm_hybrid_config& c = m->cfg;
+    const int W = c.width, unit = kWalkRow / sizeof(ET);  // elements that rows are a multiple of
+    int dev = 0, cus = 0;
+    FX_HIP(hipGetDevice(&dev));
+    FX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int few = 2 * kWalkWG;                          // rows of which every workgroup has some
+    bool ok = cus >= kWalkWG && W % unit == 0 && W <= kWalkMaxWidth && c.vocab >= few;
+    for (const HybridLayer& L : m->layers)
+        ok = ok && L.d.mixer == FLEXLLM_MIX_SHARED_KV && walk_shared_kv_ok(L.sd) && L.n_in >= few && L.k_o % unit == 0 &&
+             (L.d.ff_kind == FLEXLLM_FF_NONE || (L.d.ff_kind == FLEXLLM_FF_DENSE && L.d.ff % unit == 0 && 2 * L.d.ff >= few));
+    if (!ok) return FLEXLLM_OK;
+    std::vector<WalkPhase> phases;
+    std::vector<WalkRun> runs;
+    WalkArgs& a = m->walk;
+    size_t at = 0, longest = 0, sums = 0;
+    auto linear = [&](const void* w, int n, int k) {
+        phases.push_back({w, n, k});
+        const size_t rows = 2 * (size_t)(((n + 1) / 2 + kWalkWG - 1) / kWalkWG), s = rows * (k / unit);
+        if ((size_t)k > longest) longest = k;
+        if (s > sums) sums = s;
+    };
+    auto words = [&](size_t n) {
+        const size_t p = at;
+        at += (n + 63) / 64 * 64;
+        return (unsigned)p;
+    };
+    const int n_runs = (int)m->runs.size();
+    for (int slot = 0; slot < c.slots; slot++)
+        for (int i = 0; i < n_runs; i++) {
+            const HybridLayer& L = m->layers[m->runs[i].layer];
+            WalkRun r = {};
+            if (slot > 0) {
+                r = runs[i];
+            } else {
+                r.g1 = L.g1; r.g1b = L.g1b; r.g2 = L.g2; r.g2b = L.g2b; r.in_bias = L.in_bias; r.kv_norm = L.kv_norm;
+                r.mixer = kWalkSharedKv; r.again = m->runs[i].again; r.n_in = L.n_in; r.n_et = L.n_et; r.k_o = L.k_o;
+                r.ff = L.d.ff_kind == FLEXLLM_FF_NONE ? 0 : L.d.ff; r.glu = 1 + L.d.glu; r.limit = L.d.limit;
+                r.kv_heads = L.sd.kv_heads; r.rep = L.sd.heads / L.sd.kv_heads; r.splits = walk_splits(L.sd.heads, L.sd.dim); r.dim = L.sd.dim; r.sink = L.sd.sink; r.temp_every = L.sd.temp_every; r.capacity = L.sd.capacity;
+                r.scale = L.sd.scale; r.temp_coef = L.sd.temp_coef;
+                r.x_in = words(r.n_in); r.x_part = words((size_t)L.sd.heads * r.splits * walk_part(r.dim)); r.x_att = words(r.k_o); r.x_y = words(W);
+                linear(L.w_in, L.n_in, W);
+                linear(L.w_o, W, L.k_o);
+                if (r.ff) {
+                    r.x_hid = words(r.ff); r.x_y2 = words(W);
+                    linear(L.w_gu, 2 * r.ff, W);
+                    linear(L.w_d, W, r.ff);
+                }
+            }
+            r.rows = m->slots[slot].rows[i]; r.inv_rms = m->slots[slot].inv_rms[i];
+            runs.push_back(r);
+        }
+    a.n_phases = (int)phases.size();
+    linear(m->head, c.vocab, W);
+    a.x_cand = words(2 * kWalkWG);
+    a.lds_xs = (int)longest; a.lds_red = (int)((sums + 255) / 256 * 256);
+    if (a.n_phases + 1 > kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || walk_lds(a) + kWalkMinSlots * kWalkSlotBytes > kWalkLdsMax) return FLEXLLM_OK;
+    WalkPhase* dev_phases;
+    FX_TRY(own(m, dev_phases, phases.size()));
+    FX_TRY(own(m, m->walk_runs, runs.size()));
+    FX_HIP(hipMemcpy(dev_phases, phases.data(), sizeof(WalkPhase) * phases.size(), hipMemcpyHostToDevice));
+    FX_HIP(hipMemcpy(m->walk_runs, runs.data(), sizeof(WalkRun) * runs.size(), hipMemcpyHostToDevice));
+    a.set = at;
+    FX_TRY(own(m, a.words, 2 * at));
+    FX_HIP(hipMemset(a.words, 0xFF, 2 * at * sizeof(float)));
+    FX_TRY(own(m, a.err, 1));
+    a.n_runs = n_runs; a.width = W; a.vocab = c.vocab; a.eps = c.eps; a.embed_scale = c.embed_scale;
+    a.embed = as_bf16(m->embed); a.g_final = m->g_final;
+    a.phases = dev_phases;
+    return FLEXLLM_OK;
+}
+
 template <typename ET>
 static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, const flexllm_hybrid_layer_weights* lw) {
     const flexllm_hybrid_config& c = m->cfg;
@@ -439,6 +517,7 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
     FX_TRY(own(m, m->topk_val, kTopKParts * kTopKMax));
     FX_TRY(own(m, m->topk_idx, kTopKParts * kTopKMax));
     FX_TRY(own(m, m->gen_token, 1));
+    FX_TRY(create_walk<ET>(m));
     FX_HIP(hipDeviceSynchronize());
     return FLEXLLM_OK;
 }
@@ -792,6 +871,29 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
     return FLEXLLM_OK;
 }
 
+// Steps of one token each in one launch per kWalkLaunch of them: logits of a single one, or greedy ones (tokens_out).
+constexpr int kWalkLaunch = 64;           // bounds the time of a launch
+static bool walk_ready(const flexllm_hybrid* m, hipStream_t st) {
+    if (!m->walk.phases) return false;
+    // a captured launch would be replayed with the same set of words, and beside the host's order of launches
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+static int walk(flexllm_hybrid* m, int slot, int* token, int steps, int* tokens_out, bool head, float* logits, hipStream_t st) {
+    for (int done = 0; done < steps;) {
+        WalkArgs a = m->walk;
+        a.runs = m->walk_runs + (size_t)slot * a.n_runs;
+        a.state = m->slots[slot].pos;
+        a.token = token; a.tokens_out = tokens_out; a.logits = logits; a.head = head;
+        a.steps = steps - done < kWalkLaunch ? steps - done : kWalkLaunch;
+        a.parity = m->walk_steps & 1;
+        FX_TRY(resident_launch(st, [&] { return m->cfg.dtype == 0 ? walk_launch<bf16_t>(a, st) : walk_launch<float>(a, st); }));
+        m->walk_steps += a.steps;
+        done += a.steps;
+    }
+    return FLEXLLM_OK;
+}
+
 template <typename ET>
 static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const int* want, int n_want, float* logits, float* layers_out, hipStream_t st) {
     HybridSlot& s = m->slots[slot];
@@ -804,7 +906,9 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
         int w1 = w0;
         while (w1 < n_want && want[w1] < t0 + T) part.push_back(want[w1++] - t0);
         float* lg = n_want ? logits + (size_t)w0 * m->cfg.vocab : nullptr;
-        if (T <= kSmallTokens && (!layers_out || t0 == 0))
+        if (T == 1 && !layers_out && walk_ready(m, st))
+            FX_TRY(walk(m, slot, const_cast<int*>(tokens + t0), 1, nullptr, !part.empty(), lg, st));      // a single step leaves the token alone
+        else if (T <= kSmallTokens && (!layers_out || t0 == 0))
             FX_TRY(run_small<ET>(m, s, tokens + t0, T, s.length + T, part.data(), (int)part.size(), lg, layers_out, st));
         else
             FX_TRY(run_many<ET>(m, s, tokens + t0, T, part.data(), (int)part.size(), lg, layers_out ? layers_out + (size_t)t0 * W : nullptr, (size_t)n * W, st));
@@ -911,7 +1015,9 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
     FX_REQUIRE(!use_graph || st, "hybrid_decode: graph replay needs a non-default stream");
     if (steps == 0) return FLEXLLM_OK;
     FX_TRY(set_state_launch(s.pos, s.length, 0, st));
-    if (!use_graph) {
+    if (top_k == 0 && walk_ready(m, st)) {
+        FX_TRY(walk(m, slot, token_io, steps, tokens_out, true, nullptr, st));
+    } else if (!use_graph) {
         for (int i = 0; i < steps; i++) FX_TRY(decode_any(m, slot, s.length + steps, token_io, rands, top_k, tokens_out, st));
     } else {
         int splits = 0;                                   // of all layers together: none has fewer at more rows
@@ -951,6 +1057,17 @@ int flexllm_hybrid_generate(flexllm_hybrid* m, int slot, const int* prompt, int 
 int flexllm_hybrid_check(flexllm_hybrid* m) {
     FX_REQUIRE(m, "hybrid_check: null pointer");
     FX_HIP(hipDeviceSynchronize());
+    if (m->walk.phases) {
+        int err = 0;
+        FX_HIP(hipMemcpy(&err, m->walk.err, sizeof(err), hipMemcpyDeviceToHost));
+        if (err) {                                        // what the workgroups handed to each other is in no known state
+            FX_HIP(hipMemset(m->walk.words, 0xFF, 2 * m->walk.set * sizeof(float)));
+            FX_HIP(hipMemset(m->walk.err, 0, sizeof(err)));
+            FX_HIP(hipDeviceSynchronize());
+            set_error("decode: a wait timed out (were all %d workgroups resident?)", kWalkWG);
+            return FLEXLLM_EHIP;
+        }
+    }
     for (size_t i = 0; i < m->slots.size(); i++) {
         int st[4] = {0, 0, 0, 0};
         FX_HIP(hipMemcpy(st, m->slots[i].pos, sizeof(st), hipMemcpyDeviceToHost));

@@ -192,10 +192,12 @@ static int launch_mega(flexllm_llama* m, int* token, const float* x_in, float* l
     // An ordinary launch: one workgroup per CU fits by construction (mega_ok checks the CU count), and every barrier
     // and poll in the kernel is bounded, so work of other streams that delays some workgroups costs time, not a hang.
     // (A cooperative launch gives the same timing, but rocprofv3 of this ROCm release crashes at exit after one.)
-    if (m->w4) decode_mega_w4_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
-    else decode_mega_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
-    FX_LAUNCH_CHECK();
-    return FLEXLLM_OK;
+    return resident_launch(st, [&] {
+        if (m->w4) decode_mega_w4_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
+        else decode_mega_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
+        FX_LAUNCH_CHECK();
+        return FLEXLLM_OK;
+    });
 }
 
 static inline bool use_mega(const flexllm_llama* m) { return m->mega_ok && m->decode_mode == 0; }

@@ -60,6 +60,39 @@ void stream_scratch_release(hipStream_t st) {
     }
 }
 
+namespace {
+std::mutex g_resident_mu;
+std::map<int, hipEvent_t> g_resident;                    // per device: behind the last of these launches
+}  // namespace
+
+int resident_begin(hipStream_t st, bool& ordered) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    FX_HIP(hipStreamIsCapturing(st, &cap));
+    ordered = cap == hipStreamCaptureStatusNone;
+    if (!ordered) return FLEXLLM_OK;
+    int dev = 0;
+    FX_HIP(hipGetDevice(&dev));
+    g_resident_mu.lock();                                // the order of launches and of their events is one: held until resident_end
+    auto turn = [&] {
+        hipEvent_t& e = g_resident[dev];
+        if (!e) FX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        FX_HIP(hipStreamWaitEvent(st, e, 0));
+        return FLEXLLM_OK;
+    };
+    const int rc = turn();
+    if (rc) { ordered = false; g_resident_mu.unlock(); }
+    return rc;
+}
+int resident_end(hipStream_t st, bool ordered) {
+    if (!ordered) return FLEXLLM_OK;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipEventRecord(g_resident[dev], st);
+    g_resident_mu.unlock();
+    FX_HIP(e);
+    return FLEXLLM_OK;
+}
+
 // SplitMix64 of (seed, index): the same sequence as flexllm_amd.synth.splitmix64 on the host.
 __host__ __device__ inline uint64_t splitmix64(uint64_t seed, uint64_t idx) {
     uint64_t z = seed + (idx + 1) * 0x9E3779B97F4A7C15ull;

@@ -1,0 +1,126 @@
+"""Steps of one token as one kernel: models whose sizes it takes, against the plain statement of their equations, token by token and in
+loops of several tokens per launch, with one and several splits of the rows."""
+import numpy as np
+import pytest
+
+import lopazen_cases as lc
+from oracle import lopazen_ref
+from test_gpu_decoder_sizes import check_lopazen
+
+pytestmark = pytest.mark.gpu
+BOTH = pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+
+
+def attention(heads, kv_heads, dim, ff, coef=0.4):
+    return lc.layer(heads=heads, kv_heads=kv_heads, dim=dim, scale=dim ** -0.5, coef=coef, mlp=lc.dense(ff) if ff else None)
+
+
+# rows of one quad and of several, whole numbers of a wave's share and not (14336), the smallest vocabulary, an odd one; heads that share rows
+# in fours, in eights, alone, and in threes; no feed-forward; loops
+LOPAZEN = {
+    "rows of a quad": lc.config([attention(32, 8, 64, 2048), attention(32, 8, 64, 2048)], width=2048, vocab=512),
+    "rows of seven quads": lc.config([attention(32, 8, 64, 14336)], width=2048, vocab=517),
+    "long heads": lc.config([attention(16, 2, 128, 4096)], width=4096, vocab=600),
+    "as many key heads": lc.config([attention(32, 32, 64, 0)], width=2048, vocab=1001),
+    "heads in threes": lc.config([attention(48, 16, 128, 2048, coef=0.0)], width=2048, vocab=700),
+    "a loop": lc.config([attention(32, 8, 64, 2048), attention(16, 4, 128, 0)], width=2048, vocab=515, loop=(0, 2, 2)),
+}
+
+
+@BOTH
+@pytest.mark.parametrize("name", list(LOPAZEN))
+def test_token_by_token(name, dtype):
+    check_lopazen(LOPAZEN[name], dtype, 40, [1], [23, 1])
+
+
+@BOTH
+@pytest.mark.parametrize("dim", [64, 128])
+def test_splits_of_the_rows(dim, dtype):
+    """Around the number of rows from which on there are several splits, and where all of them have some."""
+    borders = {64: (64, 256), 128: (32, 128)}[dim]
+    for rows in {"bfloat16": borders[1], "float32": borders[1] // 2}[dtype], 8 * borders[1]:
+        check_lopazen(lc.config([attention(32, 8, dim, 0)], width=2048, vocab=512), dtype, rows + 5, [rows - 5, 1], max_pos=2112)
+
+
+@BOTH
+def test_loop_of_tokens(dtype):
+    """70 greedy tokens (two launches) are those of 70 steps, in two slots in turn, continued by a step and by another loop."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd.lopazen import Lopazen
+    cfg = LOPAZEN["a loop"]
+    w, toks = lc.weights(cfg, 5), lc.tokens(cfg, 30)
+    ref = lopazen_ref.Reference(cfg, w)
+    m = Lopazen.from_tensors(cfg, w, dtype=dtype, max_pos=256, slots=2)
+    slots = [m.pool.acquire(n) for n in "ab"]
+    for s in slots:
+        m.step(s, toks[:29])
+    got, want, token = [], toks[29:], to_device(np.array(toks[29:], np.int32))
+    for n in (1, 2, 67):
+        out = zeros((n,), np.int32)
+        m.decode(slots[0], token, n, out)
+        got += out.numpy().tolist()
+        assert token.numpy()[0] == got[-1]
+        for _ in range(n):
+            want.append(int(m.step(slots[1], want[-1:], [0])[0].argmax()))
+    m.check()
+    assert got == want[1:] and m.length(slots[0]) == m.length(slots[1]) == 99
+    last = [m.step(s, got[-1:], [0]) for s in slots]
+    assert np.array_equal(last[0], last[1])
+    err = lc.rel_err(last[0], ref.run(toks + got)[-1:])
+    assert err.max() < lc.LIMIT[dtype]
+    m.close()
+
+
+def test_tokens_outside_the_vocabulary():
+    """are reported, and taken as token 0."""
+    from flexllm_amd._lib import FlexLLMError
+    from flexllm_amd.lopazen import Lopazen
+    cfg = LOPAZEN["rows of a quad"]
+    m = Lopazen.from_tensors(cfg, lc.weights(cfg, 5), dtype="bfloat16", max_pos=64)
+    out = []
+    for t in (512, 0):
+        s = m.pool.acquire("t")
+        out.append(m.step(s, [t], [0]))
+        if t:
+            with pytest.raises(FlexLLMError, match="vocabulary"):
+                m.check()
+        m.pool.release("t")
+    m.close()
+    assert np.array_equal(*out)
+
+
+def test_infinities_and_not_a_number():
+    """An infinite row of a weight is an infinity (or, against both signs, not a number) in that place alone."""
+    from flexllm_amd.lopazen import Lopazen
+    cfg = LOPAZEN["as many key heads"]
+    w = lc.weights(cfg, 5)
+    w["embed"] = w["embed"].copy()
+    m = Lopazen.from_tensors(cfg, w, dtype="float32", max_pos=64)
+    clean = m.generate(lc.tokens(cfg, 5), 3)
+    m.close()
+    w["embed"][900, 7] = np.inf                            # the head is the embedding: one logit
+    m = Lopazen.from_tensors(cfg, w, dtype="float32", max_pos=64)
+    s = m.pool.acquire("t")
+    got = m.step(s, lc.tokens(cfg, 1), [0])[0]
+    m.close()
+    assert np.isinf(got[900]) and np.isfinite(np.delete(got, 900)).all() and len(clean) == 3
+
+
+def test_two_models_on_streams_of_their_own():
+    """Each launch needs the whole chip: they run one after the other, whatever streams they are on and threads they come from."""
+    import threading
+    from flexllm_amd.lopazen import Lopazen
+    cfg = LOPAZEN["rows of a quad"]
+    w, prompt = lc.weights(cfg, 5), lc.tokens(cfg, 12)
+    models = [Lopazen.from_tensors(cfg, w, dtype="bfloat16", max_pos=256) for _ in range(2)]
+    want = models[0].generate(prompt, 30)
+    got = {}
+
+    def work(i):
+        got[i] = [models[i].generate(prompt, 30) for _ in range(10)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert got == {i: [want] * 10 for i in range(2)}
+    [m.close() for m in models]
