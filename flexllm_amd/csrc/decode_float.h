@@ -5,6 +5,7 @@
 namespace fx {
 
 constexpr int kWalkWG = 256;               // workgroups, one per CU: all of them have to be resident at once
+constexpr int kWalkCopies = 8;            // of few words that every workgroup reads
 constexpr int kWalkMaxPhases = 512;
 constexpr int kWalkMaxWidth = 4096;
 constexpr size_t kWalkLdsMax = 160 * 1024;
@@ -16,7 +17,7 @@ struct WalkPhase {
     const void* w;
     int n, kpad;
 };
-enum WalkMixer { kWalkSharedKv = 0 };
+enum WalkMixer { kWalkSharedKv = 0, kWalkLatent = 1, kWalkGla = 2 };
 struct WalkRun {
     const float *g1, *g1b, *g2, *g2b;      // norms ahead of and behind (null: none) the two sublayers
     const float *in_bias, *kv_norm;
@@ -25,16 +26,27 @@ struct WalkRun {
     int mixer, again, n_in, n_et, k_o, ff, glu;
     float limit;
     // shared key/value rows
-    int kv_heads, rep, splits, dim, sink, temp_every, capacity;
+    int heads, kv_heads, rep, splits, dim, sink, temp_every, capacity;     // splits: of the rows, or slices of a head's columns
     float scale, temp_coef;
+    // latent rows
+    const void *uk, *uv;
+    const float *latent_norm, *cos_t, *sin_t;
+    int own_rows, window;                  // 0: the rows of an earlier run
+    // gated linear attention
+    const void* a2;
+    const float *a2_bias, *head_norm;
+    float* state;
+    int a_rank;
+    float tau;
     // where the words that the workgroups hand to each other lie, in floats from the start of a set
-    unsigned x_in, x_part, x_att, x_y, x_hid, x_y2;
+    unsigned x_in, x_ql, x_part, x_att, x_y, x_hid, x_y2;
 };
 struct WalkArgs {
     const WalkRun* runs;
     const WalkPhase* phases;
     int n_runs, n_phases;                  // without the head's phase, which is entry n_phases
-    int width, vocab, segs_max;
+    int kind;                              // mixers: shared key/value rows (kWalkSharedKv), or the others (kWalkLatent)
+    int width, vocab;
     float eps, embed_scale;
     const bf16_t* embed;
     const float* g_final;
@@ -66,5 +78,12 @@ inline int walk_splits(int heads, int dim) {
 }
 __host__ __device__ constexpr int walk_part(int dim) { return dim + 4; }
 inline bool walk_shared_kv_ok(const SharedKvDims& d) { return (d.dim == 64 || d.dim == 128) && d.dimp == d.dim && 4 * d.heads <= kWalkWG; }
+// The other two are made for one size of head: a slice of a head's columns per workgroup, 16 or 8 for each head.
+constexpr int kWalkDim = 128, kWalkRot = 64, kWalkRank = 512, kWalkRow2 = kWalkRank + kWalkRot, kWalkGlaRank = 16;
+inline int walk_slices(int heads) { return heads <= 16 ? 16 : 8; }
+inline bool walk_latent_ok(const LatentDims& d) {
+    return d.dim == kWalkDim && d.vdim == kWalkDim && d.rot_dim == kWalkRot && d.kv_rank == kWalkRank && d.kvp == kWalkRank && d.ldc == kWalkRow2 && d.heads <= 32;
+}
+inline bool walk_gla_ok(const GlaDims& d) { return d.dim == kWalkDim && d.vdim == kWalkDim && d.a_rank <= kWalkGlaRank && d.heads <= 32; }
 
 }  // namespace fx

@@ -107,9 +107,11 @@ constexpr float kWalkLog2e = 1.44269504088896340736f;
 
 struct WalkLds {                                          // ahead of the vector and the sums
     __attribute__((aligned(16))) int4 phase[kWalkMaxPhases + 1];       // address of the workgroup's rows, 1 KiB units, [pieces of 64 per row | 8 mod that | barriers]
-    __attribute__((aligned(16))) float q[128];
-    __attribute__((aligned(16))) float kx[128];
-    __attribute__((aligned(16))) float sums[kSvcWaves][128];
+    __attribute__((aligned(16))) float q[kWalkRow2];      // query; of gated linear attention query, key, decay, and what is short
+    __attribute__((aligned(16))) float kx[kWalkRow2];     // the row of this step
+    __attribute__((aligned(16))) float ql[kWalkRow2];     // latent query
+    __attribute__((aligned(16))) float sums[kSvcWaves][kWalkRank];
+    float of_head[32];
     float m[kSvcWaves], l[kSvcWaves];
     int met, ready, sent;                                 // service waves' barrier; linears whose vector is there, whose sums have left
     float norm[2][kSvcWaves];
@@ -178,18 +180,6 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
         settle();
     };
     settle();
-    // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (without that 624 us per
-    // token where it is 610; nothing asked for between linears: 658).
-    auto calm = [&](int n) {
-        while (flag(L.ready) < n) {
-            if (ahead < slots && it < tokens) {
-                ask();
-                wait_quads(0);
-            } else {
-                __builtin_amdgcn_s_sleep(1);
-            }
-        }
-    };
     int slot = 0, n = 0;
     for (int ct = 0; ct < tokens; ct++)
         for (int cp = 0; cp < phases; cp++) {
@@ -230,16 +220,35 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 at += kStrWaves;
                 while (at >= rq) at -= rq;
             };
-            calm(++n);
+            // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (without that 624 us
+            // per token where it is 610; nothing asked for between linears: 658).  When the ring is full, the first two quads move into registers.
+            i32x4 u[2][4];
+            bool taken = false;
+            n++;
+            while (flag(L.ready) < n) {
+                if (ahead < slots && it < tokens) {
+                    ask();
+                    wait_quads(0);
+                } else if (!taken && ahead >= 2 && wave + kStrWaves < total) {
+                    wait_quads(ahead - 2);
+                    read(u[0]);
+                    read(u[1]);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
+                    taken = true;
+                } else {
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
             __syncthreads();                              // the vector is there
             while (ahead < slots && ip == cp && it == ct) ask();
             if (wave < total) vector(xr, at);
             int q = wave;
             for (; q + kStrWaves < total; q += 2 * kStrWaves) {        // two at a time, which hide each other's latencies
-                wait_quads(ahead - 2);
-                i32x4 u[2][4];
-                read(u[0]);
-                read(u[1]);
+                if (!taken) {
+                    wait_quads(ahead - 2);
+                    read(u[0]);
+                    read(u[1]);
+                }
                 float v[2];
                 if (held) {
                     v[0] = dot(u[0], xr);
@@ -253,28 +262,29 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                     v[0] = dot(u[0], xr);
                     v[1] = dot(u[1], x2);
                 }
-                if (ip == cp && it == ct) {
+                if (!taken) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
-                    ask();
+                    if (ip == cp && it == ct) ask();
                     if (ip == cp && it == ct) ask();
                 }
+                taken = false;
                 multi_sum_step<2, 1>(v, lane);
                 if (lane < 2) red[q + kStrWaves * lane] = v[0];
             }
             if (q < total) {
                 wait_quads(ahead - 1);
-                i32x4 u[4];
-                read(u);
+                read(u[0]);
                 if (!held && q > wave) vector(xr, at);
-                const float v = wave_sum(dot(u, xr));
+                const float v = wave_sum(dot(u[0], xr));
                 if (lane == 0) red[q] = v;
             }
             __syncthreads();                              // the sums are there
+            while (flag(L.sent) < n) __builtin_amdgcn_s_sleep(1);      // they leave first: a store, too, stands in line
         }
 }
 
 // ---- service waves ----------------------------------------------------------------------------------------------------
-template <typename ET, int QW>
+template <typename ET, int QW, int KIND>
 struct Service {
     static constexpr int CE = Chunk<ET>::N, PL = CE / 4, QE = kQuad / sizeof(ET);      // elements of a quad
     const WalkArgs& a;
@@ -291,6 +301,12 @@ struct Service {
         : a(a_), L(L_), xs(xs_), red(red_), t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {
         wait.err = a.err;
         wait.dead = false;
+    }
+    // The thread's number as the compiler does not know it: addresses made of it are not kept in registers from layer to layer.
+    __device__ __forceinline__ int opaque() const {
+        int v = threadIdx.x;
+        asm volatile("" : "+v"(v));
+        return v;
     }
     // Barrier of the service waves among themselves: the others may stand still for the sake of their requests.
     __device__ __forceinline__ void meet() {
@@ -325,6 +341,7 @@ struct Service {
     }
     // A vector of k words as it is
     __device__ __forceinline__ void take(unsigned at, int k) {
+        const int t = opaque();
         const int n4 = k / 4, segs = k / (CE * 64);
         auto some = [&](auto n, int c0) {
             constexpr int N = decltype(n)::value;
@@ -346,6 +363,7 @@ struct Service {
     }
     // x += y (normed and times gb where there is one) + the embedding of `again`; the vector becomes norm(x) * g.
     __device__ __forceinline__ void norm(bool have, unsigned at, const float* gb, const float* g, int again_token) {
+        const int t = opaque();
         const int n4 = a.width / 4, segs = a.width / (CE * 64);
         f32x4 gv[QW], gbv[QW];
         unsigned off[QW];
@@ -367,7 +385,7 @@ struct Service {
                     if (t + kSvcT * i < n4)
 #pragma unroll
                         for (int e = 0; e < 4; e++) ss = fma_f(y[i][e], y[i][e], ss);
-                rs = root(ss);
+                rs = root(ss, (float)a.width);
             }
 #pragma unroll
             for (int i = 0; i < QW; i++)
@@ -383,7 +401,7 @@ struct Service {
             if (t + kSvcT * i < n4)
 #pragma unroll
                 for (int e = 0; e < 4; e++) ss = fma_f(x[i][e], x[i][e], ss);
-        const float rx = root(ss);
+        const float rx = root(ss, (float)a.width);
 #pragma unroll
         for (int i = 0; i < QW; i++) {
             f32x4 h;
@@ -393,14 +411,14 @@ struct Service {
         }
         vector_done();
     }
-    // 1 / rms of a vector of the model's width from the threads' sums of squares
-    __device__ __forceinline__ float root(float ss) {
+    // 1 / rms of `count` values from the threads' sums of squares
+    __device__ __forceinline__ float root(float ss, float count) {
         ss = wave_sum(ss);
         if (lane == 0) L.norm[normed][wave] = ss;
         meet();
         const float* n = L.norm[normed];
         normed ^= 1;
-        return 1.0f / sqrtf(((n[0] + n[1]) + (n[2] + n[3])) / (float)a.width + a.eps);
+        return 1.0f / sqrtf(((n[0] + n[1]) + (n[2] + n[3])) / count + a.eps);
     }
     __device__ __forceinline__ f32x4 embedding(int token, int c) const {
         const bf16x4 b = *global(reinterpret_cast<const bf16x4*>(a.embed + (size_t)token * a.width + 4 * c));
@@ -420,6 +438,7 @@ struct Service {
     // least: up to 256 rows of 64 then need no join, which is 2.4 us.
     template <int D>
     __device__ __forceinline__ void shared_kv(RunPtr r, int pos) {
+        const int t = opaque(), lane = t & 63;
         constexpr int LPK = D / CE, KS = kSvcT / LPK, U = 4, N = CE, PW = walk_part(D);
         const int G = r->kv_heads, rep = r->rep, S = r->splits, g = wg % G, idx = wg / G, split = idx / rep, head = g * rep + idx % rep;
         const int held = pos, per = max(((held + S - 1) / S + KS - 1) / KS * KS, U * KS), ns = max((held + per - 1) / per, 1);
@@ -577,7 +596,6 @@ struct Service {
                     if (t == 0) { put(part + D, mt); put(part + D + 1, lt); }
                 }
             }
-            sums_done();
         } else if (split < S) {
             for (int i = t; i < D + 2; i += kSvcT) unput(part + i);
         }
@@ -606,7 +624,406 @@ struct Service {
             const float lt = r->sink ? o[4] + __builtin_amdgcn_exp2f(-mt) : o[4];
             if (cols && s < 4) put(r->x_att + (unsigned)(head * D + c + s), (s == 0 ? o[0] : s == 1 ? o[1] : s == 2 ? o[2] : o[3]) / lt);
         }
-        sums_done();
+    }
+
+    // ---- gated linear attention: a workgroup has a slice of `cs` columns of a head's state.  The state does not hang on the step and is on
+    // its way under the wait.  The head's norm needs all slices: the outputs leave times the norm's weight and the gate, with the slice's
+    // sum of squares (in copies: a line that all workgroups ask for has them stand in line, 3 us), and who reads them divides (take_heads).  (A kernel with a workgroup per head: 8.2 us on 16 or 32 CUs.)
+    __device__ __forceinline__ void gla(RunPtr r, int pos) {
+        const int t = opaque(), lane = t & 63;
+        constexpr int D = kWalkDim, NR = kWalkGlaRank;
+        const int H = r->heads, NS = r->splits, cs = D / NS, h = wg % H, slice = wg / H, HD = H * D;
+        if (slice >= NS) return;
+        const int qd = cs / 4, c0 = slice * cs;           // float4 of a row of the slice
+        float* S = r->state + (size_t)h * D * D + c0;
+        const bool fresh = pos == 0;                      // a sequence starts from a zero state
+        f32x4 st[2];
+        int row[2];
+        const int c4 = t % qd;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            row[i] = (t + kSvcT * i) / qd;
+            if (row[i] < D && !fresh) st[i] = *global(reinterpret_cast<const f32x4*>(S + (size_t)row[i] * D + 4 * c4));
+            else st[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        float w[NR], bias = 0.0f;
+        if (t < D) {
+            const ET* src = static_cast<const ET*>(r->a2) + (size_t)(h * D + t) * kKPad;       // rows are padded with zeros
+#pragma unroll
+            for (int i = 0; i < NR / CE; i++) {
+                float v[CE];
+                const i32x4 u = *global(reinterpret_cast<const i32x4*>(src + i * CE));
+                Chunk<ET>::unpack(make_uint4(u[0], u[1], u[2], u[3]), v);
+#pragma unroll
+                for (int e = 0; e < CE; e++) w[i * CE + e] = v[e];
+            }
+            bias = *global(r->a2_bias + h * D + t);
+        }
+        const float nw = t < cs ? *global(r->head_norm + c0 + t) : 0.0f;
+        float *sq = L.q, *sk = L.q + D, *sa = L.q + 2 * D, *sv = L.q + 3 * D, *sg = sv + 16, *s1 = sg + 16;
+        if (wave == 0) {                                  // query and key
+            unsigned off[1] = {4u * (unsigned)((lane < 32 ? 0 : HD) + h * D) + 16u * (unsigned)(lane & 31)};
+            f32x4 v[1];
+            poll_words<1>(now + r->x_in, off, true, v, wait);
+            *reinterpret_cast<f32x4*>((lane < 32 ? sq : sk) + 4 * (lane & 31)) = v[0];
+        } else if (wave == 1) {                           // the slice's values and gates, the decay's input
+            const int n1 = (r->a_rank + 3) / 4, part = lane < 4 ? 0 : lane < 8 ? 1 : 2, i = part < 2 ? lane & 3 : lane - 8;
+            const bool need = part < 2 ? i < qd : i < n1;
+            const unsigned at = (unsigned)(part == 0 ? 2 * HD + h * D + c0 : part == 1 ? 3 * HD + h * D + c0 : 4 * HD);
+            unsigned off[1] = {4u * at + 16u * (unsigned)(need ? i : 0)};
+            f32x4 v[1];
+            poll_words<1>(now + r->x_in, off, need, v, wait);
+            if (part < 2) *reinterpret_cast<f32x4*>((part == 0 ? sv : sg) + 4 * i) = v[0];
+            else if (i < NR / 4) *reinterpret_cast<f32x4*>(s1 + 4 * i) = v[0];         // zeros beyond the rank
+        }
+        meet();
+        if (t < D) {
+            float z = bias;
+#pragma unroll
+            for (int i = 0; i < NR; i++) z = i < r->a_rank ? fma_f(w[i], s1[i], z) : z;
+            sa[t] = exp_f<false>(log_sigmoid_f(z) / r->tau);
+            sq[t] *= 1.0f / sqrtf((float)D);
+        }
+        meet();
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        const f32x4 v = *reinterpret_cast<const f32x4*>(sv + 4 * c4);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            if (row[i] < D) {
+                const float k = sk[row[i]], d = sa[row[i]], q = sq[row[i]];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    st[i][e] = fma_f(k, v[e], fresh ? 0.0f : st[i][e] * d);
+                    acc[e] = fma_f(st[i][e], q, acc[e]);
+                }
+                *(Global<f32x4>*)(S + (size_t)row[i] * D + 4 * c4) = st[i];
+            }
+        // over the rows: lanes of the same four columns, then the waves
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            if (qd <= 2) acc[e] += lane_xor_f<2>(acc[e]);
+            acc[e] += lane_xor_f<4>(acc[e]);
+            acc[e] += lane_xor_f<8>(acc[e]);
+            acc[e] += lane_xor_f<16>(acc[e]);
+            acc[e] += lane_xor_f<32>(acc[e]);
+        }
+        if (lane < qd) *reinterpret_cast<f32x4*>(&L.sums[wave][4 * lane]) = acc;
+        meet();
+        if (wave == 0) {
+            float x = 0.0f;
+            if (t < cs) {
+                x = (L.sums[0][t] + L.sums[1][t]) + (L.sums[2][t] + L.sums[3][t]);
+                const float g = sg[t];
+                put(r->x_att + (unsigned)(h * D + c0 + t), x * nw * (g * sigmoid_f(g)));
+            }
+            const float ss = wave_sum(x * x);
+            if (t < kWalkCopies) put(r->x_part + (unsigned)(t * kWalkWG + h * NS + slice), ss);
+        }
+    }
+    // The vector of gla(): every head over the root of its mean square.
+    __device__ __forceinline__ void take_heads(RunPtr r) {
+        const int t = opaque(), lane = t & 63;
+        const int k = r->k_o, n4 = k / 4, segs = k / (CE * 64), NS = r->splits, H = r->heads;
+        if (wave == 0) {
+            const bool need = 4 * lane < H * NS;
+            unsigned off[1] = {16u * (unsigned)(need ? lane : 0)};
+            f32x4 v[1];
+            poll_words<1>(now + r->x_part + wg % kWalkCopies * kWalkWG, off, need, v, wait);
+            float ss = (v[0][0] + v[0][1]) + (v[0][2] + v[0][3]);
+            ss += lane_xor_f<1>(ss);                      // two lanes per head, or four
+            if (NS == 16) ss += lane_xor_f<2>(ss);
+            if (need && lane % (NS / 4) == 0) L.of_head[lane / (NS / 4)] = 1.0f / sqrtf(ss / (float)kWalkDim + a.eps);
+        }
+        auto all = [&](auto n) {
+            constexpr int N = decltype(n)::value;
+            unsigned off[N];
+            f32x4 v[N];
+#pragma unroll
+            for (int i = 0; i < N; i++) off[i] = 16u * (unsigned)min(t + kSvcT * i, n4 - 1);
+            poll_words<N>(now + r->x_att, off, wave * 64 < n4, v, wait);
+            meet();
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                const int c = t + kSvcT * i;
+                if (c < n4) put_x(segs, c, v[i] * L.of_head[c / (kWalkDim / 4)]);
+            }
+        };
+        if (n4 > 2 * kSvcT) all(std::integral_constant<int, 4>());
+        else all(std::integral_constant<int, 2>());
+        vector_done();
+    }
+
+    // ---- latent attention (see latent_attn.hip), a workgroup per head and slice throughout.  The query's slice of latent columns; a split of
+    // the rows for the whole latent query; the context of all splits through the slice's rows of W_uv.  Weights and rows are on their way
+    // under the waits.  (Three kernels: 19 us.)
+    __device__ __forceinline__ void latent(RunPtr r, int pos) {
+        const int t = opaque(), lane = t & 63;
+        constexpr int D = kWalkDim, RK = kWalkRank, RW = kWalkRow2, PW = walk_part(RK), PCS = RK / CE / 64;      // pieces of a row per lane
+        const int H = r->heads, NS = r->splits, h = wg % H, slice = wg / H;
+        if (slice >= NS || pos >= r->capacity) return;
+        {   // ---- W_uk's slice of columns against the head's query
+            const int cols = RK / NS, pc = cols / CE, c0 = slice * cols, c = t % pc, g = t / pc, step = kSvcT / pc;       // 32 or 64 columns
+            constexpr int NP = 8;                         // rows per thread at most: 128 / (256 / pc), pc at most 16
+            i32x4 u[NP];
+            const auto* w = global(static_cast<const ET*>(r->uk)) + (size_t)h * D * RK + c0 + c * CE;
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                if (g + i * step < D) u[i] = *reinterpret_cast<const Global<i32x4>*>(w + (size_t)(g + i * step) * RK);
+            if (wave == 0) {
+                unsigned off[1] = {4u * (unsigned)(h * (D + kWalkRot)) + 16u * (unsigned)min(lane, 47)};
+                f32x4 v[1];
+                poll_words<1>(now + r->x_in, off, lane < 48, v, wait);
+                if (lane < 48) *reinterpret_cast<f32x4*>(L.q + 4 * lane) = v[0];
+            }
+            meet();
+            float acc[CE];
+#pragma unroll
+            for (int e = 0; e < CE; e++) acc[e] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                if (g + i * step < D) {
+                    float wv[CE];
+                    Chunk<ET>::unpack(make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]), wv);
+                    const float q = L.q[g + i * step];
+#pragma unroll
+                    for (int e = 0; e < CE; e++) acc[e] = fma_f(wv[e], q, acc[e]);
+                }
+            // over the rows: lanes of the same piece (pc 4, 8 or 16), then the waves
+#pragma unroll
+            for (int e = 0; e < CE; e++) {
+                if (pc <= 4) acc[e] += lane_xor_f<4>(acc[e]);
+                if (pc <= 8) acc[e] += lane_xor_f<8>(acc[e]);
+                acc[e] += lane_xor_f<16>(acc[e]);
+                acc[e] += lane_xor_f<32>(acc[e]);
+            }
+            if (lane < pc)
+#pragma unroll
+                for (int e = 0; e < CE; e++) L.sums[wave][lane * CE + e] = acc[e];
+            meet();
+            if (t < cols) put(r->x_ql + (unsigned)(h * RW + c0 + t), (L.sums[0][t] + L.sums[1][t]) + (L.sums[2][t] + L.sums[3][t]));
+            if (slice == 0 && wave == 3) {                // the rotated part
+                const int j = lane >> 1, rh = kWalkRot / 2;
+                const float x = L.q[D + 2 * j], y = L.q[D + 2 * j + 1], cs = *global(r->cos_t + (size_t)pos * rh + j), sn = *global(r->sin_t + (size_t)pos * rh + j);
+                put(r->x_ql + (unsigned)(h * RW + RK + lane), lane & 1 ? y * cs + x * sn : x * cs - y * sn);
+            }
+        }
+        // ---- a split of the rows: a wave takes U rows at a time, a lane 8 of their latent columns; their rotated parts, 64 columns each, lie side by
+        // side over the lanes
+        const int lo = r->window > 0 && pos - r->window + 1 > 0 ? pos - r->window + 1 : 0, end = r->own_rows ? pos : pos + 1;      // rows lo .. end-1 are in the cache
+        constexpr int U = 4;
+        const int n = end - lo, per = max(((n + NS - 1) / NS + 4 * U - 1) / (4 * U) * (4 * U), 64), ns = max((n + per - 1) / per, 1);
+        const int first = lo + slice * per, last = min(end, first + per);
+        const unsigned part = r->x_part + (unsigned)((h * NS + slice) * PW);
+        if (slice < ns) {
+            const bool own = r->own_rows && slice == ns - 1;
+            const auto* rows = global(static_cast<const ET*>(r->rows));
+            i32x4 u[U][PCS], v[U][PCS], ur, vr;
+            auto load = [&](int k0, i32x4 (&x)[U][PCS], i32x4& xr) {
+#pragma unroll
+                for (int i = 0; i < U; i++)
+#pragma unroll
+                    for (int j = 0; j < PCS; j++) x[i][j] = *reinterpret_cast<const Global<i32x4>*>(rows + (size_t)min(k0 + i, last - 1) * RW + lane * 8 + j * CE);
+                constexpr int LR = kWalkRot / CE;         // lanes per rotated part
+                xr = *reinterpret_cast<const Global<i32x4>*>(rows + (size_t)min(k0 + lane / LR, last - 1) * RW + RK + lane % LR * CE);
+            };
+            const int k1 = first + wave * U;
+            if (k1 < last) load(k1, u, ur);
+            if (own) {                                    // the row of this step: normed and rotated by each head for itself, stored by the first
+                f32x4 p[1];
+                unsigned off[1] = {4u * (unsigned)r->n_et + 16u * (unsigned)min(t, RW / 4 - 1)};
+                if (wave < 3) {
+                    poll_words<1>(now + r->x_in, off, t < RW / 4, p, wait);
+                    if (t < RW / 4) *reinterpret_cast<f32x4*>(L.kx + 4 * t) = p[0];
+                }
+                meet();
+                const float x0 = L.kx[2 * t], x1 = L.kx[2 * t + 1];
+                const float rs = root(fma_f(x0, x0, x1 * x1), (float)RK);
+                float o0 = x0 * rs * *global(r->latent_norm + 2 * t), o1 = x1 * rs * *global(r->latent_norm + 2 * t + 1);
+                float e0 = 0.0f, e1 = 0.0f;
+                if (t < kWalkRot / 2) {
+                    const float a0 = L.kx[RK + 2 * t], a1 = L.kx[RK + 2 * t + 1], cs = *global(r->cos_t + (size_t)pos * (kWalkRot / 2) + t), sn = *global(r->sin_t + (size_t)pos * (kWalkRot / 2) + t);
+                    e0 = (float)(ET)(a0 * cs - a1 * sn);
+                    e1 = (float)(ET)(a1 * cs + a0 * sn);
+                    L.kx[RK + 2 * t] = e0;
+                    L.kx[RK + 2 * t + 1] = e1;
+                }
+                o0 = (float)(ET)o0;
+                o1 = (float)(ET)o1;
+                L.kx[2 * t] = o0;
+                L.kx[2 * t + 1] = o1;
+                if (h == 0) {
+                    ET* dst = static_cast<ET*>(r->rows) + (size_t)pos * RW;
+                    auto pair = [&](ET* p, float a, float b) {
+                        if constexpr (std::is_same<ET, float>::value) {
+                            store_past(p, a);
+                            store_past(p + 1, b);
+                        } else {
+                            __attribute__((aligned(4))) ET w[2] = {(ET)a, (ET)b};
+                            store_past(reinterpret_cast<float*>(p), *reinterpret_cast<const float*>(w));
+                        }
+                    };
+                    pair(dst + 2 * t, o0, o1);
+                    if (t < kWalkRot / 2) pair(dst + RK + 2 * t, e0, e1);
+                }
+            }
+            {
+                unsigned off[1] = {4u * (unsigned)(h * RW) + 16u * (unsigned)min(t, RW / 4 - 1)};
+                f32x4 p[1];
+                if (wave < 3) {
+                    poll_words<1>(now + r->x_ql, off, t < RW / 4, p, wait);
+                    if (t < RW / 4) *reinterpret_cast<f32x4*>(L.ql + 4 * t) = p[0];
+                }
+                meet();
+            }
+            float ql[8], qr[CE], acc[8], m = -1e30f, l = 0.0f;
+            const float f = r->scale * kWalkLog2e;
+#pragma unroll
+            for (int e = 0; e < 8; e++) { ql[e] = L.ql[lane * 8 + e] * f; acc[e] = 0.0f; }
+            constexpr int LR = kWalkRot / CE;
+#pragma unroll
+            for (int e = 0; e < CE; e++) qr[e] = L.ql[RK + lane % LR * CE + e] * f;
+            auto columns = [&](const i32x4 (&x)[PCS], float (&o)[8]) {
+#pragma unroll
+                for (int j = 0; j < PCS; j++) Chunk<ET>::unpack(make_uint4(x[j][0], x[j][1], x[j][2], x[j][3]), reinterpret_cast<float (&)[CE]>(o[j * CE]));
+            };
+            auto take_rows = [&](int k0, const i32x4 (&x)[U][PCS], const i32x4& xr) {
+                float s[U], w[CE], rot = 0.0f;
+                Chunk<ET>::unpack(make_uint4(xr[0], xr[1], xr[2], xr[3]), w);
+#pragma unroll
+                for (int e = 0; e < CE; e++) rot = fma_f(w[e], qr[e], rot);
+                rot = lanes_sum<LR>(rot);                 // of row lane / LR
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    float o[8];
+                    columns(x[i], o);
+                    s[i] = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) s[i] = fma_f(o[e], ql[e], s[i]);
+                }
+                multi_sum_step<U, 1>(s, lane);            // lane i has row multi_row(i)
+                float z[U], mx = m;
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    int from = 0;                         // the lane with row i
+#pragma unroll
+                    for (int b = 1, half = U / 2; half >= 1; b *= 2, half /= 2)
+                        if (i & half) from |= b;
+                    const float v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[0]), from)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rot), i * LR));
+                    z[i] = k0 + i < last ? v : -INFINITY;
+                    mx = fmaxf(mx, z[i]);
+                }
+                const float al = __builtin_amdgcn_exp2f(m - mx);
+                m = mx;
+                l *= al;
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] *= al;
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    const float p = __builtin_amdgcn_exp2f(z[i] - mx);
+                    l += p;
+                    float o[8];
+                    columns(x[i], o);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) acc[e] = k0 + i < last ? fma_f(p, o[e], acc[e]) : acc[e];
+                }
+            };
+            for (int k0 = k1; k0 < last; k0 += 8 * U) {
+                if (k0 + 4 * U < last) load(k0 + 4 * U, v, vr);
+                take_rows(k0, u, ur);
+                if (k0 + 4 * U >= last) break;
+                if (k0 + 8 * U < last) load(k0 + 8 * U, u, ur);
+                take_rows(k0 + 4 * U, v, vr);
+            }
+            if (own && wave == 3) {                       // the row of this step
+                float o[8], s = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    o[e] = L.kx[lane * 8 + e];
+                    s = fma_f(o[e], ql[e], s);
+                }
+                s = fma_f(L.kx[RK + lane], L.ql[RK + lane] * f, s);
+                s = wave_sum(s);
+                const float mx = fmaxf(m, s), al = __builtin_amdgcn_exp2f(m - mx), p = __builtin_amdgcn_exp2f(s - mx);
+                m = mx;
+                l = l * al + p;
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] = fma_f(p, o[e], acc[e] * al);
+            }
+            if (lane == 0) { L.m[wave] = m; L.l[wave] = l; }
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) *reinterpret_cast<f32x4*>(&L.sums[wave][lane * 8 + e]) = f32x4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+            meet();
+            const float mt = fmaxf(fmaxf(L.m[0], L.m[1]), fmaxf(L.m[2], L.m[3]));
+            float lt = 0.0f, o[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int w = 0; w < kSvcWaves; w++) {
+                const float e = __builtin_amdgcn_exp2f(L.m[w] - mt);
+                lt = fma_f(L.l[w], e, lt);
+#pragma unroll
+                for (int i = 0; i < 2; i++) o[i] += e == 0.0f ? 0.0f : L.sums[w][t + kSvcT * i] * e;
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++) put(part + t + kSvcT * i, o[i]);
+            if (t == 0) { put(part + RK, mt); put(part + RK + 1, lt); }
+        } else {
+            for (int i = t; i < RK + 2; i += kSvcT) unput(part + i);
+        }
+        // ---- the context of all splits, and W_uv's rows of the slice: a wave takes every fourth one
+        {
+            const int nr = D / NS;                        // 8 or 16
+            constexpr int NP = 4;
+            i32x4 u[NP][PCS];
+            const auto* w = global(static_cast<const ET*>(r->uv)) + (size_t)(h * D + slice * nr) * RK + lane * 8;
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                if (wave + 4 * i < nr)
+#pragma unroll
+                    for (int j = 0; j < PCS; j++) u[i][j] = *reinterpret_cast<const Global<i32x4>*>(w + (size_t)(wave + 4 * i) * RK + j * CE);
+            const unsigned base = 4u * (unsigned)(h * NS * PW);
+            float ms, ls;
+            {
+                unsigned off[1] = {base + 4u * (unsigned)(min(lane, ns - 1) * PW + RK)};
+                f32x4 v[1];
+                poll_words<1, 2>(now + r->x_part, off, lane < ns, v, wait);
+                ms = lane < ns ? v[0][0] : -INFINITY;
+                ls = v[0][1];
+            }
+            const float mt = wave_max(ms), e = lane < ns ? __builtin_amdgcn_exp2f(ms - mt) : 0.0f, lt = wave_sum(e == 0.0f ? 0.0f : ls * e), share = e / lt;
+            const int half = __builtin_amdgcn_readfirstlane(t >> 7), c4 = t & 127;        // two halves of the threads take splits in turn
+            f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int s0 = 0; s0 < ns; s0 += 8) {
+                unsigned off[4];
+                f32x4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) off[i] = base + 4u * (unsigned)(min(s0 + 2 * i + half, ns - 1) * PW + 4 * c4);
+                poll_words<4>(now + r->x_part, off, true, v, wait);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int sp = s0 + 2 * i + half;
+                    const float p = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(share), min(sp, 63)));
+                    if (sp < ns && p != 0.0f) sum += v[i] * p;
+                }
+            }
+            *reinterpret_cast<f32x4*>((half ? L.kx : L.q) + 4 * c4) = sum;      // nobody reads them any more, L.sums may still be read
+            meet();
+            float ctx[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) ctx[i] = L.q[lane * 8 + i] + L.kx[lane * 8 + i];
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+                if (wave + 4 * i < nr) {
+                    float o = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < PCS; j++) {
+                        float wv[CE];
+                        Chunk<ET>::unpack(make_uint4(u[i][j][0], u[i][j][1], u[i][j][2], u[i][j][3]), wv);
+#pragma unroll
+                        for (int q = 0; q < CE; q++) o = fma_f(wv[q], ctx[j * CE + q], o);
+                    }
+                    o = wave_sum(o);
+                    if (lane == 0) put(r->x_att + (unsigned)(h * D + slice * nr + wave + 4 * i), o);
+                }
+        }
     }
 
     // ---- one token: returns the next one
@@ -634,9 +1051,17 @@ struct Service {
             RunPtr r = runs + i;
             norm(have, y, gb, r->g1, r->again ? token : -1);
             plain(r->n_in, W, r->x_in, r->in_bias);
-            if (r->dim == 64) shared_kv<64>(r, pos);
-            else shared_kv<128>(r, pos);
-            take(r->x_att, r->k_o);
+            if constexpr (KIND == kWalkSharedKv) {
+                if (r->dim == 64) shared_kv<64>(r, pos);
+                else shared_kv<128>(r, pos);
+                take(r->x_att, r->k_o);
+            } else if (r->mixer == kWalkGla) {
+                gla(r, pos);
+                take_heads(r);
+            } else {
+                latent(r, pos);
+                take(r->x_att, r->k_o);
+            }
             plain(W, r->k_o, r->x_y, nullptr);
             have = true; y = r->x_y; gb = r->g1b;
             if (r->ff == 0) continue;
@@ -651,6 +1076,7 @@ struct Service {
             plain(W, r->ff, r->x_y2, nullptr);
             y = r->x_y2; gb = r->g2b;
         }
+        if (!choose && t < 2) unput(a.x_cand + (unsigned)(2 * wg + t));        // what is not handed out in this step is unset behind the last one all the same
         if (!a.head) return 0;
         norm(have, y, gb, a.g_final, -1);
         __syncthreads();
@@ -694,7 +1120,8 @@ struct Service {
     }
 };
 
-template <typename ET, int QW>
+// KIND: models of shared key/value rows, or of latent rows and gated linear attention (kWalkLatent)
+template <typename ET, int QW, int KIND>
 __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
     constexpr int QE = kQuad / sizeof(ET);
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -714,7 +1141,7 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
         stream_waves<ET>(L, xs, red, reinterpret_cast<const char*>(red + a.lds_red), slots, phases, a.steps);
         return;
     }
-    Service<ET, QW> s(a, L, xs, red);
+    Service<ET, QW, KIND> s(a, L, xs, red);
     const int pos0 = a.state[0], step0 = a.state[1];
     int token = a.token[0];
     if ((unsigned)token >= (unsigned)a.vocab) {
@@ -757,8 +1184,9 @@ int walk_launch(const WalkArgs& a, hipStream_t st) {
         FX_LAUNCH_CHECK();
         return FLEXLLM_OK;
     };
-    static std::atomic<bool> opted2{false}, opted4{false};
-    return a.width <= 2048 ? go(walk_kernel<ET, 2>, opted2) : go(walk_kernel<ET, 4>, opted4);
+    static std::atomic<bool> opted[4];
+    if (a.kind == kWalkSharedKv) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkSharedKv>, opted[0]) : go(walk_kernel<ET, 4, kWalkSharedKv>, opted[1]);
+    return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkLatent>, opted[2]) : go(walk_kernel<ET, 4, kWalkLatent>, opted[3]);
 }
 template int walk_launch<bf16_t>(const WalkArgs&, hipStream_t);
 template int walk_launch<float>(const WalkArgs&, hipStream_t);

@@ -384,9 +384,12 @@ static int create_walk(flexllm_hybrid* m) {
     FX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     const int few = 2 * kWalkWG;                          // rows of which every workgroup has some
     bool ok = cus >= kWalkWG && W % unit == 0 && W <= kWalkMaxWidth && c.vocab >= few;
-    for (const HybridLayer& L : m->layers)
-        ok = ok && L.d.mixer == FLEXLLM_MIX_SHARED_KV && walk_shared_kv_ok(L.sd) && L.n_in >= few && L.k_o % unit == 0 &&
-             (L.d.ff_kind == FLEXLLM_FF_NONE || (L.d.ff_kind == FLEXLLM_FF_DENSE && L.d.ff % unit == 0 && 2 * L.d.ff >= few));
+    const bool shared = m->layers[0].d.mixer == FLEXLLM_MIX_SHARED_KV;
+    for (const HybridLayer& L : m->layers) {
+        ok = ok && (L.d.mixer == FLEXLLM_MIX_SHARED_KV) == shared && L.n_in >= few && L.k_o % unit == 0 && L.k_o <= kWalkMaxWidth;
+        ok = ok && (L.d.mixer == FLEXLLM_MIX_SHARED_KV ? walk_shared_kv_ok(L.sd) : L.d.mixer == FLEXLLM_MIX_LATENT ? walk_latent_ok(L.ld) : walk_gla_ok(L.gd));
+        ok = ok && (L.d.ff_kind == FLEXLLM_FF_NONE || (L.d.ff_kind == FLEXLLM_FF_DENSE && L.d.ff % unit == 0 && 2 * L.d.ff >= few));
+    }
     if (!ok) return FLEXLLM_OK;
     std::vector<WalkPhase> phases;
     std::vector<WalkRun> runs;
@@ -412,11 +415,25 @@ static int create_walk(flexllm_hybrid* m) {
                 r = runs[i];
             } else {
                 r.g1 = L.g1; r.g1b = L.g1b; r.g2 = L.g2; r.g2b = L.g2b; r.in_bias = L.in_bias; r.kv_norm = L.kv_norm;
-                r.mixer = kWalkSharedKv; r.again = m->runs[i].again; r.n_in = L.n_in; r.n_et = L.n_et; r.k_o = L.k_o;
+                r.again = m->runs[i].again; r.n_in = L.n_in; r.n_et = L.n_et; r.k_o = L.k_o; r.heads = L.d.heads; r.capacity = c.max_pos;
                 r.ff = L.d.ff_kind == FLEXLLM_FF_NONE ? 0 : L.d.ff; r.glu = 1 + L.d.glu; r.limit = L.d.limit;
-                r.kv_heads = L.sd.kv_heads; r.rep = L.sd.heads / L.sd.kv_heads; r.splits = walk_splits(L.sd.heads, L.sd.dim); r.dim = L.sd.dim; r.sink = L.sd.sink; r.temp_every = L.sd.temp_every; r.capacity = L.sd.capacity;
-                r.scale = L.sd.scale; r.temp_coef = L.sd.temp_coef;
-                r.x_in = words(r.n_in); r.x_part = words((size_t)L.sd.heads * r.splits * walk_part(r.dim)); r.x_att = words(r.k_o); r.x_y = words(W);
+                r.x_in = words(r.n_in);
+                if (shared) {
+                    r.mixer = kWalkSharedKv;
+                    r.kv_heads = L.sd.kv_heads; r.rep = L.sd.heads / L.sd.kv_heads; r.splits = walk_splits(L.sd.heads, L.sd.dim); r.dim = L.sd.dim;
+                    r.sink = L.sd.sink; r.temp_every = L.sd.temp_every; r.scale = L.sd.scale; r.temp_coef = L.sd.temp_coef;
+                    r.x_part = words((size_t)r.heads * r.splits * walk_part(r.dim));
+                } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {
+                    r.mixer = kWalkLatent;
+                    r.splits = walk_slices(r.heads); r.scale = L.ld.scale; r.window = L.ld.window; r.own_rows = L.d.kv_from < 0;
+                    r.uk = L.uk; r.uv = L.uv; r.latent_norm = L.latent_norm; r.cos_t = L.cos_t; r.sin_t = L.sin_t;
+                    r.x_ql = words((size_t)r.heads * kWalkRow2); r.x_part = words((size_t)r.heads * r.splits * walk_part(kWalkRank));
+                } else {
+                    r.mixer = kWalkGla;
+                    r.splits = walk_slices(r.heads); r.a2 = L.a2; r.a2_bias = L.a2_bias; r.head_norm = L.head_norm; r.a_rank = L.gd.a_rank; r.tau = L.gd.tau;
+                    r.x_part = words((size_t)kWalkCopies * kWalkWG);
+                }
+                r.x_att = words(r.k_o); r.x_y = words(W);
                 linear(L.w_in, L.n_in, W);
                 linear(L.w_o, W, L.k_o);
                 if (r.ff) {
@@ -425,7 +442,7 @@ static int create_walk(flexllm_hybrid* m) {
                     linear(L.w_d, W, r.ff);
                 }
             }
-            r.rows = m->slots[slot].rows[i]; r.inv_rms = m->slots[slot].inv_rms[i];
+            r.rows = m->slots[slot].rows[i]; r.inv_rms = m->slots[slot].inv_rms[i]; r.state = m->slots[slot].state[i];
             runs.push_back(r);
         }
     a.n_phases = (int)phases.size();
@@ -442,6 +459,7 @@ static int create_walk(flexllm_hybrid* m) {
     FX_TRY(own(m, a.words, 2 * at));
     FX_HIP(hipMemset(a.words, 0xFF, 2 * at * sizeof(float)));
     FX_TRY(own(m, a.err, 1));
+    a.kind = shared ? kWalkSharedKv : kWalkLatent;
     a.n_runs = n_runs; a.width = W; a.vocab = c.vocab; a.eps = c.eps; a.embed_scale = c.embed_scale;
     a.embed = as_bf16(m->embed); a.g_final = m->g_final;
     a.phases = dev_phases;

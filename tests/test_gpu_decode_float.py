@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 
 import lopazen_cases as lc
+import nifunex_cases as nc
 from oracle import lopazen_ref
-from test_gpu_decoder_sizes import check_lopazen
+from test_gpu_decoder_sizes import check_lopazen, check_nifunex
 
 pytestmark = pytest.mark.gpu
 BOTH = pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
@@ -31,6 +32,37 @@ LOPAZEN = {
 @pytest.mark.parametrize("name", list(LOPAZEN))
 def test_token_by_token(name, dtype):
     check_lopazen(LOPAZEN[name], dtype, 40, [1], [23, 1])
+
+
+def latent(heads, ff, **kw):
+    return nc.latent(heads=heads, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5, mlp=nc.dense(ff) if ff else None, **kw)
+
+
+def gla(heads, ff):
+    return nc.gla(heads=heads, dim=128, vdim=128, mlp=nc.dense(ff) if ff else None)
+
+
+# slices of 8 and of 16 columns, as many heads as there may be and fewer; windows shorter than a split and none; rows of an earlier layer
+NIFUNEX = {
+    "both kinds": nc.config([latent(16, 2048, window=40), gla(16, 2048), latent(16, 2048, window=40, kv_from=0), gla(16, 0)], width=2048, vocab=512),
+    "many heads": nc.config([gla(32, 4096), latent(32, 4096, window=None)], width=4096, vocab=515),
+    "rows of seven quads": nc.config([latent(16, 14336, scaling=None)], width=2048, vocab=519),
+    "heads that leave workgroups without a slice": nc.config([latent(32, 0), gla(32, 2048)], width=2048, vocab=600),
+}
+
+
+@BOTH
+@pytest.mark.parametrize("name", list(NIFUNEX))
+def test_token_by_token_nifunex(name, dtype):
+    check_nifunex(NIFUNEX[name], dtype, 70, [1], [50, 1])
+
+
+@BOTH
+@pytest.mark.parametrize("heads,window", [(16, 1024), (16, 300), (32, 700)])
+def test_splits_of_latent_rows(heads, window, dtype):
+    """One more than a split, the window's edge, and beyond it."""
+    cfg = nc.config([latent(heads, 0, window=window)], width=2048, vocab=512)
+    check_nifunex(cfg, dtype, window + 90, [62, 1, 1, 1, window - 68, 1, 1, 1, 1, 1, 60, 1], max_pos=1152)
 
 
 @BOTH
@@ -69,6 +101,32 @@ def test_loop_of_tokens(dtype):
     err = lc.rel_err(last[0], ref.run(toks + got)[-1:])
     assert err.max() < lc.LIMIT[dtype]
     m.close()
+
+
+@pytest.mark.parametrize("name", list(NIFUNEX)[:2])
+def test_loops_and_steps_in_turn(name):
+    """Steps hand out logits and no candidates: a loop behind one finds none of an earlier loop's."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd.nifunex import Nifunex
+    cfg = NIFUNEX[name]
+    w, toks = nc.weights(cfg, 5), nc.tokens(cfg, 12)
+    m = Nifunex.from_tensors(cfg, w, dtype="float32", max_pos=256)
+    seen = []
+    for n in (5, 5, 4, 4, 3, 3):
+        for _ in range(6):
+            slot = m.pool.acquire("t")
+            got = [int(m.step(slot, toks, [11])[0].argmax())]
+            token, out = to_device(np.array(got, np.int32)), zeros((n,), np.int32)
+            m.decode(slot, token, n, out)
+            last = m.step(slot, token, [0])
+            got += out.numpy().tolist()
+            seen.append((got, last))
+            m.pool.release("t")
+    m.check()
+    m.close()
+    for got, last in seen:
+        assert got == seen[0][0][:len(got)]
+    assert all(np.array_equal(a[1], b[1]) for a, b in zip(seen[:6], seen[6:12]))
 
 
 def test_tokens_outside_the_vocabulary():
