@@ -55,7 +55,7 @@ void stream_scratch_release(hipStream_t st);
 
 // Launches of kernels whose workgroups wait for each other and so have to be resident all at once.  Two of them side by side could each
 // hold a part of the chip and wait for the rest of it, so on a device they run one after the other, whatever streams they are
-// launched on: each waits for the event behind the one before.  (Kernels of other kinds end by themselves.)  In a
+// launched on: one on another stream than the last waits for that stream.  (Kernels of other kinds end by themselves.)  In a
 // stream that is being captured there is no such order to keep.
 int resident_begin(hipStream_t st, bool& ordered);       // takes the device's turn
 int resident_end(hipStream_t st, bool ordered);
