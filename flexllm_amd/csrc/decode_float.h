@@ -6,18 +6,24 @@ namespace fx {
 
 constexpr int kWalkWG = 256;               // workgroups, one per CU: all of them have to be resident at once
 constexpr int kWalkCopies = 8;            // of few words that every workgroup reads
-constexpr int kWalkMaxPhases = 512;
+constexpr int kWalkMaxPhases = 256;
 constexpr int kWalkMaxWidth = 4096;
 constexpr size_t kWalkLdsMax = 160 * 1024;
 constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 8, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
 constexpr int kWalkRow = 4096;             // bytes that the rows of all linears are a multiple of
 
-// A linear of the step: n rows of kpad elements, dealt to the workgroups in runs of neighbouring rows (walk_rows).
+// A linear of the step: n rows of kpad elements, dealt to the workgroups in runs of neighbouring rows (walk_rows).  The experts' products are groups of
+// such linears, one per choice, between whose products nobody waits.
 struct WalkPhase {
-    const void* w;
+    const void* w;                         // of choice `slot` of the experts: + stride elements times the expert
     int n, kpad;
+    int group, first, last;                // number of its group; first and last of it
+    int routed;                            // 0, or the number (from 1) of the mixture whose choice it waits for
+    int slot;
+    size_t stride;
+    int x_off, red_off;                    // where the vector starts in LDS, and where the sums do (in floats, the same in all workgroups)
 };
-enum WalkMixer { kWalkSharedKv = 0, kWalkLatent = 1, kWalkGla = 2 };
+enum WalkMixer { kWalkSharedKv = 0, kWalkLatent = 1, kWalkGla = 2, kWalkMixture = 3 };
 struct WalkRun {
     const float *g1, *g1b, *g2, *g2b;      // norms ahead of and behind (null: none) the two sublayers
     const float *in_bias, *kv_norm;
@@ -38,12 +44,17 @@ struct WalkRun {
     float* state;
     int a_rank;
     float tau;
+    // mixture of experts (experts 0: none)
+    int experts, top, shared_ff;
+    float shared_limit;
+    int phase;                             // of the first choice's gate/up; the down projections follow, then the shared expert's
     // where the words that the workgroups hand to each other lie, in floats from the start of a set
-    unsigned x_in, x_ql, x_part, x_att, x_y, x_hid, x_y2;
+    unsigned x_in, x_ql, x_part, x_att, x_y, x_hid, x_route, x_y2;
 };
 struct WalkArgs {
     const WalkRun* runs;
     const WalkPhase* phases;
+    int routed;                            // mixtures of a token
     int n_runs, n_phases;                  // without the head's phase, which is entry n_phases
     int kind;                              // mixers: shared key/value rows (kWalkSharedKv), or the others (kWalkLatent)
     int width, vocab;
@@ -67,7 +78,10 @@ __host__ __device__ inline int walk_rows(int n, int w) {
     const int r = 2 * (int)(((long long)w * ((n + 1) / 2)) / kWalkWG);
     return r < n ? r : n;
 }
+// Rows that a workgroup has at most.
+__host__ __device__ inline int red_rows(int n) { return 2 * (((n + 1) / 2 + kWalkWG - 1) / kWalkWG); }
 size_t walk_lds(const WalkArgs& a);        // bytes
+constexpr int kWalkExperts = 255, kWalkTop = 16;        // most
 template <typename ET> int walk_launch(const WalkArgs& a, hipStream_t st);
 // Attention over shared key/value rows: splits of the rows per query head (one workgroup each, and at least four columns of the head for
 // each in the join), and the words of a split: the sums, maximum and weight sum.

@@ -16,6 +16,7 @@
 // workgroups take part in, or with the kernel).  A result that happens to have kUnset's bits leaves as another NaN.
 // All waits are bounded: a wait that times out raises a flag, everybody then runs to the end without waiting.
 #include "decode_float.h"
+#include "route.h"
 #include <atomic>
 
 namespace fx {
@@ -106,14 +107,16 @@ __device__ __forceinline__ void group(int n, F f) {
 constexpr float kWalkLog2e = 1.44269504088896340736f;
 
 struct WalkLds {                                          // ahead of the vector and the sums
-    __attribute__((aligned(16))) int4 phase[kWalkMaxPhases + 1];       // address of the workgroup's rows, 1 KiB units, [pieces of 64 per row | 8 mod that | barriers]
+    __attribute__((aligned(16))) int4 phase[kWalkMaxPhases];           // address of the workgroup's rows, quads, quads per row (0: half a one)
+    __attribute__((aligned(16))) int4 group[kWalkMaxPhases];           // vector's and sums' places; number of the group; [last << 31 | first << 30 | wave that begins << 16 | mixture]
     __attribute__((aligned(16))) float q[kWalkRow2];      // query; of gated linear attention query, key, decay, and what is short
     __attribute__((aligned(16))) float kx[kWalkRow2];     // the row of this step
     __attribute__((aligned(16))) float ql[kWalkRow2];     // latent query
     __attribute__((aligned(16))) float sums[kSvcWaves][kWalkRank];
     float of_head[32];
+    float z[kWalkExperts + 1], choice_w[kWalkTop + 1];
     float m[kSvcWaves], l[kSvcWaves];
-    int met, ready, sent;                                 // service waves' barrier; linears whose vector is there, whose sums have left
+    int met, ready, sent, chosen;                         // service waves' barrier; linears whose vector is there, whose sums have left; mixtures that have chosen
     float norm[2][kSvcWaves];
     float bestv[2][kSvcWaves];
     int besti[2][kSvcWaves];
@@ -153,26 +156,40 @@ __device__ __forceinline__ void wait_quads(int n) {
     }
 }
 __device__ __forceinline__ int flag(const int& f) { return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)); }
-template <typename ET>
-__device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, float* red, const char* ring, int slots, int phases, int tokens) {
+// MOE: with groups of linears and rows of half a quad (the other models are 2 to 3 % faster without).
+template <typename ET, bool MOE>
+__device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, float* red, const char* ring, int slots, int phases, int tokens, int routed) {
     constexpr int CE = Chunk<ET>::N, PL = CE / 4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) - kSvcWaves;
     auto word = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
     const char* mine = ring + (size_t)wave * slots * kQuad;
     const unsigned dst = word((int)(unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)mine);
     // what is asked for next: quad iq of linear ip of token it
-    int ip = 0, it = 0, iq = wave, itotal = word(L.phase[0].z), islot = 0, ahead = 0;       // ahead: quads asked for and not taken in
+    int ip = 0, it = 0, iq = wave, itotal = word(L.phase[0].z), iorder = 0, igroup = 0, islot = 0, ahead = 0;      // ahead: quads asked for and not taken in
     auto base_of = [&](int p) { return reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(L.phase[p].y) << 32) | (unsigned)word(L.phase[p].x)); };
+    auto begins = [&](int flags) { return (wave + (flags >> 16 & 7)) & (kStrWaves - 1); };      // this wave's first quad
     const char* ibase = base_of(0);
     auto settle = [&] {                                   // on to a linear of which this wave has a quad
         while (iq >= itotal && it < tokens) {
-            iq = wave;
             if (++ip == phases) { ip = 0; it++; }
-            itotal = word(L.phase[ip].z);
-            ibase = base_of(ip);
+            const int4 ph = L.phase[ip];
+            itotal = word(ph.z);
+            ibase = reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(ph.y) << 32) | (unsigned)word(ph.x));
+            if constexpr (MOE) {
+                const int4 gr = L.group[ip];
+                const int flags = word(gr.w);
+                iq = begins(flags);
+                iorder = flags & 0xFFFF;
+                igroup = word(gr.z);
+            } else {
+                iq = wave;
+                igroup = ip;
+            }
         }
     };
+    auto known = [&] { return it < tokens && (!MOE || iorder == 0 || flag(L.chosen) >= it * routed + iorder); };       // an expert's weights have no address before the choice
     auto ask = [&] {
+        if (MOE && iorder) ibase = base_of(ip);
         quad_to_lds(ibase, (unsigned)iq * kQuad + lane * 16, dst + islot * kQuad);
         islot = islot + 1 == slots ? 0 : islot + 1;
         ahead++;
@@ -181,19 +198,27 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
     };
     settle();
     int slot = 0, n = 0;
+    float xr[4][CE];
     for (int ct = 0; ct < tokens; ct++)
         for (int cp = 0; cp < phases; cp++) {
-            const int total = word(L.phase[cp].z), rq = word(L.phase[cp].w), segs = 4 * rq;       // quads, and those of a row
-            int at = wave;                                // place of the quad in its row
-            while (at >= rq) at -= rq;
-            const bool held = kStrWaves % rq == 0;        // the same in all rows
-            float xr[4][CE];
+            const int4 ph = L.phase[cp];
+            int4 gr = make_int4(0, 0, cp, (int)(3u << 30));
+            if constexpr (MOE) gr = L.group[cp];
+            const int total = word(ph.z), rq = word(ph.w), flags = word(gr.w), cgroup = MOE ? word(gr.z) : cp;
+            const bool half = MOE && rq == 0, first = !MOE || (flags >> 30 & 1), last = !MOE || flags < 0;
+            const int segs = half ? 2 : 4 * rq, from = MOE ? begins(flags) : wave;
+            if (!first && !last && from >= total) continue;
+            const float* x0 = MOE ? xs + word(gr.x) : xs;
+            float* sums = MOE ? red + word(gr.y) : red;
+            int at = from;                                // place of the quad in its row
+            while (!half && at >= rq) at -= rq;
+            const bool held = half || kStrWaves % rq == 0;             // the same in all rows
             auto vector = [&](float (&x)[4][CE], int at) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
                     for (int q = 0; q < PL; q++) {
-                        const f32x4 v = *reinterpret_cast<const f32x4*>(xs + ((q * segs + 4 * at + i) * 64 + lane) * 4);
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(x0 + ((q * segs + (half ? i & 1 : 4 * at + i)) * 64 + lane) * 4);
 #pragma unroll
                         for (int e = 0; e < 4; e++) x[i][q * 4 + e] = v[e];
                     }
@@ -204,8 +229,7 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 slot = slot + 1 == slots ? 0 : slot + 1;
                 ahead--;
             };
-            auto dot = [&](const i32x4 (&u)[4], const float (&x)[4][CE]) {
-                float s[4];
+            auto dots = [&](const i32x4 (&u)[4], const float (&x)[4][CE], float (&s)[4]) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     float wv[CE];
@@ -214,36 +238,44 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
 #pragma unroll
                     for (int e = 0; e < CE; e++) s[i] = fma_f(wv[e], x[i][e], s[i]);
                 }
+            };
+            auto dot = [&](const i32x4 (&u)[4], const float (&x)[4][CE]) {
+                float s[4];
+                dots(u, x, s);
                 return (s[0] + s[1]) + (s[2] + s[3]);
             };
             auto next = [&] {
                 at += kStrWaves;
                 while (at >= rq) at -= rq;
             };
+            auto same = [&] { return igroup == cgroup && it == ct; };
             // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (without that 624 us
             // per token where it is 610; nothing asked for between linears: 658).  When the ring is full, the first two quads move into registers.
             i32x4 u[2][4];
             bool taken = false;
-            n++;
-            while (flag(L.ready) < n) {
-                if (ahead < slots && it < tokens) {
-                    ask();
-                    wait_quads(0);
-                } else if (!taken && ahead >= 2 && wave + kStrWaves < total) {
-                    wait_quads(ahead - 2);
-                    read(u[0]);
-                    read(u[1]);
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
-                    taken = true;
-                } else {
-                    __builtin_amdgcn_s_sleep(1);
+            if (first) {
+                n++;
+                while (flag(L.ready) < n) {
+                    if (ahead < slots && known()) {
+                        ask();
+                        wait_quads(0);
+                    } else if (!taken && ahead >= 2 && !half && from + kStrWaves < total) {
+                        wait_quads(ahead - 2);
+                        read(u[0]);
+                        read(u[1]);
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
+                        taken = true;
+                    } else {
+                        __builtin_amdgcn_s_sleep(1);
+                    }
                 }
+                __syncthreads();                          // the vector is there
+                while (ahead < slots && same()) ask();
             }
-            __syncthreads();                              // the vector is there
-            while (ahead < slots && ip == cp && it == ct) ask();
-            if (wave < total) vector(xr, at);
-            int q = wave;
-            for (; q + kStrWaves < total; q += 2 * kStrWaves) {        // two at a time, which hide each other's latencies
+            // experts' gate/up: all on the one vector, which is still there
+            if (from < total && (first || !held || half || word(gr.x) != 0 || from != wave)) vector(xr, at);
+            int q = from;
+            for (; !half && q + kStrWaves < total; q += 2 * kStrWaves) {       // two at a time, which hide each other's latencies
                 if (!taken) {
                     wait_quads(ahead - 2);
                     read(u[0]);
@@ -255,7 +287,7 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                     v[1] = dot(u[1], xr);
                 } else {
                     float x2[4][CE];
-                    if (q > wave) vector(xr, at);
+                    if (q > from) vector(xr, at);
                     next();
                     vector(x2, at);
                     next();
@@ -264,22 +296,34 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 }
                 if (!taken) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slots have been read
-                    if (ip == cp && it == ct) ask();
-                    if (ip == cp && it == ct) ask();
+                    if (same()) ask();
+                    if (same()) ask();
                 }
                 taken = false;
                 multi_sum_step<2, 1>(v, lane);
-                if (lane < 2) red[q + kStrWaves * lane] = v[0];
+                if (lane < 2) sums[q + kStrWaves * lane] = v[0];
             }
-            if (q < total) {
+            for (; q < total; q += kStrWaves) {           // the last one, or all halves
                 wait_quads(ahead - 1);
                 read(u[0]);
-                if (!held && q > wave) vector(xr, at);
-                const float v = wave_sum(dot(u[0], xr));
-                if (lane == 0) red[q] = v;
+                if (!held && q > from) vector(xr, at);
+                float s[4];
+                dots(u[0], xr, s);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (same()) ask();
+                float v[2] = {s[0] + s[1], s[2] + s[3]};
+                if (half) {
+                    multi_sum_step<2, 1>(v, lane);
+                    if (lane < 2) sums[2 * q + lane] = v[0];
+                } else {
+                    const float o = wave_sum(v[0] + v[1]);
+                    if (lane == 0) sums[q] = o;
+                }
             }
-            __syncthreads();                              // the sums are there
-            while (flag(L.sent) < n) __builtin_amdgcn_s_sleep(1);      // they leave first: a store, too, stands in line
+            if (last) {
+                __syncthreads();                          // the sums are there
+                while (flag(L.sent) < n) __builtin_amdgcn_s_sleep(1);      // they leave first: a store, too, stands in line
+            }
         }
 }
 
@@ -295,7 +339,7 @@ struct Service {
     float *now, *other;                                   // the two sets
     f32x4 x[QW];                                          // residual: float4 t + 256 i
     int normed = 0;                                       // L.norm in turn
-    int meetings = 0, ready = 0, sent = 0;
+    int meetings = 0, ready = 0, sent = 0, chosen = 0;
 
     __device__ __forceinline__ Service(const WalkArgs& a_, WalkLds& L_, float* xs_, float* red_)
         : a(a_), L(L_), xs(xs_), red(red_), t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {
@@ -328,13 +372,13 @@ struct Service {
         unput(at);
     }
     __device__ __forceinline__ void unput(unsigned at) { store_past(other + at, __int_as_float((int)kUnset)); }
-    __device__ __forceinline__ void put_x(int segs, int c, const f32x4& v) {       // float4 c of the vector
+    __device__ __forceinline__ void put_x(int segs, int c, const f32x4& v, int off = 0) {      // float4 c of the vector that starts at off
         const int at = PL == 1 ? c : (c & 1) * segs * 64 + (c >> 1);
-        *reinterpret_cast<f32x4*>(xs + 4 * at) = v;
+        *reinterpret_cast<f32x4*>(xs + off + 4 * at) = v;
     }
-    // total of local row r, of rq quads
-    __device__ __forceinline__ float total(int rq, int r) const {
-        const float* p = red + r * rq;
+    // total of local row r, of rq quads (0: half a one)
+    __device__ __forceinline__ float total(int rq, int r, int off = 0) const {
+        const float* p = red + off + r * (rq > 0 ? rq : 1);
         float s = p[0];
         for (int i = 1; i < rq; i++) s += p[i];
         return s;
@@ -1026,13 +1070,94 @@ struct Service {
         }
     }
 
-    // ---- one token: returns the next one
     __device__ __forceinline__ int rows_of(int n, int& r0) const {
         r0 = walk_rows(n, wg);
         return walk_rows(n, wg + 1) - r0;
     }
+    // ---- mixture of experts.  The choice is every workgroup's own, from the router's outputs; it gives the streams their addresses.
+    __device__ __forceinline__ void mixture(RunPtr r) {
+        const int t = opaque(), lane = t & 63;
+        const int W = a.width, E = r->experts, top = r->top, ff = r->ff, sf = r->shared_ff, kr = (E + 4) / 4 * 4;
+        int r0;
+        int rows = rows_of(2 * sf + kr, r0);
+        __syncthreads();                                  // the sums of [shared gate/up; router; shared gate] are there
+        for (int j = t; j < rows; j += kSvcT) {
+            const int row = r0 + j;
+            if (row >= 2 * sf) {                          // in copies: all workgroups at one line stand in line
+                const float z = total(W / QE, j);
+                for (int c = 0; c < kWalkCopies; c++) put(r->x_route + (unsigned)(c * kr + row - 2 * sf), z);
+            } else if ((row & 1) == 0) {
+                put(r->x_hid + (unsigned)(top * ff + row / 2), glu_f(r->glu, total(W / QE, j), total(W / QE, j + 1), r->shared_limit));
+            }
+        }
+        sums_done();
+        if (wave == 0) {
+            unsigned off[1] = {16u * (unsigned)min(lane, kr / 4 - 1)};
+            f32x4 v[1];
+            poll_words<1>(now + r->x_route + wg % kWalkCopies * kr, off, 4 * lane < kr, v, wait);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (4 * lane + e <= E) L.z[4 * lane + e] = v[0][e];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            int pick;
+            float weight;
+            route_wave(L.z, E, top, pick, weight);
+            pick = min(max(pick, 0), E - 1);              // router outputs that are not numbers choose nobody
+            if (lane < top) {
+                L.choice_w[lane] = weight;
+#pragma unroll
+                for (int k = 0; k < 2; k++) {             // gate/up and down
+                    const int p = r->phase + k * top + lane;
+                    const WalkPhase ph = a.phases[p];
+                    const uintptr_t w = reinterpret_cast<uintptr_t>(static_cast<const ET*>(ph.w) + (size_t)pick * ph.stride + (size_t)walk_rows(ph.n, wg) * ph.kpad);
+                    L.phase[p].x = (int)(unsigned)w;
+                    L.phase[p].y = (int)(unsigned)(w >> 32);
+                }
+            }
+            if (lane == 0) L.choice_w[top] = sigmoid_f(L.z[E]);
+            chosen++;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            say(L.chosen, chosen);
+        }
+        vector_done();                                    // the vector is still the same
+        rows = rows_of(2 * ff, r0);
+        __syncthreads();
+        const int wq = W / QE, all = rows / 2 * top;
+        for (int j = t; j < all; j += kSvcT) {
+            const int s = j / (rows / 2), i = j - s * (rows / 2), o = s * red_rows(2 * ff) * wq;
+            put(r->x_hid + (unsigned)(s * ff + r0 / 2 + i), glu_f(r->glu, total(wq, 2 * i, o), total(wq, 2 * i + 1, o), r->limit));
+        }
+        sums_done();
+        // the vectors of the chosen experts one after the other, then the shared one's
+        const int fsegs = ff / (CE * 64), ssegs = sf / (CE * 64), n4 = (top * ff + sf) / 4;
+        for (int c0 = 0; c0 < n4; c0 += 4 * kSvcT) {
+            unsigned off[4];
+            f32x4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) off[i] = 16u * (unsigned)min(c0 + t + kSvcT * i, n4 - 1);
+            poll_words<4>(now + r->x_hid, off, c0 + wave * 64 < n4, v, wait);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int c = c0 + t + kSvcT * i, s = min(c / (ff / 4), top);
+                if (c < n4) put_x(s < top ? fsegs : ssegs, c - s * (ff / 4), v[i], s * ff);
+            }
+        }
+        vector_done();
+        rows = rows_of(W, r0);
+        __syncthreads();
+        const int fq = ff / QE, sq = sf / QE, step = red_rows(W) * max(fq, 1);
+        for (int j = t; j < rows; j += kSvcT) {
+            float y = 0.0f;
+            for (int s = 0; s < top; s++) y = fma_f(L.choice_w[s], total(fq, j, s * step), y);
+            put(r->x_y2 + (unsigned)(r0 + j), fma_f(L.choice_w[top], total(sq, j, top * step), y));
+        }
+        sums_done();
+    }
+
+    // ---- one token: returns the next one
     // the sums of a linear of n rows of k leave as they are
     __device__ __forceinline__ void plain(int n, int k, unsigned at, const float* bias) {
+        const int t = opaque();
         int r0;
         const int rows = rows_of(n, r0);
         const float b = bias && t < rows ? *global(bias + r0 + t) : 0.0f;      // under the products
@@ -1066,6 +1191,12 @@ struct Service {
             have = true; y = r->x_y; gb = r->g1b;
             if (r->ff == 0) continue;
             norm(true, y, gb, r->g2, -1);
+            y = r->x_y2; gb = r->g2b;
+            if constexpr (KIND == kWalkMixture)
+                if (r->experts) {
+                    mixture(r);
+                    continue;
+                }
             __syncthreads();
             int r0;
             const int rows = rows_of(2 * r->ff, r0);
@@ -1074,7 +1205,6 @@ struct Service {
             sums_done();
             take(r->x_hid, r->ff);
             plain(W, r->ff, r->x_y2, nullptr);
-            y = r->x_y2; gb = r->g2b;
         }
         if (!choose && t < 2) unput(a.x_cand + (unsigned)(2 * wg + t));        // what is not handed out in this step is unset behind the last one all the same
         if (!a.head) return 0;
@@ -1120,7 +1250,7 @@ struct Service {
     }
 };
 
-// KIND: models of shared key/value rows, or of latent rows and gated linear attention (kWalkLatent)
+// KIND: models of shared key/value rows, of latent rows and gated linear attention (kWalkLatent), or of those with mixtures of experts
 template <typename ET, int QW, int KIND>
 __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
     constexpr int QE = kQuad / sizeof(ET);
@@ -1133,12 +1263,14 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
         const WalkPhase ph = a.phases[p];
         const int r0 = walk_rows(ph.n, blockIdx.x), rows = walk_rows(ph.n, blockIdx.x + 1) - r0, rq = ph.kpad / QE;
         const uintptr_t w = reinterpret_cast<uintptr_t>(static_cast<const ET*>(ph.w) + (size_t)r0 * ph.kpad);
-        L.phase[p] = make_int4((int)(unsigned)w, (int)(unsigned)(w >> 32), rows * rq, rq);
+        // choices of few quads begin with another wave in turn
+        L.phase[p] = make_int4((int)(unsigned)w, (int)(unsigned)(w >> 32), rq ? rows * rq : rows / 2, rq);
+        L.group[p] = make_int4(ph.x_off, ph.red_off, ph.group, (int)((unsigned)ph.last << 31 | (unsigned)ph.first << 30 | (unsigned)(rq == 0 && ph.slot & 1 ? kStrWaves / 2 : 0) << 16 | (unsigned)ph.routed));
     }
-    if (threadIdx.x == 0) L.met = L.ready = L.sent = 0;
+    if (threadIdx.x == 0) L.met = L.ready = L.sent = L.chosen = 0;
     __syncthreads();
     if (threadIdx.x >= kSvcT) {
-        stream_waves<ET>(L, xs, red, reinterpret_cast<const char*>(red + a.lds_red), slots, phases, a.steps);
+        stream_waves<ET, KIND == kWalkMixture>(L, xs, red, reinterpret_cast<const char*>(red + a.lds_red), slots, phases, a.steps, a.routed);
         return;
     }
     Service<ET, QW, KIND> s(a, L, xs, red);
@@ -1169,7 +1301,7 @@ static_assert(kStrWaves * kQuad == kWalkSlotBytes && kQuad == kWalkRow, "a quad 
 
 template <typename ET>
 int walk_launch(const WalkArgs& a, hipStream_t st) {
-    FX_REQUIRE(a.n_phases + 1 <= kWalkMaxPhases && a.width % 512 == 0 && a.width <= kWalkMaxWidth && a.vocab >= kWalkWG && a.steps > 0, "walk: %d linears, width %d, vocabulary %d", a.n_phases, a.width, a.vocab);
+    FX_REQUIRE(a.n_phases < kWalkMaxPhases && a.width % 512 == 0 && a.width <= kWalkMaxWidth && a.vocab >= kWalkWG && a.steps > 0, "walk: %d linears, width %d, vocabulary %d", a.n_phases, a.width, a.vocab);
     const size_t used = walk_lds(a);
     FX_REQUIRE(used + kWalkMinSlots * kWalkSlotBytes <= kWalkLdsMax, "walk: %zu bytes of LDS", used);
     int slots = (int)((kWalkLdsMax - used) / kWalkSlotBytes);
@@ -1184,8 +1316,9 @@ int walk_launch(const WalkArgs& a, hipStream_t st) {
         FX_LAUNCH_CHECK();
         return FLEXLLM_OK;
     };
-    static std::atomic<bool> opted[4];
+    static std::atomic<bool> opted[6];
     if (a.kind == kWalkSharedKv) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkSharedKv>, opted[0]) : go(walk_kernel<ET, 4, kWalkSharedKv>, opted[1]);
+    if (a.routed) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkMixture>, opted[4]) : go(walk_kernel<ET, 4, kWalkMixture>, opted[5]);
     return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkLatent>, opted[2]) : go(walk_kernel<ET, 4, kWalkLatent>, opted[3]);
 }
 template int walk_launch<bf16_t>(const WalkArgs&, hipStream_t);

@@ -4,62 +4,12 @@
 // The first two groups are requested before the prologue (residual, norms) runs, so that its latency lies under the weight
 // stream, and two groups stay in flight after that.  The R sums are reduced together (multi_sum_step).
 #include "float_ops.h"
+#include "route.h"
 #include <atomic>
 
 namespace fx {
 
-constexpr int kMaxExperts = 1024, kMaxTop = 32;
 constexpr size_t kGemvTokensLds = 128 * 1024;             // vectors of gemv_tokens_kernel
-
-// Expert choice of one token by one wave: softmax over the router outputs, the `top` largest (ties: lower index), their
-// weights divided by their sum.  Lane k < top gets choice k and its weight.  NE: 64-expert pieces (experts <= 64 NE).
-template <int NE>
-__device__ __forceinline__ void route_wave_n(const float* __restrict__ z, int experts, int top, int& pick, float& weight) {
-    const int lane = threadIdx.x & 63;
-    float v[NE];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < NE; i++) {
-        v[i] = i * 64 + lane < experts ? z[i * 64 + lane] : -INFINITY;
-        mx = fmaxf(mx, v[i]);
-    }
-    mx = wave_max(mx);
-    float den = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NE; i++) {
-        v[i] = i * 64 + lane < experts ? exp_f<false>(v[i] - mx) : -1.0f;
-        den += fmaxf(v[i], 0.0f);
-    }
-    den = wave_sum(den);
-    float sum = 0.0f;
-    pick = 0;
-    weight = 0.0f;
-    for (int k = 0; k < top; k++) {
-        float best = v[0];
-#pragma unroll
-        for (int i = 1; i < NE; i++) best = fmaxf(best, v[i]);
-        best = wave_max(best);
-        int bi = -1;                                      // lowest index that holds the maximum
-#pragma unroll
-        for (int i = 0; i < NE; i++) {
-            const unsigned long long hit = __ballot(v[i] == best);
-            if (bi < 0 && hit) {
-                const int l = __builtin_ctzll(hit);
-                bi = i * 64 + l;
-                if (lane == l) v[i] = -1.0f;
-            }
-        }
-        const float s = best / den;
-        sum += s;
-        if (lane == k) { pick = bi; weight = s; }
-    }
-    weight = weight / (sum + 1e-20f);
-}
-__device__ __forceinline__ void route_wave(const float* __restrict__ z, int experts, int top, int& pick, float& weight) {
-    if (experts <= 64) route_wave_n<1>(z, experts, top, pick, weight);
-    else if (experts <= 256) route_wave_n<4>(z, experts, top, pick, weight);
-    else route_wave_n<kMaxExperts / 64>(z, experts, top, pick, weight);
-}
 
 // VEC: the prologue keeps its vectors in registers as float4 (k a multiple of 4, at most what the S pieces per thread cover);
 // else any k, through LDS.  NT: the weights are read once on this chip and are requested as such (non-temporal): what they

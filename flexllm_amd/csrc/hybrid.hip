@@ -388,19 +388,30 @@ static int create_walk(flexllm_hybrid* m) {
     for (const HybridLayer& L : m->layers) {
         ok = ok && (L.d.mixer == FLEXLLM_MIX_SHARED_KV) == shared && L.n_in >= few && L.k_o % unit == 0 && L.k_o <= kWalkMaxWidth;
         ok = ok && (L.d.mixer == FLEXLLM_MIX_SHARED_KV ? walk_shared_kv_ok(L.sd) : L.d.mixer == FLEXLLM_MIX_LATENT ? walk_latent_ok(L.ld) : walk_gla_ok(L.gd));
-        ok = ok && (L.d.ff_kind == FLEXLLM_FF_NONE || (L.d.ff_kind == FLEXLLM_FF_DENSE && L.d.ff % unit == 0 && 2 * L.d.ff >= few));
+        const auto rows = [&](int k) { return k % unit == 0 || 2 * k == unit; };           // of whole quads, or of half a one
+        if (L.d.ff_kind == FLEXLLM_FF_DENSE) ok = ok && L.d.ff % unit == 0 && 2 * L.d.ff >= few;
+        if (L.d.ff_kind == FLEXLLM_FF_MOE)
+            ok = ok && !shared && L.d.shared_ff > 0 && rows(L.d.ff) && rows(L.d.shared_ff) && 2 * L.d.ff >= few && L.n_side >= few && L.d.experts <= kWalkExperts && L.d.top <= kWalkTop;
     }
     if (!ok) return FLEXLLM_OK;
     std::vector<WalkPhase> phases;
     std::vector<WalkRun> runs;
     WalkArgs& a = m->walk;
     size_t at = 0, longest = 0, sums = 0;
-    auto linear = [&](const void* w, int n, int k) {
-        phases.push_back({w, n, k});
-        const size_t rows = 2 * (size_t)(((n + 1) / 2 + kWalkWG - 1) / kWalkWG), s = rows * (k / unit);
-        if ((size_t)k > longest) longest = k;
-        if (s > sums) sums = s;
+    // Linears that nobody waits between are a group: experts' products of a token, whose vectors and sums lie side by side.
+    int groups = 0;
+    size_t x_off = 0, red_off = 0;
+    auto one = [&](const void* w, int n, int k, bool first, bool last, int routed = 0, int slot = 0, size_t stride = 0, bool same_x = false) {
+        const int rq = k / unit;
+        if (first) x_off = red_off = 0;
+        phases.push_back({w, n, k, groups, first, last, routed, slot, stride, (int)x_off, (int)red_off});
+        if (!same_x) x_off += k;
+        red_off += (size_t)red_rows(n) * (rq ? rq : 1);
+        if ((same_x ? (size_t)k : x_off) > longest) longest = same_x ? k : x_off;
+        if (red_off > sums) sums = red_off;
+        if (last) groups++;
     };
+    auto linear = [&](const void* w, int n, int k) { one(w, n, k, true, true); };
     auto words = [&](size_t n) {
         const size_t p = at;
         at += (n + 63) / 64 * 64;
@@ -436,7 +447,16 @@ static int create_walk(flexllm_hybrid* m) {
                 r.x_att = words(r.k_o); r.x_y = words(W);
                 linear(L.w_in, L.n_in, W);
                 linear(L.w_o, W, L.k_o);
-                if (r.ff) {
+                if (L.d.ff_kind == FLEXLLM_FF_MOE) {
+                    r.experts = L.d.experts; r.top = L.d.top; r.shared_ff = L.d.shared_ff; r.shared_limit = L.d.shared_limit;
+                    r.x_route = words((size_t)kWalkCopies * up4(r.experts + 1)); r.x_hid = words((size_t)r.top * r.ff + r.shared_ff); r.x_y2 = words(W);
+                    linear(L.w_side, L.n_side, W);
+                    r.phase = (int)phases.size();
+                    a.routed++;
+                    for (int k = 0; k < r.top; k++) one(L.w_gu, 2 * r.ff, W, k == 0, k == r.top - 1, a.routed, k, (size_t)2 * r.ff * W, true);
+                    for (int k = 0; k < r.top; k++) one(L.w_d, W, r.ff, k == 0, false, a.routed, k, (size_t)W * r.ff);
+                    one(L.w_sd, W, r.shared_ff, false, true);
+                } else if (r.ff) {
                     r.x_hid = words(r.ff); r.x_y2 = words(W);
                     linear(L.w_gu, 2 * r.ff, W);
                     linear(L.w_d, W, r.ff);
@@ -449,16 +469,21 @@ static int create_walk(flexllm_hybrid* m) {
     linear(m->head, c.vocab, W);
     a.x_cand = words(2 * kWalkWG);
     a.lds_xs = (int)longest; a.lds_red = (int)((sums + 255) / 256 * 256);
-    if (a.n_phases + 1 > kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || walk_lds(a) + kWalkMinSlots * kWalkSlotBytes > kWalkLdsMax) return FLEXLLM_OK;
-    WalkPhase* dev_phases;
-    FX_TRY(own(m, dev_phases, phases.size()));
-    FX_TRY(own(m, m->walk_runs, runs.size()));
-    FX_HIP(hipMemcpy(dev_phases, phases.data(), sizeof(WalkPhase) * phases.size(), hipMemcpyHostToDevice));
-    FX_HIP(hipMemcpy(m->walk_runs, runs.data(), sizeof(WalkRun) * runs.size(), hipMemcpyHostToDevice));
+    if (a.n_phases >= kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || walk_lds(a) + kWalkMinSlots * kWalkSlotBytes > kWalkLdsMax) return FLEXLLM_OK;
+    // one piece of memory: the words, the flag, the tables
     a.set = at;
-    FX_TRY(own(m, a.words, 2 * at));
-    FX_HIP(hipMemset(a.words, 0xFF, 2 * at * sizeof(float)));
-    FX_TRY(own(m, a.err, 1));
+    const size_t words_bytes = 2 * at * sizeof(float), runs_at = 256, phases_at = runs_at + sizeof(WalkRun) * runs.size();
+    std::vector<char> tables(phases_at + sizeof(WalkPhase) * phases.size(), 0);
+    memcpy(&tables[runs_at], runs.data(), sizeof(WalkRun) * runs.size());
+    memcpy(&tables[phases_at], phases.data(), sizeof(WalkPhase) * phases.size());
+    char* mem;
+    FX_TRY(own(m, mem, words_bytes + tables.size()));
+    FX_HIP(hipMemset(mem, 0xFF, words_bytes));
+    FX_HIP(hipMemcpy(mem + words_bytes, tables.data(), tables.size(), hipMemcpyHostToDevice));
+    a.words = reinterpret_cast<float*>(mem);
+    a.err = reinterpret_cast<int*>(mem + words_bytes);
+    m->walk_runs = reinterpret_cast<WalkRun*>(mem + words_bytes + runs_at);
+    const WalkPhase* dev_phases = reinterpret_cast<WalkPhase*>(mem + words_bytes + phases_at);
     a.kind = shared ? kWalkSharedKv : kWalkLatent;
     a.n_runs = n_runs; a.width = W; a.vocab = c.vocab; a.eps = c.eps; a.embed_scale = c.embed_scale;
     a.embed = as_bf16(m->embed); a.g_final = m->g_final;

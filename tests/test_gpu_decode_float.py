@@ -51,6 +51,24 @@ NIFUNEX = {
 }
 
 
+# the experts' rows a half of what a wave asks for at a time, and whole; few experts, one choice, the most choices
+MIXTURES = {
+    "rows of half a quad in bfloat16": (8, 3, 1024, 2048),
+    "rows of half a quad in float32": (5, 1, 512, 1024),
+    "rows of a quad": (3, 2, 2048, 4096),
+    "all of many": (16, 16, 1024, 2048),
+}
+
+
+@BOTH
+@pytest.mark.parametrize("name", list(MIXTURES))
+def test_mixtures(name, dtype):
+    experts, top, ff, shared = MIXTURES[name]
+    moe = dict(mlp=nc.moe(experts, top, ff, 0.75, shared))
+    cfg = nc.config([nc.gla(heads=16, dim=128, vdim=128, **moe), nc.latent(heads=16, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5, **moe)], width=2048, vocab=512)
+    check_nifunex(cfg, dtype, 40, [1], [30, 1])
+
+
 @BOTH
 @pytest.mark.parametrize("name", list(NIFUNEX))
 def test_token_by_token_nifunex(name, dtype):
