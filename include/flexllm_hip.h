@@ -585,7 +585,8 @@ int flexllm_hybrid_step(flexllm_hybrid* m, int slot, const int* tokens, int n, c
                         float* layers_out, void* stream);
 /* `steps` tokens from *token_io (device; fed first, the last drawn token on return) into tokens_out (device [steps]):
  * the largest logit, or with top_k > 0 a draw from the top_k largest with rands[step] (device).  use_graph: one step is
- * captured in a HIP graph and replayed (needs a stream of its own). */
+ * captured in a HIP graph and replayed (needs a stream of its own).  Where the sizes allow it, greedy steps run in one resident kernel
+ * instead, which needs the whole chip and keeps its turn with others of its kind; flexllm_hybrid_check reports a wait that timed out. */
 int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps, const float* rands, int top_k, int* tokens_out,
                           int use_graph, void* stream);
 /* Prompt to tokens in one slot: all prompt tokens but the last in one go, then the decode loop from the last one. */

@@ -87,8 +87,8 @@ def test_splits_of_latent_rows(heads, window, dtype):
 @pytest.mark.parametrize("dim", [64, 128])
 def test_splits_of_the_rows(dim, dtype):
     """Around the number of rows from which on there are several splits, and where all of them have some."""
-    borders = {64: (64, 256), 128: (32, 128)}[dim]
-    for rows in {"bfloat16": borders[1], "float32": borders[1] // 2}[dtype], 8 * borders[1]:
+    alone = {64: 256, 128: 128}[dim] // (1 if dtype == "bfloat16" else 2)
+    for rows in alone, 8 * alone:
         check_lopazen(lc.config([attention(32, 8, dim, 0)], width=2048, vocab=512), dtype, rows + 5, [rows - 5, 1], max_pos=2112)
 
 
