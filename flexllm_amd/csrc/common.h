@@ -1,9 +1,12 @@
 // Shared device helpers and host-side error plumbing for libflexllm_hip (gfx950 only).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <tuple>
 #include "../../include/flexllm_hip.h"
+#include "resident.h"
 
 namespace fx {
 
@@ -53,20 +56,20 @@ enum ScratchKind { kScratchArgmax = 0, kScratchTopK = 1, kScratchMhaDecode = 2, 
 int stream_scratch(ScratchKind kind, hipStream_t st, size_t bytes, void** out);
 void stream_scratch_release(hipStream_t st);
 
-// Launches of kernels whose workgroups wait for each other and so have to be resident all at once.  Two of them side by side could each
-// hold a part of the chip and wait for the rest of it, so on a device they run one after the other, whatever streams they are
-// launched on: one on another stream than the last waits for that stream.  (Kernels of other kinds end by themselves.)  In a
-// stream that is being captured there is no such order to keep.
-int resident_begin(hipStream_t st, bool& ordered);       // takes the device's turn
-int resident_end(hipStream_t st, bool ordered);
-template <class F>
-int resident_launch(hipStream_t st, F launch) {
-    bool ordered = false;
-    int rc = resident_begin(st, ordered);
-    if (rc) return rc;
-    rc = launch();
-    const int end = resident_end(st, ordered);
-    return rc ? rc : end;
+// Launch of a kernel whose workgroups wait for each other, in turn with the others of its kind (resident.h): its last parameter is a
+// ResidentEnd, a... are the ones ahead of it.
+int resident_launch_args(const void* kernel, int grid, int block, void** args, size_t lds, hipStream_t st, ResidentEnd& end);
+int resident_ready();                      // at the creation of what launches them
+template <class... P, class... A>
+int resident_launch(void (*kernel)(P...), int grid, int block, size_t lds, hipStream_t st, const A&... a) {
+    std::tuple<P...> values(a..., ResidentEnd{nullptr, 0});
+    return std::apply([&](P&... v) {
+        void* args[] = {&v...};
+        return resident_launch_args(reinterpret_cast<const void*>(kernel), grid, block, args, lds, st, std::get<sizeof...(P) - 1>(values));
+    }, values);
+}
+__device__ __forceinline__ void resident_done(const ResidentEnd& end) {
+    if (end.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(end.word, end.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- cross-lane exchange

@@ -1252,7 +1252,7 @@ struct Service {
 
 // KIND: models of shared key/value rows, of latent rows and gated linear attention (kWalkLatent), or of those with mixtures of experts
 template <typename ET, int QW, int KIND>
-__global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
+__global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, ResidentEnd end) {
     constexpr int QE = kQuad / sizeof(ET);
     extern __shared__ __attribute__((aligned(16))) char lds[];
     WalkLds& L = *reinterpret_cast<WalkLds*>(lds);
@@ -1293,6 +1293,7 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots) {
         a.state[0] = pos0 + a.steps;
         a.state[1] = step0 + a.steps;
     }
+    resident_done(end);
 }
 
 // What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.
@@ -1312,9 +1313,7 @@ int walk_launch(const WalkArgs& a, hipStream_t st) {
             FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWalkLdsMax));
             opted_in.store(true, std::memory_order_release);
         }
-        k<<<kWalkWG, kWalkT, lds, st>>>(a, slots);
-        FX_LAUNCH_CHECK();
-        return FLEXLLM_OK;
+        return resident_launch(k, kWalkWG, kWalkT, lds, st, a, slots);
     };
     static std::atomic<bool> opted[6];
     if (a.kind == kWalkSharedKv) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkSharedKv>, opted[0]) : go(walk_kernel<ET, 4, kWalkSharedKv>, opted[1]);

@@ -1393,7 +1393,13 @@ __device__ __forceinline__ void decode_mega_body(const MegaParams& p) {
 #endif
 }
 
-__global__ __launch_bounds__(kMegaT, 1) void decode_mega_kernel(MegaParams p) { decode_mega_body<false>(p); }
-__global__ __launch_bounds__(kMegaT, 1) void decode_mega_w4_kernel(MegaParams p) { decode_mega_body<true>(p); }
+__global__ __launch_bounds__(kMegaT, 1) void decode_mega_kernel(MegaParams p, ResidentEnd end) {
+    decode_mega_body<false>(p);
+    resident_done(end);
+}
+__global__ __launch_bounds__(kMegaT, 1) void decode_mega_w4_kernel(MegaParams p, ResidentEnd end) {
+    decode_mega_body<true>(p);
+    resident_done(end);
+}
 
 }  // namespace fx

@@ -394,6 +394,7 @@ static int create_walk(flexllm_hybrid* m) {
             ok = ok && !shared && L.d.shared_ff > 0 && rows(L.d.ff) && rows(L.d.shared_ff) && 2 * L.d.ff >= few && L.n_side >= few && L.d.experts <= kWalkExperts && L.d.top <= kWalkTop;
     }
     if (!ok) return FLEXLLM_OK;
+    FX_TRY(resident_ready());
     std::vector<WalkPhase> phases;
     std::vector<WalkRun> runs;
     WalkArgs& a = m->walk;
@@ -930,7 +931,7 @@ static int walk(flexllm_hybrid* m, int slot, int* token, int steps, int* tokens_
         a.token = token; a.tokens_out = tokens_out; a.logits = logits; a.head = head;
         a.steps = steps - done < kWalkLaunch ? steps - done : kWalkLaunch;
         a.parity = m->walk_steps & 1;
-        FX_TRY(resident_launch(st, [&] { return m->cfg.dtype == 0 ? walk_launch<bf16_t>(a, st) : walk_launch<float>(a, st); }));
+        FX_TRY(m->cfg.dtype == 0 ? walk_launch<bf16_t>(a, st) : walk_launch<float>(a, st));
         m->walk_steps += a.steps;
         done += a.steps;
     }

@@ -192,12 +192,7 @@ static int launch_mega(flexllm_llama* m, int* token, const float* x_in, float* l
     // An ordinary launch: one workgroup per CU fits by construction (mega_ok checks the CU count), and every barrier
     // and poll in the kernel is bounded, so work of other streams that delays some workgroups costs time, not a hang.
     // (A cooperative launch gives the same timing, but rocprofv3 of this ROCm release crashes at exit after one.)
-    return resident_launch(st, [&] {
-        if (m->w4) decode_mega_w4_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
-        else decode_mega_kernel<<<kMegaWG, kMegaT, sizeof(MegaLds), st>>>(p);
-        FX_LAUNCH_CHECK();
-        return FLEXLLM_OK;
-    });
+    return resident_launch(m->w4 ? decode_mega_w4_kernel : decode_mega_kernel, kMegaWG, kMegaT, sizeof(MegaLds), st, p);
 }
 
 static inline bool use_mega(const flexllm_llama* m) { return m->mega_ok && m->decode_mode == 0; }
@@ -349,6 +344,7 @@ int flexllm_llama_create(flexllm_llama** out, const flexllm_llama_config* cfg, c
         // the persistent kernel needs all its workgroups resident at once and is compiled for these shapes
         m->mega_ok = cus >= kMegaWG && c.hidden == 2048 && c.kv_hidden == 512 && c.inter == 8192 && c.q_heads == 32 &&
                      c.kv_heads == 8 && c.max_pos <= 32 * kChunk && kArgmaxParts >= kMegaWG;
+        if (m->mega_ok) FX_TRY(resident_ready());
     }
     FX_TRY_HIP(hipDeviceSynchronize());
 #undef FX_TRY

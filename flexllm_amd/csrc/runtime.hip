@@ -3,7 +3,6 @@
 #include <hip/hip_fp16.h>
 #include <map>
 #include <mutex>
-#include <set>
 #include <stdarg.h>
 #include <string.h>
 #include <tuple>
@@ -61,66 +60,13 @@ void stream_scratch_release(hipStream_t st) {
     }
 }
 
-namespace {
-// Per device: the stream of the last of these launches, and an event behind it.  An event costs 17 us of the stream's time, so on streams
-// whose end is known here (those of flexllm_rt_stream_create, and the null stream, which has none) it is recorded only when a
-// launch on another stream has to wait; on all others at once, since they could be gone by then.
-struct Resident { hipStream_t last = nullptr; hipEvent_t event = nullptr; bool any = false, recorded = false; };
-std::mutex g_resident_mu;
-std::map<int, Resident> g_resident;
-std::set<hipStream_t> g_own_streams;
-}  // namespace
-
-int resident_begin(hipStream_t st, bool& ordered) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    FX_HIP(hipStreamIsCapturing(st, &cap));
-    ordered = cap == hipStreamCaptureStatusNone;
-    if (!ordered) return FLEXLLM_OK;
-    int dev = 0;
-    FX_HIP(hipGetDevice(&dev));
-    g_resident_mu.lock();                                // the order of launches and of their events is one: held until resident_end
-    auto turn = [&] {
-        Resident& r = g_resident[dev];
-        if (!r.event) FX_HIP(hipEventCreateWithFlags(&r.event, hipEventDisableTiming));
-        if (!r.any || (!r.recorded && r.last == st)) return FLEXLLM_OK;
-        if (!r.recorded) {
-            FX_HIP(hipStreamIsCapturing(r.last, &cap));
-            if (cap != hipStreamCaptureStatusNone) return FLEXLLM_OK;      // cannot be waited for; the launch was ahead of the capture
-            const hipError_t idle = hipStreamQuery(r.last);
-            if (idle == hipSuccess) { r.any = false; return FLEXLLM_OK; }
-            (void)hipGetLastError();                     // "not ready" is no error of the next launch
-            FX_HIP(hipEventRecord(r.event, r.last));
-            r.recorded = true;
-        }
-        FX_HIP(hipStreamWaitEvent(st, r.event, 0));
-        return FLEXLLM_OK;
-    };
-    const int rc = turn();
-    if (rc) { ordered = false; g_resident_mu.unlock(); }
-    return rc;
-}
-int resident_end(hipStream_t st, bool ordered) {
-    if (!ordered) return FLEXLLM_OK;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) {
-        Resident& r = g_resident[dev];
-        r.last = st;
-        r.any = true;
-        r.recorded = st && !g_own_streams.count(st);
-        if (r.recorded) e = hipEventRecord(r.event, st);
-    }
-    g_resident_mu.unlock();
-    FX_HIP(e);
+int resident_launch_args(const void* kernel, int grid, int block, void** args, size_t lds, hipStream_t st, ResidentEnd& end) {
+    FX_HIP(resident_run(kernel, grid, block, args, lds, st, end));
     return FLEXLLM_OK;
 }
-// A stream of this library begins, or ends with all its work done.
-void own_stream(hipStream_t st, bool there) {
-    std::lock_guard<std::mutex> lk(g_resident_mu);
-    if (there) { g_own_streams.insert(st); return; }
-    g_own_streams.erase(st);
-    for (auto& r : g_resident)
-        if (r.second.any && r.second.last == st && !r.second.recorded) r.second.any = false;      // it has been waited for
+int resident_ready() {
+    FX_HIP(resident_prepare());
+    return FLEXLLM_OK;
 }
 
 // SplitMix64 of (seed, index): the same sequence as flexllm_amd.synth.splitmix64 on the host.
@@ -208,13 +154,11 @@ int flexllm_rt_stream_create(void** stream) {
     FX_REQUIRE(stream, "stream is null");
     hipStream_t s;
     FX_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    own_stream(s, true);
     *stream = s;
     return FLEXLLM_OK;
 }
 int flexllm_rt_stream_destroy(void* stream) {
     FX_HIP(hipStreamSynchronize(as_stream(stream)));
-    own_stream(as_stream(stream), false);
     stream_scratch_release(as_stream(stream));         // the stand-alone entry points' scratch of this stream
     FX_HIP(hipStreamDestroy(as_stream(stream)));
     return FLEXLLM_OK;
