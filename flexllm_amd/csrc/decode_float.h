@@ -7,6 +7,7 @@ namespace fx {
 constexpr int kWalkWG = 256;               // workgroups, one per CU: all of them have to be resident at once
 constexpr int kWalkCopies = 8;            // of few words that every workgroup reads
 constexpr int kWalkMaxPhases = 256;
+constexpr int kWalkPolls = 1 << 20;        // about a second
 constexpr int kWalkMaxWidth = 4096;
 constexpr size_t kWalkLdsMax = 160 * 1024;
 constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 8, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
@@ -65,7 +66,9 @@ struct WalkArgs {
     size_t set;
     unsigned x_cand;                       // candidates of the arg-max
     int parity;                            // set of the first token
-    int* err;                              // raised when a wait has timed out
+    int* err;                              // raised when a wait has timed out, and
+    int* told;                             // the same in host memory
+    int polls;                             // of a word, behind which a wait times out
     int* state;                            // HybridSlot::pos
     int* token;                            // token fed in; after greedy steps the last one found
     int* tokens_out;                       // greedy steps: tokens_out[state[1] + step]; null: a single step

@@ -14,7 +14,8 @@
 // which holds kUnset until then; readers poll the places themselves, 16 bytes per lane.  There are two sets of places, for tokens in
 // turn: who writes a word of one set puts kUnset back in the other one, whose readers were done a token ago (a token ends with an exchange that all
 // workgroups take part in, or with the kernel).  A result that happens to have kUnset's bits leaves as another NaN.
-// All waits are bounded: a wait that times out raises a flag, everybody then runs to the end without waiting.
+// All waits are bounded: a wait that times out raises a flag, everybody then runs to the end without waiting.  The host has a copy of the
+// flag, and refuses further steps until it has been asked for.
 #include "decode_float.h"
 #include "route.h"
 #include <atomic>
@@ -23,7 +24,7 @@ namespace fx {
 
 constexpr int kSvcWaves = 4, kSvcT = kSvcWaves * 64, kStrWaves = 8, kWalkT = kSvcT + kStrWaves * 64;
 constexpr unsigned kUnset = 0xFFFFFFFFu;
-constexpr int kWalkSpin = 1 << 20, kWalkErrPeriod = 64;
+constexpr int kWalkErrPeriod = 64;
 constexpr int kQuad = 4096;                               // bytes that a stream wave asks for at a time: 4 x 16 per lane
 
 // Pointers out of tables are global ones: as the generic ones that the compiler takes them for, their loads would count as LDS accesses
@@ -35,12 +36,17 @@ using RunPtr = const WalkRun __attribute__((address_space(4)))*;       // read-o
 __device__ __forceinline__ bool unset(float v) { return (unsigned)__float_as_int(v) == kUnset; }
 
 struct Wait {
-    int* err;
+    const WalkArgs& a;
     bool dead;
     __device__ __forceinline__ bool give_up(int it) {
-        if (it % kWalkErrPeriod != 0) return false;
-        if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) dead = true;
-        else if (it >= kWalkSpin) { __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); dead = true; }
+        if (it % kWalkErrPeriod != 0 && it < a.polls) return false;
+        if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+            dead = true;
+        } else if (it >= a.polls) {
+            __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.told, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            dead = true;
+        }
         return dead;
     }
 };
@@ -334,18 +340,15 @@ struct Service {
     const WalkArgs& a;
     WalkLds& L;
     float *xs, *red;
-    const int t, lane, wave, wg;
     Wait wait;
+    const int t, lane, wave, wg;
     float *now, *other;                                   // the two sets
     f32x4 x[QW];                                          // residual: float4 t + 256 i
     int normed = 0;                                       // L.norm in turn
     int meetings = 0, ready = 0, sent = 0, chosen = 0;
 
     __device__ __forceinline__ Service(const WalkArgs& a_, WalkLds& L_, float* xs_, float* red_)
-        : a(a_), L(L_), xs(xs_), red(red_), t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {
-        wait.err = a.err;
-        wait.dead = false;
-    }
+        : a(a_), L(L_), xs(xs_), red(red_), wait{a_, false}, t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {}
     // The thread's number as the compiler does not know it: addresses made of it are not kept in registers from layer to layer.
     __device__ __forceinline__ int opaque() const {
         int v = threadIdx.x;

@@ -98,6 +98,8 @@ struct flexllm_hybrid {
     fx::WalkArgs walk = {};
     fx::WalkRun* walk_runs = nullptr;         // [slots][runs]
     unsigned walk_steps = 0;                  // steps taken so far
+    int walk_polls = fx::kWalkPolls;
+    int* told = nullptr;                      // host memory: a wait of a step has timed out
 };
 
 namespace fx {
@@ -471,6 +473,10 @@ static int create_walk(flexllm_hybrid* m) {
     a.x_cand = words(2 * kWalkWG);
     a.lds_xs = (int)longest; a.lds_red = (int)((sums + 255) / 256 * 256);
     if (a.n_phases >= kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || walk_lds(a) + kWalkMinSlots * kWalkSlotBytes > kWalkLdsMax) return FLEXLLM_OK;
+    void* told = nullptr;
+    FX_HIP(hipHostMalloc(&told, 64, hipHostMallocPortable));
+    a.told = m->told = static_cast<int*>(told);
+    *m->told = 0;
     // one piece of memory: the words, the flag, the tables
     a.set = at;
     const size_t words_bytes = 2 * at * sizeof(float), runs_at = 256, phases_at = runs_at + sizeof(WalkRun) * runs.size();
@@ -931,6 +937,7 @@ static int walk(flexllm_hybrid* m, int slot, int* token, int steps, int* tokens_
         a.token = token; a.tokens_out = tokens_out; a.logits = logits; a.head = head;
         a.steps = steps - done < kWalkLaunch ? steps - done : kWalkLaunch;
         a.parity = m->walk_steps & 1;
+        a.polls = m->walk_polls;
         FX_TRY(m->cfg.dtype == 0 ? walk_launch<bf16_t>(a, st) : walk_launch<float>(a, st));
         m->walk_steps += a.steps;
         done += a.steps;
@@ -1022,7 +1029,22 @@ int flexllm_hybrid_destroy(flexllm_hybrid* m) {
     if (m->graph) (void)hipGraphExecDestroy(m->graph);
     for (void* p : m->pool) (void)hipFree(p);
     for (void* p : m->owned) (void)hipFree(p);
+    if (m->told) (void)hipHostFree(m->told);
     delete m;
+    return FLEXLLM_OK;
+}
+
+int flexllm_hybrid_timed_out(const flexllm_hybrid* m) {
+    FX_REQUIRE(m, "hybrid_timed_out: null pointer");
+    if (m->told && __atomic_load_n(m->told, __ATOMIC_ACQUIRE)) {
+        set_error("decode: a wait timed out (were all %d workgroups resident?); what the slots hold is in no known state", kWalkWG);
+        return FLEXLLM_EHIP;
+    }
+    return FLEXLLM_OK;
+}
+int flexllm_hybrid_set_wait_limit(flexllm_hybrid* m, int polls) {
+    FX_REQUIRE(m && polls >= 0, "hybrid_set_wait_limit: %d polls", polls);
+    m->walk_polls = polls ? polls : kWalkPolls;
     return FLEXLLM_OK;
 }
 
@@ -1044,6 +1066,7 @@ int flexllm_hybrid_step(flexllm_hybrid* m, int slot, const int* tokens, int n, c
     FX_REQUIRE(m->slots[slot].length + n <= m->cfg.max_pos, "hybrid_step: %d tokens on top of %d exceed max_pos=%d", n, m->slots[slot].length, m->cfg.max_pos);
     for (int i = 0; i < n_want; i++)
         FX_REQUIRE(want[i] >= 0 && want[i] < n && (i == 0 || want[i] > want[i - 1]), "hybrid_step: want[%d]=%d is not ascending in 0..%d", i, want[i], n - 1);
+    FX_TRY(flexllm_hybrid_timed_out(m));
     hipStream_t st = as_stream(stream);
     return m->cfg.dtype == 0 ? run_step<bf16_t>(m, slot, tokens, n, want, n_want, logits, layers_out, st)
                              : run_step<float>(m, slot, tokens, n, want, n_want, logits, layers_out, st);
@@ -1057,6 +1080,7 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
     FX_REQUIRE(s.length + steps <= m->cfg.max_pos, "hybrid_decode: %d steps on top of %d tokens exceed max_pos=%d", steps, s.length, m->cfg.max_pos);
     hipStream_t st = as_stream(stream);
     FX_REQUIRE(!use_graph || st, "hybrid_decode: graph replay needs a non-default stream");
+    FX_TRY(flexllm_hybrid_timed_out(m));
     if (steps == 0) return FLEXLLM_OK;
     FX_TRY(set_state_launch(s.pos, s.length, 0, st));
     if (top_k == 0 && walk_ready(m, st)) {
@@ -1108,8 +1132,9 @@ int flexllm_hybrid_check(flexllm_hybrid* m) {
             FX_HIP(hipMemset(m->walk.words, 0xFF, 2 * m->walk.set * sizeof(float)));
             FX_HIP(hipMemset(m->walk.err, 0, sizeof(err)));
             FX_HIP(hipDeviceSynchronize());
-            set_error("decode: a wait timed out (were all %d workgroups resident?)", kWalkWG);
-            return FLEXLLM_EHIP;
+            const int rc = flexllm_hybrid_timed_out(m);
+            __atomic_store_n(m->told, 0, __ATOMIC_RELEASE);
+            return rc;
         }
     }
     for (size_t i = 0; i < m->slots.size(); i++) {

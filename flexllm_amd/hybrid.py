@@ -140,10 +140,14 @@ class HybridModel:
                                         want.ctypes.data_as(C.c_void_p) if want.size else None, want.size,
                                         C.c_void_p(logits.ptr) if logits else None, C.c_void_p(res.ptr) if res else None, _s(st)))
         st.sync()
+        if lib().flexllm_hybrid_timed_out(self.handle):
+            self.check()
         out = logits.numpy() if logits else None
         return (out, res.numpy()) if layers else out
 
     def decode(self, slot, token_io, steps, tokens_out, rands=None, top_k=0, use_graph=True, stream=None):
+        """`steps` tokens from the device array token_io into tokens_out.  Does not wait for them: check() says, once they are
+        there, whether they are valid, and so does the next step."""
         check(lib().flexllm_hybrid_decode(self.handle, int(slot), C.c_void_p(token_io.ptr), int(steps),
                                           C.c_void_p(rands.ptr) if rands is not None else None, int(top_k),
                                           C.c_void_p(tokens_out.ptr), int(use_graph), _s(stream or self.stream())))
@@ -173,8 +177,12 @@ class HybridModel:
         return out.numpy()[:int(steps)].tolist()
 
     def check(self):
-        """Synchronise and raise if a token id outside the vocabulary was fed in."""
+        """Synchronise and raise if a wait of the resident decode kernel timed out or a token id outside the vocabulary was fed in."""
         check(lib().flexllm_hybrid_check(self.handle))
+
+    def set_wait_limit(self, polls):
+        """Polls (about 1 us each) after which a wait of the resident decode kernel times out; 0: the default, 2**20."""
+        check(lib().flexllm_hybrid_set_wait_limit(self.handle, int(polls)))
 
     def close(self):
         if self.handle:

@@ -586,14 +586,20 @@ int flexllm_hybrid_step(flexllm_hybrid* m, int slot, const int* tokens, int n, c
 /* `steps` tokens from *token_io (device; fed first, the last drawn token on return) into tokens_out (device [steps]):
  * the largest logit, or with top_k > 0 a draw from the top_k largest with rands[step] (device).  use_graph: one step is
  * captured in a HIP graph and replayed (needs a stream of its own).  Where the sizes allow it, greedy steps run in one resident kernel
- * instead, which needs the whole chip and keeps its turn with others of its kind; flexllm_hybrid_check reports a wait that timed out. */
+ * instead, which needs the whole chip and keeps its turn with others of its kind (flexllm_hybrid_timed_out). */
 int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps, const float* rands, int top_k, int* tokens_out,
                           int use_graph, void* stream);
 /* Prompt to tokens in one slot: all prompt tokens but the last in one go, then the decode loop from the last one. */
 int flexllm_hybrid_generate(flexllm_hybrid* m, int slot, const int* prompt, int n_prompt, int steps, const float* rands, int top_k,
                             int* tokens_out, int use_graph, void* stream);
-/* Synchronises and reports a token id outside the vocabulary (FLEXLLM_EINVAL; id 0 was used). */
+/* Synchronises and reports a wait of the resident kernel that timed out (FLEXLLM_EHIP, once: the model can be used again, its slots are to be
+ * reset) or a token id outside the vocabulary (FLEXLLM_EINVAL; id 0 was used). */
 int flexllm_hybrid_check(flexllm_hybrid* m);
+/* FLEXLLM_EHIP if a wait of the resident kernel, in work that has ended, has timed out since the last flexllm_hybrid_check: what came of that work
+ * is not valid, and steps are refused until the check.  Does not synchronise. */
+int flexllm_hybrid_timed_out(const flexllm_hybrid* m);
+/* Polls of a word (about 1 us each) behind which such a wait times out; 0: the default, 2^20. */
+int flexllm_hybrid_set_wait_limit(flexllm_hybrid* m, int polls);
 /* The GEMM behind the prompt path on its own: a [m][k], w [n][k] of the element type (dtype as in the configuration),
  * k % 64 == 0.  Columns below n_split go to y (element type, [m][n_split], or with glu [m][n_split/2]: rows 2i / 2i+1 of w
  * are gate and up of unit i), the others to y32 (float32 [m][n - n_split]); n_split must keep pairs together.

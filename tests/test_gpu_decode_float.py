@@ -165,6 +165,56 @@ def test_tokens_outside_the_vocabulary():
     assert np.array_equal(*out)
 
 
+def shared_rows(dtype="float32", **kw):
+    from flexllm_amd.lopazen import Lopazen
+    cfg = LOPAZEN["rows of a quad"]
+    return cfg, Lopazen.from_tensors(cfg, lc.weights(cfg, 5), dtype=dtype, max_pos=256, **kw)
+
+
+def latent_rows_and_gla(dtype="float32", **kw):
+    from flexllm_amd.nifunex import Nifunex
+    cfg = NIFUNEX["both kinds"]
+    return cfg, Nifunex.from_tensors(cfg, nc.weights(cfg, 5), dtype=dtype, max_pos=256, **kw)
+
+
+def mixture(dtype="float32", **kw):
+    from flexllm_amd.nifunex import Nifunex
+    moe = dict(mlp=nc.moe(8, 3, 1024, 0.75, 2048))
+    cfg = nc.config([nc.gla(heads=16, dim=128, vdim=128, **moe), latent(16, 0, window=None)], width=2048, vocab=512)
+    return cfg, Nifunex.from_tensors(cfg, nc.weights(cfg, 5), dtype=dtype, max_pos=256, **kw)
+
+
+KINDS = pytest.mark.parametrize("make", [shared_rows, latent_rows_and_gla, mixture])
+
+
+@KINDS
+def test_waits_that_time_out(make):
+    """are an error of the step, and of whatever comes behind a loop; the model is as before once it has been asked."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd._lib import FlexLLMError
+    cfg, m = make()
+    toks = [7, 100, 33, 250, 4]
+    want = m.generate(toks, 70)
+    token, out = to_device(np.array([7], np.int32)), zeros((70,), np.int32)
+    slot = m.pool.acquire("t")
+    m.set_wait_limit(1)                                    # the first word that is not there yet
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.step(slot, toks[:1], [0])
+    m.check()
+    m.decode(slot, token, 70, out)
+    m.stream().sync()
+    m.set_wait_limit(0)
+    for call in (lambda: m.decode(slot, token, 1, out), lambda: m.step(slot, toks), lambda: m.step(slot, toks[:1], [0])):
+        with pytest.raises(FlexLLMError, match="timed out"):
+            call()
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.check()
+    m.pool.release("t")
+    assert m.generate(toks, 70) == want
+    m.check()
+    m.close()
+
+
 def test_infinities_and_not_a_number():
     """An infinite row of a weight is an infinity (or, against both signs, not a number) in that place alone."""
     from flexllm_amd.lopazen import Lopazen
