@@ -99,6 +99,7 @@ struct flexllm_hybrid {
     fx::WalkRun* walk_runs = nullptr;         // [slots][runs]
     unsigned walk_steps = 0;                  // steps taken so far
     int walk_polls = fx::kWalkPolls;
+    int decode_mode = 0;                      // 1: not in one kernel
     int* told = nullptr;                      // host memory: a wait of a step has timed out
 };
 
@@ -924,7 +925,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
 // Steps of one token each in one launch per kWalkLaunch of them: logits of a single one, or greedy ones (tokens_out).
 constexpr int kWalkLaunch = 64;           // bounds the time of a launch
 static bool walk_ready(const flexllm_hybrid* m, hipStream_t st) {
-    if (!m->walk.phases) return false;
+    if (!m->walk.phases || m->decode_mode != 0) return false;
     // a captured launch would be replayed with the same set of words, and beside the host's order of launches
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
@@ -1040,6 +1041,11 @@ int flexllm_hybrid_timed_out(const flexllm_hybrid* m) {
         set_error("decode: a wait timed out (were all %d workgroups resident?); what the slots hold is in no known state", kWalkWG);
         return FLEXLLM_EHIP;
     }
+    return FLEXLLM_OK;
+}
+int flexllm_hybrid_set_decode_mode(flexllm_hybrid* m, int mode) {
+    FX_REQUIRE(m && (mode == 0 || mode == 1), "hybrid_set_decode_mode: mode %d", mode);
+    m->decode_mode = mode;
     return FLEXLLM_OK;
 }
 int flexllm_hybrid_set_wait_limit(flexllm_hybrid* m, int polls) {

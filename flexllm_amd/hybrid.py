@@ -180,6 +180,11 @@ class HybridModel:
         """Synchronise and raise if a wait of the resident decode kernel timed out or a token id outside the vocabulary was fed in."""
         check(lib().flexllm_hybrid_check(self.handle))
 
+    def set_decode_mode(self, mode):
+        """0 (default): steps of one token in the resident kernel where the sizes allow it; 1: in a chain of kernels, for a
+        device that other processes use too."""
+        check(lib().flexllm_hybrid_set_decode_mode(self.handle, int(mode)))
+
     def set_wait_limit(self, polls):
         """Polls (about 1 us each) after which a wait of the resident decode kernel times out; 0: the default, 2**20."""
         check(lib().flexllm_hybrid_set_wait_limit(self.handle, int(polls)))

@@ -598,6 +598,9 @@ int flexllm_hybrid_check(flexllm_hybrid* m);
 /* FLEXLLM_EHIP if a wait of the resident kernel, in work that has ended, has timed out since the last flexllm_hybrid_check: what came of that work
  * is not valid, and steps are refused until the check.  Does not synchronise. */
 int flexllm_hybrid_timed_out(const flexllm_hybrid* m);
+/* 0 (default): steps of one token in the resident kernel where the sizes allow it; 1: in a chain of kernels that end by themselves, for devices
+ * shared with other processes. */
+int flexllm_hybrid_set_decode_mode(flexllm_hybrid* m, int mode);
 /* Polls of a word (about 1 us each) behind which such a wait times out; 0: the default, 2^20. */
 int flexllm_hybrid_set_wait_limit(flexllm_hybrid* m, int polls);
 /* The GEMM behind the prompt path on its own: a [m][k], w [n][k] of the element type (dtype as in the configuration),

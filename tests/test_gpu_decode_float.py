@@ -215,6 +215,40 @@ def test_waits_that_time_out(make):
     m.close()
 
 
+@KINDS
+def test_chain_of_kernels_in_its_place(make):
+    """Switched off, single tokens and loops, with and without a graph, are a chain of kernels, which waits for nothing; and on again."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd._lib import FlexLLMError
+    cfg, m = make()
+    toks = [7, 100, 33, 250, 4]
+    token, out = to_device(np.array([9], np.int32)), zeros((20,), np.int32)
+
+    def request(use_graph=True):
+        slot = m.pool.acquire("t")
+        first = m.step(slot, toks, [4])
+        token.copy_from(np.array([9], np.int32))
+        m.decode(slot, token, 20, out, use_graph=use_graph)
+        got = (first, m.step(slot, toks[:1], [0]), out.numpy().tolist())
+        m.check()
+        m.pool.release("t")
+        return got
+
+    want = request()
+    m.set_wait_limit(1)                                    # the resident kernel would give up
+    m.set_decode_mode(1)
+    for use_graph in True, False:
+        got = request(use_graph)
+        assert np.array_equal(got[0], want[0]) and got[2] == want[2]
+        assert lc.rel_err(got[1], want[1]).max() < lc.LIMIT["float32"]
+    with pytest.raises(FlexLLMError, match="mode"):
+        m.set_decode_mode(2)
+    m.set_decode_mode(0)
+    with pytest.raises(FlexLLMError, match="timed out"):
+        request()
+    m.close()
+
+
 def test_infinities_and_not_a_number():
     """An infinite row of a weight is an infinity (or, against both signs, not a number) in that place alone."""
     from flexllm_amd.lopazen import Lopazen
