@@ -924,11 +924,21 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
 
 // Steps of one token each in one launch per kWalkLaunch of them: logits of a single one, or greedy ones (tokens_out).
 constexpr int kWalkLaunch = 64;           // bounds the time of a launch
+constexpr int kWalkMaskWords = 32;        // of a stream's CUs
 static bool walk_ready(const flexllm_hybrid* m, hipStream_t st) {
     if (!m->walk.phases || m->decode_mode != 0) return false;
     // a captured launch would be replayed with the same set of words, and beside the host's order of launches
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+    // a stream may be confined to some of the CUs (0.2 us to ask)
+    uint32_t mask[kWalkMaskWords] = {0};
+    if (hipExtStreamGetCUMask(st, kWalkMaskWords, mask) != hipSuccess) {
+        (void)hipGetLastError();                          // no error of the next launch
+        return false;
+    }
+    int cus = 0;
+    for (const uint32_t m : mask) cus += __builtin_popcount(m);
+    return cus >= kWalkWG;
 }
 static int walk(flexllm_hybrid* m, int slot, int* token, int steps, int* tokens_out, bool head, float* logits, hipStream_t st) {
     for (int done = 0; done < steps;) {

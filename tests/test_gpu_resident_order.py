@@ -89,6 +89,33 @@ def test_callers_streams():
     t.destroy()
 
 
+def test_a_stream_with_half_of_the_chip():
+    """The workgroups that have to be there all at once do not fit: its tokens come from the chain of kernels."""
+    from flexllm_amd import to_device, zeros
+    half, all_of_it = [CallersStream(), CallersStream()]
+    for s, word in (half, 0), (all_of_it, 0xFFFFFFFF):
+        s.destroy()
+        hip()("hipExtStreamCreateWithCUMask", C.byref(s.handle), 8, (C.c_uint32 * 8)(*[0xFFFFFFFF] * 4 + [word] * 4))
+    m = lopazen()
+    prompt, token, out, got = lc.tokens(CFG, 20), to_device(np.array([0], np.int32)), zeros((30,), np.int32), []
+    for mode, s in (1, None), (0, half), (0, all_of_it):
+        m.set_decode_mode(mode)
+        slot = m.pool.acquire("r")
+        m.step(slot, prompt[:-1])
+        token.copy_from(np.array(prompt[-1:], np.int32))
+        if s is half:
+            m.set_wait_limit(1)                            # the resident kernel would give up
+        m.decode(slot, token, 30, out, stream=s)
+        m.check()
+        m.set_wait_limit(0)
+        got.append(out.numpy().tolist())
+        m.pool.release("r")
+    assert got[0] == got[1] and got[0][:3] == got[2][:3]
+    m.close()
+    half.destroy()
+    all_of_it.destroy()
+
+
 def test_two_designs_and_ordinary_work():
     """Llama's decode kernel, a decoder's, and prompts of a third model, whose kernels hold a part of the chip now and then."""
     from flexllm_amd import llama
