@@ -193,7 +193,13 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
             }
         }
     };
-    auto known = [&] { return it < tokens && (!MOE || iorder == 0 || flag(L.chosen) >= it * routed + iorder); };       // an expert's weights have no address before the choice
+    auto known = [&] {                                    // an expert's weights have no address before the choice
+        if (it >= tokens) return false;
+        if (!MOE || iorder == 0) return true;
+        const bool yes = flag(L.chosen) >= it * routed + iorder;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");         // the addresses are read behind the flag
+        return yes;
+    };
     auto ask = [&] {
         if (MOE && iorder) ibase = base_of(ip);
         quad_to_lds(ibase, (unsigned)iq * kQuad + lane * 16, dst + islot * kQuad);
