@@ -10,7 +10,7 @@ constexpr int kWalkMaxPhases = 256;
 constexpr int kWalkPolls = 1 << 20;        // about a second
 constexpr int kWalkMaxWidth = 4096;
 constexpr size_t kWalkLdsMax = 160 * 1024;
-constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 8, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
+constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 4, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
 constexpr int kWalkRow = 4096;             // bytes that the rows of all linears are a multiple of
 
 // A linear of the step: n rows of kpad elements, dealt to the workgroups in runs of neighbouring rows (walk_rows).  The experts' products are groups of

@@ -148,17 +148,13 @@ __device__ __forceinline__ void quad_to_lds(const char* base, unsigned voff, uns
                  "s_mov_b32 m0, %0"
                  : "=&s"(saved_m0) : "v"(voff), "s"(base), "s"(dst) : "memory");
 }
-// Until all but the youngest n quads have arrived.
+// Until all but the youngest n quads have arrived; n at most 3, since a ring has at most four.
 __device__ __forceinline__ void wait_quads(int n) {
     switch (n) {
         case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
         case 1: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
         case 2: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
-        case 3: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
-        case 4: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;
-        case 5: asm volatile("s_waitcnt vmcnt(20)" ::: "memory"); break;
-        case 6: asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); break;
-        default: asm volatile("s_waitcnt vmcnt(28)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
     }
 }
 __device__ __forceinline__ int flag(const int& f) { return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)); }
@@ -1308,14 +1304,14 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, Res
 // What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.
 size_t walk_lds(const WalkArgs& a) { return sizeof(WalkLds) + sizeof(float) * ((size_t)a.lds_xs + a.lds_red); }
 static_assert(kStrWaves * kQuad == kWalkSlotBytes && kQuad == kWalkRow, "a quad per wave");
+static_assert((kWalkLdsMax - sizeof(WalkLds)) / kWalkSlotBytes == kWalkMaxSlots, "wait_quads counts as many");
 
 template <typename ET>
 int walk_launch(const WalkArgs& a, hipStream_t st) {
     FX_REQUIRE(a.n_phases < kWalkMaxPhases && a.width % 512 == 0 && a.width <= kWalkMaxWidth && a.vocab >= kWalkWG && a.steps > 0, "walk: %d linears, width %d, vocabulary %d", a.n_phases, a.width, a.vocab);
     const size_t used = walk_lds(a);
     FX_REQUIRE(used + kWalkMinSlots * kWalkSlotBytes <= kWalkLdsMax, "walk: %zu bytes of LDS", used);
-    int slots = (int)((kWalkLdsMax - used) / kWalkSlotBytes);
-    if (slots > kWalkMaxSlots) slots = kWalkMaxSlots;
+    const int slots = (int)((kWalkLdsMax - used) / kWalkSlotBytes);
     const size_t lds = used + slots * kWalkSlotBytes;
     auto go = [&](auto* k, std::atomic<bool>& opted_in) {
         if (!opted_in.load(std::memory_order_acquire)) {
