@@ -1107,7 +1107,6 @@ struct Service {
             int pick;
             float weight;
             route_wave(L.z, E, top, pick, weight);
-            pick = min(max(pick, 0), E - 1);              // router outputs that are not numbers choose nobody
             if (lane < top) {
                 L.choice_w[lane] = weight;
 #pragma unroll

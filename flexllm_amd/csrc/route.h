@@ -7,7 +7,8 @@ namespace fx {
 constexpr int kMaxExperts = 1024, kMaxTop = 32;
 
 // Expert choice of one token by one wave: softmax over the router outputs, the `top` largest (ties: lower index), their
-// weights divided by their sum.  Lane k < top gets choice k and its weight.  NE: 64-expert pieces (experts <= 64 NE).
+// weights divided by their sum.  Lane k < top gets choice k, an expert's number whatever the outputs are, and its weight.
+// NE: 64-expert pieces (experts <= 64 NE).
 template <int NE>
 __device__ __forceinline__ void route_wave_n(const float* __restrict__ z, int experts, int top, int& pick, float& weight) {
     const int lane = threadIdx.x & 63;
@@ -49,6 +50,8 @@ __device__ __forceinline__ void route_wave_n(const float* __restrict__ z, int ex
         if (lane == k) { pick = bi; weight = s; }
     }
     weight = weight / (sum + 1e-20f);
+    // where outputs are not numbers there may be nothing left to take, or only lanes without an expert
+    pick = min(max(pick, 0), experts - 1);
 }
 __device__ __forceinline__ void route_wave(const float* __restrict__ z, int experts, int top, int& pick, float& weight) {
     if (experts <= 64) route_wave_n<1>(z, experts, top, pick, weight);

@@ -380,6 +380,26 @@ def test_errors():
     m.close()
 
 
+@BOTH
+@pytest.mark.parametrize("experts,top", [(8, 3), (64, 6), (130, 4)])
+def test_router_outputs_that_are_no_numbers(experts, top, dtype):
+    """choose some expert, not a place outside of the experts' weights: that token's logits are no numbers, those of earlier steps what they
+    are without it.  As a prompt, in steps of several tokens and of one; numbers of experts that fill a wave and that do not."""
+    moe = dict(mlp=nc.moe(experts, top, 40, 0.75, 56))
+    cfg = nc.config([nc.gla(**moe), nc.latent(**moe)])
+    w, toks = nc.weights(cfg, 5), nc.tokens(cfg, 40)
+    w["embed"] = w["embed"].copy()
+    w["embed"][299, 3], w["embed"][298, 4] = np.nan, np.inf
+    toks = [t % 290 for t in toks]
+    for cuts in [40], [4], [1]:
+        for bad in 299, 298:
+            m = model(cfg, w, dtype)
+            want, got = run(m, toks, cuts), run(m, toks[:21] + [bad] + toks[22:], cuts)
+            ahead = 21 // cuts[0] * cuts[0]
+            assert np.isfinite(want).all() and np.array_equal(got[:ahead], want[:ahead]) and np.isnan(got[21]).all()
+            m.close()
+
+
 def test_command_line_and_trace(tmp_path):
     """A model folder through the generation command and through the trace runner."""
     from flexllm_amd import loader
