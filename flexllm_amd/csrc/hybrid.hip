@@ -44,6 +44,7 @@ struct HybridLayer {
     void *w_side = nullptr, *w_sd = nullptr;  // mixture: [shared gate/up; router; shared gate row], shared down
     int n_side = 0;
     float* kv_norm = nullptr;                 // product of the query and key norms' weights
+    bool clear_o = false, clear_d = false, clear_sd = false;      // clear_pads ahead of a prompt's w_o, w_d, w_sd
     LatentDims ld = {};
     SharedKvDims sd = {};
     GlaDims gd = {};
@@ -114,7 +115,7 @@ static int halloc(std::vector<void*>& list, void** p, size_t bytes) {
         return e == hipErrorOutOfMemory ? FLEXLLM_ENOMEM : FLEXLLM_EHIP;
     }
     list.push_back(*p);
-    FX_HIP(hipMemset(*p, 0, n));             // padding columns are multiplied by zero weights: they have to be finite
+    FX_HIP(hipMemset(*p, 0, n));             // padding columns are multiplied by zero weights: they have to be finite (see clear_pads)
     return FLEXLLM_OK;
 }
 #define FX_TRY(expr)              \
@@ -499,6 +500,19 @@ static int create_walk(flexllm_hybrid* m) {
     return FLEXLLM_OK;
 }
 
+// Layers whose padding columns others write to (clear_pads).
+static void note_pads(std::vector<HybridLayer>& layers) {
+    const auto differ = [&](auto k_of, auto clear) {
+        for (HybridLayer& L : layers)
+            if (k_of(L) % kKPad)
+                for (const HybridLayer& o : layers)
+                    if (k_of(o) && k_of(o) != k_of(L)) L.*clear = true;
+    };
+    differ([](const HybridLayer& L) { return L.k_o; }, &HybridLayer::clear_o);
+    differ([](const HybridLayer& L) { return L.d.ff_kind == FLEXLLM_FF_NONE ? 0 : L.d.ff; }, &HybridLayer::clear_d);
+    differ([](const HybridLayer& L) { return L.d.ff_kind == FLEXLLM_FF_MOE ? L.d.shared_ff : 0; }, &HybridLayer::clear_sd);
+}
+
 template <typename ET>
 static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, const flexllm_hybrid_layer_weights* lw) {
     const flexllm_hybrid_config& c = m->cfg;
@@ -516,6 +530,7 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
         m->head = head.dst;
     }
     for (int i = 0; i < c.layers; i++) FX_TRY(create_layer<ET>(m, i, lw[i]));
+    note_pads(m->layers);
     m->slots.resize(c.slots);
     for (HybridSlot& s : m->slots) {
         const int n = (int)m->runs.size();
@@ -770,6 +785,20 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
 }
 
 // ---- many tokens --------------------------------------------------------------------------------------------------------
+// A product multiplies its rows' padding columns, k .. ld-1, by zero weights.  Layers share the rows' memory: where their k differ, one's padding is
+// another's values, of an earlier request perhaps, and what is infinite or not a number there would be in every sum.
+template <typename ET>
+__global__ __launch_bounds__(256) void clear_pads_kernel(ET* __restrict__ p, int ld, int rows, int k) {
+    const int pads = ld - k;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < (size_t)rows * pads; i += (size_t)gridDim.x * 256) p[i / pads * ld + k + i % pads] = (ET)0.0f;
+}
+template <typename ET>
+static int clear_pads(void* p, int ld, int rows, int k, hipStream_t st) {
+    const size_t blocks = ((size_t)rows * (ld - k) + 255) / 256;
+    clear_pads_kernel<ET><<<(int)(blocks < 2048 ? blocks : 2048), 256, 0, st>>>(static_cast<ET*>(p), ld, rows, k);
+    FX_LAUNCH_CHECK();
+    return FLEXLLM_OK;
+}
 template <typename ET>
 static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, const int* want, int n_want, float* logits, float* layers_out,
                     size_t layer_stride, hipStream_t st) {
@@ -858,6 +887,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         } else {
             FX_TRY(gla_steps<ET>(L.gd, proj, ldp, 0, m->lf32, nf, static_cast<ET*>(L.a2), L.a2_bias, L.head_norm, s.state[r], s.pos, 0, T, att, lda, 0, st));
         }
+        if (L.clear_o) FX_TRY(clear_pads<ET>(att, lda, T, L.k_o, st));
         FX_TRY(to_y(att, lda, L.w_o, L.k_o));
         pend.gb = L.g1b;
         if (L.d.ff_kind == FLEXLLM_FF_NONE) continue;
@@ -867,6 +897,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
             g = gemm(m->lh, kw, L.w_gu, T, 2 * L.d.ff, W);
             g.n_split = 2 * L.d.ff; g.glu = 1 + L.d.glu; g.limit = L.d.limit; g.y = m->lhid; g.ldy = kf;
             FX_TRY(gemm_float<ET>(g, st));
+            if (L.clear_d) FX_TRY(clear_pads<ET>(m->lhid, kf, T, L.d.ff, st));
             FX_TRY(to_y(m->lhid, kf, L.w_d, L.d.ff));
             pend.gb = L.g2b;
             continue;
@@ -886,11 +917,13 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         g.n_split = 2 * L.d.ff; g.glu = 1 + L.d.glu; g.limit = L.d.limit; g.y = m->lhid; g.ldy = kf;
         g.row_src = m->lrow_src; g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)2 * L.d.ff * kw; g.group_rows = T * top / L.d.experts;
         FX_TRY(gemm_grouped<ET>(g, tile, st));
+        if (L.clear_d) FX_TRY(clear_pads<ET>(m->lhid, kf, T * top, L.d.ff, st));
         g = gemm(m->lhid, kf, L.w_d, T * top, W, L.d.ff);
         g.n_split = 0; g.y32 = m->lys; g.ldy32 = W;
         g.tiles = m->ltiles; g.n_tiles = m->lntiles; g.max_tiles = max_tiles; g.w_stride = (size_t)W * kf; g.group_rows = T * top / L.d.experts;
         FX_TRY(gemm_grouped<ET>(g, tile, st));
         if (sf) {
+            if (L.clear_sd) FX_TRY(clear_pads<ET>(m->lhs, ks, T, sf, st));
             FX_TRY(to_y(m->lhs, ks, L.w_sd, sf));
             pend.route = m->lroute; pend.ld_route = ldr; pend.experts = L.d.experts;
         }

@@ -8,6 +8,7 @@ import sys
 import numpy as np
 import pytest
 
+import lopazen_cases as lc
 import nifunex_cases as nc
 from oracle import nifunex_ref
 
@@ -398,6 +399,35 @@ def test_router_outputs_that_are_no_numbers(experts, top, dtype):
             ahead = 21 // cuts[0] * cuts[0]
             assert np.isfinite(want).all() and np.array_equal(got[:ahead], want[:ahead]) and np.isnan(got[21]).all()
             m.close()
+
+
+LEFT = {
+    "sizes that need padding": nc.config([nc.gla(mlp=nc.dense()), nc.gla(heads=3, dim=36, vdim=20, mlp=nc.moe()), nc.gla(heads=1, mlp=nc.moe(5, 3, 24, 1.5, 20))]),
+    "shared rows": lc.mixed(),
+}
+
+
+@BOTH
+@pytest.mark.parametrize("name", list(LEFT))
+def test_what_a_request_leaves_behind(name, dtype):
+    """Values that are not numbers stay in their own sequence: not in padding columns, which layers of other sizes use for values, nor
+    in rows, states and workspaces that the next sequence takes over."""
+    from flexllm_amd.registry import model_class
+    cfg = LEFT[name]
+    cases = lc if cfg["architecture"] == "Lopazen" else nc
+    w = cases.weights(cfg, 5)
+    w["embed"] = w["embed"].copy()
+    w["embed"][299, 3], w["embed"][298, 4] = np.nan, np.inf
+    toks, logits = [t % 290 for t in nc.tokens(cfg, 200)], np.arange(298)
+    m = model_class(cfg["architecture"]).from_tensors(cfg, w, dtype=dtype, max_pos=512)
+    for cuts in [40], [5], [1]:
+        want = run(m, toks[:40], cuts)[:, logits]
+        assert np.isfinite(want).all()
+        for bad in 299, 298:
+            for bad_cuts in [200], [4], [1]:
+                assert np.isnan(run(m, toks[:33] + [bad] + toks[34:], bad_cuts)[33, logits]).all()
+                assert np.array_equal(run(m, toks[:40], cuts)[:, logits], want), (cuts, bad, bad_cuts)
+    m.close()
 
 
 def test_command_line_and_trace(tmp_path):
