@@ -463,8 +463,9 @@ template int latent_decode<float>(const LatentDims&, const float*, int, const fl
 // the slots of that product's k dimension are assigned to the keys in accumulator order (slot j of half-wave h = key
 // 8 * (j / 4) + 4 * h + j % 4 of each 16), which the reads of the transposed values follow.
 // LDS: keys in planes of 8 dims [plane][64 keys][16 B], values in planes of 4 keys [plane][value row][8 B].
-// Planes beyond a head's own dims meet zeros on the query side, value rows beyond vdim are not stored: both may hold any
-// finite value, so no load is conditional.
+// Planes beyond a head's own dims meet zeros on the query side and repeat the head's own, value rows beyond vdim are not stored: no load is
+// conditional.  Values behind the last row are what an earlier prompt left: in the tile that has any they are set to zero, since
+// a weight of zero leaves what is infinite or not a number.
 constexpr int kFlashK = 64;
 
 template <int DK, int DV, int NW>
@@ -531,6 +532,14 @@ __global__ __launch_bounds__(NW * 64, (DV > 128 || NW < 4) ? 1 : 2) void latent_
     };
     load(kb0);
     for (int kb = kb0; kb <= kb1; kb += kFlashK) {
+        if (kb + kFlashK > rows) {
+#pragma unroll
+            for (int i = 0; i < VCH; i++) {
+                const int left = rows - kb - ((t + T * i) & 7) * 8;       // of the piece's eight keys
+#pragma unroll
+                for (int w = 0; w < 4; w++) rv[i][w] = left >= 2 * w + 2 ? rv[i][w] : left == 2 * w + 1 ? rv[i][w] & 0xFFFF : 0;
+            }
+        }
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < KCH; i++) {

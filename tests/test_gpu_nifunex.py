@@ -404,6 +404,8 @@ def test_router_outputs_that_are_no_numbers(experts, top, dtype):
 LEFT = {
     "sizes that need padding": nc.config([nc.gla(mlp=nc.dense()), nc.gla(heads=3, dim=36, vdim=20, mlp=nc.moe()), nc.gla(heads=1, mlp=nc.moe(5, 3, 24, 1.5, 20))]),
     "shared rows": lc.mixed(),
+    "latent rows": nc.mixed(),
+    "latent rows, long heads": nc.config([nc.gla(mlp=nc.dense(64)), nc.latent(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=512, window=None, mlp=nc.dense(64))], width=128),
 }
 
 
@@ -420,13 +422,13 @@ def test_what_a_request_leaves_behind(name, dtype):
     w["embed"][299, 3], w["embed"][298, 4] = np.nan, np.inf
     toks, logits = [t % 290 for t in nc.tokens(cfg, 200)], np.arange(298)
     m = model_class(cfg["architecture"]).from_tensors(cfg, w, dtype=dtype, max_pos=512)
-    for cuts in [40], [5], [1]:
-        want = run(m, toks[:40], cuts)[:, logits]
+    for n, cuts in (40, [40]), (63, [63]), (25, [5]), (25, [1]):
+        want = run(m, toks[:n], cuts)[:, logits]
         assert np.isfinite(want).all()
         for bad in 299, 298:
             for bad_cuts in [200], [4], [1]:
                 assert np.isnan(run(m, toks[:33] + [bad] + toks[34:], bad_cuts)[33, logits]).all()
-                assert np.array_equal(run(m, toks[:40], cuts)[:, logits], want), (cuts, bad, bad_cuts)
+                assert np.array_equal(run(m, toks[:n], cuts)[:, logits], want), (cuts, bad, bad_cuts)
     m.close()
 
 
