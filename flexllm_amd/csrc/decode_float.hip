@@ -484,7 +484,7 @@ struct Service {
     // ---- attention over shared key/value rows (see shared_kv_attn.hip): a workgroup takes a split of the rows for one query head;
     // the heads that share rows are on one die.  (All four heads of a key/value head in one workgroup and four times the splits: 2.9 us
     // instead of 1.9 for 1531 rows, for the norms and sums of four heads.)  A split has a batch of rows for every group of lanes at
-    // least: up to 256 rows of 64 then need no join, which is 2.4 us.
+    // least: up to 128 rows of 64 (64 of 128, half as many in float32) need no join, which is 2.4 us.
     template <int D>
     __device__ __forceinline__ void shared_kv(RunPtr r, int pos) {
         const int t = opaque(), lane = t & 63;

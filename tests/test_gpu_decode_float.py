@@ -75,6 +75,30 @@ def test_token_by_token_nifunex(name, dtype):
     check_nifunex(NIFUNEX[name], dtype, 70, [1], [50, 1])
 
 
+# float32: rows of one quad and of three, which no wave has the same part of in all rows
+FLOAT32 = {
+    "shared rows of a quad": lc.config([attention(16, 4, 64, 1024)], width=1024, vocab=512),
+    "shared rows of three quads": lc.config([attention(48, 16, 64, 3072)], width=3072, vocab=515),
+    "both kinds, rows of a quad": nc.config([latent(8, 1024, window=40), gla(8, 1024)], width=1024, vocab=512),
+    "both kinds, rows of three quads": nc.config([gla(24, 3072), latent(24, 3072, window=None)], width=3072, vocab=515),
+    "mixtures, rows of a quad": nc.config([gla(8, 0) | dict(mlp=nc.moe(5, 2, 512, 0.75, 1024)), latent(8, 0) | dict(mlp=nc.moe(4, 2, 1024, 0.75, 512))], width=1024, vocab=512),
+}
+
+
+@pytest.mark.parametrize("name", list(FLOAT32))
+def test_sizes_of_float32_alone(name):
+    from flexllm_amd._lib import FlexLLMError
+    from flexllm_amd.registry import model_class
+    cfg = FLOAT32[name]
+    cases, checked = (lc, check_lopazen) if cfg["architecture"] == "Lopazen" else (nc, check_nifunex)
+    checked(cfg, "float32", 40, [1], [30, 1])
+    m = model_class(cfg["architecture"]).from_tensors(cfg, cases.weights(cfg, 5), dtype="float32", max_pos=64)
+    m.set_wait_limit(1)                                    # it is the resident kernel that they take
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.step(m.pool.acquire("t"), [1], [0])
+    m.close()
+
+
 @BOTH
 @pytest.mark.parametrize("heads,window", [(16, 1024), (16, 300), (32, 700)])
 def test_splits_of_latent_rows(heads, window, dtype):
@@ -86,10 +110,37 @@ def test_splits_of_latent_rows(heads, window, dtype):
 @BOTH
 @pytest.mark.parametrize("dim", [64, 128])
 def test_splits_of_the_rows(dim, dtype):
-    """Around the number of rows from which on there are several splits, and where all of them have some."""
-    alone = {64: 256, 128: 128}[dim] // (1 if dtype == "bfloat16" else 2)
-    for rows in alone, 8 * alone:
+    """Around the number of rows from which on there are two splits, three, and where all of them have some."""
+    alone = {64: 128, 128: 64}[dim] // (1 if dtype == "bfloat16" else 2)
+    for rows in alone, 2 * alone, 16 * alone:
         check_lopazen(lc.config([attention(32, 8, dim, 0)], width=2048, vocab=512), dtype, rows + 5, [rows - 5, 1], max_pos=2112)
+
+
+@BOTH
+@pytest.mark.parametrize("rows_of", [64, 128, "latent"])
+def test_splits_inside_a_loop(rows_of, dtype):
+    """The second split, and with it the writers and readers of the words, comes in the middle of one launch: as step by step."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd.lopazen import Lopazen
+    from flexllm_amd.nifunex import Nifunex
+    if rows_of == "latent":
+        cfg, alone = nc.config([latent(16, 2048, window=None)] * 2, width=2048, vocab=512), 64
+        m = Nifunex.from_tensors(cfg, nc.weights(cfg, 5), dtype=dtype, max_pos=256, slots=2)
+    else:
+        cfg, alone = lc.config([attention(32, 8, rows_of, 2048)] * 2, width=2048 * rows_of // 64, vocab=512), {64: 128, 128: 64}[rows_of] // (1 if dtype == "bfloat16" else 2)
+        m = Lopazen.from_tensors(cfg, lc.weights(cfg, 5), dtype=dtype, max_pos=256, slots=2)
+    toks = lc.tokens(cfg, alone - 4)
+    a, b = [m.pool.acquire(n) for n in "ab"]
+    for s in a, b:
+        m.step(s, toks[:-1])
+    token, out, one_by_one = to_device(np.array(toks[-1:], np.int32)), zeros((12,), np.int32), toks[-1:]
+    m.decode(a, token, 12, out)
+    for _ in range(12):
+        one_by_one.append(int(m.step(b, one_by_one[-1:], [0])[0].argmax()))
+    m.check()
+    assert out.numpy().tolist() == one_by_one[1:]
+    assert np.array_equal(m.step(a, [3], [0]), m.step(b, [3], [0]))
+    m.close()
 
 
 @BOTH
@@ -255,15 +306,81 @@ def test_infinities_and_not_a_number():
     cfg = LOPAZEN["as many key heads"]
     w = lc.weights(cfg, 5)
     w["embed"] = w["embed"].copy()
-    m = Lopazen.from_tensors(cfg, w, dtype="float32", max_pos=64)
-    clean = m.generate(lc.tokens(cfg, 5), 3)
-    m.close()
     w["embed"][900, 7] = np.inf                            # the head is the embedding: one logit
     m = Lopazen.from_tensors(cfg, w, dtype="float32", max_pos=64)
     s = m.pool.acquire("t")
     got = m.step(s, lc.tokens(cfg, 1), [0])[0]
+    m.check()
     m.close()
-    assert np.isinf(got[900]) and np.isfinite(np.delete(got, 900)).all() and len(clean) == 3
+    assert np.isinf(got[900]) and np.isfinite(np.delete(got, 900)).all()
+
+
+# Tokens whose embeddings, and weights whose rows, are not finite: what is not a number goes through every exchange
+NOT_FINITE = {
+    "shared rows": (LOPAZEN["rows of a quad"], ["l0.mix.k", "l0.mlp.up", "l1.mix.q"]),
+    "latent rows and gla": (NIFUNEX["both kinds"], ["l0.mix.dkv", "l1.mix.v", "l1.mlp.gate"]),
+    "mixtures": (nc.config([gla(16, 0) | dict(mlp=nc.moe(8, 3, 1024, 0.75, 2048)), latent(16, 0, window=None) | dict(mlp=nc.moe(8, 3, 1024, 0.75, 2048))], width=2048, vocab=512),
+                 ["l0.mlp.router", "l0.mlp.shared.up", "l1.mlp.shared.sg"]),
+}
+
+
+@BOTH
+@pytest.mark.parametrize("name", list(NOT_FINITE))
+def test_what_is_not_finite(name, dtype):
+    """No wait takes it for a word that is not there; the places are those of the chain of kernels; a sequence in another slot is not
+    touched by it.  A loop whose logits are all no numbers finds token 0."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd.registry import model_class
+    cfg, infinite = NOT_FINITE[name]
+    cases = lc if cfg["architecture"] == "Lopazen" else nc
+    base = cases.weights(cfg, 5)
+    base["embed"] = base["embed"].copy()
+    base["embed"][300, 5], base["embed"][301, 9], base["embed"][302, 5:8] = np.inf, np.nan, [np.inf, -np.inf, np.nan]
+    if "head" not in base:                                 # logits of their own, then, are no numbers: 300 to 302 are left out below
+        others = np.delete(np.arange(cfg["vocab"]), [300, 301, 302])
+    else:
+        others = np.arange(cfg["vocab"])
+    clean = [7, 100, 33, 250, 4]
+
+    def model(w):
+        m = model_class(cfg["architecture"]).from_tensors(cfg, w, dtype=dtype, max_pos=256, slots=2)
+        return m, m.pool.acquire("bad"), m.pool.acquire("good")
+
+    def steps(m, slot, toks):
+        return np.stack([m.step(slot, [t], [0])[0] for t in toks])
+
+    m, bad, good = model(base)
+    want = steps(m, good, clean)
+    assert np.isfinite(want[:, others]).all()
+    for t in 300, 301, 302:
+        m.pool.release("bad")
+        bad = m.pool.acquire("bad")
+        got = steps(m, bad, [8, t, 9])
+        assert np.isfinite(got[0, others]).all() and np.isnan(got[1, others]).all()
+        token, out = to_device(np.array([t], np.int32)), zeros((9,), np.int32)
+        m.decode(bad, token, 9, out)
+        m.check()
+        assert out.numpy().tolist() == [0] * 9
+        m.pool.release("good")
+        good = m.pool.acquire("good")
+        assert np.array_equal(steps(m, good, clean)[:, others], want[:, others])
+    m.check()
+    m.close()
+    for t in infinite:
+        w = dict(base, **{t: base[t].copy()})
+        w[t].reshape(-1)[w[t].size // 2 + 11] = np.inf     # a row in the middle
+        m, bad, good = model(w)
+        got = steps(m, bad, clean)
+        m.check()
+        m.set_decode_mode(1)
+        chain = steps(m, good, clean)
+        m.check()
+        m.close()
+        for kind in np.isnan, np.isposinf, np.isneginf:
+            assert np.array_equal(kind(got), kind(chain)), (t, kind)
+        finite = np.isfinite(chain).all(0)
+        if finite.any():
+            assert cases.rel_err(got[:, finite], chain[:, finite]).max() < cases.LIMIT[dtype]
 
 
 def test_two_models_on_streams_of_their_own():
