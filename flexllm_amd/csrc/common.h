@@ -68,8 +68,9 @@ int resident_launch(void (*kernel)(P...), int grid, int block, size_t lds, hipSt
         return resident_launch_args(reinterpret_cast<const void*>(kernel), grid, block, args, lds, st, std::get<sizeof...(P) - 1>(values));
     }, values);
 }
+// by one thread of the first workgroup
 __device__ __forceinline__ void resident_done(const ResidentEnd& end) {
-    if (end.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(end.word, end.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (end.word) __hip_atomic_store(end.word, end.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- cross-lane exchange

@@ -1297,7 +1297,7 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, Res
         a.state[0] = pos0 + a.steps;
         a.state[1] = step0 + a.steps;
     }
-    resident_done(end);
+    if (blockIdx.x == 0 && threadIdx.x == 0) resident_done(end);
 }
 
 // What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.

@@ -521,7 +521,7 @@ __device__ __forceinline__ int mega_dot_row(const i32x4 (&wr)[NCH], const int8_t
 // activations, int4 weights two per byte, int4 output head); attention, exchanges and wave roles are the same, the
 // weight rows are half as long: a stream wave then holds all 16 of its gate/up rows in registers.
 template <bool W4>
-__device__ __forceinline__ void decode_mega_body(const MegaParams& p) {
+__device__ __forceinline__ void decode_mega_body(const MegaParams& p, const ResidentEnd& end) {
     extern __shared__ __attribute__((aligned(16))) unsigned char mega_smem[];   // sizeof(MegaLds) > the static 64 KiB limit
     MegaLds& L = *reinterpret_cast<MegaLds*>(mega_smem);
     const int t = threadIdx.x, wg = blockIdx.x;
@@ -1387,6 +1387,7 @@ __device__ __forceinline__ void decode_mega_body(const MegaParams& p) {
         p.state[2] = (int)bar.epoch;
         p.state[4] = (int)(seq0 + (unsigned)(steps_done * p.n_layers));
         if (greedy) { p.token[0] = tok; p.state[0] = pos0 + steps_done; p.state[1] = step_base + steps_done; }
+        resident_done(end);
     }
 #ifdef FX_MEGA_FINE_STAMPS
     if (p.timeline && is_t0()) p.timeline[p.n_layers * 12 + 2 + 64 + kMegaWG + wg] = wall_clock64();     // workgroup exit
@@ -1394,12 +1395,10 @@ __device__ __forceinline__ void decode_mega_body(const MegaParams& p) {
 }
 
 __global__ __launch_bounds__(kMegaT, 1) void decode_mega_kernel(MegaParams p, ResidentEnd end) {
-    decode_mega_body<false>(p);
-    resident_done(end);
+    decode_mega_body<false>(p, end);
 }
 __global__ __launch_bounds__(kMegaT, 1) void decode_mega_w4_kernel(MegaParams p, ResidentEnd end) {
-    decode_mega_body<true>(p);
-    resident_done(end);
+    decode_mega_body<true>(p, end);
 }
 
 }  // namespace fx
