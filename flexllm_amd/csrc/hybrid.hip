@@ -12,6 +12,8 @@
 // next sublayer's first kernel takes it in.
 #include "decode_float.h"
 #include "logits_kernels.h"
+#include <algorithm>
+#include <limits.h>
 #include <math.h>
 #include <string.h>
 #include <vector>
@@ -99,6 +101,7 @@ struct flexllm_hybrid {
     fx::WalkArgs walk = {};
     fx::WalkRun* walk_runs = nullptr;         // [slots][runs]
     unsigned walk_steps = 0;                  // steps taken so far
+    int walk_rows = INT_MAX;                  // rows held, from which on the chain of kernels is faster
     int walk_polls = fx::kWalkPolls;
     int decode_mode = 0;                      // 1: not in one kernel
     int* told = nullptr;                      // host memory: a wait of a step has timed out
@@ -435,6 +438,7 @@ static int create_walk(flexllm_hybrid* m) {
                 r.ff = L.d.ff_kind == FLEXLLM_FF_NONE ? 0 : L.d.ff; r.glu = 1 + L.d.glu; r.limit = L.d.limit;
                 r.x_in = words(r.n_in);
                 if (shared) {
+                    m->walk_rows = std::min(m->walk_rows, walk_shared_kv_rows(L.sd, W, sizeof(ET)));
                     r.mixer = kWalkSharedKv;
                     r.kv_heads = L.sd.kv_heads; r.rep = L.sd.heads / L.sd.kv_heads; r.splits = walk_splits(L.sd.heads, L.sd.dim); r.dim = L.sd.dim;
                     r.sink = L.sd.sink; r.temp_every = L.sd.temp_every; r.scale = L.sd.scale; r.temp_coef = L.sd.temp_coef;
@@ -958,8 +962,8 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
 // Steps of one token each in one launch per kWalkLaunch of them: logits of a single one, or greedy ones (tokens_out).
 constexpr int kWalkLaunch = 64;           // bounds the time of a launch
 constexpr int kWalkMaskWords = 32;        // of a stream's CUs
-static bool walk_ready(const flexllm_hybrid* m, hipStream_t st) {
-    if (!m->walk.phases || m->decode_mode != 0) return false;
+static bool walk_ready(const flexllm_hybrid* m, int held, hipStream_t st) {
+    if (!m->walk.phases || m->decode_mode != 0 || held >= m->walk_rows) return false;
     // a captured launch would be replayed with the same set of words, and beside the host's order of launches
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
@@ -1001,7 +1005,7 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
         int w1 = w0;
         while (w1 < n_want && want[w1] < t0 + T) part.push_back(want[w1++] - t0);
         float* lg = n_want ? logits + (size_t)w0 * m->cfg.vocab : nullptr;
-        if (T == 1 && !layers_out && walk_ready(m, st))
+        if (T == 1 && !layers_out && walk_ready(m, s.length, st))
             FX_TRY(walk(m, slot, const_cast<int*>(tokens + t0), 1, nullptr, !part.empty(), lg, st));      // a single step leaves the token alone
         else if (T <= kSmallTokens && (!layers_out || t0 == 0))
             FX_TRY(run_small<ET>(m, s, tokens + t0, T, s.length + T, part.data(), (int)part.size(), lg, layers_out, st));
@@ -1132,11 +1136,14 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
     FX_TRY(flexllm_hybrid_timed_out(m));
     if (steps == 0) return FLEXLLM_OK;
     FX_TRY(set_state_launch(s.pos, s.length, 0, st));
-    if (top_k == 0 && walk_ready(m, st)) {
-        FX_TRY(walk(m, slot, token_io, steps, tokens_out, true, nullptr, st));
-    } else if (!use_graph) {
-        for (int i = 0; i < steps; i++) FX_TRY(decode_any(m, slot, s.length + steps, token_io, rands, top_k, tokens_out, st));
-    } else {
+    int done = 0;                                         // in one kernel, as far as that is the faster way
+    if (top_k == 0 && walk_ready(m, s.length, st)) {
+        done = std::min(steps, m->walk_rows - s.length);
+        FX_TRY(walk(m, slot, token_io, done, tokens_out, true, nullptr, st));
+    }
+    if (done < steps && !use_graph) {
+        for (int i = done; i < steps; i++) FX_TRY(decode_any(m, slot, s.length + steps, token_io, rands, top_k, tokens_out, st));
+    } else if (done < steps) {
         int splits = 0;                                   // of all layers together: none has fewer at more rows
         for (const HybridLayer& L : m->layers)
             if (L.d.mixer == FLEXLLM_MIX_SHARED_KV) splits += shared_kv_split_count(L.sd, 1, s.length + steps);
@@ -1156,7 +1163,7 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
             FX_HIP(e);
             m->graph_slot = slot; m->graph_topk = top_k; m->graph_io = token_io; m->graph_out = tokens_out; m->graph_rands = rands; m->graph_stream = st; m->graph_splits = splits;
         }
-        for (int i = 0; i < steps; i++) FX_HIP(hipGraphLaunch(m->graph, st));
+        for (int i = done; i < steps; i++) FX_HIP(hipGraphLaunch(m->graph, st));
     }
     s.length += steps;
     return FLEXLLM_OK;

@@ -75,6 +75,41 @@ def test_token_by_token_nifunex(name, dtype):
     check_nifunex(NIFUNEX[name], dtype, 70, [1], [50, 1])
 
 
+def test_long_sequences_leave_the_resident_kernel():
+    """From some number of rows on the chain of kernels is faster: a loop goes on in it where it gets there, steps too."""
+    from flexllm_amd import to_device, zeros
+    from flexllm_amd._lib import FlexLLMError
+    from flexllm_amd.lopazen import Lopazen
+    border = 8 * ((384 * 1024 + 160 * 1024) // (128 * 4))  # eight splits of the rows
+    cfg = lc.config([attention(32, 8, 128, 0)], width=1024, vocab=512)
+    m = Lopazen.from_tensors(cfg, lc.weights(cfg, 5), dtype="float32", max_pos=border + 64, slots=2)
+    toks = lc.tokens(cfg, border - 5)
+    a, b = [m.pool.acquire(n) for n in "ab"]
+    for s in a, b:
+        m.step(s, toks[:-1])                               # border - 6 rows
+    token, out = to_device(np.array(toks[-1:], np.int32)), zeros((20,), np.int32)
+    got = {}
+    for s, mode, graph in (a, 0, True), (b, 1, False):
+        m.set_decode_mode(mode)
+        token.copy_from(np.array(toks[-1:], np.int32))
+        m.decode(s, token, 3, out, use_graph=graph)
+        first = out.numpy()[:3].tolist()
+        m.decode(s, token, 17, out, use_graph=graph)
+        got[s] = first + out.numpy()[:17].tolist(), m.step(s, [3], [0])
+        m.check()
+    assert m.length(a) == border + 15 and got[a][0] == got[b][0]
+    assert lc.rel_err(got[a][1], got[b][1]).max() < lc.LIMIT["float32"]
+    m.set_decode_mode(0)
+    m.set_wait_limit(1)                                    # the resident kernel would give up
+    m.step(a, [3], [0])
+    m.pool.release("b")
+    b = m.pool.acquire("b")
+    m.step(b, toks[:-5])
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.step(b, [3], [0])
+    m.close()
+
+
 # float32: rows of one quad and of three, which no wave has the same part of in all rows
 FLOAT32 = {
     "shared rows of a quad": lc.config([attention(16, 4, 64, 1024)], width=1024, vocab=512),
