@@ -104,7 +104,8 @@ inline int walk_shared_kv_rows(const SharedKvDims& d, int width, int es) {
     return (int)(per_split * walk_splits(d.heads, d.dim));
 }
 inline bool walk_shared_kv_ok(const SharedKvDims& d) { return (d.dim == 64 || d.dim == 128) && d.dimp == d.dim && 4 * d.heads <= kWalkWG; }
-// The other two are made for one size of head: a slice of a head's columns per workgroup, 16 or 8 for each head.
+// The other two are made for one size of head: a slice of a head's columns per workgroup, 16 or 8 for each head, and which lane holds which
+// columns of a row is fixed when they are compiled.  Other sizes keep the chain of kernels, which takes any.
 constexpr int kWalkDim = 128, kWalkRot = 64, kWalkRank = 512, kWalkRow2 = kWalkRank + kWalkRot, kWalkGlaRank = 16;
 inline int walk_slices(int heads) { return heads <= 16 ? 16 : 8; }
 inline bool walk_latent_ok(const LatentDims& d) {

@@ -5,7 +5,7 @@
 // kernels of their own every link costs 3.5 us of launch and ramp beside its stream of weights: 16 layers of 2048, feed-forward 8192, bfloat16, 1531
 // tokens held, take 43 us each for 122 MB (17 us at the rate of a read stream).  Here a link costs an exchange between resident
 // workgroups, 1.3 us behind the slowest of them, and the weights, which do not hang on the activations, are asked for ahead of it: 33 us per
-// layer, 771 -> 615 us per token (four layers of 4096: 535 -> 478; ten layers, six of them twice, float32: 1098 -> 922).
+// layer, 771 -> 595 us per token (four layers of 4096: 535 -> 466; ten layers, six of them twice, float32: 1098 -> 903).
 // Eight of a workgroup's twelve waves ("stream waves") do nothing but walk through the workgroup's rows of all linears.  The other four ("service
 // waves") wait for the vectors, norm them, attend, finish the sums.  They meet at workgroup barriers: the vector is in LDS / the sums
 // are in LDS.  Answers of vector memory return to a wave in order, so a wave that streams could not see a word of another workgroup before its weights.
@@ -257,8 +257,8 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 while (at >= rq) at -= rq;
             };
             auto same = [&] { return igroup == cgroup && it == ct; };
-            // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (without that 624 us
-            // per token where it is 610; nothing asked for between linears: 658).  When the ring is full, the first two quads move into registers.
+            // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (16 layers of 2048, before
+            // the registers below: 610 us per token, 624 without that, 658 with nothing asked for between linears).  When the ring is full, the first two quads move into registers.
             i32x4 u[2][4];
             bool taken = false;
             if (first) {
