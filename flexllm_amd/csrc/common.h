@@ -60,6 +60,7 @@ void stream_scratch_release(hipStream_t st);
 // ResidentEnd, a... are the ones ahead of it.
 int resident_launch_args(const void* kernel, int grid, int block, void** args, size_t lds, hipStream_t st, ResidentEnd& end);
 int resident_ready();                      // at the creation of what launches them
+int resident_makes_room(hipStream_t st);   // behind the last kernel of a call that has many of other kinds
 template <class... P, class... A>
 int resident_launch(void (*kernel)(P...), int grid, int block, size_t lds, hipStream_t st, const A&... a) {
     std::tuple<P...> values(a..., ResidentEnd{nullptr, 0});

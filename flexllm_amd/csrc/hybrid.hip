@@ -1001,6 +1001,7 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
     const int W = m->cfg.width;
     std::vector<int> part;
     int w0 = 0;
+    bool chain = false;
     for (int t0 = 0; t0 < n;) {
         const int T = n - t0 < kPieceTokens ? n - t0 : kPieceTokens;
         part.clear();
@@ -1009,7 +1010,7 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
         float* lg = n_want ? logits + (size_t)w0 * m->cfg.vocab : nullptr;
         if (T == 1 && !layers_out && walk_ready(m, s.length, st))
             FX_TRY(walk(m, slot, const_cast<int*>(tokens + t0), 1, nullptr, !part.empty(), lg, st));      // a single step leaves the token alone
-        else if (T <= kSmallTokens && (!layers_out || t0 == 0))
+        else if (chain = true; T <= kSmallTokens && (!layers_out || t0 == 0))
             FX_TRY(run_small<ET>(m, s, tokens + t0, T, s.length + T, part.data(), (int)part.size(), lg, layers_out, st));
         else
             FX_TRY(run_many<ET>(m, s, tokens + t0, T, part.data(), (int)part.size(), lg, layers_out ? layers_out + (size_t)t0 * W : nullptr, (size_t)n * W, st));
@@ -1018,7 +1019,7 @@ static int run_step(flexllm_hybrid* m, int slot, const int* tokens, int n, const
         w0 = w1;
         t0 += T;
     }
-    return FLEXLLM_OK;
+    return chain ? resident_makes_room(st) : FLEXLLM_OK;
 }
 
 // One token of the decode loop: *token_io -> logits -> next token, position and step advance on the device.
@@ -1168,7 +1169,7 @@ int flexllm_hybrid_decode(flexllm_hybrid* m, int slot, int* token_io, int steps,
         for (int i = done; i < steps; i++) FX_HIP(hipGraphLaunch(m->graph, st));
     }
     s.length += steps;
-    return FLEXLLM_OK;
+    return done < steps ? resident_makes_room(st) : FLEXLLM_OK;
 }
 
 int flexllm_hybrid_generate(flexllm_hybrid* m, int slot, const int* prompt, int n_prompt, int steps, const float* rands, int top_k,

@@ -552,7 +552,7 @@ int flexllm_llama_decode_hidden(flexllm_llama* m, const float* x_in, int pos, fl
         int rc = decode_head(m, logits, st);
         if (rc) return rc;
     }
-    return FLEXLLM_OK;
+    return resident_makes_room(st);
 }
 
 int flexllm_llama_decode_greedy(flexllm_llama* m, int* token_io, int pos0, int steps, int* tokens_out, int use_graph,
@@ -576,7 +576,7 @@ int flexllm_llama_decode_greedy(flexllm_llama* m, int* token_io, int pos0, int s
             int rc = greedy_step(m, token_io, tokens_out, st);
             if (rc) return rc;
         }
-        return FLEXLLM_OK;
+        return resident_makes_room(st);
     }
     FX_REQUIRE(st != nullptr, "llama_decode_greedy: graph replay needs a non-default stream");
     if (!m->graph_exec || m->graph_token_io != token_io || m->graph_tokens_out != tokens_out || m->graph_stream != st) {
@@ -596,7 +596,7 @@ int flexllm_llama_decode_greedy(flexllm_llama* m, int* token_io, int pos0, int s
         m->graph_stream = st;
     }
     for (int s = 0; s < steps; s++) FX_HIP(hipGraphLaunch(m->graph_exec, st));
-    return FLEXLLM_OK;
+    return resident_makes_room(st);
 }
 
 int flexllm_llama_decode_sample(flexllm_llama* m, int* token_io, int pos0, int steps, const float* rands, int top_k,
@@ -634,7 +634,7 @@ int flexllm_llama_decode_sample(flexllm_llama* m, int* token_io, int pos0, int s
         topk_sample_kernel<256><<<1, 256, 0, st>>>(m->topk_val, m->topk_idx, kTopKParts * top_k, top_k, rands, 1, 1, out);
         FX_LAUNCH_CHECK();
     }
-    return FLEXLLM_OK;
+    return resident_makes_room(st);
 }
 
 int flexllm_llama_generate(flexllm_llama* m, const int* prompt, int n_prompt, int steps, const float* rands, int top_k,
@@ -668,6 +668,10 @@ int flexllm_llama_generate(flexllm_llama* m, const int* prompt, int n_prompt, in
     }
     copy_int_kernel<<<1, 1, 0, st>>>(prompt + s, m->gen_token);
     FX_LAUNCH_CHECK();
+    if (rows > 0) {
+        const int rc = resident_makes_room(st);
+        if (rc) return rc;
+    }
     if (steps == 0) return FLEXLLM_OK;
     if (top_k == 0) return flexllm_llama_decode_greedy(m, m->gen_token, s, steps, tokens_out, 0, stream);
     return flexllm_llama_decode_sample(m, m->gen_token, s, steps, rands, top_k, tokens_out, stream);
@@ -675,12 +679,12 @@ int flexllm_llama_generate(flexllm_llama* m, const int* prompt, int n_prompt, in
 
 int flexllm_llama_prefill_hidden(flexllm_llama* m, const float* x_in, int s, float* hidden_out, void* stream) {
     FX_REQUIRE(m && x_in, "llama_prefill_hidden: null pointer");
-    if (m->w4)
-        return llama_prefill_run_w4a4(m->cfg, m->layers.data(), m->layers4.data(), m->gamma, m->q_s, m->k_s, m->v_s, m->a_s,
-                                      m->rope_sin, m->rope_cos, m->k_cache, m->v_cache, m->cache_layer_bytes, &m->pws, x_in, s,
-                                      hidden_out, as_stream(stream));
-    return llama_prefill_run(m->cfg, m->layers.data(), m->gamma, m->q_s, m->k_s, m->v_s, m->a_s, m->rope_sin, m->rope_cos,
-                             m->k_cache, m->v_cache, m->cache_layer_bytes, &m->pws, x_in, s, hidden_out, as_stream(stream));
+    const int rc = m->w4 ? llama_prefill_run_w4a4(m->cfg, m->layers.data(), m->layers4.data(), m->gamma, m->q_s, m->k_s, m->v_s, m->a_s,
+                                                  m->rope_sin, m->rope_cos, m->k_cache, m->v_cache, m->cache_layer_bytes, &m->pws, x_in, s,
+                                                  hidden_out, as_stream(stream))
+                         : llama_prefill_run(m->cfg, m->layers.data(), m->gamma, m->q_s, m->k_s, m->v_s, m->a_s, m->rope_sin, m->rope_cos,
+                                             m->k_cache, m->v_cache, m->cache_layer_bytes, &m->pws, x_in, s, hidden_out, as_stream(stream));
+    return rc ? rc : resident_makes_room(as_stream(stream));
 }
 
 }  // extern "C"

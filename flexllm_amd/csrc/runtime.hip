@@ -64,6 +64,10 @@ int resident_launch_args(const void* kernel, int grid, int block, void** args, s
     FX_HIP(resident_run(kernel, grid, block, args, lds, st, end));
     return FLEXLLM_OK;
 }
+int resident_makes_room(hipStream_t st) {
+    FX_HIP(resident_works(st));
+    return FLEXLLM_OK;
+}
 int resident_ready() {
     FX_HIP(resident_prepare());
     return FLEXLLM_OK;

@@ -14,15 +14,16 @@ extern "C" hipError_t hipExtLaunchKernel(const void*, dim3, dim3, void**, size_t
 #include <vector>
 
 namespace {
-struct Launch { hipStream_t stream; int device; fx::ResidentEnd end; long behind; bool ended; };      // behind: the launch whose event its stream waits for
+struct Launch { hipStream_t stream; int device; fx::ResidentEnd end; std::set<long> behind; bool ended; };      // behind: those whose events its stream waits for
 std::mutex mu;
 std::vector<Launch> launches;
-std::map<int, long> last;                      // of a device
-std::map<hipStream_t, long> waits;             // of a stream: the latest launch that it waits for
-std::map<hipEvent_t, long> events;             // launch that carries the event
+std::map<int, long> last;                      // resident launch of a device
+std::map<hipStream_t, std::set<long>> waits;   // of a stream
+std::map<hipEvent_t, long> events;             // launch that carries the event, or that it stands behind
+std::set<long> owed;                           // ends of calls of other kinds that the next resident launch has to wait for
 std::set<hipStream_t> capturing;
-std::atomic<int> bad{0}, made{0}, carried{0}, waited{0};
-std::atomic<bool> stop{false};
+std::atomic<int> bad{0}, made{0}, carried{0}, waited{0}, recorded{0};
+std::atomic<bool> stop{false}, threaded{false};      // with threads, a call may end while a launch is on its way: the next one waits for it
 thread_local hipStream_t mine = nullptr;       // the caller's stream: no call may name another one
 thread_local int device = 0;
 thread_local fx::ResidentEnd* end_of = nullptr;
@@ -44,7 +45,9 @@ void run_device() {
             Launch& l = launches[i];
             if (l.ended || busy.count(l.stream)) continue;
             busy.insert(l.stream);
-            if ((l.behind >= 0 && !launches[l.behind].ended) || rand() % 3) continue;
+            bool free = rand() % 3 == 0;
+            for (long b : l.behind) free = free && launches[b].ended;
+            if (!free) continue;
             l.ended = true;
             if (l.end.word) __atomic_store_n(l.end.word, l.end.ticket, __ATOMIC_RELEASE);
         }
@@ -53,7 +56,8 @@ void run_device() {
 hipError_t launch(hipStream_t st, hipEvent_t end) {
     std::lock_guard<std::mutex> lk(mu);
     if (fail_next) { fail_next = false; return hipErrorLaunchFailure; }
-    const long n = (long)launches.size(), behind = waits.count(st) ? waits[st] : -1;
+    const long n = (long)launches.size();
+    const std::set<long> behind = waits[st];
     if (capturing.count(st)) {
         if (end || end_of->word) wrong("a captured launch takes part in the order");
         return hipSuccess;
@@ -61,8 +65,11 @@ hipError_t launch(hipStream_t st, hipEvent_t end) {
     if (last.count(device)) {
         const long p = last[device];
         const bool one_stream = launches[p].stream == st && st != hipStreamPerThread;
-        if (!one_stream && !launches[p].ended && behind < p) wrong("launch " + std::to_string(n) + " beside launch " + std::to_string(p));
+        if (!one_stream && !launches[p].ended && !behind.count(p)) wrong("launch " + std::to_string(n) + " beside launch " + std::to_string(p));
     }
+    for (long o : owed)
+        if (!threaded && launches[o].stream != st && !launches[o].ended && !behind.count(o)) wrong("launch " + std::to_string(n) + " ahead of call " + std::to_string(o));
+    owed.clear();
     launches.push_back({st, device, *end_of, behind, false});
     last[device] = n;
     if (end) { events[end] = n; carried++; }
@@ -87,15 +94,17 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
     named("hipEventRecord", st);
     std::lock_guard<std::mutex> lk(mu);
     if (capturing.count(st)) wrong("an event joins a stream's capture");
-    events[e] = last.count(device) ? last[device] : -1;
-    carried++;
+    for (long i = 0; i < (long)launches.size(); i++)
+        if (launches[i].stream == st) events[e] = i;
+    owed.insert(events[e]);
+    recorded++;
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t st, hipEvent_t e, unsigned) {
     named("hipStreamWaitEvent", st);
     std::lock_guard<std::mutex> lk(mu);
     if (!events.count(e)) wrong("a wait for an event that no launch carries");
-    else if (!waits.count(st) || waits[st] < events[e]) waits[st] = events[e];
+    else waits[st].insert(events[e]);
     waited++;
     return hipSuccess;
 }
@@ -113,6 +122,17 @@ static int go(int stream) {
     fx::ResidentEnd end;
     end_of = &end;
     return (int)fx::resident_run(nullptr, 256, 512, nullptr, 0, mine, end);
+}
+// a call of kernels of other kinds: whether an event is left behind it
+static bool ordinary(int stream) {
+    mine = handle(stream);
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        if (!capturing.count(mine)) launches.push_back({mine, device, {nullptr, 0}, waits[mine], false});
+    }
+    const int before = recorded;
+    if (fx::resident_works(mine) != hipSuccess) wrong("a call's end is refused");
+    return recorded != before;
 }
 static void set_capturing(int stream, bool on) {
     std::lock_guard<std::mutex> lk(mu);
@@ -159,16 +179,48 @@ int main() {
     go(4);
     device = 0;
     go(1);
+    // calls of other kinds: their turn comes ahead of the next launch on another stream
+    drain();
+    std::this_thread::sleep_for(std::chrono::nanoseconds(fx::kWorkNs));
+    if (ordinary(1) || ordinary(2)) wrong("an event where no resident launch was made");
+    go(1);
+    go(1);
+    if (ordinary(1)) wrong("an event on the only stream with resident launches");
+    if (!ordinary(2) || !ordinary(3) || !ordinary(0)) wrong("no event behind a call beside resident launches");
+    go(1);
+    go(1);
+    ordinary(2);
+    go(2);
+    if (!ordinary(2) || !ordinary(1)) wrong("no event where two streams have resident launches");
+    go(1);
+    go(2);
+    set_capturing(2, true);
+    if (ordinary(2)) wrong("an event into a capture");
+    set_capturing(2, false);
+    for (int i = 0; i < 3 * fx::kWorks; i++) ordinary(100 + i);       // more streams than places: the oldest ones are given up
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        while (owed.size() > (size_t)fx::kWorks) owed.erase(owed.begin());
+    }
+    go(1);
+    drain();
+    const int made_before = made;
     size_t n = launches.size();
+    threaded = true;
     std::vector<std::thread> threads;
     for (int k = 0; k < 4; k++)
-        threads.emplace_back([k] { for (int i = 0; i < 500; i++) go(k < 2 ? k : k == 2 ? -1 : 3 + i / 100 % 3); });
+        threads.emplace_back([k] {
+            for (int i = 0; i < 500; i++) {
+                go(k < 2 ? k : k == 2 ? -1 : 3 + i / 100 % 3);
+                if (i % 7 == k) ordinary(k);
+            }
+        });
     for (auto& t : threads) t.join();
     drain();
     stop = true;
     dev.join();
     n = launches.size() - n;
-    printf("%zu launches, %d events carried, %d waits\n", launches.size(), carried.load(), waited.load());
-    if (n != 2000 || made != 4) wrong("launches are missing, or too much was made");      // a word and an event for each of two devices
+    printf("%zu launches and calls, %d events carried, %d recorded, %d waits\n", launches.size(), carried.load(), recorded.load(), waited.load());
+    if (n < 2280 || made_before != 4 + fx::kWorks || made != made_before) wrong("launches are missing, or too much was made");      // a word and an event for each of two devices, the calls' events
     return bad != 0;
 }

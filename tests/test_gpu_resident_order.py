@@ -2,6 +2,7 @@
 gives what it gives alone."""
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -114,6 +115,40 @@ def test_a_stream_with_half_of_the_chip():
     m.close()
     half.destroy()
     all_of_it.destroy()
+
+
+def test_prompts_beside_decoding():
+    """Loops of tokens and the prompts of another stream take turns: the prompts do not wait for a gap between loops kernel by kernel."""
+    from flexllm_amd import to_device, zeros
+    a, b = lopazen(), lopazen()
+    prompt, token, out = to_device(np.array(lc.tokens(CFG, 200), np.int32)), to_device(np.array([3], np.int32)), zeros((16,), np.int32)
+    done, stop = [], threading.Event()
+
+    def prompts():
+        while not stop.is_set():
+            s = b.pool.acquire("p")
+            b.step(s, prompt)
+            b.pool.release("p")
+            done.append(1)
+
+    slot = a.pool.acquire("d")
+    a.decode(slot, token, 16, out)
+    a.stream().sync()
+    t = threading.Thread(target=prompts)
+    t.start()
+    while not done:
+        time.sleep(0.01)
+    before = len(done)
+    for _ in range(25):                                    # 400 tokens
+        a.decode(slot, token, 16, out)
+        a.stream().sync()
+    served = len(done) - before
+    stop.set()
+    t.join()
+    a.check()
+    assert served >= 12, served                            # a prompt per loop; kernel by kernel it is one per five
+    a.close()
+    b.close()
 
 
 def test_two_designs_and_ordinary_work():
