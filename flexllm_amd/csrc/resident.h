@@ -22,9 +22,11 @@ struct ResidentEnd {
 // Launches on one stream, or behind the last one's end, need nothing.  Where another stream's launch is still at work, the next one waits
 // for the event that it carries; it carries one for kSpell launches behind such a meeting, since an event costs 4.2 us of the stream's
 // time, and the word 0.2 (a short kernel and one of 100 us in turn; one step of Llama on a caller's stream 303.4 us with an event
-// behind each, 297.6 so).  The first launch of such a meeting finds no event and holds its caller until the word is there.
+// behind each, 297.6 so).  The first launch of such a meeting finds no event and holds its caller until the word is there, or for
+// a minute: that stream may wait for something that this caller does next.
 // In a stream that is being captured there is no order to keep: the launch runs when its graph does.
 constexpr int kMaxDevices = 64, kSpell = 64;
+constexpr long long kHoldNs = 60000000000;
 
 // Calls of many kernels that end by themselves (prompts, steps of several tokens, sampled tokens), on other streams than the resident
 // launches: between two of those one kernel gets in, so that a prompt of 150 kernels beside loops of 16 tokens takes a second.  Such a call
@@ -98,7 +100,7 @@ inline hipError_t resident_run(const void* kernel, int grid, int block, void** a
     // hipStreamPerThread is another stream in every thread
     if ((st != t->last || st == hipStreamPerThread) && !t->done()) {
         if (t->carries) e = hipStreamWaitEvent(st, t->end, 0);
-        else while (!t->done()) std::this_thread::sleep_for(std::chrono::microseconds(20));
+        else for (const long long until = resident_clock() + kHoldNs; !t->done() && resident_clock() < until;) std::this_thread::sleep_for(std::chrono::microseconds(20));
         if (e != hipSuccess) return e;
         t->spell = kSpell;
     }
