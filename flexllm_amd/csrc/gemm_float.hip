@@ -1,54 +1,16 @@
-// Floating-point GEMMs for prefill: C[m][n] = sum_k A[m][k] * W[n][k], both operands K-contiguous.
-//
-// bfloat16: the direct-load kernel of the int8 path (gemm_i8.h) on v_mfma_f32_32x32x16_bf16.  A lane's operand is the
-// same 16 bytes of a row as in the int8 instruction, so the LDS stage layout, the chunk rotation and the software
-// pipeline carry over with K counted in bytes.  Additions: rows of A may be gathered, groups of rows may have a weight
-// matrix each (experts), the epilogue adds a bias, splits the columns between an ET and a float32 output and applies the
-// gated unit to interleaved gate/up columns.
-//
-// float32: the same kernel on v_mfma_f32_32x32x2_f32 (full float32 products and sums).  The 16 bytes that a lane holds are four k of
-// a row, and instruction e of four takes its e-th: the two halves of the wave then stand for k apart, the same ones in
-// both operands, and a sum does not mind.  (A register-staged 64 x 64 tile, which this took the place of: 333 x 2048 x 8192 345 us,
-// now 173; 2048 x 4096 x 4096 950 us, now 602.)
+// Floating-point GEMMs for prefill: C[m][n] = sum_k A[m][k] * W[n][k], both operands K-contiguous, on the walk of gemm_walk.h.
+// Rows of A may be gathered, groups of rows may have a weight matrix each (experts), the epilogue adds a bias, splits the columns
+// between an ET and a float32 output and applies the gated unit to interleaved gate/up columns.
+#include <atomic>
 #include "float_ops.h"
-#include "gemm_i8.h"
+#include "gemm_walk.h"
 
 namespace fx {
 
-struct GemmTile { int row0, row_end, group; };
-
-// Which tile this workgroup works on: row tiles fastest inside a range of weight columns per XCD, as in gemm_i8_kernel.
-template <int BM, int BN>
-__device__ __forceinline__ bool gemm_pick_tile(const GemmArgs& g, int tiles_m, int tiles_n, GemmTile& t, int& col0) {
-    const int tile = blockIdx.x;
-    int tm, tn;
-    if ((tiles_n & 7) == 0) {
-        const int xcd = tile & 7, idx = tile >> 3;
-        tn = xcd * (tiles_n >> 3) + idx / tiles_m;
-        tm = idx % tiles_m;
-    } else {
-        tm = tile % tiles_m;
-        tn = tile / tiles_m;
-    }
-    col0 = tn * BN;
-    if (g.tiles) {
-        if (tm >= g.n_tiles[0]) return false;
-        const int4 e = g.tiles[tm];
-        t.group = e.x; t.row0 = e.y; t.row_end = e.z;
-    } else {
-        t.group = 0; t.row0 = tm * BM; t.row_end = min(g.m, t.row0 + BM);
-    }
-    return true;
-}
-
-// One row's four consecutive columns col..col+3 of the accumulator tile.
+// One row's four consecutive columns col..col+3.
 template <typename ET>
 __device__ __forceinline__ void gemm_store4(const GemmArgs& g, int row, int col, float (&v)[4], bool vec) {
     ET* y = static_cast<ET*>(g.y);
-    if (g.bias) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] += g.bias[min(col + e, g.n - 1)];
-    }
     if (vec) {
         if (col >= g.n) return;
         if (col >= g.n_split) {
@@ -77,186 +39,147 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs& g, int row, int col,
     }
 }
 
-// The accumulator tile of a wave turns through a private LDS patch so that a lane owns four consecutive columns.
-template <typename ET, int TM, int TN>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const GemmTile& t, int col0, int wm, int wn, int lane, float* patch,
-                                              f32x16 (&acc)[TM][TN]) {
-    constexpr int EP = 36;
-    const int pr = lane >> 3, pc = (lane & 7) * 4;
-    // four columns never straddle the split, and every store address is a multiple of the store's size
-    const bool vec = (g.n & 3) == 0 && (g.n_split & 3) == 0 && (g.ldy & 3) == 0 && (g.ldy32 & 3) == 0;
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) patch[((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * EP + (lane & 31)] = acc[i][j][r];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const int lr = p * 8 + pr, row = t.row0 + wm + i * 32 + lr;
-                const f32x4 q = *reinterpret_cast<const f32x4*>(patch + lr * EP + pc);
-                float v[4] = {q[0], q[1], q[2], q[3]};
-                if (row < t.row_end) gemm_store4<ET>(g, row, col0 + wn + j * 32 + pc, v, vec);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
-}
+// How the outputs of a product may leave.  kWide: columns below n_split, or those from there on, in whole 16-byte pieces (rows and outputs
+// start on such a border); kQuad: four columns never straddle the split and every store address is a multiple of the store's size;
+// kSingle: one by one.
+enum GemmStores { kSingle = 0, kQuad = 1, kWide = 2 };
 
-// A stage is 128 bytes of k of the tile's rows and columns; STAGES of them form the ring in LDS.
-// What bounds it: with one workgroup per CU the trip of a stage's bytes, so that everything LDS holds is in flight (two stages of
-// 128 x 128 in four waves, of which a CU could hold two: 213 us for 777 x 4096 x 14336, 224 tiles; four stages, eight waves: 117 us), and for the
-// largest tile LDS itself, which hands out 6 KiB of operands for 8 matrix instructions per wave.
-template <typename ET, int BM, int BN, int STAGES, int WPE, int NW>
-__global__ __launch_bounds__(NW * 64, WPE) void gemm_float_dma_kernel(GemmArgs g, int tiles_m, int tiles_n) {
-    constexpr int BKB = 128, GW = NW, WGN = GW / 2;
-    constexpr int WM = BM / 2, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
-    constexpr int CPR = BKB / 16, RPI = 64 / CPR;
-    constexpr int A_INSTR = BM / (GW * RPI), B_INSTR = BN / (GW * RPI);
-    static_assert(A_INSTR >= 1 && B_INSTR >= 1 && TM >= 1 && TN >= 1, "tile too small for this wave count");
-    constexpr int STAGE = (BM + BN) * BKB, KS = BKB / 32;
-    auto rot = [](int r) { return (r >> 1) & 7; };
-    extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
-
-    GemmTile tl;
-    int col0;
-    // scalar registers for the ends of the part: divisions are made in vector ones, and the loop would carry them along
-    const int part = blockIdx.y, stages = g.k * (int)sizeof(ET) / BKB;
-    const int k0 = __builtin_amdgcn_readfirstlane(part * stages / g.parts);
-    if (!gemm_pick_tile<BM, BN>(g, tiles_m, tiles_n, tl, col0)) return;
-    g.y32 += part * g.part_stride;
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
-    const int8_t* const a = static_cast<const int8_t*>(g.a) + (size_t)k0 * BKB;
-    const int8_t* const w = static_cast<const int8_t*>(g.w) + (size_t)tl.group * g.w_stride * sizeof(ET) + (size_t)k0 * BKB;
-
-    unsigned offa[A_INSTR], offb[B_INSTR];
+// A wave's outputs that all lie on one side of the split: J blocks of 16 columns at a time become 64 consecutive bytes of a row, 16 per
+// lane (GLU: the unit, 0: none; OT: type of the outputs).
+template <typename OT, class W, int GLU, bool BIAS>
+__device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias, float limit, int row0, int row_end, f32x4 (&acc)[W::MIv][W::NIv]) {
+    constexpr int R = (int)sizeof(OT) / (GLU ? 2 : 1), J = 4 / R, NI = W::NIv, MI = W::MIv;   // R: words of a lane's four columns
+    const int lane = threadIdx.x & 63, row_bytes = ldy * (int)sizeof(OT);
+    const TileRows out(y + (size_t)row0 * ldy, row_end - row0, row_bytes);
+    const int at = (lane & 15) * row_bytes + (lane >> 4) * 16;
 #pragma unroll
-    for (int j = 0; j < A_INSTR; j++) {
-        const int r = (wave * A_INSTR + j) * RPI + lane / CPR;
-        int row = min(tl.row0 + r, tl.row_end - 1);
-        if (g.row_src) row = g.row_src[row];
-        offa[j] = (unsigned)row * (unsigned)(g.lda * sizeof(ET)) + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
-    }
+    for (int j0 = 0; j0 < NI; j0 += J) {
+        f32x4 b[J];
+        if constexpr (BIAS) {
 #pragma unroll
-    for (int j = 0; j < B_INSTR; j++) {
-        const int r = (wave * B_INSTR + j) * RPI + lane / CPR;
-        offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)(g.ldw * sizeof(ET)) + (unsigned)(((lane % CPR) ^ rot(r)) * 16);
-    }
-    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)gemm_smem;
-    auto issue_stage = [&](int kt) {
-        const unsigned sb = lds0 + (unsigned)(kt % STAGES) * STAGE;
-        const size_t koff = (size_t)kt * BKB;
+            for (int j = 0; j < J; j++)
 #pragma unroll
-        for (int j = 0; j < A_INSTR; j++) gemm_dma_issue(a + koff, offa[j], sb + (wave * A_INSTR + j) * 1024);
-#pragma unroll
-        for (int j = 0; j < B_INSTR; j++) gemm_dma_issue(w + koff, offb[j], sb + BM * BKB + (wave * B_INSTR + j) * 1024);
-    };
-
-    f32x16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    const int nk = __builtin_amdgcn_readfirstlane((part + 1) * stages / g.parts) - k0;
-    constexpr int PER = A_INSTR + B_INSTR;
-    // everything the compiler loaded itself (tile table, gathered row numbers) has to be in before the counted loads start
-    gemm_wait_vmcnt<0>();
-#pragma unroll
-    for (int s0 = 0; s0 < STAGES - 1; s0++)
-        if (s0 < nk) issue_stage(s0);
-    const int fr = lane & 31, fg = lane >> 5;
-    using Frag = std::conditional_t<std::is_same<ET, float>::value, f32x4, bf16x8>;
-    auto read_frags = [&](int kt, int ks, Frag (&fa)[TM], Frag (&fb)[TN]) {
-        const int8_t* sa = gemm_smem + (kt % STAGES) * STAGE;
-        const int8_t* sb = sa + BM * BKB;
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int r = wm + i * 32 + fr;
-            fa[i] = *reinterpret_cast<const Frag*>(sa + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
+                for (int e = 0; e < 4; e++) b[j][e] = bias[(j0 + j) * 16 + (lane >> 4) * 4 + e];
         }
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int r = wn + j * 32 + fr;
-            fb[j] = *reinterpret_cast<const Frag*>(sb + r * BKB + (((ks * 2 + fg) ^ rot(r)) * 16));
-        }
-    };
-    auto mma = [&](const Frag (&fa)[TM], const Frag (&fb)[TN]) {
+        for (int i = 0; i < MI; i++) {
+            uint32_t w[J][R];
 #pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                if constexpr (std::is_same<ET, float>::value) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][e], fb[j][e], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < J; j++) {
+                f32x4 v = acc[i][j0 + j];
+                if constexpr (BIAS) v += b[j];
+                OT o[GLU ? 2 : 4];
+                if constexpr (GLU != 0) {
+                    o[0] = (OT)glu_f(GLU, v[0], v[1], limit);
+                    o[1] = (OT)glu_f(GLU, v[2], v[3], limit);
                 } else {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-                }
-            }
-    };
-    auto wait_stage = [&](int kt) {
-        const int younger = min(STAGES - 2, nk - 1 - kt);
-        if (younger >= 2) gemm_wait_vmcnt<2 * PER>();
-        else if (younger == 1) gemm_wait_vmcnt<PER>();
-        else gemm_wait_vmcnt<0>();
-    };
-    static_assert(STAGES <= 4 && 2 * PER < 64, "the wait distinguishes up to two younger stages");
-
-    Frag fa0[TM], fb0[TN], fa1[TM], fb1[TN];
-    wait_stage(0);
-    __syncthreads();
-    read_frags(0, 0, fa0, fb0);
-    // The last stage stands by itself, a branch less in the loop: 2 x 72 x 9024, one tile of 141 stages, 36.7 -> 31.0 us.
-    auto stage = [&](int kt, auto more) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ks += 2) {
-            read_frags(kt, ks + 1, fa1, fb1);
-            if (more && ks == 0 && kt + STAGES - 1 < nk) issue_stage(kt + STAGES - 1);
-            __builtin_amdgcn_sched_barrier(0);
-            mma(fa0, fb0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (ks + 2 < KS) {
-                read_frags(kt, ks + 2, fa0, fb0);
-            } else if (more) {
-                wait_stage(kt + 1);
-                __syncthreads();
-                read_frags(kt + 1, 0, fa0, fb0);
+                    for (int e = 0; e < 4; e++) o[e] = (OT)v[e];
+                }
+                __builtin_memcpy(w[j], o, sizeof(o));
             }
-            __builtin_amdgcn_sched_barrier(0);
-            mma(fa1, fb1);
-            __builtin_amdgcn_sched_barrier(0);
+            join_blocks<R>(w);
+            out.put(&w[0][0], at + i * 16 * row_bytes + j0 * 16 * (int)sizeof(OT) / (GLU ? 2 : 1));
+            __builtin_amdgcn_sched_barrier(0);                 // one piece after the other: all at once are more than the registers hold
         }
-    };
-    for (int kt = 0; kt < nk - 1; kt++) stage(kt, std::true_type());
-    stage(nk - 1, std::false_type());
+    }
+}
+
+template <typename ET, class W>
+__device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_end, int col0, int stores, int8_t* smem, f32x4 (&acc)[W::MIv][W::NIv]) {
+    constexpr int NI = W::NIv, MI = W::MIv, J = std::is_same<ET, float>::value ? 2 : 4;
+    const int lane = threadIdx.x & 63, fg = lane >> 4, fr = lane & 15, end = col0 + NI * 16;
+    const float* bias = g.bias ? g.bias + col0 : nullptr;
+    if (stores == kWide && col0 >= g.n_split && end <= g.n) {
+        float* y = g.y32 + (col0 - g.n_split);
+        if (bias) return gemm_out_wide<float, W, 0, true>(y, g.ldy32, bias, 0.0f, row0, row_end, acc);
+        return gemm_out_wide<float, W, 0, false>(y, g.ldy32, bias, 0.0f, row0, row_end, acc);
+    }
+    if constexpr (NI % J == 0) {
+        if (stores == kWide && end <= g.n_split && !(bias && g.glu)) {
+            ET* y = static_cast<ET*>(g.y);
+            if (g.glu == kGluClamped) return gemm_out_wide<ET, W, kGluClamped, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, acc);
+            if (g.glu == kGluGelu) return gemm_out_wide<ET, W, kGluGelu, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, acc);
+            if (bias) return gemm_out_wide<ET, W, 0, true>(y + col0, g.ldy, bias, 0.0f, row0, row_end, acc);
+            return gemm_out_wide<ET, W, 0, false>(y + col0, g.ldy, bias, 0.0f, row0, row_end, acc);
+        }
+    }
+    // Any other: sixteen columns of the wave's rows at a time through LDS, so that a loop can take them (the walk has left it behind: the
+    // barrier is for the other waves' reads).
     __syncthreads();
-    gemm_epilogue<ET, TM, TN>(g, tl, col0, wm, wn, lane, reinterpret_cast<float*>(gemm_smem) + wave * (32 * 36), acc);
+    float* patch = reinterpret_cast<float*>(smem) + W::wave() * (MI * 256);
+    f32x4* mine = reinterpret_cast<f32x4*>(patch) + lane;
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+#pragma unroll
+        for (int i = 0; i < MI; i++) mine[i * 64] = acc[i][j];          // a lane reads back what it wrote
+#pragma clang loop unroll(disable)
+        for (int i = 0; i < MI; i++) {
+            const int row = row0 + i * 16 + fr;
+            const f32x4 q = mine[i * 64];
+            const int col = col0 + j * 16 + fg * 4;
+            float v[4] = {q[0], q[1], q[2], q[3]};
+            if (g.bias) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] += g.bias[min(col + e, g.n - 1)];
+            }
+            if (row < row_end) gemm_store4<ET>(g, row, col, v, stores != kSingle);
+        }
+    }
 }
 
-constexpr int gemm_float_lds(int bm, int bn, int stages, int nw) {
-    const int ring = stages * (bm + bn) * 128, epi = nw * 32 * 36 * 4;
-    return ring > epi ? ring : epi;
+template <typename ET, int WM, int MI, int NI, int NA, int NB>
+struct FloatWalk : GemmWalk<ET, WM, MI, NI, NA, NB> { static constexpr int MIv = MI, NIv = NI; };
+
+template <typename ET, class W>
+__global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmArgs g, int tiles_m, int tiles_n, int stores) {
+    extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
+    int tm, tn, group = 0, row0, row_end;
+    gemm_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    if (g.tiles) {
+        if (tm >= g.n_tiles[0]) return;
+        const int4 e = g.tiles[tm];
+        group = e.x; row0 = e.y; row_end = e.z;
+    } else {
+        row0 = tm * W::BM; row_end = min(g.m, row0 + W::BM);
+    }
+    const int col0 = tn * W::BN;
+    // scalar registers for the ends of the part: divisions are made in vector ones, and the loop would carry them along
+    const int part = blockIdx.y, stages = g.k * (int)sizeof(ET) / 128;
+    const int k0 = __builtin_amdgcn_readfirstlane(part * stages / g.parts), k1 = __builtin_amdgcn_readfirstlane((part + 1) * stages / g.parts);
+    g.y32 += part * g.part_stride;
+    unsigned offa[W::AI], offb[W::BI];
+#pragma unroll
+    for (int j = 0; j < W::AI; j++) {
+        const int r = W::load_row_a(j);
+        int row = min(row0 + r, row_end - 1);
+        if (g.row_src) row = g.row_src[row];
+        offa[j] = (unsigned)row * (unsigned)(g.lda * sizeof(ET)) + W::load_byte(r);
+    }
+#pragma unroll
+    for (int j = 0; j < W::BI; j++) {
+        const int r = W::load_row_b(j);
+        offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)(g.ldw * sizeof(ET)) + W::load_byte(r);
+    }
+    f32x4 acc[W::MIv][W::NIv];
+    W::run(static_cast<const int8_t*>(g.a) + (size_t)k0 * 128, static_cast<const int8_t*>(g.w) + (size_t)group * g.w_stride * sizeof(ET) + (size_t)k0 * 128, offa, offb,
+           k1 - k0, gemm_smem, acc);
+    const int r0 = row0 + W::row_of_wave(), c0 = col0 + W::col_of_wave();
+    gemm_out<ET, W>(g, r0, row_end, c0, stores, gemm_smem, acc);
 }
 
-template <typename ET, int BM, int BN, int STAGES, int WPE, int NW>
-static int launch_dma(const GemmArgs& g, hipStream_t st) {
-    constexpr int lds = gemm_float_lds(BM, BN, STAGES, NW);
+template <typename ET, int WM, int MI, int NI, int NA, int NB>
+static int launch_walk(const GemmArgs& g, hipStream_t st) {
+    using W = FloatWalk<ET, WM, MI, NI, NA, NB>;
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float_walk_kernel<ET, W>), hipFuncAttributeMaxDynamicSharedMemorySize, W::kLds));
         opted_in.store(true, std::memory_order_release);
     }
-    const int tm = g.tiles ? g.max_tiles : (g.m + BM - 1) / BM, tn = (g.n + BN - 1) / BN;
-    gemm_float_dma_kernel<ET, BM, BN, STAGES, WPE, NW><<<dim3(tm * tn, g.parts), NW * 64, lds, st>>>(g, tm, tn);
+    const int tm = g.tiles ? g.max_tiles : (g.m + W::BM - 1) / W::BM, tn = (g.n + W::BN - 1) / W::BN;
+    const bool quad = (g.n & 3) == 0 && (g.n_split & 3) == 0 && (g.ldy & 3) == 0 && (g.ldy32 & 3) == 0;
+    const bool wide = quad && rows_fit(g.ldy, sizeof(ET)) && rows_fit(g.ldy32, 4) && g.ldy % (16 / (int)sizeof(ET)) == 0 && ((reinterpret_cast<uintptr_t>(g.y) | reinterpret_cast<uintptr_t>(g.y32)) & 15) == 0;
+    gemm_float_walk_kernel<ET, W><<<dim3(tm * tn, g.parts), 256, W::kLds, st>>>(g, tm, tn, wide ? kWide : quad ? kQuad : kSingle);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
@@ -306,17 +229,15 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
 }
 
 // The tile whose rounds over the chip take the least time.  cost: of one stage of a round, and `round` once per round, in 0.01 us, as
-// measured where all CUs are busy; per_cu: workgroups that a CU holds at a time.  The bfloat16 ones are those that lose least over 520 sizes of 1
-// to 4096 rows and 64 to 14336 k: the tiles picked are 0.6 % from the best ones on average.  What a round costs besides its stages decides where k
-// is short and the outputs' stores bound the product: 2409 x 5608 x 256 23.7 us on 256 x 256, 20.5 on 128 x 128 twice per CU,
-// where 1621 x 22276 x 320 takes 54.8 us on 128 x 256 and 63.4 on those; 2070 x 9468 x 5632 293 us on 128 x 128, 253 on 128 x 256.
+// measured where all CUs are busy; per_cu: workgroups that the rule counts with per CU.  The bfloat16 ones were set by 520 sizes of 1
+// to 4096 rows and 64 to 14336 k on an earlier kernel; on this one the tiles picked are 1.1 % from the best ones on average over 44 sizes.  What a
+// round costs besides its stages decides where k is short and the outputs' stores bound the product: 2806 x 6656 x 512 29 us on 160 rows
+// of 256 columns and on 128 x 128 twice per CU, 37 on 128 x 256 and 38 on 128 x 128.
 //
-// bfloat16 (64 k): 777 x 28672 x 4096 takes 256 x 256 (2 rounds, 230 us; 128 x 128: 7 rounds, 255 us), 1531 x 16384 x 2048 128 x 256 (3
-// rounds, 113 us; 256 x 256: 2 rounds, 141 us), 777 x 4096 x 14336 128 x 128 (1 round, 117 us; 128 x 256: 170 us), 1024 x 2048 x 2048
-// 64 x 128 (14.4 us; 128 x 128: 19.4 us).  128 x 128 in four waves with two stages fits twice into a CU: 3700 x 2064 x 8576, 493 tiles,
-// takes one round of it (130 us; two rounds of the one with four stages: 181 us).
-// float32 (32 k): 333 x 16384 x 2048 takes 64 x 128 (251 us; 64 x 64: 265, 128 x 128: 289 us), 333 x 2048 x 8192 64 x 64 (173 us; 64 x 128:
-// 276 us), 2048 x 4096 x 4096 128 x 128 (602 us, 114 TFLOP/s; 64 x 64: 656 us).
+// bfloat16 (64 k): 777 x 28672 x 4096 takes 256 columns (169 us; 128 x 128: 222 us), 1531 x 16384 x 2048 too (86 us; 123), 777 x 4096 x 14336
+// 128 x 128 (1 round, 99 us; 128 x 256: 159 us), 1024 x 2048 x 2048 64 x 128 (16.0 us; 128 x 128: 21.4 us).  128 x 128 with two stages fits
+// twice into a CU: 1389 x 6528 x 640 22.5 us, 27.5 on the one with five stages.
+// float32 (32 k): 333 x 16384 x 2048 takes 64 x 128 (196 us; 128 x 128: 244 us), 333 x 2048 x 8192 64 x 64 (135 us; 64 x 128: 248 us).
 struct GemmTileCost { int bm, bn, cost, round, per_cu; };
 template <typename ET> struct GemmTiles;
 template <> struct GemmTiles<bf16_t> {
@@ -335,6 +256,23 @@ static int gemm_cheapest_tile(const GemmArgs& g, int parts, long& best) {
         i++;
     }
     return pick;
+}
+
+// bfloat16 products whose tile has 256 columns share their rows out anew: any multiple of 32 from 128 to 256 rows is a tile of its own on the
+// same walk, and the one whose rounds cost least is taken (as above, in 0.01 us; the choices of 44 sizes of 120 to 4096 rows are 0.2 % from
+// the best ones on average).  777 x 28672 x 4096 takes 224 rows (170 us; 256: 185, 128: 211), 1531 x 16384 x 2048 192 (88 us; 256: 111,
+// 128: 103), 2596 x 3712 x 2560 160 (51 us; 256: 63, 128: 69), 722 x 10496 x 10112 128 (140 us; 160: 171, 256: 186).
+struct GemmWideRows { int rows, stage, round; };
+constexpr GemmWideRows kGemmWideRows[] = {{256, 135, 1100}, {224, 119, 1000}, {192, 105, 900}, {160, 99, 800}, {128, 83, 700}};
+static int gemm_wide_rows(int m, int k, int n, int parts) {
+    const long stages = ((long)k * 2 / 128 + parts - 1) / parts;
+    long best = 0;
+    int rows = 0;
+    for (const GemmWideRows& t : kGemmWideRows) {
+        const long tiles = (long)((m + t.rows - 1) / t.rows) * ((n + 255) / 256) * parts, cost = (tiles + 255) / 256 * (t.stage * stages + t.round);
+        if (!rows || cost < best) { best = cost; rows = t.rows; }
+    }
+    return rows;
 }
 
 // Few rows of a long k leave most CUs without a tile, so k is shared out.  A part costs its sums' way to memory and back (8 bytes
@@ -375,28 +313,31 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
     }
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
-        case 0: return launch_dma<bf16_t, 256, 256, 2, 2, 8>(g, st);
-        case 1: return launch_dma<bf16_t, 128, 256, 3, 2, 8>(g, st);
-        case 2: return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
-        case 3: return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
-        case 4: return launch_dma<bf16_t, 64, 64, 4, 2, 4>(g, st);
-        default: return launch_dma<bf16_t, 128, 128, 2, 2, 4>(g, st);
+        case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
+            case 256: return launch_walk<bf16_t, 2, 8, 8, 3, 2>(g, st);
+            case 224: return launch_walk<bf16_t, 2, 7, 8, 3, 2>(g, st);
+            case 192: return launch_walk<bf16_t, 2, 6, 8, 3, 2>(g, st);
+            case 160: return launch_walk<bf16_t, 2, 5, 8, 3, 2>(g, st);
+            default: return launch_walk<bf16_t, 2, 4, 8, 4, 3>(g, st);
+        }
+        case 2: return launch_walk<bf16_t, 2, 4, 4, 5, 5>(g, st);
+        case 3: return launch_walk<bf16_t, 2, 2, 4, 6, 6>(g, st);
+        case 4: return launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
+        default: return launch_walk<bf16_t, 2, 4, 4, 2, 2>(g, st);
     }
 }
 
-// Experts: their weights are read once and little else, so the tiles keep as many bytes in flight as LDS holds (64 experts of
-// 2048 x 2048 and 2048 x 1024, 1024 tokens, top 6: 134 us on average with two stages in four waves, 122 with four in eight;
-// the weights alone are 73 us at 5.5 TB/s).  With fewer than 45 rows per expert most of a wide tile's rows are none, and three workgroups per
-// CU on 64 x 64 hide more of each other's trips (the mixture's whole prompt of 9 rows 1711 -> 1666 us, 333 rows 2743 -> 2669, 450 rows
-// 2830 -> 2772; 500 rows, 47 per expert, 2841 and 2850, 600 rows 3093 and 3143).
+// Experts: their weights are read once and little else, so the tiles keep as many bytes in flight as LDS holds (1024 tokens, top 6 of
+// 64 experts of 2048 x 2048 and 2048 x 1024: 143 and 90 us; the weights alone are 98 and 49 at 5.5 TB/s).  With fewer than 45 rows
+// per expert most of a wide tile's rows are none, and three workgroups per CU on 64 x 64 hide more of each other's trips.
 template <int BM>
 static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
-    if constexpr (BM == 128) return launch_dma<bf16_t, 128, 128, 4, 2, 8>(g, st);
-    else if (g.group_rows < 45) return launch_dma<bf16_t, 64, 64, 3, 3, 4>(g, st);
-    else return launch_dma<bf16_t, 64, 128, 4, 2, 8>(g, st);
+    if constexpr (BM == 128) return launch_walk<bf16_t, 2, 4, 4, 5, 5>(g, st);
+    else if (g.group_rows < 45) return launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
+    else return launch_walk<bf16_t, 2, 2, 4, 6, 6>(g, st);
 }
 
 // ---- float32 -----------------------------------------------------------------------------------------------------
@@ -408,9 +349,9 @@ int gemm_float<float>(const GemmArgs& args, hipStream_t st) {
     FX_REQUIRE(!g.tiles, "gemm_float: a tile table goes to gemm_grouped");
     long cost;
     switch (gemm_cheapest_tile<float>(g, g.parts, cost)) {
-        case 0: return launch_dma<float, 128, 128, 4, 2, 8>(g, st);
-        case 1: return launch_dma<float, 64, 128, 4, 2, 8>(g, st);
-        default: return launch_dma<float, 64, 64, 4, 2, 4>(g, st);
+        case 0: return launch_walk<float, 2, 4, 4, 5, 5>(g, st);
+        case 1: return launch_walk<float, 2, 2, 4, 6, 6>(g, st);
+        default: return launch_walk<float, 2, 2, 2, 3, 3>(g, st);
     }
 }
 
@@ -419,8 +360,8 @@ static int gemm_grouped_f32(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 4);
     if (rc) return rc;
-    if constexpr (BM == 128) return launch_dma<float, 128, 64, 4, 2, 4>(g, st);
-    else return launch_dma<float, 64, 64, 4, 2, 4>(g, st);
+    if constexpr (BM == 128) return launch_walk<float, 2, 4, 2, 3, 3>(g, st);
+    else return launch_walk<float, 2, 2, 2, 3, 3>(g, st);
 }
 
 template <typename ET>
@@ -457,6 +398,16 @@ int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, in
     *cols = t.bn;
     *per_cu = t.per_cu;
     return FLEXLLM_OK;
+}
+
+int flexllm_linear_float_gemm_rows(int m, int k, int n, int dtype, int parts) {
+    FX_REQUIRE((dtype == 0 || dtype == 1) && m > 0 && n > 0 && k > 0 && k % kKPad == 0 && parts > 0, "linear_float_gemm_rows: m=%d k=%d n=%d dtype=%d", m, k, n, dtype);
+    GemmArgs g;
+    g.m = m; g.k = k; g.n = n;
+    long cost;
+    if (dtype) return GemmTiles<float>::list[gemm_cheapest_tile<float>(g, parts, cost)].bm;
+    const GemmTileCost& t = GemmTiles<bf16_t>::list[gemm_cheapest_tile<bf16_t>(g, parts, cost)];
+    return t.bn == 256 ? gemm_wide_rows(m, k, n, parts) : t.bm;
 }
 
 int flexllm_linear_float_gemm_parts(int m, int k, int n, int dtype, int most) {

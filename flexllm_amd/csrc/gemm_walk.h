@@ -1,0 +1,273 @@
+// The walk over k that the GEMMs of many rows share (int8, bfloat16 and float32): C[m][n] = sum_k A[m][k] * W[n][k], both operands
+// K-contiguous, on 16 x 16 matrix instructions.
+//
+// Four waves per workgroup, one per SIMD, as a grid of WM x 4/WM; a wave's tile is MI x NI blocks of 16 x 16.  Rows go global -> LDS by
+// direct loads in stages of 128 bytes of k (whole lines; halves of them reach 14.5 TB/s where lines reach 23), through a ring of NA
+// stages of A and one of NB stages of W.  A lane's 16 bytes of a row are one operand, so nothing is transposed; the 16-byte chunks of
+// row r are stored rotated by (r >> 1) & 7, which is applied on the global side of the load, and the operand reads are free of conflicts.
+//
+// What bounds it.  A 256 x 256 tile reads 32 KiB of operands from LDS per 16 KiB that arrive, against 48 with eight waves of 128 x 64: with
+// those, LDS was busy all the time and the matrix cores 55 % of it.  Now they are busy for 80 % of the cycles and the chip's power
+// holds the clock at 1.9 GHz (16 x 16 instructions take less of it than 32 x 32 ones: those kept it at 1.66 GHz, at 88 %, and took 4 to
+// 6 % more time).  What it took: each matrix instruction has at most an operand read and one half of a direct load behind it; the
+// loads of a stage are spread over one and a half k-steps (in a burst they queue up and the matrix instructions behind them
+// wait), and A is a stage further ahead than W, which is what fits into 160 KiB.
+// bfloat16, before (eight waves, 32 x 32 instructions) and now, us: 4096 x 4096 x 14336 (m, n, k) 407 and 320, 1504 TFLOP/s; 4096 x 28672 x 4096 879
+// and 706; 4096 x 4096 x 4096 127 and 98; 777 x 4096 x 14336 on 128 x 128 113 and 99; 1024 x 2048 x 2048 on 64 x 128 16.6 and 16.0.
+// float32: 333 x 16384 x 2048 205 and 182, 333 x 2048 x 8192 150 and 135.
+//
+// The operands of the matrix instruction are exchanged: W's rows are its rows, A's rows its columns.  A lane then holds four
+// consecutive columns n of one row m, and the outputs leave without a turn through LDS.
+#pragma once
+#include "elem.h"
+
+namespace fx {
+
+template <typename ET> struct MatrixOp;
+template <> struct MatrixOp<int8_t> {
+    using Frag = i32x4; using Acc = i32x4;
+    static __device__ __forceinline__ void mma(const Frag& w, const Frag& a, Acc& c) { c = __builtin_amdgcn_mfma_i32_16x16x64_i8(w, a, c, 0, 0, 0); }
+};
+template <> struct MatrixOp<bf16_t> {
+    using Frag = bf16x8; using Acc = f32x4;
+    static __device__ __forceinline__ void mma(const Frag& w, const Frag& a, Acc& c) { c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, c, 0, 0, 0); }
+};
+template <> struct MatrixOp<float> {     // 16 bytes are four k of a row; an instruction takes the same one of every lane, in both operands
+    using Frag = f32x4; using Acc = f32x4;
+    static __device__ __forceinline__ void mma(const Frag& w, const Frag& a, Acc& c) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e ^ 1], a[e ^ 1], c, 0, 0, 0);   // any order will do
+    }
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {                 // s_waitcnt vmcnt(N) only; the count is a 6-bit split immediate
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+// The tile of workgroup `id`.  Ids go to the eight dies in turn, each with an L2 of its own: of every 256 tiles (a round over the chip) a
+// die takes 32 in a row, which are eight row tiles by four column tiles.  They read 12 stages of rows per stage where 32 row
+// tiles by one column tile read 33.
+__device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int total = tiles_m * tiles_n, round = id & ~255, in = id & 255, left = min(total - round, 256), die = in & 7;
+    const int t = round + die * (left >> 3) + min(die, left & 7) + (in >> 3);
+    constexpr int G = 8;
+    const int group = t / (G * tiles_n), rows = min(G, tiles_m - group * G), o = t - group * G * tiles_n;
+    tm = group * G + o % rows;
+    tn = o / rows;
+}
+
+// R words of each of 4/R blocks, as lanes hold them (lane group g of 16 lanes has words g*R .. g*R + R - 1 of a block's row), become four
+// consecutive words per lane: group g then has words 4g .. 4g + 3 of the row through all the blocks, in the order w[0][0], w[0][1] ...
+template <int R>
+__device__ __forceinline__ void join_blocks(uint32_t (&w)[4 / R][R]) {
+    auto swap32 = [](uint32_t& a, uint32_t& b) { const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false); a = r[0]; b = r[1]; };
+    auto swap16 = [](uint32_t& a, uint32_t& b) { const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false); a = r[0]; b = r[1]; };
+    if constexpr (R == 2) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) { swap32(w[0][r], w[1][r]); swap16(w[0][r], w[1][r]); }
+    } else if constexpr (R == 1) {
+        swap32(w[0][0], w[2][0]); swap32(w[1][0], w[3][0]);
+        swap16(w[0][0], w[1][0]); swap16(w[2][0], w[3][0]);
+    }
+}
+
+// Rows of an output (or a residual) as a tile sees them: 16-byte accesses at byte offsets behind its first row.  What lies behind the last
+// row is neither written nor read (zeros come back), and neither is offset kNowhere: no branch stands around a store, so that
+// loads issued ahead of stores are not waited for together with them.  A tile's rows have to stay below 2 GiB (rows_fit).
+constexpr int kNowhere = -1;
+inline bool rows_fit(int ld, int bytes) { return (size_t)256 * ld * bytes < (1ull << 31); }
+struct TileRows {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ TileRows(void* first_row, int rows, int row_bytes)
+        : r(__builtin_amdgcn_make_buffer_rsrc(first_row, 0, rows > 0 ? rows * row_bytes : 0, 0x00027000)) {}
+    __device__ __forceinline__ void put(const uint32_t* w, int at) const {
+        const i32x4 v = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, at, 0, 0);
+    }
+    __device__ __forceinline__ f32x4 get(int at) const {
+        const i32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
+        return {__int_as_float(v[0]), __int_as_float(v[1]), __int_as_float(v[2]), __int_as_float(v[3])};
+    }
+};
+
+template <typename ET, int WM, int MI, int NI, int NA, int NB>
+struct GemmWalk {
+    using Op = MatrixOp<ET>;
+    using Frag = typename Op::Frag;
+    using Acc = typename Op::Acc;
+    static constexpr int WN = 4 / WM, BM = WM * MI * 16, BN = WN * NI * 16;
+    static constexpr int RA = (BM + 31) / 32 * 32, RB = BN;    // rows in LDS: every wave issues the same number of loads, of eight rows each
+    static constexpr int AI = RA / 32, BI = RB / 32, PER = AI + BI;
+    static constexpr int ASZ = RA * 128, BSZ = RB * 128, kLds = NA * ASZ + NB * BSZ;
+    static_assert(WM == 1 || WM == 2, "waves along the rows");
+    static_assert(RB % 32 == 0 && (NA == NB || NA == NB + 1) && NB >= 2 && kLds <= 160 * 1024, "ring");
+    // waves per SIMD that registers have to leave room for: as many workgroups as LDS does, two waves' worth of registers where that is enough
+    static constexpr int per_cu() { return kSumsApart ? 1 : 160 * 1024 / kLds < 2 ? 2 : 160 * 1024 / kLds < 3 ? 2 : 3; }
+    // a wave's loads in flight behind those of the stage that a wait is for, `younger` stages behind it
+    static constexpr int in_flight(int younger) {
+        const int a = younger < NA - 1 ? younger : NA - 1, b = younger < NB - 1 ? younger : NB - 1;
+        // loads of stage s go out behind the barrier of stage s - NB (W) and s - NA (A), W ahead of A
+        return NA == NB ? (a < NB - 2 ? a : NB - 2) * PER : (a < NB - 1 ? a : NB - 1) * AI + (b < NB - 2 ? b : NB - 2) * BI;
+    }
+    static_assert((NB - 1) * PER < 64, "wait count");
+    // Beyond a wave's 256 vector registers the sums live in the accumulation registers.
+    static constexpr bool kSumsApart = (MI * NI + 2 * (MI + NI)) * 4 > 210;
+
+    // Place, counted in matrix instructions behind a barrier, at which the j-th load of W (A) is aimed; it goes out behind the next matrix
+    // instruction, in the same stage.
+    static constexpr int NM = MI * NI, NR = MI + NI, KS = 2;
+    static constexpr int SB = NM / 2 > BI ? NM / 2 : BI, SA = KS * NM - SB < NM ? KS * NM - SB : NM;
+    static constexpr int slot_b(int j) { return j * SB / BI; }
+    static constexpr int slot_a(int j) { return SB + j * SA / AI + (SB + j * SA / AI == NM - 1); }
+    static constexpr int early() {                             // A's loads inside the last k-step
+        int n = 0;
+        for (int j = 0; j < AI; j++) n += slot_a(j) + 1 < NM;
+        return n;
+    }
+    static_assert(SB < NM && SA >= 2 * AI && slot_b(BI - 1) + 1 <= SB && slot_a(AI - 1) + 1 < KS * NM, "places of the loads");
+
+    static __device__ __forceinline__ int rot(int r) { return (r >> 1) & 7; }
+    static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+    static __device__ __forceinline__ int row_of_wave() { return (wave() / WN) * (MI * 16); }
+    static __device__ __forceinline__ int col_of_wave() { return (wave() % WN) * (NI * 16); }
+    // row of the tile that this lane's j-th load of A (W) is for, and the lane's byte within the 128 of the stage
+    static __device__ __forceinline__ int load_row_a(int j) { return (wave() * AI + j) * 8 + ((int)threadIdx.x & 63) / 8; }
+    static __device__ __forceinline__ int load_row_b(int j) { return (wave() * BI + j) * 8 + ((int)threadIdx.x & 63) / 8; }
+    static __device__ __forceinline__ unsigned load_byte(int r) { return (unsigned)((((int)threadIdx.x & 7) ^ rot(r)) * 16); }
+
+    // a, w: first byte of k of the operands; offa, offb: byte offsets of this lane's loads behind them; nk: stages.  Nothing else of the
+    // workgroup may be on its way to LDS.  Ends with every wave's loads and reads of LDS complete, without a barrier.
+    static __device__ __forceinline__ void run(const int8_t* a, const int8_t* w, const unsigned (&offa)[AI], const unsigned (&offb)[BI], int nk, int8_t* smem,
+                                               Acc (&acc)[MI][NI]) {
+        const int lane = threadIdx.x & 63, wv = wave();
+        const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+        const unsigned lds_a = lds0 + wv * (AI * 1024), lds_b = lds0 + NA * ASZ + wv * (BI * 1024);
+        // A direct load takes its LDS address from m0.  In two halves, with a matrix instruction between them: the address has to be
+        // in m0 one wait state ahead of the load.  Nothing else in this loop uses m0.
+        auto aim = [&](unsigned base, int j) __attribute__((always_inline)) { asm volatile("s_add_u32 m0, %0, %1" :: "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc"); };
+        auto load = [&](const int8_t* p, unsigned off) __attribute__((always_inline)) { asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p) : "memory"); };
+        auto load_now = [&](const int8_t* p, unsigned off, unsigned base, int j) __attribute__((always_inline)) {
+            aim(base, j);
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p) : "memory");
+        };
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NI; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[i][j][r] = 0;
+        // Zeros of its own for every block: from one shared zero the compiler cannot keep the sums in place, and the loop is full of moves.
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NI; j++) {
+                if constexpr (kSumsApart) asm volatile("" : "+a"(acc[i][j])); else asm volatile("" : "+v"(acc[i][j]));
+            }
+        wait_vmcnt<0>();                                        // what the compiler loaded itself stays out of the counts
+        // Behind the barrier of stage e: W's loads of stage e + NB over the first half of the last k-step, then A's of e + NA over
+        // as many matrix instructions as a k-step has.
+        constexpr int early_a = early();
+#pragma unroll
+        for (int s = 0; s < NA; s++) {
+#pragma unroll
+            for (int j = 0; j < BI; j++)
+                if (s < NB && s < nk) load_now(w + (size_t)s * 128, offb[j], lds_b + s * BSZ, j);
+#pragma unroll
+            for (int j = 0; j < AI; j++)
+                if ((s < NA - 1 || j < early_a) && s < nk) load_now(a + (size_t)s * 128, offa[j], lds_a + s * ASZ, j);
+        }
+        const int fr = lane & 15, fg = lane >> 4;
+        int at[KS];
+#pragma unroll
+        for (int s = 0; s < KS; s++) at[s] = fr * 128 + (((s * 4 + fg) ^ rot(fr)) * 16);
+        const int8_t* const read_a = smem + row_of_wave() * 128;
+        const int8_t* const read_b = smem + NA * ASZ + col_of_wave() * 128;
+        Frag fa[2][MI], fb[2][NI];
+        auto read = [&](unsigned sa, unsigned sb, int ks, int set, int q) __attribute__((always_inline)) {       // q-th of the reads of a k-step
+            if (q == 0) fa[set][0] = *reinterpret_cast<const Frag*>(read_a + sa + at[ks]);
+            else if (q <= NI) fb[set][q - 1] = *reinterpret_cast<const Frag*>(read_b + sb + at[ks] + (q - 1) * 2048);
+            else fa[set][q - NI] = *reinterpret_cast<const Frag*>(read_a + sa + at[ks] + (q - NI) * 2048);
+        };
+        auto wait_stage = [&](int younger) __attribute__((always_inline)) {
+            if (younger >= NB) wait_vmcnt<in_flight(NB)>();
+            else if (NB > 4 && younger == 4) wait_vmcnt<in_flight(4)>();
+            else if (NB > 3 && younger == 3) wait_vmcnt<in_flight(3)>();
+            else if (NB > 2 && younger == 2) wait_vmcnt<in_flight(2)>();
+            else if (younger == 1) wait_vmcnt<in_flight(1)>();
+            else wait_vmcnt<0>();
+        };
+        static_assert(NB <= 6, "the wait tells up to four younger stages apart");
+        // Stage 0 is in when what was asked for behind it is out: all of the stages 1 .. NA - 1 that there are, as far as they are asked for.
+        {
+            constexpr int full = (NB - 1) * BI + (NA - 2) * AI + early_a;
+            if (nk >= NA) wait_vmcnt<(full < 63 ? full : 63)>();
+            else wait_vmcnt<0>();
+        }
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < NR; q++) read(0, 0, 0, 0, q);
+        // ring slots of the last, this and the next stage; the last one's are refilled
+        unsigned a0 = (NA - 1) * ASZ, a1 = 0, a2 = ASZ, b0 = (NB - 1) * BSZ, b1 = 0, b2 = BSZ;
+        const int8_t* pa = a + (size_t)(NA - 1) * 128;           // stage kt - 1 + NA
+        const int8_t* pb = w + (size_t)(NB - 1) * 128;           // stage kt - 1 + NB
+        auto stage = [&](int left, auto next, auto full) __attribute__((always_inline)) {   // left: stages behind this one
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                constexpr bool kNext = decltype(next)::value, kFull = decltype(full)::value;
+                const bool last = s == KS - 1;
+                if (last && kNext) {
+                    if constexpr (kFull) wait_vmcnt<in_flight(NB)>(); else wait_stage(left - 1);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int x = 0; x < NM; x++) {
+                    Op::mma(fb[s & 1][x % NI], fa[s & 1][x / NI], acc[x / NI][x % NI]);
+                    // operands of the next k-step, evenly over the first half of the matrix instructions
+                    constexpr int RS = NM / 2 / NR > 0 ? NM / 2 / NR : 1;
+                    if (x % RS == 0 && x / RS < NR) {
+                        if (!last) read(a1, b1, s + 1, (s + 1) & 1, x / RS);
+                        else if (kNext) read(a2, b2, 0, (s + 1) & 1, x / RS);
+                    }
+                    if constexpr (NR > NM) {                     // more reads than matrix instructions: the rest behind the last one
+                        if (x == NM - 1) {
+#pragma unroll
+                            for (int q = NM; q < NR; q++) {
+                                if (!last) read(a1, b1, s + 1, (s + 1) & 1, q);
+                                else if (kNext) read(a2, b2, 0, (s + 1) & 1, q);
+                            }
+                        }
+                    }
+                    // place behind the barrier of this stage (last k-step) or of the one before
+                    const int p = last ? x : (s + 1) * NM + x;
+                    const unsigned sa = last ? a1 : a0, sb = last ? b1 : b0;
+                    const bool there_a = kFull || left + (last ? 0 : 1) >= NA, there_b = kFull || left + (last ? 0 : 1) >= NB;
+#pragma unroll
+                    for (int j = 0; j < BI; j++) {
+                        if (p == slot_b(j) + 1 && there_b) load(pb + (last ? 128 : 0), offb[j]);
+                        if (p == slot_b(j) && there_b) aim(lds_b + sb, j);
+                    }
+#pragma unroll
+                    for (int j = 0; j < AI; j++) {
+                        if (p == slot_a(j) + 1 && there_a) load(pa + (last ? 128 : 0), offa[j]);
+                        if (p == slot_a(j) && there_a) aim(lds_a + sa, j);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            pa += 128; pb += 128;
+            a0 = a1; a1 = a2; a2 = a2 == (NA - 1) * ASZ ? 0 : a2 + ASZ;
+            b0 = b1; b1 = b2; b2 = b2 == (NB - 1) * BSZ ? 0 : b2 + BSZ;
+        };
+        int left = nk - 1;
+        for (; left >= NA; left--) stage(left, std::true_type(), std::true_type());
+        for (; left >= 1; left--) stage(left, std::true_type(), std::false_type());
+        stage(0, std::false_type(), std::false_type());
+    }
+};
+
+}  // namespace fx

@@ -611,6 +611,9 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
                               int dtype, void* stream);
 /* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
 int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
+/* A bfloat16 product whose tile has 256 columns shares its rows out anew: the rows that a workgroup takes (128 to 256; of any other product
+ * those of its tile), negative: an error code.  parts: 1, or those that k is shared out in.  Needs no GPU. */
+int flexllm_linear_float_gemm_rows(int m, int k, int n, int dtype, int parts);
 /* Parts (at most `most`) that k of such a product is shared out in where its reader adds the parts' sums up; negative: an error code.
  * Needs no GPU. */
 int flexllm_linear_float_gemm_parts(int m, int k, int n, int dtype, int most);
