@@ -10,6 +10,7 @@
 #pragma once
 #include "attn_decode_kernels.h"
 #include "common.h"
+#include "gemm_walk.h"
 #include <atomic>
 #include <type_traits>
 
@@ -221,6 +222,56 @@ struct QkvEpiArgs {
     const float *b_x = nullptr, *w_sum = nullptr;
 };
 
+// q/k/v from the dequantised tile [BM tokens][BN channels], pitch BN + 1: RoPE, static quantisation, the stores into q8 and the caches.
+template <int BM, int BN, int NW>
+__device__ __forceinline__ void qkv_tile_out(const float* tile, int row0, int col0, int m, int n, const QkvEpiArgs& qa) {
+    constexpr int TP = BN + 1;
+    const int t = threadIdx.x;
+    // four waves at a time take a block of 64 tokens x one head
+    constexpr int HM = BM / 64, HN = BN / 64, TEAMS = NW / 4;
+    const int sel = t & 63, part = (t >> 6) & 3;
+    for (int blk = t >> 8; blk < HM * HN; blk += TEAMS) {
+        const int tr = (blk % HM) * 64, tc = (blk / HM) * 64, head = (col0 + tc) / kHd;      // 0..q_heads-1 q, then k heads, then v heads
+        if (col0 + tc >= n) break;
+        const float* sub = tile + tr * TP + tc;
+        if (head < qa.q_heads + qa.kv_heads) {
+            // RoPE + static quantisation: thread = (token sel, pairs 8*part .. 8*part+7)
+            const int row = row0 + tr + sel, pos = qa.pos0 + row;
+            if (row < m) {
+                const bool is_q = head < qa.q_heads;
+                const int hk = is_q ? head : head - qa.q_heads;
+                const float div = is_q ? 8.0f * qa.q_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
+                const float* sn = qa.sin_t + (size_t)pos * 32 + part * 8;
+                const float* cs = qa.cos_t + (size_t)pos * 32 + part * 8;
+                uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float t0 = sub[sel * TP + part * 8 + j], t1 = sub[sel * TP + part * 8 + j + 32];
+                    const float o0 = t0 * cs[j] - t1 * sn[j];
+                    const float o1 = t0 * sn[j] + t1 * cs[j];
+                    lo[j >> 2] |= (uint32_t)(static_q8(o0, div) & 0xff) << (8 * (j & 3));
+                    hi[j >> 2] |= (uint32_t)(static_q8(o1, div) & 0xff) << (8 * (j & 3));
+                }
+                int8_t* dst = is_q ? qa.q8 + ((size_t)row * qa.q_heads + hk) * kHd : qa.kc + k_index(hk, pos, qa.max_pos);
+                *reinterpret_cast<uint2*>(dst + part * 8) = make_uint2(lo[0], lo[1]);
+                *reinterpret_cast<uint2*>(dst + part * 8 + 32) = make_uint2(hi[0], hi[1]);
+            }
+        } else {
+            // V: thread = (channel sel, 16 consecutive positions 16*part ..): one 16-byte run of the transposed cache block
+            const int hv = head - qa.q_heads - qa.kv_heads;
+            const int rbase = row0 + tr + part * 16;
+            if (rbase < m) {                               // m is a multiple of 32 (checked by the launcher)
+                const float div = 1.0f * qa.v_s[hv];
+                uint32_t wv4[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    wv4[i >> 2] |= (uint32_t)(static_q8(sub[(part * 16 + i) * TP + sel], div) & 0xff) << (8 * (i & 3));
+                *reinterpret_cast<uint4*>(qa.vc + v_index(hv, qa.pos0 + rbase, sel, qa.max_pos)) = make_uint4(wv4[0], wv4[1], wv4[2], wv4[3]);
+            }
+        }
+    }
+}
+
 __device__ __forceinline__ void gemm_dma_issue(const int8_t* base, unsigned voff, unsigned lds_dst) {
     unsigned saved_m0;
     asm volatile("s_mov_b32 %0, m0\n\t"
@@ -242,7 +293,7 @@ __device__ __forceinline__ void gemm_wait_vmcnt() {            // s_waitcnt vmcn
 // for again one stage later: measured with the loads alone (no math, 128 x 256 tiles at K = 2048), the chip moves
 // 23 TB/s into LDS in whole 128-byte lines and 14.5 TB/s in halves.  With 128-byte rows the slot rotation is
 // s ^ ((r >> 1) & 7): two rows span the 64 banks, so 16 consecutive rows of one chunk fall on 16 different bank groups.
-// NW = waves per workgroup, 4 (2x2 wave grid) or 8 (2x4): eight waves let a 256x256 tile keep two waves per SIMD.
+// NW = waves per workgroup, 4 (2x2 wave grid) or 8 (2x4).
 template <int BM, int BN, int EPI, int kDmaStages, int WPE, int BKB, int NW>   // at most 4 stages (the wait below distinguishes up to 2 younger ones)
 __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ w,
                                                           int32_t* __restrict__ c_out, const float* __restrict__ s_x,
@@ -401,49 +452,7 @@ __global__ __launch_bounds__(NW * 64, WPE) void gemm_i8_dma_kernel(const int8_t*
                 }
         }
         __syncthreads();
-        // four waves at a time take a block of 64 tokens x one head
-        constexpr int HM = BM / 64, HN = BN / 64, TEAMS = NW / 4;
-        const int sel = t & 63, part = (t >> 6) & 3;
-        for (int blk = t >> 8; blk < HM * HN; blk += TEAMS) {
-            const int tr = (blk % HM) * 64, tc = (blk / HM) * 64, head = (col0 + tc) / kHd;      // 0..q_heads-1 q, then k heads, then v heads
-            if (col0 + tc >= n) break;
-            const float* sub = tile + tr * TP + tc;
-            if (head < qa.q_heads + qa.kv_heads) {
-                // RoPE + static quantisation: thread = (token sel, pairs 8*part .. 8*part+7)
-                const int row = row0 + tr + sel, pos = qa.pos0 + row;
-                if (row < m) {
-                    const bool is_q = head < qa.q_heads;
-                    const int hk = is_q ? head : head - qa.q_heads;
-                    const float div = is_q ? 8.0f * qa.q_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
-                    const float* sn = qa.sin_t + (size_t)pos * 32 + part * 8;
-                    const float* cs = qa.cos_t + (size_t)pos * 32 + part * 8;
-                    uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};
-#pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const float t0 = sub[sel * TP + part * 8 + j], t1 = sub[sel * TP + part * 8 + j + 32];
-                        const float o0 = t0 * cs[j] - t1 * sn[j];
-                        const float o1 = t0 * sn[j] + t1 * cs[j];
-                        lo[j >> 2] |= (uint32_t)(static_q8(o0, div) & 0xff) << (8 * (j & 3));
-                        hi[j >> 2] |= (uint32_t)(static_q8(o1, div) & 0xff) << (8 * (j & 3));
-                    }
-                    int8_t* dst = is_q ? qa.q8 + ((size_t)row * qa.q_heads + hk) * kHd : qa.kc + k_index(hk, pos, qa.max_pos);
-                    *reinterpret_cast<uint2*>(dst + part * 8) = make_uint2(lo[0], lo[1]);
-                    *reinterpret_cast<uint2*>(dst + part * 8 + 32) = make_uint2(hi[0], hi[1]);
-                }
-            } else {
-                // V: thread = (channel sel, 16 consecutive positions 16*part ..): one 16-byte run of the transposed cache block
-                const int hv = head - qa.q_heads - qa.kv_heads;
-                const int rbase = row0 + tr + part * 16;
-                if (rbase < m) {                               // m is a multiple of 32 (checked by the launcher)
-                    const float div = 1.0f * qa.v_s[hv];
-                    uint32_t wv4[4] = {0, 0, 0, 0};
-#pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        wv4[i >> 2] |= (uint32_t)(static_q8(sub[(part * 16 + i) * TP + sel], div) & 0xff) << (8 * (i & 3));
-                    *reinterpret_cast<uint4*>(qa.vc + v_index(hv, qa.pos0 + rbase, sel, qa.max_pos)) = make_uint4(wv4[0], wv4[1], wv4[2], wv4[3]);
-                }
-            }
-        }
+        qkv_tile_out<BM, BN, NW>(tile, row0, col0, m, n, qa);
         return;
     }
     constexpr bool kAsym = EPI == kDmaDequantAsym || EPI == kDmaSwigluAsym;      // + zero point x row sum of the dequantised weights
@@ -565,6 +574,214 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
     return FLEXLLM_OK;
 }
 
+// static_q8 (attn_decode_kernels.h) of four values that share a divisor, without a division each, packed.  quant_vector rounds as the quotient does up to
+// 255; what is beyond is clamped either way.
+__device__ __forceinline__ uint32_t static_q8x4(const float (&v)[4], float div) {
+    int n[4];
+    quant_vector<4>(v, div, n);
+#pragma unroll
+    for (int e = 0; e < 4; e++) n[e] = max(min(n[e], 127), -128);
+    return pack4_i8(n[0], n[1], n[2], n[3]);
+}
+
+// Tiles of 256 columns, 128-byte rows: the walk of gemm_walk.h.  Before (gemm_i8_dma_kernel, eight waves of 32 x 32 instructions) and now, us:
+// 2528 x 16384 x 2048 (m, n, k) 110 and 101, 1531 x 16384 x 2048 69 and 64, 2528 x 2048 x 8192 58.2 and 53.8, 4096 x 2048 x 8192 74 and 62,
+// 1024 x 16384 x 2048 with the gated unit 43.8 and 38.  A product of a short k is bound by what stands around the walk: of
+// 2528 x 16384 x 2048's 100 us three rounds take 19 us of walk each (16 stages of 0.8 us), the rest are the first stages' trips and the
+// outputs.  Smaller tiles stay on the other kernel, whose eight waves hide more of each other's trips (1024 x 2048 x 8192 on
+// 64 x 128 28.5 us, 28.6 here; on 128 x 128 34.6 and 38.3).
+template <int MI> using WideI8 = GemmWalk<int8_t, 2, MI, 8, MI == 4 ? 4 : 3, MI == 4 ? 3 : 2>;      // 32 * MI rows
+
+template <int EPI, int MI>
+__global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int32_t* __restrict__ c_out,
+                                                                                 const float* __restrict__ s_x, const float* __restrict__ w_s, const float* __restrict__ residual,
+                                                                                 float* __restrict__ y, int m, int k, int n, int tiles_m, int tiles_n, QkvEpiArgs qa) {
+    using W = WideI8<MI>;
+    constexpr int NI = 8;
+    extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
+    int tm, tn;
+    gemm_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    const int row0 = tm * W::BM, col0 = tn * W::BN;
+    unsigned offa[W::AI], offb[W::BI];
+#pragma unroll
+    for (int j = 0; j < W::AI; j++) {
+        const int r = W::load_row_a(j);
+        offa[j] = (unsigned)min(row0 + r, m - 1) * (unsigned)k + W::load_byte(r);
+    }
+#pragma unroll
+    for (int j = 0; j < W::BI; j++) {
+        const int r = W::load_row_b(j);
+        offb[j] = (unsigned)min(col0 + r, n - 1) * (unsigned)k + W::load_byte(r);
+    }
+    i32x4 acc[MI][NI];
+    W::run(a, w, offa, offb, k / 128, gemm_smem, acc);
+    const int lane = threadIdx.x & 63, fr = lane & 15, fg = lane >> 4;
+    const int wr = W::row_of_wave(), wc = W::col_of_wave();
+    if constexpr (EPI == kDmaQkv) {
+        // A wave has 64 tokens x two heads.  Channels c and c + 32 of a token are in blocks j and j + 2 of one lane, so RoPE stays in registers, and the
+        // quantised head of a token leaves in 16-byte pieces.
+        static_assert(MI == 4 && NI == 8, "64 tokens x two heads per wave");
+        constexpr int TP = 64 + 16;                            // V only: a head's bytes [channel][token], turned through LDS
+        int8_t* const turn = gemm_smem + W::wave() * (64 * TP);
+        __syncthreads();                                       // all waves are done with the stage buffers
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            const int c0 = col0 + wc + hh * 64, head = c0 / kHd;      // 0..q_heads-1 q, then k heads, then v heads
+            if (c0 >= n) break;
+            const bool asym = qa.b_x != nullptr;               // asymmetric activations: + zero point x row sum of the dequantised weights
+            f32x4 ws[4], wq[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                ws[j] = *reinterpret_cast<const f32x4*>(w_s + c0 + j * 16 + fg * 4);
+                wq[j] = asym ? *reinterpret_cast<const f32x4*>(qa.w_sum + c0 + j * 16 + fg * 4) : f32x4{};
+            }
+            const bool is_q = head < qa.q_heads, is_v = head >= qa.q_heads + qa.kv_heads;
+            const int hk = is_q ? head : is_v ? head - qa.q_heads - qa.kv_heads : head - qa.q_heads;
+            const float div = is_q ? 8.0f * qa.q_s[hk] : is_v ? 1.0f * qa.v_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const int row = row0 + wr + i * 16 + fr, r = min(row, m - 1), pos = qa.pos0 + r;
+                const float sx = s_x[r], bx = asym ? qa.b_x[r] : 0.0f;
+                f32x4 v[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[j][e] = (float)acc[i][hh * 4 + j][e] * sx * ws[j][e];
+                    if (asym) v[j] = v[j] + bx * wq[j];
+                }
+                if (is_v) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float x[4] = {v[j][0], v[j][1], v[j][2], v[j][3]};
+                        const uint32_t q = static_q8x4(x, div);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) turn[(j * 16 + fg * 4 + e) * TP + i * 16 + fr] = (int8_t)(q >> (8 * e));
+                    }
+                    continue;
+                }
+                uint32_t o[4][1];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const f32x4 sn = *reinterpret_cast<const f32x4*>(qa.sin_t + (size_t)pos * 32 + j * 16 + fg * 4);
+                    const f32x4 cs = *reinterpret_cast<const f32x4*>(qa.cos_t + (size_t)pos * 32 + j * 16 + fg * 4);
+                    float lo[4], hi[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        lo[e] = v[j][e] * cs[e] - v[j + 2][e] * sn[e];
+                        hi[e] = v[j][e] * sn[e] + v[j + 2][e] * cs[e];
+                    }
+                    o[j][0] = static_q8x4(lo, div);
+                    o[j + 2][0] = static_q8x4(hi, div);
+                }
+                join_blocks<1>(o);
+                int8_t* dst = is_q ? qa.q8 + ((size_t)row * qa.q_heads + hk) * kHd : qa.kc + k_index(hk, pos, qa.max_pos);
+                if (row < m) *reinterpret_cast<uint4*>(dst + fg * 16) = make_uint4(o[0][0], o[1][0], o[2][0], o[3][0]);
+            }
+            if (is_v) {
+                // the patch is private to the wave, whose LDS operations complete in order
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                // lane = channel; 16 consecutive positions are one run of the transposed cache block
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const int row = row0 + wr + p * 16;            // m is a multiple of 32 (checked by the launcher)
+                    const uint4 run = *reinterpret_cast<const uint4*>(turn + lane * TP + p * 16);
+                    if (row < m) *reinterpret_cast<uint4*>(qa.vc + v_index(hk, qa.pos0 + row, lane, qa.max_pos)) = run;
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            }
+        }
+        return;
+    } else {
+        constexpr bool kAsym = EPI == kDmaDequantAsym || EPI == kDmaSwigluAsym, kUnit = EPI == kDmaSwiglu || EPI == kDmaSwigluAsym;
+        constexpr int J = kUnit ? 2 : 1;                       // blocks of 16 columns whose outputs leave together, 64 bytes of a row
+        const int rows = m - row0 - wr, ld = kUnit ? n >> 1 : n;
+        const TileRows out(EPI == kDmaRaw ? reinterpret_cast<float*>(c_out) + (size_t)(row0 + wr) * ld : y + (size_t)(row0 + wr) * ld, rows, ld * 4);
+        const bool has_res = !kUnit && EPI != kDmaRaw && residual != nullptr;
+        const TileRows res(const_cast<float*>(has_res ? residual + (size_t)(row0 + wr) * n : y), has_res ? rows : 0, n * 4);
+        float sx[MI], bx[MI];
+        if constexpr (EPI != kDmaRaw) {
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const int row = min(row0 + wr + i * 16 + fr, m - 1);
+                sx[i] = s_x[row];
+                if constexpr (kAsym) bx[i] = qa.b_x[row];
+            }
+        }
+        // byte of the lane's 16 in the tile's first row; they lie inside or behind the row as a whole
+        auto place = [&](int j0) __attribute__((always_inline)) {
+            const int col = col0 + wc + j0 * 16 + (kUnit ? fg * 8 : fg * 4);
+            return col < n ? (kUnit ? col * 2 : col * 4) + fr * ld * 4 : kNowhere;
+        };
+        // residuals of the next columns are asked for ahead of the stores of these: a wait for loads is one for the stores before them, too
+        f32x4 rs[2][MI];
+        auto residuals = [&](int j0) __attribute__((always_inline)) {
+            const int at = place(j0);
+#pragma unroll
+            for (int i = 0; i < MI; i++) rs[(j0 / J) & 1][i] = res.get(at == kNowhere ? kNowhere : at + i * 16 * ld * 4);
+        };
+        if (has_res) residuals(0);
+#pragma unroll
+        for (int j0 = 0; j0 < NI; j0 += J) {
+            f32x4 ws[J], wq[J];
+            const int at = place(j0);
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const int c = min(col0 + wc + (j0 + j) * 16 + fg * 4, n - 4);
+                if constexpr (EPI != kDmaRaw) ws[j] = *reinterpret_cast<const f32x4*>(w_s + c);
+                if constexpr (kAsym) wq[j] = *reinterpret_cast<const f32x4*>(qa.w_sum + c);
+            }
+            if (has_res && j0 + J < NI) residuals(j0 + J);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                uint32_t o[J][4 / J];
+#pragma unroll
+                for (int j = 0; j < J; j++) {
+                    const i32x4 q = acc[i][j0 + j];
+                    if constexpr (EPI == kDmaRaw) {
+                        __builtin_memcpy(o[j], &q, 16);
+                    } else {
+                        f32x4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[e] = (float)q[e] * sx[i] * ws[j][e];
+                        if constexpr (kAsym) v = v + bx[i] * wq[j];
+                        if constexpr (kUnit) {
+                            // weight rows are interleaved (2c gate, 2c+1 up)
+                            const float h[2] = {v[1] * silu_f(v[0]), v[3] * silu_f(v[2])};
+                            __builtin_memcpy(o[j], h, 8);
+                        } else {
+                            if (has_res) v = v + rs[(j0 / J) & 1][i];
+                            __builtin_memcpy(o[j], &v, 16);
+                        }
+                    }
+                }
+                join_blocks<4 / J>(o);
+                out.put(&o[0][0], at == kNowhere ? kNowhere : at + i * 16 * ld * 4);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+}
+
+template <int EPI, int MI>
+inline int launch_gemm_walk(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s, const float* residual, float* y, int m, int k, int n,
+                            hipStream_t st, QkvEpiArgs qa) {
+    using W = WideI8<MI>;
+    static std::atomic<bool> opted_in{false};
+    if (!opted_in.load(std::memory_order_acquire)) {
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_i8_walk_kernel<EPI, MI>), hipFuncAttributeMaxDynamicSharedMemorySize, W::kLds));
+        opted_in.store(true, std::memory_order_release);
+    }
+    const int tm = (m + W::BM - 1) / W::BM, tn = (n + W::BN - 1) / W::BN;
+    gemm_i8_walk_kernel<EPI, MI><<<tm * tn, 256, W::kLds, st>>>(a, w, c, s_x, w_s, residual, y, m, k, n, tm, tn, qa);
+    FX_LAUNCH_CHECK();
+    return FLEXLLM_OK;
+}
+
 // The direct-load kernel runs on the tile whose rounds over the 256 CUs (per_cu at a time) cost least, in about 0.01 us: per stage, and
 // once per round for what lies around them (first loads, epilogue).  Rows of a stage are whole 128-byte lines where k
 // allows, 64 bytes where it is a multiple of 64 alone.
@@ -579,8 +796,9 @@ inline int launch_gemm_dma(const int8_t* a, const int8_t* w, int32_t* c, const f
 // two of the one with four stages.  64 x 64 with three stages fits three times: 1536 x 2048 x 2048, 768 tiles, 14.4 us in one
 // round of it, 15.8 on 128 x 128; 393 x 9536 x 128 7.5 us, 9.5 on 128 x 128 twice per CU.  The q/k/v
 // epilogue turns whole heads, for which small tiles are no better: 1024 x 3072 x 2048 stays on 128 x 128.
-// The costs are the ones that lose least over 384 sizes (128-byte rows) and 136 sizes (64-byte rows) of 1 to 4096 rows and 64 to 14336 k: their
-// tiles are 0.6 and 0.2 % from the best ones on average.
+// The costs are the ones that lost least over 384 sizes (128-byte rows) and 136 sizes (64-byte rows) of 1 to 4096 rows and 64 to 14336 k with
+// every tile on this kernel (0.6 and 0.2 % from the best ones on average); with the wide ones on the walk it is 3.4 % over 44 sizes, most of it
+// at k below 1152.
 struct GemmI8Tile { int bm, bn, stage, round, per_cu; };
 constexpr GemmI8Tile kGemmI8Tiles[2][7] = {
     {{256, 256, 126, 2000, 1}, {128, 256, 81, 1140, 1}, {128, 128, 74, 400, 1}, {64, 128, 60, 410, 1}, {64, 64, 27, 450, 1}, {64, 64, 77, 350, 3}, {128, 128, 112, 950, 2}},
@@ -598,6 +816,20 @@ inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
     return pick;
 }
 
+// Products on 128-byte rows whose tile has 256 columns share their rows out anew, as bfloat16 ones do (gemm_float.hip); costs in 0.01 us.
+struct GemmI8Rows { int rows, stage, round; };
+constexpr GemmI8Rows kGemmI8Rows[] = {{256, 110, 1500}, {224, 99, 1350}, {192, 88, 1200}, {160, 80, 1050}, {128, 70, 900}};
+inline int gemm_i8_rows(int m, int k, int n, bool qkv) {
+    if (qkv) return 128;                                       // blocks of 64 tokens
+    long best = 0;
+    int rows = 0;
+    for (const GemmI8Rows& t : kGemmI8Rows) {
+        const long tiles = (long)((m + t.rows - 1) / t.rows) * ((n + 255) / 256), cost = (tiles + 255) / 256 * (t.stage * (k / 128) + t.round);
+        if (!rows || cost < best) { best = cost; rows = t.rows; }
+    }
+    return rows;
+}
+
 template <int EPI>
 inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const float* s_x, const float* w_s, const float* residual, float* y,
                              int m, int k, int n, hipStream_t st, QkvEpiArgs qa = QkvEpiArgs()) {
@@ -611,13 +843,27 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
         if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 64);
         return FX_GEMM_TILE(64, 64, 4, 2, 64);
     }
+    // the gated unit's 16 bytes of output are eight columns
+    // (a head's 64 bytes leave in 16-byte pieces, too, and the scales and tables are read in such)
+    const auto bits = [](auto... p) { return (reinterpret_cast<uintptr_t>(p) | ...); };
+    if (EPI == kDmaQkv && pick < 2 && (bits(qa.q8, qa.kc, qa.vc, qa.sin_t, qa.cos_t, w_s, qa.w_sum) & 15)) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
+    const bool wide = rows_fit(n, 4) && ((EPI != kDmaSwiglu && EPI != kDmaSwigluAsym) || (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0));
+    if (pick < 2 && wide) {
+#define FX_GEMM_ROWS(MI) launch_gemm_walk<EPI, MI>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa)
+        if constexpr (EPI != kDmaQkv) switch (gemm_i8_rows(m, k, n, false)) {
+            case 256: return FX_GEMM_ROWS(8);
+            case 224: return FX_GEMM_ROWS(7);
+            case 192: return FX_GEMM_ROWS(6);
+            case 160: return FX_GEMM_ROWS(5);
+        }
+        return FX_GEMM_ROWS(4);
+#undef FX_GEMM_ROWS
+    }
     if constexpr (EPI != kDmaQkv) {
-        if (pick == 0) return FX_GEMM_TILE(256, 256, 2, 2, 128, 8);
         if (pick == 5) return FX_GEMM_TILE(64, 64, 3, 3, 128);
         if (pick == 6) return FX_GEMM_TILE(128, 128, 2, 2, 128);
     }
-    if (pick == 1) return FX_GEMM_TILE(128, 256, 3, 2, 128, 8);
-    if (pick == 2) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
+    if (pick <= 2) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
     if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 128, 8);
     return FX_GEMM_TILE(64, 64, 4, 2, 128);
 #undef FX_GEMM_TILE

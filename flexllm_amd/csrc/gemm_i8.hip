@@ -57,4 +57,10 @@ int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* co
     return FLEXLLM_OK;
 }
 
+int flexllm_linear_i8_gemm_rows(int m, int k, int n, int qkv) {
+    FX_REQUIRE(m > 0 && n > 0 && k > 0 && k % 64 == 0, "linear_i8_gemm_rows: m=%d k=%d n=%d", m, k, n);
+    const GemmI8Tile& t = kGemmI8Tiles[k % 128 != 0][gemm_i8_tile(m, k, n, qkv != 0)];
+    return k % 128 == 0 && t.bn == 256 ? gemm_i8_rows(m, k, n, qkv != 0) : t.bm;
+}
+
 }  // extern "C"

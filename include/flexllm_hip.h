@@ -141,6 +141,9 @@ int flexllm_linear_i8_gemm(const int8_t* a, const int8_t* w, int32_t* acc, int m
 /* Rows and columns of the tile that an int8 product (qkv: the fused q/k/v projection) of these sizes runs on, and how many of them
  * a CU holds at a time.  Needs no GPU. */
 int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols, int* per_cu);
+/* A product whose tile has 256 columns shares its rows out anew: the rows that a workgroup takes (128 to 256; of any other product those of
+ * its tile), negative: an error code.  Needs no GPU. */
+int flexllm_linear_i8_gemm_rows(int m, int k, int n, int qkv);
 /* The same exact product with UNSIGNED 8-bit activations (0..255), the reference's is_uint_input instantiation of its
  * int8 arrays (Modules/MHA.h:339-344, :854-859 with is_uint_input = true; Modules/PE.h:526-583, is_uint_A): used for
  * P.V with the uint8 softmax probabilities as a stand-alone stage.  a [m][k] uint8, w [n][k] int8, acc [m][n] int32;
@@ -611,8 +614,7 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
                               int dtype, void* stream);
 /* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
 int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
-/* A bfloat16 product whose tile has 256 columns shares its rows out anew: the rows that a workgroup takes (128 to 256; of any other product
- * those of its tile), negative: an error code.  parts: 1, or those that k is shared out in.  Needs no GPU. */
+/* The rows that a workgroup takes, as flexllm_linear_i8_gemm_rows; parts: 1, or those that k is shared out in.  Needs no GPU. */
 int flexllm_linear_float_gemm_rows(int m, int k, int n, int dtype, int parts);
 /* Parts (at most `most`) that k of such a product is shared out in where its reader adds the parts' sums up; negative: an error code.
  * Needs no GPU. */

@@ -7,11 +7,15 @@ def test_every_number_of_rows_is_under_test():
     for rows, (m, n) in gpu.FLOAT.items():
         for k in gpu.FLOAT_K:
             assert lib().flexllm_linear_float_gemm_rows(m, k, n, 0, 1) == rows
+    for (rows, k), (m, n) in gpu.INT.items():
+        assert lib().flexllm_linear_i8_gemm_rows(m, k, n, 0) == rows
 
 
 def test_rows_that_measured_best():
     """Sizes at which another number of rows was 5 to 40 % slower; few rows stay on their tile."""
     from flexllm_amd import lib
-    f = lambda *s: lib().flexllm_linear_float_gemm_rows(*s, 0, 1)  # noqa: E731
+    f, i = (lambda *s: lib().flexllm_linear_float_gemm_rows(*s, 0, 1)), (lambda *s: lib().flexllm_linear_i8_gemm_rows(*s, 0))
     assert f(777, 4096, 28672) == f(2528, 2048, 16384) == 224 and f(1531, 2048, 16384) == 192 and f(2596, 2560, 3712) == 160
     assert f(1024, 2048, 16384) == 256 and f(2528, 8192, 2048) == 128 and f(777, 14336, 4096) == 128 and f(1024, 2048, 2048) == 64
+    assert i(777, 4096, 28672) == 224 and i(1531, 2048, 16384) == 192 and i(1024, 2048, 16384) == 256
+    assert i(2528, 8192, 2048) == lib().flexllm_linear_i8_gemm_rows(2528, 2048, 3072, 1) == 128
