@@ -92,6 +92,14 @@ struct TileRows {
     }
 };
 
+// The workgroup's barrier alone: what has to be waited for is waited for explicitly ahead of it.  No memory access moves across it.
+__device__ __forceinline__ void barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
 template <typename ET, int WM, int MI, int NI, int NA, int NB>
 struct GemmWalk {
     using Op = MatrixOp<ET>;
@@ -205,8 +213,7 @@ struct GemmWalk {
             if (nk >= NA) wait_vmcnt<(full < 63 ? full : 63)>();
             else wait_vmcnt<0>();
         }
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        barrier();
 #pragma unroll
         for (int q = 0; q < NR; q++) read(0, 0, 0, 0, q);
         // ring slots of the last, this and the next stage; the last one's are refilled
@@ -221,8 +228,7 @@ struct GemmWalk {
                 if (last && kNext) {
                     if constexpr (kFull) wait_vmcnt<in_flight(NB)>(); else wait_stage(left - 1);
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    __builtin_amdgcn_s_barrier();
-                    __builtin_amdgcn_sched_barrier(0);
+                    barrier();
                 }
 #pragma unroll
                 for (int x = 0; x < NM; x++) {

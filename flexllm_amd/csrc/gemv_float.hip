@@ -4,6 +4,7 @@
 // The first two groups are requested before the prologue (residual, norms) runs, so that its latency lies under the weight
 // stream, and two groups stay in flight after that.  The R sums are reduced together (multi_sum_step).
 #include "float_ops.h"
+#include "gemm_walk.h"
 #include "route.h"
 #include <atomic>
 
@@ -369,129 +370,210 @@ static int gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
 }
 
 // bfloat16 weights on the matrix cores: a float32 vector is the sum of three bfloat16 parts to 24 bits and their products with the
-// weights are exact in float32, so three instructions per 16 rows x 32 k give what the float32 products give (vector
+// weights are exact in float32, so two instructions per 16 rows x 32 k (at most 8 tokens: two parts lie side by side) give what the float32 products give (vector
 // instructions: 16384 x 2048 for 5 tokens 24 us, the weights' stream is 10).  A workgroup of eight waves walks tiles of 16 rows; the
-// waves share its stretch of k (KW steps of 32 each), whose vectors lie in LDS as [part][token][stretch, padded by 16 bytes: the
-// tokens of an operand read are then on different banks], and meet through LDS per tile, two tiles' weights in flight.
-constexpr int kMfmaTokens = 16, kMfmaWaves = 8;
-constexpr float kBf16Max = 3.38953139e38f;
-constexpr int gemv_mfma_row(int stretch) { return stretch * 2 + 16; }      // bytes of a token's part
-template <int KW>
-__global__ __launch_bounds__(kMfmaWaves * 64) void gemv_mfma_kernel(GemvArgs g, int tokens, int group) {
-    constexpr int NT = kMfmaWaves * 64, STRETCH = KW * kMfmaWaves * 32, ROW = gemv_mfma_row(STRETCH);
-    extern __shared__ __attribute__((aligned(16))) int8_t xp[];    // [3][group][ROW]
+// waves share a unit of UK of k, of which a tile has UNITS, and meet through LDS per tile.
+// What bounds it: the weights' stream, and that hangs on how it is asked for.  The operand of the instruction is 64 bytes of each of 16 rows; asked
+// for like that, 67 MB take 17.5 us without any arithmetic, as 1 KiB of one row per request 11.5.  So the weights go to LDS in
+// such requests (16-byte chunk c of row r at place c ^ r, for reads without conflicts), two units of 64 KiB of them in flight, and a
+// unit's place is free for the next but one as soon as its operands are in registers.  The vectors' parts stay in registers, each wave's
+// own stretch of k.
+// Before (operands straight from memory) and now, 5 tokens, us: 16384 x 2048 21.5 and 14.4, 2048 x 8192 13.2 and 9.3, 28672 x 4096 49.8 and
+// 39.6 (8 tokens 81 and 44), 4096 x 14336 28.0 and 21.0, 2560 x 2048 6.7 and 6.6, 2048 x 2048 4.9 and 5.2.  What the last two are made of: 2 us
+// until the vectors are in and taken apart, 1.5 more until the first unit is, 1 for the sums' way through LDS.
+constexpr int kMfmaTokens = 8, kMfmaWaves = 8;
+template <int UK, int UNITS>
+__global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs g, int tokens, int group) {
+    constexpr int STRETCH = UK * UNITS, SW = UK / kMfmaWaves / 32, SL = UK / kMfmaWaves;      // matrix k-steps and k of a wave in a unit
+    constexpr int UB = UK * 2, SLOT = 16 * UB, SLOTS = 128 * 1024 / SLOT, PER = SLOT / 1024 / kMfmaWaves;   // PER: requests of a wave per unit
+    static_assert(kMfmaTokens * SL * 4 <= PER * 1024, "a wave's vectors fit into its part of a unit's place");
+    extern __shared__ __attribute__((aligned(16))) int8_t ring[];
     __shared__ float red[2][kMfmaWaves][16 * 17];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int part = blockIdx.x % g.parts, walker = blockIdx.x / g.parts, walkers = gridDim.x / g.parts;
     const int tok0 = blockIdx.y * group, nt = min(group, tokens - tok0), k0 = part * STRETCH, tiles = (g.n + 15) / 16;
-    for (int i = t; i < nt * (STRETCH / 4); i += NT) {
-        const int j = i / (STRETCH / 4), c = i - j * (STRETCH / 4), k = k0 + 4 * c;
-        const float* x = g.x + (size_t)(tok0 + j) * g.ldx;
-        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-        if ((g.k & 3) == 0 && (g.ldx & 3) == 0) {
-            if (k < g.k) v = *reinterpret_cast<const f32x4*>(x + k);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = k + e < g.k ? x[k + e] : 0.0f;
-        }
-        auto split = [&](auto big) {
-#pragma unroll
-            for (int p = 0; p < 3; p++) {
-                bf16x4 b;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    // what is beyond the largest bfloat16 lies in the rest (a part that rounds to infinity would leave infinity
-                    // less infinity); an infinity has no rest
-                    const bool finite = !big || isfinite(v[e]);
-                    b[e] = (bf16_t)(big && finite ? fminf(fmaxf(v[e], -kBf16Max), kBf16Max) : v[e]);
-                    v[e] = finite ? v[e] - (float)b[e] : 0.0f;
-                }
-                *reinterpret_cast<bf16x4*>(xp + (p * group + j) * ROW + c * 8) = b;
-            }
-        };
-        if (fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) > kBf16Max) split(std::true_type());
-        else split(std::false_type());                    // not a number stays what it is in every part
-    }
-    const int wk = wave * (KW * 32) + (lane >> 4) * 8;    // this lane's k within the stretch
-    const bf16_t* w = static_cast<const bf16_t*>(g.w) + k0 + wk;
-    bf16x8 buf[2][KW];
-    auto load = [&](int b, int tile) {
-        const bf16_t* row = w + (size_t)min(tile * 16 + (lane & 15), g.n - 1) * g.kpad;
-#pragma unroll
-        for (int s = 0; s < KW; s++)
-            if (k0 + wave * (KW * 32) + s * 32 < g.kpad) buf[b][s] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(row + s * 32));
-            else
-#pragma unroll
-                for (int e = 0; e < 8; e++) buf[b][s][e] = (bf16_t)0.0f;
+    const int mine = (tiles - walker + walkers - 1) / walkers, total = mine * UNITS;          // tiles and units of this workgroup
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)ring;
+    // the weights are read once on this chip, the vectors by every workgroup
+    auto request = [&](const void* base, unsigned off, unsigned to, auto once) __attribute__((always_inline)) {
+        if constexpr (decltype(once)::value) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" :: "s"(to), "v"(off), "s"(base) : "memory");
+        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(off), "s"(base) : "memory");
     };
-    load(0, walker);
-    if (walker + walkers < tiles) load(1, walker + walkers);
-    __syncthreads();
-    const int8_t* xl = xp + min(lane & 15, nt - 1) * ROW + wk * 2;
-    // Not a number may be of the parts' own making, where an infinite weight meets parts of zero or of both signs: the same sum with
-    // a float32 product per weight has the right of it.
-    auto whole = [&](int row, int j) __attribute__((always_inline)) {
-        const bf16_t* wr = static_cast<const bf16_t*>(g.w) + (size_t)row * g.kpad + k0;
-        float s = 0.0f;
-        for (int c = 0; c < min(STRETCH, g.kpad - k0); c += 8) {
-            const bf16x8 u = *reinterpret_cast<const bf16x8*>(wr + c);
-            bf16x8 b[3];
+    auto request_unit = [&](int u) __attribute__((always_inline)) {
+        const int tile = walker + u / UNITS * walkers, h = u % UNITS, last = min(16, g.n - tile * 16) - 1;
+        const int8_t* base = static_cast<const int8_t*>(g.w) + (size_t)tile * 16 * g.kpad * 2;
 #pragma unroll
-            for (int p = 0; p < 3; p++) b[p] = *reinterpret_cast<const bf16x8*>(xp + (p * group + j) * ROW + c * 2);
-#pragma unroll
-            for (int e = 0; e < 8; e++) s = fma_f((float)u[e], (float)b[0][e] + ((float)b[1][e] + (float)b[2][e]), s);
+        for (int q = 0; q < PER; q++) {
+            const int p = wave * PER + q, r = p / (UB / 1024), seg = p % (UB / 1024);
+            // what is behind the row's end (any of its bytes will do) meets zeros
+            const int kb = min((k0 + h * UK) * 2 + seg * 1024 + (lane ^ r) * 16, g.kpad * 2 - 16);
+            request(base, (unsigned)(min(r, last) * g.kpad * 2 + kb), lds0 + (u % SLOTS) * SLOT + p * 1024, std::true_type());
         }
+    };
+    // a wave's vectors [token][SL], in the last place's part that only this wave's requests write
+    int8_t* const xs = ring + (SLOTS - 1) * SLOT + wave * (PER * 1024);
+    constexpr int XC = SL / 4, XN = kMfmaTokens * XC / 64;    // 16-byte chunks of a token, and of a lane
+    const bool vec = (g.k & 3) == 0 && (g.ldx & 3) == 0 && (reinterpret_cast<uintptr_t>(g.x) & 15) == 0;
+    auto request_vectors = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < XN; i++) {
+            const int c = i * 64 + lane, j = min(c / XC, nt - 1), k = k0 + h * UK + wave * SL + c % XC * 4;
+            if (i * 64 < nt * XC) request(g.x + (size_t)tok0 * g.ldx, (unsigned)(j * g.ldx + min(k, g.k - 4)) * 4u, lds0 + (unsigned)(xs - ring) + i * 1024, std::false_type());
+        }
+    };
+    // The instruction has 16 columns for at most 8 tokens: columns 0 to 7 are the tokens' first and third part, 8 to 15 their second.
+    bf16x8 xf[UNITS * SW][2];
+    const int j0 = min(lane & 7, nt - 1), second = (lane >> 3) & 1, gq = lane >> 4;
+    constexpr int JI = 64 / XC;                               // tokens that a round of the wave's lanes covers
+    const int put0 = ((((lane % XC) >> 1) ^ (lane / XC)) << 4) + (lane & 1) * 8 + lane / XC * (SL * 2), row0 = second * kMfmaTokens + j0;
+    const int8_t* const get0 = xs + row0 * (SL * 2);
+    auto take_vectors = [&](int h) __attribute__((always_inline)) {
+        const int first = k0 + h * UK + wave * SL;            // k of the wave's stretch
+        f32x4 v[XN];
+#pragma unroll
+        for (int i = 0; i < XN; i++) {
+            if (i * JI >= nt) break;
+            if (vec) {
+                v[i] = *reinterpret_cast<const f32x4*>(xs + (i * 64 + lane) * 16);
+            } else {
+                const float* x = g.x + (size_t)(tok0 + min(i * JI + lane / XC, nt - 1)) * g.ldx;
+                for (int e = 0; e < 4; e++) v[i][e] = x[min(first + lane % XC * 4 + e, g.k - 1)];
+            }
+        }
+        if (first + SL > g.k) {
+#pragma unroll
+            for (int i = 0; i < XN; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[i][e] = first + lane % XC * 4 + e < g.k ? v[i][e] : 0.0f;
+        }
+        // A part is the upper half of the bits, so three of them are the value and none rounds up to infinity.  What is left of an infinity
+        // is not a number, which makes the sums such (see `whole`).  Parts lie as [2][token][SL], chunk c of 16 bytes at place c ^ row:
+        // the 16 columns of an operand read are on different banks.
+        auto put = [&](int i, int to) __attribute__((always_inline)) {
+            const int row = to * kMfmaTokens + i * JI;
+            uint2 o;
+            o.x = __builtin_amdgcn_perm(__float_as_uint(v[i][1]), __float_as_uint(v[i][0]), 0x07060302u);
+            o.y = __builtin_amdgcn_perm(__float_as_uint(v[i][3]), __float_as_uint(v[i][2]), 0x07060302u);
+            *reinterpret_cast<uint2*>(xs + (put0 ^ (row << 4)) + row * (SL * 2)) = o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[i][e] -= __uint_as_float(__float_as_uint(v[i][e]) & 0xFFFF0000u);
+        };
+        auto get = [&](int s) { return *reinterpret_cast<const bf16x8*>(get0 + (((s * 4 + gq) ^ row0) << 4)); };
+#pragma unroll
+        for (int i = 0; i < XN; i++) {
+            if (i * JI >= nt) break;
+            put(i, 0);
+            put(i, 1);
+        }
+#pragma unroll
+        for (int s = 0; s < SW; s++) xf[h * SW + s][0] = get(s);
+#pragma unroll
+        for (int i = 0; i < XN; i++) {
+            if (i * JI >= nt) break;
+            put(i, 0);
+        }
+        const uint32_t keep = second ? 0u : ~0u;
+#pragma unroll
+        for (int s = 0; s < SW; s++) {
+            i32x4 b = __builtin_bit_cast(i32x4, get(s));
+#pragma unroll
+            for (int e = 0; e < 4; e++) b[e] &= keep;
+            xf[h * SW + s][1] = __builtin_bit_cast(bf16x8, b);
+        }
+    };
+    auto all_read = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    if (vec) request_vectors(0);
+#pragma unroll
+    for (int u = 0; u < SLOTS - 1; u++)
+        if (u < total) request_unit(u);
+    if (vec) {
+        if (total >= SLOTS - 1) wait_vmcnt<(SLOTS - 1) * PER>();
+        else if (total == 2) wait_vmcnt<2 * PER>();
+        else wait_vmcnt<PER>();
+    }
+    take_vectors(0);
+    if constexpr (UNITS == 2) {
+        all_read();
+        if (vec) { request_vectors(1); wait_vmcnt<0>(); }
+        take_vectors(1);
+    }
+    all_read();
+    if (SLOTS - 1 < total) request_unit(SLOTS - 1);
+    // Not a number may be of the parts' own making, where an infinite weight meets parts of zero or of both signs (or, behind the row's
+    // end, zeros) or a value is infinite: the same sum with a float32 product per weight has the right of it.
+    auto whole = [&](int row, int j) __attribute__((always_inline)) {
+        const bf16_t* wr = static_cast<const bf16_t*>(g.w) + (size_t)row * g.kpad;
+        const float* x = g.x + (size_t)(tok0 + j) * g.ldx;
+        float s = 0.0f;
+        for (int k = k0; k < min(k0 + STRETCH, g.k); k++) s = fma_f((float)wr[k], x[k], s);
         return s;
     };
-    auto process = [&](int b, int tile) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < KW; s++)
-#pragma unroll
-            for (int p = 2; p >= 0; p--)                  // the small parts first
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(buf[b][s], *reinterpret_cast<const bf16x8*>(xl + p * group * ROW + s * 64), acc, 0, 0, 0);
-        if (tile + 2 * walkers < tiles) load(b, tile + 2 * walkers);      // ahead of the branches below
-#pragma unroll
-        for (int i = 0; i < 4; i++) red[b][wave][((lane >> 4) * 4 + i) * 17 + (lane & 15)] = acc[i];
-        __syncthreads();                                  // red alternates with the buffer: one barrier per tile is enough
-        const int r = t & 15, j = t >> 4, row = tile * 16 + r, tok = tok0 + j;
+    auto finish = [&](int i) __attribute__((always_inline)) {
+        const int r = t & 15, j = t >> 4, row = (walker + i * walkers) * 16 + r, tok = tok0 + j;
         if (j < nt && row < g.n) {
-            auto total = [&](int i) {
-                const float* p = red[b][0] + (r + i) * 17 + j;
+            auto sum = [&](int o) {
+                const float* p = red[i & 1][0] + (r + o) * 17 + j;
                 float v[kMfmaWaves];
 #pragma unroll
-                for (int q = 0; q < kMfmaWaves; q++) v[q] = p[q * 16 * 17];
+                for (int q = 0; q < kMfmaWaves; q++) v[q] = p[q * 16 * 17] + p[q * 16 * 17 + 8];
                 float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-                if (isnan(s)) s = whole(min(row + i, g.n - 1), j);
-                return g.bias ? s + g.bias[min(row + i, g.n - 1)] : s;
+                if (isnan(s)) s = whole(min(row + o, g.n - 1), j);
+                return g.bias ? s + g.bias[min(row + o, g.n - 1)] : s;
             };
-            if (row >= g.n_split) g.out32[part * g.part_stride + (size_t)tok * g.ldo32 + row - g.n_split] = total(0);
-            else if (!g.glu) g.out[(size_t)tok * g.ldo + row] = total(0);
-            else if ((row & 1) == 0) g.out[(size_t)tok * g.ldo + (row >> 1)] = glu_f(g.glu, total(0), total(1), g.limit);
+            if (row >= g.n_split) g.out32[part * g.part_stride + (size_t)tok * g.ldo32 + row - g.n_split] = sum(0);
+            else if (!g.glu) g.out[(size_t)tok * g.ldo + row] = sum(0);
+            else if ((row & 1) == 0) g.out[(size_t)tok * g.ldo + (row >> 1)] = glu_f(g.glu, sum(0), sum(1), g.limit);
         }
     };
-    for (int tile = walker; tile < tiles; tile += 2 * walkers) {
-        process(0, tile);
-        if (tile + walkers < tiles) process(1, tile + walkers);
+    const int8_t* const mine_in = ring + (lane & 15) * UB;
+    for (int i = 0; i < mine; i++) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int h = 0; h < UNITS; h++) {
+            const int u = i * UNITS + h, younger = total - 1 - u;
+            if (younger >= SLOTS - 1) wait_vmcnt<(SLOTS - 1) * PER>();
+            else if (SLOTS > 3 && younger == 2) wait_vmcnt<2 * PER>();
+            else if (SLOTS > 2 && younger == 1) wait_vmcnt<PER>();
+            else wait_vmcnt<0>();
+            all_read();                                        // the last tile's sums have left
+            barrier();
+            bf16x8 wf[SW];
+            const int8_t* in = mine_in + (u % SLOTS) * SLOT;
+#pragma unroll
+            for (int s = 0; s < SW; s++) {
+                const int c = wave * (SL / 8) + s * 4 + gq;      // chunk of the row, in KiB of 64 chunks that are rotated each by itself
+                wf[s] = *reinterpret_cast<const bf16x8*>(in + (c ^ (lane & 15)) * 16);
+            }
+            all_read();
+            barrier();
+            if (u + SLOTS < total) request_unit(u + SLOTS);
+            if (h == 0 && i > 0) finish(i - 1);
+#pragma unroll
+            for (int s = 0; s < SW; s++)
+#pragma unroll
+                for (int p = 1; p >= 0; p--)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[h * SW + s][p], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[i & 1][wave][(gq * 4 + e) * 17 + (lane & 15)] = acc[e];
     }
+    __syncthreads();
+    finish(mine - 1);
 }
 
-template <int KW>
+template <int UK, int UNITS>
 static int launch_gemv_mfma(const GemvArgs& g, int tokens, hipStream_t st) {
-    constexpr int STRETCH = KW * kMfmaWaves * 32, fit = (int)(kGemvTokensLds / (3 * gemv_mfma_row(STRETCH)));
-    constexpr int most = fit < kMfmaTokens ? fit : kMfmaTokens;
-    static_assert(most >= 4, "tokens that fit");
+    constexpr int lds = 128 * 1024;
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mfma_kernel<KW>), hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTokensLds));
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mfma_kernel<UK, UNITS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         opted_in.store(true, std::memory_order_release);
     }
-    const int groups = (tokens + most - 1) / most, group = (tokens + groups - 1) / groups, tiles = (g.n + 15) / 16;
-    const size_t lds = (size_t)3 * group * gemv_mfma_row(STRETCH);
-    int walkers = 256 / (g.parts * groups);               // one workgroup per CU: a second one does not speed the stream up
+    const int groups = (tokens + kMfmaTokens - 1) / kMfmaTokens, group = (tokens + groups - 1) / groups, tiles = (g.n + 15) / 16;
+    int walkers = 256 / (g.parts * groups);               // one workgroup per CU
     if (walkers < 1) walkers = 1;
     if (walkers > tiles) walkers = tiles;
-    gemv_mfma_kernel<KW><<<dim3(walkers * g.parts, groups), kMfmaWaves * 64, lds, st>>>(g, tokens, group);
+    gemv_mfma_kernel<UK, UNITS><<<dim3(walkers * g.parts, groups), kMfmaWaves * 64, lds, st>>>(g, tokens, group);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
@@ -518,9 +600,9 @@ int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     if (pro == 0 && tokens > 1 && !g.per_token) {
         if constexpr (std::is_same<ET, bf16_t>::value) {
             const int stretch = (g.kpad + g.parts - 1) / g.parts;
-            if (stretch <= 1024) return launch_gemv_mfma<4>(g, tokens, st);
-            if (stretch <= 2048) return launch_gemv_mfma<8>(g, tokens, st);
-            if (stretch <= 4096) return launch_gemv_mfma<16>(g, tokens, st);
+            if (stretch <= 1024) return launch_gemv_mfma<1024, 1>(g, tokens, st);
+            if (stretch <= 2048) return launch_gemv_mfma<2048, 1>(g, tokens, st);
+            if (stretch <= 4096) return launch_gemv_mfma<2048, 2>(g, tokens, st);
             FX_REQUIRE(g.parts == 1, "gemv_float: %d parts of k=%d", g.parts, g.k);
         }
         return gemv_tokens<ET>(g, tokens, st);
