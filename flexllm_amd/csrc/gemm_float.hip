@@ -4,6 +4,7 @@
 #include <atomic>
 #include "float_ops.h"
 #include "gemm_walk.h"
+#include "gemm_few.h"
 
 namespace fx {
 
@@ -236,7 +237,8 @@ static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
 //
 // bfloat16 (64 k): 777 x 28672 x 4096 takes 256 columns (169 us; 128 x 128: 222 us), 1531 x 16384 x 2048 too (86 us; 123), 777 x 4096 x 14336
 // 128 x 128 (1 round, 99 us; 128 x 256: 159 us), 1024 x 2048 x 2048 64 x 128 (16.0 us; 128 x 128: 21.4 us).  128 x 128 with two stages fits
-// twice into a CU: 1389 x 6528 x 640 22.5 us, 27.5 on the one with five stages.
+// twice into a CU: 1389 x 6528 x 640 22.5 us, 27.5 on the one with more stages.  (Four stages on the others: 777 x 2560 x 2048 18.6 us, five 19.4,
+// three 19.7; 41 x 2048 x 8192 in eight parts on 64 x 64 9.1, six 9.3, three 10.0.)
 // float32 (32 k): 333 x 16384 x 2048 takes 64 x 128 (196 us; 128 x 128: 244 us), 333 x 2048 x 8192 64 x 64 (135 us; 64 x 128: 248 us).
 struct GemmTileCost { int bm, bn, cost, round, per_cu; };
 template <typename ET> struct GemmTiles;
@@ -311,6 +313,7 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         FX_LAUNCH_CHECK();
         g.n = g.n_split;
     }
+    if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
         case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
@@ -320,9 +323,9 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
             case 160: return launch_walk<bf16_t, 2, 5, 8, 3, 2>(g, st);
             default: return launch_walk<bf16_t, 2, 4, 8, 4, 3>(g, st);
         }
-        case 2: return launch_walk<bf16_t, 2, 4, 4, 5, 5>(g, st);
-        case 3: return launch_walk<bf16_t, 2, 2, 4, 6, 6>(g, st);
-        case 4: return launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
+        case 2: return launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
+        case 3: return launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
+        case 4: return launch_walk<bf16_t, 2, 2, 2, 4, 4>(g, st);
         default: return launch_walk<bf16_t, 2, 4, 4, 2, 2>(g, st);
     }
 }
@@ -335,9 +338,9 @@ static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
-    if constexpr (BM == 128) return launch_walk<bf16_t, 2, 4, 4, 5, 5>(g, st);
+    if constexpr (BM == 128) return launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
     else if (g.group_rows < 45) return launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
-    else return launch_walk<bf16_t, 2, 2, 4, 6, 6>(g, st);
+    else return launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
 }
 
 // ---- float32 -----------------------------------------------------------------------------------------------------
@@ -349,8 +352,8 @@ int gemm_float<float>(const GemmArgs& args, hipStream_t st) {
     FX_REQUIRE(!g.tiles, "gemm_float: a tile table goes to gemm_grouped");
     long cost;
     switch (gemm_cheapest_tile<float>(g, g.parts, cost)) {
-        case 0: return launch_walk<float, 2, 4, 4, 5, 5>(g, st);
-        case 1: return launch_walk<float, 2, 2, 4, 6, 6>(g, st);
+        case 0: return launch_walk<float, 2, 4, 4, 4, 4>(g, st);
+        case 1: return launch_walk<float, 2, 2, 4, 4, 4>(g, st);
         default: return launch_walk<float, 2, 2, 2, 3, 3>(g, st);
     }
 }
@@ -406,6 +409,7 @@ int flexllm_linear_float_gemm_rows(int m, int k, int n, int dtype, int parts) {
     g.m = m; g.k = k; g.n = n;
     long cost;
     if (dtype) return GemmTiles<float>::list[gemm_cheapest_tile<float>(g, parts, cost)].bm;
+    if (gemm_few_ok(m, k, n, parts)) return m <= 16 ? 16 : 32;
     const GemmTileCost& t = GemmTiles<bf16_t>::list[gemm_cheapest_tile<bf16_t>(g, parts, cost)];
     return t.bn == 256 ? gemm_wide_rows(m, k, n, parts) : t.bm;
 }

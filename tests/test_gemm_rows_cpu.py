@@ -19,3 +19,11 @@ def test_rows_that_measured_best():
     assert f(1024, 2048, 16384) == 256 and f(2528, 8192, 2048) == 128 and f(777, 14336, 4096) == 128 and f(1024, 2048, 2048) == 64
     assert i(777, 4096, 28672) == 224 and i(1531, 2048, 16384) == 192 and i(1024, 2048, 16384) == 256
     assert i(2528, 8192, 2048) == lib().flexllm_linear_i8_gemm_rows(2528, 2048, 3072, 1) == 128
+
+
+def test_few_rows_are_one_pass():
+    from flexllm_amd import lib
+    import test_gpu_gemm_few as few
+    f = lambda m, k, n, parts=1: lib().flexllm_linear_float_gemm_rows(m, k, n, 0, parts)  # noqa: E731
+    assert all(f(m, k, n) == (16 if m <= 16 else 32) for m, n in few.FEW for k in few.K)
+    assert f(33, 2048, 16384) == f(9, 4160, 16384) == f(9, 2048, 8188) == f(9, 2048, 16384, 2) == 64
