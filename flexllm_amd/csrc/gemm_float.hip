@@ -47,8 +47,9 @@ enum GemmStores { kSingle = 0, kQuad = 1, kWide = 2 };
 
 // A wave's outputs that all lie on one side of the split: J blocks of 16 columns at a time become 64 consecutive bytes of a row, 16 per
 // lane (GLU: the unit, 0: none; OT: type of the outputs).
+// cols: those that there are from the wave's first one on, a multiple of what 16 bytes of output are made of.
 template <typename OT, class W, int GLU, bool BIAS>
-__device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias, float limit, int row0, int row_end, f32x4 (&acc)[W::MIv][W::NIv]) {
+__device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias, float limit, int row0, int row_end, int cols, f32x4 (&acc)[W::MIv][W::NIv]) {
     constexpr int R = (int)sizeof(OT) / (GLU ? 2 : 1), J = 4 / R, NI = W::NIv, MI = W::MIv;   // R: words of a lane's four columns
     const int lane = threadIdx.x & 63, row_bytes = ldy * (int)sizeof(OT);
     const TileRows out(y + (size_t)row0 * ldy, row_end - row0, row_bytes);
@@ -60,8 +61,9 @@ __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias,
 #pragma unroll
             for (int j = 0; j < J; j++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) b[j][e] = bias[(j0 + j) * 16 + (lane >> 4) * 4 + e];
+                for (int e = 0; e < 4; e++) b[j][e] = bias[min((j0 + j) * 16 + (lane >> 4) * 4 + e, cols - 1)];
         }
+        const bool there = j0 * 16 + (lane >> 4) * (4 * J) < cols;
 #pragma unroll
         for (int i = 0; i < MI; i++) {
             uint32_t w[J][R];
@@ -69,6 +71,7 @@ __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias,
             for (int j = 0; j < J; j++) {
                 f32x4 v = acc[i][j0 + j];
                 if constexpr (BIAS) v += b[j];
+                else asm volatile("" : "+v"(v));                  // out of the accumulation registers here, a block at a time
                 OT o[GLU ? 2 : 4];
                 if constexpr (GLU != 0) {
                     o[0] = (OT)glu_f(GLU, v[0], v[1], limit);
@@ -80,29 +83,41 @@ __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias,
                 __builtin_memcpy(w[j], o, sizeof(o));
             }
             join_blocks<R>(w);
-            out.put(&w[0][0], at + i * 16 * row_bytes + j0 * 16 * (int)sizeof(OT) / (GLU ? 2 : 1));
+            out.put(&w[0][0], there ? at + i * 16 * row_bytes + j0 * 16 * (int)sizeof(OT) / (GLU ? 2 : 1) : kNowhere);
             __builtin_amdgcn_sched_barrier(0);                 // one piece after the other: all at once are more than the registers hold
         }
     }
 }
 
-template <typename ET, class W>
+// OUT: forms of the outputs that a kernel of tiles of 256 columns is made for (all of them in one are more than its registers hold beside the
+// sums, and spilled sums have come back wrong).  kOutAny: all, at run time.
+enum GemmOut { kOutAny = 0, kOutPlain = 1, kOutBias = 2, kOutClamped = 3, kOutGelu = 4 };
+template <typename ET, class W, int OUT>
 __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_end, int col0, int stores, int8_t* smem, f32x4 (&acc)[W::MIv][W::NIv]) {
     constexpr int NI = W::NIv, MI = W::MIv, J = std::is_same<ET, float>::value ? 2 : 4;
     const int lane = threadIdx.x & 63, fg = lane >> 4, fr = lane & 15, end = col0 + NI * 16;
-    const float* bias = g.bias ? g.bias + col0 : nullptr;
-    if (stores == kWide && col0 >= g.n_split && end <= g.n) {
-        float* y = g.y32 + (col0 - g.n_split);
-        if (bias) return gemm_out_wide<float, W, 0, true>(y, g.ldy32, bias, 0.0f, row0, row_end, acc);
-        return gemm_out_wide<float, W, 0, false>(y, g.ldy32, bias, 0.0f, row0, row_end, acc);
-    }
-    if constexpr (NI % J == 0) {
-        if (stores == kWide && end <= g.n_split && !(bias && g.glu)) {
-            ET* y = static_cast<ET*>(g.y);
-            if (g.glu == kGluClamped) return gemm_out_wide<ET, W, kGluClamped, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, acc);
-            if (g.glu == kGluGelu) return gemm_out_wide<ET, W, kGluGelu, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, acc);
-            if (bias) return gemm_out_wide<ET, W, 0, true>(y + col0, g.ldy, bias, 0.0f, row0, row_end, acc);
-            return gemm_out_wide<ET, W, 0, false>(y + col0, g.ldy, bias, 0.0f, row0, row_end, acc);
+    const float* bias = g.bias + col0;
+    ET* const y = static_cast<ET*>(g.y);
+    float* const y32 = g.y32 + (col0 - g.n_split);
+    const int cols = g.n_split - col0, cols32 = g.n - col0;
+    if constexpr (OUT == kOutClamped || OUT == kOutGelu) {
+        return gemm_out_wide<ET, W, OUT == kOutGelu ? kGluGelu : kGluClamped, false>(y + (col0 >> 1), g.ldy, nullptr, g.limit, row0, row_end, cols, acc);
+    } else if constexpr (OUT != kOutAny) {
+        if (col0 >= g.n_split) gemm_out_wide<float, W, 0, OUT == kOutBias>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
+        else gemm_out_wide<ET, W, 0, OUT == kOutBias>(y + col0, g.ldy, bias, 0.0f, row0, row_end, cols, acc);
+        return;
+    } else {
+        if (stores == kWide && col0 >= g.n_split) {
+            if (g.bias) return gemm_out_wide<float, W, 0, true>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
+            return gemm_out_wide<float, W, 0, false>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
+        }
+        if constexpr (NI % J == 0) {
+            if (stores == kWide && (end <= g.n_split || g.n_split == g.n) && !(g.bias && g.glu)) {
+                if (g.glu == kGluClamped) return gemm_out_wide<ET, W, kGluClamped, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, cols, acc);
+                if (g.glu == kGluGelu) return gemm_out_wide<ET, W, kGluGelu, false>(y + (col0 >> 1), g.ldy, bias, g.limit, row0, row_end, cols, acc);
+                if (g.bias) return gemm_out_wide<ET, W, 0, true>(y + col0, g.ldy, bias, 0.0f, row0, row_end, cols, acc);
+                return gemm_out_wide<ET, W, 0, false>(y + col0, g.ldy, bias, 0.0f, row0, row_end, cols, acc);
+            }
         }
     }
     // Any other: sixteen columns of the wave's rows at a time through LDS, so that a loop can take them (the walk has left it behind: the
@@ -132,7 +147,7 @@ __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_en
 template <typename ET, int WM, int MI, int NI, int NA, int NB>
 struct FloatWalk : GemmWalk<ET, WM, MI, NI, NA, NB> { static constexpr int MIv = MI, NIv = NI; };
 
-template <typename ET, class W>
+template <typename ET, class W, int OUT>
 __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmArgs g, int tiles_m, int tiles_n, int stores) {
     extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
     int tm, tn, group = 0, row0, row_end;
@@ -162,27 +177,56 @@ __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmA
         const int r = W::load_row_b(j);
         offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)(g.ldw * sizeof(ET)) + W::load_byte(r);
     }
+    // Workgroups that walk in step all ask for the same bytes of rows that lie a power of two apart, and some of the memory's channels have it all.  So
+    // each die begins an eighth of k further on (many parts of k are spread by themselves; float32 waits for its products): bfloat16, 41 rows,
+    // 28672 x 4096 50.7 -> 43.7 us, 1531 x 2560 x 2048 22.9 -> 21.8, 777 x 2048 x 8192 in two parts 35.1 -> 34.4; in eight parts 41 x 2048 x 8192
+    // 9.4 without and 10.5 with it.
+    int first = 0;
+    if constexpr (sizeof(ET) == 2 && W::kTurned)
+        if (g.parts <= 2) first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x & 7) * (k1 - k0) / 8);
     f32x4 acc[W::MIv][W::NIv];
     W::run(static_cast<const int8_t*>(g.a) + (size_t)k0 * 128, static_cast<const int8_t*>(g.w) + (size_t)group * g.w_stride * sizeof(ET) + (size_t)k0 * 128, offa, offb,
-           k1 - k0, gemm_smem, acc);
+           k1 - k0, gemm_smem, acc, first);
     const int r0 = row0 + W::row_of_wave(), c0 = col0 + W::col_of_wave();
-    gemm_out<ET, W>(g, r0, row_end, c0, stores, gemm_smem, acc);
+    gemm_out<ET, W, OUT>(g, r0, row_end, c0, stores, gemm_smem, acc);
 }
 
-template <typename ET, int WM, int MI, int NI, int NA, int NB>
-static int launch_walk(const GemmArgs& g, hipStream_t st) {
-    using W = FloatWalk<ET, WM, MI, NI, NA, NB>;
+// Whole pieces: rows and outputs start on 16 bytes, and both sides of the split are a multiple of the columns that a piece is made of.
+template <typename ET>
+static int gemm_stores(const GemmArgs& g) {
+    const int piece = 16 / (int)sizeof(ET);
+    if ((g.n & 3) || (g.n_split & 3) || (g.ldy & 3) || (g.ldy32 & 3)) return kSingle;
+    const bool wide = rows_fit(g.ldy, sizeof(ET)) && rows_fit(g.ldy32, 4) && g.ldy % piece == 0 && g.n_split % (g.glu ? 2 * piece : piece) == 0 &&
+                      ((reinterpret_cast<uintptr_t>(g.y) | reinterpret_cast<uintptr_t>(g.y32)) & 15) == 0;
+    return wide ? kWide : kQuad;
+}
+// Tiles of 256 columns know no other way; a wave's 128 columns lie on one side of the split, and with a gated unit there is only one.
+static bool gemm_wide_ok(const GemmArgs& g) {
+    return gemm_stores<bf16_t>(g) == kWide && (g.n_split == g.n || (!g.glu && g.n_split % 128 == 0)) && !(g.bias && g.glu);
+}
+
+template <typename ET, class W, int OUT>
+static int launch_walk_out(const GemmArgs& g, hipStream_t st) {
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float_walk_kernel<ET, W>), hipFuncAttributeMaxDynamicSharedMemorySize, W::kLds));
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_float_walk_kernel<ET, W, OUT>), hipFuncAttributeMaxDynamicSharedMemorySize, W::kLds));
         opted_in.store(true, std::memory_order_release);
     }
     const int tm = g.tiles ? g.max_tiles : (g.m + W::BM - 1) / W::BM, tn = (g.n + W::BN - 1) / W::BN;
-    const bool quad = (g.n & 3) == 0 && (g.n_split & 3) == 0 && (g.ldy & 3) == 0 && (g.ldy32 & 3) == 0;
-    const bool wide = quad && rows_fit(g.ldy, sizeof(ET)) && rows_fit(g.ldy32, 4) && g.ldy % (16 / (int)sizeof(ET)) == 0 && ((reinterpret_cast<uintptr_t>(g.y) | reinterpret_cast<uintptr_t>(g.y32)) & 15) == 0;
-    gemm_float_walk_kernel<ET, W><<<dim3(tm * tn, g.parts), 256, W::kLds, st>>>(g, tm, tn, wide ? kWide : quad ? kQuad : kSingle);
+    gemm_float_walk_kernel<ET, W, OUT><<<dim3(tm * tn, g.parts), 256, W::kLds, st>>>(g, tm, tn, gemm_stores<ET>(g));
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
+}
+template <typename ET, int WM, int MI, int NI, int NA, int NB>
+static int launch_walk(const GemmArgs& g, hipStream_t st) {
+    using W = FloatWalk<ET, WM, MI, NI, NA, NB>;
+    if constexpr (W::kSumsApart) {
+        if (g.glu == kGluClamped) return launch_walk_out<ET, W, kOutClamped>(g, st);
+        if (g.glu == kGluGelu) return launch_walk_out<ET, W, kOutGelu>(g, st);
+        return g.bias ? launch_walk_out<ET, W, kOutBias>(g, st) : launch_walk_out<ET, W, kOutPlain>(g, st);
+    } else {
+        return launch_walk_out<ET, W, kOutAny>(g, st);
+    }
 }
 
 // A few float32 output columns (router rows, low-rank gate inputs): 16 rows x 16 columns per workgroup on
@@ -316,7 +360,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
     if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
-        case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
+        case 0: case 1: switch (gemm_wide_ok(g) ? gemm_wide_rows(g.m, g.k, g.n, g.parts) : 0) {
+            case 0: return launch_walk<bf16_t, 2, 4, 4, 2, 2>(g, st);
             case 256: return launch_walk<bf16_t, 2, 8, 8, 3, 2>(g, st);
             case 224: return launch_walk<bf16_t, 2, 7, 8, 3, 2>(g, st);
             case 192: return launch_walk<bf16_t, 2, 6, 8, 3, 2>(g, st);

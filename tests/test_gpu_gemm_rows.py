@@ -9,18 +9,36 @@ from test_gpu_prefill import fx  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 # rows of a workgroup: rows and columns of a product
-FLOAT = {128: (300, 12284), 160: (1299, 12284), 192: (1632, 12288), 224: (2076, 6140), 256: (1151, 12284)}
+FLOAT = {128: (300, 12272), 160: (1299, 12272), 192: (1632, 12288), 224: (2076, 6128), 256: (1151, 12272)}
 FLOAT_K = [320, 576]
 INT = {(128, 1152): (300, 12284), (160, 1152): (1558, 6144), (192, 1152): (1632, 6140), (224, 384): (2076, 6144), (224, 1152): (1928, 6140),
        (256, 384): (1151, 12284), (256, 1152): (1151, 12288)}
 
 
 @pytest.mark.parametrize("k", FLOAT_K)
-@pytest.mark.parametrize("split,glu", [("all", 0), ("all", 1), ("half", 2), ("none", 0)])
+@pytest.mark.parametrize("split,glu", [("all", 0), ("all", 1), ("all", 2), ("half", 0), ("half", 2), ("none", 0), ("odd", 0)])
 @pytest.mark.parametrize("rows", FLOAT)
 def test_rows_bfloat16(rows, split, glu, k):
+    """Outputs on either side of a split between waves; a split inside a wave's columns goes to other tiles."""
     m, n = FLOAT[rows]
-    floats.test_gemm_tiles(m, n, {"all": n, "half": n // 512 * 256 + 64, "none": 0}[split], glu, k, "bfloat16")
+    floats.test_gemm_tiles(m, n, {"all": n, "half": n // 512 * 256 + 128, "none": 0, "odd": n // 512 * 256 + 64}[split], glu, k, "bfloat16")
+
+
+@pytest.mark.parametrize("rows", FLOAT)
+def test_bias(rows):
+    """Added in float32 ahead of the rounding, on both sides of the split, columns that do not fill the last wave among them."""
+    import numpy as np
+    import lopazen_cases as lc
+    from flexllm_amd import ops, to_device
+    from flexllm_amd.loader import from_bf16, to_bf16
+    (m, n), k = FLOAT[rows], 320
+    split, r = n // 512 * 256, np.random.default_rng(rows)
+    a, w, bias = lc.round_bf16(r.standard_normal((m, k))), lc.round_bf16(r.standard_normal((n, k))), r.standard_normal(n).astype(np.float32)
+    y, y32 = ops.linear_float(to_device(to_bf16(a)), to_device(to_bf16(w)), split, bias=to_device(bias))
+    want = a.astype(np.float64) @ w.astype(np.float64).T + bias
+    d = 1e-5 * np.sqrt(k)                                 # as for the tiles
+    assert np.all(np.abs(from_bf16(y.numpy()) - want[:, :split]) <= 2.0 ** -8 * np.abs(want[:, :split]) + d)
+    assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * np.abs(want[:, split:]) + d)
 
 
 @pytest.mark.parametrize("rows,k", INT)
