@@ -177,16 +177,9 @@ __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmA
         const int r = W::load_row_b(j);
         offb[j] = (unsigned)min(col0 + r, g.n - 1) * (unsigned)(g.ldw * sizeof(ET)) + W::load_byte(r);
     }
-    // Workgroups that walk in step all ask for the same bytes of rows that lie a power of two apart, and some of the memory's channels have it all.  So
-    // each die begins an eighth of k further on (many parts of k are spread by themselves; float32 waits for its products): bfloat16, 41 rows,
-    // 28672 x 4096 50.7 -> 43.7 us, 1531 x 2560 x 2048 22.9 -> 21.8, 777 x 2048 x 8192 in two parts 35.1 -> 34.4; in eight parts 41 x 2048 x 8192
-    // 9.4 without and 10.5 with it.
-    int first = 0;
-    if constexpr (sizeof(ET) == 2 && W::kTurned)
-        if (g.parts <= 2) first = __builtin_amdgcn_readfirstlane((int)(blockIdx.x & 7) * (k1 - k0) / 8);
     f32x4 acc[W::MIv][W::NIv];
     W::run(static_cast<const int8_t*>(g.a) + (size_t)k0 * 128, static_cast<const int8_t*>(g.w) + (size_t)group * g.w_stride * sizeof(ET) + (size_t)k0 * 128, offa, offb,
-           k1 - k0, gemm_smem, acc, first);
+           k1 - k0, gemm_smem, acc);
     const int r0 = row0 + W::row_of_wave(), c0 = col0 + W::col_of_wave();
     gemm_out<ET, W, OUT>(g, r0, row_end, c0, stores, gemm_smem, acc);
 }

@@ -145,13 +145,10 @@ struct GemmWalk {
     static __device__ __forceinline__ int load_row_b(int j) { return (wave() * BI + j) * 8 + ((int)threadIdx.x & 63) / 8; }
     static __device__ __forceinline__ unsigned load_byte(int r) { return (unsigned)((((int)threadIdx.x & 7) ^ rot(r)) * 16); }
 
-    // Tiles of 128 columns and less may begin at any stage of k and come round to it (`first`).  Of the wide ones the loop has no registers left for that.
-    static constexpr bool kTurned = !kSumsApart;
     // a, w: first byte of k of the operands; offa, offb: byte offsets of this lane's loads behind them; nk: stages.  Nothing else of the
     // workgroup may be on its way to LDS.  Ends with every wave's loads and reads of LDS complete, without a barrier.
     static __device__ __forceinline__ void run(const int8_t* a, const int8_t* w, const unsigned (&offa)[AI], const unsigned (&offb)[BI], int nk, int8_t* smem,
-                                               Acc (&acc)[MI][NI], int first = 0) {
-        const int start = kTurned ? first : 0;
+                                               Acc (&acc)[MI][NI]) {
         const int lane = threadIdx.x & 63, wv = wave();
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
         const unsigned lds_a = lds0 + wv * (AI * 1024), lds_b = lds0 + NA * ASZ + wv * (BI * 1024);
@@ -180,15 +177,14 @@ struct GemmWalk {
         // Behind the barrier of stage e: W's loads of stage e + NB over the first half of the last k-step, then A's of e + NA over
         // as many matrix instructions as a k-step has.
         constexpr int early_a = early();
-        auto at_k = [&](int s) { const int k = start + s; return kTurned && k >= nk ? k - nk : k; };
 #pragma unroll
         for (int s = 0; s < NA; s++) {
 #pragma unroll
             for (int j = 0; j < BI; j++)
-                if (s < NB && s < nk) load_now(w + (size_t)at_k(s) * 128, offb[j], lds_b + s * BSZ, j);
+                if (s < NB && s < nk) load_now(w + (size_t)s * 128, offb[j], lds_b + s * BSZ, j);
 #pragma unroll
             for (int j = 0; j < AI; j++)
-                if ((s < NA - 1 || j < early_a) && s < nk) load_now(a + (size_t)at_k(s) * 128, offa[j], lds_a + s * ASZ, j);
+                if ((s < NA - 1 || j < early_a) && s < nk) load_now(a + (size_t)s * 128, offa[j], lds_a + s * ASZ, j);
         }
         const int fr = lane & 15, fg = lane >> 4;
         int at[KS];
@@ -222,11 +218,10 @@ struct GemmWalk {
         for (int q = 0; q < NR; q++) read(0, 0, 0, 0, q);
         // ring slots of the last, this and the next stage; the last one's are refilled
         unsigned a0 = (NA - 1) * ASZ, a1 = 0, a2 = ASZ, b0 = (NB - 1) * BSZ, b1 = 0, b2 = BSZ;
-        int ka = nk >= NA ? at_k(NA - 1) : 0, kb = nk >= NA ? at_k(NB - 1) : 0;      // places of the stages kt - 1 + NA and kt - 1 + NB
+        int ka = NA - 1, kb = NB - 1;                            // stages kt - 1 + NA and kt - 1 + NB (as numbers: pointers cost the wide tiles spills)
         // left: stages behind this one.  loads: 2 all, 1 what is left for the last stages (the rest of the last barrier's, and W's where it is a stage
         // behind A), 0 none.  No branches among them: those cost a short walk 2 % (250 x 2560 x 2048 in four parts, eight stages on 128 x 128, 11.4 us and 11.2).
         auto stage = [&](int left, auto next, auto loads) __attribute__((always_inline)) {
-            const int ka1 = kTurned && ka + 1 == nk ? 0 : ka + 1, kb1 = kTurned && kb + 1 == nk ? 0 : kb + 1;
 #pragma unroll
             for (int s = 0; s < KS; s++) {
                 constexpr bool kNext = decltype(next)::value;
@@ -261,18 +256,18 @@ struct GemmWalk {
                     const bool there_a = kLoads == 2 || (kLoads == 1 && !last), there_b = kLoads == 2 || (kLoads == 1 && NA > NB && last);
 #pragma unroll
                     for (int j = 0; j < BI; j++) {
-                        if (p == slot_b(j) + 1 && there_b) load(w + (size_t)(last ? kb1 : kb) * 128, offb[j]);
+                        if (p == slot_b(j) + 1 && there_b) load(w + (size_t)(last ? kb + 1 : kb) * 128, offb[j]);
                         if (p == slot_b(j) && there_b) aim(lds_b + sb, j);
                     }
 #pragma unroll
                     for (int j = 0; j < AI; j++) {
-                        if (p == slot_a(j) + 1 && there_a) load(a + (size_t)(last ? ka1 : ka) * 128, offa[j]);
+                        if (p == slot_a(j) + 1 && there_a) load(a + (size_t)(last ? ka + 1 : ka) * 128, offa[j]);
                         if (p == slot_a(j) && there_a) aim(lds_a + sa, j);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            ka = ka1; kb = kb1;
+            ka++; kb++;
             a0 = a1; a1 = a2; a2 = a2 == (NA - 1) * ASZ ? 0 : a2 + ASZ;
             b0 = b1; b1 = b2; b2 = b2 == (NB - 1) * BSZ ? 0 : b2 + BSZ;
         };
