@@ -618,36 +618,51 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
     const int lane = threadIdx.x & 63, fr = lane & 15, fg = lane >> 4;
     const int wr = W::row_of_wave(), wc = W::col_of_wave();
     if constexpr (EPI == kDmaQkv) {
-        // A wave has 64 tokens x two heads.  Channels c and c + 32 of a token are in blocks j and j + 2 of one lane, so RoPE stays in registers, and the
-        // quantised head of a token leaves in 16-byte pieces.
+        // A wave has 64 tokens x two heads.  Channels c and c + 32 of a token are in blocks j and j + 2 of one lane, so RoPE stays in registers, and
+        // the quantised head of a token leaves in 16-byte pieces.  Everything that has to be read is asked for at once: one wave per SIMD
+        // waits for each trip (2528 x 3072 x 2048, asked for token by token 34.4 us, 32.0 so).
         static_assert(MI == 4 && NI == 8, "64 tokens x two heads per wave");
-        constexpr int TP = 64 + 16;                            // V only: a head's bytes [channel][token], turned through LDS
+        constexpr int TP = 64 + 16, HEADS = 2;                 // TP: V only, a head's bytes [channel][token], turned through LDS
         int8_t* const turn = gemm_smem + W::wave() * (64 * TP);
-        __syncthreads();                                       // all waves are done with the stage buffers
+        const bool asym = qa.b_x != nullptr;                   // asymmetric activations: + zero point x row sum of the dequantised weights
+        f32x4 sn[MI][2], cs[MI][2], ws[HEADS][4], wq[HEADS][4];
+        float sx[MI], bx[MI];
 #pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-            const int c0 = col0 + wc + hh * 64, head = c0 / kHd;      // 0..q_heads-1 q, then k heads, then v heads
-            if (c0 >= n) break;
-            const bool asym = qa.b_x != nullptr;               // asymmetric activations: + zero point x row sum of the dequantised weights
-            f32x4 ws[4], wq[4];
+        for (int i = 0; i < MI; i++) {
+            const int r = min(row0 + wr + i * 16 + fr, m - 1);
+            sx[i] = s_x[r];
+            bx[i] = asym ? qa.b_x[r] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                sn[i][j] = *reinterpret_cast<const f32x4*>(qa.sin_t + (size_t)(qa.pos0 + r) * 32 + j * 16 + fg * 4);
+                cs[i][j] = *reinterpret_cast<const f32x4*>(qa.cos_t + (size_t)(qa.pos0 + r) * 32 + j * 16 + fg * 4);
+            }
+        }
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                ws[j] = *reinterpret_cast<const f32x4*>(w_s + c0 + j * 16 + fg * 4);
-                wq[j] = asym ? *reinterpret_cast<const f32x4*>(qa.w_sum + c0 + j * 16 + fg * 4) : f32x4{};
+                const int c = min(col0 + wc + hh * 64 + j * 16 + fg * 4, n - 4);
+                ws[hh][j] = *reinterpret_cast<const f32x4*>(w_s + c);
+                wq[hh][j] = asym ? *reinterpret_cast<const f32x4*>(qa.w_sum + c) : f32x4{};
             }
+        __syncthreads();                                       // all waves are done with the stage buffers
+#pragma unroll
+        for (int hh = 0; hh < HEADS; hh++) {
+            const int c0 = col0 + wc + hh * 64, head = c0 / kHd;      // 0..q_heads-1 q, then k heads, then v heads
+            if (c0 >= n) break;
             const bool is_q = head < qa.q_heads, is_v = head >= qa.q_heads + qa.kv_heads;
             const int hk = is_q ? head : is_v ? head - qa.q_heads - qa.kv_heads : head - qa.q_heads;
             const float div = is_q ? 8.0f * qa.q_s[hk] : is_v ? 1.0f * qa.v_s[hk] : 1.0f * qa.k_s[hk];     // sqrt(head_dim) folded into the Q scale
 #pragma unroll
             for (int i = 0; i < MI; i++) {
-                const int row = row0 + wr + i * 16 + fr, r = min(row, m - 1), pos = qa.pos0 + r;
-                const float sx = s_x[r], bx = asym ? qa.b_x[r] : 0.0f;
+                const int row = row0 + wr + i * 16 + fr, pos = qa.pos0 + row;
                 f32x4 v[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[j][e] = (float)acc[i][hh * 4 + j][e] * sx * ws[j][e];
-                    if (asym) v[j] = v[j] + bx * wq[j];
+                    for (int e = 0; e < 4; e++) v[j][e] = (float)acc[i][hh * 4 + j][e] * sx[i] * ws[hh][j][e];
+                    if (asym) v[j] = v[j] + bx[i] * wq[hh][j];
                 }
                 if (is_v) {
 #pragma unroll
@@ -662,13 +677,11 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
                 uint32_t o[4][1];
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    const f32x4 sn = *reinterpret_cast<const f32x4*>(qa.sin_t + (size_t)pos * 32 + j * 16 + fg * 4);
-                    const f32x4 cs = *reinterpret_cast<const f32x4*>(qa.cos_t + (size_t)pos * 32 + j * 16 + fg * 4);
                     float lo[4], hi[4];
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        lo[e] = v[j][e] * cs[e] - v[j + 2][e] * sn[e];
-                        hi[e] = v[j][e] * sn[e] + v[j + 2][e] * cs[e];
+                        lo[e] = v[j][e] * cs[i][j][e] - v[j + 2][e] * sn[i][j][e];
+                        hi[e] = v[j][e] * sn[i][j][e] + v[j + 2][e] * cs[i][j][e];
                     }
                     o[j][0] = static_q8x4(lo, div);
                     o[j + 2][0] = static_q8x4(hi, div);
@@ -845,9 +858,12 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
     }
     // the gated unit's 16 bytes of output are eight columns
     // (a head's 64 bytes leave in 16-byte pieces, too, and the scales and tables are read in such)
-    const auto bits = [](auto... p) { return (reinterpret_cast<uintptr_t>(p) | ...); };
-    if (EPI == kDmaQkv && pick < 2 && (bits(qa.q8, qa.kc, qa.vc, qa.sin_t, qa.cos_t, w_s, qa.w_sum) & 15)) return FX_GEMM_TILE(128, 128, 4, 2, 128, 8);
-    const bool wide = rows_fit(n, 4) && ((EPI != kDmaSwiglu && EPI != kDmaSwigluAsym) || (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0));
+    if constexpr (EPI == kDmaQkv) {
+        const auto bits = [](auto... p) { return (reinterpret_cast<uintptr_t>(p) | ...); };
+        // (on 128 x 128 the eight waves of the other kernel hide more of it: 1024 x 3072 x 2048 19.1 us, 20.4 as a walk)
+        if (pick == 1 && !(bits(qa.q8, qa.kc, qa.vc, qa.sin_t, qa.cos_t, w_s, qa.w_sum) & 15)) return launch_gemm_walk<EPI, 4>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
+    }
+    const bool wide = EPI != kDmaQkv && rows_fit(n, 4) && ((EPI != kDmaSwiglu && EPI != kDmaSwigluAsym) || (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0));
     if (pick < 2 && wide) {
 #define FX_GEMM_ROWS(MI) launch_gemm_walk<EPI, MI>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa)
         if constexpr (EPI != kDmaQkv) switch (gemm_i8_rows(m, k, n, false)) {
@@ -855,8 +871,8 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
             case 224: return FX_GEMM_ROWS(7);
             case 192: return FX_GEMM_ROWS(6);
             case 160: return FX_GEMM_ROWS(5);
+            default: return FX_GEMM_ROWS(4);
         }
-        return FX_GEMM_ROWS(4);
 #undef FX_GEMM_ROWS
     }
     if constexpr (EPI != kDmaQkv) {
