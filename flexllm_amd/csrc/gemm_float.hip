@@ -297,12 +297,13 @@ static int gemm_cheapest_tile(const GemmArgs& g, int parts, long& best) {
     return pick;
 }
 
-// bfloat16 products whose tile has 256 columns share their rows out anew: any multiple of 32 from 128 to 256 rows is a tile of its own on the
+// bfloat16 products whose tile has 256 columns share their rows out anew: any multiple of 32 from 96 to 256 rows is a tile of its own on the
 // same walk, and the one whose rounds cost least is taken (as above, in 0.01 us; the choices of 44 sizes of 120 to 4096 rows are 0.2 % from
 // the best ones on average).  777 x 28672 x 4096 takes 224 rows (170 us; 256: 185, 128: 211), 1531 x 16384 x 2048 192 (88 us; 256: 111,
-// 128: 103), 2596 x 3712 x 2560 160 (51 us; 256: 63, 128: 69), 722 x 10496 x 10112 128 (140 us; 160: 171, 256: 186).
+// 128: 103), 2596 x 3712 x 2560 160 (51 us; 256: 63, 128: 69), 722 x 10496 x 10112 128 (140 us; 160: 171, 256: 186),
+// 2528 x 2048 x 8192 96 (90 us; 128: 97, 160: 114; 64 rows, a trip of W for half the products, 139).
 struct GemmWideRows { int rows, stage, round; };
-constexpr GemmWideRows kGemmWideRows[] = {{256, 135, 1100}, {224, 119, 1000}, {192, 105, 900}, {160, 99, 800}, {128, 83, 700}};
+constexpr GemmWideRows kGemmWideRows[] = {{256, 135, 1100}, {224, 119, 1000}, {192, 105, 900}, {160, 99, 800}, {128, 83, 700}, {96, 70, 620}};
 static int gemm_wide_rows(int m, int k, int n, int parts) {
     const long stages = ((long)k * 2 / 128 + parts - 1) / parts;
     long best = 0;
@@ -359,7 +360,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
             case 224: return launch_walk<bf16_t, 2, 7, 8, 3, 2>(g, st);
             case 192: return launch_walk<bf16_t, 2, 6, 8, 3, 2>(g, st);
             case 160: return launch_walk<bf16_t, 2, 5, 8, 3, 2>(g, st);
-            default: return launch_walk<bf16_t, 2, 4, 8, 4, 3>(g, st);
+            case 128: return launch_walk<bf16_t, 2, 4, 8, 4, 3>(g, st);
+            default: return launch_walk<bf16_t, 2, 3, 8, 4, 3>(g, st);
         }
         case 2: return launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
         case 3: return launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);

@@ -830,6 +830,7 @@ inline int gemm_i8_tile(int m, int k, int n, bool qkv) {
 }
 
 // Products on 128-byte rows whose tile has 256 columns share their rows out anew, as bfloat16 ones do (gemm_float.hip); costs in 0.01 us.
+// 96 rows, which bfloat16 has too, make 2528 x 2048 x 8192 alone 8 % faster and the w4a4 prompt of 2528 around it 1.5 % slower (4350, 4415 us).
 struct GemmI8Rows { int rows, stage, round; };
 constexpr GemmI8Rows kGemmI8Rows[] = {{256, 110, 1500}, {224, 99, 1350}, {192, 88, 1200}, {160, 80, 1050}, {128, 70, 900}};
 inline int gemm_i8_rows(int m, int k, int n, bool qkv) {

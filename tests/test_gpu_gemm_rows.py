@@ -9,7 +9,7 @@ from test_gpu_prefill import fx  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 # rows of a workgroup: rows and columns of a product
-FLOAT = {128: (300, 12272), 160: (1299, 12272), 192: (1632, 12288), 224: (2076, 6128), 256: (1151, 12272)}
+FLOAT = {96: (371, 12272), 128: (589, 12272), 160: (1299, 12272), 192: (1632, 12288), 224: (2076, 6128), 256: (1151, 12272)}
 FLOAT_K = [320, 576]
 INT = {(128, 1152): (300, 12284), (160, 1152): (1558, 6144), (192, 1152): (1632, 6140), (224, 384): (2076, 6144), (224, 1152): (1928, 6140),
        (256, 384): (1151, 12284), (256, 1152): (1151, 12288)}
