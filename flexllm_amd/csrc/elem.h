@@ -40,13 +40,9 @@ __device__ __forceinline__ void store_past(float* p, float v) { __hip_atomic_sto
 __device__ __forceinline__ float load_past(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 __device__ __forceinline__ float fma_f(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-// 1 / d for d of 1 to 2^126: the hardware's reciprocal (1 ulp) and one step of Newton's method, within 0.51 ulp like the division (0.5), in
-// 3 instructions for its 10.
-__device__ __forceinline__ float rcp_f(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fma_f(fma_f(-d, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float sigmoid_f(float v) { return rcp_f(1.0f + exp_f(-v)); }
+// A division: exp_f is infinite far below zero (the cube in gelu gets there from a gate of -877 on), where a reciprocal with a step of
+// Newton's method is not a number, and the quotient is 0.
+__device__ __forceinline__ float sigmoid_f(float v) { return 1.0f / (1.0f + exp_f(-v)); }
 
 // log(sigmoid(z)) = min(z, 0) - log(1 + exp(-|z|)): no cancellation and no overflow for any z
 __device__ __forceinline__ float log_sigmoid_f(float z) { return fminf(z, 0.0f) - log1pf(exp_f(-fabsf(z))); }
