@@ -52,7 +52,7 @@ template <typename OT, class W, int GLU, bool BIAS>
 __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias, float limit, int row0, int row_end, int cols, f32x4 (&acc)[W::MIv][W::NIv]) {
     constexpr int R = (int)sizeof(OT) / (GLU ? 2 : 1), J = 4 / R, NI = W::NIv, MI = W::MIv;   // R: words of a lane's four columns
     const int lane = threadIdx.x & 63, row_bytes = ldy * (int)sizeof(OT);
-    const TileRows out(y + (size_t)row0 * ldy, row_end - row0, row_bytes);
+    const TileRows out(y + (size_t)row0 * ldy, row_end - row0, MI * 16, row_bytes);
     const int at = (lane & 15) * row_bytes + (lane >> 4) * 16;
 #pragma unroll
     for (int j0 = 0; j0 < NI; j0 += J) {

@@ -712,9 +712,9 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
         constexpr bool kAsym = EPI == kDmaDequantAsym || EPI == kDmaSwigluAsym, kUnit = EPI == kDmaSwiglu || EPI == kDmaSwigluAsym;
         constexpr int J = kUnit ? 2 : 1;                       // blocks of 16 columns whose outputs leave together, 64 bytes of a row
         const int rows = m - row0 - wr, ld = kUnit ? n >> 1 : n;
-        const TileRows out(EPI == kDmaRaw ? reinterpret_cast<float*>(c_out) + (size_t)(row0 + wr) * ld : y + (size_t)(row0 + wr) * ld, rows, ld * 4);
+        const TileRows out(EPI == kDmaRaw ? reinterpret_cast<float*>(c_out) + (size_t)(row0 + wr) * ld : y + (size_t)(row0 + wr) * ld, rows, MI * 16, ld * 4);
         const bool has_res = !kUnit && EPI != kDmaRaw && residual != nullptr;
-        const TileRows res(const_cast<float*>(has_res ? residual + (size_t)(row0 + wr) * n : y), has_res ? rows : 0, n * 4);
+        const TileRows res(const_cast<float*>(has_res ? residual + (size_t)(row0 + wr) * n : y), has_res ? rows : 0, MI * 16, n * 4);
         float sx[MI], bx[MI];
         if constexpr (EPI != kDmaRaw) {
 #pragma unroll

@@ -75,13 +75,15 @@ __device__ __forceinline__ void join_blocks(uint32_t (&w)[4 / R][R]) {
 
 // Rows of an output (or a residual) as a tile sees them: 16-byte accesses at byte offsets behind its first row.  What lies behind the last
 // row is neither written nor read (zeros come back), and neither is offset kNowhere: no branch stands around a store, so that
-// loads issued ahead of stores are not waited for together with them.  A tile's rows have to stay below 2 GiB (rows_fit).
+// loads issued ahead of stores are not waited for together with them.  A tile's rows have to stay below 2 GiB (rows_fit): of the rows that are
+// left of the matrix only the tile's own `most` count, all of them can be more bytes than 32 bits say.
 constexpr int kNowhere = -1;
 inline bool rows_fit(int ld, int bytes) { return (size_t)256 * ld * bytes < (1ull << 31); }
 struct TileRows {
     __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ TileRows(void* first_row, int rows, int row_bytes)
-        : r(__builtin_amdgcn_make_buffer_rsrc(first_row, 0, rows > 0 ? rows * row_bytes : 0, 0x00027000)) {}
+    static __host__ __device__ constexpr int bytes(int left, int most, int row_bytes) { return left <= 0 ? 0 : (left < most ? left : most) * row_bytes; }
+    __device__ __forceinline__ TileRows(void* first_row, int left, int most, int row_bytes)
+        : r(__builtin_amdgcn_make_buffer_rsrc(first_row, 0, bytes(left, most, row_bytes), 0x00027000)) {}
     __device__ __forceinline__ void put(const uint32_t* w, int at) const {
         const i32x4 v = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
         __builtin_amdgcn_raw_buffer_store_b128(v, r, at, 0, 0);
@@ -91,6 +93,8 @@ struct TileRows {
         return {__int_as_float(v[0]), __int_as_float(v[1]), __int_as_float(v[2]), __int_as_float(v[3])};
     }
 };
+
+static_assert(TileRows::bytes(65536, 128, 65536) == 128 * 65536 && TileRows::bytes(5, 128, 65536) == 5 * 65536 && TileRows::bytes(-3, 128, 65536) == 0, "bytes of a tile's rows");
 
 // The workgroup's barrier alone: what has to be waited for is waited for explicitly ahead of it.  No memory access moves across it.
 __device__ __forceinline__ void barrier() {

@@ -46,3 +46,22 @@ def test_rows_int8(fx, oracle, rows, k):  # noqa: F811
     m, n = INT[rows, k]
     ints.test_tiles(fx, oracle, m, k, n)
     ints.test_half_line_tiles_with_the_gated_unit(fx, m, k, n)
+
+
+def test_outputs_of_4_gib(fx):  # noqa: F811
+    """The bytes of the rows behind a tile's first one need more than 32 bits: first rows, rows on both sides of 2 GiB, last rows."""
+    import numpy as np
+    from flexllm_amd import synth
+    m, k, n = 65536, 1024, 16384
+    assert fx.lib().flexllm_linear_i8_gemm_rows(m, k, n, 0) == 256      # on the wide tiles
+    a, w = synth.device_i8((m, k), 3), synth.device_i8((n, k), 4)
+    s_x, w_s, res = synth.device_uniform_f32((m,), 5, 0.01, 0.02), synth.device_uniform_f32((n,), 6, 1e-3, 1e-2), synth.device_uniform_f32((m, n), 7, -1, 1)
+    rows = np.r_[0:4, 126:130, 32766:32770, 65404:65412, 65534:65536]
+    ha, hw = a.numpy()[rows].astype(np.float64), w.numpy().astype(np.float64)
+    want = (ha @ hw.T).astype(np.int64).astype(np.int32)
+    some = lambda y: np.stack([y.view(4 * n * int(r), (n,)).numpy() for r in rows])  # noqa: E731
+    acc = fx.ops.linear_i8_gemm(a, w)
+    assert np.array_equal(some(acc), want)
+    del acc
+    y = fx.ops.linear_i8_gemm_dequant(a, s_x, w, w_s, residual=res)
+    assert np.array_equal(some(y), (want.astype(np.float32) * s_x.numpy()[rows, None]) * w_s.numpy() + some(res))
