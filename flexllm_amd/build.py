@@ -2,6 +2,7 @@
 import fcntl
 import glob
 import os
+import re
 import subprocess
 import sys
 
@@ -15,6 +16,7 @@ FLAGS = [
     # the reference's arithmetic has no fused multiply-add: keep mul and add separate
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-Rpass-analysis=kernel-resource-usage",           # read by resources()
     "-Wall", "-Wno-unused-function", *os.environ.get("FLEXLLM_EXTRA_FLAGS", "").split(),
 ]
 
@@ -62,13 +64,47 @@ def build(verbose=False, jobs=8, srcs=None, out=LIB, obj_dir=os.path.join(CSRC, 
     return out
 
 
+# Kernels that count their loads in flight themselves and hold nearly as many sums as there are registers.  They have to do without memory of
+# the compiler's own: a form of the wide GEMMs that spilled sums gave wrong ones on some sizes, for a reason that was not found.
+WITHOUT_SPILLS = ("gemm_float_walk_kernel", "gemm_i8_walk_kernel", "gemm_i8_dma_kernel", "gemm_few_kernel", "gemv_mfma_kernel")
+
+
+def resources(out):
+    """({kernel: {"ScratchSize": bytes per lane, "VGPRs Spill": registers, ...}}, the other lines) of what hipcc prints."""
+    kernels, rest, kernel, remark = {}, [], None, False
+    for line in out.splitlines():
+        if "[-Rpass-analysis=kernel-resource-usage]" in line:
+            remark = True
+            while rest and rest[-1].startswith("In file included from "):
+                rest.pop()
+            name, _, value = line.split("remark:")[1].partition(":")
+            name, value = name.split("[")[0].strip(), value.split("[-R")[0].strip()
+            if name == "Function Name":
+                kernel = kernels.setdefault(value, {})
+            elif value.isdigit():
+                kernel[name] = int(value)
+        elif remark and re.match(r"\s*\d* \| ", line):      # the source line of a remark
+            continue
+        elif "packed-fp32-ops" not in line:
+            remark = False
+            rest.append(line)
+    return kernels, rest
+
+
+def spilled(kernels):
+    """Names of those of `kernels` that must not use memory of the compiler's own and do."""
+    return [n for n, r in kernels.items() if any(k in n for k in WITHOUT_SPILLS) and (r["ScratchSize"] or r["VGPRs Spill"])]
+
+
 def _drain(procs):
     while procs:
         src, p = procs.pop(0)
         out, _ = p.communicate()
-        lines = [l for l in out.splitlines() if "packed-fp32-ops" not in l]
+        kernels, lines = resources(out)
         if p.returncode != 0:
             raise RuntimeError("hipcc failed on %s:\n%s" % (src, "\n".join(lines)))
+        if spilled(kernels):
+            raise RuntimeError("%s: kernels that have to stay in registers do not:\n%s" % (src, "\n".join(spilled(kernels))))
         if lines:
             print("\n".join(lines), file=sys.stderr)
 

@@ -90,7 +90,7 @@ __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias,
 }
 
 // OUT: forms of the outputs that a kernel of tiles of 256 columns is made for (all of them in one are more than its registers hold beside the
-// sums, and spilled sums have come back wrong).  kOutAny: all, at run time.
+// sums, and spilled sums have come back wrong: the build refuses such kernels).  kOutAny: all, at run time.
 enum GemmOut { kOutAny = 0, kOutPlain = 1, kOutBias = 2, kOutClamped = 3, kOutGelu = 4 };
 template <typename ET, class W, int OUT>
 __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_end, int col0, int stores, int8_t* smem, f32x4 (&acc)[W::MIv][W::NIv]) {
