@@ -33,8 +33,7 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
             const int p = wave * PER + q, r = p / (UB / 1024), seg = p % (UB / 1024);
             // what is behind the row's end (any of its bytes will do) is not looked at
             const int kb = min((k0 + h * UK) * 2 + seg * 1024 + (lane ^ r) * 16, g.k * 2 - 16);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                         :: "s"(lds0 + (u % SLOTS) * SLOT + p * 1024), "v"((unsigned)(min(r, last) * g.ldw * 2 + kb)), "s"(base) : "memory");
+            load_to_lds<true>(base, (unsigned)(min(r, last) * g.ldw * 2 + kb), lds0 + (u % SLOTS) * SLOT + p * 1024);
         }
     };
     bf16x8 af[UNITS * SW][NG];

@@ -104,6 +104,16 @@ __device__ __forceinline__ void barrier() {
     asm volatile("" ::: "memory");
 }
 
+// A direct load, global -> LDS: 16 bytes per lane from byte `off` behind base, to 16 bytes per lane from LDS address `to` on, which the
+// instruction takes from m0 (one wait state after it was written).  m0 is an output, so that the compiler knows that what it may have there itself
+// is gone.  ONCE: read once on this chip.
+template <bool ONCE = false>
+__device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsigned to) {
+    unsigned m0;
+    if constexpr (ONCE) asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3 nt" : "=&{m0}"(m0) : "s"(to), "v"(off), "s"(base) : "memory");
+    else asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" : "=&{m0}"(m0) : "s"(to), "v"(off), "s"(base) : "memory");
+}
+
 template <typename ET, int WM, int MI, int NI, int NA, int NB>
 struct GemmWalk {
     using Op = MatrixOp<ET>;
@@ -156,13 +166,16 @@ struct GemmWalk {
         const int lane = threadIdx.x & 63, wv = wave();
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
         const unsigned lds_a = lds0 + wv * (AI * 1024), lds_b = lds0 + NA * ASZ + wv * (BI * 1024);
-        // A direct load takes its LDS address from m0.  In two halves, with a matrix instruction between them: the address has to be
-        // in m0 one wait state ahead of the load.  Nothing else in this loop uses m0.
-        auto aim = [&](unsigned base, int j) __attribute__((always_inline)) { asm volatile("s_add_u32 m0, %0, %1" :: "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc"); };
-        auto load = [&](const int8_t* p, unsigned off) __attribute__((always_inline)) { asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p) : "memory"); };
+        // A direct load in two halves, with a matrix instruction between them: the address has to be in m0 one wait state ahead of the load.
+        // What `aim` leaves in m0 is an operand of `load`, so that the compiler puts nothing of its own there between them.
+        unsigned m0 = 0;
+        auto aim = [&](unsigned base, int j) __attribute__((always_inline)) {
+            asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(m0) : "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc");
+        };
+        auto load = [&](const int8_t* p, unsigned off) __attribute__((always_inline)) { asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p), "{m0}"(m0) : "memory"); };
         auto load_now = [&](const int8_t* p, unsigned off, unsigned base, int j) __attribute__((always_inline)) {
             aim(base, j);
-            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p) : "memory");
+            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p), "{m0}"(m0) : "memory");
         };
 #pragma unroll
         for (int i = 0; i < MI; i++)

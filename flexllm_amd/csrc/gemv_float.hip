@@ -394,11 +394,6 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
     const int tok0 = blockIdx.y * group, nt = min(group, tokens - tok0), k0 = part * STRETCH, tiles = (g.n + 15) / 16;
     const int mine = (tiles - walker + walkers - 1) / walkers, total = mine * UNITS;          // tiles and units of this workgroup
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)ring;
-    // the weights are read once on this chip, the vectors by every workgroup
-    auto request = [&](const void* base, unsigned off, unsigned to, auto once) __attribute__((always_inline)) {
-        if constexpr (decltype(once)::value) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" :: "s"(to), "v"(off), "s"(base) : "memory");
-        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(to), "v"(off), "s"(base) : "memory");
-    };
     auto request_unit = [&](int u) __attribute__((always_inline)) {
         const int tile = walker + u / UNITS * walkers, h = u % UNITS, last = min(16, g.n - tile * 16) - 1;
         const int8_t* base = static_cast<const int8_t*>(g.w) + (size_t)tile * 16 * g.kpad * 2;
@@ -407,7 +402,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
             const int p = wave * PER + q, r = p / (UB / 1024), seg = p % (UB / 1024);
             // what is behind the row's end (any of its bytes will do) meets zeros
             const int kb = min((k0 + h * UK) * 2 + seg * 1024 + (lane ^ r) * 16, g.kpad * 2 - 16);
-            request(base, (unsigned)(min(r, last) * g.kpad * 2 + kb), lds0 + (u % SLOTS) * SLOT + p * 1024, std::true_type());
+            load_to_lds<true>(base, (unsigned)(min(r, last) * g.kpad * 2 + kb), lds0 + (u % SLOTS) * SLOT + p * 1024);      // the vectors are read by every workgroup
         }
     };
     // a wave's vectors [token][SL], in the last place's part that only this wave's requests write
@@ -418,7 +413,7 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
 #pragma unroll
         for (int i = 0; i < XN; i++) {
             const int c = i * 64 + lane, j = min(c / XC, nt - 1), k = k0 + h * UK + wave * SL + c % XC * 4;
-            if (i * 64 < nt * XC) request(g.x + (size_t)tok0 * g.ldx, (unsigned)(j * g.ldx + min(k, g.k - 4)) * 4u, lds0 + (unsigned)(xs - ring) + i * 1024, std::false_type());
+            if (i * 64 < nt * XC) load_to_lds(g.x + (size_t)tok0 * g.ldx, (unsigned)(j * g.ldx + min(k, g.k - 4)) * 4u, lds0 + (unsigned)(xs - ring) + i * 1024);
         }
     };
     // The instruction has 16 columns for at most 8 tokens: columns 0 to 7 are the tokens' first and third part, 8 to 15 their second.

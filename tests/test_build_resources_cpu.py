@@ -52,3 +52,12 @@ a.hip:9:1: error: other"""
     kernels, rest = build.resources(out)
     assert kernels == {"gemm_few_kernel": {"ScratchSize": 16, "VGPRs Spill": 4}} and build.spilled(kernels) == ["gemm_few_kernel"]
     assert rest == out.splitlines()[:4] + ["a.hip:9:1: error: other"]
+
+
+def test_the_compiler_knows_who_writes_m0():
+    """m0 has the LDS address of a direct load: a statement that writes it puts back what was there, or names it among its operands."""
+    for f in glob.glob(os.path.join(build.CSRC, "*")):
+        if f.endswith((".h", ".hip")):
+            for asm in re.findall(r"\basm volatile\((.*?)\);", open(f).read(), re.S):
+                if "global_load_lds" in asm or re.search(r"\bm0\b", asm):
+                    assert "{m0}" in asm or ("s_mov_b32 %0, m0" in asm and "s_mov_b32 m0, %0" in asm), (f, asm)
