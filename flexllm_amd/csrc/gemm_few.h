@@ -117,10 +117,18 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
 
 // k of a part, in units of 64.
 inline int gemm_few_len(int k, int parts) { return ((k / 64 + parts - 1) / parts) * 64; }
-// Products of at most 32 rows run here where a workgroup has two tiles or more: their weights' stream is long enough to pay for the
-// start (A into registers) and the sums.  The tiles of the wide GEMMs and this, us: 16384 x 2048, 9 rows 17.6 and 13.2, 32 rows 18.0 and
-// 16.3; 28672 x 4096 51 and 38, 51 and 44; 2560 x 2048 5.8 and 5.4, 6.2 and 7.3 (stays); two passes over the weights for 41 rows 18.0 and 23.8.
-inline bool gemm_few_ok(int m, int k, int n, int parts) { return m <= kFewMost && parts == 1 && k <= 4096 && n >= 8192; }
+// Products of at most 32 rows run here where a workgroup has two tiles or more, so that their weights' stream is long enough to pay for
+// the start (A into registers) and the sums, and where k fills the units: a place in the ring that is half empty is half as much in flight, and an
+// instruction on nothing takes as long as another.  The tiles of the wide GEMMs and this, us: 16384 x 2048, 9 rows 17.6 and 13.8, 32 rows 18.0 and 16.9; 28672 x
+// 4096 53 and 38, 53 and 44; 8192 x 512, 16 rows 6.3 and 5.2, 32 rows 6.5 and 6.4 (stays).  Units that are not full: 12300 x 3072, 16 rows 18.6 and 17.6, 17 rows
+// 19.0 and 20.1 (stays); 20480 x 2112, 16 rows 19.3 and 21.0 (stays); 16384 x 1088, 32 rows 10.2 and 12.2 (stays).  k below 512: 8192 x 64, 16 rows
+// 3.9 and 5.0 (stays).  Over 240 sizes of 8 to 32 rows, 64 to 4096 k and 8192 to 28672 columns the choice is 1.1 % from the better one on average, and at
+// most 1.6 % behind the tiles.
+inline bool gemm_few_ok(int m, int k, int n, int parts) {
+    if (m > kFewMost || parts != 1 || k > 4096 || n < 8192) return false;
+    const int units = k <= 1024 ? 1024 : k <= 2048 ? 2048 : 4096;
+    return m <= 16 ? k >= 512 && (k <= 1024 || k * 4 >= units * 3) : k > 1024 && k * 8 >= units * 7;
+}
 
 template <int UK, int UNITS, int NG>
 static int launch_few(const GemmArgs& g, hipStream_t st) {
@@ -141,7 +149,7 @@ static int launch_few(const GemmArgs& g, hipStream_t st) {
 inline int gemm_few(const GemmArgs& g, hipStream_t st) {
     const int len = gemm_few_len(g.k, g.parts);
     if (g.m <= 16) return len <= 1024 ? launch_few<1024, 1, 1>(g, st) : len <= 2048 ? launch_few<2048, 1, 1>(g, st) : launch_few<2048, 2, 1>(g, st);
-    return len <= 1024 ? launch_few<1024, 1, 2>(g, st) : len <= 2048 ? launch_few<2048, 1, 2>(g, st) : launch_few<2048, 2, 2>(g, st);
+    return len <= 2048 ? launch_few<2048, 1, 2>(g, st) : launch_few<2048, 2, 2>(g, st);
 }
 
 }  // namespace fx

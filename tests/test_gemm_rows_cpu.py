@@ -25,5 +25,10 @@ def test_few_rows_are_one_pass():
     from flexllm_amd import lib
     import test_gpu_gemm_few as few
     f = lambda m, k, n, parts=1: lib().flexllm_linear_float_gemm_rows(m, k, n, 0, parts)  # noqa: E731
-    assert all(f(m, k, n) == (16 if m <= 16 else 32) for m, n in few.FEW for k in few.K)
+    for m, n in few.FEW:
+        rows = 16 if m <= 16 else 32
+        assert all(f(m, k, n) == rows for k in few.FILLED[rows])
+        # units that k does not fill, and short ones, cost more than the tiles' stages (5 to 50 % more)
+        assert all(f(m, k, n) == 64 for k in (64, 448, 1088, 2112, 3008))
+    assert f(17, 1024, 16384) == f(32, 1536, 8192) == f(32, 3520, 8192) == 64
     assert f(33, 2048, 16384) == f(9, 4160, 16384) == f(9, 2048, 8188) == f(9, 2048, 16384, 2) == 64
