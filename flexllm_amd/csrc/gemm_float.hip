@@ -150,6 +150,7 @@ struct FloatWalk : GemmWalk<ET, WM, MI, NI, NA, NB> { static constexpr int MIv =
 template <typename ET, class W, int OUT>
 __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmArgs g, int tiles_m, int tiles_n, int stores) {
     extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
+    if constexpr (!W::kSumsApart) arguments(g.a, g.w, g.lda, g.ldw, g.m, g.n, g.k, g.row_src, g.tiles, g.n_tiles, g.w_stride, g.parts, g.part_stride, tiles_m, tiles_n);
     int tm, tn, group = 0, row0, row_end;
     gemm_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
     if (g.tiles) {
@@ -160,9 +161,13 @@ __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmA
         row0 = tm * W::BM; row_end = min(g.m, row0 + W::BM);
     }
     const int col0 = tn * W::BN;
-    // scalar registers for the ends of the part: divisions are made in vector ones, and the loop would carry them along
     const int part = blockIdx.y, stages = g.k * (int)sizeof(ET) / 128;
-    const int k0 = __builtin_amdgcn_readfirstlane(part * stages / g.parts), k1 = __builtin_amdgcn_readfirstlane((part + 1) * stages / g.parts);
+    int k0 = 0, k1 = stages;
+    if (g.parts > 1) {
+        // scalar registers: divisions are made in vector ones, and the loop would carry them along
+        k0 = __builtin_amdgcn_readfirstlane(part * stages / g.parts);
+        k1 = __builtin_amdgcn_readfirstlane((part + 1) * stages / g.parts);
+    }
     g.y32 += part * g.part_stride;
     unsigned offa[W::AI], offb[W::BI];
 #pragma unroll

@@ -49,13 +49,19 @@ __device__ __forceinline__ void wait_vmcnt() {                 // s_waitcnt vmcn
 // The tile of workgroup `id`.  Ids go to the eight dies in turn, each with an L2 of its own: of every 256 tiles (a round over the chip) a
 // die takes 32 in a row, which are eight row tiles by four column tiles.  They read 12 stages of rows per stage where 32 row
 // tiles by one column tile read 33.
+// Quotients stand ahead of the first load, so they are float ones put right by the remainder (exact: a quotient of tiles is below 2^20, and the
+// float one below half off); a division of integers takes three times the instructions.
+__device__ __forceinline__ int quotient(int a, int d) {
+    const int q = (int)((float)a * __builtin_amdgcn_rcpf((float)d)), r = a - q * d;
+    return __builtin_amdgcn_readfirstlane(q + (r >= d) - (r < 0));
+}
 __device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
     const int total = tiles_m * tiles_n, round = id & ~255, in = id & 255, left = min(total - round, 256), die = in & 7;
     const int t = round + die * (left >> 3) + min(die, left & 7) + (in >> 3);
     constexpr int G = 8;
-    const int group = t / (G * tiles_n), rows = min(G, tiles_m - group * G), o = t - group * G * tiles_n;
-    tm = group * G + o % rows;
-    tn = o / rows;
+    const int group = tiles_m <= G ? 0 : quotient(t, G * tiles_n), rows = min(G, tiles_m - group * G), o = t - group * G * tiles_n;
+    tn = rows == G ? o / G : quotient(o, rows);
+    tm = group * G + o - tn * rows;
 }
 
 // R words of each of 4/R blocks, as lanes hold them (lane group g of 16 lanes has words g*R .. g*R + R - 1 of a block's row), become four
@@ -95,6 +101,16 @@ struct TileRows {
 };
 
 static_assert(TileRows::bytes(65536, 128, 65536) == 128 * 65536 && TileRows::bytes(5, 128, 65536) == 5 * 65536 && TileRows::bytes(-3, 128, 65536) == 0, "bytes of a tile's rows");
+
+// A kernel's arguments come from memory, and each group of them that is asked for behind a branch or an index is a trip of its own ahead of
+// the first load.  Values that stand here are in scalar registers from here on, so that they are asked for together at the start
+// (three trips one after the other before, us: 24 x 8192 x 512 5.81 and 5.48, 41 x 2560 x 2048 9.41 and 9.11; the two trips of the wide tiles stay, with the
+// arguments in registers their sums do not fit).
+template <typename... T>
+__device__ __forceinline__ void arguments(const T&... v) {
+    auto one = [](const auto& x) __attribute__((always_inline)) { asm volatile("" :: "s"(x)); };
+    (one(v), ...);
+}
 
 // The workgroup's barrier alone: what has to be waited for is waited for explicitly ahead of it.  No memory access moves across it.
 __device__ __forceinline__ void barrier() {

@@ -32,3 +32,20 @@ def test_few_rows_are_one_pass():
         assert all(f(m, k, n) == 64 for k in (64, 448, 1088, 2112, 3008))
     assert f(17, 1024, 16384) == f(32, 1536, 8192) == f(32, 3520, 8192) == 64
     assert f(33, 2048, 16384) == f(9, 4160, 16384) == f(9, 2048, 8188) == f(9, 2048, 16384, 2) == 64
+
+
+def test_quotients_of_tile_numbers():
+    """A workgroup's tile by float quotients put right by the remainder (gemm_walk.h): exact for every number of tiles that a call can
+    have, wherever within an ulp the reciprocal lies."""
+    import numpy as np
+    r = np.random.default_rng(1)
+    d = np.concatenate([np.arange(1, 300), np.exp(r.uniform(0, np.log(2.0 ** 21), 4000)).astype(np.int64)])
+    q = np.exp(r.uniform(0, np.log(2.0 ** 18), len(d))).astype(np.int64)
+    for off in (-1, 0, 1):
+        a = np.clip(q * d + off, 0, 2 ** 31 - 1)
+        inv = np.float32(1) / d.astype(np.float32)
+        for rcp in (inv, np.nextafter(inv, np.float32(0)), np.nextafter(inv, np.float32(2))):
+            got = (a.astype(np.float32) * rcp).astype(np.int64)
+            rest = a - got * d
+            got += (rest >= d).astype(np.int64) - (rest < 0)
+            assert np.array_equal(got, a // d)
