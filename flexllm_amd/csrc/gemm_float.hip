@@ -89,24 +89,79 @@ __device__ __forceinline__ void gemm_out_wide(OT* y, int ldy, const float* bias,
     }
 }
 
+// Outputs of any form: up to 64 columns of the wave's rows at a time turn through LDS, so that a loop can take them and lanes side by side store what
+// is side by side.  (Before, a loop of a lane's own four columns: sixteen rows per store.)
+template <typename ET, class W>
+__device__ __forceinline__ void gemm_out_loose(const GemmArgs& g, int row0, int row_end, int col0, int stores, int8_t* smem, f32x4 (&acc)[W::MIv][W::NIv]) {
+    constexpr int MI = W::MIv, NI = W::NIv, J = NI < 4 || 4 * MI * 16 * 68 * 4 > W::kLds ? 2 : 4, C = J * 16, P = C + 4;      // P: of 16 rows no two begin on the same banks
+    static_assert(NI % J == 0 && 4 * MI * 16 * P * 4 <= W::kLds, "a patch per wave");
+    const int lane = threadIdx.x & 63, fg = lane >> 4, fr = lane & 15, rows = min(MI * 16, row_end - row0);
+    __syncthreads();                                           // the walk has left LDS behind in this wave alone
+    float* const patch = reinterpret_cast<float*>(smem) + W::wave() * (MI * 16 * P);
+    auto settled = []() __attribute__((always_inline)) {       // a wave's own LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+#pragma unroll
+    for (int j0 = 0; j0 < NI; j0 += J) {
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < MI; i++) *reinterpret_cast<f32x4*>(patch + (i * 16 + fr) * P + j * 16 + fg * 4) = acc[i][j0 + j];
+        settled();
+        if (stores == kSingle && !g.glu) {
+            constexpr int R = 64 / C;
+            const int c = lane % C, col = col0 + j0 * 16 + c;
+            const float b = g.bias ? g.bias[min(col, g.n - 1)] : 0.0f;
+            auto each = [&](auto* to, int ld) __attribute__((always_inline)) {
+#pragma unroll 4
+                for (int r = lane / C; r < rows; r += R) {
+                    float v = patch[r * P + c];
+                    if (g.bias) v += b;
+                    to[(size_t)r * ld] = v;
+                }
+            };
+            if (col < g.n_split) each(static_cast<ET*>(g.y) + (size_t)row0 * g.ldy + col, g.ldy);
+            else if (col < g.n) each(g.y32 + (size_t)row0 * g.ldy32 + (col - g.n_split), g.ldy32);
+        } else {
+            constexpr int L = C / 4, R = 64 / L;
+            const int c = lane % L * 4, col = col0 + j0 * 16 + c;
+            f32x4 b = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (g.bias)
+#pragma unroll
+                for (int e = 0; e < 4; e++) b[e] = g.bias[min(col + e, g.n - 1)];
+#pragma unroll 2
+            for (int r = lane / L; r < rows; r += R) {
+                f32x4 q = *reinterpret_cast<const f32x4*>(patch + r * P + c);
+                if (g.bias) q += b;
+                float v[4] = {q[0], q[1], q[2], q[3]};
+                gemm_store4<ET>(g, row0 + r, col, v, stores != kSingle);
+            }
+        }
+        settled();
+    }
+}
+
 // OUT: forms of the outputs that a kernel of tiles of 256 columns is made for (all of them in one are more than its registers hold beside the
-// sums, and spilled sums have come back wrong: the build refuses such kernels).  kOutAny: all, at run time.
-enum GemmOut { kOutAny = 0, kOutPlain = 1, kOutBias = 2, kOutClamped = 3, kOutGelu = 4 };
+// sums, and spilled sums have come back wrong: the build refuses such kernels).  kOutAny: all, at run time; kOutLoose: what does not leave in
+// whole 16-byte pieces.
+enum GemmOut { kOutAny = 0, kOutPlain = 1, kOutBias = 2, kOutClamped = 3, kOutGelu = 4, kOutLoose = 5 };
 template <typename ET, class W, int OUT>
 __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_end, int col0, int stores, int8_t* smem, f32x4 (&acc)[W::MIv][W::NIv]) {
-    constexpr int NI = W::NIv, MI = W::MIv, J = std::is_same<ET, float>::value ? 2 : 4;
-    const int lane = threadIdx.x & 63, fg = lane >> 4, fr = lane & 15, end = col0 + NI * 16;
+    constexpr int NI = W::NIv, J = std::is_same<ET, float>::value ? 2 : 4;
+    const int end = col0 + NI * 16;
     const float* bias = g.bias + col0;
     ET* const y = static_cast<ET*>(g.y);
     float* const y32 = g.y32 + (col0 - g.n_split);
     const int cols = g.n_split - col0, cols32 = g.n - col0;
     if constexpr (OUT == kOutClamped || OUT == kOutGelu) {
         return gemm_out_wide<ET, W, OUT == kOutGelu ? kGluGelu : kGluClamped, false>(y + (col0 >> 1), g.ldy, nullptr, g.limit, row0, row_end, cols, acc);
-    } else if constexpr (OUT != kOutAny) {
+    } else if constexpr (OUT == kOutPlain || OUT == kOutBias) {
         if (col0 >= g.n_split) gemm_out_wide<float, W, 0, OUT == kOutBias>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
         else gemm_out_wide<ET, W, 0, OUT == kOutBias>(y + col0, g.ldy, bias, 0.0f, row0, row_end, cols, acc);
         return;
-    } else {
+    } else if constexpr (OUT == kOutAny) {
         if (stores == kWide && col0 >= g.n_split) {
             if (g.bias) return gemm_out_wide<float, W, 0, true>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
             return gemm_out_wide<float, W, 0, false>(y32, g.ldy32, bias, 0.0f, row0, row_end, cols32, acc);
@@ -120,28 +175,7 @@ __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_en
             }
         }
     }
-    // Any other: sixteen columns of the wave's rows at a time through LDS, so that a loop can take them (the walk has left it behind: the
-    // barrier is for the other waves' reads).
-    __syncthreads();
-    float* patch = reinterpret_cast<float*>(smem) + W::wave() * (MI * 256);
-    f32x4* mine = reinterpret_cast<f32x4*>(patch) + lane;
-#pragma unroll
-    for (int j = 0; j < NI; j++) {
-#pragma unroll
-        for (int i = 0; i < MI; i++) mine[i * 64] = acc[i][j];          // a lane reads back what it wrote
-#pragma clang loop unroll(disable)
-        for (int i = 0; i < MI; i++) {
-            const int row = row0 + i * 16 + fr;
-            const f32x4 q = mine[i * 64];
-            const int col = col0 + j * 16 + fg * 4;
-            float v[4] = {q[0], q[1], q[2], q[3]};
-            if (g.bias) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[e] += g.bias[min(col + e, g.n - 1)];
-            }
-            if (row < row_end) gemm_store4<ET>(g, row, col, v, stores != kSingle);
-        }
-    }
+    gemm_out_loose<ET, W>(g, row0, row_end, col0, stores, smem, acc);
 }
 
 template <typename ET, int WM, int MI, int NI, int NA, int NB>
@@ -198,7 +232,8 @@ static int gemm_stores(const GemmArgs& g) {
                       ((reinterpret_cast<uintptr_t>(g.y) | reinterpret_cast<uintptr_t>(g.y32)) & 15) == 0;
     return wide ? kWide : kQuad;
 }
-// Tiles of 256 columns know no other way; a wave's 128 columns lie on one side of the split, and with a gated unit there is only one.
+// Tiles of 256 columns have kernels of their own for these forms; a wave's 128 columns lie on one side of the split, and with a gated unit there is
+// only one.
 static bool gemm_wide_ok(const GemmArgs& g) {
     return gemm_stores<bf16_t>(g) == kWide && (g.n_split == g.n || (!g.glu && g.n_split % 128 == 0)) && !(g.bias && g.glu);
 }
@@ -219,6 +254,7 @@ template <typename ET, int WM, int MI, int NI, int NA, int NB>
 static int launch_walk(const GemmArgs& g, hipStream_t st) {
     using W = FloatWalk<ET, WM, MI, NI, NA, NB>;
     if constexpr (W::kSumsApart) {
+        if (!gemm_wide_ok(g)) return launch_walk_out<ET, W, kOutLoose>(g, st);
         if (g.glu == kGluClamped) return launch_walk_out<ET, W, kOutClamped>(g, st);
         if (g.glu == kGluGelu) return launch_walk_out<ET, W, kOutGelu>(g, st);
         return g.bias ? launch_walk_out<ET, W, kOutBias>(g, st) : launch_walk_out<ET, W, kOutPlain>(g, st);
@@ -359,8 +395,7 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
     if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
-        case 0: case 1: switch (gemm_wide_ok(g) ? gemm_wide_rows(g.m, g.k, g.n, g.parts) : 0) {
-            case 0: return launch_walk<bf16_t, 2, 4, 4, 2, 2>(g, st);
+        case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
             case 256: return launch_walk<bf16_t, 2, 8, 8, 3, 2>(g, st);
             case 224: return launch_walk<bf16_t, 2, 7, 8, 3, 2>(g, st);
             case 192: return launch_walk<bf16_t, 2, 6, 8, 3, 2>(g, st);

@@ -614,7 +614,7 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
                               int dtype, void* stream);
 /* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
 int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
-/* The rows that a workgroup takes, as flexllm_linear_i8_gemm_rows (where the outputs leave in whole 16-byte pieces), or 16 or 32 where few rows of a long bfloat16 product are one pass over the
+/* The rows that a workgroup takes, as flexllm_linear_i8_gemm_rows, or 16 or 32 where few rows of a long bfloat16 product are one pass over the
  * weights without tiles; parts: 1, or those that k is shared out in.  Needs no GPU. */
 int flexllm_linear_float_gemm_rows(int m, int k, int n, int dtype, int parts);
 /* Parts (at most `most`) that k of such a product is shared out in where its reader adds the parts' sums up; negative: an error code.

@@ -19,9 +19,44 @@ INT = {(128, 1152): (300, 12284), (160, 1152): (1558, 6144), (192, 1152): (1632,
 @pytest.mark.parametrize("split,glu", [("all", 0), ("all", 1), ("all", 2), ("half", 0), ("half", 2), ("none", 0), ("odd", 0)])
 @pytest.mark.parametrize("rows", FLOAT)
 def test_rows_bfloat16(rows, split, glu, k):
-    """Outputs on either side of a split between waves; a split inside a wave's columns goes to other tiles."""
+    """Outputs on either side of a split between waves, and of one inside a wave's columns."""
     m, n = FLOAT[rows]
     floats.test_gemm_tiles(m, n, {"all": n, "half": n // 512 * 256 + 128, "none": 0, "odd": n // 512 * 256 + 64}[split], glu, k, "bfloat16")
+
+
+# outputs that do not leave in whole 16-byte pieces: one by one, four at a time, a unit's in both ways, on two sides of a split inside four columns
+@pytest.mark.parametrize("cut,split,glu", [(13, None, 0), (4, None, 0), (10, None, 1), (8, None, 2), (6, 3002, 0), (4, 3004, 2), (13, 3001, 0)])
+@pytest.mark.parametrize("rows", FLOAT)
+def test_rows_bfloat16_in_pieces(rows, cut, split, glu):
+    m, n = FLOAT[rows]
+    n = (n + 255) // 256 * 256 - cut
+    from flexllm_amd import lib
+    assert lib().flexllm_linear_float_gemm_rows(m, 320, n, 0, 1) == rows
+    floats.test_gemm_tiles(m, n, n if split is None else split, glu, 320, "bfloat16")
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("m,n,split,glu", [(129, 771, 771, 0), (129, 770, 770, 1), (70, 515, 258, 0), (300, 2049, 1025, 0), (1300, 331, 331, 0), (33, 70, 35, 0),
+                                           (2100, 1030, 1030, 2), (2600, 2053, 2053, 0), (1300, 1924, 964, 2)])
+def test_small_tiles_in_pieces(m, n, split, glu, dtype):
+    floats.test_gemm_tiles(m, n, split, glu, 320, dtype)
+
+
+@pytest.mark.parametrize("rows,m,n", [(r, *FLOAT[r]) for r in FLOAT] + [(0, 129, 772), (0, 1300, 330), (0, 40, 132)])
+@pytest.mark.parametrize("cut", [0, 2])
+def test_unit_behind_a_bias(rows, m, n, cut):
+    import numpy as np
+    import lopazen_cases as lc
+    from flexllm_amd import ops, to_device
+    from flexllm_amd.loader import from_bf16, to_bf16
+    from oracle import lopazen_ref
+    n, k, r = n - cut, 320, np.random.default_rng(rows + m)
+    a, w, bias = lc.round_bf16(r.standard_normal((m, k))), lc.round_bf16(r.standard_normal((n, k))), r.standard_normal(n).astype(np.float32)
+    y = from_bf16(ops.linear_float(to_device(to_bf16(a)), to_device(to_bf16(w)), n, 2, bias=to_device(bias))[0].numpy())
+    want = a.astype(np.float64) @ w.astype(np.float64).T + bias
+    g, u = want[:, 0::2], want[:, 1::2]
+    first, d = lopazen_ref.gelu(g) * u, 1e-5 * np.sqrt(k)      # bounds as for the tiles
+    assert np.all(np.abs(y - first) <= 5e-3 * np.abs(first) + d * (1.2 * (np.abs(u) + 1) + np.abs(g)))
 
 
 @pytest.mark.parametrize("rows", FLOAT)
