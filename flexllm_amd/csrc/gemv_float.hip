@@ -379,13 +379,18 @@ static int gemv_tokens(const GemvArgs& g, int tokens, hipStream_t st) {
 // unit's place is free for the next but one as soon as its operands are in registers.  The vectors' parts stay in registers, each wave's
 // own stretch of k.
 // Before (operands straight from memory) and now, 5 tokens, us: 16384 x 2048 21.5 and 14.4, 2048 x 8192 13.2 and 9.3, 28672 x 4096 49.8 and
-// 39.6 (8 tokens 81 and 44), 4096 x 14336 28.0 and 21.0, 2560 x 2048 6.7 and 6.6, 2048 x 2048 4.9 and 5.2.  What the last two are made of: 2 us
-// until the vectors are in and taken apart, 1.5 more until the first unit is, 1 for the sums' way through LDS.
+// 39.6 (8 tokens 81 and 44), 4096 x 14336 28.0 and 21.0.
+// ONE: where a workgroup has one tile of one unit there is no stream, only a chain of trips, and the weights come to registers in the operands' own
+// shape: asked for together with the vectors they are a trip less than through LDS.  us, 5 tokens, before the stream through LDS, on it, now: 2048 x 2048 7.2, 6.7,
+// 5.9, in two parts 5.3, 5.7, 4.8; 4096 x 2048 8.0, 7.5, 6.8; 1024 x 1024 4.9, 5.1, 4.5; 4000 x 1088 6.4, 6.6, 6.1; 4096 x 256 4.2, 5.1, 4.5 (what is left there is
+// that each wave takes its vectors apart by itself, and at k of 256 two of eight have any).
 constexpr int kMfmaTokens = 8, kMfmaWaves = 8;
-template <int UK, int UNITS>
+template <int UK, int UNITS, bool ONE>
 __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs g, int tokens, int group) {
+    static_assert(!ONE || UNITS == 1, "ONE: a workgroup has one tile of one unit at most");
+    arguments(g.w, g.x, g.n, g.k, g.kpad, g.ldx, g.parts, tokens, group, gridDim.x);
     constexpr int STRETCH = UK * UNITS, SW = UK / kMfmaWaves / 32, SL = UK / kMfmaWaves;      // matrix k-steps and k of a wave in a unit
-    constexpr int UB = UK * 2, SLOT = 16 * UB, SLOTS = 128 * 1024 / SLOT, PER = SLOT / 1024 / kMfmaWaves;   // PER: requests of a wave per unit
+    constexpr int UB = UK * 2, SLOT = 16 * UB, SLOTS = ONE ? 1 : 128 * 1024 / SLOT, PER = SLOT / 1024 / kMfmaWaves;   // PER: requests of a wave per unit
     static_assert(kMfmaTokens * SL * 4 <= PER * 1024, "a wave's vectors fit into its part of a unit's place");
     extern __shared__ __attribute__((aligned(16))) int8_t ring[];
     __shared__ float red[2][kMfmaWaves][16 * 17];
@@ -422,18 +427,30 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
     constexpr int JI = 64 / XC;                               // tokens that a round of the wave's lanes covers
     const int put0 = ((((lane % XC) >> 1) ^ (lane / XC)) << 4) + (lane & 1) * 8 + lane / XC * (SL * 2), row0 = second * kMfmaTokens + j0;
     const int8_t* const get0 = xs + row0 * (SL * 2);
+    bf16x8 direct[ONE ? SW : 1];
     auto take_vectors = [&](int h) __attribute__((always_inline)) {
         const int first = k0 + h * UK + wave * SL;            // k of the wave's stretch
         f32x4 v[XN];
+        auto row_of = [&](int i) __attribute__((always_inline)) { return g.x + (size_t)(tok0 + min(i * JI + lane / XC, nt - 1)) * g.ldx; };
+        if (vec) {
 #pragma unroll
-        for (int i = 0; i < XN; i++) {
-            if (i * JI >= nt) break;
-            if (vec) {
-                v[i] = *reinterpret_cast<const f32x4*>(xs + (i * 64 + lane) * 16);
-            } else {
-                const float* x = g.x + (size_t)(tok0 + min(i * JI + lane / XC, nt - 1)) * g.ldx;
-                for (int e = 0; e < 4; e++) v[i][e] = x[min(first + lane % XC * 4 + e, g.k - 1)];
+            for (int i = 0; i < XN; i++) {
+                if (i * JI >= nt) break;
+                v[i] = ONE ? *reinterpret_cast<const f32x4*>(row_of(i) + min(first + lane % XC * 4, g.k - 4)) : *reinterpret_cast<const f32x4*>(xs + (i * 64 + lane) * 16);
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < XN; i++) {
+                if (i * JI >= nt) break;
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[i][e] = row_of(i)[min(first + lane % XC * 4 + e, g.k - 1)];
+            }
+        }
+        if constexpr (ONE) {
+            const bf16_t* row = static_cast<const bf16_t*>(g.w) + (size_t)min(walker * 16 + (lane & 15), g.n - 1) * g.kpad;
+#pragma unroll
+            for (int s = 0; s < SW; s++) direct[s] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(row + min(first + s * 32 + gq * 8, g.kpad - 8)));
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (first + SL > g.k) {
 #pragma unroll
@@ -477,23 +494,27 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
         }
     };
     auto all_read = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
-    if (vec) request_vectors(0);
+    if constexpr (ONE) {
+        take_vectors(0);
+    } else {
+        if (vec) request_vectors(0);
 #pragma unroll
-    for (int u = 0; u < SLOTS - 1; u++)
-        if (u < total) request_unit(u);
-    if (vec) {
-        if (total >= SLOTS - 1) wait_vmcnt<(SLOTS - 1) * PER>();
-        else if (total == 2) wait_vmcnt<2 * PER>();
-        else wait_vmcnt<PER>();
-    }
-    take_vectors(0);
-    if constexpr (UNITS == 2) {
+        for (int u = 0; u < SLOTS - 1; u++)
+            if (u < total) request_unit(u);
+        if (vec) {
+            if (total >= SLOTS - 1) wait_vmcnt<(SLOTS - 1) * PER>();
+            else if (total == 2) wait_vmcnt<2 * PER>();
+            else wait_vmcnt<PER>();
+        }
+        take_vectors(0);
+        if constexpr (UNITS == 2) {
+            all_read();
+            if (vec) { request_vectors(1); wait_vmcnt<0>(); }
+            take_vectors(1);
+        }
         all_read();
-        if (vec) { request_vectors(1); wait_vmcnt<0>(); }
-        take_vectors(1);
+        if (SLOTS - 1 < total) request_unit(SLOTS - 1);
     }
-    all_read();
-    if (SLOTS - 1 < total) request_unit(SLOTS - 1);
     // Not a number may be of the parts' own making, where an infinite weight meets parts of zero or of both signs (or, behind the row's
     // end, zeros) or a value is infinite: the same sum with a float32 product per weight has the right of it.
     auto whole = [&](int row, int j) __attribute__((always_inline)) {
@@ -520,6 +541,17 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
             else if ((row & 1) == 0) g.out[(size_t)tok * g.ldo + (row >> 1)] = glu_f(g.glu, sum(0), sum(1), g.limit);
         }
     };
+    if constexpr (ONE) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < SW; s++)
+#pragma unroll
+            for (int p = 1; p >= 0; p--) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(direct[s], xf[s][p], acc, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[0][wave][(gq * 4 + e) * 17 + (lane & 15)] = acc[e];
+        __syncthreads();
+        return finish(0);
+    }
     const int8_t* const mine_in = ring + (lane & 15) * UB;
     for (int i = 0; i < mine; i++) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -556,21 +588,27 @@ __global__ __launch_bounds__(kMfmaWaves * 64, 2) void gemv_mfma_kernel(GemvArgs 
     finish(mine - 1);
 }
 
-template <int UK, int UNITS>
-static int launch_gemv_mfma(const GemvArgs& g, int tokens, hipStream_t st) {
-    constexpr int lds = 128 * 1024;
+template <int UK, int UNITS, bool ONE>
+static int launch_gemv_mfma(const GemvArgs& g, int tokens, int walkers, int groups, hipStream_t st) {
+    constexpr int lds = ONE ? UK * 32 : 128 * 1024;
     static std::atomic<bool> opted_in{false};
     if (!opted_in.load(std::memory_order_acquire)) {
-        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mfma_kernel<UK, UNITS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mfma_kernel<UK, UNITS, ONE>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         opted_in.store(true, std::memory_order_release);
     }
-    const int groups = (tokens + kMfmaTokens - 1) / kMfmaTokens, group = (tokens + groups - 1) / groups, tiles = (g.n + 15) / 16;
-    int walkers = 256 / (g.parts * groups);               // one workgroup per CU
-    if (walkers < 1) walkers = 1;
-    if (walkers > tiles) walkers = tiles;
-    gemv_mfma_kernel<UK, UNITS><<<dim3(walkers * g.parts, groups), kMfmaWaves * 64, lds, st>>>(g, tokens, group);
+    gemv_mfma_kernel<UK, UNITS, ONE><<<dim3(walkers * g.parts, groups), kMfmaWaves * 64, lds, st>>>(g, tokens, (tokens + groups - 1) / groups);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
+}
+static int gemv_mfma(const GemvArgs& g, int tokens, int stretch, hipStream_t st) {
+    const int groups = (tokens + kMfmaTokens - 1) / kMfmaTokens, tiles = (g.n + 15) / 16;
+    int walkers = 256 / (g.parts * groups);               // one workgroup per CU
+    if (walkers < 1) walkers = 1;
+    const bool one = tiles <= walkers;
+    if (one) walkers = tiles;
+    if (stretch <= 1024) return one ? launch_gemv_mfma<1024, 1, true>(g, tokens, walkers, groups, st) : launch_gemv_mfma<1024, 1, false>(g, tokens, walkers, groups, st);
+    if (stretch <= 2048) return one ? launch_gemv_mfma<2048, 1, true>(g, tokens, walkers, groups, st) : launch_gemv_mfma<2048, 1, false>(g, tokens, walkers, groups, st);
+    return launch_gemv_mfma<2048, 2, false>(g, tokens, walkers, groups, st);
 }
 
 // k of a workgroup: 1024, 2048 or 4096.  Parts of a product whose reader adds them: as few as that takes, one more doubling where the
@@ -595,9 +633,7 @@ int gemv_float(const GemvArgs& g, int pro, int tokens, hipStream_t st) {
     if (pro == 0 && tokens > 1 && !g.per_token) {
         if constexpr (std::is_same<ET, bf16_t>::value) {
             const int stretch = (g.kpad + g.parts - 1) / g.parts;
-            if (stretch <= 1024) return launch_gemv_mfma<1024, 1>(g, tokens, st);
-            if (stretch <= 2048) return launch_gemv_mfma<2048, 1>(g, tokens, st);
-            if (stretch <= 4096) return launch_gemv_mfma<2048, 2>(g, tokens, st);
+            if (stretch <= 4096) return gemv_mfma(g, tokens, stretch, st);
             FX_REQUIRE(g.parts == 1, "gemv_float: %d parts of k=%d", g.parts, g.k);
         }
         return gemv_tokens<ET>(g, tokens, st);
