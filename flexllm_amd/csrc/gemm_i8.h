@@ -724,23 +724,24 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
                 if constexpr (kAsym) bx[i] = qa.b_x[row];
             }
         }
-        // byte of the lane's 16 in the tile's first row; they lie inside or behind the row as a whole
-        auto place = [&](int j0) __attribute__((always_inline)) {
-            const int col = col0 + wc + j0 * 16 + (kUnit ? fg * 8 : fg * 4);
-            return col < n ? (kUnit ? col * 2 : col * 4) + fr * ld * 4 : kNowhere;
+        // byte of the lane's 16 in the tile's first row.  They lie inside or behind the row as a whole, or (a unit whose rows end in the middle: it
+        // makes them of eight columns, and n is a multiple of 4) their first half does: that leaves by itself.
+        constexpr int PC = kUnit ? 8 : 4;                      // columns that 16 bytes of output are made of
+        auto place = [&](int j0, int cols) __attribute__((always_inline)) {
+            const int col = col0 + wc + j0 * 16 + fg * PC;
+            return col + cols <= n ? (kUnit ? col * 2 : col * 4) + fr * ld * 4 : kNowhere;
         };
         // residuals of the next columns are asked for ahead of the stores of these: a wait for loads is one for the stores before them, too
         f32x4 rs[2][MI];
         auto residuals = [&](int j0) __attribute__((always_inline)) {
-            const int at = place(j0);
+            const int at = place(j0, PC);
 #pragma unroll
             for (int i = 0; i < MI; i++) rs[(j0 / J) & 1][i] = res.get(at == kNowhere ? kNowhere : at + i * 16 * ld * 4);
         };
-        if (has_res) residuals(0);
-#pragma unroll
-        for (int j0 = 0; j0 < NI; j0 += J) {
+        auto columns = [&](int j0, auto ends) __attribute__((always_inline)) {      // ends: the first halves of those 16 bytes that the row ends in
+            constexpr bool kEnds = decltype(ends)::value;
             f32x4 ws[J], wq[J];
-            const int at = place(j0);
+            const int at = kEnds && place(j0, PC) != kNowhere ? kNowhere : place(j0, kEnds ? 4 : PC);
 #pragma unroll
             for (int j = 0; j < J; j++) {
                 const int c = min(col0 + wc + (j0 + j) * 16 + fg * 4, n - 4);
@@ -773,8 +774,20 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
                     }
                 }
                 join_blocks<4 / J>(o);
-                out.put(&o[0][0], at == kNowhere ? kNowhere : at + i * 16 * ld * 4);
+                const int to = at == kNowhere ? kNowhere : at + i * 16 * ld * 4;
+                if constexpr (kEnds) out.put_half(&o[0][0], to); else out.put(&o[0][0], to);
                 __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if (has_res) residuals(0);
+#pragma unroll
+        for (int j0 = 0; j0 < NI; j0 += J) columns(j0, std::false_type());
+        if constexpr (kUnit) {
+            const int left = n - (col0 + wc);
+            if ((left & 4) && left > 0 && left < NI * 16) {
+#pragma unroll
+                for (int j0 = 0; j0 < NI; j0 += J)
+                    if (left / (J * 16) == j0 / J) columns(j0, std::true_type());
             }
         }
     }
@@ -857,15 +870,14 @@ inline int launch_gemm_tiles(const int8_t* a, const int8_t* w, int32_t* c, const
         if (pick == 3) return FX_GEMM_TILE(64, 128, 4, 2, 64);
         return FX_GEMM_TILE(64, 64, 4, 2, 64);
     }
-    // the gated unit's 16 bytes of output are eight columns
-    // (a head's 64 bytes leave in 16-byte pieces, too, and the scales and tables are read in such)
+    // (a head's 64 bytes leave in 16-byte pieces, and the scales and tables are read in such)
     if constexpr (EPI == kDmaQkv) {
         const auto bits = [](auto... p) { return (reinterpret_cast<uintptr_t>(p) | ...); };
         // (on 128 x 128 the eight waves of the other kernel hide more of it: 1024 x 3072 x 2048 19.1 us, 20.4 as a walk)
         if (pick == 1 && !(bits(qa.q8, qa.kc, qa.vc, qa.sin_t, qa.cos_t, w_s, qa.w_sum) & 15)) return launch_gemm_walk<EPI, 4>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa);
     }
-    const bool wide = EPI != kDmaQkv && rows_fit(n, 4) && ((EPI != kDmaSwiglu && EPI != kDmaSwigluAsym) || (n % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0));
-    if (pick < 2 && wide) {
+    // (Units whose rows end inside 16 bytes went to 128 x 128 for a while: 1531 x 16388 x 2048 70 us ahead of the walk, 92 there, 64 here.)
+    if (pick < 2 && EPI != kDmaQkv && rows_fit(n, 4)) {
 #define FX_GEMM_ROWS(MI) launch_gemm_walk<EPI, MI>(a, w, c, s_x, w_s, residual, y, m, k, n, st, qa)
         if constexpr (EPI != kDmaQkv) switch (gemm_i8_rows(m, k, n, false)) {
             case 256: return FX_GEMM_ROWS(8);

@@ -79,7 +79,7 @@ __device__ __forceinline__ void join_blocks(uint32_t (&w)[4 / R][R]) {
     }
 }
 
-// Rows of an output (or a residual) as a tile sees them: 16-byte accesses at byte offsets behind its first row.  What lies behind the last
+// Rows of an output (or a residual) as a tile sees them: 16-byte accesses at byte offsets (of whole words) behind its first row.  What lies behind the last
 // row is neither written nor read (zeros come back), and neither is offset kNowhere: no branch stands around a store, so that
 // loads issued ahead of stores are not waited for together with them.  A tile's rows have to stay below 2 GiB (rows_fit): of the rows that are
 // left of the matrix only the tile's own `most` count, all of them can be more bytes than 32 bits say.
@@ -93,6 +93,11 @@ struct TileRows {
     __device__ __forceinline__ void put(const uint32_t* w, int at) const {
         const i32x4 v = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
         __builtin_amdgcn_raw_buffer_store_b128(v, r, at, 0, 0);
+    }
+    __device__ __forceinline__ void put_half(const uint32_t* w, int at) const {      // the first 8 of the 16 bytes
+        using i32x2 = int __attribute__((ext_vector_type(2)));
+        const i32x2 v = {(int)w[0], (int)w[1]};
+        __builtin_amdgcn_raw_buffer_store_b64(v, r, at, 0, 0);
     }
     __device__ __forceinline__ f32x4 get(int at) const {
         const i32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);

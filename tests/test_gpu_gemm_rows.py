@@ -83,6 +83,27 @@ def test_rows_int8(fx, oracle, rows, k):  # noqa: F811
     ints.test_half_line_tiles_with_the_gated_unit(fx, m, k, n)
 
 
+@pytest.mark.parametrize("off", [0, 1, 2])
+@pytest.mark.parametrize("rows,k", INT)
+def test_units_that_end_inside_16_bytes(fx, rows, k, off):  # noqa: F811
+    """A row of the unit's outputs ends in the middle of a lane's 16 bytes, and starts on any word: each row whole, and nothing behind the last."""
+    import numpy as np
+    m, n = INT[rows, k]
+    for n in ((n + 255) // 256 * 256 - 4, (n + 255) // 256 * 256 - 116):
+        assert fx.lib().flexllm_linear_i8_gemm_rows(m, k, n, 0) == rows
+        r = np.random.default_rng(m + k + n)
+        a, w = [fx.to_device(r.integers(-127, 128, s).astype(np.int8)) for s in ((m, k), (n, k))]
+        s_x, w_s = [fx.to_device(r.uniform(lo, hi, c).astype(np.float32)) for lo, hi, c in ((.01, .02, m), (1e-3, 1e-2, n))]
+        y = fx.ops.linear_i8_gemm_dequant(a, s_x, w, w_s).numpy()
+        want = fx.ops.swiglu_f32(*(fx.to_device(np.ascontiguousarray(y[:, i::2])) for i in (0, 1))).numpy()
+        size = m * (n // 2)
+        buf = fx.to_device(np.full(size + 16, 77.0, np.float32))
+        fx.ops.linear_i8_gemm_swiglu(a, s_x, w, w_s, out=buf.view(4 * off, (m, n // 2)))
+        got = buf.numpy()
+        assert np.array_equal(got[off:off + size].reshape(m, n // 2), want)
+        assert (got[:off] == 77.0).all() and (got[off + size:] == 77.0).all()
+
+
 def test_outputs_of_4_gib(fx):  # noqa: F811
     """The bytes of the rows behind a tile's first one need more than 32 bits: first rows, rows on both sides of 2 GiB, last rows."""
     import numpy as np
