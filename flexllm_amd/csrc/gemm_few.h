@@ -15,14 +15,13 @@ namespace fx {
 constexpr int kFewMost = 32;                              // rows of A in a pass over the weights
 
 template <int UK, int UNITS, int NG>                      // 16 * NG rows of A
-__global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {     // len: k of a part
+__global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g) {
     constexpr int NW = 8, SL = UK / NW, SW = SL / 32;      // k and matrix k-steps of a wave in a unit
     constexpr int UB = UK * 2, SLOT = 16 * UB, SLOTS = 128 * 1024 / SLOT, PER = SLOT / 1024 / NW;      // PER: requests of a wave per unit
     extern __shared__ __attribute__((aligned(16))) int8_t ring[];
     __shared__ float red[NW][NG][16 * 17];
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), gq = lane >> 4;
-    const int part = blockIdx.x % g.parts, walker = blockIdx.x / g.parts, walkers = gridDim.x / g.parts;
-    const int row0 = blockIdx.y * (16 * NG), rows = min(16 * NG, g.m - row0), k0 = part * len, k1 = min(g.k, k0 + len), tiles = (g.n + 15) / 16;
+    const int walker = blockIdx.x, walkers = gridDim.x, tiles = (g.n + 15) / 16;
     const int mine = (tiles - walker + walkers - 1) / walkers, total = mine * UNITS;          // tiles and units of this workgroup
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)ring;
     auto request_unit = [&](int u) __attribute__((always_inline)) {
@@ -32,7 +31,7 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
         for (int q = 0; q < PER; q++) {
             const int p = wave * PER + q, r = p / (UB / 1024), seg = p % (UB / 1024);
             // what is behind the row's end (any of its bytes will do) is not looked at
-            const int kb = min((k0 + h * UK) * 2 + seg * 1024 + (lane ^ r) * 16, g.k * 2 - 16);
+            const int kb = min(h * UK * 2 + seg * 1024 + (lane ^ r) * 16, g.k * 2 - 16);
             load_to_lds<true>(base, (unsigned)(min(r, last) * g.ldw * 2 + kb), lds0 + (u % SLOTS) * SLOT + p * 1024);
         }
     };
@@ -40,13 +39,13 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
     int steps[UNITS];                                     // k-steps of this wave that there are
 #pragma unroll
     for (int h = 0; h < UNITS; h++) {
-        const int first = k0 + h * UK + wave * SL;
-        steps[h] = max(0, min(SW, (k1 - first) / 32));
+        const int first = h * UK + wave * SL;
+        steps[h] = max(0, min(SW, (g.k - first) / 32));
 #pragma unroll
         for (int s = 0; s < SW; s++)
 #pragma unroll
             for (int q = 0; q < NG; q++)
-                af[h * SW + s][q] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(g.a) + (size_t)(row0 + min(q * 16 + (lane & 15), rows - 1)) * g.lda +
+                af[h * SW + s][q] = *reinterpret_cast<const bf16x8*>(static_cast<const bf16_t*>(g.a) + (size_t)min(q * 16 + (lane & 15), g.m - 1) * g.lda +
                                                                      min(first + s * 32, g.k - 32) + gq * 8);
     }
     wait_vmcnt<0>();                                      // results come in the order of the requests
@@ -64,14 +63,14 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
         return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
     };
     auto finish = [&](int i, float s) __attribute__((always_inline)) {
-        const int col = (walker + i * walkers) * 16 + r, row = row0 + j;
+        const int col = (walker + i * walkers) * 16 + r;
         if (g.bias) s += g.bias[min(col, g.n - 1)];
         const float up = lane_xor_f<1>(s);
-        if (j >= rows || col >= g.n) return;
+        if (j >= g.m || col >= g.n) return;
         bf16_t* y = static_cast<bf16_t*>(g.y);
-        if (col >= g.n_split) g.y32[part * g.part_stride + (size_t)row * g.ldy32 + col - g.n_split] = s;
-        else if (!g.glu) y[(size_t)row * g.ldy + col] = (bf16_t)s;
-        else if ((col & 1) == 0) y[(size_t)row * g.ldy + (col >> 1)] = (bf16_t)glu_f(g.glu, s, up, g.limit);
+        if (col >= g.n_split) g.y32[(size_t)j * g.ldy32 + col - g.n_split] = s;
+        else if (!g.glu) y[(size_t)j * g.ldy + col] = (bf16_t)s;
+        else if ((col & 1) == 0) y[(size_t)j * g.ldy + (col >> 1)] = (bf16_t)glu_f(g.glu, s, up, g.limit);
     };
     const int8_t* const in0 = ring + (lane & 15) * UB;
     for (int i = 0; i < mine; i++) {
@@ -115,8 +114,6 @@ __global__ __launch_bounds__(512, 2) void gemm_few_kernel(GemmArgs g, int len) {
     finish(mine - 1, sums());
 }
 
-// k of a part, in units of 64.
-inline int gemm_few_len(int k, int parts) { return ((k / 64 + parts - 1) / parts) * 64; }
 // Products of at most 32 rows run here where a workgroup has two tiles or more, so that their weights' stream is long enough to pay for
 // the start (A into registers) and the sums, and where k fills the units: a place in the ring that is half empty is half as much in flight, and an
 // instruction on nothing takes as long as another.  The tiles of the wide GEMMs and this, us: 16384 x 2048, 9 rows 17.6 and 13.8, 32 rows 18.0 and 16.9; 28672 x
@@ -138,18 +135,13 @@ static int launch_few(const GemmArgs& g, hipStream_t st) {
         FX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_few_kernel<UK, UNITS, NG>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         opted_in.store(true, std::memory_order_release);
     }
-    const int groups = (g.m + 16 * NG - 1) / (16 * NG), tiles = (g.n + 15) / 16;
-    int walkers = 256 / (g.parts * groups);               // one workgroup per CU
-    if (walkers < 1) walkers = 1;
-    if (walkers > tiles) walkers = tiles;
-    gemm_few_kernel<UK, UNITS, NG><<<dim3(walkers * g.parts, groups), 512, lds, st>>>(g, gemm_few_len(g.k, g.parts));
+    gemm_few_kernel<UK, UNITS, NG><<<256, 512, lds, st>>>(g);      // one workgroup per CU, of two tiles or more
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
 inline int gemm_few(const GemmArgs& g, hipStream_t st) {
-    const int len = gemm_few_len(g.k, g.parts);
-    if (g.m <= 16) return len <= 1024 ? launch_few<1024, 1, 1>(g, st) : len <= 2048 ? launch_few<2048, 1, 1>(g, st) : launch_few<2048, 2, 1>(g, st);
-    return len <= 2048 ? launch_few<2048, 1, 2>(g, st) : launch_few<2048, 2, 2>(g, st);
+    if (g.m <= 16) return g.k <= 1024 ? launch_few<1024, 1, 1>(g, st) : g.k <= 2048 ? launch_few<2048, 1, 1>(g, st) : launch_few<2048, 2, 1>(g, st);
+    return g.k <= 2048 ? launch_few<2048, 1, 2>(g, st) : launch_few<2048, 2, 2>(g, st);
 }
 
 }  // namespace fx

@@ -1,7 +1,7 @@
 // The walk over k that the GEMMs of many rows share (int8, bfloat16 and float32): C[m][n] = sum_k A[m][k] * W[n][k], both operands
 // K-contiguous, on 16 x 16 matrix instructions.
 //
-// Four waves per workgroup, one per SIMD, as a grid of WM x 4/WM; a wave's tile is MI x NI blocks of 16 x 16.  Rows go global -> LDS by
+// Four waves per workgroup, one per SIMD, as a grid of two by two; a wave's tile is MI x NI blocks of 16 x 16.  Rows go global -> LDS by
 // direct loads in stages of 128 bytes of k (whole lines; halves of them reach 14.5 TB/s where lines reach 23), through a ring of NA
 // stages of A and one of NB stages of W.  A lane's 16 bytes of a row are one operand, so nothing is transposed; the 16-byte chunks of
 // row r are stored rotated by (r >> 1) & 7, which is applied on the global side of the load, and the operand reads are free of conflicts.
@@ -144,8 +144,8 @@ struct GemmWalk {
     static constexpr int RA = (BM + 31) / 32 * 32, RB = BN;    // rows in LDS: every wave issues the same number of loads, of eight rows each
     static constexpr int AI = RA / 32, BI = RB / 32, PER = AI + BI;
     static constexpr int ASZ = RA * 128, BSZ = RB * 128, kLds = NA * ASZ + NB * BSZ;
-    static_assert(WM == 1 || WM == 2, "waves along the rows");
-    static_assert(RB % 32 == 0 && (NA == NB || NA == NB + 1) && NB >= 2 && kLds <= 160 * 1024, "ring");
+    static_assert(WM == 2, "waves along the rows");
+    static_assert(RB % 32 == 0 && (NA == NB || NA == NB + 1) && NB >= 2 && NB <= 4 && kLds <= 160 * 1024, "ring");
     // waves per SIMD that registers have to leave room for: as many workgroups as LDS does, two waves' worth of registers where that is enough
     static constexpr int per_cu() { return kSumsApart ? 1 : 160 * 1024 / kLds < 2 ? 2 : 160 * 1024 / kLds < 3 ? 2 : 3; }
     // a wave's loads in flight behind those of the stage that a wait is for, `younger` stages behind it
@@ -170,6 +170,7 @@ struct GemmWalk {
         return n;
     }
     static_assert(SB < NM && SA >= 2 * AI && slot_b(BI - 1) + 1 <= SB && slot_a(AI - 1) + 1 < KS * NM, "places of the loads");
+    static_assert(NR <= NM, "an operand read behind a matrix instruction");
 
     static __device__ __forceinline__ int rot(int r) { return (r >> 1) & 7; }
     static __device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
@@ -238,13 +239,11 @@ struct GemmWalk {
         };
         auto wait_stage = [&](int younger) __attribute__((always_inline)) {
             if (younger >= NB) wait_vmcnt<in_flight(NB)>();
-            else if (NB > 4 && younger == 4) wait_vmcnt<in_flight(4)>();
             else if (NB > 3 && younger == 3) wait_vmcnt<in_flight(3)>();
             else if (NB > 2 && younger == 2) wait_vmcnt<in_flight(2)>();
             else if (younger == 1) wait_vmcnt<in_flight(1)>();
             else wait_vmcnt<0>();
         };
-        static_assert(NB <= 6, "the wait tells up to four younger stages apart");
         // Stage 0 is in when what was asked for behind it is out: all of the stages 1 .. NA - 1 that there are, as far as they are asked for.
         {
             constexpr int full = (NB - 1) * BI + (NA - 2) * AI + early_a;
@@ -278,15 +277,6 @@ struct GemmWalk {
                     if (x % RS == 0 && x / RS < NR) {
                         if (!last) read(a1, b1, s + 1, (s + 1) & 1, x / RS);
                         else if (kNext) read(a2, b2, 0, (s + 1) & 1, x / RS);
-                    }
-                    if constexpr (NR > NM) {                     // more reads than matrix instructions: the rest behind the last one
-                        if (x == NM - 1) {
-#pragma unroll
-                            for (int q = NM; q < NR; q++) {
-                                if (!last) read(a1, b1, s + 1, (s + 1) & 1, q);
-                                else if (kNext) read(a2, b2, 0, (s + 1) & 1, q);
-                            }
-                        }
                     }
                     // place behind the barrier of this stage (last k-step) or of the one before
                     const int p = last ? x : (s + 1) * NM + x;

@@ -138,8 +138,8 @@ int flexllm_linear_i8_gemv_swiglu(const int8_t* x, const float* s_x, const int8_
  * pref_Linear_Layer_i4xi4 (Modules/Linear_Layer.h:293-341) with the int8 systolic array
  * (Modules/MHA.h:113-187, Modules/PE.h:526-583).  k % 64 == 0. */
 int flexllm_linear_i8_gemm(const int8_t* a, const int8_t* w, int32_t* acc, int m, int k, int n, void* stream);
-/* Rows and columns of the tile that an int8 product (qkv: the fused q/k/v projection) of these sizes runs on, and how many of them
- * a CU holds at a time.  Needs no GPU. */
+/* Rows and columns of the tile that is chosen for an int8 product (qkv: the fused q/k/v projection) of these sizes, and how many of them
+ * a CU holds at a time; where it has 256 columns, flexllm_linear_i8_gemm_rows says how many rows of them a workgroup takes.  Needs no GPU. */
 int flexllm_linear_i8_gemm_tile(int m, int k, int n, int qkv, int* rows, int* cols, int* per_cu);
 /* A product whose tile has 256 columns shares its rows out anew: the rows that a workgroup takes (128 to 256; of any other product those of
  * its tile), negative: an error code.  Needs no GPU. */
@@ -612,7 +612,8 @@ int flexllm_hybrid_set_wait_limit(flexllm_hybrid* m, int polls);
  * bias [n] or NULL is added first; glu: 0, or 1 + FLEXLLM_GLU_*. */
 int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, void* y, float* y32, int m, int k, int n, int n_split, int glu, float limit,
                               int dtype, void* stream);
-/* Rows and columns of the tile that such a product runs on, and how many of them a CU holds at a time.  Needs no GPU. */
+/* Rows and columns of the tile that is chosen for such a product, and how many of them a CU holds at a time; where it has 256 columns, and for
+ * few rows, flexllm_linear_float_gemm_rows says what a workgroup takes.  Needs no GPU. */
 int flexllm_linear_float_gemm_tile(int m, int k, int n, int dtype, int* rows, int* cols, int* per_cu);
 /* The rows that a workgroup takes, as flexllm_linear_i8_gemm_rows, or 16 or 32 where few rows of a long bfloat16 product are one pass over the
  * weights without tiles; parts: 1, or those that k is shared out in.  Needs no GPU. */
