@@ -7,9 +7,9 @@
 // row r are stored rotated by (r >> 1) & 7, which is applied on the global side of the load, and the operand reads are free of conflicts.
 //
 // What bounds it.  A 256 x 256 tile reads 32 KiB of operands from LDS per 16 KiB that arrive, against 48 with eight waves of 128 x 64: with
-// those, LDS was busy all the time and the matrix cores 55 % of it.  Now they are busy for 80 % of the cycles and the chip's power
-// holds the clock at 1.9 GHz (16 x 16 instructions take less of it than 32 x 32 ones: those kept it at 1.66 GHz, at 88 %, and took 4 to
-// 6 % more time).  What it took: each matrix instruction has at most an operand read and one half of a direct load behind it; the
+// those, LDS was busy all the time and the matrix cores 55 % of it.  Now they are busy for 73 to 78 % of the cycles of a long walk, and the chip's
+// power holds the clock at 1.76 to 1.85 GHz (counters of 4096 x 28672 x 4096, 4096 x 4096 x 4096 and 4096 x 16384 x 4096; 16 x 16 instructions take less of
+// it than 32 x 32 ones, which took 4 to 6 % more time).  What it took: each matrix instruction has at most an operand read and one half of a direct load behind it; the
 // loads of a stage are spread over one and a half k-steps (in a burst they queue up and the matrix instructions behind them
 // wait), and A is a stage further ahead than W, which is what fits into 160 KiB.
 // bfloat16, before (eight waves, 32 x 32 instructions) and now, us: 4096 x 4096 x 14336 (m, n, k) 407 and 320, 1504 TFLOP/s; 4096 x 28672 x 4096 879
