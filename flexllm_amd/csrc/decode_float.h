@@ -10,6 +10,7 @@ constexpr int kWalkMaxPhases = 256;
 constexpr int kWalkPolls = 1 << 20;        // about a second
 constexpr int kWalkMaxWidth = 4096;
 constexpr size_t kWalkLdsMax = 160 * 1024;
+constexpr size_t kWalkMixerLds = 16 * 1024;
 constexpr int kWalkMinSlots = 2, kWalkMaxSlots = 4, kWalkSlotBytes = 32 * 1024;       // of the weights' ring
 constexpr int kWalkRow = 4096;             // bytes that the rows of all linears are a multiple of
 
@@ -22,7 +23,7 @@ struct WalkPhase {
     int routed;                            // 0, or the number (from 1) of the mixture whose choice it waits for
     int slot;
     size_t stride;
-    int x_off, red_off;                    // where the vector starts in LDS, and where the sums do (in floats, the same in all workgroups)
+    int x_off, red_off;                    // where the vector starts in LDS (element of those ahead of it), and where the sums do (in floats, the same in all workgroups)
 };
 enum WalkMixer { kWalkSharedKv = 0, kWalkLatent = 1, kWalkGla = 2, kWalkMixture = 3 };
 struct WalkRun {
@@ -74,7 +75,9 @@ struct WalkArgs {
     int* tokens_out;                       // greedy steps: tokens_out[state[1] + step]; null: a single step
     float* logits;                         // null: not wanted
     int steps, head;
+    int parts;                             // vectors lie in LDS as three bfloat16 parts, for the matrix cores
     int lds_xs, lds_red;                   // floats
+    int lds_head;                          // where the head's sums lie from the other linears': beside its vector, where that of a feed-forward is longer
 };
 // Rows r0 .. r1-1 of n belong to workgroup w: pairs of rows stay together.
 __host__ __device__ inline int walk_rows(int n, int w) {
@@ -83,6 +86,13 @@ __host__ __device__ inline int walk_rows(int n, int w) {
 }
 // Rows that a workgroup has at most.
 __host__ __device__ inline int red_rows(int n) { return 2 * (((n + 1) / 2 + kWalkWG - 1) / kWalkWG); }
+// Sums that a row of k leaves in LDS: with parts one for each stream wave that has blocks of it, otherwise one for each quad (of qe elements).  And those of n rows.
+constexpr int kBlockK = 512, kWalkStreams = 8;
+__host__ __device__ inline int walk_sums(bool parts, int k, int qe) {
+    const int n = parts ? k / kBlockK : k / qe;
+    return parts && n > kWalkStreams ? kWalkStreams : n > 0 ? n : 1;
+}
+__host__ __device__ inline int walk_red(bool parts, int n, int k, int qe) { return (parts ? (red_rows(n) + 3) / 4 * 4 : red_rows(n)) * walk_sums(parts, k, qe); }
 size_t walk_lds(const WalkArgs& a);        // bytes
 constexpr int kWalkExperts = 255, kWalkTop = 16;        // most
 template <typename ET> int walk_launch(const WalkArgs& a, hipStream_t st);

@@ -112,17 +112,21 @@ __device__ __forceinline__ void group(int n, F f) {
 
 constexpr float kWalkLog2e = 1.44269504088896340736f;
 
-struct WalkLds {                                          // ahead of the vector and the sums
-    __attribute__((aligned(16))) int4 phase[kWalkMaxPhases];           // address of the workgroup's rows, quads, quads per row (0: half a one)
-    __attribute__((aligned(16))) int4 group[kWalkMaxPhases];           // vector's and sums' places; number of the group; [last << 31 | first << 30 | wave that begins << 16 | mixture]
+// A linear of the workgroup.  phase: address of its rows; quads and quads per row (0: half a one), with parts rows and blocks of k.  group, for mixtures: the vector's and the
+// sums' places; number of the group; [last << 31 | first << 30 | wave that begins << 16 | mixture].
+struct WalkTables { int4 *phase, *group; };
+struct MixerLds {                                         // where the vector lies otherwise: nobody needs that while the mixers are at work
     __attribute__((aligned(16))) float q[kWalkRow2];      // query; of gated linear attention query, key, decay, and what is short
     __attribute__((aligned(16))) float kx[kWalkRow2];     // the row of this step
     __attribute__((aligned(16))) float ql[kWalkRow2];     // latent query
     __attribute__((aligned(16))) float sums[kSvcWaves][kWalkRank];
-    float of_head[32];
+};
+static_assert(sizeof(MixerLds) <= kWalkMixerLds, "room for the mixers");
+struct WalkLds {                                          // ahead of the tables, the vector and the sums
+    __attribute__((aligned(16))) float of_head[32];
     float z[kWalkExperts + 1], choice_w[kWalkTop + 1];
     float m[kSvcWaves], l[kSvcWaves];
-    int met, ready, sent, chosen;                         // service waves' barrier; linears whose vector is there, whose sums have left; mixtures that have chosen
+    int met, ready, done, sent, chosen;                   // service waves' barrier; linears (free: shares) whose vector is there, shares whose sums are; linears whose sums have left; mixtures that have chosen
     float norm[2][kSvcWaves];
     float bestv[2][kSvcWaves];
     int besti[2][kSvcWaves];
@@ -157,28 +161,37 @@ __device__ __forceinline__ void wait_quads(int n) {
         default: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
     }
 }
+// A wave's part in a count that others wait for: what it has written to LDS before is there.
+__device__ __forceinline__ void add(int& f) {
+    if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(&f, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 __device__ __forceinline__ int flag(const int& f) { return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)); }
+// Between linears the waves ask and look for the vector in turn.  FREE: they do not stand still until a quad is there, and the two kinds of waves meet by counts;
+// otherwise a wave has one quad at a time on its way, and they meet at barriers, for which all have to be there.  16 layers of 2048, 24 tokens behind 1531 rows:
+// 19170 us with barriers, 18500 free; latent rows and gated linear attention 19390 and 19110; with mixtures 15200 and 15470, whose choice is one more chain of words
+// that requests stand in the way of.
+template <int KIND> constexpr bool kFree = KIND != kWalkMixture;
 // MOE: with groups of linears and rows of half a quad (the other models are 2 to 3 % faster without).
-template <typename ET, bool MOE>
-__device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, float* red, const char* ring, int slots, int phases, int tokens, int routed) {
+template <typename ET, bool MOE, bool FREE>
+__device__ __forceinline__ void stream_waves(WalkLds& L, WalkTables T, const float* xs, float* red, const char* ring, int slots, int phases, int tokens, int routed, int head, int head_off) {
     constexpr int CE = Chunk<ET>::N, PL = CE / 4;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) - kSvcWaves;
     auto word = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
     const char* mine = ring + (size_t)wave * slots * kQuad;
     const unsigned dst = word((int)(unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)mine);
     // what is asked for next: quad iq of linear ip of token it
-    int ip = 0, it = 0, iq = wave, itotal = word(L.phase[0].z), iorder = 0, igroup = 0, islot = 0, ahead = 0;      // ahead: quads asked for and not taken in
-    auto base_of = [&](int p) { return reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(L.phase[p].y) << 32) | (unsigned)word(L.phase[p].x)); };
+    int ip = 0, it = 0, iq = wave, itotal = word(T.phase[0].z), iorder = 0, igroup = 0, islot = 0, ahead = 0;      // ahead: quads asked for and not taken in
+    auto base_of = [&](int p) { return reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(T.phase[p].y) << 32) | (unsigned)word(T.phase[p].x)); };
     auto begins = [&](int flags) { return (wave + (flags >> 16 & 7)) & (kStrWaves - 1); };      // this wave's first quad
     const char* ibase = base_of(0);
     auto settle = [&] {                                   // on to a linear of which this wave has a quad
         while (iq >= itotal && it < tokens) {
             if (++ip == phases) { ip = 0; it++; }
-            const int4 ph = L.phase[ip];
+            const int4 ph = T.phase[ip];
             itotal = word(ph.z);
             ibase = reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(ph.y) << 32) | (unsigned)word(ph.x));
             if constexpr (MOE) {
-                const int4 gr = L.group[ip];
+                const int4 gr = T.group[ip];
                 const int flags = word(gr.w);
                 iq = begins(flags);
                 iorder = flags & 0xFFFF;
@@ -209,15 +222,15 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
     float xr[4][CE];
     for (int ct = 0; ct < tokens; ct++)
         for (int cp = 0; cp < phases; cp++) {
-            const int4 ph = L.phase[cp];
+            const int4 ph = T.phase[cp];
             int4 gr = make_int4(0, 0, cp, (int)(3u << 30));
-            if constexpr (MOE) gr = L.group[cp];
+            if constexpr (MOE) gr = T.group[cp];
             const int total = word(ph.z), rq = word(ph.w), flags = word(gr.w), cgroup = MOE ? word(gr.z) : cp;
             const bool half = MOE && rq == 0, first = !MOE || (flags >> 30 & 1), last = !MOE || flags < 0;
             const int segs = half ? 2 : 4 * rq, from = MOE ? begins(flags) : wave;
             if (!first && !last && from >= total) continue;
             const float* x0 = MOE ? xs + word(gr.x) : xs;
-            float* sums = MOE ? red + word(gr.y) : red;
+            float* sums = red + (MOE ? word(gr.y) : cp == head ? head_off : 0);
             int at = from;                                // place of the quad in its row
             while (!half && at >= rq) at -= rq;
             const bool held = half || kStrWaves % rq == 0;             // the same in all rows
@@ -257,17 +270,16 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 while (at >= rq) at -= rq;
             };
             auto same = [&] { return igroup == cgroup && it == ct; };
-            // Requests stand in the way of the service waves' words, so between linears each wave has one quad at a time on its way (16 layers of 2048, before
-            // the registers below: 610 us per token, 624 without that, 658 with nothing asked for between linears).  When the ring is full, the first two quads move into registers.
+            // When the ring is full, the linear's first quads move into registers.
             i32x4 u[2][4];
             bool taken = false;
             if (first) {
                 n++;
-                while (flag(L.ready) < n) {
+                while (flag(L.ready) < (FREE ? kSvcWaves * n : n)) {
                     if (ahead < slots && known()) {
                         ask();
-                        wait_quads(0);
-                    } else if (!taken && ahead >= 2 && !half && from + kStrWaves < total) {
+                        if constexpr (!FREE) wait_quads(0);
+                    } else if (!taken && ahead == slots && ahead >= 2 && !half && from + kStrWaves < total) {
                         wait_quads(ahead - 2);
                         read(u[0]);
                         read(u[1]);
@@ -277,7 +289,8 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                         __builtin_amdgcn_s_sleep(1);
                     }
                 }
-                __syncthreads();                          // the vector is there
+                if constexpr (FREE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                else __syncthreads();                     // the vector is there
                 while (ahead < slots && same()) ask();
             }
             // experts' gate/up: all on the one vector, which is still there
@@ -329,28 +342,292 @@ __device__ __forceinline__ void stream_waves(const WalkLds& L, const float* xs, 
                 }
             }
             if (last) {
-                __syncthreads();                          // the sums are there
+                if constexpr (FREE) add(L.done);
+                else __syncthreads();                     // the sums are there
+                while (flag(L.sent) < n) __builtin_amdgcn_s_sleep(1);      // they leave first: a store, too, stands in line
+            }
+        }
+}
+
+// bfloat16 weights on the matrix cores.  A quad is 1 KiB, 512 of k, of four neighbouring rows (a block); a float32 vector is the sum of three
+// bfloat16 parts to 24 bits, and their products with the weights are exact in float32.  An instruction (16 x 16 x 32) takes 256 bytes of each row: its rows
+// are 4 weight rows x 4 pieces of k, its columns 3 parts x the same 4 pieces, and where the pieces meet are the sums.  So 512 weights take one
+// instruction for 20 of a lane's own, operands come in requests of 1 KiB of one row, and a wave that stays in a block of k keeps the vector in 16 registers.
+// In LDS 16 bytes c of row r lie at place c ^ 2r, of part p at c ^ 2p: eight lanes that read together are on different banks.
+__device__ __forceinline__ void block_to_lds(const char* base, const unsigned (&voff)[4], unsigned dst) {
+    unsigned saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\t"
+                 "s_mov_b32 m0, %6\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %5 nt\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %2, %5 nt\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %3, %5 nt\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %4, %5 nt\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(base), "s"(dst) : "memory", "scc");
+}
+template <bool MOE, bool FREE>
+__device__ __forceinline__ void stream_parts(WalkLds& L, WalkTables T, const float* xs, float* red, const char* ring, int slots, int phases, int tokens, int routed, int head, int head_off) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) - kSvcWaves;
+    auto word = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const char* mine = ring + (size_t)wave * slots * kQuad;
+    const unsigned dst = word((int)(unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)mine);
+    // as an operand's row lane & 15 is row or part lane & 3 of piece lane >> 2 & 3, of which this lane has 16 bytes
+    const int row = lane & 3, part = min(row, 2), piece = lane >> 4 << 2 | (lane >> 2 & 3);
+    const bool meets = row < 3 && (lane >> 2 & 3) == lane >> 4;
+    const char* get = mine + row * 1024 + (piece ^ 2 * row) * 16;
+    // what is asked for next: block ikb of rows 4 irg .. of linear ip of token it
+    int ip = 0, it = 0, irg = 0, ikb = wave, irows = 0, inkb = 1, iorder = 0, igroup = 0, islot = 0, ahead = 0;      // ahead: quads asked for and not taken in
+    auto address = [&](const int4& ph) { return reinterpret_cast<const char*>(((unsigned long long)(unsigned)word(ph.y) << 32) | (unsigned)word(ph.x)); };
+    auto begins = [&](int flags) { return (wave + (flags >> 16 & 7)) & (kStrWaves - 1); };      // this wave's first quad
+    const char* ibase = nullptr;
+    auto start = [&] {
+        const int4 ph = T.phase[ip];
+        irows = word(ph.z);
+        inkb = word(ph.w);
+        ibase = address(ph);
+        irg = 0;
+        ikb = wave;
+        igroup = ip;
+        if constexpr (MOE) {
+            const int4 gr = T.group[ip];
+            const int flags = word(gr.w);
+            ikb = begins(flags);
+            iorder = flags & 0xFFFF;
+            igroup = word(gr.z);
+        }
+    };
+    auto settle = [&] {                                   // on to a linear of which this wave has a quad
+        for (;;) {
+            while (ikb >= inkb) { ikb -= inkb; irg++; }
+            if (4 * irg < irows || it >= tokens) break;
+            if (++ip == phases) { ip = 0; it++; }
+            start();
+        }
+    };
+    auto known = [&] {                                    // an expert's weights have no address before the choice
+        if (it >= tokens) return false;
+        if (!MOE || iorder == 0) return true;
+        const bool yes = flag(L.chosen) >= it * routed + iorder;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");         // the addresses are read behind the flag
+        return yes;
+    };
+    auto ask = [&] {
+        if (MOE && iorder) ibase = address(T.phase[ip]);
+        const unsigned stride = (unsigned)inkb * 1024u;
+        const int left = irows - 1 - 4 * irg;             // a last group of fewer rows has the last one again
+        unsigned voff[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) voff[r] = (unsigned)min(r, left) * stride + (unsigned)(lane ^ 2 * r) * 16u;
+        block_to_lds(ibase + (size_t)(4 * irg) * stride + (size_t)ikb * 1024, voff, dst + islot * kQuad);
+        islot = islot + 1 == slots ? 0 : islot + 1;
+        ahead++;
+        ikb += kStrWaves;
+        settle();
+    };
+    start();
+    settle();
+    int slot = 0, n = 0;
+    i32x4 x[4];                                           // the vector's operands of a block
+    for (int ct = 0; ct < tokens; ct++)
+        for (int cp = 0; cp < phases; cp++) {
+            const int4 ph = T.phase[cp];
+            int4 gr = make_int4(0, 0, cp, (int)(3u << 30));
+            if constexpr (MOE) gr = T.group[cp];
+            const int rows = word(ph.z), nkb = word(ph.w), flags = word(gr.w), cgroup = MOE ? word(gr.z) : cp;
+            const bool first = !MOE || (flags >> 30 & 1), last = !MOE || flags < 0;
+            const int total = (rows + 3) / 4 * nkb, from = MOE ? begins(flags) : wave;
+            if (!first && !last && from >= total) continue;
+            const char* x0 = reinterpret_cast<const char*>(MOE ? xs + word(gr.x) : xs);
+            const char* x_get = x0 + part * nkb * 1024 + (piece ^ 2 * part) * 16;
+            float* sums = red + (MOE ? word(gr.y) : cp == head ? head_off : 0);
+            const bool held = nkb <= kStrWaves;           // one block of k per wave
+            const int per = min(nkb, kStrWaves);          // sums of a row
+            auto vector = [&](i32x4 (&v)[4], int kb) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const i32x4*>(x_get + kb * 1024 + i * 256);
+            };
+            auto read = [&](i32x4 (&u)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) u[i] = *reinterpret_cast<const i32x4*>(get + slot * kQuad + i * 256);
+                slot = slot + 1 == slots ? 0 : slot + 1;
+                ahead--;
+            };
+            auto products = [&](const i32x4 (&u)[4], const i32x4 (&v)[4], f32x4& acc) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, u[i]), __builtin_bit_cast(bf16x8, v[i]), acc, 0, 0, 0);
+            };
+            // the sums of G groups of rows leave; group i is i * step behind rg
+            bool bad = false;
+            auto leave = [&](auto groups, float (&v)[4 * decltype(groups)::value], int rg, int step) {
+                constexpr int G = decltype(groups)::value;
+#pragma unroll
+                for (int i = 0; i < 4 * G; i++) v[i] = meets ? v[i] : 0.0f;
+                multi_sum_step<4 * G, 1>(v, lane);
+                const int of = multi_row<4 * G>(lane & (4 * G - 1)), r = 4 * (rg + of / 4 * step) + (of & 3);
+                bad = bad || isnan(v[0]);
+                if (lane < 4 * G) sums[r * per + (from & (per - 1))] = v[0];
+            };
+            auto same = [&] { return igroup == cgroup && it == ct; };
+            // When the ring is full, the linear's first quads move into registers.
+            i32x4 u[4][4];
+            int taken = 0;
+            auto all_read = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };      // the slots that have been read are free
+            if (first) {
+                n++;
+                while (flag(L.ready) < (FREE ? kSvcWaves * n : n)) {
+                    if (ahead < slots && known()) {
+                        ask();
+                        if constexpr (!FREE) wait_quads(0);
+                    } else if (taken < (FREE && held ? 4 : 2) && ahead == slots && from + kStrWaves * taken < total) {
+                        wait_quads(ahead - 1);
+                        if (taken == 0) read(u[0]);
+                        else if (taken == 1) read(u[1]);
+                        else if (taken == 2) read(u[2]);
+                        else read(u[3]);
+                        all_read();
+                        taken++;
+                    } else {
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                }
+                if constexpr (FREE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                else __syncthreads();                     // the vector is there
+                while (ahead < slots && same()) ask();
+            }
+            auto fetch = [&](int count) {                 // the next quads, of which the first may be there already
+                if (taken < 1) {
+                    wait_quads(ahead - count);
+                    read(u[0]);
+                    if (count == 2) read(u[1]);
+                } else if (taken < count) {
+                    wait_quads(ahead - 1);
+                    read(u[1]);
+                }
+            };
+            auto used = [&] {                             // two of them: the others move up
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    u[0][i] = u[2][i];
+                    u[1][i] = u[3][i];
+                }
+                taken = max(taken - 2, 0);
+            };
+            auto refill = [&] {
+                all_read();
+                while (ahead < slots && same()) ask();
+            };
+            int kb = from, rg = 0, q = from;
+            while (kb >= nkb) { kb -= nkb; rg++; }
+            if (held) {
+                // experts' gate/up: all on the one vector, which is still there
+                if (from < total && (first || word(gr.x) != 0 || from != wave)) vector(x, kb);
+                const int step = kStrWaves / nkb;
+                for (; q + kStrWaves < total; q += 2 * kStrWaves, rg += 2 * step) {       // two at a time, which hide each other's latencies
+                    fetch(2);
+                    f32x4 acc[2] = {};
+                    products(u[0], x, acc[0]);
+                    products(u[1], x, acc[1]);
+                    refill();
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) v[i] = acc[i / 4][i % 4];
+                    leave(std::integral_constant<int, 2>(), v, rg, step);
+                    used();
+                }
+                if (q < total) {
+                    fetch(1);
+                    f32x4 acc = {};
+                    products(u[0], x, acc);
+                    refill();
+                    float v[4] = {acc[0], acc[1], acc[2], acc[3]};
+                    leave(std::integral_constant<int, 1>(), v, rg, 0);
+                }
+            } else {                                      // several blocks of each group of rows
+                f32x4 acc = {};
+                auto block = [&](const i32x4 (&u)[4], const i32x4 (&v)[4]) {
+                    products(u, v, acc);
+                    kb += kStrWaves;
+                    if (kb < nkb) return;
+                    float o[4] = {acc[0], acc[1], acc[2], acc[3]};
+                    leave(std::integral_constant<int, 1>(), o, rg, 0);
+                    acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    rg++;
+                    kb -= nkb;
+                };
+                for (; q < total; q += 2 * kStrWaves) {
+                    const int count = q + kStrWaves < total ? 2 : 1;
+                    fetch(count);
+                    taken = 0;
+                    i32x4 x2[4];
+                    vector(x, kb);
+                    vector(x2, kb + kStrWaves < nkb ? kb + kStrWaves : kb + kStrWaves - nkb);
+                    refill();
+                    block(u[0], x);
+                    if (count == 2) block(u[1], x2);
+                }
+            }
+            // Not a number may be of the parts' own making, where an infinite weight meets parts of zero or of both signs or a value is infinite (what is left of it is
+            // no number): the same sum with a float32 product per weight has the right of it.
+            if (__builtin_amdgcn_ballot_w64(bad)) {
+                all_read();
+                for (int q = from; q < total; q += kStrWaves) {
+                    const int r = q / nkb * 4, kb0 = q % nkb;
+                    if (!held && kb0 >= kStrWaves) continue;
+                    for (int i = 0; i < 4; i++) {
+                        float& sum = sums[(r + i) * per + (from & (per - 1))];
+                        if (!isnan(sum)) continue;
+                        const char* w = address(T.phase[cp]) + (size_t)min(r + i, rows - 1) * nkb * 1024;
+                        float s = 0.0f;
+                        for (int kb = kb0; kb < nkb; kb += kStrWaves) {
+                            float wv[8];
+                            const i32x4 u = *global(reinterpret_cast<const i32x4*>(w + (size_t)kb * 1024 + lane * 16));
+                            Chunk<bf16_t>::unpack(make_uint4(u[0], u[1], u[2], u[3]), wv);
+#pragma unroll
+                            for (int e = 0; e < 8; e++) {
+                                auto at = [&](int p) { return __uint_as_float((unsigned)*reinterpret_cast<const unsigned short*>(x0 + (size_t)p * nkb * 1024 + ((kb * 64 + lane) ^ 2 * p) * 16 + 2 * e) << 16); };
+                                const float h = at(0);
+                                s = fma_f(wv[e], fabsf(h) < INFINITY ? (h + at(1)) + at(2) : h, s);
+                            }
+                        }
+                        s = wave_sum(s);
+                        if (lane == 0) sum = s;
+                    }
+                }
+            }
+            if (last) {
+                if constexpr (FREE) add(L.done);
+                else __syncthreads();                     // the sums are there
                 while (flag(L.sent) < n) __builtin_amdgcn_s_sleep(1);      // they leave first: a store, too, stands in line
             }
         }
 }
 
 // ---- service waves ----------------------------------------------------------------------------------------------------
-template <typename ET, int QW, int KIND>
+template <typename ET, int QW, int KIND, bool PARTS>
 struct Service {
     static constexpr int CE = Chunk<ET>::N, PL = CE / 4, QE = kQuad / sizeof(ET);      // elements of a quad
+    static constexpr bool FREE = kFree<KIND>;
     const WalkArgs& a;
     WalkLds& L;
+    WalkTables T;
+    MixerLds& M;
     float *xs, *red;
     Wait wait;
     const int t, lane, wave, wg;
     float *now, *other;                                   // the two sets
     f32x4 x[QW];                                          // residual: float4 t + 256 i
     int normed = 0;                                       // L.norm in turn
-    int meetings = 0, ready = 0, sent = 0, chosen = 0;
+    int meetings = 0, ready = 0, sums = 0, sent = 0, chosen = 0;
 
-    __device__ __forceinline__ Service(const WalkArgs& a_, WalkLds& L_, float* xs_, float* red_)
-        : a(a_), L(L_), xs(xs_), red(red_), wait{a_, false}, t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {}
+    __device__ __forceinline__ Service(const WalkArgs& a_, WalkLds& L_, WalkTables T_, float* xs_, float* red_)
+        : a(a_), L(L_), T(T_), M(*reinterpret_cast<MixerLds*>(xs_)), xs(xs_), red(red_), wait{a_, false}, t(threadIdx.x), lane(threadIdx.x & 63), wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), wg(blockIdx.x) {}
     // The thread's number as the compiler does not know it: addresses made of it are not kept in registers from layer to layer.
     __device__ __forceinline__ int opaque() const {
         int v = threadIdx.x;
@@ -360,16 +637,29 @@ struct Service {
     // Barrier of the service waves among themselves: the others may stand still for the sake of their requests.
     __device__ __forceinline__ void meet() {
         meetings += kSvcWaves;
-        if (lane == 0) __hip_atomic_fetch_add(&L.met, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        add(L.met);
         while (__hip_atomic_load(&L.met, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < meetings) {}
     }
     __device__ __forceinline__ void say(int& f, int n) {
         if (t == 0) __hip_atomic_store(&f, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    // to the stream waves: the vector is there; then, behind put(): the sums have left
+    // to the stream waves: the vector is there
     __device__ __forceinline__ void vector_done() {
-        say(L.ready, ++ready);
-        __syncthreads();
+        if constexpr (FREE) {
+            add(L.ready);
+        } else {
+            say(L.ready, ++ready);
+            __syncthreads();
+        }
+    }
+    // until the sums of all stream waves are there; then, behind put(): they have left
+    __device__ __forceinline__ void sums_there() {
+        if constexpr (FREE) {
+            sums += kStrWaves;
+            while (__hip_atomic_load(&L.done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < sums) __builtin_amdgcn_s_sleep(1);
+        } else {
+            __syncthreads();
+        }
     }
     __device__ __forceinline__ void sums_done() { say(L.sent, ++sent); }
     __device__ __forceinline__ void put(unsigned at, float v) {
@@ -377,21 +667,42 @@ struct Service {
         unput(at);
     }
     __device__ __forceinline__ void unput(unsigned at) { store_past(other + at, __int_as_float((int)kUnset)); }
-    __device__ __forceinline__ void put_x(int segs, int c, const f32x4& v, int off = 0) {      // float4 c of the vector that starts at off
-        const int at = PL == 1 ? c : (c & 1) * segs * 64 + (c >> 1);
-        *reinterpret_cast<f32x4*>(xs + off + 4 * at) = v;
+    __device__ __forceinline__ void put_x(int k, int c, f32x4 v, int off = 0) {      // float4 c of the vector of k that starts at element off
+        if constexpr (PARTS) {                            // part p's 16 bytes c at place c ^ 2p, see stream_parts
+            char* x = reinterpret_cast<char*>(xs) + 6 * off + 8 * (c & 1);
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                uint2 o;
+                o.x = __builtin_amdgcn_perm(__float_as_uint(v[1]), __float_as_uint(v[0]), 0x07060302u);
+                o.y = __builtin_amdgcn_perm(__float_as_uint(v[3]), __float_as_uint(v[2]), 0x07060302u);
+                *reinterpret_cast<uint2*>(x + 2 * p * k + ((c >> 1) ^ 2 * p) * 16) = o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] -= __uint_as_float(__float_as_uint(v[e]) & 0xFFFF0000u);
+            }
+        } else {
+            const int at = PL == 1 ? c : (c & 1) * (k / CE) + (c >> 1);
+            *reinterpret_cast<f32x4*>(xs + off + 4 * at) = v;
+        }
     }
-    // total of local row r, of rq quads (0: half a one)
-    __device__ __forceinline__ float total(int rq, int r, int off = 0) const {
-        const float* p = red + off + r * (rq > 0 ? rq : 1);
+    // total of local row r of k
+    __device__ __forceinline__ float total(int k, int r, int off = 0) const {
+        const int n = walk_sums(PARTS, k, QE);
+        const float* p = red + off + r * n;
+        if constexpr (PARTS) {
+            if (n == 2) return p[0] + p[1];
+            f32x4 v = *reinterpret_cast<const f32x4*>(p);
+            if (n == 8) v += *reinterpret_cast<const f32x4*>(p + 4);
+            return (v[0] + v[1]) + (v[2] + v[3]);
+        }
         float s = p[0];
-        for (int i = 1; i < rq; i++) s += p[i];
+        for (int i = 1; i < n; i++) s += p[i];
         return s;
     }
     // A vector of k words as it is
     __device__ __forceinline__ void take(unsigned at, int k) {
         const int t = opaque();
-        const int n4 = k / 4, segs = k / (CE * 64);
+        const int n4 = k / 4;
+        meet();                                           // the mixer's values lie where the vector will
         auto some = [&](auto n, int c0) {
             constexpr int N = decltype(n)::value;
             unsigned off[N];
@@ -401,7 +712,7 @@ struct Service {
             poll_words<N>(now + at, off, c0 + wave * 64 < n4, v, wait);
 #pragma unroll
             for (int i = 0; i < N; i++)
-                if (c0 + t + kSvcT * i < n4) put_x(segs, c0 + t + kSvcT * i, v[i]);
+                if (c0 + t + kSvcT * i < n4) put_x(k, c0 + t + kSvcT * i, v[i]);
         };
         int c0 = 0;
         while (n4 - c0 > 4 * kSvcT) { some(std::integral_constant<int, 8>(), c0); c0 += 8 * kSvcT; }
@@ -413,7 +724,7 @@ struct Service {
     // x += y (normed and times gb where there is one) + the embedding of `again`; the vector becomes norm(x) * g.
     __device__ __forceinline__ void norm(bool have, unsigned at, const float* gb, const float* g, int again_token) {
         const int t = opaque();
-        const int n4 = a.width / 4, segs = a.width / (CE * 64);
+        const int n4 = a.width / 4;
         f32x4 gv[QW], gbv[QW];
         unsigned off[QW];
 #pragma unroll
@@ -456,7 +767,7 @@ struct Service {
             f32x4 h;
 #pragma unroll
             for (int e = 0; e < 4; e++) h[e] = x[i][e] * rx * gv[i][e];
-            if (t + kSvcT * i < n4) put_x(segs, t + kSvcT * i, h);
+            if (t + kSvcT * i < n4) put_x(a.width, t + kSvcT * i, h);
         }
         vector_done();
     }
@@ -526,8 +837,8 @@ struct Service {
                 const bool isq = lane < D / 4, isk = own && lane >= D / 4 && lane < D / 2;
                 off[0] = isq ? 4u * (unsigned)(head * D) + 16u * (unsigned)lane : 4u * (unsigned)(r->n_et + g * D) + 16u * (unsigned)(isk ? lane - D / 4 : 0);
                 poll_words<1>(now + r->x_in, off, isq || isk, v, wait);
-                if (isq) *reinterpret_cast<f32x4*>(L.q + 4 * lane) = v[0];
-                if (isk) *reinterpret_cast<f32x4*>(L.kx + 4 * (lane - D / 4)) = v[0];
+                if (isq) *reinterpret_cast<f32x4*>(M.q + 4 * lane) = v[0];
+                if (isk) *reinterpret_cast<f32x4*>(M.kx + 4 * (lane - D / 4)) = v[0];
             }
             meet();
             float qv[N], acc[N], m = -1e30f, l = 0.0f;    // m finite, so that differences stay defined
@@ -535,7 +846,7 @@ struct Service {
                 float ss = 0.0f;
 #pragma unroll
                 for (int q = 0; q < N; q += 4) {
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(L.q + col + q);
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(M.q + col + q);
 #pragma unroll
                     for (int e = 0; e < 4; e++) { qv[q + e] = v[e]; ss = fma_f(v[e], v[e], ss); }
                 }
@@ -588,7 +899,7 @@ struct Service {
                 float v[N], ss = 0.0f;
 #pragma unroll
                 for (int e = 0; e < N; e++) {
-                    v[e] = L.kx[col + e];
+                    v[e] = M.kx[col + e];
                     ss = fma_f(v[e], v[e], ss);
                     v[e] = (float)(ET)v[e];               // as a later step reads it
                 }
@@ -622,7 +933,7 @@ struct Service {
             for (int mask = LPK, half = N / 2; mask < 64 && half > 0; mask *= 2, half /= 2)
                 if (lane & mask) r0 += half;
 #pragma unroll
-            for (int i = 0; i < LEFT; i++) L.sums[wave][col + r0 + i] = acc[i];
+            for (int i = 0; i < LEFT; i++) M.sums[wave][col + r0 + i] = acc[i];
             meet();
             // and the waves
             if (t < D) {
@@ -632,7 +943,7 @@ struct Service {
 #pragma unroll
                 for (int i = 0; i < kSvcWaves; i++) {
                     const float e = __builtin_amdgcn_exp2f(L.m[i] - mt);
-                    v += e == 0.0f ? 0.0f : L.sums[i][t] * e;
+                    v += e == 0.0f ? 0.0f : M.sums[i][t] * e;
                     lt = fma_f(L.l[i], e, lt);
                 }
                 if (sink) lt += __builtin_amdgcn_exp2f(-mt);
@@ -709,7 +1020,7 @@ struct Service {
             bias = *global(r->a2_bias + h * D + t);
         }
         const float nw = t < cs ? *global(r->head_norm + c0 + t) : 0.0f;
-        float *sq = L.q, *sk = L.q + D, *sa = L.q + 2 * D, *sv = L.q + 3 * D, *sg = sv + 16, *s1 = sg + 16;
+        float *sq = M.q, *sk = M.q + D, *sa = M.q + 2 * D, *sv = M.q + 3 * D, *sg = sv + 16, *s1 = sg + 16;
         if (wave == 0) {                                  // query and key
             unsigned off[1] = {4u * (unsigned)((lane < 32 ? 0 : HD) + h * D) + 16u * (unsigned)(lane & 31)};
             f32x4 v[1];
@@ -756,12 +1067,12 @@ struct Service {
             acc[e] += lane_xor_f<16>(acc[e]);
             acc[e] += lane_xor_f<32>(acc[e]);
         }
-        if (lane < qd) *reinterpret_cast<f32x4*>(&L.sums[wave][4 * lane]) = acc;
+        if (lane < qd) *reinterpret_cast<f32x4*>(&M.sums[wave][4 * lane]) = acc;
         meet();
         if (wave == 0) {
             float x = 0.0f;
             if (t < cs) {
-                x = (L.sums[0][t] + L.sums[1][t]) + (L.sums[2][t] + L.sums[3][t]);
+                x = (M.sums[0][t] + M.sums[1][t]) + (M.sums[2][t] + M.sums[3][t]);
                 const float g = sg[t];
                 put(r->x_att + (unsigned)(h * D + c0 + t), x * nw * (g * sigmoid_f(g)));
             }
@@ -772,7 +1083,7 @@ struct Service {
     // The vector of gla(): every head over the root of its mean square.
     __device__ __forceinline__ void take_heads(RunPtr r) {
         const int t = opaque(), lane = t & 63;
-        const int k = r->k_o, n4 = k / 4, segs = k / (CE * 64), NS = r->splits, H = r->heads;
+        const int k = r->k_o, n4 = k / 4, NS = r->splits, H = r->heads;
         if (wave == 0) {
             const bool need = 4 * lane < H * NS;
             unsigned off[1] = {16u * (unsigned)(need ? lane : 0)};
@@ -794,7 +1105,7 @@ struct Service {
 #pragma unroll
             for (int i = 0; i < N; i++) {
                 const int c = t + kSvcT * i;
-                if (c < n4) put_x(segs, c, v[i] * L.of_head[c / (kWalkDim / 4)]);
+                if (c < n4) put_x(k, c, v[i] * L.of_head[c / (kWalkDim / 4)]);
             }
         };
         if (n4 > 2 * kSvcT) all(std::integral_constant<int, 4>());
@@ -822,7 +1133,7 @@ struct Service {
                 unsigned off[1] = {4u * (unsigned)(h * (D + kWalkRot)) + 16u * (unsigned)min(lane, 47)};
                 f32x4 v[1];
                 poll_words<1>(now + r->x_in, off, lane < 48, v, wait);
-                if (lane < 48) *reinterpret_cast<f32x4*>(L.q + 4 * lane) = v[0];
+                if (lane < 48) *reinterpret_cast<f32x4*>(M.q + 4 * lane) = v[0];
             }
             meet();
             float acc[CE];
@@ -833,7 +1144,7 @@ struct Service {
                 if (g + i * step < D) {
                     float wv[CE];
                     Chunk<ET>::unpack(make_uint4(u[i][0], u[i][1], u[i][2], u[i][3]), wv);
-                    const float q = L.q[g + i * step];
+                    const float q = M.q[g + i * step];
 #pragma unroll
                     for (int e = 0; e < CE; e++) acc[e] = fma_f(wv[e], q, acc[e]);
                 }
@@ -847,12 +1158,12 @@ struct Service {
             }
             if (lane < pc)
 #pragma unroll
-                for (int e = 0; e < CE; e++) L.sums[wave][lane * CE + e] = acc[e];
+                for (int e = 0; e < CE; e++) M.sums[wave][lane * CE + e] = acc[e];
             meet();
-            if (t < cols) put(r->x_ql + (unsigned)(h * RW + c0 + t), (L.sums[0][t] + L.sums[1][t]) + (L.sums[2][t] + L.sums[3][t]));
+            if (t < cols) put(r->x_ql + (unsigned)(h * RW + c0 + t), (M.sums[0][t] + M.sums[1][t]) + (M.sums[2][t] + M.sums[3][t]));
             if (slice == 0 && wave == 3) {                // the rotated part
                 const int j = lane >> 1, rh = kWalkRot / 2;
-                const float x = L.q[D + 2 * j], y = L.q[D + 2 * j + 1], cs = *global(r->cos_t + (size_t)pos * rh + j), sn = *global(r->sin_t + (size_t)pos * rh + j);
+                const float x = M.q[D + 2 * j], y = M.q[D + 2 * j + 1], cs = *global(r->cos_t + (size_t)pos * rh + j), sn = *global(r->sin_t + (size_t)pos * rh + j);
                 put(r->x_ql + (unsigned)(h * RW + RK + lane), lane & 1 ? y * cs + x * sn : x * cs - y * sn);
             }
         }
@@ -882,24 +1193,24 @@ struct Service {
                 unsigned off[1] = {4u * (unsigned)r->n_et + 16u * (unsigned)min(t, RW / 4 - 1)};
                 if (wave < 3) {
                     poll_words<1>(now + r->x_in, off, t < RW / 4, p, wait);
-                    if (t < RW / 4) *reinterpret_cast<f32x4*>(L.kx + 4 * t) = p[0];
+                    if (t < RW / 4) *reinterpret_cast<f32x4*>(M.kx + 4 * t) = p[0];
                 }
                 meet();
-                const float x0 = L.kx[2 * t], x1 = L.kx[2 * t + 1];
+                const float x0 = M.kx[2 * t], x1 = M.kx[2 * t + 1];
                 const float rs = root(fma_f(x0, x0, x1 * x1), (float)RK);
                 float o0 = x0 * rs * *global(r->latent_norm + 2 * t), o1 = x1 * rs * *global(r->latent_norm + 2 * t + 1);
                 float e0 = 0.0f, e1 = 0.0f;
                 if (t < kWalkRot / 2) {
-                    const float a0 = L.kx[RK + 2 * t], a1 = L.kx[RK + 2 * t + 1], cs = *global(r->cos_t + (size_t)pos * (kWalkRot / 2) + t), sn = *global(r->sin_t + (size_t)pos * (kWalkRot / 2) + t);
+                    const float a0 = M.kx[RK + 2 * t], a1 = M.kx[RK + 2 * t + 1], cs = *global(r->cos_t + (size_t)pos * (kWalkRot / 2) + t), sn = *global(r->sin_t + (size_t)pos * (kWalkRot / 2) + t);
                     e0 = (float)(ET)(a0 * cs - a1 * sn);
                     e1 = (float)(ET)(a1 * cs + a0 * sn);
-                    L.kx[RK + 2 * t] = e0;
-                    L.kx[RK + 2 * t + 1] = e1;
+                    M.kx[RK + 2 * t] = e0;
+                    M.kx[RK + 2 * t + 1] = e1;
                 }
                 o0 = (float)(ET)o0;
                 o1 = (float)(ET)o1;
-                L.kx[2 * t] = o0;
-                L.kx[2 * t + 1] = o1;
+                M.kx[2 * t] = o0;
+                M.kx[2 * t + 1] = o1;
                 if (h == 0) {
                     ET* dst = static_cast<ET*>(r->rows) + (size_t)pos * RW;
                     auto pair = [&](ET* p, float a, float b) {
@@ -920,17 +1231,17 @@ struct Service {
                 f32x4 p[1];
                 if (wave < 3) {
                     poll_words<1>(now + r->x_ql, off, t < RW / 4, p, wait);
-                    if (t < RW / 4) *reinterpret_cast<f32x4*>(L.ql + 4 * t) = p[0];
+                    if (t < RW / 4) *reinterpret_cast<f32x4*>(M.ql + 4 * t) = p[0];
                 }
                 meet();
             }
             float ql[8], qr[CE], acc[8], m = -1e30f, l = 0.0f;
             const float f = r->scale * kWalkLog2e;
 #pragma unroll
-            for (int e = 0; e < 8; e++) { ql[e] = L.ql[lane * 8 + e] * f; acc[e] = 0.0f; }
+            for (int e = 0; e < 8; e++) { ql[e] = M.ql[lane * 8 + e] * f; acc[e] = 0.0f; }
             constexpr int LR = kWalkRot / CE;
 #pragma unroll
-            for (int e = 0; e < CE; e++) qr[e] = L.ql[RK + lane % LR * CE + e] * f;
+            for (int e = 0; e < CE; e++) qr[e] = M.ql[RK + lane % LR * CE + e] * f;
             auto columns = [&](const i32x4 (&x)[PCS], float (&o)[8]) {
 #pragma unroll
                 for (int j = 0; j < PCS; j++) Chunk<ET>::unpack(make_uint4(x[j][0], x[j][1], x[j][2], x[j][3]), reinterpret_cast<float (&)[CE]>(o[j * CE]));
@@ -987,10 +1298,10 @@ struct Service {
                 float o[8], s = 0.0f;
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    o[e] = L.kx[lane * 8 + e];
+                    o[e] = M.kx[lane * 8 + e];
                     s = fma_f(o[e], ql[e], s);
                 }
-                s = fma_f(L.kx[RK + lane], L.ql[RK + lane] * f, s);
+                s = fma_f(M.kx[RK + lane], M.ql[RK + lane] * f, s);
                 s = wave_sum(s);
                 const float mx = fmaxf(m, s), al = __builtin_amdgcn_exp2f(m - mx), p = __builtin_amdgcn_exp2f(s - mx);
                 m = mx;
@@ -1000,7 +1311,7 @@ struct Service {
             }
             if (lane == 0) { L.m[wave] = m; L.l[wave] = l; }
 #pragma unroll
-            for (int e = 0; e < 8; e += 4) *reinterpret_cast<f32x4*>(&L.sums[wave][lane * 8 + e]) = f32x4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
+            for (int e = 0; e < 8; e += 4) *reinterpret_cast<f32x4*>(&M.sums[wave][lane * 8 + e]) = f32x4{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]};
             meet();
             const float mt = fmaxf(fmaxf(L.m[0], L.m[1]), fmaxf(L.m[2], L.m[3]));
             float lt = 0.0f, o[2] = {0.0f, 0.0f};
@@ -1009,7 +1320,7 @@ struct Service {
                 const float e = __builtin_amdgcn_exp2f(L.m[w] - mt);
                 lt = fma_f(L.l[w], e, lt);
 #pragma unroll
-                for (int i = 0; i < 2; i++) o[i] += e == 0.0f ? 0.0f : L.sums[w][t + kSvcT * i] * e;
+                for (int i = 0; i < 2; i++) o[i] += e == 0.0f ? 0.0f : M.sums[w][t + kSvcT * i] * e;
             }
 #pragma unroll
             for (int i = 0; i < 2; i++) put(part + t + kSvcT * i, o[i]);
@@ -1053,11 +1364,11 @@ struct Service {
                     if (sp < ns && p != 0.0f) sum += v[i] * p;
                 }
             }
-            *reinterpret_cast<f32x4*>((half ? L.kx : L.q) + 4 * c4) = sum;      // nobody reads them any more, L.sums may still be read
+            *reinterpret_cast<f32x4*>((half ? M.kx : M.q) + 4 * c4) = sum;      // nobody reads them any more, M.sums may still be read
             meet();
             float ctx[8];
 #pragma unroll
-            for (int i = 0; i < 8; i++) ctx[i] = L.q[lane * 8 + i] + L.kx[lane * 8 + i];
+            for (int i = 0; i < 8; i++) ctx[i] = M.q[lane * 8 + i] + M.kx[lane * 8 + i];
 #pragma unroll
             for (int i = 0; i < NP; i++)
                 if (wave + 4 * i < nr) {
@@ -1085,14 +1396,14 @@ struct Service {
         const int W = a.width, E = r->experts, top = r->top, ff = r->ff, sf = r->shared_ff, kr = (E + 4) / 4 * 4;
         int r0;
         int rows = rows_of(2 * sf + kr, r0);
-        __syncthreads();                                  // the sums of [shared gate/up; router; shared gate] are there
+        sums_there();                                    // the sums of [shared gate/up; router; shared gate] are there
         for (int j = t; j < rows; j += kSvcT) {
             const int row = r0 + j;
             if (row >= 2 * sf) {                          // in copies: all workgroups at one line stand in line
-                const float z = total(W / QE, j);
+                const float z = total(W, j);
                 for (int c = 0; c < kWalkCopies; c++) put(r->x_route + (unsigned)(c * kr + row - 2 * sf), z);
             } else if ((row & 1) == 0) {
-                put(r->x_hid + (unsigned)(top * ff + row / 2), glu_f(r->glu, total(W / QE, j), total(W / QE, j + 1), r->shared_limit));
+                put(r->x_hid + (unsigned)(top * ff + row / 2), glu_f(r->glu, total(W, j), total(W, j + 1), r->shared_limit));
             }
         }
         sums_done();
@@ -1114,8 +1425,8 @@ struct Service {
                     const int p = r->phase + k * top + lane;
                     const WalkPhase ph = a.phases[p];
                     const uintptr_t w = reinterpret_cast<uintptr_t>(static_cast<const ET*>(ph.w) + (size_t)pick * ph.stride + (size_t)walk_rows(ph.n, wg) * ph.kpad);
-                    L.phase[p].x = (int)(unsigned)w;
-                    L.phase[p].y = (int)(unsigned)(w >> 32);
+                    T.phase[p].x = (int)(unsigned)w;
+                    T.phase[p].y = (int)(unsigned)(w >> 32);
                 }
             }
             if (lane == 0) L.choice_w[top] = sigmoid_f(L.z[E]);
@@ -1125,15 +1436,15 @@ struct Service {
         }
         vector_done();                                    // the vector is still the same
         rows = rows_of(2 * ff, r0);
-        __syncthreads();
-        const int wq = W / QE, all = rows / 2 * top;
+        sums_there();
+        const int all = rows / 2 * top;
         for (int j = t; j < all; j += kSvcT) {
-            const int s = j / (rows / 2), i = j - s * (rows / 2), o = s * red_rows(2 * ff) * wq;
-            put(r->x_hid + (unsigned)(s * ff + r0 / 2 + i), glu_f(r->glu, total(wq, 2 * i, o), total(wq, 2 * i + 1, o), r->limit));
+            const int s = j / (rows / 2), i = j - s * (rows / 2), o = s * walk_red(PARTS, 2 * ff, W, QE);
+            put(r->x_hid + (unsigned)(s * ff + r0 / 2 + i), glu_f(r->glu, total(W, 2 * i, o), total(W, 2 * i + 1, o), r->limit));
         }
         sums_done();
         // the vectors of the chosen experts one after the other, then the shared one's
-        const int fsegs = ff / (CE * 64), ssegs = sf / (CE * 64), n4 = (top * ff + sf) / 4;
+        const int n4 = (top * ff + sf) / 4;
         for (int c0 = 0; c0 < n4; c0 += 4 * kSvcT) {
             unsigned off[4];
             f32x4 v[4];
@@ -1143,17 +1454,17 @@ struct Service {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int c = c0 + t + kSvcT * i, s = min(c / (ff / 4), top);
-                if (c < n4) put_x(s < top ? fsegs : ssegs, c - s * (ff / 4), v[i], s * ff);
+                if (c < n4) put_x(s < top ? ff : sf, c - s * (ff / 4), v[i], s * ff);
             }
         }
         vector_done();
         rows = rows_of(W, r0);
-        __syncthreads();
-        const int fq = ff / QE, sq = sf / QE, step = red_rows(W) * max(fq, 1);
+        sums_there();
+        const int step = walk_red(PARTS, W, ff, QE);
         for (int j = t; j < rows; j += kSvcT) {
             float y = 0.0f;
-            for (int s = 0; s < top; s++) y = fma_f(L.choice_w[s], total(fq, j, s * step), y);
-            put(r->x_y2 + (unsigned)(r0 + j), fma_f(L.choice_w[top], total(sq, j, top * step), y));
+            for (int s = 0; s < top; s++) y = fma_f(L.choice_w[s], total(ff, j, s * step), y);
+            put(r->x_y2 + (unsigned)(r0 + j), fma_f(L.choice_w[top], total(sf, j, top * step), y));
         }
         sums_done();
     }
@@ -1165,8 +1476,8 @@ struct Service {
         int r0;
         const int rows = rows_of(n, r0);
         const float b = bias && t < rows ? *global(bias + r0 + t) : 0.0f;      // under the products
-        __syncthreads();                                  // the sums are there
-        for (int j = t; j < rows; j += kSvcT) put(at + (unsigned)(r0 + j), total(k / QE, j) + (j == t ? b : bias ? *global(bias + r0 + j) : 0.0f));
+        sums_there();                                    // the sums are there
+        for (int j = t; j < rows; j += kSvcT) put(at + (unsigned)(r0 + j), total(k, j) + (j == t ? b : bias ? *global(bias + r0 + j) : 0.0f));
         sums_done();
     }
     __device__ __forceinline__ int step(int token, int pos, bool choose) {
@@ -1201,11 +1512,11 @@ struct Service {
                     mixture(r);
                     continue;
                 }
-            __syncthreads();
+            sums_there();
             int r0;
             const int rows = rows_of(2 * r->ff, r0);
             for (int j = t; j < rows / 2; j += kSvcT)
-                put(r->x_hid + (unsigned)(r0 / 2 + j), glu_f(r->glu, total(W / QE, 2 * j), total(W / QE, 2 * j + 1), r->limit));
+                put(r->x_hid + (unsigned)(r0 / 2 + j), glu_f(r->glu, total(W, 2 * j), total(W, 2 * j + 1), r->limit));
             sums_done();
             take(r->x_hid, r->ff);
             plain(W, r->ff, r->x_y2, nullptr);
@@ -1213,13 +1524,13 @@ struct Service {
         if (!choose && t < 2) unput(a.x_cand + (unsigned)(2 * wg + t));        // what is not handed out in this step is unset behind the last one all the same
         if (!a.head) return 0;
         norm(have, y, gb, a.g_final, -1);
-        __syncthreads();
+        sums_there();
         int r0;
         const int rows = rows_of(a.vocab, r0);
         float best = -INFINITY;
         int bi = 0x7fffffff;
         for (int j = t; j < rows; j += kSvcT) {
-            const float v = total(W / QE, j);
+            const float v = total(W, j, a.lds_head);
             if (a.logits) a.logits[r0 + j] = v;
             if (v > best) { best = v; bi = r0 + j; }
         }
@@ -1254,30 +1565,37 @@ struct Service {
     }
 };
 
-// KIND: models of shared key/value rows, of latent rows and gated linear attention (kWalkLatent), or of those with mixtures of experts
-template <typename ET, int QW, int KIND>
+// KIND: models of shared key/value rows, of latent rows and gated linear attention (kWalkLatent), or of those with mixtures of experts.  PARTS: the
+// vectors lie as three bfloat16 parts.
+template <typename ET, int QW, int KIND, bool PARTS>
 __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, ResidentEnd end) {
     constexpr int QE = kQuad / sizeof(ET);
     extern __shared__ __attribute__((aligned(16))) char lds[];
     WalkLds& L = *reinterpret_cast<WalkLds*>(lds);
-    float* xs = reinterpret_cast<float*>(lds + sizeof(WalkLds));
+    WalkTables T;
+    T.phase = reinterpret_cast<int4*>(lds + sizeof(WalkLds));
+    T.group = T.phase + a.n_phases + 1;
+    float* xs = reinterpret_cast<float*>(T.group + (KIND == kWalkMixture ? a.n_phases + 1 : 0));
     float* red = xs + a.lds_xs;
     const int phases = a.n_phases + (a.head ? 1 : 0);
     for (int p = threadIdx.x; p < phases; p += kWalkT) {
         const WalkPhase ph = a.phases[p];
         const int r0 = walk_rows(ph.n, blockIdx.x), rows = walk_rows(ph.n, blockIdx.x + 1) - r0, rq = ph.kpad / QE;
         const uintptr_t w = reinterpret_cast<uintptr_t>(static_cast<const ET*>(ph.w) + (size_t)r0 * ph.kpad);
+        T.phase[p] = make_int4((int)(unsigned)w, (int)(unsigned)(w >> 32), PARTS ? rows : rq ? rows * rq : rows / 2, PARTS ? ph.kpad / kBlockK : rq);
         // choices of few quads begin with another wave in turn
-        L.phase[p] = make_int4((int)(unsigned)w, (int)(unsigned)(w >> 32), rq ? rows * rq : rows / 2, rq);
-        L.group[p] = make_int4(ph.x_off, ph.red_off, ph.group, (int)((unsigned)ph.last << 31 | (unsigned)ph.first << 30 | (unsigned)(rq == 0 && ph.slot & 1 ? kStrWaves / 2 : 0) << 16 | (unsigned)ph.routed));
+        if (KIND == kWalkMixture)
+            T.group[p] = make_int4(PARTS ? ph.x_off / 2 * 3 : ph.x_off, p == a.n_phases ? a.lds_head : ph.red_off, ph.group, (int)((unsigned)ph.last << 31 | (unsigned)ph.first << 30 | (unsigned)(rq == 0 && ph.slot & 1 ? kStrWaves / 2 : 0) << 16 | (unsigned)ph.routed));
     }
-    if (threadIdx.x == 0) L.met = L.ready = L.sent = L.chosen = 0;
+    if (threadIdx.x == 0) L.met = L.ready = L.done = L.sent = L.chosen = 0;
     __syncthreads();
     if (threadIdx.x >= kSvcT) {
-        stream_waves<ET, KIND == kWalkMixture>(L, xs, red, reinterpret_cast<const char*>(red + a.lds_red), slots, phases, a.steps, a.routed);
+        const char* ring = reinterpret_cast<const char*>(red + a.lds_red);
+        if constexpr (PARTS) stream_parts<KIND == kWalkMixture, kFree<KIND>>(L, T, xs, red, ring, slots, phases, a.steps, a.routed, a.n_phases, a.lds_head);
+        else stream_waves<ET, KIND == kWalkMixture, kFree<KIND>>(L, T, xs, red, ring, slots, phases, a.steps, a.routed, a.n_phases, a.lds_head);
         return;
     }
-    Service<ET, QW, KIND> s(a, L, xs, red);
+    Service<ET, QW, KIND, PARTS> s(a, L, T, xs, red);
     const int pos0 = a.state[0], step0 = a.state[1];
     int token = a.token[0];
     if ((unsigned)token >= (unsigned)a.vocab) {
@@ -1301,9 +1619,9 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, Res
 }
 
 // What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.
-size_t walk_lds(const WalkArgs& a) { return sizeof(WalkLds) + sizeof(float) * ((size_t)a.lds_xs + a.lds_red); }
-static_assert(kStrWaves * kQuad == kWalkSlotBytes && kQuad == kWalkRow, "a quad per wave");
-static_assert((kWalkLdsMax - sizeof(WalkLds)) / kWalkSlotBytes == kWalkMaxSlots, "wait_quads counts as many");
+size_t walk_lds(const WalkArgs& a) { return sizeof(WalkLds) + (a.n_phases + 1) * sizeof(int4) * (a.routed ? 2 : 1) + sizeof(float) * ((size_t)a.lds_xs + a.lds_red); }
+static_assert(kStrWaves * kQuad == kWalkSlotBytes && kQuad == kWalkRow && kStrWaves == kWalkStreams, "a quad per wave");
+static_assert((kWalkLdsMax - sizeof(WalkLds) - kWalkMixerLds) / kWalkSlotBytes == kWalkMaxSlots, "wait_quads counts as many");
 
 template <typename ET>
 int walk_launch(const WalkArgs& a, hipStream_t st) {
@@ -1319,10 +1637,16 @@ int walk_launch(const WalkArgs& a, hipStream_t st) {
         }
         return resident_launch(k, kWalkWG, kWalkT, lds, st, a, slots);
     };
-    static std::atomic<bool> opted[6];
-    if (a.kind == kWalkSharedKv) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkSharedKv>, opted[0]) : go(walk_kernel<ET, 4, kWalkSharedKv>, opted[1]);
-    if (a.routed) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkMixture>, opted[4]) : go(walk_kernel<ET, 4, kWalkMixture>, opted[5]);
-    return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkLatent>, opted[2]) : go(walk_kernel<ET, 4, kWalkLatent>, opted[3]);
+    static std::atomic<bool> opted[2][6];
+    auto kind = [&](auto parts) {
+        constexpr bool P = decltype(parts)::value;
+        if (a.kind == kWalkSharedKv) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkSharedKv, P>, opted[P][0]) : go(walk_kernel<ET, 4, kWalkSharedKv, P>, opted[P][1]);
+        if (a.routed) return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkMixture, P>, opted[P][4]) : go(walk_kernel<ET, 4, kWalkMixture, P>, opted[P][5]);
+        return a.width <= 2048 ? go(walk_kernel<ET, 2, kWalkLatent, P>, opted[P][2]) : go(walk_kernel<ET, 4, kWalkLatent, P>, opted[P][3]);
+    };
+    if constexpr (std::is_same<ET, bf16_t>::value)
+        if (a.parts) return kind(std::true_type());
+    return kind(std::false_type());
 }
 template int walk_launch<bf16_t>(const WalkArgs&, hipStream_t);
 template int walk_launch<float>(const WalkArgs&, hipStream_t);

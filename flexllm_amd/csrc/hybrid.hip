@@ -407,18 +407,21 @@ static int create_walk(flexllm_hybrid* m) {
     std::vector<WalkPhase> phases;
     std::vector<WalkRun> runs;
     WalkArgs& a = m->walk;
-    size_t at = 0, longest = 0, sums = 0;
+    size_t at = 0, longest = 0, sums[2] = {0, 0};
     // Linears that nobody waits between are a group: experts' products of a token, whose vectors and sums lie side by side.
     int groups = 0;
-    size_t x_off = 0, red_off = 0;
+    size_t x_off = 0, red_off[2] = {0, 0};
+    std::vector<int> red_offs[2];                         // without and with parts
     auto one = [&](const void* w, int n, int k, bool first, bool last, int routed = 0, int slot = 0, size_t stride = 0, bool same_x = false) {
-        const int rq = k / unit;
-        if (first) x_off = red_off = 0;
-        phases.push_back({w, n, k, groups, first, last, routed, slot, stride, (int)x_off, (int)red_off});
+        if (first) x_off = red_off[0] = red_off[1] = 0;
+        phases.push_back({w, n, k, groups, first, last, routed, slot, stride, (int)x_off, 0});
         if (!same_x) x_off += k;
-        red_off += (size_t)red_rows(n) * (rq ? rq : 1);
-        if ((same_x ? (size_t)k : x_off) > longest) longest = same_x ? k : x_off;
-        if (red_off > sums) sums = red_off;
+        longest = std::max(longest, same_x ? (size_t)k : x_off);
+        for (int p = 0; p < 2; p++) {
+            red_offs[p].push_back((int)red_off[p]);
+            red_off[p] += walk_red(p, n, k, unit);
+            sums[p] = std::max(sums[p], red_off[p]);
+        }
         if (last) groups++;
     };
     auto linear = [&](const void* w, int n, int k) { one(w, n, k, true, true); };
@@ -477,10 +480,22 @@ static int create_walk(flexllm_hybrid* m) {
             runs.push_back(r);
         }
     a.n_phases = (int)phases.size();
+    const size_t others[2] = {sums[0], sums[1]};
     linear(m->head, c.vocab, W);
     a.x_cand = words(2 * kWalkWG);
-    a.lds_xs = (int)longest; a.lds_red = (int)((sums + 255) / 256 * 256);
-    if (a.n_phases >= kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || walk_lds(a) + kWalkMinSlots * kWalkSlotBytes > kWalkLdsMax) return FLEXLLM_OK;
+    // bfloat16 weights meet vectors in parts, half as long again in LDS, where that leaves the ring its slots (mixtures of up to 14336 elements, say)
+    bool fits = false;
+    for (int p = sizeof(ET) == 2; p >= 0 && !fits; p--) {
+        const size_t xw = p ? W / 2 * 3 : W, head = walk_red(p, c.vocab, W, unit);
+        a.parts = p;
+        a.lds_xs = (int)std::max(p ? longest / 2 * 3 : longest, kWalkMixerLds / sizeof(float));
+        a.lds_red = (int)((others[p] + 255) / 256 * 256);
+        if (xw + head > (size_t)a.lds_xs + a.lds_red) a.lds_red = (int)((xw + head - a.lds_xs + 255) / 256 * 256);
+        a.lds_head = (int)xw - a.lds_xs;
+        for (size_t i = 0; i < phases.size(); i++) phases[i].red_off = red_offs[p][i];
+        fits = walk_lds(a) + kWalkMinSlots * kWalkSlotBytes <= kWalkLdsMax;
+    }
+    if (a.n_phases >= kWalkMaxPhases || at * sizeof(float) >= (size_t)1 << 31 || !fits) return FLEXLLM_OK;
     void* told = nullptr;
     FX_HIP(hipHostMalloc(&told, 64, hipHostMallocPortable));
     a.told = m->told = static_cast<int*>(told);

@@ -34,6 +34,20 @@ def test_token_by_token(name, dtype):
     check_lopazen(LOPAZEN[name], dtype, 40, [1], [23, 1])
 
 
+# bfloat16: feed-forwards of 12 and of 16 blocks of 512, of which eight waves have one or two each; the longest vector beside many rows of the head
+@pytest.mark.parametrize("width,ff,vocab", [(2048, 6144, 514), (2048, 8192, 514), (4096, 14336, 128257)])
+def test_long_vectors_in_bfloat16(width, ff, vocab):
+    from flexllm_amd._lib import FlexLLMError
+    from flexllm_amd.lopazen import Lopazen
+    cfg = lc.config([attention(32, 8, 64, ff)], width=width, vocab=vocab)
+    check_lopazen(cfg, "bfloat16", 40, [1], [23, 1])
+    m = Lopazen.from_tensors(cfg, lc.weights(cfg, 5), dtype="bfloat16", max_pos=64)
+    m.set_wait_limit(1)                                    # it is the resident kernel that they take
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.step(m.pool.acquire("t"), [1], [0])
+    m.close()
+
+
 def latent(heads, ff, **kw):
     return nc.latent(heads=heads, dim=128, rot_dim=64, vdim=128, kv_rank=512, scale=192 ** -0.5, mlp=nc.dense(ff) if ff else None, **kw)
 
