@@ -146,11 +146,11 @@ template <typename ET> int shared_kv_store(const SharedKvDims& d, const float* k
 // Few tokens (any size): splits of the visible rows, joined by the one that ends last.  k as above for tokens whose rows are not
 // in the cache yet (they are stored on the way), null when shared_kv_store has been there.  q [tokens][ldq] (heads x dimp),
 // not normed, and o [tokens][ldo] (heads x dim) are ET, or float32 with f32.  norm_w [dimp]: product of the two norms'
-// weights.  Scratch: shared_kv_scratch floats per token; tickets: heads * kTicketPitch ints per
+// weights.  Scratch: shared_kv_scratch(d, 1) floats per token, or shared_kv_scratch(d, most) for any number of tokens up to `most`; tickets: heads * kTicketPitch ints per
 // token (a memory line each: arrivals at one line stand in line), zero before the first call and left zero.  held: rows that
 // there will be at most, as far as the host knows (shared_kv_split_count goes by it); more are correct all the same.
 constexpr int kTicketPitch = 64;
-size_t shared_kv_scratch(const SharedKvDims& d);
+size_t shared_kv_scratch(const SharedKvDims& d, int most);
 int shared_kv_split_count(const SharedKvDims& d, int tokens, int rows);
 template <typename ET> int shared_kv_splits(const SharedKvDims& d, const void* q, int ldq, const float* k, int ldk, const float* norm_w, SharedKvRows<ET> c,
                                             const int* state, int tok0, int tokens, int held, float* scratch, int* tickets, void* o, int ldo, int f32, hipStream_t st);

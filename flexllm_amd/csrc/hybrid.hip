@@ -25,9 +25,12 @@ constexpr int kPieceTokens = 4096;
 constexpr int kHeadRows = 256;          // rows of logits formed at a time
 constexpr int kMaxParts = 8;            // parts that the k of a product with few rows is shared out in,
 constexpr int kPartRows = 4096;         // and rows of all parts together
-// Prompts without a matrix-core attention (float32, long heads) take the attention kernels for few tokens in slices of this many
+// Prompts without a matrix-core attention over latent rows (float32, long heads) take the attention kernels for few tokens in slices of this many
 // (333 tokens of ten layers in float32: 16 at a time 17.2 ms, 64 at a time 14.7 ms: more workgroups per launch, fewer splits to join).
 constexpr int kAbsorbTokens = 64;
+// Tokens of a launch of the splits over shared rows, where the heads or the type keep a prompt from the matrix cores: the more there are, the fewer
+// splits and chains of trips (16 layers of 2048, float32, 333 tokens, a prompt and 5 steps: 64 at a time 12150 us, 128 11810, 512 11680).
+constexpr int kSplitTokens = 512;
 
 static inline int up4(int v) { return (v + 3) / 4 * 4; }
 
@@ -311,7 +314,7 @@ static int create_layer(flexllm_hybrid* m, int i, const flexllm_hybrid_layer_wei
         for (int e = 0; e < d.dim; e++) v[e] *= u[e];
         v.resize(s.dimp, 0.0f);
         FX_TRY(own_floats(m, L.kv_norm, v));
-        const size_t a = shared_kv_scratch(s);
+        const size_t a = shared_kv_scratch(s, 1);
         if (a > m->absorbed) m->absorbed = a;
     } else {
         const int HD = d.heads * d.dim, HV = d.heads * d.vdim;
@@ -590,12 +593,17 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
     FX_TRY(own(m, m->pick, T * m->max_top));
     FX_TRY(own(m, m->pick_w, T * m->max_top));
     int heads = 1, slice = kSmallTokens;
+    size_t scratch = kSmallTokens * m->absorbed;
     for (const HybridLayer& L : m->layers) {
         heads = L.d.heads > heads ? L.d.heads : heads;
-        const bool flash = std::is_same<ET, bf16_t>::value && (L.d.mixer == FLEXLLM_MIX_LATENT ? latent_flash_ok(L.ld) : shared_kv_flash_ok(L.sd));
-        if (L.d.mixer != FLEXLLM_MIX_GLA && !flash) slice = kAbsorbTokens;
+        if (L.d.mixer == FLEXLLM_MIX_LATENT && !(std::is_same<ET, bf16_t>::value && latent_flash_ok(L.ld)))
+            scratch = std::max(scratch, kAbsorbTokens * latent_absorbed_scratch(L.ld));
+        if (L.d.mixer == FLEXLLM_MIX_SHARED_KV && !(std::is_same<ET, bf16_t>::value && shared_kv_flash_ok(L.sd))) {
+            slice = kSplitTokens;
+            scratch = std::max(scratch, shared_kv_scratch(L.sd, kSplitTokens));
+        }
     }
-    FX_TRY(own(m, m->scratch, slice * m->absorbed + 1));
+    FX_TRY(own(m, m->scratch, scratch + 1));
     FX_TRY(own(m, m->tickets, (size_t)slice * heads * kTicketPitch));
     FX_TRY(own(m, m->logits, c.vocab));
     FX_TRY(own(m, m->want, kPieceTokens));
@@ -874,8 +882,8 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
                 if (flash) FX_TRY(shared_kv_flash(L.sd, proj, ldp, L.kv_norm, rows, pos0, T, att, lda, st));
             }
             if (!flash)
-                for (int t0 = 0; t0 < T; t0 += kAbsorbTokens) {
-                    const int n = T - t0 < kAbsorbTokens ? T - t0 : kAbsorbTokens;
+                for (int t0 = 0; t0 < T; t0 += kSplitTokens) {
+                    const int n = T - t0 < kSplitTokens ? T - t0 : kSplitTokens;
                     FX_TRY(shared_kv_splits<ET>(L.sd, proj + (size_t)t0 * ldp, ldp, nullptr, 0, L.kv_norm, rows, s.pos, t0, n, pos0 + t0 + n, m->scratch, m->tickets, att + (size_t)t0 * lda, lda, 0, st));
                 }
         } else if (L.d.mixer == FLEXLLM_MIX_LATENT) {

@@ -102,7 +102,11 @@ static int kv_split_count(const SharedKvDims& d, int tokens, int rows) {
     return s < most ? s : most;
 }
 int shared_kv_split_count(const SharedKvDims& d, int tokens, int rows) { return kv_split_count(d, tokens, rows); }
-size_t shared_kv_scratch(const SharedKvDims& d) { return (size_t)d.heads * kv_split_count(d, 1, d.capacity) * (d.dimp + kKvStats); }
+size_t shared_kv_scratch(const SharedKvDims& d, int most) {
+    size_t splits = 0;                                    // of all tokens together
+    for (int t = 1; t <= most; t++) splits = std::max(splits, (size_t)t * kv_split_count(d, t, d.capacity));
+    return (size_t)d.heads * splits * (d.dimp + kKvStats);
+}
 
 // N consecutive float32 (N a multiple of 4, 16-byte aligned), zeros where there are none.
 template <int N>
