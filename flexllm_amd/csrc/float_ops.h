@@ -30,7 +30,7 @@ template <typename ET> int gemm_float(const GemmArgs& g, hipStream_t st);
 template <typename ET> int gemm_parts(const GemmArgs& g, int most);
 // The grouped form; the table is cut for tiles of tile_rows (64 or 128) rows, gemm_group_tile_rows says which suits.
 template <typename ET> int gemm_grouped(const GemmArgs& g, int tile_rows, hipStream_t st);
-int gemm_group_tile_rows(int rows_per_group);
+template <typename ET> int gemm_group_tile_rows(int rows_per_group);
 
 // ---- linears of one token (csrc/gemv_float.hip) ----------------------------------------------------------------
 // The vector is float32.  Prologue 0: x [tokens][ldx] as it is.  Prologue 1: h = norm(x + normb(y)), where the y part is

@@ -178,15 +178,15 @@ __device__ __forceinline__ void gemm_out(const GemmArgs& g, int row0, int row_en
     gemm_out_loose<ET, W>(g, row0, row_end, col0, stores, smem, acc);
 }
 
-template <typename ET, int WM, int MI, int NI, int NA, int NB>
-struct FloatWalk : GemmWalk<ET, WM, MI, NI, NA, NB> { static constexpr int MIv = MI, NIv = NI; };
+template <typename ET, int WM, int MI, int NI, int NA, int NB, bool ONCE = false>
+struct FloatWalk : GemmWalk<ET, WM, MI, NI, NA, NB, ONCE> { static constexpr int MIv = MI, NIv = NI; };
 
 template <typename ET, class W, int OUT>
 __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmArgs g, int tiles_m, int tiles_n, int stores) {
     extern __shared__ __attribute__((aligned(16))) int8_t gemm_smem[];
     if constexpr (!W::kSumsApart) arguments(g.a, g.w, g.lda, g.ldw, g.m, g.n, g.k, g.row_src, g.tiles, g.n_tiles, g.w_stride, g.parts, g.part_stride, tiles_m, tiles_n);
     int tm, tn, group = 0, row0, row_end;
-    gemm_tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    gemm_tile_of<W::kOnce ? 1 : 8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
     if (g.tiles) {
         if (tm >= g.n_tiles[0]) return;
         const int4 e = g.tiles[tm];
@@ -250,9 +250,9 @@ static int launch_walk_out(const GemmArgs& g, hipStream_t st) {
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
 }
-template <typename ET, int WM, int MI, int NI, int NA, int NB>
+template <typename ET, int WM, int MI, int NI, int NA, int NB, bool ONCE = false>
 static int launch_walk(const GemmArgs& g, hipStream_t st) {
-    using W = FloatWalk<ET, WM, MI, NI, NA, NB>;
+    using W = FloatWalk<ET, WM, MI, NI, NA, NB, ONCE>;
     if constexpr (W::kSumsApart) {
         if (!gemm_wide_ok(g)) return launch_walk_out<ET, W, kOutLoose>(g, st);
         if (g.glu == kGluClamped) return launch_walk_out<ET, W, kOutClamped>(g, st);
@@ -293,7 +293,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_narrow_kernel(GemmArgs g, int n
     if (row0 + rr < g.m && col0 + cc < g.n) g.y32[(size_t)(row0 + rr) * g.ldy32 + (col0 + cc - g.n_split)] = g.bias ? v + g.bias[col0 + cc] : v;
 }
 
-int gemm_group_tile_rows(int rows_per_group) { return rows_per_group >= 96 ? 128 : 64; }
+// 128 rows where most of a group's rows fill most of them.  bfloat16, 8 layers of 64 experts, a whole prompt on 64 and on 128 rows: 65 rows per expert 3261 and 3125 us, 93
+// rows 4025 and 3526.
+template <typename ET>
+int gemm_group_tile_rows(int rows_per_group) { return rows_per_group >= (sizeof(ET) == 2 ? 60 : 96) ? 128 : 64; }
+template int gemm_group_tile_rows<bf16_t>(int);
+template int gemm_group_tile_rows<float>(int);
 
 static int gemm_check(GemmArgs& g, size_t a_rows, int es) {
     if (!g.ldw) g.ldw = g.k;
@@ -412,15 +417,17 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
 
 // Experts: their weights are read once and little else, so the tiles keep as many bytes in flight as LDS holds (1024 tokens, top 6 of
 // 64 experts of 2048 x 2048 and 2048 x 1024: 143 and 90 us; the weights alone are 98 and 49 at 5.5 TB/s).  With fewer than 45 rows
-// per expert most of a wide tile's rows are none, and three workgroups per CU on 64 x 64 hide more of each other's trips.
+// per expert most of a wide tile's rows are none, and three workgroups per CU on 64 x 64 hide more of each other's trips.  Where an expert's rows are
+// one tile its weights are read once, past what the caches hold of the rows, and a die takes all columns of an expert: 64 rows 2429 -> 2217 us (a whole
+// prompt of 8 layers), 500 2983 -> 2827, 1024 3667 -> 3574.  Up to 112 rows on average on 128: at 122 many experts have two tiles (4230 -> 4239 us), at 188 4918 -> 5284.
 template <int BM>
 static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
-    if constexpr (BM == 128) return launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
-    else if (g.group_rows < 45) return launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
-    else return launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
+    if constexpr (BM == 128) return g.group_rows <= 112 ? launch_walk<bf16_t, 2, 4, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
+    else if (g.group_rows < 45) return launch_walk<bf16_t, 2, 2, 2, 3, 3, true>(g, st);
+    else return launch_walk<bf16_t, 2, 2, 4, 4, 4, true>(g, st);
 }
 
 // ---- float32 -----------------------------------------------------------------------------------------------------

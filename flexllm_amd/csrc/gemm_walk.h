@@ -55,10 +55,12 @@ __device__ __forceinline__ int quotient(int a, int d) {
     const int q = (int)((float)a * __builtin_amdgcn_rcpf((float)d)), r = a - q * d;
     return __builtin_amdgcn_readfirstlane(q + (r >= d) - (r < 0));
 }
+// Groups of rows that have a W each: one row tile by all column tiles, which share its rows (ROWS 1).
+template <int ROWS = 8>
 __device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
     const int total = tiles_m * tiles_n, round = id & ~255, in = id & 255, left = min(total - round, 256), die = in & 7;
     const int t = round + die * (left >> 3) + min(die, left & 7) + (in >> 3);
-    constexpr int G = 8;
+    constexpr int G = ROWS;
     const int group = tiles_m <= G ? 0 : quotient(t, G * tiles_n), rows = min(G, tiles_m - group * G), o = t - group * G * tiles_n;
     tn = rows == G ? o / G : quotient(o, rows);
     tm = group * G + o - tn * rows;
@@ -135,8 +137,10 @@ __device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsi
     else asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" : "=&{m0}"(m0) : "s"(to), "v"(off), "s"(base) : "memory");
 }
 
-template <typename ET, int WM, int MI, int NI, int NA, int NB>
+// ONCE: W is read by one row tile alone, and does not take the place of what is read again in the caches.
+template <typename ET, int WM, int MI, int NI, int NA, int NB, bool ONCE = false>
 struct GemmWalk {
+    static constexpr bool kOnce = ONCE;
     using Op = MatrixOp<ET>;
     using Frag = typename Op::Frag;
     using Acc = typename Op::Acc;
@@ -189,16 +193,19 @@ struct GemmWalk {
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
         const unsigned lds_a = lds0 + wv * (AI * 1024), lds_b = lds0 + NA * ASZ + wv * (BI * 1024);
         // A direct load in two halves, with a matrix instruction between them: the address has to be in m0 one wait state ahead of the load.
-        // What `aim` leaves in m0 is an operand of `load`, so that the compiler puts nothing of its own there between them.
+        // What `aim` leaves in m0 is an operand of `load_a` and `load_w`, so that the compiler puts nothing of its own there between them.
         unsigned m0 = 0;
         auto aim = [&](unsigned base, int j) __attribute__((always_inline)) {
             asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(m0) : "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc");
         };
-        auto load = [&](const int8_t* p, unsigned off) __attribute__((always_inline)) { asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p), "{m0}"(m0) : "memory"); };
-        auto load_now = [&](const int8_t* p, unsigned off, unsigned base, int j) __attribute__((always_inline)) {
-            aim(base, j);
-            asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(p), "{m0}"(m0) : "memory");
+        auto load_a = [&](unsigned off, int stage) __attribute__((always_inline)) {
+            asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(a + (size_t)stage * 128), "{m0}"(m0) : "memory");
         };
+        auto load_w = [&](unsigned off, int stage) __attribute__((always_inline)) {
+            if constexpr (ONCE) asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
+            else asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
+        };
+        auto settle = [] __attribute__((always_inline)) { asm volatile("s_nop 0" ::: "memory"); };
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -220,10 +227,10 @@ struct GemmWalk {
         for (int s = 0; s < NA; s++) {
 #pragma unroll
             for (int j = 0; j < BI; j++)
-                if (s < NB && s < nk) load_now(w + (size_t)s * 128, offb[j], lds_b + s * BSZ, j);
+                if (s < NB && s < nk) { aim(lds_b + s * BSZ, j); settle(); load_w(offb[j], s); }
 #pragma unroll
             for (int j = 0; j < AI; j++)
-                if ((s < NA - 1 || j < early_a) && s < nk) load_now(a + (size_t)s * 128, offa[j], lds_a + s * ASZ, j);
+                if ((s < NA - 1 || j < early_a) && s < nk) { aim(lds_a + s * ASZ, j); settle(); load_a(offa[j], s); }
         }
         const int fr = lane & 15, fg = lane >> 4;
         int at[KS];
@@ -284,12 +291,12 @@ struct GemmWalk {
                     const bool there_a = kLoads == 2 || (kLoads == 1 && !last), there_b = kLoads == 2 || (kLoads == 1 && NA > NB && last);
 #pragma unroll
                     for (int j = 0; j < BI; j++) {
-                        if (p == slot_b(j) + 1 && there_b) load(w + (size_t)(last ? kb + 1 : kb) * 128, offb[j]);
+                        if (p == slot_b(j) + 1 && there_b) load_w(offb[j], last ? kb + 1 : kb);
                         if (p == slot_b(j) && there_b) aim(lds_b + sb, j);
                     }
 #pragma unroll
                     for (int j = 0; j < AI; j++) {
-                        if (p == slot_a(j) + 1 && there_a) load(a + (size_t)(last ? ka + 1 : ka) * 128, offa[j]);
+                        if (p == slot_a(j) + 1 && there_a) load_a(offa[j], last ? ka + 1 : ka);
                         if (p == slot_a(j) && there_a) aim(lds_a + sa, j);
                     }
                     __builtin_amdgcn_sched_barrier(0);

@@ -935,7 +935,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
         g = gemm(m->lh, kw, L.w_side, T, L.n_side, W);
         g.n_split = 2 * sf; g.glu = 1 + L.d.glu; g.limit = L.d.shared_limit; g.y = m->lhs; g.ldy = ks; g.y32 = m->lroute; g.ldy32 = ldr;
         FX_TRY(gemm_float<ET>(g, st));
-        const int tile = gemm_group_tile_rows(T * top / L.d.experts);
+        const int tile = gemm_group_tile_rows<ET>(T * top / L.d.experts);
         MoePlan p;
         p.pick = m->lpick; p.pick_w = m->lpick_w; p.pos_of = m->lpos_of; p.row_src = m->lrow_src; p.counts = m->lcounts; p.tiles = m->ltiles; p.n_tiles = m->lntiles;
         FX_TRY(moe_plan(m->lroute, ldr, T, L.d.experts, top, tile, p, st));

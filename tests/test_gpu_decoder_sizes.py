@@ -112,6 +112,13 @@ def test_gemm_tiles(m, n, split, glu, k, dtype):
         assert np.all(np.abs(y32.numpy() - want[:, split:]) <= 1e-5 * np.abs(want[:, split:]) + d)
 
 
+# both sides of the rows per expert from which on there are tiles of 128 rows, and up to which experts' weights are read once; uneven shares of them
+@BOTH
+@pytest.mark.parametrize("experts,top,ff,tokens", [(4, 2, 72, 100), (2, 1, 40, 119), (2, 1, 40, 120), (4, 2, 200, 225), (4, 2, 72, 227)])
+def test_grouped_tiles_of_few_rows(experts, top, ff, tokens, dtype):
+    check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=192), dtype, tokens, [tokens])
+
+
 # grouped products of the experts: tiles of 64 rows, narrow and wide ones, and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
 @BOTH
 @pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70), (4, 2, 100, 130), (2, 1, 40, 130)])
