@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256, WideI8<MI>::per_cu()) void gemm_i8_walk_kernel
         offb[j] = (unsigned)min(col0 + r, n - 1) * (unsigned)k + W::load_byte(r);
     }
     i32x4 acc[MI][NI];
-    W::run(a, w, offa, offb, k / 128, gemm_smem, acc);
+    W::run(a, w, offa, offb, k / 128, gemm_smem, acc, OneTile());
     const int lane = threadIdx.x & 63, fr = lane & 15, fg = lane >> 4;
     const int wr = W::row_of_wave(), wc = W::col_of_wave();
     if constexpr (EPI == kDmaQkv) {

@@ -51,13 +51,14 @@ __device__ __forceinline__ void wait_vmcnt() {                 // s_waitcnt vmcn
 // tiles by one column tile read 33.
 // Quotients stand ahead of the first load, so they are float ones put right by the remainder (exact: a quotient of tiles is below 2^20, and the
 // float one below half off); a division of integers takes three times the instructions.
-__device__ __forceinline__ int quotient(int a, int d) {
+__device__ __forceinline__ int quotient_of_lane(int a, int d) {
     const int q = (int)((float)a * __builtin_amdgcn_rcpf((float)d)), r = a - q * d;
-    return __builtin_amdgcn_readfirstlane(q + (r >= d) - (r < 0));
+    return q + (r >= d) - (r < 0);
 }
+__device__ __forceinline__ int quotient(int a, int d) { return __builtin_amdgcn_readfirstlane(quotient_of_lane(a, d)); }
 // Groups of rows that have a W each: one row tile by all column tiles, which share its rows (ROWS 1).
-template <int ROWS = 8>
-__device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
+template <int ROWS = 8, class Q>
+__device__ __forceinline__ void gemm_tile_by(Q quotient, int id, int tiles_m, int tiles_n, int& tm, int& tn) {
     const int total = tiles_m * tiles_n, round = id & ~255, in = id & 255, left = min(total - round, 256), die = in & 7;
     const int t = round + die * (left >> 3) + min(die, left & 7) + (in >> 3);
     constexpr int G = ROWS;
@@ -65,6 +66,11 @@ __device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, i
     tn = rows == G ? o / G : quotient(o, rows);
     tm = group * G + o - tn * rows;
 }
+
+template <int ROWS = 8>
+__device__ __forceinline__ void gemm_tile_of(int id, int tiles_m, int tiles_n, int& tm, int& tn) { gemm_tile_by<ROWS>(quotient, id, tiles_m, tiles_n, tm, tn); }
+template <int ROWS = 8>                                        // an id of every lane's own
+__device__ __forceinline__ void gemm_tile_of_lane(int id, int tiles_m, int tiles_n, int& tm, int& tn) { gemm_tile_by<ROWS>(quotient_of_lane, id, tiles_m, tiles_n, tm, tn); }
 
 // R words of each of 4/R blocks, as lanes hold them (lane group g of 16 lanes has words g*R .. g*R + R - 1 of a block's row), become four
 // consecutive words per lane: group g then has words 4g .. 4g + 3 of the row through all the blocks, in the order w[0][0], w[0][1] ...
@@ -137,6 +143,25 @@ __device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsi
     else asm volatile("s_mov_b32 %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" : "=&{m0}"(m0) : "s"(to), "v"(off), "s"(base) : "memory");
 }
 
+// The tile of a workgroup that walks one.  A workgroup that walks several (kMany) says besides: more(), whether another tile follows; rows() and cols(),
+// which put the offsets of that one's loads in the place of this one's; out(), this one's outputs, behind which the other one is this one.
+// kTurned: a tile begins at a stage first() of k and ends ahead of it.  Workgroups that begin together and read W once otherwise ask for the same bytes of
+// rows that lie a power of two apart, and those come from a few of the memory's channels (64 experts of 64 x 64 tiles: whole prompt of 64 tokens 2196 -> 2150 us).
+struct OneTile {
+    static constexpr bool kMany = false, kTurned = false;
+    __device__ int first(int) const { return 0; }
+    __device__ int first_of_next(int) const { return 0; }
+    template <class... X> __device__ void rows(X&...) const {}
+    template <class... X> __device__ void cols(X&...) const {}
+};
+__device__ __forceinline__ int first_stage(int group, int tn, int nk) { const int f = tn * 5 + group * 3; return f - quotient(f, nk) * nk; }
+struct OneTurned : OneTile {
+    static constexpr bool kTurned = true;
+    int group, tn;
+    __device__ __forceinline__ OneTurned(int group, int tn) : group(group), tn(tn) {}
+    __device__ __forceinline__ int first(int nk) const { return first_stage(group, tn, nk); }
+};
+
 // ONCE: W is read by one row tile alone, and does not take the place of what is read again in the caches.
 template <typename ET, int WM, int MI, int NI, int NA, int NB, bool ONCE = false>
 struct GemmWalk {
@@ -187,38 +212,50 @@ struct GemmWalk {
 
     // a, w: first byte of k of the operands; offa, offb: byte offsets of this lane's loads behind them; nk: stages.  Nothing else of the
     // workgroup may be on its way to LDS.  Ends with every wave's loads and reads of LDS complete, without a barrier.
-    static __device__ __forceinline__ void run(const int8_t* a, const int8_t* w, const unsigned (&offa)[AI], const unsigned (&offb)[BI], int nk, int8_t* smem,
-                                               Acc (&acc)[MI][NI]) {
+    // Of several tiles (nk >= NA) the ring goes on from one to the next: the last stages of a tile ask for the first ones of the tile behind it, which are on
+    // their way while the outputs leave, and the place of a tile takes neither the trips ahead of its first stage nor the drain behind its last.
+    template <class T>
+    static __device__ __forceinline__ void run(const int8_t* a, const int8_t* w, unsigned (&offa)[AI], unsigned (&offb)[BI], int nk, int8_t* smem,
+                                               Acc (&acc)[MI][NI], T tiles) {
         const int lane = threadIdx.x & 63, wv = wave();
         const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
         const unsigned lds_a = lds0 + wv * (AI * 1024), lds_b = lds0 + NA * ASZ + wv * (BI * 1024);
         // A direct load in two halves, with a matrix instruction between them: the address has to be in m0 one wait state ahead of the load.
         // What `aim` leaves in m0 is an operand of `load_a` and `load_w`, so that the compiler puts nothing of its own there between them.
         unsigned m0 = 0;
+        int first = 0;
+        if constexpr (T::kTurned) first = tiles.first(nk);
+        auto at_k = [&](int stage) __attribute__((always_inline)) {
+            if constexpr (T::kTurned) stage = stage + first >= nk ? stage + first - nk : stage + first;
+            return (size_t)stage * 128;
+        };
         auto aim = [&](unsigned base, int j) __attribute__((always_inline)) {
             asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(m0) : "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc");
         };
         auto load_a = [&](unsigned off, int stage) __attribute__((always_inline)) {
-            asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(a + (size_t)stage * 128), "{m0}"(m0) : "memory");
+            asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(a + at_k(stage)), "{m0}"(m0) : "memory");
         };
         auto load_w = [&](unsigned off, int stage) __attribute__((always_inline)) {
-            if constexpr (ONCE) asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
-            else asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
+            if constexpr (ONCE) asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(off), "s"(w + at_k(stage)), "{m0}"(m0) : "memory");
+            else asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(w + at_k(stage)), "{m0}"(m0) : "memory");
         };
         auto settle = [] __attribute__((always_inline)) { asm volatile("s_nop 0" ::: "memory"); };
+        auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int j = 0; j < NI; j++)
+                for (int j = 0; j < NI; j++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[i][j][r] = 0;
-        // Zeros of its own for every block: from one shared zero the compiler cannot keep the sums in place, and the loop is full of moves.
+                    for (int r = 0; r < 4; r++) acc[i][j][r] = 0;
+            // Zeros of its own for every block: from one shared zero the compiler cannot keep the sums in place, and the loop is full of moves.
 #pragma unroll
-        for (int i = 0; i < MI; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int j = 0; j < NI; j++) {
-                if constexpr (kSumsApart) asm volatile("" : "+a"(acc[i][j])); else asm volatile("" : "+v"(acc[i][j]));
-            }
+                for (int j = 0; j < NI; j++) {
+                    if constexpr (kSumsApart) asm volatile("" : "+a"(acc[i][j])); else asm volatile("" : "+v"(acc[i][j]));
+                }
+        };
+        clear();
         wait_vmcnt<0>();                                        // what the compiler loaded itself stays out of the counts
         // Behind the barrier of stage e: W's loads of stage e + NB over the first half of the last k-step, then A's of e + NA over
         // as many matrix instructions as a k-step has.
@@ -265,12 +302,16 @@ struct GemmWalk {
         int ka = NA - 1, kb = NB - 1;                            // stages kt - 1 + NA and kt - 1 + NB (as numbers: pointers cost the wide tiles spills)
         // left: stages behind this one.  loads: 2 all, 1 what is left for the last stages (the rest of the last barrier's, and W's where it is a stage
         // behind A), 0 none.  No branches among them: those cost a short walk 2 % (250 x 2560 x 2048 in four parts, eight stages on 128 x 128, 11.4 us and 11.2).
-        auto stage = [&](int left, auto next, auto loads) __attribute__((always_inline)) {
+        // turn, where another tile follows: 1 from the last k-step on A's loads are that one's, 2 W's are, 4 the next stage is that one's and is read behind the outputs.
+        auto turning = [&](int left, auto next, auto loads, auto turn) __attribute__((always_inline)) {
 #pragma unroll
             for (int s = 0; s < KS; s++) {
                 constexpr bool kNext = decltype(next)::value;
                 constexpr int kLoads = decltype(loads)::value;
+                constexpr int kTurn = decltype(turn)::value;
                 const bool last = s == KS - 1;
+                if constexpr (kTurn & 1) { if (last) { tiles.rows(offa); ka = -1; } }
+                if constexpr (kTurn & 2) { if (last) { tiles.cols(offb, w); kb = -1; if constexpr (T::kTurned) first = tiles.first_of_next(nk); } }
                 if (last && kNext) {
                     if constexpr (kLoads > 0) wait_vmcnt<in_flight(NA - 2)>(); else wait_stage(left - 1);
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -283,7 +324,7 @@ struct GemmWalk {
                     constexpr int RS = NM / 2 / NR > 0 ? NM / 2 / NR : 1;
                     if (x % RS == 0 && x / RS < NR) {
                         if (!last) read(a1, b1, s + 1, (s + 1) & 1, x / RS);
-                        else if (kNext) read(a2, b2, 0, (s + 1) & 1, x / RS);
+                        else if (kNext && !(kTurn & 4)) read(a2, b2, 0, (s + 1) & 1, x / RS);
                     }
                     // place behind the barrier of this stage (last k-step) or of the one before
                     const int p = last ? x : (s + 1) * NM + x;
@@ -306,13 +347,30 @@ struct GemmWalk {
             a0 = a1; a1 = a2; a2 = a2 == (NA - 1) * ASZ ? 0 : a2 + ASZ;
             b0 = b1; b1 = b2; b2 = b2 == (NB - 1) * BSZ ? 0 : b2 + BSZ;
         };
+        auto stage = [&](int left, auto next, auto loads) __attribute__((always_inline)) { turning(left, next, loads, std::integral_constant<int, 0>()); };
         int left = nk - 1;
+        if constexpr (T::kMany) {
+            using All = std::integral_constant<int, 2>;
+            while (tiles.more()) {
+                for (; left >= NA; left--) stage(left, std::true_type(), All());
+                if constexpr (NA > NB) turning(left--, std::true_type(), All(), std::integral_constant<int, 1>());
+                turning(left--, std::true_type(), All(), std::integral_constant<int, (NA > NB ? 2 : 3)>());
+                for (; left >= 1; left--) stage(left, std::true_type(), All());
+                turning(0, std::true_type(), All(), std::integral_constant<int, 4>());
+                tiles.out(acc);
+                clear();
+#pragma unroll
+                for (int q = 0; q < NR; q++) read(a1, b1, 0, 0, q);
+                left = nk - 1;
+            }
+        }
         if (nk >= NA) {
             for (; left >= NA; left--) stage(left, std::true_type(), std::integral_constant<int, 2>());
             stage(left--, std::true_type(), std::integral_constant<int, 1>());
         }
         for (; left >= 1; left--) stage(left, std::true_type(), std::integral_constant<int, 0>());     // everything is on its way
         stage(0, std::false_type(), std::integral_constant<int, 0>());
+        if constexpr (T::kMany) tiles.out(acc);
     }
 };
 

@@ -119,6 +119,13 @@ def test_grouped_tiles_of_few_rows(experts, top, ff, tokens, dtype):
     check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=192), dtype, tokens, [tokens])
 
 
+# workgroups that walk several tiles of experts: tiles of 64 and of 128 rows, weights read once and not, a last column tile that is not full, more tiles than a
+# workgroup lists at a time, fewer than there are CUs
+@pytest.mark.parametrize("experts,top,ff,tokens", [(20, 2, 1024, 470), (12, 2, 1000, 470), (8, 2, 1032, 700), (4, 1, 328, 257), (4, 2, 4096, 4096)])
+def test_grouped_tiles_of_one_workgroup(experts, top, ff, tokens):
+    check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=256), "bfloat16", tokens, [tokens], max_pos=max(512, tokens))
+
+
 # grouped products of the experts: tiles of 64 rows, narrow and wide ones, and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
 @BOTH
 @pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70), (4, 2, 100, 130), (2, 1, 40, 130)])
