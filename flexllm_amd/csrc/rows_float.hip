@@ -1,6 +1,7 @@
 // Row kernels of the floating-point layers: weight packing, embedding rows, and the fused
 // residual + norm after a sublayer + norm before the next one (with the mixture's weighted sum in front).
 #include "float_ops.h"
+#include "gemm_walk.h"
 
 namespace fx {
 
@@ -40,7 +41,16 @@ static __global__ __launch_bounds__(256) void embed_bf16_kernel(const bf16_t* __
         tk = 0;
     }
     const bf16_t* s = table + (size_t)tk * width;
-    for (int i = threadIdx.x; i < width; i += 256) x[(size_t)blockIdx.x * width + i] = (float)s[i] * scale;
+    float* const to = x + (size_t)blockIdx.x * width;
+    if (width % 8 == 0) {                                  // rows start on 16 bytes
+        for (int i = threadIdx.x * 8; i < width; i += 256 * 8) {
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(s + i);
+#pragma unroll
+            for (int h = 0; h < 8; h += 4) *reinterpret_cast<f32x4*>(to + i + h) = f32x4{(float)v[h] * scale, (float)v[h + 1] * scale, (float)v[h + 2] * scale, (float)v[h + 3] * scale};
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i < width; i += 256) to[i] = (float)s[i] * scale;
 }
 int embed_rows_bf16(const bf16_t* table, float scale, const int* tokens, int n, float* x, int width, int vocab, int* err, hipStream_t st) {
     embed_bf16_kernel<<<n, 256, 0, st>>>(table, scale, tokens, x, width, vocab, err);
@@ -119,67 +129,92 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
 }
 
 // The same for widths that are a multiple of 4 and at most 256 * 4 * V: the row stays in registers, 16-byte accesses.
-template <typename ET, int V>
+// What bounds it: up to a few hundred rows the chain of trips to memory, so that all that does not hang on another trip's answer is asked for at the
+// start (norm weights, all parts of y, the places of a mixture's rows, then those rows together); with thousands of rows the memory's rate.
+//TIMES
+template <typename ET, int V, bool MIX>
 __global__ __launch_bounds__(256) void norm_rows_vec_kernel(RowArgs a) {
+    arguments(a.x, a.x_new, a.x0, a.y, a.ldy, a.y_parts, a.y_stride, a.gb, a.g, a.width, a.h, a.ldh, a.rows_src, a.ys, a.top);
     __shared__ float red[4];
     const int t = threadIdx.x, r = blockIdx.x, n4 = a.width >> 2;
-    const float* x = a.x + (size_t)(a.rows_src ? a.rows_src[r] : r) * a.width;
-    float* x_new = (a.x_new ? a.x_new : a.x) + (size_t)r * a.width;
-    const bool mix = a.ys != nullptr, have_y = a.y || mix;
-    f32x4 v[V];
+    const bool have_y = a.y || MIX, post = have_y && a.gb;
+    int at[V];                                             // a lane behind the row's end reads its last piece and has zeros
+    bool in[V];
 #pragma unroll
-    for (int i = 0; i < V; i++) {
-        const int c = t + i * 256;
-        v[i] = c < n4 ? *reinterpret_cast<const f32x4*>(x + c * 4) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < V; i++) { in[i] = t + i * 256 < n4; at[i] = min(t + i * 256, n4 - 1) * 4; }
+    auto get = [&](f32x4 (&d)[V], const float* from) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < V; i++) d[i] = *reinterpret_cast<const f32x4*>(from + at[i]);
+    };
+    f32x4 v[V], y[V], x0[V], gb[V], g[V];
+    get(v, a.x + (size_t)(a.rows_src ? a.rows_src[r] : r) * a.width);
+    if (a.y) get(y, a.y + (size_t)r * a.ldy);
+    if (a.x0) get(x0, a.x0 + (size_t)r * a.width);
+    if (post) get(gb, a.gb);
+    if (a.h) get(g, a.g);
+    if (a.y)
+        for (int p = 1; p < a.y_parts; p += 3) {
+            f32x4 u[3][V];
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                if (p + q < a.y_parts) get(u[q], a.y + (p + q) * a.y_stride + (size_t)r * a.ldy);
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                if (p + q < a.y_parts)
+#pragma unroll
+                    for (int i = 0; i < V; i++) y[i] += u[q][i];
+        }
+    if constexpr (MIX) {
+        constexpr int K = V > 2 ? 4 : 8;
+        const float sg = a.y ? sigmoid_f(a.route[(size_t)r * a.ld_route + a.experts]) : 1.0f;
+        f32x4 sum[V];
+#pragma unroll
+        for (int i = 0; i < V; i++) sum[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k0 = 0; k0 < a.top; k0 += K) {
+            f32x4 u[K][V];
+            float w[K];
+            int pos[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const int k1 = r * a.top + min(k0 + k, a.top - 1);
+                w[k] = a.pick_w[k1];
+                pos[k] = a.pos_of[k1];
+            }
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if (k0 + k < a.top) get(u[k], a.ys + (size_t)pos[k] * a.ldy);
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if (k0 + k < a.top)
+#pragma unroll
+                    for (int i = 0; i < V; i++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) sum[i][e] = fma_f(w[k], u[k][i][e], sum[i][e]);
+        }
+#pragma unroll
+        for (int i = 0; i < V; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[i][e] = a.y ? fma_f(sg, y[i][e], sum[i][e]) : sum[i][e];
     }
     if (have_y || a.x0) {
-        f32x4 y[V];
-        float ss = 0.0f, sg = 1.0f;
-        if (mix && a.y) sg = sigmoid_f(a.route[(size_t)r * a.ld_route + a.experts]);
+        float rs = 1.0f;
+        if (post) {
+            float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < V; i++) {
-            const int c = t + i * 256;
-            y[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (c < n4) {
-                if (mix) {
-                    for (int k = 0; k < a.top; k++) {
-                        const float w = a.pick_w[r * a.top + k];
-                        const f32x4 u = *reinterpret_cast<const f32x4*>(a.ys + (size_t)a.pos_of[r * a.top + k] * a.ldy + c * 4);
+            for (int i = 0; i < V; i++)
 #pragma unroll
-                        for (int e = 0; e < 4; e++) y[i][e] = fma_f(w, u[e], y[i][e]);
-                    }
-                    if (a.y) {
-                        const f32x4 u = sum_parts<f32x4>(a, (size_t)r * a.ldy + c * 4);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) y[i][e] = fma_f(sg, u[e], y[i][e]);
-                    }
-                } else if (a.y) {
-                    y[i] = sum_parts<f32x4>(a, (size_t)r * a.ldy + c * 4);
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; e++) ss = fma_f(y[i][e], y[i][e], ss);
+                for (int e = 0; e < 4; e++) ss = in[i] ? fma_f(y[i][e], y[i][e], ss) : ss;
+            rs = 1.0f / sqrtf(block_sum<4>(ss, red) / (float)a.width + a.eps);
         }
-        const bool post = have_y && a.gb;
-        const float rs = post ? 1.0f / sqrtf(block_sum<4>(ss, red) / (float)a.width + a.eps) : 1.0f;
+        float* x_new = (a.x_new ? a.x_new : a.x) + (size_t)r * a.width;
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const int c = t + i * 256;
-            if (c >= n4) continue;
-            if (post) {
-                const f32x4 gb = *reinterpret_cast<const f32x4*>(a.gb + c * 4);
+            if (have_y) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[i][e] = v[i][e] + y[i][e] * rs * gb[e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[i][e] = v[i][e] + y[i][e];
+                for (int e = 0; e < 4; e++) v[i][e] = v[i][e] + (post ? y[i][e] * rs * gb[i][e] : y[i][e]);
             }
-            if (a.x0) {
-                const f32x4 u = *reinterpret_cast<const f32x4*>(a.x0 + (size_t)r * a.width + c * 4);
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[i][e] += u[e];
-            }
-            if (!a.rows_src) *reinterpret_cast<f32x4*>(x_new + c * 4) = v[i];
+            if (a.x0) v[i] += x0[i];
+            if (in[i] && !a.rows_src) *reinterpret_cast<f32x4*>(x_new + at[i]) = v[i];
         }
     }
     if (!a.h) return;
@@ -187,23 +222,21 @@ __global__ __launch_bounds__(256) void norm_rows_vec_kernel(RowArgs a) {
 #pragma unroll
     for (int i = 0; i < V; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) ss = fma_f(v[i][e], v[i][e], ss);
+        for (int e = 0; e < 4; e++) ss = in[i] ? fma_f(v[i][e], v[i][e], ss) : ss;
     const float rx = 1.0f / sqrtf(block_sum<4>(ss, red) / (float)a.width + a.eps);
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const int c = t + i * 256;
-        if (c >= n4) continue;
-        const f32x4 g = *reinterpret_cast<const f32x4*>(a.g + c * 4);
+        if (!in[i]) continue;
         f32x4 o;
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = v[i][e] * rx * g[e];
+        for (int e = 0; e < 4; e++) o[e] = v[i][e] * rx * g[i][e];
         if (a.h_f32 || std::is_same<ET, float>::value) {
-            *reinterpret_cast<f32x4*>(static_cast<float*>(a.h) + (size_t)r * a.ldh + c * 4) = o;
+            *reinterpret_cast<f32x4*>(static_cast<float*>(a.h) + (size_t)r * a.ldh + at[i]) = o;
         } else {
             bf16x4 b;
 #pragma unroll
             for (int e = 0; e < 4; e++) b[e] = (bf16_t)o[e];
-            *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(a.h) + (size_t)r * a.ldh + c * 4) = b;
+            *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(a.h) + (size_t)r * a.ldh + at[i]) = b;
         }
     }
 }
@@ -212,9 +245,14 @@ template <typename ET>
 int norm_rows(const RowArgs& a, hipStream_t st) {
     FX_REQUIRE(a.x && a.rows > 0 && a.width > 0 && a.width <= 16384 && (!a.h || (a.g && a.ldh >= a.width)), "norm_rows: rows=%d width=%d", a.rows, a.width);
     const bool vec = a.width % 4 == 0 && a.ldy % 4 == 0 && a.ldh % 4 == 0;
-    if (vec && a.width <= 1024) norm_rows_vec_kernel<ET, 1><<<a.rows, 256, 0, st>>>(a);
-    else if (vec && a.width <= 2048) norm_rows_vec_kernel<ET, 2><<<a.rows, 256, 0, st>>>(a);
-    else if (vec && a.width <= 4096) norm_rows_vec_kernel<ET, 4><<<a.rows, 256, 0, st>>>(a);
+    auto launch = [&](auto mix) {
+        constexpr bool MIX = decltype(mix)::value;
+        if (a.width <= 1024) norm_rows_vec_kernel<ET, 1, MIX><<<a.rows, 256, 0, st>>>(a);
+        else if (a.width <= 2048) norm_rows_vec_kernel<ET, 2, MIX><<<a.rows, 256, 0, st>>>(a);
+        else norm_rows_vec_kernel<ET, 4, MIX><<<a.rows, 256, 0, st>>>(a);
+    };
+    if (vec && a.width <= 4096 && a.ys) launch(std::true_type());
+    else if (vec && a.width <= 4096) launch(std::false_type());
     else norm_rows_kernel<ET><<<a.rows, 256, a.width * sizeof(float), st>>>(a);
     FX_LAUNCH_CHECK();
     return FLEXLLM_OK;
