@@ -675,16 +675,18 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 }
 
 // A linear behind a norm, for T tokens of a step: every token reads the weights (from L2, behind the first) under its own norm's
-// prologue while that is cheap, else the norms have a launch of their own (5 us) ahead of one pass over the weights.
-// Rows of at most 4 KiB, a piece per thread, are cheap up to four tokens: 16 layers of 2048, bfloat16, three tokens 945 us against 1107
-// (with a recurrence in every second layer 1208 and 1370), four 1013 and 1114 (1349 and 1480), six 1243 and 1203.
-// Longer rows and more tokens while the bytes read again are few.  A mixture of 8 layers of 2048 in float32, four tokens, 4161 rows
-// (97 MiB) read again or not: 1369 and 1404 us; five tokens (130 MiB) 1655 and 1686; 16 layers of 2048 in float32, two tokens, 16384 rows (128
-// MiB): 1541 and 1453, five, 3072 rows (96 MiB): 1680 and 1750.  Four layers of 4096 in bfloat16, two tokens, 28672 rows (224 MiB): 633 and 579,
-// in float32 (16 KiB), four tokens, up to 240 MiB: 1224 and 1175.
+// prologue while the bytes read again are few, else the norms have a launch of their own (3.7 us) ahead of one pass over the weights.
+// bfloat16, 16 layers of 2048, whole steps, us, by tokens, where up to four read rows of 4 KiB again whatever their number, and now: 2 946 and 925, 3 1050
+// and 960, 4 1117 and 942; with a recurrence in every second layer 1129 and 1084, 1293 and 1148, 1402 and 1204.  Limits of 0, 20 and 40 MiB are
+// the same to 1 % there; a mixture's shared linears (17 MB) want to be read again by two tokens: 836 with 0, 812 with 20, 790 with 40.
+// float32: rows of at most 4 KiB, a piece per thread, up to four tokens.  Longer rows and more tokens while the bytes read again are few.  A mixture of 8
+// layers of 2048, four tokens, 4161 rows (97 MiB) read again or not: 1369 and 1404 us; five tokens (130 MiB) 1655 and 1686; 16 layers of 2048, two
+// tokens, 16384 rows (128 MiB): 1541 and 1453, five, 3072 rows (96 MiB): 1680 and 1750; four layers of 4096 (16 KiB), four tokens, up to 240 MiB: 1224 and 1175.
 static bool short_rows(int kpad, int es) { return kpad * es <= 4096; }
 static bool reads_again(int T, int n, int kpad, int es) {
-    return T == 1 || (T <= 4 && short_rows(kpad, es)) || (size_t)(T - 1) * n * kpad * es <= (size_t)(kpad * es > 8192 ? 72 : T == 2 ? 104 : 240) << 20;
+    const size_t again = (size_t)(T - 1) * n * kpad * es;
+    if (es == 2) return again <= (size_t)40 << 20;
+    return T == 1 || (T <= 4 && short_rows(kpad, es)) || again <= (size_t)(kpad * es > 8192 ? 72 : T == 2 ? 104 : 240) << 20;
 }
 
 // ---- one to kSmallTokens tokens, behind which there are at most `held` ------------------------------------------------
@@ -743,7 +745,8 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
     auto to_y = [&](const void* w, int k, const float* v, int ldv, const float* gb, bool shared) {      // shared: k may be shared out
         GemvArgs a = base(w, W, k);
         a.x = v; a.ldx = ldv; a.n_split = 0; a.out32 = m->y; a.ldo32 = W;
-        a.per_token = T > 1 && T <= 4 && short_rows(kw, sizeof(ET));      // then the next linear's prologue takes the sum as it is
+        // each token for itself: then the next linear's prologue takes the sum as it is
+        a.per_token = T > 1 && T <= 4 && short_rows(kw, sizeof(ET)) && (sizeof(ET) == 4 || !shared);
         if (T > 1 && !a.per_token && shared) { a.parts = gemv_parts<ET>(W, a.kpad, kMaxParts); a.part_stride = (size_t)T * W; }
         pending(gb, a.parts);
         return gemv_float<ET>(a, 0, T, st);

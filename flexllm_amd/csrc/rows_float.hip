@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(RowArgs a) {
 // The same for widths that are a multiple of 4 and at most 256 * 4 * V: the row stays in registers, 16-byte accesses.
 // What bounds it: up to a few hundred rows the chain of trips to memory, so that all that does not hang on another trip's answer is asked for at the
 // start (norm weights, all parts of y, the places of a mixture's rows, then those rows together); with thousands of rows the memory's rate.
-//TIMES
+// us, requests: lopazen-1b 5 tokens 1024 -> 973, 100 tokens 1400 -> 1345, nifunex-1b-moe 64 tokens 2125 -> 2094; 1000 rows and more as before.
 template <typename ET, int V, bool MIX>
 __global__ __launch_bounds__(256) void norm_rows_vec_kernel(RowArgs a) {
     arguments(a.x, a.x_new, a.x0, a.y, a.ldy, a.y_parts, a.y_stride, a.gb, a.g, a.width, a.h, a.ldh, a.rows_src, a.ys, a.top);

@@ -174,6 +174,13 @@ def test_experts_down(top, ff, shared, width, dtype):
     check_nifunex(cfg, dtype, 20, [1], [3])
 
 
+# gate/up weights that two tokens of a step just still read again, and just not; three and four tokens do not
+@pytest.mark.parametrize("ff", [5120, 5121])
+def test_step_of_several_tokens_reads_weights_once(ff):
+    check_lopazen(lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff)), lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(72))], width=2048),
+                  "bfloat16", 12, [2], [3], [4])
+
+
 @BOTH
 @pytest.mark.parametrize("ff", [88, 2050])
 def test_infinite_units(ff, dtype):
