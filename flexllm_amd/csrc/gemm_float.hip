@@ -507,6 +507,10 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         g.n = g.n_split;
     }
     if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
+    // With one row tile the weights are read once: past what the caches hold of the rows, and from another stage of k on in every workgroup.  Whole prompts, us:
+    // layers of 2048 (16), 33 rows 1197 -> 1136, 64 1273 -> 1232, 128 1423 -> 1416; of 4096 (4), 33 764 -> 695, 65 804 -> 716, 128 865 -> 813.  Where row tiles
+    // share the weights the turned stages give nothing up to 500 rows and cost 2 to 4 % beyond.
+    const bool one = g.m <= 64, one_wide = g.m <= 128;
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
         case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
@@ -517,9 +521,9 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
             case 128: return launch_walk<bf16_t, 2, 4, 8, 4, 3>(g, st);
             default: return launch_walk<bf16_t, 2, 3, 8, 4, 3>(g, st);
         }
-        case 2: return launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
-        case 3: return launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
-        case 4: return launch_walk<bf16_t, 2, 2, 2, 4, 4>(g, st);
+        case 2: return one_wide ? launch_walk<bf16_t, 2, 4, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
+        case 3: return one ? launch_walk<bf16_t, 2, 2, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
+        case 4: return one ? launch_walk<bf16_t, 2, 2, 2, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 2, 2, 4, 4>(g, st);
         default: return launch_walk<bf16_t, 2, 4, 4, 2, 2>(g, st);
     }
 }

@@ -154,7 +154,8 @@ struct OneTile {
     template <class... X> __device__ void rows(X&...) const {}
     template <class... X> __device__ void cols(X&...) const {}
 };
-__device__ __forceinline__ int first_stage(int group, int tn, int nk) { const int f = tn * 5 + group * 3; return f - quotient(f, nk) * nk; }
+// (As many stages as a ring holds are asked for at once, in whatever order: those stay in theirs.)
+__device__ __forceinline__ int first_stage(int group, int tn, int nk) { const int f = tn * 5 + group * 3; return nk <= 4 ? 0 : f - quotient(f, nk) * nk; }
 struct OneTurned : OneTile {
     static constexpr bool kTurned = true;
     int group, tn;

@@ -42,6 +42,14 @@ def test_small_tiles_in_pieces(m, n, split, glu, dtype):
     floats.test_gemm_tiles(m, n, split, glu, 320, dtype)
 
 
+# one row tile, whose weights are read once and from another stage of k on in every workgroup: one stage, as many as the ring holds and more, the first row
+# that takes a second tile
+@pytest.mark.parametrize("k", floats.GEMM_K)
+@pytest.mark.parametrize("m,n,split,glu", [(33, 132, 132, 0), (64, 2060, 1030, 0), (64, 16380, 16380, 1), (65, 6144, 6144, 2), (100, 2048, 0, 0), (128, 12286, 12286, 0), (129, 6144, 6144, 0)])
+def test_one_row_tile(m, n, split, glu, k):
+    floats.test_gemm_tiles(m, n, split, glu, k, "bfloat16")
+
+
 @pytest.mark.parametrize("rows,m,n", [(r, *FLOAT[r]) for r in FLOAT] + [(0, 129, 772), (0, 1300, 330), (0, 40, 132)])
 @pytest.mark.parametrize("cut", [0, 2])
 def test_unit_behind_a_bias(rows, m, n, cut):
