@@ -6,6 +6,8 @@
 // tokens held, take 43 us each for 122 MB (17 us at the rate of a read stream).  Here a link costs an exchange between resident
 // workgroups, 1.3 us behind the slowest of them, and the weights, which do not hang on the activations, are asked for ahead of it: 33 us per
 // layer, 771 -> 595 us per token (four layers of 4096: 535 -> 466; ten layers, six of them twice, float32: 1098 -> 903).
+// bfloat16 products on the matrix cores, the vector as three parts: 595 -> 566 us per token, with latent and recurrent layers in turn 713 -> 692, with mixtures
+// 520 -> 516; four layers of 4096, whose quads are the weights' stream, 462 and 461, 522 and 525.
 // Eight of a workgroup's twelve waves ("stream waves") do nothing but walk through the workgroup's rows of all linears.  The other four ("service
 // waves") wait for the vectors, norm them, attend, finish the sums.  They meet at workgroup barriers: the vector is in LDS / the sums
 // are in LDS.  Answers of vector memory return to a wave in order, so a wave that streams could not see a word of another workgroup before its weights.
