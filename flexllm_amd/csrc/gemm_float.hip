@@ -221,8 +221,7 @@ __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmA
     }
     f32x4 acc[W::MIv][W::NIv];
     const int8_t *const a = static_cast<const int8_t*>(g.a) + (size_t)k0 * 128, *const w = static_cast<const int8_t*>(g.w) + (size_t)group * g.w_stride * sizeof(ET) + (size_t)k0 * 128;
-    if constexpr (W::kOnce) W::run(a, w, offa, offb, k1 - k0, gemm_smem, acc, OneTurned(group, tn));
-    else W::run(a, w, offa, offb, k1 - k0, gemm_smem, acc, OneTile());
+    W::run(a, w, offa, offb, k1 - k0, gemm_smem, acc, OneTile());
     const int r0 = row0 + W::row_of_wave(), c0 = col0 + W::col_of_wave();
     gemm_out<ET, W, OUT>(g, r0, row_end, c0, stores, gemm_smem, acc);
 }
@@ -231,11 +230,11 @@ __global__ __launch_bounds__(256, W::per_cu()) void gemm_float_walk_kernel(GemmA
 // rows lie is three trips (tile table, row numbers, rows), then the ring filled and the outputs left.  A workgroup makes the trips once for kListed tiles
 // (the offsets of their rows and what else there is to a tile stand in LDS behind the ring), and the ring goes on from one to the next.  Whole prompts of 8 layers
 // of 64 experts, top 6, us: 500 tokens 2850 -> 2698, 700 3120 -> 2950, 1024 3565 -> 3470, 2000 4920 -> 4690, 4000 8040 -> 7610 (of these, where experts are one tile, 1.5 to 2 %
-// are the turned stages).  The weights come at 4.1 TB/s where the tiles of 1024 tokens are 4.2 to 5 rounds of 256.
+// were tiles that began at different stages of k, which they do no more).  The weights come at 4.1 TB/s where the tiles of 1024 tokens are 4.2 to 5 rounds of 256.
 constexpr int kListed = 16;
 template <typename ET, class W, int OUT>
 struct GroupTiles {
-    static constexpr bool kMany = true, kTurned = W::kOnce;
+    static constexpr bool kMany = true;
     static constexpr int kRowsAt = W::kLds, kTileAt = kRowsAt + kListed * W::BM * 4, kLds = kTileAt + kListed * 16;
     static_assert(kLds <= 160 * 1024, "ring and list");
     const GemmArgs& g;
@@ -246,9 +245,6 @@ struct GroupTiles {
         return make_int4(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y), __builtin_amdgcn_readfirstlane(t.z), __builtin_amdgcn_readfirstlane(t.w));
     }
     __device__ __forceinline__ bool more() const { return at + 1 < count; }
-    __device__ __forceinline__ int first_of(int i, int nk) const { const int4 t = tile(i); return first_stage(t.x, t.w, nk); }
-    __device__ __forceinline__ int first(int nk) const { return first_of(at, nk); }
-    __device__ __forceinline__ int first_of_next(int nk) const { return first_of(at + 1, nk); }
     __device__ __forceinline__ void rows_of(int i, unsigned (&offa)[W::AI]) const {
         const unsigned* const off = reinterpret_cast<const unsigned*>(smem + kRowsAt) + i * W::BM;
 #pragma unroll
@@ -507,9 +503,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         g.n = g.n_split;
     }
     if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
-    // With one row tile the weights are read once: past what the caches hold of the rows, and from another stage of k on in every workgroup.  Whole prompts, us:
-    // layers of 2048 (16), 33 rows 1197 -> 1136, 64 1273 -> 1232, 128 1423 -> 1416; of 4096 (4), 33 764 -> 695, 65 804 -> 716, 128 865 -> 813.  Where row tiles
-    // share the weights the turned stages give nothing up to 500 rows and cost 2 to 4 % beyond.
+    // With one row tile the weights are read once: past what the caches hold of the rows.  Whole prompts, us, read by ordinary loads and so: layers of 2048 (16),
+    // 33 rows 1196 and 1157, 64 1268 and 1252, 128 1416 and 1417; of 4096 (4), 33 760 and 734, 64 786 and 771, 128 867 and 852.
     const bool one = g.m <= 64, one_wide = g.m <= 128;
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
@@ -531,8 +526,8 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
 // Experts: their weights are read once and little else, so the tiles keep as many bytes in flight as LDS holds (1024 tokens, top 6 of
 // 64 experts of 2048 x 2048 and 2048 x 1024: 143 and 90 us; the weights alone are 98 and 49 at 5.5 TB/s).  With fewer than 45 rows
 // per expert most of a wide tile's rows are none, and three workgroups per CU on 64 x 64 hide more of each other's trips.  Where an expert's rows are
-// one tile its weights are read once, past what the caches hold of the rows, and a die takes all columns of an expert: 64 rows 2429 -> 2217 us (a whole
-// prompt of 8 layers), 500 2983 -> 2827, 1024 3667 -> 3574.  Up to 112 rows on average on 128: at 122 many experts have two tiles (4230 -> 4239 us), at 188 4918 -> 5284.
+// one tile its weights are read once, past what the caches hold of the rows, and a die takes all columns of an expert: 64 rows 2394 -> 2265 us (a whole
+// prompt of 8 layers), 500 2886 -> 2793, 1024 3588 -> 3537.  Up to 112 rows on average on 128: at 122 many experts have two tiles (4230 -> 4239 us), at 188 4918 -> 5284.
 template <int BM>
 static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;

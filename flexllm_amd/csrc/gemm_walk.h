@@ -145,22 +145,13 @@ __device__ __forceinline__ void load_to_lds(const void* base, unsigned off, unsi
 
 // The tile of a workgroup that walks one.  A workgroup that walks several (kMany) says besides: more(), whether another tile follows; rows() and cols(),
 // which put the offsets of that one's loads in the place of this one's; out(), this one's outputs, behind which the other one is this one.
-// kTurned: a tile begins at a stage first() of k and ends ahead of it.  Workgroups that begin together and read W once otherwise ask for the same bytes of
-// rows that lie a power of two apart, and those come from a few of the memory's channels (64 experts of 64 x 64 tiles: whole prompt of 64 tokens 2196 -> 2150 us).
+// Every tile walks k from its beginning: a sum's order does not hang on where its tile lies or on how many rows there are.  (Workgroups that read W once and begin
+// together ask for the same bytes of rows a power of two apart.  Begun at different stages of k, products of up to 128 rows were 2 to 5 % faster, but a row's sums
+// were then others than on the tiles of longer prompts, and what is rounded to bfloat16 behind them as well.)
 struct OneTile {
-    static constexpr bool kMany = false, kTurned = false;
-    __device__ int first(int) const { return 0; }
-    __device__ int first_of_next(int) const { return 0; }
+    static constexpr bool kMany = false;
     template <class... X> __device__ void rows(X&...) const {}
     template <class... X> __device__ void cols(X&...) const {}
-};
-// (As many stages as a ring holds are asked for at once, in whatever order: those stay in theirs.)
-__device__ __forceinline__ int first_stage(int group, int tn, int nk) { const int f = tn * 5 + group * 3; return nk <= 4 ? 0 : f - quotient(f, nk) * nk; }
-struct OneTurned : OneTile {
-    static constexpr bool kTurned = true;
-    int group, tn;
-    __device__ __forceinline__ OneTurned(int group, int tn) : group(group), tn(tn) {}
-    __device__ __forceinline__ int first(int nk) const { return first_stage(group, tn, nk); }
 };
 
 // ONCE: W is read by one row tile alone, and does not take the place of what is read again in the caches.
@@ -224,21 +215,15 @@ struct GemmWalk {
         // A direct load in two halves, with a matrix instruction between them: the address has to be in m0 one wait state ahead of the load.
         // What `aim` leaves in m0 is an operand of `load_a` and `load_w`, so that the compiler puts nothing of its own there between them.
         unsigned m0 = 0;
-        int first = 0;
-        if constexpr (T::kTurned) first = tiles.first(nk);
-        auto at_k = [&](int stage) __attribute__((always_inline)) {
-            if constexpr (T::kTurned) stage = stage + first >= nk ? stage + first - nk : stage + first;
-            return (size_t)stage * 128;
-        };
         auto aim = [&](unsigned base, int j) __attribute__((always_inline)) {
             asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(m0) : "s"(__builtin_amdgcn_readfirstlane(base)), "i"(j * 1024) : "scc");
         };
         auto load_a = [&](unsigned off, int stage) __attribute__((always_inline)) {
-            asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(a + at_k(stage)), "{m0}"(m0) : "memory");
+            asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(a + (size_t)stage * 128), "{m0}"(m0) : "memory");
         };
         auto load_w = [&](unsigned off, int stage) __attribute__((always_inline)) {
-            if constexpr (ONCE) asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(off), "s"(w + at_k(stage)), "{m0}"(m0) : "memory");
-            else asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(w + at_k(stage)), "{m0}"(m0) : "memory");
+            if constexpr (ONCE) asm volatile("global_load_lds_dwordx4 %0, %1 nt" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
+            else asm volatile("global_load_lds_dwordx4 %0, %1" :: "v"(off), "s"(w + (size_t)stage * 128), "{m0}"(m0) : "memory");
         };
         auto settle = [] __attribute__((always_inline)) { asm volatile("s_nop 0" ::: "memory"); };
         auto clear = [&]() __attribute__((always_inline)) {
@@ -312,7 +297,7 @@ struct GemmWalk {
                 constexpr int kTurn = decltype(turn)::value;
                 const bool last = s == KS - 1;
                 if constexpr (kTurn & 1) { if (last) { tiles.rows(offa); ka = -1; } }
-                if constexpr (kTurn & 2) { if (last) { tiles.cols(offb, w); kb = -1; if constexpr (T::kTurned) first = tiles.first_of_next(nk); } }
+                if constexpr (kTurn & 2) { if (last) { tiles.cols(offb, w); kb = -1; } }
                 if (last && kNext) {
                     if constexpr (kLoads > 0) wait_vmcnt<in_flight(NA - 2)>(); else wait_stage(left - 1);
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -126,6 +126,23 @@ def test_grouped_tiles_of_one_workgroup(experts, top, ff, tokens):
     check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=256), "bfloat16", tokens, [tokens], max_pos=max(512, tokens))
 
 
+# tiles of 64 x 64, 64 x 128 and 128 x 128, with more stages of k than the ring holds
+@pytest.mark.parametrize("tokens", [40, 50, 100])
+def test_experts_in_another_order(tokens):
+    """An expert's sums do not hang on its number: with two experts that change places, logits stay the same bit for bit."""
+    from flexllm_amd.nifunex import Nifunex
+    cfg = nc.config([nc.gla(heads=1, mlp=nc.moe(2, 2, 512, 1.5, 0))], width=1024)
+    w, toks = nc.weights(cfg, 11), nc.tokens(cfg, tokens)
+    other = {n: w[n.replace(".e0.", ".e#.").replace(".e1.", ".e0.").replace(".e#.", ".e1.")] for n in w}
+    other["l0.mlp.router"] = w["l0.mlp.router"][::-1].copy()
+    got = []
+    for weights in w, other:
+        m = Nifunex.from_tensors(cfg, weights, dtype="bfloat16", max_pos=128)
+        got.append(logits(m, toks, [tokens]))
+        m.close()
+    assert np.array_equal(got[0], got[1])
+
+
 # grouped products of the experts: tiles of 64 rows, narrow and wide ones, and of 128 rows, experts with a tile and a row more, columns that do not fill a tile
 @BOTH
 @pytest.mark.parametrize("experts,top,ff,tokens", [(2, 1, 40, 200), (3, 2, 100, 194), (4, 4, 72, 129), (8, 1, 130, 70), (4, 2, 100, 130), (2, 1, 40, 130)])

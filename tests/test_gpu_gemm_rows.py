@@ -42,12 +42,27 @@ def test_small_tiles_in_pieces(m, n, split, glu, dtype):
     floats.test_gemm_tiles(m, n, split, glu, 320, dtype)
 
 
-# one row tile, whose weights are read once and from another stage of k on in every workgroup: one stage, as many as the ring holds and more, the first row
+# one row tile, whose weights are read once: one stage, as many as the ring holds and more, the first row
 # that takes a second tile
 @pytest.mark.parametrize("k", floats.GEMM_K)
 @pytest.mark.parametrize("m,n,split,glu", [(33, 132, 132, 0), (64, 2060, 1030, 0), (64, 16380, 16380, 1), (65, 6144, 6144, 2), (100, 2048, 0, 0), (128, 12286, 12286, 0), (129, 6144, 6144, 0)])
 def test_one_row_tile(m, n, split, glu, k):
     floats.test_gemm_tiles(m, n, split, glu, k, "bfloat16")
+
+
+# one row tile and several, tiles of 64 to 256 rows, one stage of k and more than the ring holds
+@pytest.mark.parametrize("k", [64, 448, 2048])
+@pytest.mark.parametrize("n", [2048, 6144, 16384])
+def test_sums_of_a_row_are_the_same_on_every_tile(n, k):
+    """bfloat16: k is walked from its beginning everywhere, so that a row's sums are the same bit for bit however many rows there are."""
+    import numpy as np
+    from flexllm_amd import ops, to_device
+    from flexllm_amd.loader import to_bf16
+    r = np.random.default_rng(n + k)
+    a, w = to_bf16(r.standard_normal((1000, k)).astype(np.float32)), to_device(to_bf16(r.standard_normal((n, k)).astype(np.float32)))
+    want = ops.linear_float(to_device(a), w, 0, 0, 3.0)[1].numpy()
+    for m in 33, 64, 65, 100, 128, 129, 400:
+        assert np.array_equal(ops.linear_float(to_device(a[:m]), w, 0, 0, 3.0)[1].numpy(), want[:m]), m
 
 
 @pytest.mark.parametrize("rows,m,n", [(r, *FLOAT[r]) for r in FLOAT] + [(0, 129, 772), (0, 1300, 330), (0, 40, 132)])
