@@ -10,7 +10,9 @@ namespace fx {
 // weight rows 2i / 2i+1 are gate and up of unit i, and the gated unit of the pair leaves in column i); the columns from
 // n_split on leave as float32 in y32.  bias [n]: added to every row ahead of all that.  row_src: row r of A is read at row row_src[r].  tiles: grouped form, one weight
 // matrix per group (w_stride elements apart); rows of a group are contiguous in C, and tiles[i] = {group, first row,
-// end row, 0} for the *n_tiles tiles of `tile_rows` rows each.
+// end row, 0} for the *n_tiles tiles of `tile_rows` rows each.  from_memory: W will not be in the caches at its next use either, and where one row tile
+// reads it, it passes them by (bfloat16).
+constexpr size_t kCacheBytes = (size_t)256 << 20;       // of the memory-side cache
 struct GemmArgs {
     const void* a = nullptr; const void* w = nullptr;
     int lda = 0, ldw = 0, m = 0, n = 0, k = 0;           // ldw 0: rows of W are k long
@@ -23,6 +25,7 @@ struct GemmArgs {
     const int4* tiles = nullptr; const int* n_tiles = nullptr; int max_tiles = 0;
     size_t w_stride = 0;
     int group_rows = 0;                                   // rows that a group has on average
+    bool from_memory = false;
     int parts = 1; size_t part_stride = 0;                // n_split 0 only: k in `parts` parts, whose sums leave part_stride apart in y32
 };
 template <typename ET> int gemm_float(const GemmArgs& g, hipStream_t st);

@@ -503,9 +503,10 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
         g.n = g.n_split;
     }
     if (!g.row_src && gemm_few_ok(g.m, g.k, g.n, g.parts)) return gemm_few(g, st);
-    // With one row tile the weights are read once: past what the caches hold of the rows.  Whole prompts, us, read by ordinary loads and so: layers of 2048 (16),
-    // 33 rows 1196 and 1157, 64 1268 and 1252, 128 1416 and 1417; of 4096 (4), 33 760 and 734, 64 786 and 771, 128 867 and 852.
-    const bool one = g.m <= 64, one_wide = g.m <= 128;
+    // With one row tile the weights are read once: past what the caches hold of the rows, unless the caches hold the weights too.  Whole prompts, us, weights read by
+    // ordinary loads and past the caches: layers of 2048 (16), 33 rows 1196 and 1157, 64 1268 and 1252, 128 1416 and 1417; of 4096 (4), 33 760 and 734, 64 786 and 771, 128
+    // 867 and 852.  Layers of 1024, 64 rows, by all weights: 125 MB 261 and 283, 243 MB 444 and 484, 365 MB 668 and 634, 487 MB 868 and 825.
+    const bool one = g.from_memory && g.m <= 64, one_wide = g.from_memory && g.m <= 128;
     long cost;
     switch (gemm_cheapest_tile<bf16_t>(g, g.parts, cost)) {
         case 0: case 1: switch (gemm_wide_rows(g.m, g.k, g.n, g.parts)) {
@@ -528,14 +529,15 @@ int gemm_float<bf16_t>(const GemmArgs& args, hipStream_t st) {
 // per expert most of a wide tile's rows are none, and three workgroups per CU on 64 x 64 hide more of each other's trips.  Where an expert's rows are
 // one tile its weights are read once, past what the caches hold of the rows, and a die takes all columns of an expert: 64 rows 2394 -> 2265 us (a whole
 // prompt of 8 layers), 500 2886 -> 2793, 1024 3588 -> 3537.  Up to 112 rows on average on 128: at 122 many experts have two tiles (4230 -> 4239 us), at 188 4918 -> 5284.
+// Not where the caches hold all weights: 125 MB in two layers of 16 experts, 64 tokens 275 us and 290, 200 299 and 314; 250 MB 507 and 493, 536 and 528.
 template <int BM>
 static int gemm_grouped_bf16(const GemmArgs& args, hipStream_t st) {
     GemmArgs g = args;
     int rc = gemm_check(g, g.m, 2);
     if (rc) return rc;
-    if constexpr (BM == 128) return g.group_rows <= 112 ? launch_walk<bf16_t, 2, 4, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
-    else if (g.group_rows < 45) return launch_walk<bf16_t, 2, 2, 2, 3, 3, true>(g, st);
-    else return launch_walk<bf16_t, 2, 2, 4, 4, 4, true>(g, st);
+    if constexpr (BM == 128) return g.from_memory && g.group_rows <= 112 ? launch_walk<bf16_t, 2, 4, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 4, 4, 4, 4>(g, st);
+    else if (g.group_rows < 45) return g.from_memory ? launch_walk<bf16_t, 2, 2, 2, 3, 3, true>(g, st) : launch_walk<bf16_t, 2, 2, 2, 3, 3>(g, st);
+    else return g.from_memory ? launch_walk<bf16_t, 2, 2, 4, 4, 4, true>(g, st) : launch_walk<bf16_t, 2, 2, 4, 4, 4>(g, st);
 }
 
 // ---- float32 -----------------------------------------------------------------------------------------------------
@@ -583,6 +585,7 @@ int flexllm_linear_float_gemm(const void* a, const void* w, const float* bias, v
     GemmArgs g;
     g.a = a; g.w = w; g.lda = k; g.m = m; g.n = n; g.k = k; g.n_split = n_split; g.glu = glu; g.limit = limit; g.bias = bias;
     g.y = y; g.ldy = glu ? n_split / 2 : n_split; g.y32 = y32; g.ldy32 = n - n_split;
+    g.from_memory = n > 0 && k > 0 && (size_t)n * k * (dtype ? 4 : 2) > kCacheBytes;
     return dtype == 0 ? gemm_float<bf16_t>(g, as_stream(stream)) : gemm_float<float>(g, as_stream(stream));
 }
 

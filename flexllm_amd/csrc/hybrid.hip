@@ -79,6 +79,7 @@ struct flexllm_hybrid {
     float* g_final = nullptr;
     // largest sizes over the layers
     int max_et = 0, max_f32 = 0, max_att = 0, max_ff = 0, max_slots_ff = 1, max_shared = 0, max_route = 4, max_experts = 0, max_top = 1;
+    size_t weights = 0;                       // bytes of the matrices that every request reads
     size_t absorbed = 0;                      // scratch floats per token of the attention kernels for few tokens
     // one-token workspace
     float *x0 = nullptr, *xa = nullptr, *xb = nullptr, *proj = nullptr, *f32 = nullptr, *att = nullptr, *y = nullptr, *hn = nullptr, *hid = nullptr, *hs = nullptr, *route = nullptr;
@@ -149,7 +150,10 @@ struct Packer {
     ET* dst = nullptr;
     int k, kpad, next = 0;
     Packer(flexllm_hybrid* m_, int k_) : m(m_), k(k_), kpad(pad_k(k_)) {}
-    int alloc(size_t rows) { return halloc(m->owned, reinterpret_cast<void**>(&dst), rows * kpad * sizeof(ET)); }
+    int alloc(size_t rows) {
+        m->weights += rows * kpad * sizeof(ET);
+        return halloc(m->owned, reinterpret_cast<void**>(&dst), rows * kpad * sizeof(ET));
+    }
     int put(const uint16_t* src, int n, const char* what, int step = 1, int off = 0) {
         FX_REQUIRE(src, "hybrid_create: missing tensor %s", what);
         FX_TRY(pack_rows<ET>(as_bf16(src), dst + (size_t)next * kpad, n, k, kpad, step, off, nullptr));
@@ -547,6 +551,7 @@ static int create_model(flexllm_hybrid* m, const flexllm_hybrid_weights& w, cons
     FX_TRY(own_norm(m, m->g_final, w.final_norm, W, c.norm_add, "final.norm"));
     if (w.head == w.embed && std::is_same<ET, bf16_t>::value && pad_k(W) == W) {
         m->head = m->embed;                               // tied, and already in the head's layout
+        m->weights += (size_t)c.vocab * W * sizeof(ET);
     } else {
         Packer<ET> head(m, W);
         FX_TRY(head.alloc(c.vocab));
@@ -851,6 +856,7 @@ static int run_many(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T, 
     auto gemm = [&](const void* a, int lda, const void* w, int rows, int n, int k) {
         GemmArgs g;
         g.a = a; g.lda = lda; g.w = w; g.m = rows; g.n = n; g.k = pad_k(k);
+        g.from_memory = m->weights > kCacheBytes;
         return g;
     };
     // a product that the next row kernel takes in, which adds the parts that k is shared out in

@@ -126,6 +126,12 @@ def test_grouped_tiles_of_one_workgroup(experts, top, ff, tokens):
     check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=256), "bfloat16", tokens, [tokens], max_pos=max(512, tokens))
 
 
+# weights beyond the caches, which one row tile of 64 and of 128 rows reads past them, and two tiles do not: outputs that leave in whole pieces, and not
+@pytest.mark.parametrize("ff", [8192, 1030])
+def test_weights_beyond_the_caches(ff):
+    check_lopazen(lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff))], width=2048, vocab=66000), "bfloat16", 129, [129], [128, 1], [100, 29], [64, 65], [33], max_pos=160)
+
+
 # tiles of 64 x 64, 64 x 128 and 128 x 128, with more stages of k than the ring holds
 @pytest.mark.parametrize("tokens", [40, 50, 100])
 def test_experts_in_another_order(tokens):
