@@ -288,7 +288,7 @@ struct GemmWalk {
         int ka = NA - 1, kb = NB - 1;                            // stages kt - 1 + NA and kt - 1 + NB (as numbers: pointers cost the wide tiles spills)
         // left: stages behind this one.  loads: 2 all, 1 what is left for the last stages (the rest of the last barrier's, and W's where it is a stage
         // behind A), 0 none.  No branches among them: those cost a short walk 2 % (250 x 2560 x 2048 in four parts, eight stages on 128 x 128, 11.4 us and 11.2).
-        // turn, where another tile follows: 1 from the last k-step on A's loads are that one's, 2 W's are, 4 the next stage is that one's and is read behind the outputs.
+        // turn, where another tile follows: 1 from the last k-step on the loads are that one's, 2 the next stage is that one's and is read behind the outputs.
         auto turning = [&](int left, auto next, auto loads, auto turn) __attribute__((always_inline)) {
 #pragma unroll
             for (int s = 0; s < KS; s++) {
@@ -296,8 +296,13 @@ struct GemmWalk {
                 constexpr int kLoads = decltype(loads)::value;
                 constexpr int kTurn = decltype(turn)::value;
                 const bool last = s == KS - 1;
-                if constexpr (kTurn & 1) { if (last) { tiles.rows(offa); ka = -1; } }
-                if constexpr (kTurn & 2) { if (last) { tiles.cols(offb, w); kb = -1; } }
+                if constexpr (kTurn & 1) {
+                    if (last) {
+                        tiles.rows(offa);
+                        tiles.cols(offb, w);
+                        ka = kb = -1;
+                    }
+                }
                 if (last && kNext) {
                     if constexpr (kLoads > 0) wait_vmcnt<in_flight(NA - 2)>(); else wait_stage(left - 1);
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -310,7 +315,7 @@ struct GemmWalk {
                     constexpr int RS = NM / 2 / NR > 0 ? NM / 2 / NR : 1;
                     if (x % RS == 0 && x / RS < NR) {
                         if (!last) read(a1, b1, s + 1, (s + 1) & 1, x / RS);
-                        else if (kNext && !(kTurn & 4)) read(a2, b2, 0, (s + 1) & 1, x / RS);
+                        else if (kNext && !(kTurn & 2)) read(a2, b2, 0, (s + 1) & 1, x / RS);
                     }
                     // place behind the barrier of this stage (last k-step) or of the one before
                     const int p = last ? x : (s + 1) * NM + x;
@@ -336,13 +341,13 @@ struct GemmWalk {
         auto stage = [&](int left, auto next, auto loads) __attribute__((always_inline)) { turning(left, next, loads, std::integral_constant<int, 0>()); };
         int left = nk - 1;
         if constexpr (T::kMany) {
+            static_assert(NA == NB, "rows and columns turn to the next tile in the same stage");
             using All = std::integral_constant<int, 2>;
             while (tiles.more()) {
                 for (; left >= NA; left--) stage(left, std::true_type(), All());
-                if constexpr (NA > NB) turning(left--, std::true_type(), All(), std::integral_constant<int, 1>());
-                turning(left--, std::true_type(), All(), std::integral_constant<int, (NA > NB ? 2 : 3)>());
+                turning(left--, std::true_type(), All(), std::integral_constant<int, 1>());
                 for (; left >= 1; left--) stage(left, std::true_type(), All());
-                turning(0, std::true_type(), All(), std::integral_constant<int, 4>());
+                turning(0, std::true_type(), All(), std::integral_constant<int, 2>());
                 tiles.out(acc);
                 clear();
 #pragma unroll

@@ -126,6 +126,27 @@ def test_grouped_tiles_of_one_workgroup(experts, top, ff, tokens):
     check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=256), "bfloat16", tokens, [tokens], max_pos=max(512, tokens))
 
 
+def by_experts(mlp, w, pre, h):
+    """nifunex_ref.mixture, an expert's rows at a time."""
+    out = np.zeros_like(h)
+    picks = [nifunex_ref.route(z, mlp["router"]["top"]) for z in h @ w[pre + "router"].T]
+    for e in range(mlp["router"]["experts"]):
+        rows = [(t, a) for t, (pick, wt) in enumerate(picks) for i, a in zip(pick, wt) if i == e]
+        if rows:
+            t, a = np.array([r[0] for r in rows]), np.array([r[1] for r in rows])
+            out[t] += a[:, None] * nifunex_ref.feed_forward(w, "%se%d." % (pre, e), h[t], mlp["expert"]["limit"])
+    return out
+
+
+# more tiles than CUs, and k of more stages than the ring holds: an odd number of them, so that tiles begin at every place of it, and not.  Where all weights lie in the
+# caches (100 MB and less) tiles of 128 rows; beyond them (more than 256 MiB) tiles of 64 and of 128 rows, gate/up and down products with several tiles per workgroup
+@pytest.mark.parametrize("experts,top,ff,tokens,width", [(8, 2, 1032, 700, 320), (8, 2, 2056, 700, 448), (6, 2, 2048, 700, 1024),
+                                                         (22, 2, 2048, 520, 1024), (21, 2, 2048, 500, 1088), (22, 2, 1088, 900, 2048), (21, 2, 2048, 900, 1088)])
+def test_grouped_tiles_of_many_stages(experts, top, ff, tokens, width, monkeypatch):
+    monkeypatch.setattr(nifunex_ref, "mixture", by_experts)
+    check_nifunex(nc.config([nc.gla(heads=1, mlp=nc.moe(experts, top, ff, 1.5, 0))], width=width), "bfloat16", tokens, [tokens], max_pos=1024)
+
+
 # weights beyond the caches, which one row tile of 64 and of 128 rows reads past them, and two tiles do not: outputs that leave in whole pieces, and not
 @pytest.mark.parametrize("ff", [8192, 1030])
 def test_weights_beyond_the_caches(ff):
