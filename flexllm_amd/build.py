@@ -66,7 +66,7 @@ def build(verbose=False, jobs=8, srcs=None, out=LIB, obj_dir=os.path.join(CSRC, 
 
 # Kernels that count their loads in flight themselves and hold nearly as many sums as there are registers.  They have to do without memory of
 # the compiler's own: a form of the wide GEMMs that spilled sums gave wrong ones on some sizes, for a reason that was not found.
-WITHOUT_SPILLS = ("gemm_float_walk_kernel", "gemm_float_groups_kernel", "gemm_i8_walk_kernel", "gemm_i8_dma_kernel", "gemm_few_kernel", "gemv_mfma_kernel")
+WITHOUT_SPILLS = ("gemm_float_walk_kernel", "gemm_float_groups_kernel", "gemm_i8_walk_kernel", "gemm_i8_dma_kernel", "gemm_few_kernel", "gemv_mfma_kernel", "walk_kernel")
 
 
 def resources(out):

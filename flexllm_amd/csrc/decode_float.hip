@@ -790,6 +790,7 @@ struct Service {
         return v;
     }
     __device__ __forceinline__ void embed(int token) {
+        const int t = opaque();
 #pragma unroll
         for (int i = 0; i < QW; i++) x[i] = embedding(token, min(t + kSvcT * i, a.width / 4 - 1));
     }
@@ -1516,13 +1517,14 @@ struct Service {
                 }
             sums_there();
             int r0;
-            const int rows = rows_of(2 * r->ff, r0);
+            const int t = opaque(), rows = rows_of(2 * r->ff, r0);
             for (int j = t; j < rows / 2; j += kSvcT)
                 put(r->x_hid + (unsigned)(r0 / 2 + j), glu_f(r->glu, total(W, 2 * j), total(W, 2 * j + 1), r->limit));
             sums_done();
             take(r->x_hid, r->ff);
             plain(W, r->ff, r->x_y2, nullptr);
         }
+        const int t = opaque();
         if (!choose && t < 2) unput(a.x_cand + (unsigned)(2 * wg + t));        // what is not handed out in this step is unset behind the last one all the same
         if (!a.head) return 0;
         norm(have, y, gb, a.g_final, -1);
@@ -1604,20 +1606,21 @@ __global__ __launch_bounds__(kWalkT) void walk_kernel(WalkArgs a, int slots, Res
         if (blockIdx.x == 0 && threadIdx.x == 0) a.state[3] = 2;
         token = 0;
     }
+    const auto first = [&] { return blockIdx.x == 0 && s.opaque() == 0; };
     for (int i = 0; i < a.steps; i++) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");             // rows that other workgroups stored a token ago
         const int set = (a.parity + i) & 1;
         s.now = a.words + set * a.set;
         s.other = a.words + (1 - set) * a.set;
         token = s.step(token, pos0 + i, a.tokens_out != nullptr);
-        if (a.tokens_out && blockIdx.x == 0 && threadIdx.x == 0) a.tokens_out[step0 + i] = token;
+        if (a.tokens_out && first()) a.tokens_out[step0 + i] = token;
     }
-    if (a.tokens_out && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (a.tokens_out && first()) {
         a.token[0] = token;
         a.state[0] = pos0 + a.steps;
         a.state[1] = step0 + a.steps;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) resident_done(end);
+    if (first()) resident_done(end);
 }
 
 // What the ring of the stream waves is given besides: as much as is left, in slots of a quad for each of them.

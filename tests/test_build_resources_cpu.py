@@ -18,7 +18,7 @@ __global__ __launch_bounds__(1024, 8) void NAME(const float* x, float* y) {
 """
 
 
-@pytest.mark.parametrize("name,refused", [("gemm_few_kernel", True), ("some_kernel", False)])
+@pytest.mark.parametrize("name,refused", [("gemm_few_kernel", True), ("walk_kernel", True), ("some_kernel", False)])
 def test_spills(tmp_path, name, refused):
     src = tmp_path / "k.hip"
     src.write_text(SOURCE.replace("NAME", name).replace("for (int i", "_Pragma(\"unroll\") for (int i"))
