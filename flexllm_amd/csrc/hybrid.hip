@@ -681,16 +681,19 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 
 // A linear behind a norm, for T tokens of a step: every token reads the weights (from L2, behind the first) under its own norm's
 // prologue while the bytes read again are few, else the norms have a launch of their own (3.7 us) ahead of one pass over the weights.
-// bfloat16, 16 layers of 2048, whole steps, us, by tokens, where up to four read rows of 4 KiB again whatever their number, and now: 2 946 and 925, 3 1050
-// and 960, 4 1117 and 942; with a recurrence in every second layer 1129 and 1084, 1293 and 1148, 1402 and 1204.  Limits of 0, 20 and 40 MiB are
-// the same to 1 % there; a mixture's shared linears (17 MB) want to be read again by two tokens: 836 with 0, 812 with 20, 790 with 40.
+// bfloat16: while 40 MiB are, or less than 64 for two to four tokens and rows of at most 4 KiB (a product whose sum the next one's prologue takes in: less
+// than 32).  Whole steps, us, by tokens, with one pass from 40 MiB on and down products always in one pass, and where up to four tokens read rows of 4 KiB again
+// whatever their number: 8 layers of 1024, feed-forward 4096, 2 (16 MiB) 342 and 320, 3 (32) 364 and 346, 4 (48) 368 and 354; feed-forward 8192, 2 (32) 398 and 381, 3 (64)
+// 413 and 420, 4 (96) 397 and 432; 8 layers of 512, 2048, 2 to 4 tokens 324 and 294, 318 and 287, 332 and 302; of 1536, 6144, 2 (36) 416 and 383, 3 (72) 434 and 427, 4 (108)
+// 430 and 440; 6 layers of 2048, 4096, 2 (32) 329 and 312, 3 (64) 346 and 346, 4 (96) 345 and 370; 8192, 2 (64) 383 and 386, 3 390 and 428.  Longer rows, 4 layers of 2560, 2
+// tokens (80 MiB) 342 and 382, of 3072 (96) 365 and 411.  A mixture's shared linears (17 MB) want to be read again by two tokens: 836 with a limit of 0, 812 with 20, 790 with 40.
 // float32: rows of at most 4 KiB, a piece per thread, up to four tokens.  Longer rows and more tokens while the bytes read again are few.  A mixture of 8
 // layers of 2048, four tokens, 4161 rows (97 MiB) read again or not: 1369 and 1404 us; five tokens (130 MiB) 1655 and 1686; 16 layers of 2048, two
 // tokens, 16384 rows (128 MiB): 1541 and 1453, five, 3072 rows (96 MiB): 1680 and 1750; four layers of 4096 (16 KiB), four tokens, up to 240 MiB: 1224 and 1175.
 static bool short_rows(int kpad, int es) { return kpad * es <= 4096; }
 static bool reads_again(int T, int n, int kpad, int es) {
     const size_t again = (size_t)(T - 1) * n * kpad * es;
-    if (es == 2) return again <= (size_t)40 << 20;
+    if (es == 2) return again <= (size_t)40 << 20 || (T <= 4 && short_rows(kpad, es) && again < (size_t)64 << 20);
     return T == 1 || (T <= 4 && short_rows(kpad, es)) || again <= (size_t)(kpad * es > 8192 ? 72 : T == 2 ? 104 : 240) << 20;
 }
 
@@ -782,7 +785,10 @@ static int run_small(flexllm_hybrid* m, HybridSlot& s, const int* tokens, int T,
             a = base(L.w_gu, 2 * L.d.ff, W);
             a.n_split = 2 * L.d.ff; a.glu = 1 + L.d.glu; a.limit = L.d.limit; a.out = m->hid; a.ldo = L.d.ff;
             FX_TRY(norm_linear(a, L.g2));
-            FX_TRY(to_y(L.w_d, L.d.ff, m->hid, L.d.ff, L.g2b, true));
+            // in parts, unless the next linear takes the sum as it is and the weights read again are few
+            const bool whole = T <= 4 && short_rows(kw, sizeof(ET)) && (size_t)(T - 1) * W * pad_k(L.d.ff) * sizeof(ET) < (size_t)32 << 20 && r + 1 < runs &&
+                               reads_again(T, m->layers[m->runs[r + 1].layer].n_in, kw, sizeof(ET));
+            FX_TRY(to_y(L.w_d, L.d.ff, m->hid, L.d.ff, L.g2b, !whole));
         } else if (L.d.ff_kind == FLEXLLM_FF_MOE) {
             const int sf = L.d.shared_ff, ldr = L.n_side - 2 * sf;
             a = base(L.w_side, L.n_side, W);

@@ -218,8 +218,9 @@ def test_experts_down(top, ff, shared, width, dtype):
     check_nifunex(cfg, dtype, 20, [1], [3])
 
 
-# gate/up weights that two tokens of a step just still read again, and just not; three and four tokens do not
-@pytest.mark.parametrize("ff", [5120, 5121])
+# gate/up weights that two tokens of a step just still read again, and just not (8191 and 8192; as many as longer rows could be: 5120 and 5121), down products whose
+# sums leave whole, and in parts; three and four tokens do not read them again
+@pytest.mark.parametrize("ff", [5120, 5121, 8191, 8192])
 def test_step_of_several_tokens_reads_weights_once(ff):
     check_lopazen(lc.config([lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(ff)), lc.layer(heads=2, kv_heads=1, dim=32, mlp=lc.dense(72))], width=2048),
                   "bfloat16", 12, [2], [3], [4])
