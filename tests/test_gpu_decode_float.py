@@ -370,6 +370,7 @@ NOT_FINITE = {
     "latent rows and gla": (NIFUNEX["both kinds"], ["l0.mix.dkv", "l1.mix.v", "l1.mlp.gate"]),
     "mixtures": (nc.config([gla(16, 0) | dict(mlp=nc.moe(8, 3, 1024, 0.75, 2048)), latent(16, 0, window=None) | dict(mlp=nc.moe(8, 3, 1024, 0.75, 2048))], width=2048, vocab=512),
                  ["l0.mlp.router", "l0.mlp.shared.up", "l1.mlp.shared.sg"]),
+    "rows of 12 blocks": (lc.config([attention(32, 8, 64, 6144)], width=2048, vocab=512), ["l0.mlp.down"]),
 }
 
 
@@ -430,6 +431,71 @@ def test_what_is_not_finite(name, dtype):
         finite = np.isfinite(chain).all(0)
         if finite.any():
             assert cases.rel_err(got[:, finite], chain[:, finite]).max() < cases.LIMIT[dtype]
+
+
+# an infinite weight in rows of 12 blocks of k and of 28, of which a wave has one or two and three or four, in a wave's first block and in a later one; in rows of four
+# blocks, in the query in a workgroup's last group of two rows instead of four; clamped gates and units, which leave finite logits (a gate where it is above zero).
+# "units": two hidden values beyond float32 instead, where their gates are above zero.  What is not finite behind a down product is no number in all logits.
+LONG_ROWS = [(6144, "l0.mlp.down", 0, 3), (6144, "l0.mlp.down", 1031, 6000), (14336, "l0.mlp.down", 1029, 11000), (6144, "l0.mix.q", 1029, 2000),
+             (6144, "l0.mlp.gate", 3071, 5), (6144, "l0.mlp.up", 6143, 2047), (14336, "l0.mlp.up", 77, 1030), (6144, "units", 700, 5000), (14336, "units", 5, 14000)]
+
+
+@BOTH
+@pytest.mark.parametrize("ff,name,row,col", LONG_ROWS)
+def test_not_finite_in_long_rows(ff, name, row, col, dtype):
+    """The places that are no number, infinite and finite are those of the chain of kernels, and the finite ones agree."""
+    from flexllm_amd.registry import model_class
+    clamped = name.endswith(("gate", "up"))
+    cfg = nc.config([gla(16, ff)], width=2048, vocab=514) if clamped else lc.config([attention(32, 8, 64, ff)], width=2048, vocab=514)
+    w = (nc if clamped else lc).weights(cfg, 5)
+    if name == "units":
+        for unit in row, col:
+            w["l0.mlp.gate"][unit] = lc.round_bf16(w["l0.mlp.gate"][unit] * np.float32(1e4))
+            w["l0.mlp.up"][unit] = lc.round_bf16(w["l0.mlp.up"][unit] * np.float32(1e36))
+            w["l0.mlp.down"][::3, unit] = 0.0              # no number with an infinite unit
+    else:
+        w[name][row, col] = np.inf
+    m = model_class(cfg["architecture"]).from_tensors(cfg, w, dtype=dtype, max_pos=64, slots=2)
+    got = []
+    for i, mode in enumerate((0, 1)):
+        m.set_decode_mode(mode)
+        slot = m.pool.acquire(str(i))
+        got.append(np.stack([m.step(slot, [t], [0])[0] for t in (7, 100, 33, 250, 4, 19, 60, 301)]))
+        m.check()
+    m.close()
+    for kind in np.isnan, np.isposinf, np.isneginf:
+        assert np.array_equal(kind(got[0]), kind(got[1])), kind
+    finite = np.isfinite(got[1]).all(1)
+    assert finite.all() == name.endswith("up") and (finite.any() or not clamped)
+    if clamped:                                            # (the tail of a gelu times a unit of 1e36 is finite and has no digits to agree in)
+        assert lc.rel_err(got[0][finite], got[1][finite]).max() < lc.LIMIT[dtype]
+
+
+# a head of so many rows that its sums leave no room for a vector in three parts: bfloat16 weights meet it as it is, waves meet by counts all the same
+@pytest.mark.parametrize("kind", ["shared rows", "latent rows and gla"])
+def test_vectors_that_lie_whole(kind):
+    from flexllm_amd._lib import FlexLLMError
+    from flexllm_amd.lopazen import Lopazen
+    from flexllm_amd.nifunex import Nifunex
+    vocab = 600064                                         # 2344 rows per workgroup, 8 sums each: 73 KiB beside 24 KiB of the vector
+    if kind == "shared rows":
+        m = Lopazen.synthetic(lc.config([attention(32, 8, 64, 6144), attention(32, 8, 64, 2048)], width=4096, vocab=vocab), dtype="bfloat16", max_pos=64, slots=2)
+    else:
+        m = Nifunex.synthetic(nc.config([latent(16, 6144, window=40), gla(16, 2048)], width=4096, vocab=vocab), dtype="bfloat16", max_pos=64, slots=2)
+    toks, got = [7, 100, 599999, 250, 4, 300001], []
+    for i, mode in enumerate((0, 1)):
+        m.set_decode_mode(mode)
+        slot = m.pool.acquire(str(i))
+        got.append(np.stack([m.step(slot, [t], [0])[0] for t in toks]))
+        m.check()
+    # Both have float32 activations; what may differ are cached rows, on one side or the other of a bfloat16 step: 2^-8 at worst.
+    assert lc.rel_err(got[0], got[1]).max() < 2.0 ** -8
+    m.set_decode_mode(0)
+    m.set_wait_limit(1)                                    # it is the resident kernel that they take
+    m.pool.release("0")
+    with pytest.raises(FlexLLMError, match="timed out"):
+        m.step(m.pool.acquire("0"), [1], [0])
+    m.close()
 
 
 def test_two_models_on_streams_of_their_own():
