@@ -106,9 +106,10 @@ inline int walk_splits(int heads, int dim) {
 __host__ __device__ constexpr int walk_part(int dim) { return dim + 4; }
 // Rows up to which this is the faster way.  A split's workgroup reads its rows for one query head, 43 us per MB; the kernels of the chain
 // (shared_kv_attn.hip) read a row once for up to four heads, in up to eight times as many splits, but have a few us of launches in every layer, more
-// beside wider linears.  Two layers, 32 heads on 8 of 64, width 2048, bfloat16, us per token in one kernel and in the chain: 24000 rows 93 and 100,
-// 32000 104 and 105, 48000 125 and 113, 128000 255 and 156.  The two meet at 0.53 to 0.88 MB per split there (widths of 2048, heads of 64
-// and 128, alone on their rows and up to eight, both types), 0.51 at 1024, 0.86 to 1.25 at 4096: the line is within 7 % of the better side.
+// beside wider linears.  Two layers, 32 heads on 8 of 64, width 2048, bfloat16, us per token in one kernel and in the chain: 24000 rows 94 and 98,
+// 32000 104 and 103, 48000 125 and 110; four layers with feed-forwards of 8192 at 32000 rows 235 and 250.  With two layers the two meet at 0.5 to 0.8 MB per split (widths
+// of 2048, heads of 64 and 128, alone on their rows and up to eight, both types), 0.51 at 1024, 0.75 to 1.2 at 4096; more layers' linears move that on: the
+// line is within 12 % of the better side.
 inline int walk_shared_kv_rows(const SharedKvDims& d, int width, int es) {
     const long long per_split = (384 * 1024 + 160LL * width) / ((long long)d.dim * es);
     return (int)(per_split * walk_splits(d.heads, d.dim));

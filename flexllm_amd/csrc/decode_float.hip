@@ -9,9 +9,16 @@
 // bfloat16 products on the matrix cores, the vector as three parts: 595 -> 566 us per token, with latent and recurrent layers in turn 713 -> 692, with mixtures
 // 520 -> 516; four layers of 4096, whose quads are the weights' stream, 462 and 461, 522 and 525.
 // Eight of a workgroup's twelve waves ("stream waves") do nothing but walk through the workgroup's rows of all linears.  The other four ("service
-// waves") wait for the vectors, norm them, attend, finish the sums.  They meet at workgroup barriers: the vector is in LDS / the sums
-// are in LDS.  Answers of vector memory return to a wave in order, so a wave that streams could not see a word of another workgroup before its weights.
-//
+// waves") wait for the vectors, norm them, attend, finish the sums.  Answers of vector memory return to a wave in order, so a wave that streams could not see a word of
+// another workgroup before its weights.
+// The two kinds meet twice in every linear, by counts in LDS that are added to with release and read with acquire (kFree), in models with mixtures at workgroup barriers in
+// the same two places:
+//   L.ready, one from each service wave: its share of the vector is in LDS, and it has read the sums of the linear before.  Behind all four the stream waves read the
+//     vector and write sums.
+//   L.done, one from each stream wave: its sums are in LDS, and it has read the vector for the last time.  Behind all eight the service waves read the sums, and the vector's
+//     place is theirs: the mixers' values lie over it, until all service waves have met (take, norm) and put the next vector there.  The head's sums, which may lie
+//     behind its vector where a longer one would, are read before the service waves meet in the next token's first norm.
+//   L.sent guards nothing: stream waves ask for more once the sums have left, so that the words stand ahead of their requests.
 // Words between workgroups: a float32 goes past the L2 caches (which do not see each other's lines) to a place of its own per layer run,
 // which holds kUnset until then; readers poll the places themselves, 16 bytes per lane.  There are two sets of places, for tokens in
 // turn: who writes a word of one set puts kUnset back in the other one, whose readers were done a token ago (a token ends with an exchange that all
@@ -139,7 +146,7 @@ struct WalkLds {                                          // ahead of the tables
 // number.  Each wave has a ring of `slots` quads in LDS.  The trip is direct (the compiler does not see it: a wait names how many
 // younger quads are on their way), so a request holds no register and may be made at any time.  When it is made matters: a CU takes
 // 32 KiB of requests or so, then the wave that asks stands still until bytes arrive.  Freed slots are therefore filled at once only from the same
-// linear; what belongs to the next ones is asked for behind the barrier that hands the sums on, beside the exchange.  (With register buffers that the
+// linear; what belongs to the next ones is asked for behind the sums, beside the exchange.  (With register buffers that the
 // compiler waits for, refilled on the spot, the last products of a linear wait until the next one's first quads are asked for: gate/up of
 // 16384 x 2048 8.7 us behind a full ring, 7.1 so.  Eight waves: with four, one per SIMD, a quad's 100 instructions are not hidden, 13 us.)
 __device__ __forceinline__ void quad_to_lds(const char* base, unsigned voff, unsigned dst) {
@@ -355,7 +362,8 @@ __device__ __forceinline__ void stream_waves(WalkLds& L, WalkTables T, const flo
 // bfloat16 parts to 24 bits, and their products with the weights are exact in float32.  An instruction (16 x 16 x 32) takes 256 bytes of each row: its rows
 // are 4 weight rows x 4 pieces of k, its columns 3 parts x the same 4 pieces, and where the pieces meet are the sums.  So 512 weights take one
 // instruction for 20 of a lane's own, operands come in requests of 1 KiB of one row, and a wave that stays in a block of k keeps the vector in 16 registers.
-// In LDS 16 bytes c of row r lie at place c ^ 2r, of part p at c ^ 2p: eight lanes that read together are on different banks.
+// In LDS 16 bytes c of row r lie at place c ^ 2r, of part p at c ^ 2p: eight neighbouring lanes that read 16 bytes each are on different banks.  (Counted: a quad takes 86
+// cycles of its CU's LDS, 23 of them conflicts; the matrix cores are busy for 3 % of a token.)
 __device__ __forceinline__ void block_to_lds(const char* base, const unsigned (&voff)[4], unsigned dst) {
     unsigned saved_m0;
     asm volatile("s_mov_b32 %0, m0\n\t"

@@ -685,8 +685,8 @@ static int many_workspace(flexllm_hybrid* m, int rows) {
 // than 32).  Whole steps, us, by tokens, with one pass from 40 MiB on and down products always in one pass, and where up to four tokens read rows of 4 KiB again
 // whatever their number: 8 layers of 1024, feed-forward 4096, 2 (16 MiB) 342 and 320, 3 (32) 364 and 346, 4 (48) 368 and 354; feed-forward 8192, 2 (32) 398 and 381, 3 (64)
 // 413 and 420, 4 (96) 397 and 432; 8 layers of 512, 2048, 2 to 4 tokens 324 and 294, 318 and 287, 332 and 302; of 1536, 6144, 2 (36) 416 and 383, 3 (72) 434 and 427, 4 (108)
-// 430 and 440; 6 layers of 2048, 4096, 2 (32) 329 and 312, 3 (64) 346 and 346, 4 (96) 345 and 370; 8192, 2 (64) 383 and 386, 3 390 and 428.  Longer rows, 4 layers of 2560, 2
-// tokens (80 MiB) 342 and 382, of 3072 (96) 365 and 411.  A mixture's shared linears (17 MB) want to be read again by two tokens: 836 with a limit of 0, 812 with 20, 790 with 40.
+// 430 and 440; 6 layers of 2048, 4096, 2 (32) 329 and 312, 3 (64) 346 and 346, 4 (96) 345 and 370; 8192, 2 (64) 383 and 386, 3 390 and 428.  Longer rows, 2
+// tokens, 4 layers of 2560 (80 MiB) 342 and 382, of 3072 (96) 365 and 411, 3 of 4096 (224, too many for either) 410 and 410.  A mixture's shared linears (17 MB) want to be read again by two tokens: 836 with a limit of 0, 812 with 20, 790 with 40.
 // float32: rows of at most 4 KiB, a piece per thread, up to four tokens.  Longer rows and more tokens while the bytes read again are few.  A mixture of 8
 // layers of 2048, four tokens, 4161 rows (97 MiB) read again or not: 1369 and 1404 us; five tokens (130 MiB) 1655 and 1686; 16 layers of 2048, two
 // tokens, 16384 rows (128 MiB): 1541 and 1453, five, 3072 rows (96 MiB): 1680 and 1750; four layers of 4096 (16 KiB), four tokens, up to 240 MiB: 1224 and 1175.
