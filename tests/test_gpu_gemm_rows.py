@@ -65,6 +65,23 @@ def test_sums_of_a_row_are_the_same_on_every_tile(n, k):
         assert np.array_equal(ops.linear_float(to_device(a[:m]), w, 0, 0, 3.0)[1].numpy(), want[:m]), m
 
 
+def test_weights_beyond_the_caches():
+    """A product whose weights are more than 256 MiB reads them past the caches where one row tile does: the same bit for bit as its halves, which do not."""
+    import numpy as np
+    from flexllm_amd import ops, synth, to_device
+    from flexllm_amd.loader import to_bf16
+    k, half = 2048, 35002
+    w = synth.device_uniform_bf16((2 * half, k), 7, -1.0, 1.0)
+    parts = [to_device(p) for p in np.split(w.numpy(), 2)]
+    a = to_bf16(np.random.default_rng(3).standard_normal((129, k)).astype(np.float32))
+    for m in 33, 64, 65, 100, 128, 129:
+        x = to_device(a[:m])
+        for split, glu in (0, 0), (half, 2):               # all columns float32; gated units
+            got = ops.linear_float(x, w, 2 * split, glu, 3.0)[not split].numpy()
+            want = np.concatenate([ops.linear_float(x, p, split, glu, 3.0)[not split].numpy() for p in parts], 1)
+            assert np.array_equal(got, want), (m, glu)
+
+
 @pytest.mark.parametrize("rows,m,n", [(r, *FLOAT[r]) for r in FLOAT] + [(0, 129, 772), (0, 1300, 330), (0, 40, 132)])
 @pytest.mark.parametrize("cut", [0, 2])
 def test_unit_behind_a_bias(rows, m, n, cut):
